@@ -1685,7 +1685,8 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             if (L.attn_mfma && kv_mode == KV_BF16 && !all_decode && max_n >= 16 && lay_attn_mfma_fits(dk, ev, a.vpool != nullptr)) {
                 const auto& tm = tiles64[sp.heads / sp.kv_heads];
                 a.tiles = (const int2*)(L.d_tab + tm.first); a.ntiles = tm.second;
-                launch_lay_attn_mfma(a, s);
+                if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) launch_lay_attn_tile(a, s);
+                else launch_lay_attn_mfma(a, s);
             } else
                 launch_lay_attn(a, kv_mode, s);
         };

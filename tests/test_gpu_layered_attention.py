@@ -1,0 +1,89 @@
+"""GPU: the tiled matrix-core attention of prompt passes (kernels_layered_attn.hip) against the f32 FMA kernel on the same cache, at the
+edges of its tiles and masks.
+
+One attention layer without a feed-forward, bfloat16 format, the same portions with the matrix-core kernels on and off.  Both read the same
+pages; the matrix cores read the query rounded to bfloat16 where the FMA kernel keeps 32 bits.  With keys and queries of unit variance
+that moves a score by 2^-9 / sqrt(3) = 1.1e-3 in the mean square (d independent roundings of d products of size d^-1/2), the weights by the
+same share and the largest logit by no more; everything else (weights as a 16-bit hi + lo pair, exp and log of the hardware units, the
+bfloat16 rounding of the attention rows on their way into the output projection, which tips 0.3 % of the elements over) is below 3e-4.
+8e-3 of the largest logit is seven times that."""
+import numpy as np
+import pytest
+
+from tests import gibipel_util as GI
+from tests import gizezen_util as GZ
+from tests import korupel_util as KO
+from tests import mononex_util as MO
+
+pytestmark = pytest.mark.gpu
+
+TOL = 8e-3
+
+
+def _run(tmp_path, U, cfg, portions, seed, **kw):
+    """Logits of every fourth position and of the last 70, with the matrix-core kernels on, then off."""
+    from crane_amd.backend import Model
+    P = U.random_weights(cfg, seed)
+    n = sum(portions)
+    toks = U.tokens(n, cfg["vocab"], seed + 1)
+    m = Model.from_pretrained(U.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=4, max_seq_len=2048, **kw)
+    try:
+        got = []
+        for on in (1, 0):
+            m.debug_set("lay_attn_mfma", on)
+            s, at, rows = m.seq_alloc(), 0, []
+            for k in portions:
+                want = [i for i in range(k) if i % 4 == 0 or i >= k - 70]
+                rows.append(m.step_batch([(s, toks[at:at + k], want)])[0])
+                at += k
+            got.append(np.concatenate(rows).astype(np.float64))
+            m.seq_free(s)
+        return got
+    finally:
+        m.close()
+
+
+def _check(got):
+    assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() < TOL * np.abs(got[1]).max()
+
+
+# key / value sizes on both sides of the padded sizes (64, 128); query rows per position 1, 3, 4; portions that start inside a tile and
+# end on, before and behind a tile's edge; windows shorter than a tile, around it and over the whole context
+@pytest.mark.parametrize("d,e,heads,kv,size,portions", [
+    (16, 16, 4, 4, 7, (65, 16, 130)), (64, 80, 6, 2, 64, (100, 200)), (80, 64, 4, 1, 65, (63, 64, 65)), (128, 128, 8, 2, 1000, (300, 17)),
+    (112, 128, 4, 1, 128, (190, 150)), (96, 48, 3, 3, 200, (64, 128, 100))])
+@pytest.mark.parametrize("page", [64, 128])
+def test_window_and_one_in_the_denominator(tmp_path, d, e, heads, kv, size, portions, page):
+    mx = GZ.attn(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size, rot_dims=16)
+    _check(_run(tmp_path, GZ, GZ.config([GZ.layer(mx, None)], vocab=96, width=64), portions, 3, kv_block_size=page))
+
+
+# first tokens kept in front of the window (fewer than a tile, more than a tile, reaching into the window), a logarithmic distance term,
+# values that are the keys
+@pytest.mark.parametrize("d,heads,kv,size,keep,portions", [(32, 4, 2, 20, 3, (70, 150)), (128, 4, 1, 90, 70, (100, 260)), (48, 5, 5, 300, 128, (330,)),
+                                                           (64, 2, 1, 5, 64, (130, 67))])
+def test_kept_first_tokens_and_distance_term(tmp_path, d, heads, kv, size, keep, portions):
+    mx = KO.attn(heads=heads, kv_heads=kv, dim=d, size=size, keep_first=keep)
+    _check(_run(tmp_path, KO, KO.config([KO.layer("attention", None, **mx)], vocab=96, width=64), portions, 5))
+
+
+# position blocks (a query sees its own block only), a linear distance term, a sink, a gate per element; block edges on and off tile edges
+@pytest.mark.parametrize("d,e,heads,kv,size,portions", [(32, 16, 6, 2, 50, (200, 30)), (128, 112, 4, 2, 64, (129, 70)), (64, 64, 2, 2, 200, (150, 150))])
+def test_position_blocks_and_sink(tmp_path, d, e, heads, kv, size, portions):
+    mx = MO.attn(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size)
+    _check(_run(tmp_path, MO, MO.config([MO.layer("attention", None, **mx)], vocab=96, width=64), portions, 7))
+
+
+# mean rows of the blocks in front of the window: fewer than a tile of them, more than a tile, blocks that end in another page
+@pytest.mark.parametrize("d,e,heads,kv,size,pool,portions", [(32, 16, 4, 2, 20, 6, (120, 100)), (128, 128, 4, 1, 30, 4, (300, 40)), (64, 96, 2, 2, 70, 64, (250, 65))])
+def test_block_rows(tmp_path, d, e, heads, kv, size, pool, portions):
+    lf = GI.left(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size, pool=pool)
+    cfg = GI.config([GI.layer(lf, GI.right(), None)], vocab=96, width=64)
+    _check(_run(tmp_path, GI, cfg, portions, 9))
+
+
+# many key heads and query blocks, window shorter than the portion
+@pytest.mark.parametrize("d,e,size,portions", [(16, 16, 300, (1025,)), (128, 128, 2000, (40, 1100)), (64, 80, 33, (1090,))])
+def test_many_heads(tmp_path, d, e, size, portions):
+    mx = GZ.attn(heads=64, kv_heads=64, dim=d, vdim=e, size=size, rot_dims=16)
+    _check(_run(tmp_path, GZ, GZ.config([GZ.layer(mx, None)], vocab=96, width=64), portions, 11))
