@@ -6,31 +6,11 @@
 
 #include "dev_common.h"
 #include "layered.h"
+#include "layered_dev.h"
 
 namespace cm {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-__device__ __forceinline__ float lay_act(float v, int act, float param = 1.f) {
-    switch (act) {
-        case LACT_RELU2: { const float r = fmaxf(v, 0.f); return r * r; }
-        case LACT_LOGSIG: return param * (fminf(v, 0.f) - log1pf(expf(-fabsf(v))));      // ln sigmoid(v), no overflow either way
-        case LACT_SOFTCAP: return param * tanhf(v / param);
-        case LACT_SILU: return v / (1.f + __expf(-v));
-        case LACT_SIGMOID: return 1.f / (1.f + __expf(-v));
-        case LACT_GELU_TANH: {
-            const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
-            return 0.5f * v * (1.f + tanhf(u));
-        }
-        default: return v;
-    }
-}
-// capped gated product: g = min(g, cap), u = clamp(u, -cap, cap): g sigmoid(1.702 g) (u + 1)
-__device__ __forceinline__ float lay_capglu(float g, float u, float cap) {
-    g = fminf(g, cap);
-    u = fminf(fmaxf(u, -cap), cap);
-    return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
-}
 
 // sum over the block (blockDim.x a multiple of 64, every thread calls); red: >= blockDim.x / 64 floats of LDS
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -712,7 +692,7 @@ __global__ __launch_bounds__(256) void lgemm_bf16_kernel(LGemmArgs a) {
 // few rows (decode steps): the matrix is streamed ONCE with 16-byte non-temporal loads, one wave per two output columns, every
 // row of A (at most LV_MAXM, L2-resident) against each weight fragment; the wave's lanes split K.  bfloat16 format: A is rounded
 // on the fly, so a row gives the same products here and in the tiled kernel.
-constexpr int LV_MAXM = 8;
+constexpr int LV_MAXM = LAY_ROW_KERNEL_ROWS;
 template <bool BF16, bool DUAL>
 __global__ __launch_bounds__(256) void lgemv_kernel(LGemmArgs a) {
     const int g = blockIdx.z;

@@ -1,0 +1,199 @@
+// Products of the layer-list decoders' mixtures of experts (bfloat16 format, more rows than the streaming row kernel takes):
+// C[p] = act(A[row(p)] W_g^T) * (A[row(p)] W2_g^T) or A[row(p)] W_g^T, rows sorted by expert, one matrix (pair) per expert.
+//
+// A block makes BM x BN outputs with four waves (2 x 2) on v_mfma_f32_16x16x32_bf16.  Both operands are bfloat16 rows with K contiguous
+// and go from memory into LDS without passing registers (global_load_lds_dwordx4: 8 rows x 128 bytes per wave instruction, k-tiles of 64
+// elements = whole cache lines); the rows of A are gathered by their token there, for nothing.  The LDS image of such a load is linear in
+// the lane, so the bank swizzle sits on the source: slot p of a row holds its 16-byte chunk p ^ ((row >> 1) & 7), and fragment reads undo
+// it.  ST stages, one barrier per k-tile; two blocks share a CU, so one multiplies while the other waits.
+//
+// Which (row tile, expert) a block has follows from the group offsets in device memory: the tiles of all experts are numbered through and
+// every block finds its own with one scan over the offsets (at most 64 experts: a wave's lanes), so the grid is rows / BM + experts tiles
+// high whatever the router chose -- not experts x rows / BM, of which a 16-expert launch filled a quarter.  Tiles that share weight
+// columns have consecutive numbers on one XCD: its L2 serves them.
+//
+// Bound: LDS.  A wave's k-step of 64 x 64 outputs reads 8 KB of fragments for 16 products (256 cycles); four waves of two blocks ask for the
+// LDS ports' full 128 bytes a cycle.  64 x 64 tiles: the latency of the weights' first touch and the L2's traffic per product.
+// Measured (us per launch, gate-and-up / down; the 64 x 64 kernel without a pipeline that this replaces in brackets): 8192 rows, 16 experts of
+// 2048 x 4096: 395 / 235 (2481 / 1566), 0.70 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 22.5 / 14.2 (60 / 50).
+#include <algorithm>
+
+#include "dev_common.h"
+#include "kernels.h"
+#include "layered.h"
+#include "layered_dev.h"
+
+namespace cm {
+
+namespace {
+
+constexpr int BK = 64;
+
+__device__ __forceinline__ void lds_load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(gsrc), "s"(lds_base)
+                 : "memory");
+}
+
+template <int BM, int BN, int ST, bool DUAL>
+__global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int mtiles, int ntiles) {
+    constexpr int WM = BM / 2, WN = BN / 2, NI = WM / 16, NJ = WN / 16, APC = BM / 8, NL = (BM + BN) / 32;      // NL: loads per wave and k-tile
+    constexpr int NC = DUAL ? WN / 2 : WN;                                // output columns of a wave
+    constexpr int STAGE = (BM + BN) * BK;
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    const int per = (int)gridDim.x >> 3, bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (bid >= mtiles * ntiles) return;
+    const int nt = bid / mtiles, mt = bid - nt * mtiles;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    int g = 0, p0 = mt * BM, rows = min(BM, a.M - p0);
+    if (a.grp_off) {
+        int o0 = 0, o1 = 0;
+        if (lane < a.groups) { o0 = a.grp_off[lane]; o1 = a.grp_off[lane + 1]; }
+        const int mine = (o1 - o0 + BM - 1) / BM;
+        int incl = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(incl, d); if (lane >= d) incl += v; }
+        const unsigned long long reach = __ballot(mt < incl);
+        if (reach == 0) return;                                           // behind the last expert's last tile
+        g = __builtin_ctzll(reach);
+        p0 = __builtin_amdgcn_readlane(o0, g) + (mt - __builtin_amdgcn_readlane(incl - mine, g)) * BM;
+        rows = min(BM, __builtin_amdgcn_readlane(o1, g) - p0);
+    }
+    const uint16_t* W = a.W + (size_t)g * a.w_stride;
+    const uint16_t* W2 = DUAL ? a.W2 + (size_t)g * a.w_stride : nullptr;
+    const int n0 = nt * (DUAL ? BN / 2 : BN);
+
+    // this lane's share of the loads: piece wave + 4 i covers 8 rows of A (pieces below APC) or of the weight tile.  Rows past the end repeat
+    // the last one; their outputs are not stored.  DUAL: a wave's columns of the weight tile are NC rows of W, then the same NC of W2
+    const int prow = lane >> 3, pslot = lane & 7;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;                       // LDS offset of the dynamic segment (low half of the flat address)
+    const uint16_t* src[NL];
+    uint32_t dst[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int p = wave + 4 * i;
+        const bool isA = p < APC;
+        const int row = (isA ? p : p - APC) * 8 + prow;
+        const int kc = (pslot ^ ((row >> 1) & 7)) << 3;
+        if (isA) {
+            const int r = p0 + min(row, rows - 1);
+            src[i] = a.A + (size_t)(a.a_idx ? a.a_idx[r] / a.a_div : r) * a.lda + kc;
+        } else {
+            const int c = row / WN, q = row - c * WN;
+            const bool second = DUAL && q >= NC;
+            const int n = min(n0 + c * NC + (second ? q - NC : q), a.N - 1);
+            src[i] = (second ? W2 : W) + (size_t)n * a.K + kc;
+        }
+        dst[i] = lds0 + (uint32_t)((isA ? p * 8 : BM + (p - APC) * 8) * BK) * 2u;
+    }
+    const int nk = a.K / BK;
+    auto request = [&](int t) __attribute__((always_inline)) {            // past the end: the last tile again, into a stage nobody reads
+        const int tc = min(t, nk - 1);
+        const uint32_t at = (uint32_t)((t % ST) * STAGE) * 2u;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) lds_load16(src[i] + (size_t)tc * BK, dst[i] + at);
+    };
+    f32x4 acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, lg = lane >> 4, sw = (fr >> 1) & 7;
+#pragma unroll
+    for (int t = 0; t < ST - 1; ++t) request(t);
+    for (int t = 0; t < nk; ++t) {
+        // this wave's share of tile t has landed and its reads of tile t - 1 are done; behind the barrier that holds for every wave
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * NL) : "memory");
+        request(t + ST - 1);
+        const uint16_t* As = lds + (t % ST) * STAGE + wm * WM * BK;
+        const uint16_t* Bs = lds + (t % ST) * STAGE + (BM + wn * WN) * BK;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int fk = ((s * 4 + lg) ^ sw) << 3;
+            bf16x8 af[NI], bf[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) bf[j] = *(const bf16x8*)&Bs[(j * 16 + fr) * BK + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) af[i] = *(const bf16x8*)&As[(i * 16 + fr) * BK + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail: none may land after the block is gone
+    // D of a product: column = lane % 16, rows 4 (lane / 16) + r
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = wm * WM + i * 16 + lg * 4 + r;
+            if (m >= rows) continue;
+            const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
+#pragma unroll
+            for (int j = 0; j < NC / 16; ++j) {
+                const int n = n0 + wn * NC + j * 16 + fr;
+                if (n >= a.N) continue;
+                const float v = acc[i][j][r];
+                if (DUAL) {
+                    const float u = acc[i][j + NJ / 2][r];
+                    ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(a.act == LACT_CAPGLU ? lay_capglu(v, u, a.act_param) : lay_act(v, a.act) * u);
+                } else ((float*)a.C)[row * a.ldc + n] = v;
+            }
+        }
+}
+
+// row tiles of a launch; grouped: every expert ends in at most one ragged tile, and none has more than M rows
+template <int BM>
+int mtiles(const LTileArgs& a) {
+    return a.grp_off ? std::min((a.total + BM - 1) / BM + a.groups, a.groups * ((a.M + BM - 1) / BM)) : (a.M + BM - 1) / BM;
+}
+
+template <int BM, int BN, int ST, bool DUAL>
+void go(const LTileArgs& a, hipStream_t s) {
+    constexpr size_t lds = (size_t)ST * (BM + BN) * BK * sizeof(uint16_t);
+    static DevOnce attr;
+    attr.run([&] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tile_gemm_kernel<BM, BN, ST, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    });
+    const int cols = DUAL ? BN / 2 : BN, mt = mtiles<BM>(a), nt = (a.N + cols - 1) / cols;
+    hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL>), dim3((unsigned)((mt * nt + 7) / 8 * 8)), dim3(256), lds, s, a, mt, nt);
+}
+
+}  // namespace
+
+bool lay_tile_gemm_fits(int N, int K, int groups) { return N > 0 && K >= 2 * BK && K % BK == 0 && groups <= 64; }
+
+void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s) {
+    if (a.M <= 0 || a.N <= 0) return;
+    // 128 x 128 tiles where they still give the chip 320 blocks and a group fills half a tile of rows; measured (us, gate-and-up, 128 / 64
+    // tiles): 16 experts of 2048 x 4096 -- 2048 tokens 395 / 685, 300 tokens (75 rows, 832 blocks) 156 / 168, 128 tokens (32 rows) 151 / 142;
+    // 14 of 768 x 1024 -- 2048 tokens 63 / 75, 700 tokens (432 blocks) 35 / 34; one matrix pair 2048 x 4096 -- 1200 rows (320 blocks) 66 / 79,
+    // 600 rows (160) 64 / 46
+    const int total = a.grp_off ? a.total : a.M, groups = a.grp_off ? a.groups : 1;
+    const int blocks = mtiles<128>(a) * ((a.N + (a.W2 ? 63 : 127)) / (a.W2 ? 64 : 128));
+    const bool wide = blocks >= LAY_TILE_WIDE_BLOCKS && total >= 64 * groups;
+    if (a.W2) { if (wide) go<128, 128, 2, true>(a, s); else go<64, 64, 3, true>(a, s); }
+    else { if (wide) go<128, 128, 2, false>(a, s); else go<64, 64, 3, false>(a, s); }
+}
+
+// rows of f32, gathered and scaled -> bfloat16: out[p] = x[idx[p] / div] * scale[idx[p]]
+__global__ __launch_bounds__(256) void lay_round_scaled_kernel(const float* __restrict__ x, int ldx, const int32_t* __restrict__ idx, int div,
+                                                               const float* __restrict__ scale, uint16_t* __restrict__ out, int K) {
+    const int p = blockIdx.x, at = idx[p];
+    const float* xr = x + (size_t)(at / div) * ldx;
+    const float sc = scale[at];
+    for (int k = threadIdx.x * 2; k < K; k += 512) {                      // K is even (a multiple of the k-tile)
+        *(uint32_t*)(out + (size_t)p * K + k) = pack_bf16x2(xr[k] * sc, xr[k + 1] * sc);
+    }
+}
+void launch_lay_round_scaled(const float* x, int ldx, const int32_t* idx, int div, const float* scale, uint16_t* out, int P, int K, hipStream_t s) {
+    if (P <= 0) return;
+    hipLaunchKernelGGL(lay_round_scaled_kernel, dim3((unsigned)P), dim3(256), 0, s, x, ldx, idx, div, scale, out, K);
+}
+
+}  // namespace cm

@@ -68,6 +68,7 @@ struct Layered {
     bool attn_mfma = true;             // bfloat16 format, prompt passes: the matrix-core attention (cm_debug_set("lay_attn_mfma", 0): never)
     bool fused_prep = true;            // query / key norm + rotation + cache append in one launch (cm_debug_set("lay_fused_prep", 0): single operations)
     uint16_t* Abf = nullptr;           // [cap rounded up to 256][widest K] bf16 A operand
+    uint16_t* Asc = nullptr;           // [cap][top][W] bf16 rows times their expert's weight (scale_input)
     float *G1 = nullptr, *G2 = nullptr;   // [cap][widest dense ff] the two products of a gated feed-forward
     float* U = nullptr;                // lightning attention, chunk-parallel form: [chunks of a pass][widest H d e] f32
     size_t u_stride = 0;
@@ -120,6 +121,56 @@ static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipSt
         return;
     }
     launch_lgemm(g, bf, groups, s);
+}
+
+// the experts of a pass over `T` rows of h (choices sorted by expert in L.srt / L.off, weights in L.wsel): their outputs, and those of the expert
+// that every token uses, into L.YS [token][slots][W].  bfloat16 format, more rows than the row kernel takes, sizes of whole k-tiles: the rows are
+// rounded once and everything runs on the tile kernel, the inner rows bfloat16 as the second product reads them
+static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const LayeredLayerW& w, const float* h, int T, int W, int slots, hipStream_t s) {
+    LGemmArgs gu;
+    gu.A = h; gu.lda = W; gu.a_idx = L.srt; gu.a_div = slots; gu.a_scale = sp.scale_input ? L.wsel : nullptr;
+    gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
+    gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W; gu.grp_off = L.off; gu.act = sp.expert_act; gu.act_param = sp.limit;
+    LGemmArgs dn;
+    dn.A = L.HH; dn.lda = sp.ff; dn.W = w.down; dn.w_stride = (size_t)W * sp.ff;
+    dn.C = L.YS; dn.ldc = W; dn.c_idx = L.srt; dn.M = T; dn.N = W; dn.K = sp.ff; dn.grp_off = L.off;
+    LGemmArgs su, sdn;
+    const bool every = sp.shared_ff > 0 && slots > sp.top;
+    if (every) {                           // row `top` of the token's rows
+        su.A = h; su.lda = W; su.W = w.sh_gate; su.W2 = w.sh_up; su.C = L.HS; su.ldc = sp.shared_ff; su.M = T; su.N = sp.shared_ff;
+        su.K = W; su.act = sp.expert_act; su.act_param = sp.shared_limit;
+        sdn.A = L.HS; sdn.lda = sp.shared_ff; sdn.W = w.sh_down; sdn.C = L.YS + (size_t)sp.top * W; sdn.ldc = slots * W; sdn.M = T;
+        sdn.N = W; sdn.K = sp.shared_ff;
+    }
+    const bool tiles = !L.f32 && L.shared_gemm && L.Abf && T > LAY_ROW_KERNEL_ROWS && (!sp.scale_input || L.Asc);
+    auto tile = [&](const LGemmArgs& g, const uint16_t* A, bool gather) {
+        LTileArgs t;
+        t.A = A; t.lda = g.K; t.W = g.W; t.W2 = g.W2; t.w_stride = g.w_stride; t.C = g.C; t.ldc = g.ldc; t.c_idx = g.c_idx;
+        t.M = g.M; t.N = g.N; t.K = g.K; t.act = g.act; t.act_param = g.act_param;
+        if (gather) { t.a_idx = g.a_idx; t.a_div = g.a_div; }
+        if (g.grp_off) { t.grp_off = g.grp_off; t.groups = sp.experts; t.total = T * sp.top; }
+        launch_lay_tile_gemm(t, s);
+    };
+    const bool routed = tiles && lay_tile_gemm_fits(sp.ff, W, sp.experts) && lay_tile_gemm_fits(W, sp.ff, sp.experts);
+    const bool shared = tiles && every && lay_tile_gemm_fits(sp.shared_ff, W, 1) && lay_tile_gemm_fits(W, sp.shared_ff, 1);
+    if ((routed && !sp.scale_input) || shared) launch_lay_round_rows(h, W, L.Abf, T, W, s);
+    if (routed) {
+        if (sp.scale_input) launch_lay_round_scaled(h, W, L.srt, slots, L.wsel, L.Asc, T * sp.top, W, s);
+        tile(gu, sp.scale_input ? L.Asc : L.Abf, !sp.scale_input);
+        tile(dn, (const uint16_t*)L.HH, false);
+    }
+    if (shared) {
+        tile(su, L.Abf, false);
+        tile(sdn, (const uint16_t*)L.HS, false);
+    }
+    if (!routed) {
+        lay_gemm(m, L, gu, sp.experts, s);
+        lay_gemm(m, L, dn, sp.experts, s);
+    }
+    if (!shared && every) {
+        lay_gemm(m, L, su, 1, s);
+        lay_gemm(m, L, sdn, 1, s);
+    }
 }
 
 static void need(bool ok, const char* what) { if (!ok) throw CmError(CM_ERR_INVALID, std::string("config.json: ") + what); }
@@ -1414,6 +1465,9 @@ void Model::alloc_runtime_layered() {
         const size_t rows = (cap + 255) / 256 * 256;
         L.Abf = dalloc<uint16_t>(rows * (size_t)max_k);
         CM_HIP(hipMemsetAsync(L.Abf, 0, rows * (size_t)max_k * sizeof(uint16_t), stream));
+        int scaled_top = 0;
+        for (const LayerSpec& sp : L.spec) if (sp.mlp == LMLP_MOE && sp.scale_input) scaled_top = std::max(scaled_top, sp.top);
+        if (scaled_top) L.Asc = dalloc<uint16_t>(cap * (size_t)scaled_top * W);
         if (dense_ff) { L.G1 = dalloc<float>(cap * (size_t)dense_ff); L.G2 = dalloc<float>(cap * (size_t)dense_ff); }
         ensure_gemm_workspace();
     }
@@ -1990,25 +2044,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
                     launch_lay_router(L.Hc, w.router, L.sel, L.wsel, T, W, sp.experts, sp.top, s, &sp.router, nullptr, slots, L.Z);
                     launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, sp.experts, s, sp.top, slots);
-                    LGemmArgs gu;
-                    gu.A = L.Hc; gu.lda = W; gu.a_idx = L.srt; gu.a_div = slots; gu.a_scale = sp.scale_input ? L.wsel : nullptr;
-                    gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
-                    gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W; gu.grp_off = L.off; gu.act = sp.expert_act; gu.act_param = sp.limit;
-                    lay_gemm(*this, L, gu, sp.experts, s);
-                    LGemmArgs dn;
-                    dn.A = L.HH; dn.lda = sp.ff; dn.W = w.down; dn.w_stride = (size_t)W * sp.ff;
-                    dn.C = L.YS; dn.ldc = W; dn.c_idx = L.srt; dn.M = T; dn.N = W; dn.K = sp.ff; dn.grp_off = L.off;
-                    lay_gemm(*this, L, dn, sp.experts, s);
-                    if (sp.shared_ff > 0) {        // the expert every token uses: row `top` of the token's rows
-                        LGemmArgs su;
-                        su.A = L.Hc; su.lda = W; su.W = w.sh_gate; su.W2 = w.sh_up; su.C = L.HS; su.ldc = sp.shared_ff; su.M = T; su.N = sp.shared_ff;
-                        su.K = W; su.act = sp.expert_act; su.act_param = sp.shared_limit;
-                        lay_gemm(*this, L, su, 1, s);
-                        LGemmArgs sdn;
-                        sdn.A = L.HS; sdn.lda = sp.shared_ff; sdn.W = w.sh_down; sdn.C = L.YS + (size_t)sp.top * W; sdn.ldc = slots * W; sdn.M = T;
-                        sdn.N = W; sdn.K = sp.shared_ff;
-                        lay_gemm(*this, L, sdn, 1, s);
-                    }
+                    lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s);
                     padd.y = L.YS; padd.nsum = slots; padd.wsel = sp.scale_input ? nullptr : L.wsel;
                 }
                 if (L.capture || li + 1 == L.spec.size()) add_norm(nullptr, nullptr, 0.f, nullptr);
@@ -2078,25 +2114,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     const int outs = sp.experts + sp.router.identity, slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
                     launch_lay_router(L.X, w.router, L.sel, L.wsel, T, W, outs, sp.top, s, &sp.router, w.correction, slots, L.Z);
                     launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, outs, s, sp.top, slots);
-                    LGemmArgs gu;
-                    gu.A = L.X; gu.lda = W; gu.a_idx = L.srt; gu.a_div = slots;
-                    gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
-                    gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W; gu.grp_off = L.off; gu.act = LACT_SILU;
-                    lay_gemm(*this, L, gu, sp.experts, s);
-                    LGemmArgs dn;
-                    dn.A = L.HH; dn.lda = sp.ff; dn.W = w.down; dn.w_stride = (size_t)W * sp.ff;
-                    dn.C = L.YS; dn.ldc = W; dn.c_idx = L.srt; dn.M = T; dn.N = W; dn.K = sp.ff; dn.grp_off = L.off;
-                    lay_gemm(*this, L, dn, sp.experts, s);
-                    if (sp.shared_ff > 0) {        // the expert every token uses: row `top` of the token's rows, weight 1
-                        LGemmArgs su;
-                        su.A = L.X; su.lda = W; su.W = w.sh_gate; su.W2 = w.sh_up; su.C = L.HS; su.ldc = sp.shared_ff; su.M = T; su.N = sp.shared_ff;
-                        su.K = W; su.act = LACT_SILU;
-                        lay_gemm(*this, L, su, 1, s);
-                        LGemmArgs sdn;
-                        sdn.A = L.HS; sdn.lda = sp.shared_ff; sdn.W = w.sh_down; sdn.C = L.YS + (size_t)sp.top * W; sdn.ldc = slots * W; sdn.M = T;
-                        sdn.N = W; sdn.K = sp.shared_ff;
-                        lay_gemm(*this, L, sdn, 1, s);
-                    }
+                    lay_experts(*this, L, sp, w, L.X, T, W, slots, s);
                     post_norm(L.YS, w.norm2b, L.wsel, slots);
                     if (sp.router.identity > 0) { pend.sel_top = sp.top; pend.n_real = sp.experts; }      // identity rows are taken in the combine
                 }
@@ -2137,15 +2155,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 } else {
                     launch_lay_router(L.Hc, w.router, L.sel, L.wsel, T, W, sp.experts, sp.top, s, nullptr, nullptr, 0, L.Z);
                     launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, sp.experts, s);
-                    LGemmArgs gu;
-                    gu.A = L.Hc; gu.lda = W; gu.a_idx = L.srt; gu.a_div = sp.top;
-                    gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
-                    gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W; gu.grp_off = L.off; gu.act = LACT_SILU;
-                    lay_gemm(*this, L, gu, sp.experts, s);
-                    LGemmArgs dn;
-                    dn.A = L.HH; dn.lda = sp.ff; dn.W = w.down; dn.w_stride = (size_t)W * sp.ff;
-                    dn.C = L.YS; dn.ldc = W; dn.c_idx = L.srt; dn.M = T; dn.N = W; dn.K = sp.ff; dn.grp_off = L.off;
-                    lay_gemm(*this, L, dn, sp.experts, s);
+                    lay_experts(*this, L, sp, w, L.Hc, T, W, sp.top, s);
                     post_norm(L.YS, w.norm2b, L.wsel, sp.top);
                 }
             }

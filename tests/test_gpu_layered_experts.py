@@ -1,0 +1,69 @@
+"""GPU: the tile kernel of the experts' products (kernels_layered_gemm.hip) against the plain kernels on the same rounded operands, at the
+edges of its tiles.
+
+One layer, bfloat16 format, the same step with the tile kernels on and off.  Both round the experts' inputs and inner rows to bfloat16 and
+add up the exact products in f32, in another order: a sum of K = 128 .. 320 terms moves by about 1e-6 of itself, an inner row's element lands
+on the other side of a rounding boundary with probability 1e-6 / 2^-8 and is then 2^-8 off -- 3e-5 in the mean square, and the same once more
+in the head's input.  1e-3 of the largest logit is over ten times that; the router reads the same rows on both sides, so the choices agree."""
+import numpy as np
+import pytest
+
+from tests import gibipel_util as GI
+from tests import gizezen_util as GZ
+from tests import korupel_util as KO
+from tests import nevotar_util as NE
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-3
+
+
+def _check(tmp_path, U, cfg, n, seed):
+    from crane_amd.backend import Model
+    m = Model.from_pretrained(U.write_checkpoint(str(tmp_path / "ckpt"), cfg, U.random_weights(cfg, seed)), compute_dtype="bfloat16", max_seqs=4,
+                              max_seq_len=2560, prefill_chunk=2560)
+    toks = U.tokens(n, cfg["vocab"], seed + 1)
+    want = [i for i in range(n) if i % 8 == 0 or i >= n - 66]
+    got = []
+    try:
+        for on in (1, 0):
+            m.debug_set("lay_shared_gemm", on)
+            s = m.seq_alloc()
+            got.append(m.step_batch([(s, toks, want)])[0].astype(np.float64))
+            m.seq_free(s)
+    finally:
+        m.close()
+    assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() < TOL * np.abs(got[1]).max()
+
+
+# one row more than the row kernel takes, groups of no or one row, ragged last tiles, output columns that end inside a tile, inner sizes of
+# the smallest and of odd numbers of k-tiles, the most groups the kernel numbers and one more (which the plain kernel keeps)
+@pytest.mark.parametrize("n", [9, 65, 200])
+@pytest.mark.parametrize("width,ff,shared,experts,top", [(128, 128, 128, 6, 2), (192, 320, 192, 4, 4), (320, 192, 0, 64, 3), (128, 192, 320, 65, 2)])
+def test_softmax_routed_experts_and_a_shared_one(tmp_path, n, width, ff, shared, experts, top):
+    cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=experts, top=top, ff=ff, shared=shared))], vocab=96, width=width)
+    _check(tmp_path, GZ, cfg, n, 3)
+
+
+# 128 x 128 tiles: enough rows and columns for 320 of them
+def test_wide_tiles(tmp_path):
+    cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=8, top=4, ff=576, shared=192))], vocab=96, width=1216)
+    _check(tmp_path, GZ, cfg, 2500, 5)
+
+
+def test_weights_on_the_experts_inputs_and_the_capped_product(tmp_path):
+    cfg = NE.config([NE.layer("attention", NE.attn(), NE.moe(experts=6, top=3, ff=192, shared=128))], vocab=96, width=192)
+    for n in (9, 150):
+        _check(tmp_path, NE, cfg, n, 7)
+
+
+def test_identity_experts(tmp_path):
+    cfg = GI.config([GI.layer(GI.left(), GI.right(), GI.moe(experts=5, top=2, ff=128, identity=3, groups=2, keep=1, shared=192))], vocab=96, width=128)
+    for n in (9, 150):
+        _check(tmp_path, GI, cfg, n, 9)
+
+
+def test_sigmoid_routed_experts_without_a_shared_one(tmp_path):
+    cfg = KO.config([KO.layer("attention", KO.moe(experts=5, top=2, ff=192), **KO.attn())], vocab=96, width=192)
+    for n in (33, 150):
+        _check(tmp_path, KO, cfg, n, 11)
