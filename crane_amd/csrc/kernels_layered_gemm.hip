@@ -126,25 +126,30 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int 
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail: none may land after the block is gone
-    // D of a product: column = lane % 16, rows 4 (lane / 16) + r
+    // D of a product: column = lane % 16, rows 4 (lane / 16) + r.  f: the outputs' function, chosen once per block
+    auto store = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = wm * WM + i * 16 + lg * 4 + r;
-            if (m >= rows) continue;
-            const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
+            for (int r = 0; r < 4; ++r) {
+                const int m = wm * WM + i * 16 + lg * 4 + r;
+                if (m >= rows) continue;
+                const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
 #pragma unroll
-            for (int j = 0; j < NC / 16; ++j) {
-                const int n = n0 + wn * NC + j * 16 + fr;
-                if (n >= a.N) continue;
-                const float v = acc[i][j][r];
-                if (DUAL) {
-                    const float u = acc[i][j + NJ / 2][r];
-                    ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(a.act == LACT_CAPGLU ? lay_capglu(v, u, a.act_param) : lay_act(v, a.act) * u);
-                } else ((float*)a.C)[row * a.ldc + n] = v;
+                for (int j = 0; j < NC / 16; ++j) {
+                    const int n = n0 + wn * NC + j * 16 + fr;
+                    if (n >= a.N) continue;
+                    if (DUAL) ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(f(acc[i][j][r], acc[i][j + (DUAL ? NJ / 2 : 0)][r], n));
+                    else ((float*)a.C)[row * a.ldc + n] = f(acc[i][j][r], 0.f, n);
+                }
             }
-        }
+    };
+    if (DUAL) {
+        if (a.act == LACT_SILU) store([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
+        else if (a.act == LACT_CAPGLU) store([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
+        else store([&](float v, float u, int) { return lay_act(v, a.act) * u; });
+    } else if (!a.bias && a.act == LACT_NONE && a.act2 == LACT_NONE) store([](float v, float, int) { return v; });
+    else store([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
 }
 
 // row tiles of a launch; grouped: every expert ends in at most one ragged tile, and none has more than M rows

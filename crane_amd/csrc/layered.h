@@ -208,7 +208,7 @@ constexpr int LAY_ROW_KERNEL_ROWS = 8;
 void launch_lgemm(const LGemmArgs& a, bool bf16, int groups, hipStream_t s);
 
 // products over bfloat16 rows on matrix-core tiles (kernels_layered_gemm.hip).  W2 given: C (bfloat16) = act(A W^T) * (A W2^T); else C (f32) =
-// A W^T.  grp_off: rows [grp_off[g], grp_off[g + 1]) use matrix g; `total` rows in all groups, at most M in one.  A row of output row p:
+// A W^T + bias, columns below act_split through act, the others through act2.  grp_off: rows [grp_off[g], grp_off[g + 1]) use matrix g; `total` rows in all groups, at most M in one.  A row of output row p:
 // a_idx ? a_idx[p] / a_div : p; output row: c_idx ? c_idx[p] : p.  K a multiple of 64, at most 64 groups; A, W, W2 and their rows 16-byte aligned
 struct LTileArgs {
     const uint16_t* A = nullptr; int lda = 0;
@@ -218,7 +218,8 @@ struct LTileArgs {
     const int32_t* c_idx = nullptr;
     int M = 0, N = 0, K = 0;
     const int32_t* grp_off = nullptr; int groups = 1, total = 0;
-    int act = LACT_NONE; float act_param = 1.f;
+    const float* bias = nullptr;
+    int act = LACT_NONE, act2 = LACT_NONE, act_split = 0; float act_param = 1.f;
 };
 constexpr int LAY_TILE_WIDE_BLOCKS = 320;       // 128 x 128 tiles from this many blocks on (launch_lay_tile_gemm)
 bool lay_tile_gemm_fits(int N, int K, int groups);

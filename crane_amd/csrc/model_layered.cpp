@@ -93,6 +93,19 @@ void LayeredDeleter::operator()(Layered* p) const { delete p; }
 // one projection of a pass: the shared matrix-core GEMM where it applies, else the kernels of kernels_layered.hip
 static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipStream_t s) {
     const bool bf = !L.f32;
+    // the tile kernel with bias and activation in its epilogue, instead of (split sums, their reduction,) a product and an activation sweep.  Below
+    // 32 rows the alternative is the plain kernel (24 rows, four layers: 840 -> 632 us at width 1024, 2747 -> 1890 at 4096); from there on the
+    // shared GEMM, whose split sums win while the tiles are few for the depth: 64 rows 644 against 663 us (26 and 16 tiles, K 1024) and 1884
+    // against 1955 (98 and 64 tiles, K 4096), but 128 rows 704 / 689 (52 and 32) and 2016 / 2022 (196 and 128), 700 rows 921 / 878, 2947 / 2916
+    if (bf && L.shared_gemm && L.Abf && groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && !g.W2 && g.M > LAY_ROW_KERNEL_ROWS &&
+        lay_tile_gemm_fits(g.N, g.K, 1) && (g.M < 32 || (size_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * 32 >= (size_t)g.K)) {
+        launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
+        LTileArgs t;
+        t.A = L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.N; t.K = g.K; t.bias = g.bias;
+        t.act = g.act; t.act2 = g.act2; t.act_split = g.act_split; t.act_param = g.act_param;
+        launch_lay_tile_gemm(t, s);
+        return;
+    }
     if (bf && L.shared_gemm && L.Abf && groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && g.M >= 32 && g.N % 128 == 0 && g.K % 32 == 0 &&
         (!g.W2 || (g.ldc == g.N && L.G1 && L.G2))) {
         launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
