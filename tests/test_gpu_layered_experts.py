@@ -8,6 +8,7 @@ in the head's input.  1e-3 of the largest logit is over ten times that; the rout
 import numpy as np
 import pytest
 
+from oracle import gizezen_oracle as O
 from tests import gibipel_util as GI
 from tests import gizezen_util as GZ
 from tests import korupel_util as KO
@@ -67,3 +68,24 @@ def test_sigmoid_routed_experts_without_a_shared_one(tmp_path):
     cfg = KO.config([KO.layer("attention", KO.moe(experts=5, top=2, ff=192), **KO.attn())], vocab=96, width=192)
     for n in (33, 150):
         _check(tmp_path, KO, cfg, n, 11)
+
+
+# the router's row kernel against the oracle in the float32 format: logits below, at and above its register sizes (16, 20, 32; more stay on the
+# block-per-token form), one and two tokens per wave, a last wave with one of two
+@pytest.mark.parametrize("experts,shared", [(16, 0), (16, 28), (20, 28), (32, 0), (32, 28)])
+@pytest.mark.parametrize("n", [9, 1025])
+def test_router_rows(tmp_path, experts, shared, n):
+    from crane_amd.backend import Model
+    cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=experts, top=3, ff=24, shared=shared))], vocab=61, width=72)
+    P = GZ.random_weights(cfg, 13)
+    toks = GZ.tokens(n, cfg["vocab"], 14)
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="float32", max_seqs=2, max_seq_len=1088)
+    try:
+        got = m.step_batch([(m.seq_alloc(), toks, list(range(n)))])[0].astype(np.float64)
+    finally:
+        m.close()
+    want = O.forward(cfg, P, toks)
+    # float32 sums against float64: 1e-4 of the largest logit, as in the family's own tests; a choice within 1e-6 of a tie may fall the other way
+    # for one position in a thousand
+    off = np.abs(got - want).max(-1) / np.abs(want).max()
+    assert np.quantile(off, 0.998) < 1e-4, (float(off.max()), int(off.argmax()))
