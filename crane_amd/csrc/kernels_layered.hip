@@ -1494,10 +1494,15 @@ void launch_lay_attn(const LAttnArgs& a0, int kvt, hipStream_t s) {
         else if (narrow) lay_attn_go<KV_BF16, 32, 16>(a, grid, lds, s);
         else lay_attn_go<KV_BF16, 64, 16>(a, grid, lds, s);
     }
-    // the merge: one thread per output element, blocks of 256 over a tile's 16 rows
-    if (nsplit > 1)
-        hipLaunchKernelGGL(lay_attn_merge_kernel, dim3((unsigned)a.ntiles, (unsigned)a.G, (unsigned)std::max(1, std::min(16, LA_BQ * a.e / 1024))),
-                           dim3(256), 0, s, a, nsplit);
+    if (nsplit > 1) launch_lay_attn_merge(a, nsplit, s);
+}
+// the merge: one thread per output element, blocks of 256 over a tile's 16 rows
+void launch_lay_attn_merge(const LAttnArgs& a0, int nsplit, hipStream_t s) {
+    LAttnArgs a = a0;
+    if (!a.gbuf) { a.gbuf = a.proj + a.g_off; a.ldg = a.ldp; }
+    if (a.e <= 0) a.e = a.d;
+    hipLaunchKernelGGL(lay_attn_merge_kernel, dim3((unsigned)a.ntiles, (unsigned)a.G, (unsigned)std::max(1, std::min(16, LA_BQ * a.e / 1024))),
+                       dim3(256), 0, s, a, nsplit);
 }
 int lay_attn_key_tile(int d, int e, bool own_v) { return (d > 128 || lay_attn_lds(d, e, own_v, 64) > LDS_PLAIN) ? 32 : 64; }
 

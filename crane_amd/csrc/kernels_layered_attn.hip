@@ -13,7 +13,7 @@
 //     register), and only tiles on the edge of somebody's mask are masked.
 //   * rows are staged once per block, two LDS buffers, requested two tiles ahead, one barrier per tile.
 // Measured (us per launch): 2048 tokens, 32 query heads of 128 on 8 key heads, causal: 106 (325 TFLOP/s; the form with transposed stores and
-// the weights through LDS: 1590); a mixed batch of 24 single tokens and 300 prompt rows, 8 heads on 2, window 1024: 27 (174).  Blocks of
+// the weights through LDS: 1590); a mixed batch of 24 single tokens and 300 prompt rows, 8 heads on 2, window 1024: 24 (174).  Blocks of
 // 128 rows (two query groups per wave, half the fragment reads per product): 100 at the first size, 3 % slower at 1024 tokens; not kept.
 // Rounding points are the older form's: q rounded to bfloat16 once, scores, running maximum / sum and weights f32, the weights as a
 // bfloat16 hi + lo pair (two products), exp2 and log on the hardware units.
@@ -36,144 +36,73 @@ __device__ __forceinline__ void lds_barrier() {        // LDS hand-off only: req
     asm volatile("" ::: "memory");
 }
 
-// DP / EP: key / value size the registers and LDS rows are laid out for (64 or 128; the key rows' padding is zero).  A block takes 64 query
-// rows, 16 per wave, row qi = (position in the portion) * nrep + (query head in the group).  POOL: the walk starts with the mean rows of
-// position blocks.
-template <int DP, int EP, bool POOL>
-__global__ __launch_bounds__(256, 2) void lay_attn_tile_kernel(LAttnArgs a, bool qvec, bool ovec) {
-    constexpr int KLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16;
-    constexpr int KC = DP / 8, VC = EP / 8, KPT = KT * KC / 256, VPT = KT * VC / 256;   // 16-byte chunks per row / per thread
-    extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-    uint16_t* const Ks = smem;                         // [2][64][KLD]
-    uint16_t* const Vs = smem + 2 * KT * KLD;          // [2][64][VLD]
-    const int g = blockIdx.x;
-    const int2 tile_id = a.tiles[blockIdx.y];
-    const LaySegDev sg = a.segs[tile_id.x];
-    const int nrep = a.H / a.G, d = a.d, e = a.e;
-    const int q0 = tile_id.y, nq = min(64, sg.n * nrep - q0);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lg = lane >> 4;
-    const int win = (int)min(a.win, 1ll << 30), keep = (int)min(a.keep, 1ll << 30), chunk = (int)min(a.chunk, 1ll << 30);
-    const int pool = POOL ? (int)min(a.pool, 1ll << 30) : 0;
-
-    const int qr = wave * 16 + lr;
-    const bool qok = qr < nq;
-    const int qi = q0 + (qok ? qr : 0), lp = qi / nrep, qhead = g * nrep + (qi - lp * nrep), qrow = sg.row0 + lp;
-    const int qpos = qok ? sg.start_pos + lp : -1;     // -1: sees nothing where masks are applied
-    const int qclo = chunk > 0 && qok ? qpos / chunk * chunk : 0;
-    const float r1 = a.bias != LBIAS_NONE ? a.r1[qhead] * L2E : 0.f, r2 = a.bias == LBIAS_LOG ? a.r2[qhead] : 0.f;
-    float m = -INFINITY, l = 0.f;
-    if (a.sink && qok) { m = a.sink[qhead] * L2E; l = lg == 0 ? 1.f : 0.f; }       // the four lane groups' sums meet at the end
-    bf16x8 qf[NKS];
-    const float* src = a.proj + (size_t)qrow * a.ldp + a.q_off + qhead * d;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-        const int c = ks * 32 + lg * 8;
-        u32x4 pk = {0u, 0u, 0u, 0u};
-        if (qok && c < d) {
-            float x[8];
-            if (qvec) {
-                const f32x4 x0 = *(const f32x4*)(src + c), x1 = *(const f32x4*)(src + c + 4);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) { x[i] = x0[i]; x[4 + i] = x1[i]; }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = src[c + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) pk[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
-        }
-        qf[ks] = __builtin_bit_cast(bf16x8, pk);
+// The key walk of query rows [q0, q0 + nq) of a portion: `front` tiles of block rows (POOL) or of the kept first tokens that lie in front of the
+// window's first tile, then the window from a multiple of 64 on.
+struct Walk {
+    int pmin, pmax, main0, front, ntile, blocks, vis_lo;      // everybody sees [vis_lo, pmin]
+    int win, keep, chunk, pool;
+    template <bool POOL>
+    __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int q0, int nq, int nrep) {
+        win = (int)min(a.win, 1ll << 30); keep = (int)min(a.keep, 1ll << 30); chunk = (int)min(a.chunk, 1ll << 30);
+        pool = POOL ? (int)min(a.pool, 1ll << 30) : 0;
+        pmin = sg.start_pos + q0 / nrep; pmax = sg.start_pos + (q0 + nq - 1) / nrep;
+        int main_lo = max(0, pmin - win + 1);
+        if (chunk > 0) main_lo = max(main_lo, pmin / chunk * chunk);
+        main0 = main_lo / KT * KT;
+        blocks = POOL ? max(0, (pmax - win + 1) / pool) : 0;
+        front = POOL ? (blocks + KT - 1) / KT : min((keep + KT - 1) / KT, main0 / KT);
+        ntile = front + (pmax - main0) / KT + 1;
+        vis_lo = max(pmax - win + 1, chunk > 0 ? pmax / chunk * chunk : 0);
     }
-    // the key walk: `front` tiles of block rows (POOL) or of the kept first tokens that lie in front of the window's first tile, then the
-    // window from a multiple of 64 on
-    const int pmin = sg.start_pos + q0 / nrep, pmax = sg.start_pos + (q0 + nq - 1) / nrep;
-    int main_lo = max(0, pmin - win + 1);
-    if (chunk > 0) main_lo = max(main_lo, pmin / chunk * chunk);
-    const int main0 = main_lo / KT * KT;
-    const int blocks = POOL ? max(0, (pmax - win + 1) / pool) : 0;
-    const int front = POOL ? (blocks + KT - 1) / KT : min((keep + KT - 1) / KT, main0 / KT);
-    const int ntile = front + (pmax - main0) / KT + 1;
-    const int vis_lo = max(pmax - win + 1, chunk > 0 ? pmax / chunk * chunk : 0);      // everybody sees [vis_lo, pmin]
-    auto first_of = [&](int t) __attribute__((always_inline)) { return t < front ? t * KT : main0 + (t - front) * KT; };
+    __device__ __forceinline__ int first(int t) const { return t < front ? t * KT : main0 + (t - front) * KT; }
+};
+// cached row of block b's mean (keys' row index; the values' follows the same count)
+__device__ __forceinline__ size_t block_row(const LAttnArgs& a, const LaySegDev& sg, int g, int b, int pool) {
+    const int lpg = (b * pool + pool - 1) / a.page;
+    return ((size_t)a.bt[sg.bt_off + lpg] * a.G + g) * a.pool_rows + (b - (int)(((long long)lpg * a.page) / pool));
+}
 
-    // page of every position tile; lane i holds that of tile 64 grp + i
-    int pgs_grp = 0;
-    auto load_pages = [&](int grp) __attribute__((always_inline)) {
-        const int j = min(first_of(min(grp * 64 + lane, ntile - 1)), pmax);
-        return a.bt[sg.bt_off + j / a.page];
-    };
-    int pgs = load_pages(0);
-    struct Rows { u32x4 k[KPT], v[VPT]; };
-    const int Gv = a.v_div > 1 ? a.G / a.v_div : a.G, gv = a.v_div > 1 ? g / a.v_div : g;
-    auto fetch = [&](int t_, Rows& rg) __attribute__((always_inline)) {
-        const int t = min(t_, ntile - 1);              // past the end: the last tile again, parked into a buffer nobody reads
-        const int j0 = first_of(t);
-        if ((t >> 6) != pgs_grp) { pgs_grp = t >> 6; pgs = load_pages(pgs_grp); }      // (uniform)
-        if (POOL && t < front) {
+// elements c .. c + 7 of a query row in f32 (zero outside)
+__device__ __forceinline__ void query8(const float* src, int c, int d, bool ok, bool qvec, float (&x)[8]) {
 #pragma unroll
-            for (int i = 0; i < KPT; ++i) {
-                const int idx = tid + 256 * i, b = min(j0 + idx / KC, blocks - 1), c = (idx % KC) * 8;
-                const int lpg = (b * pool + pool - 1) / a.page;
-                const size_t row = ((size_t)a.bt[sg.bt_off + lpg] * a.G + g) * a.pool_rows + (b - (int)(((long long)lpg * a.page) / pool));
-                rg.k[i] = (u32x4){0u, 0u, 0u, 0u};
-                if (c < d) rg.k[i] = ld16((const uint16_t*)a.pk_pool + row * d + c);
-            }
+    for (int i = 0; i < 8; ++i) x[i] = 0.f;
+    if (!ok || c >= d) return;
+    if (qvec) {
+        const f32x4 x0 = *(const f32x4*)(src + c), x1 = *(const f32x4*)(src + c + 4);
 #pragma unroll
-            for (int i = 0; i < VPT; ++i) {
-                const int idx = tid + 256 * i, b = min(j0 + idx / VC, blocks - 1), c = (idx % VC) * 8;
-                const int lpg = (b * pool + pool - 1) / a.page;
-                const size_t row = ((size_t)a.bt[sg.bt_off + lpg] * a.G + g) * a.pool_rows + (b - (int)(((long long)lpg * a.page) / pool));
-                rg.v[i] = (u32x4){0u, 0u, 0u, 0u};
-                if (c < e) rg.v[i] = a.pv_pool ? ld16((const uint16_t*)a.pv_pool + row * e + c) : ld16((const uint16_t*)a.pk_pool + row * d + c);
-            }
-            return;
-        }
-        const int pg = __builtin_amdgcn_readlane(pgs, t & 63), r0 = j0 % a.page, last = pmax - j0;      // rows past the newest position: that one again
-        const uint16_t* kp = (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + r0) * d;
-        const uint16_t* vp = a.vpool ? (const uint16_t*)a.vpool + (((size_t)pg * Gv + gv) * a.page + r0) * e : kp;
-        const int ldv = a.vpool ? e : d;
+        for (int i = 0; i < 4; ++i) { x[i] = x0[i]; x[4 + i] = x1[i]; }
+    } else {
 #pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            const int idx = tid + 256 * i, row = min(idx / KC, last), c = (idx % KC) * 8;
-            rg.k[i] = (u32x4){0u, 0u, 0u, 0u};
-            if (c < d) rg.k[i] = ld16(kp + (size_t)row * d + c);
-        }
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-            const int idx = tid + 256 * i, row = min(idx / VC, last), c = (idx % VC) * 8;
-            rg.v[i] = (u32x4){0u, 0u, 0u, 0u};
-            if (c < e) rg.v[i] = ld16(vp + (size_t)row * ldv + c);
-        }
-    };
-    auto park = [&](int buf, const Rows& rg) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < KPT; ++i) { const int idx = tid + 256 * i; *(u32x4*)&Ks[(buf * KT + idx / KC) * KLD + (idx % KC) * 8] = rg.k[i]; }
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) { const int idx = tid + 256 * i; *(u32x4*)&Vs[(buf * KT + idx / VC) * VLD + (idx % VC) * 8] = rg.v[i]; }
-    };
+        for (int i = 0; i < 8; ++i) x[i] = src[c + i];
+    }
+}
 
-    f32x4 o[NNT];
-#pragma unroll
-    for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const float scale = a.scale * L2E;                 // scores in units of log 2
-
-    auto tile = [&](int t, Rows& rg_new, const Rows& rg_next) __attribute__((always_inline)) {
-        fetch(t + 2, rg_new);
-        const uint16_t* Kb = Ks + (t & 1) * KT * KLD;
-        const uint16_t* Vb = Vs + (t & 1) * KT * VLD;
-        f32x4 s[4];
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-            s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const bf16x8 kf = *(const bf16x8*)&Kb[(tt * 16 + lr) * KLD + ks * 32 + lg * 8];
-                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[tt], 0, 0, 0);
-            }
-        }
-        const int j0 = first_of(t);
-        const bool blk = POOL && t < front;
-        const bool full = t >= front && j0 >= vis_lo && j0 + KT - 1 <= pmin;
+// a lane's query (column lane % 16 of the transposed scores) and its running softmax.  PARTS: bfloat16 parts of a weight
+struct Query {
+    bool ok;
+    int pos, head, row, clo;
+    float r1, r2, m, l;
+    // pos -1: sees nothing where masks are applied.  first: this wave starts the running pair from the sink
+    __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int g, int qr, int q0, int nq, int nrep, int chunk, int lg, bool first) {
+        ok = qr < nq;
+        const int qi = q0 + (ok ? qr : 0), lp = qi / nrep;
+        head = g * nrep + (qi - lp * nrep);
+        row = sg.row0 + lp;
+        pos = ok ? sg.start_pos + lp : -1;
+        clo = chunk > 0 && ok ? pos / chunk * chunk : 0;
+        r1 = a.bias != LBIAS_NONE ? a.r1[head] * L2E : 0.f;
+        r2 = a.bias == LBIAS_LOG ? a.r2[head] : 0.f;
+        m = -INFINITY; l = 0.f;
+        if (a.sink && ok && first) { m = a.sink[head] * L2E; l = lg == 0 ? 1.f : 0.f; }     // the four lane groups' sums meet at the end
+    }
+    // scores of tile t (products in s, keys 16 tt + 4 lg + r) -> weights in PARTS bfloat16 parts, the running pair moved on, o rescaled when a
+    // new maximum appears in the wave.  p[..][h]: keys 16 (2 h) + 4 lg + 0 .. 3, then 16 (2 h + 1) + 4 lg + 0 .. 3
+    template <bool POOL, int PARTS, int NNT>
+    __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int lg, f32x4 (&s)[4], bf16x8 (&p)[PARTS][2], f32x4 (&o)[NNT]) {
+        const float scale = a.scale * L2E;             // scores in units of log 2
+        const int j0 = w.first(t);
+        const bool blk = POOL && t < w.front;
+        const bool full = t >= w.front && j0 >= w.vis_lo && j0 + KT - 1 <= w.pmin;
         float mt = -INFINITY;
         if (full && a.bias == LBIAS_NONE) {
 #pragma unroll
@@ -181,23 +110,29 @@ __global__ __launch_bounds__(256, 2) void lay_attn_tile_kernel(LAttnArgs a, bool
 #pragma unroll
                 for (int r = 0; r < 4; ++r) { s[tt][r] *= scale; mt = fmaxf(mt, s[tt][r]); }
         } else {
+            // (the distance term and the kind of tile are settled outside the loops: a branch per score kept the vector units at a third)
+            auto each = [&](auto penalty, auto visible) __attribute__((always_inline)) {
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+                for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int j = j0 + tt * 16 + lg * 4 + r, dist = qpos - j;
-                    const bool vis = blk ? j < blocks && (j + 1) * pool <= qpos - win + 1
-                                         : dist >= 0 && ((dist < win && j >= qclo) || j < keep);
-                    float sc = s[tt][r] * scale;
-                    if (!blk) sc -= a.bias == LBIAS_LOG ? r1 * __logf(1.f + r2 * (float)max(dist, 0)) : r1 * (float)dist;
-                    s[tt][r] = vis ? sc : -INFINITY;
-                    mt = fmaxf(mt, s[tt][r]);
-                }
+                    for (int r = 0; r < 4; ++r) {
+                        const int j = j0 + tt * 16 + lg * 4 + r, dist = pos - j;
+                        const float sc = s[tt][r] * scale - penalty(dist);
+                        s[tt][r] = visible(j, dist) ? sc : -INFINITY;
+                        mt = fmaxf(mt, s[tt][r]);
+                    }
+            };
+            // bitwise: no short-circuit branches
+            const auto window = [&](int j, int dist) { return (bool)((dist >= 0) & (((dist < w.win) & (j >= clo)) | (j < w.keep))); };
+            if (blk) each([](int) { return 0.f; }, [&](int j, int) { return (bool)((j < w.blocks) & ((j + 1) * w.pool <= pos - w.win + 1)); });
+            else if (a.bias == LBIAS_NONE) each([](int) { return 0.f; }, window);
+            else if (a.bias == LBIAS_LOG) each([&](int dist) { return r1 * __logf(1.f + r2 * (float)max(dist, 0)); }, window);   // (absolute error 1e-7)
+            else each([&](int dist) { return r1 * (float)dist; }, window);
         }
         mt = fmaxf(mt, __shfl_xor(mt, 16));
         mt = fmaxf(mt, __shfl_xor(mt, 32));
         const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.f : mn;    // nothing seen so far: every weight is exp2(-inf) = 0
-        if (__any(mn > m)) {                           // a new maximum somewhere in the wave
+        if (__any(mn > m)) {
             const float corr = __builtin_amdgcn_exp2f(m - ms);
             l *= corr;
 #pragma unroll
@@ -206,83 +141,378 @@ __global__ __launch_bounds__(256, 2) void lay_attn_tile_kernel(LAttnArgs a, bool
                 for (int r = 0; r < 4; ++r) o[n][r] *= corr;
             m = mn;
         }
-        bf16x8 ph[2], pl[2];
         float psum = 0.f;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            u32x4 hi, lo;
+            u32x4 part[PARTS];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {              // keys 16 (2 h) + 4 lg + {0, 1}, {2, 3}, then 16 (2 h + 1) + ...
-                const float p0 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1)] - ms);
-                const float p1 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1) + 1] - ms);
+            for (int q = 0; q < 4; ++q) {
+                float p0 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1)] - ms);
+                float p1 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1) + 1] - ms);
                 psum += p0 + p1;
-                hi[q] = pack_bf16x2(p0, p1);
-                lo[q] = pack_bf16x2(p0 - bf16_lo(hi[q]), p1 - bf16_hi(hi[q]));
+#pragma unroll
+                for (int k = 0; k < PARTS; ++k) {
+                    const uint32_t pk = pack_bf16x2(p0, p1);
+                    part[k][q] = pk;
+                    p0 -= bf16_lo(pk); p1 -= bf16_hi(pk);
+                }
             }
-            ph[h] = __builtin_bit_cast(bf16x8, hi);
-            pl[h] = __builtin_bit_cast(bf16x8, lo);
+#pragma unroll
+            for (int k = 0; k < PARTS; ++k) p[k][h] = __builtin_bit_cast(bf16x8, part[k]);
         }
         l += psum;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int n = 0; n < NNT; ++n) {
-                bf16x4 v2[2];
-#pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const uint16_t* vp = &Vb[((2 * h + k) * 16 + lg * 4 + (lr >> 2)) * VLD + n * 16 + (lr & 3) * 4];
-                    v2[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)vp);
-                }
-                const bf16x8 vf = __builtin_shufflevector(v2[0], v2[1], 0, 1, 2, 3, 4, 5, 6, 7);
-                o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph[h], o[n], 0, 0, 0);
-                o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl[h], o[n], 0, 0, 0);
-            }
-        park((t + 1) & 1, rg_next);                    // that buffer was last read one tile ago, behind that tile's barrier
-        lds_barrier();
-    };
-    Rows ra, rb;
-    fetch(0, ra);
-    fetch(1, rb);
-    park(0, ra);
-    lds_barrier();
-    for (int t = 0; t < ntile; t += 2) {
-        tile(t, ra, rb);
-        if (t + 1 < ntile) tile(t + 1, rb, ra);
     }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
-    if (!qok) return;
-    const float* gp = a.gbuf + (size_t)qrow * a.ldg + (a.gate == LGATE_ELEM ? qhead * e : qhead);
-    const float inv = (a.gate == LGATE_HEAD ? gp[0] : 1.f) / l * a.out_scale;
-    float* out = a.out + (size_t)qrow * a.ldo + qhead * e;
+};
+// O^T += V^T P^T of one tile from its rows in LDS
+template <int VLD, int PARTS, int NNT>
+__device__ __forceinline__ void values(const uint16_t* Vb, int lr, int lg, const bf16x8 (&p)[PARTS][2], f32x4 (&o)[NNT]) {
 #pragma unroll
-    for (int n = 0; n < NNT; ++n) {
-        const int c = n * 16 + lg * 4;
-        if (c >= e) continue;
-        f32x4 v;
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = o[n][r] * inv * (a.gate == LGATE_ELEM ? gp[c + r] : 1.f);
-        if (ovec) *(f32x4*)(out + c) = v;
-        else {
+        for (int n = 0; n < NNT; ++n) {
+            bf16x4 v2[2];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) out[c + r] = v[r];
+            for (int k = 0; k < 2; ++k) {
+                const uint16_t* vp = &Vb[((2 * h + k) * 16 + lg * 4 + (lr >> 2)) * VLD + n * 16 + (lr & 3) * 4];
+                v2[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)vp);
+            }
+            const bf16x8 vf = __builtin_shufflevector(v2[0], v2[1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int k = 0; k < PARTS; ++k) o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p[k][h], o[n], 0, 0, 0);
         }
+}
+// four output elements c .. c + 3 of a query: v times inv times the gate
+__device__ __forceinline__ void put4(const LAttnArgs& a, int row, int head, int c, const f32x4& o, float l, bool ovec) {
+    const float* gp = a.gbuf + (size_t)row * a.ldg + (a.gate == LGATE_ELEM ? head * a.e : head);
+    const float inv = (a.gate == LGATE_HEAD ? gp[0] : 1.f) / l * a.out_scale;
+    float* out = a.out + (size_t)row * a.ldo + head * a.e + c;
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = o[r] * inv * (a.gate == LGATE_ELEM ? gp[c + r] : 1.f);
+    if (ovec) *(f32x4*)out = v;
+    else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[r] = v[r];
     }
 }
 
-template <int DP, int EP, bool POOL>
+// ---- prompt passes.  DP / EP: key / value size the registers and LDS rows are laid out for (64 or 128).  A block
+// takes 64 query rows, 16 per wave, row qi = (position in the portion) * nrep + (query head in the group).  POOL: the walk starts with the mean
+// rows of position blocks.  KS: groups of four waves that share the key tiles (each with buffers of its own; their sums meet in LDS)
+template <int DP, int EP, bool POOL, int KS>
+__global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kernel(LAttnArgs a, bool qvec, bool ovec) {
+    constexpr int KLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16;
+    constexpr int KC = DP / 8, VC = EP / 8, KPT = KT * KC / 256, VPT = KT * VC / 256;   // 16-byte chunks per row / per thread
+    extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+    const int tid = threadIdx.x & 255, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+    const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8), wave = tid >> 6;
+    uint16_t* const Ks = smem + grp * 2 * KT * (KLD + VLD);       // [2][64][KLD]
+    uint16_t* const Vs = Ks + 2 * KT * KLD;                       // [2][64][VLD]
+    const int g = blockIdx.x;
+    const int2 tile_id = a.tiles[blockIdx.y];
+    const LaySegDev sg = a.segs[tile_id.x];
+    const int nrep = a.H / a.G, d = a.d, e = a.e;
+    const int q0 = tile_id.y, nq = min(64, sg.n * nrep - q0);
+    Walk w;
+    w.init<POOL>(a, sg, q0, nq, nrep);
+    Query q;
+    q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk, lg, grp == 0);
+    bf16x8 qf[NKS];                                    // rounded once
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+        float x[8];
+        query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, ks * 32 + lg * 8, d, q.ok, qvec, x);
+        u32x4 pk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
+        qf[ks] = __builtin_bit_cast(bf16x8, pk);
+    }
+
+    // page of every position tile; lane i holds that of tile 64 grp + i
+    int pgs_grp = 0;
+    auto load_pages = [&](int grp64) __attribute__((always_inline)) {
+        const int j = min(w.first(min(grp64 * 64 + lane, w.ntile - 1)), w.pmax);
+        return a.bt[sg.bt_off + j / a.page];
+    };
+    int pgs = load_pages(0);
+    struct Rows { u32x4 k[KPT], v[VPT]; };
+    const int Gv = a.v_div > 1 ? a.G / a.v_div : a.G, gv = a.v_div > 1 ? g / a.v_div : g, ldv = a.vpool ? e : d;
+    // this thread's rows and 16-byte column of a tile.  Columns of the padding hold column 0 (their queries' are zero): no load under a branch
+    static_assert(256 % KC == 0 && 256 % VC == 0, "one column per thread");
+    const int kr0 = tid / KC, vr0 = tid / VC;
+    const int kc = (tid % KC) * 8 < d ? (tid % KC) * 8 : 0, vc = (tid % VC) * 8 < e ? (tid % VC) * 8 : 0;
+    auto fetch = [&](int t_, Rows& rg) __attribute__((always_inline)) {
+        const int t = min(t_, w.ntile - 1);            // past the end: the last tile again, parked into a buffer nobody reads
+        const int j0 = w.first(t);
+        if ((t >> 6) != pgs_grp) { pgs_grp = t >> 6; pgs = load_pages(pgs_grp); }      // (uniform)
+        if (POOL && t < w.front) {
+            const uint16_t* vpool = a.pv_pool ? (const uint16_t*)a.pv_pool : (const uint16_t*)a.pk_pool;
+#pragma unroll
+            for (int i = 0; i < KPT; ++i)
+                rg.k[i] = ld16((const uint16_t*)a.pk_pool + block_row(a, sg, g, min(j0 + kr0 + i * (256 / KC), w.blocks - 1), w.pool) * d + kc);
+#pragma unroll
+            for (int i = 0; i < VPT; ++i)
+                rg.v[i] = ld16(vpool + block_row(a, sg, g, min(j0 + vr0 + i * (256 / VC), w.blocks - 1), w.pool) * ldv + vc);
+            return;
+        }
+        const int pg = __builtin_amdgcn_readlane(pgs, t & 63), r0 = j0 % a.page, last = w.pmax - j0;   // rows past the newest position: that one again
+        const uint16_t* kp = (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + r0) * d;
+        const uint16_t* vp = a.vpool ? (const uint16_t*)a.vpool + (((size_t)pg * Gv + gv) * a.page + r0) * e : kp;
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) rg.k[i] = ld16(kp + min(kr0 + i * (256 / KC), last) * d + kc);
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) rg.v[i] = ld16(vp + min(vr0 + i * (256 / VC), last) * ldv + vc);
+    };
+    auto park = [&](int buf, const Rows& rg) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KPT; ++i) *(u32x4*)&Ks[(buf * KT + kr0 + i * (256 / KC)) * KLD + (tid % KC) * 8] = rg.k[i];
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) *(u32x4*)&Vs[(buf * KT + vr0 + i * (256 / VC)) * VLD + (tid % VC) * 8] = rg.v[i];
+    };
+
+    f32x4 o[NNT];
+#pragma unroll
+    for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // step i: tile KS i + grp of this group; the rows of step i + 2 are requested at its top, those of step i + 1 parked at its bottom
+    auto step = [&](int i, Rows& rg_new, const Rows& rg_next) __attribute__((always_inline)) {
+        const int t = KS * i + grp;
+        fetch(t + 2 * KS, rg_new);
+        if (KS == 1 || t < w.ntile) {                  // (uniform) the last step of an odd walk: the other group's only
+            const uint16_t* Kb = Ks + (i & 1) * KT * KLD;
+            f32x4 s[4];
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) {
+                s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < NKS; ++ks) {
+                    const bf16x8 kf = *(const bf16x8*)&Kb[(tt * 16 + lr) * KLD + ks * 32 + lg * 8];
+                    s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], s[tt], 0, 0, 0);
+                }
+            }
+            bf16x8 p[2][2];
+            q.template weights<POOL>(a, w, t, lg, s, p, o);
+            values<VLD>(Vs + (i & 1) * KT * VLD, lr, lg, p, o);
+        }
+        park((i + 1) & 1, rg_next);                    // that buffer was last read one step ago, behind that step's barrier
+        lds_barrier();
+    };
+    Rows ra, rb;
+    fetch(grp, ra);
+    fetch(grp + KS, rb);
+    park(0, ra);
+    lds_barrier();
+    const int steps = (w.ntile + KS - 1) / KS;
+    for (int i = 0; i < steps; i += 2) {
+        step(i, ra, rb);
+        if (i + 1 < steps) step(i + 1, rb, ra);
+    }
+    float l = q.l, c0 = 1.f;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (KS == 2) {                                     // group 1 leaves its sums, group 0 takes them in
+        float* po = (float*)smem;                      // [4 waves][NNT][64 lanes][4], then [4 waves][64 lanes] maxima and sums
+        float* pm = po + 4 * NNT * 64 * 4;
+        if (grp == 1) {
+#pragma unroll
+            for (int n = 0; n < NNT; ++n) *(f32x4*)&po[((wave * NNT + n) * 64 + lane) * 4] = o[n];
+            pm[wave * 64 + lane] = q.m;
+            pm[256 + wave * 64 + lane] = l;
+        }
+        lds_barrier();
+        if (grp == 1) return;
+        const float m1 = pm[wave * 64 + lane], l1 = pm[256 + wave * 64 + lane];
+        const float mn = fmaxf(q.m, m1), ms = mn == -INFINITY ? 0.f : mn;
+        const float c1 = __builtin_amdgcn_exp2f(m1 - ms);
+        c0 = __builtin_amdgcn_exp2f(q.m - ms);
+        l = l * c0 + l1 * c1;
+#pragma unroll
+        for (int n = 0; n < NNT; ++n) {
+            const f32x4 p = *(const f32x4*)&po[((wave * NNT + n) * 64 + lane) * 4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[n][r] = o[n][r] * c0 + p[r] * c1;
+        }
+    }
+    if (!q.ok) return;
+#pragma unroll
+    for (int n = 0; n < NNT; ++n) {
+        const int c = n * 16 + lg * 4;
+        if (c < e) put4(a, q.row, q.head, c, o[n], l, ovec);
+    }
+}
+
+template <int DP, int EP, bool POOL, int KS>
 void go(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
-    constexpr size_t lds = (size_t)2 * KT * (DP + 8 + EP + 16) * sizeof(uint16_t);
+    constexpr size_t lds = (size_t)KS * 2 * KT * (DP + 8 + EP + 16) * sizeof(uint16_t);
+    static_assert(KS == 1 || lds >= (size_t)(4 * (EP / 16) * 64 * 4 + 512) * sizeof(float), "the groups' sums");
     static DevOnce attr;
     attr.run([&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_tile_kernel<DP, EP, POOL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_tile_kernel<DP, EP, POOL, KS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    hipLaunchKernelGGL((lay_attn_tile_kernel<DP, EP, POOL>), dim3((unsigned)a.G, (unsigned)a.ntiles), dim3(256), lds, s, a, qvec, ovec);
+    hipLaunchKernelGGL((lay_attn_tile_kernel<DP, EP, POOL, KS>), dim3((unsigned)a.G, (unsigned)a.ntiles), dim3(256 * KS), lds, s, a, qvec, ovec);
 }
+
+// ---- decode steps: few query rows (tiles of 16, lay_attn_kernel's), each wave on key tiles of its own.  Keys go from the pages straight into
+// fragments, values through a private LDS tile (no barrier inside the walk); a tile's keys are requested as soon as the one before has been
+// multiplied, its values as soon as the one before is in LDS.  The eight waves' sums meet in LDS once; gridDim.z > 1: they leave a partial
+// sum for lay_attn_merge_kernel instead.  Queries and weights keep their 24 bits, as in lay_attn_kernel: three bfloat16 parts each, three
+// products per tile (the launch waits for memory, not for the matrix cores).
+constexpr int DW = 8;
+template <int DP, int EP, bool POOL>
+__global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
+    constexpr int QLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16, VC = EP / 8, VPL = KT * VC / 64;
+    extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+    __shared__ float pm[DW][16], pl_[DW][16];
+    uint16_t* const Qs = smem + DW * KT * VLD;         // [3 parts][16][QLD]
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint16_t* const Vw = smem + wave * KT * VLD;       // [64][VLD] of this wave
+    const int g = blockIdx.x;
+    const int2 tile_id = a.tiles[blockIdx.y];
+    const LaySegDev sg = a.segs[tile_id.x];
+    const int nrep = a.H / a.G, d = a.d, e = a.e;
+    const int q0 = tile_id.y, nq = min(16, sg.n * nrep - q0);
+    Walk w;
+    w.init<POOL>(a, sg, q0, nq, nrep);
+    const int t_first = (int)blockIdx.z * DW + wave, t_step = DW * (int)gridDim.z;
+    Query q;
+    q.init(a, sg, g, lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
+    int pgs_grp = 0;                                   // lane i: page of this wave's tile 64 grp + i
+    auto load_pages = [&](int grp) __attribute__((always_inline)) {
+        const int j = min(w.first(min(t_first + (grp * 64 + lane) * t_step, w.ntile - 1)), w.pmax);
+        return a.bt[sg.bt_off + j / a.page];
+    };
+    int pgs = load_pages(0);
+    const int Gv = a.v_div > 1 ? a.G / a.v_div : a.G, gv = a.v_div > 1 ? g / a.v_div : g;
+    u32x4 kr[4][NKS], vr[VPL];
+    auto page_of = [&](int i) __attribute__((always_inline)) {
+        if ((i >> 6) != pgs_grp) { pgs_grp = i >> 6; pgs = load_pages(pgs_grp); }      // (uniform)
+        return __builtin_amdgcn_readlane(pgs, i & 63);
+    };
+    auto fetch_k = [&](int i) __attribute__((always_inline)) {
+        const int t = t_first + i * t_step;
+        if (t >= w.ntile) return;                      // (uniform)
+        const int j0 = w.first(t), pg = page_of(i), last = w.pmax - j0;
+        const uint16_t* kp = (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + j0 % a.page) * d;
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            const uint16_t* row = kp + min(tt * 16 + lr, last) * d;
+            if (POOL && t < w.front) row = (const uint16_t*)a.pk_pool + block_row(a, sg, g, min(j0 + tt * 16 + lr, w.blocks - 1), w.pool) * d;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) kr[tt][ks] = ld16(row + (ks * 32 + lg * 8 < d ? ks * 32 + lg * 8 : 0));     // no load under a branch
+        }
+    };
+    auto fetch_v = [&](int i) __attribute__((always_inline)) {
+        const int t = t_first + i * t_step;
+        if (t >= w.ntile) return;
+        const int j0 = w.first(t), pg = page_of(i), last = w.pmax - j0, r0 = j0 % a.page;
+        const uint16_t* vp = a.vpool ? (const uint16_t*)a.vpool + (((size_t)pg * Gv + gv) * a.page + r0) * e
+                                     : (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + r0) * d;
+        const int ldv = a.vpool ? e : d, c = (lane % VC) * 8 < e ? (lane % VC) * 8 : 0;
+#pragma unroll
+        for (int k = 0; k < VPL; ++k) {
+            const int row = lane / VC + k * (64 / VC);
+            const uint16_t* src = vp + min(row, last) * ldv;
+            if (POOL && t < w.front) {
+                const size_t br = block_row(a, sg, g, min(j0 + row, w.blocks - 1), w.pool);
+                src = a.pv_pool ? (const uint16_t*)a.pv_pool + br * e : (const uint16_t*)a.pk_pool + br * d;
+            }
+            vr[k] = ld16(src + c);
+        }
+    };
+    f32x4 o[NNT];
+#pragma unroll
+    for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    fetch_k(0);
+    fetch_v(0);
+    for (int ks = wave; ks < NKS; ks += DW) {
+        float x[8];
+        query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, ks * 32 + lg * 8, d, q.ok, qvec, x);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            u32x4 pk;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                pk[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
+                x[2 * i] -= bf16_lo(pk[i]); x[2 * i + 1] -= bf16_hi(pk[i]);
+            }
+            *(u32x4*)&Qs[(k * 16 + lr) * QLD + ks * 32 + lg * 8] = pk;
+        }
+    }
+    lds_barrier();
+    for (int i = 0, t = t_first; t < w.ntile; ++i, t += t_step) {
+        f32x4 s[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+            for (int k = 2; k >= 0; --k) {             // the smallest part first
+                const bf16x8 qf = *(const bf16x8*)&Qs[(k * 16 + lr) * QLD + ks * 32 + lg * 8];
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[tt][ks]), qf, s[tt], 0, 0, 0);
+            }
+        fetch_k(i + 1);
+#pragma unroll
+        for (int k = 0; k < VPL; ++k) *(u32x4*)&Vw[(lane / VC + k * (64 / VC)) * VLD + (lane % VC) * 8] = vr[k];
+        fetch_v(i + 1);
+        bf16x8 p[3][2];
+        q.template weights<POOL>(a, w, t, lg, s, p, o);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the wave's own tile is in LDS
+        values<VLD>(Vw, lr, lg, p, o);
+    }
+    float l = q.l;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (lg == 0) { pm[wave][lr] = q.m; pl_[wave][lr] = l; }
+    __syncthreads();                                   // every wave's value tile has been read: its place holds the sums
+    float* po = (float*)smem;                          // [wave][NNT][64 lanes][4]
+#pragma unroll
+    for (int n = 0; n < NNT; ++n) *(f32x4*)&po[((wave * NNT + n) * 64 + lane) * 4] = o[n];
+    __syncthreads();
+    float M = -INFINITY, L = 0.f, cw[DW];
+#pragma unroll
+    for (int k = 0; k < DW; ++k) M = fmaxf(M, pm[k][lr]);
+    const float ms = M == -INFINITY ? 0.f : M;
+#pragma unroll
+    for (int k = 0; k < DW; ++k) { cw[k] = __builtin_amdgcn_exp2f(pm[k][lr] - ms); L = fmaf(pl_[k][lr], cw[k], L); }
+    const int nsplit = (int)gridDim.z;
+    const size_t pr = (((size_t)blockIdx.y * a.G + g) * nsplit + blockIdx.z) * 16 + lr;
+    if (nsplit > 1 && wave == 0 && lg == 0) { a.part_ml[pr * 2] = M * 0.6931471805599453f; a.part_ml[pr * 2 + 1] = L; }     // the merge works in e
+    for (int n = wave; n < NNT; n += DW) {
+        const int c = n * 16 + lg * 4;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < DW; ++k) {
+            const f32x4 p = *(const f32x4*)&po[((k * NNT + n) * 64 + lane) * 4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = fmaf(p[r], cw[k], v[r]);
+        }
+        if (c >= e) continue;
+        if (nsplit > 1) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a.part_o[pr * e + c + r] = v[r];
+        } else if (q.ok) put4(a, q.row, q.head, c, v, L, ovec);
+    }
+}
+template <int DP, int EP, bool POOL>
+void go_few(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
+    constexpr size_t lds = ((size_t)DW * KT * (EP + 16) + 3 * 16 * (DP + 8)) * sizeof(uint16_t);
+    static_assert(lds >= (size_t)DW * (EP / 16) * 64 * 4 * sizeof(float), "the waves' sums");
+    static DevOnce attr;
+    attr.run([&] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_few_kernel<DP, EP, POOL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    });
+    hipLaunchKernelGGL((lay_attn_few_kernel<DP, EP, POOL>), dim3((unsigned)a.G, (unsigned)a.ntiles, (unsigned)nsplit), dim3(DW * 64), lds, s, a, qvec, ovec);
+}
+// nsplit 0: the prompt kernel
 template <int DP, int EP>
-void go_sizes(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
-    if (a.pool > 0) go<DP, EP, true>(a, qvec, ovec, s);
-    else go<DP, EP, false>(a, qvec, ovec, s);
+void go_sizes(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
+    // one block per CU at most: two groups of waves share the key tiles (a mixed batch of 24 single tokens and 300 prompt rows on 8 heads:
+    // 24 us against 27); more blocks share the CUs by themselves
+    const bool two = (long long)a.ntiles * a.G <= 256;
+    if (nsplit > 0) { if (a.pool > 0) go_few<DP, EP, true>(a, nsplit, qvec, ovec, s); else go_few<DP, EP, false>(a, nsplit, qvec, ovec, s); }
+    else if (a.pool > 0) { if (two) go<DP, EP, true, 2>(a, qvec, ovec, s); else go<DP, EP, true, 1>(a, qvec, ovec, s); }
+    else { if (two) go<DP, EP, false, 2>(a, qvec, ovec, s); else go<DP, EP, false, 1>(a, qvec, ovec, s); }
 }
 
 }  // namespace
@@ -291,15 +521,34 @@ bool lay_attn_tile_fits(int d, int e, bool own_v, int page) {
     return d > 0 && e > 0 && d % 16 == 0 && e % 16 == 0 && d <= 128 && e <= 128 && (own_v || e <= d) && page % KT == 0;
 }
 
-void launch_lay_attn_tile(const LAttnArgs& a0, hipStream_t s) {
-    if (a0.ntiles <= 0) return;
+static void launch(const LAttnArgs& a0, int nsplit, hipStream_t s) {
     LAttnArgs a = a0;
     if (!a.gbuf) { a.gbuf = a.proj + a.g_off; a.ldg = a.ldp; }
     if (a.e <= 0) a.e = a.d;
     const bool qvec = a.ldp % 4 == 0 && a.q_off % 4 == 0 && ((uintptr_t)a.proj & 15) == 0;
     const bool ovec = a.ldo % 4 == 0 && ((uintptr_t)a.out & 15) == 0;
-    if (a.d <= 64) { if (a.e <= 64) go_sizes<64, 64>(a, qvec, ovec, s); else go_sizes<64, 128>(a, qvec, ovec, s); }
-    else { if (a.e <= 64) go_sizes<128, 64>(a, qvec, ovec, s); else go_sizes<128, 128>(a, qvec, ovec, s); }
+    if (a.d <= 64) { if (a.e <= 64) go_sizes<64, 64>(a, nsplit, qvec, ovec, s); else go_sizes<64, 128>(a, nsplit, qvec, ovec, s); }
+    else { if (a.e <= 64) go_sizes<128, 64>(a, nsplit, qvec, ovec, s); else go_sizes<128, 128>(a, nsplit, qvec, ovec, s); }
+}
+
+void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s) {
+    if (a.ntiles > 0) launch(a, 0, s);
+}
+
+int lay_attn_few_split(long long visible, int blocks, int parts) {
+    // one key tile per wave, then more blocks and a merge: a further tile in the same wave costs about 4 us (its keys and values are two trips to
+    // memory), the merge 6.  Eight tokens of four layers of width 4096, 32 heads on 8: context 3500 5.02 - 5.20 ms with one, 5.17 - 5.23 with two
+    // tiles per wave; context 100 (no split) 4.96
+    const long long tiles = (visible + KT - 1) / KT + 1;
+    if (tiles <= DW) return 1;
+    return (int)std::max(1ll, std::min({(tiles + DW - 1) / DW, 256ll / std::max(1, blocks), (long long)parts / std::max(1, blocks)}));
+}
+
+void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s) {
+    if (a.ntiles <= 0) return;
+    const int nsplit = a.part_o && a.part_ml && a.nsplit > 1 ? a.nsplit : 1;
+    launch(a, nsplit, s);
+    if (nsplit > 1) launch_lay_attn_merge(a, nsplit, s);
 }
 
 }  // namespace cm

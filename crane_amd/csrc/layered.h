@@ -317,6 +317,11 @@ bool lay_attn_mfma_fits(int d, int e, bool own_v);         // sizes the matrix-c
 // and long cached rows
 void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
+// the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can
+// see, blocks of an unsplit launch, scratch parts)
+void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s);
+int lay_attn_few_split(long long visible, int blocks, int parts);
+void launch_lay_attn_merge(const LAttnArgs& a, int nsplit, hipStream_t s);
 
 struct LLightArgs {
     const float* proj; int ldp, q_off, k_off, v_off; // activated projection rows

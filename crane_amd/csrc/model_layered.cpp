@@ -1740,10 +1740,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             a.r1 = w.r1; a.r2 = w.r2; a.H = sp.heads; a.G = sp.kv_heads; a.d = dk; a.page = page;
             a.scale = sp.scale; a.win = sp.win; a.keep = sp.keep; a.chunk = sp.chunk;
             a.bias = sp.bias; a.gate = sp.gate; a.sink = sp.sink ? w.sink : nullptr;
+            long long seen = std::min<long long>(max_len, sp.win + sp.keep);
+            if (sp.chunk > 0) seen = std::min(seen, sp.chunk);
+            if (sp.pool > 0) seen = std::min<long long>(max_len, sp.win + max_len / sp.pool);
             {   // few query tiles and many visible keys (decode steps): share a tile's keys among blocks
-                long long seen = std::min<long long>(max_len, sp.win + sp.keep);
-                if (sp.chunk > 0) seen = std::min(seen, sp.chunk);
-                if (sp.pool > 0) seen = std::min<long long>(max_len, sp.win + max_len / sp.pool);
                 const int kt = lay_attn_key_tile(dk, ev, a.vpool != nullptr);
                 const int key_tiles = (int)((seen + kt - 1) / kt), blocks = std::max(1, a.ntiles * sp.kv_heads);
                 a.nsplit = std::max(1, std::min({32, key_tiles, 256 / blocks, Layered::ATT_PARTS / blocks}));
@@ -1754,6 +1754,9 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 a.tiles = (const int2*)(L.d_tab + tm.first); a.ntiles = tm.second;
                 if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) launch_lay_attn_tile(a, s);
                 else launch_lay_attn_mfma(a, s);
+            } else if (L.attn_mfma && kv_mode == KV_BF16 && lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
+                a.nsplit = lay_attn_few_split(seen, a.ntiles * sp.kv_heads, Layered::ATT_PARTS);
+                launch_lay_attn_few(a, s);
             } else
                 launch_lay_attn(a, kv_mode, s);
         };

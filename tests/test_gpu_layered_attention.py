@@ -87,3 +87,63 @@ def test_block_rows(tmp_path, d, e, heads, kv, size, pool, portions):
 def test_many_heads(tmp_path, d, e, size, portions):
     mx = GZ.attn(heads=64, kv_heads=64, dim=d, vdim=e, size=size, rot_dims=16)
     _check(_run(tmp_path, GZ, GZ.config([GZ.layer(mx, None)], vocab=96, width=64), portions, 11))
+
+
+# ---- decode steps: the kernel for few query rows keeps 24 bits of queries and weights (three bfloat16 parts each), as the FMA kernel does, so the
+# attention rows agree to a few 1e-6 and what is left is the output projection's rounding of 0.1 % of them: 1e-3 of the largest logit
+TOL_FEW = 1e-3
+
+
+def _few(tmp_path, U, cfg, contexts, steps, seed, **kw):
+    """Three sequences with contexts of their own step together, `steps` tokens each per step; matrix-core kernels on, then off."""
+    from crane_amd.backend import Model
+    P = U.random_weights(cfg, seed)
+    n = max(contexts) + sum(steps)
+    toks = [U.tokens(n, cfg["vocab"], seed + 1 + i) for i in range(len(contexts))]
+    m = Model.from_pretrained(U.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=8, max_seq_len=4096, **kw)
+    got = []
+    try:
+        for on in (1, 0):
+            m.debug_set("lay_attn_mfma", on)
+            seqs, rows, at = [m.seq_alloc() for _ in contexts], [], list(contexts)
+            for s, t, c in zip(seqs, toks, contexts):
+                if c:
+                    m.step_batch([(s, t[:c], [])], want_logits=False)      # one layer: the cached rows do not depend on the attention
+            for k in steps:
+                rows.append(m.step_batch([(s, t[a:a + k], list(range(k))) for s, t, a in zip(seqs, toks, at)])[0])
+                at = [a + k for a in at]
+            got.append(np.concatenate(rows).astype(np.float64))
+            for s in seqs:
+                m.seq_free(s)
+    finally:
+        m.close()
+    assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() < TOL_FEW * np.abs(got[1]).max()
+
+
+# no context, one short of a tile, a tile, one more; more tiles than waves; one and several 16-row tiles per sequence; every key in one wave's
+# first tile or spread over blocks (more than 24 tiles: partial sums and a merge)
+@pytest.mark.parametrize("d,e,heads,kv,size,contexts,steps", [
+    (16, 16, 4, 4, 7, (0, 63, 64), (1, 1, 15)), (64, 80, 6, 2, 64, (65, 127, 600), (1, 3, 1)), (128, 128, 8, 2, 1000, (1, 700, 1300), (1, 1)),
+    (112, 48, 4, 1, 4000, (1600, 2500, 3100), (1, 6)), (80, 128, 16, 1, 3000, (1535, 1536, 2200), (1, 1))])
+@pytest.mark.parametrize("page", [64, 128])
+def test_decode_window_and_one_in_the_denominator(tmp_path, d, e, heads, kv, size, contexts, steps, page):
+    mx = GZ.attn(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size, rot_dims=16)
+    _few(tmp_path, GZ, GZ.config([GZ.layer(mx, None)], vocab=96, width=64), contexts, steps, 13, kv_block_size=page)
+
+
+@pytest.mark.parametrize("d,heads,kv,size,keep,contexts", [(32, 4, 2, 20, 3, (0, 150, 400)), (128, 4, 1, 90, 70, (60, 161, 700)), (48, 5, 5, 300, 128, (330, 5, 1000))])
+def test_decode_kept_first_tokens_and_distance_term(tmp_path, d, heads, kv, size, keep, contexts):
+    mx = KO.attn(heads=heads, kv_heads=kv, dim=d, size=size, keep_first=keep)
+    _few(tmp_path, KO, KO.config([KO.layer("attention", None, **mx)], vocab=96, width=64), contexts, (1, 1, 4), 15)
+
+
+@pytest.mark.parametrize("d,e,heads,kv,size,contexts", [(32, 16, 6, 2, 50, (49, 99, 100)), (128, 112, 4, 2, 64, (63, 64, 500)), (64, 64, 2, 2, 3000, (2999, 1, 2000))])
+def test_decode_position_blocks_and_sink(tmp_path, d, e, heads, kv, size, contexts):
+    mx = MO.attn(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size)
+    _few(tmp_path, MO, MO.config([MO.layer("attention", None, **mx)], vocab=96, width=64), contexts, (1, 2, 1), 17)
+
+
+@pytest.mark.parametrize("d,e,heads,kv,size,pool,contexts", [(32, 16, 4, 2, 20, 6, (19, 26, 300)), (128, 128, 4, 1, 30, 4, (33, 700, 1900)), (64, 96, 2, 2, 70, 64, (133, 134, 64))])
+def test_decode_block_rows(tmp_path, d, e, heads, kv, size, pool, contexts):
+    lf = GI.left(heads=heads, kv_heads=kv, dim=d, vdim=e, size=size, pool=pool)
+    _few(tmp_path, GI, GI.config([GI.layer(lf, GI.right(), None)], vocab=96, width=64), contexts, (1, 1, 3), 19)
