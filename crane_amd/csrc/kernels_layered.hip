@@ -695,7 +695,13 @@ __global__ __launch_bounds__(256) void lgemm_bf16_kernel(LGemmArgs a) {
 constexpr int LV_MAXM = LAY_ROW_KERNEL_ROWS;
 template <bool BF16, bool DUAL>
 __global__ __launch_bounds__(256) void lgemv_kernel(LGemmArgs a) {
-    const int g = blockIdx.z;
+    int g = blockIdx.z;
+    if (a.beside.W && g == (int)gridDim.z - 1) {         // the product beside the groups
+        a.A = a.beside.A; a.lda = a.beside.lda; a.W = a.beside.W; a.W2 = a.beside.W2; a.C = a.beside.C; a.ldc = a.beside.ldc;
+        a.N = a.beside.N; a.K = a.beside.K; a.act_param = a.beside.act_param;
+        a.a_idx = nullptr; a.a_scale = nullptr; a.c_idx = nullptr; a.grp_off = nullptr; a.w_stride = 0; a.a_goff = 0; a.c_goff = 0;
+        g = 0;
+    }
     int base = 0, rows = a.M;
     if (a.grp_off) { base = a.grp_off[g]; rows = a.grp_off[g + 1] - base; }
     if (rows <= 0) return;
@@ -817,7 +823,7 @@ void launch_lay_round_rows(const float* x, int ldx, uint16_t* out, int M, int K,
 void launch_lgemm(const LGemmArgs& a, bool bf16, int groups, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0 || groups <= 0) return;
     if (a.M <= LV_MAXM) {
-        const dim3 gv((unsigned)((a.N + 7) / 8), 1, (unsigned)groups);
+        const dim3 gv((unsigned)((std::max(a.N, a.beside.W ? a.beside.N : 0) + 7) / 8), 1, (unsigned)(groups + (a.beside.W ? 1 : 0)));
         if (bf16) {
             if (a.W2) hipLaunchKernelGGL((lgemv_kernel<true, true>), gv, dim3(256), 0, s, a);
             else hipLaunchKernelGGL((lgemv_kernel<true, false>), gv, dim3(256), 0, s, a);
@@ -2157,6 +2163,65 @@ __global__ __launch_bounds__(1024) void lay_moe_plan_kernel(const int32_t* __res
 }
 void launch_lay_moe_plan(const int32_t* sel, int32_t* off, int32_t* srt, int n, int E, hipStream_t s, int top, int slots) {
     hipLaunchKernelGGL(lay_moe_plan_kernel, dim3(1), dim3(1024), (size_t)E * sizeof(int), s, sel, off, srt, n, E, top, slots);
+}
+
+// decode steps: router logits, choice and plan in one block (three launches of 4.3, 5.6 and 2.6 us, each waiting for the one before, as one of
+// 7.9).  A wave per (token, logit) in lgemv_kernel's order of additions, a wave per token for the choice, the rows of an expert in token order
+__global__ __launch_bounds__(1024) void lay_router_decode_kernel(const float* __restrict__ h, const uint16_t* __restrict__ wr, int32_t* __restrict__ sel,
+                                                                 float* __restrict__ wsel, int32_t* __restrict__ off, int32_t* __restrict__ srt, int T,
+                                                                 int W, int E, int top, RouterSpec rs, const float* __restrict__ correction, int slots,
+                                                                 int per_tok) {
+    extern __shared__ float zs[];          // [T][per_tok]: logits, scores, groups, chosen scores; then [T top] choices
+    int* chosen = (int*)(zs + (size_t)T * per_tok);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = E + (rs.shared_gate ? 1 : 0), P = T * top;
+    for (int i = wave; i < T * n; i += 16) {
+        const int t = i / n, ex = i - t * n;
+        const float* hr = h + (size_t)t * W;
+        const uint16_t* w = wr + (size_t)ex * W;
+        float acc = 0.f;
+#pragma unroll 4
+        for (int k = lane * 8; k < W; k += 512) {
+            const u32x4 wv = ld16(w + k);
+            const f32x4 xa = *(const f32x4*)(hr + k), xb = *(const f32x4*)(hr + k + 4);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float x0 = c < 2 ? xa[2 * c] : xb[2 * c - 4], x1 = c < 2 ? xa[2 * c + 1] : xb[2 * c - 3];
+                acc = fmaf(bf16_lo(wv[c]), x0, acc);
+                acc = fmaf(bf16_hi(wv[c]), x1, acc);
+            }
+        }
+        acc = wave_sum(acc);
+        if (lane == 0) zs[(size_t)t * per_tok + ex] = acc;
+    }
+    __syncthreads();
+    if (wave < T) {
+        lay_router_choose(zs + (size_t)wave * per_tok, wave, lane, sel, wsel, E, top, rs, correction, slots);
+        __threadfence_block();             // the choices lane 0 wrote to memory are read back below
+        for (int k = lane; k < top; k += 64) chosen[wave * top + k] = sel[(size_t)wave * top + k];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < P; i += 1024) {
+        const int e = chosen[i];
+        int at = 0;
+        for (int j = 0; j < P; ++j) at += chosen[j] < e || (chosen[j] == e && j < i);
+        srt[at] = (i / top) * slots + i % top;
+    }
+    for (int e = threadIdx.x; e <= E; e += 1024) {
+        int before = 0;
+        for (int j = 0; j < P; ++j) before += chosen[j] < e;
+        off[e] = before;
+    }
+}
+bool lay_router_decode_fits(int T, int W, int E, int top, const RouterSpec& rs) {
+    const size_t per_tok = (size_t)2 * E + (rs.shared_gate ? 1 : 0) + rs.groups + top;
+    return T <= LAY_ROW_KERNEL_ROWS && W % 8 == 0 && top <= 64 && (size_t)T * (per_tok + top) * sizeof(float) <= LDS_PLAIN;
+}
+void launch_lay_router_decode(const float* h, const uint16_t* wr, int32_t* sel, float* wsel, int32_t* off, int32_t* srt, int T, int W, int E, int top,
+                              hipStream_t s, const RouterSpec& rs, const float* correction, int slots) {
+    if (T <= 0) return;
+    const int per_tok = 2 * E + (rs.shared_gate ? 1 : 0) + rs.groups + top;
+    hipLaunchKernelGGL(lay_router_decode_kernel, dim3(1), dim3(1024), (size_t)T * (per_tok + top) * sizeof(float), s, h, wr, sel, wsel, off, srt, T, W, E,
+                       top, rs, rs.correction ? correction : nullptr, slots > top ? slots : top, per_tok);
 }
 
 // arg-max of every row, lowest index among equals

@@ -201,6 +201,15 @@ struct LGemmArgs {
     size_t a_goff = 0, c_goff = 0;
     const float* mul = nullptr; int ldm = 0;         // C[p][n] *= mul[p ldm + g c_goff + n] after the activation
     const float* a_scale = nullptr;                  // with a_idx: the A row of output row p is multiplied by a_scale[a_idx[p]] (before any rounding)
+    // up to LAY_ROW_KERNEL_ROWS rows: one more product of its own sizes over rows 0 .. M - 1 in the same launch (act and the presence of a second
+    // matrix are the main product's)
+    struct Beside {
+        const float* A = nullptr; int lda = 0;
+        const uint16_t *W = nullptr, *W2 = nullptr;
+        float* C = nullptr; int ldc = 0;
+        int N = 0, K = 0;
+        float act_param = 1.f;
+    } beside;
 };
 // bf16 = true: A rounded to bfloat16, matrix cores, f32 accumulation; false: f32 FMA throughout.  Up to 8 rows (per group): the
 // streaming row kernel instead of tiles.
@@ -303,6 +312,10 @@ void launch_lay_qk_prep(float* proj, int ldp, int q_off, int k_off, int v_off, i
                         float eps, int dims, bool half, const float* freq, float mag, void* kpool, void* vpool, int kvt, const int32_t* bt,
                         const LaySegDev* segs, const int32_t* rowseg, int T, int page, hipStream_t s, int pool = 0, int pool_rows = 0,
                         void* pk_pool = nullptr, void* pv_pool = nullptr, const LQkPrepExtra* extra = nullptr);
+// decode steps (at most LAY_ROW_KERNEL_ROWS rows): logits, choice and the rows sorted by expert in one launch (lay_router_decode_fits)
+bool lay_router_decode_fits(int T, int W, int E, int top, const RouterSpec& rs);
+void launch_lay_router_decode(const float* h, const uint16_t* wr, int32_t* sel, float* wsel, int32_t* off, int32_t* srt, int T, int W, int E, int top,
+                              hipStream_t s, const RouterSpec& rs, const float* correction, int slots);
 inline int lay_pool_rows(int page, long long pool) { return pool >= page ? 1 : (int)((page + pool - 1) / pool); }
 void launch_lay_attn(const LAttnArgs& a, int kvt, hipStream_t s);    // kvt: KV_BF16 | KV_F32
 bool lay_attn_fits(int d, int e, bool own_v);                         // sizes the kernel can hold in LDS and registers

@@ -176,11 +176,16 @@ static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const Layered
         tile(su, L.Abf, false);
         tile(sdn, (const uint16_t*)L.HS, false);
     }
+    const bool beside = every && T <= LAY_ROW_KERNEL_ROWS;        // decode steps: the expert of every token rides in the same two launches
+    if (beside) {
+        gu.beside = {su.A, su.lda, su.W, su.W2, su.C, su.ldc, su.N, su.K, su.act_param};
+        dn.beside = {sdn.A, sdn.lda, sdn.W, nullptr, sdn.C, sdn.ldc, sdn.N, sdn.K, 1.f};
+    }
     if (!routed) {
         lay_gemm(m, L, gu, sp.experts, s);
         lay_gemm(m, L, dn, sp.experts, s);
     }
-    if (!shared && every) {
+    if (!shared && every && !beside) {
         lay_gemm(m, L, su, 1, s);
         lay_gemm(m, L, sdn, 1, s);
     }
@@ -1855,6 +1860,15 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             else launch_lay_add_gnorm(L.X, nullptr, padd.y, padd.nsum, nw_, out, T, W, L.norm_groups, cfg.eps, s, padd.wsel);
             padd.y = nullptr; padd.wsel = nullptr;
         };
+        // choices and weights of every row of h, and the rows sorted by expert
+        auto route = [&](const float* h, const uint16_t* wr, int outs, int top, const RouterSpec& rs, const float* correction, int slots) {
+            if (lay_router_decode_fits(T, W, outs, top, rs)) {
+                launch_lay_router_decode(h, wr, L.sel, L.wsel, L.off, L.srt, T, W, outs, top, s, rs, correction, slots);
+                return;
+            }
+            launch_lay_router(h, wr, L.sel, L.wsel, T, W, outs, top, s, &rs, correction, slots, L.Z);
+            launch_lay_moe_plan(L.sel, L.off, L.srt, T * top, outs, s, top, slots);
+        };
         const float *par_y1 = nullptr, *par_y2 = nullptr;       // parallel layers: sublayer outputs not yet added to the residual
         for (size_t li = 0; li < L.spec.size(); ++li) {
             const LayerSpec& sp = L.spec[li];
@@ -2058,8 +2072,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     // scale_input: an expert's weight multiplies its INPUT, the rows of the grouped product are w h and the combine is a plain
                     // sum; otherwise the weights join in the combine
                     const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
-                    launch_lay_router(L.Hc, w.router, L.sel, L.wsel, T, W, sp.experts, sp.top, s, &sp.router, nullptr, slots, L.Z);
-                    launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, sp.experts, s, sp.top, slots);
+                    route(L.Hc, w.router, sp.experts, sp.top, sp.router, nullptr, slots);
                     lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s);
                     padd.y = L.YS; padd.nsum = slots; padd.wsel = sp.scale_input ? nullptr : L.wsel;
                 }
@@ -2128,8 +2141,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 } else if (sp.mlp == LMLP_MOE) {
                     flush_post();
                     const int outs = sp.experts + sp.router.identity, slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
-                    launch_lay_router(L.X, w.router, L.sel, L.wsel, T, W, outs, sp.top, s, &sp.router, w.correction, slots, L.Z);
-                    launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, outs, s, sp.top, slots);
+                    route(L.X, w.router, outs, sp.top, sp.router, w.correction, slots);
                     lay_experts(*this, L, sp, w, L.X, T, W, slots, s);
                     post_norm(L.YS, w.norm2b, L.wsel, slots);
                     if (sp.router.identity > 0) { pend.sel_top = sp.top; pend.n_real = sp.experts; }      // identity rows are taken in the combine
@@ -2169,8 +2181,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     lay_gemm(*this, L, dn, 1, s);
                     post_norm(L.Y, w.norm2b, nullptr, 0);
                 } else {
-                    launch_lay_router(L.Hc, w.router, L.sel, L.wsel, T, W, sp.experts, sp.top, s, nullptr, nullptr, 0, L.Z);
-                    launch_lay_moe_plan(L.sel, L.off, L.srt, T * sp.top, sp.experts, s);
+                    route(L.Hc, w.router, sp.experts, sp.top, RouterSpec(), nullptr, sp.top);
                     lay_experts(*this, L, sp, w, L.Hc, T, W, sp.top, s);
                     post_norm(L.YS, w.norm2b, L.wsel, sp.top);
                 }

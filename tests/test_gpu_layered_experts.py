@@ -72,8 +72,9 @@ def test_sigmoid_routed_experts_without_a_shared_one(tmp_path):
 
 # the router's row kernel against the oracle in the float32 format: logits below, at and above its register sizes (16, 20, 32; more stay on the
 # block-per-token form), one and two tokens per wave, a last wave with one of two
-@pytest.mark.parametrize("experts,shared", [(16, 0), (16, 28), (20, 28), (32, 0), (32, 28)])
-@pytest.mark.parametrize("n", [9, 1025])
+# (up to 8 rows: logits, choice and plan in one block, the expert of every token beside the groups)
+@pytest.mark.parametrize("experts,shared", [(3, 28), (16, 0), (16, 28), (20, 28), (32, 0), (32, 28), (70, 12)])
+@pytest.mark.parametrize("n", [1, 3, 8, 9, 1025])
 def test_router_rows(tmp_path, experts, shared, n):
     from crane_amd.backend import Model
     cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=experts, top=3, ff=24, shared=shared))], vocab=61, width=72)
