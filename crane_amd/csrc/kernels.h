@@ -140,8 +140,9 @@ struct GemmArgs {
     int ksplit_cap = 0;        // split-K of the 128-wide kernel: at most this many blocks (0: the default 768; the vision tower passes 512)
     int ksplit;             // set by launch_gemm
     int dbg = 0;            // kernels_gemmw4.hip timing experiments (CM_GEMMW4_DBG); 0 in production
-    int wide256 = 1;        // 0: never the LDS-DMA kernels (kernels_gemm256.hip / kernels_gemmw4.hip), 1: automatic, 2: always kernels_gemmw4.hip,
+    int wide256 = 1;        // 0: never the LDS-DMA kernels (kernels_gemm_rows.hip / kernels_gemm256.hip / kernels_gemmw4.hip), 1: automatic, 2: always kernels_gemmw4.hip,
                             // 3: kernels_gemm256.hip only -- A/B switch, cm_debug_set("gemm256")
+                            // 4: kernels_gemm_rows.hip where its rule takes the sizes, else as 0 (the head of a decode group)
     // GEPI_RESADD with ldc == N only: ALSO write RMSNorm(C row) * norm_w as bf16 hi + lo planes [M][N] -- the A operand of the NEXT
     // GEMM (rmsnorm_rows_kernel's arithmetic).  Fused into the split-K reduction launch when the GEMM splits K (a large decode
     // group: one launch less per projection), a separate rmsnorm_rows launch otherwise -- launch_gemm does either.
@@ -151,6 +152,11 @@ struct GemmArgs {
     uint16_t* norm_lo = nullptr;
     float norm_eps = 0.f;
 };
+
+// 9 .. 128 rows with hi + lo activations (kernels_gemm_rows.hip): K slices for these sizes (0: not taken) and the launch (a.ksplit set; more than
+// one slice: partial tiles in a.ws)
+int gemm_rows_split(int M, int N, int K, size_t ws_floats);
+bool launch_gemm_rows(const GemmArgs& a, int epi, hipStream_t s);
 
 // one sequence of a multi-sequence prompt pass (Model::prefill_multi): rows [row0, row0 + S) of the pass at positions start_pos...,
 // page table at block_table + bt_off

@@ -1,0 +1,170 @@
+// Products of a decode group of 9 .. 64 rows (the narrow ones up to 128) and of prompts that short: C[M, N] (+)= A[M, K] . W[N, K]^T with the
+// activations as bf16 hi + lo planes, two MFMAs per product -- gemm256_kernel's arithmetic and epilogues on tiles made for a launch that waits
+// for its weights.
+//
+// What bounds it: the weight stream.  gemm256_kernel's tiles are 192 or 256 columns wide: 96 .. 128 workgroups for a 24576-column projection,
+// on half of the chip.  Here a workgroup of four waves owns 128 columns, one workgroup on each CU, with two (at 32 rows: three) weight tiles of
+// 16 KB in flight under the one it multiplies; the activations come out of the L2.  Tiles go from memory into LDS without passing registers
+// (8 rows x 128 bytes per wave instruction, the bank swizzle on the source address: slot p of a row holds its 16-byte chunk
+// p ^ ((row >> 1) & 7)), ST stages, one barrier per k-tile.  Narrow projections split K and leave f32 partial tiles for the fixed-order
+// reduction kernels.  Measured (us per launch with its reduction, 32 rows, gemm256_kernel / gemm_bf16_kernel -> here):
+//   width 4096:  gate_up (24576 x 4096) 50.3 -> 46.6 (4.3 TB/s), down (4096 x 12288) 34.4 -> 24.8, qkv (6144 x 4096) 17.5 -> 14.9, o 15.0 -> 11.8;
+//                the whole layer at 16 / 32 / 64 / 128 rows 114 / 117 / 125 / 160 -> 95 / 98 / 113 / 149
+//   width 2048 (I 6144): layer 54 -> 40;  width 1024 (I 3072): 40 -> 31;  lm_head (151936 x 4096) 385 -> 277 (4.5 TB/s), 391 -> 290 at 64 rows
+// Tiles of 64 columns, weight loads that bypass the caches, two workgroups per CU with fewer stages, a k start of its own per workgroup and
+// two k-tiles per barrier were all no faster.
+#include "dev_common.h"
+#include "kernels.h"
+
+namespace cm {
+
+namespace {
+
+constexpr int RBK = 64, RBN = 128;
+
+__device__ __forceinline__ void rows_load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
+}
+
+template <int BM, int ST, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs a) {
+    constexpr int GM = BM == 32 ? 1 : 2, GN = 4 / GM, WM = BM / GM, WN = RBN / GN, NI = WM / 16, NJ = WN / 16;      // waves GM x GN, WM x WN outputs each
+    constexpr int PLANE = BM * RBK, STAGE = 2 * PLANE + RBN * RBK;
+    constexpr int APC = BM / 8, NL = (2 * APC + RBN / 8) / 4;                          // pieces per plane / requests per wave and k-tile
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / GN, wn = wave % GN;
+    const int tiles = a.N / RBN, ks = (int)blockIdx.x / tiles, n0 = ((int)blockIdx.x - ks * tiles) * RBN;
+    const int K = a.K, kpb = K / RBK / a.ksplit, kbeg = ks * kpb;
+
+    const int prow = lane >> 3, pslot = lane & 7;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+    const uint16_t* src[NL];
+    uint32_t dst[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int p = wave + 4 * i, plane = p / APC;                                   // 0: hi, 1: lo, 2 and up: weights
+        const int r0 = (plane < 2 ? p - plane * APC : p - 2 * APC) * 8, row = r0 + prow;
+        const size_t kc = (size_t)kbeg * RBK + (size_t)((pslot ^ ((row >> 1) & 7)) << 3);
+        const bool isw = plane >= 2;
+        src[i] = isw ? a.W + (size_t)(n0 + row) * K + kc : (plane ? a.A_lo : a.A_hi) + (size_t)min(row, a.M - 1) * K + kc;
+        dst[i] = lds0 + (uint32_t)((isw ? 2 * PLANE : plane * PLANE) + r0 * RBK) * 2u;
+    }
+    auto request = [&](int t) __attribute__((always_inline)) {                          // past the end: the last tile again, into a stage nobody reads
+        const size_t at = (size_t)min(t, kpb - 1) * RBK;
+        const uint32_t stage = (uint32_t)((t % ST) * STAGE) * 2u;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) rows_load16(src[i] + at, dst[i] + stage);
+    };
+    f32x4 acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, lg = lane >> 4, sw = (fr >> 1) & 7;
+#pragma unroll
+    for (int t = 0; t < ST - 1; ++t) request(t);
+    for (int t = 0; t < kpb; ++t) {
+        // this wave's share of tile t has landed and its reads of tile t - 1 are done; behind the barrier that holds for every wave
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * NL) : "memory");
+        request(t + ST - 1);
+        const uint16_t* S = lds + (t % ST) * STAGE;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int fk = ((s * 4 + lg) ^ sw) << 3;
+            bf16x8 ah[NI], al[NI], bf[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) bf[j] = *(const bf16x8*)&S[2 * PLANE + (wn * WN + j * 16 + fr) * RBK + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                ah[i] = *(const bf16x8*)&S[(wm * WM + i * 16 + fr) * RBK + fk];
+                al[i] = *(const bf16x8*)&S[PLANE + (wm * WM + i * 16 + fr) * RBK + fk];
+            }
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bf[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bf[j], acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                    // no request of the tail may land after the block is gone
+    // D of a product: column = lane % 16, rows 4 (lane / 16) + r
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = wm * WM + i * 16 + lg * 4 + r;
+            const bool ok = m < a.M;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int n = n0 + wn * WN + j * 16 + fr;
+                float v = acc[i][j][r];
+                if (EPI == GEPI_PARTIAL) {
+                    if (ok) a.ws[((size_t)ks * a.M + m) * a.N + n] = v;
+                    continue;
+                }
+                if (a.bias != nullptr) v += a.bias[n];
+                if (EPI == GEPI_STORE) {
+                    if (ok) a.C[(size_t)m * a.ldc + n] = v;
+                } else if (EPI == GEPI_RESADD) {
+                    if (ok) a.C[(size_t)m * a.ldc + n] += v;
+                } else {                                                                // GEPI_SILUMUL: even column = gate_j, odd column = up_j
+                    const float up = dpp_mov<0xB1>(v);                                  // lane ^ 1
+                    if (((lane & 1) == 0) && ok) {
+                        const float h = (v / (1.0f + expf(-v))) * up;
+                        const size_t off = (size_t)m * (a.N / 2) + (n >> 1);
+                        const uint16_t hh = f32_to_bf16(h);
+                        a.H_hi[off] = hh;
+                        if (a.H_lo) a.H_lo[off] = f32_to_bf16(h - bf16_to_f32(hh));
+                    }
+                }
+            }
+        }
+}
+
+template <int BM, int ST, int EPI>
+void go(const GemmArgs& a, hipStream_t s) {
+    constexpr size_t lds = (size_t)ST * (2 * BM + RBN) * RBK * sizeof(uint16_t);
+    static DevOnce attr;
+    attr.run([&] { (void)hipFuncSetAttribute((const void*)gemm_rows_kernel<BM, ST, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+    hipLaunchKernelGGL((gemm_rows_kernel<BM, ST, EPI>), dim3((unsigned)(a.N / RBN * a.ksplit)), dim3(256), lds, s, a);
+}
+template <int BM, int ST>
+void go_epi(const GemmArgs& a, int epi, hipStream_t s) {
+    if (a.ksplit > 1) go<BM, ST, GEPI_PARTIAL>(a, s);
+    else if (epi == GEPI_STORE) go<BM, ST, GEPI_STORE>(a, s);
+    else if (epi == GEPI_RESADD) go<BM, ST, GEPI_RESADD>(a, s);
+    else go<BM, ST, GEPI_SILUMUL>(a, s);
+}
+
+}  // namespace
+
+// Where the lines lie (both sides measured, old kernels / these, us): more than one round of workgroups pays only while the last round is well
+// filled -- 272 tiles (34816 x 5120, 64 rows) 98 / 124, 1187 tiles 391 / 290; above 64 rows a launch is bound by its MFMAs as much as by the
+// weights, and wide projections stay with the wider tiles -- 192 tiles at 128 rows 62 / 78, 1187 tiles 405 / 405, while 32 .. 48 tiles split 4
+// ways 46 / 40 and 28 / 27.  A slice of K keeps at least four k-tiles: the pipeline's fill costs two or three.
+int gemm_rows_split(int M, int N, int K, size_t ws_floats) {
+    if (M < 9 || M > 128 || N % RBN != 0 || K % RBK != 0) return 0;
+    const int tiles = N / RBN, nk = K / RBK, rounds = (tiles + 255) / 256;
+    if (tiles > 256 && tiles * 10 < rounds * 256 * 9) return 0;
+    if (M > 64 && tiles > 128) return 0;
+    int ks = 1;
+    while (ks < 8 && 2 * ks * tiles <= 256 && nk % (2 * ks) == 0 && nk / (2 * ks) >= 4 && (size_t)2 * ks * M * N <= ws_floats) ks *= 2;
+    return ks;
+}
+
+// a.ksplit set by the caller (1: epilogue `epi`; > 1: partial tiles, the caller runs the reduction)
+bool launch_gemm_rows(const GemmArgs& a, int epi, hipStream_t s) {
+    if (a.M > 128 || a.A_lo == nullptr || a.N % RBN != 0 || a.K % (RBK * a.ksplit) != 0 || epi == GEPI_ACT_SPLIT) return false;
+    if (a.M <= 32) go_epi<32, 4>(a, epi, s);
+    else if (a.M <= 64) go_epi<64, 3>(a, epi, s);
+    else go_epi<128, 3>(a, epi, s);
+    return true;
+}
+
+}  // namespace cm

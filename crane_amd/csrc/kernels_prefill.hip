@@ -1334,6 +1334,16 @@ static bool norm_fused(const GemmArgs& a) {
     return env != 0 && a.norm_w != nullptr && a.ldc == a.N && a.N % 4 == 0;
 }
 
+// the reduction behind a launch that left partial tiles of a.ksplit K slices
+static void launch_splitk(GemmArgs& a, int epi, hipStream_t s) {
+    const int eb = (int)std::min<size_t>(((size_t)a.M * (a.N / 4) + 255) / 256, 2048);
+    if (epi == GEPI_STORE) launch_splitk_epilogue<GEPI_STORE>(a, eb, s);
+    else if (epi == GEPI_RESADD && norm_fused(a)) { launch_splitk_resadd_norm(a, s); a.norm_w = nullptr; }
+    else if (epi == GEPI_RESADD) launch_splitk_epilogue<GEPI_RESADD>(a, eb, s);
+    else if (epi == GEPI_ACT_SPLIT) launch_splitk_epilogue<GEPI_ACT_SPLIT>(a, eb, s);
+    else launch_splitk_epilogue<GEPI_SILUMUL>(a, eb, s);
+}
+
 // Large M (>= 512 rows): the LDS-DMA kernel on full cache lines (kernels_gemm256.hip; 128-row tiles with hi + lo activations,
 // 256-row tiles with plain bf16) where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost
 // model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
@@ -1347,7 +1357,7 @@ static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
     // than the 64-row one (the launch is not bound by its MFMAs), 8 rows run on the batched GEMVs
     static const int min_m2 = getenv("CM_GEMM256_MIN_M") ? atoi(getenv("CM_GEMM256_MIN_M")) : 9;
     static const int min_blocks = getenv("CM_GEMM256_MIN_BLOCKS") ? atoi(getenv("CM_GEMM256_MIN_BLOCKS")) : 128;
-    if (!env || !a.wide256 || a.M < (a.A_lo ? min_m2 : 512) || a.K % 64 != 0) return false;
+    if (!env || !a.wide256 || a.wide256 == 4 || a.M < (a.A_lo ? min_m2 : 512) || a.K % 64 != 0) return false;
     // round 6: the one-wave-per-SIMD kernel (kernels_gemmw4.hip) -- built, bit-compatible, measured 0 .. 4 % SLOWER than the ping-pong kernel
     // on every prompt shape, so it is opt-in: CM_GEMMW4 = 1 from `w4_min` rows on, GemmArgs::wide256 = 2 (cm_debug_set "gemm256" = 2) always
     static const int w4_env = getenv("CM_GEMMW4") ? atoi(getenv("CM_GEMMW4")) : 0;
@@ -1382,14 +1392,7 @@ static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
     a.ksplit = best_ks;
     if (w4) { if (!launch_gemmw4(a, epi, best_bn, s)) return false; }
     else if (!launch_gemm256(a, epi, best_bn, s)) return false;
-    if (best_ks > 1) {
-        const int eb = (int)std::min<size_t>(((size_t)a.M * (a.N / 4) + 255) / 256, 2048);
-        if (epi == GEPI_STORE) launch_splitk_epilogue<GEPI_STORE>(a, eb, s);
-        else if (epi == GEPI_RESADD && norm_fused(a)) { launch_splitk_resadd_norm(a, s); a.norm_w = nullptr; }
-        else if (epi == GEPI_RESADD) launch_splitk_epilogue<GEPI_RESADD>(a, eb, s);
-        else if (epi == GEPI_ACT_SPLIT) launch_splitk_epilogue<GEPI_ACT_SPLIT>(a, eb, s);
-        else launch_splitk_epilogue<GEPI_SILUMUL>(a, eb, s);
-    }
+    if (best_ks > 1) launch_splitk(a, epi, s);
     return true;
 }
 
@@ -1435,8 +1438,20 @@ bool launch_gemm(const GemmArgs& a0, int epi, hipStream_t s) {
     }
     return true;
 }
+
+// 9 .. 128 rows: the tiles of kernels_gemm_rows.hip where its rule takes the sizes
+static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
+    static const int env = getenv("CM_GEMM256") ? atoi(getenv("CM_GEMM256")) : 1;
+    if (!env || (a.wide256 != 1 && a.wide256 != 4) || a.A_lo == nullptr || epi == GEPI_ACT_SPLIT) return false;
+    const int ks = gemm_rows_split(a.M, a.N, a.K, a.ws ? a.ws_floats : 0);
+    if (ks == 0) return false;
+    a.ksplit = ks;
+    if (!launch_gemm_rows(a, epi, s)) return false;
+    if (ks > 1) launch_splitk(a, epi, s);
+    return true;
+}
 static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
-    if (try_gemm256(a, epi, s)) return true;
+    if (try_gemm_rows(a, epi, s) || try_gemm256(a, epi, s)) return true;
     const int tiles_m = (a.M + GBM - 1) / GBM;
     const bool split = a.A_lo != nullptr;
     // 256-wide tiles (one 8-wave block per CU) when they give every CU at least two blocks (1024-token gate||up: 428 -> ~370 us;
@@ -1469,12 +1484,7 @@ static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
         } else
         if (split) hipLaunchKernelGGL((gemm_bf16_kernel<2, GEPI_PARTIAL, 128>), dim3(tiles * a.ksplit), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((gemm_bf16_kernel<1, GEPI_PARTIAL, 128>), dim3(tiles * a.ksplit), dim3(256), 0, s, a);
-        const int eb = (int)std::min<size_t>(((size_t)a.M * (a.N / 4) + 255) / 256, 2048);
-        if (epi == GEPI_STORE) launch_splitk_epilogue<GEPI_STORE>(a, eb, s);
-        else if (epi == GEPI_RESADD && norm_fused(a)) { launch_splitk_resadd_norm(a, s); a.norm_w = nullptr; }
-        else if (epi == GEPI_RESADD) launch_splitk_epilogue<GEPI_RESADD>(a, eb, s);
-        else if (epi == GEPI_ACT_SPLIT) launch_splitk_epilogue<GEPI_ACT_SPLIT>(a, eb, s);
-        else launch_splitk_epilogue<GEPI_SILUMUL>(a, eb, s);
+        launch_splitk(a, epi, s);
         return true;
     }
 #define CM_GEMM(SP, EP) hipLaunchKernelGGL((gemm_bf16_kernel<SP, EP, 128>), dim3(tiles), dim3(256), 0, s, a)

@@ -1683,10 +1683,11 @@ void Model::lm_head_rows(int nb, bool want_rows) {
         // Large groups: the head as ONE MFMA GEMM over the rows of the group (final RMSNorm rows as bf16 hi + lo, like the
         // projections of the step) + a row arg-max over the logits it wrote.  The matrix-core GEMV is issue-bound from ~17 rows
         // on: 1.25 ms per 64-row pass over the 1.24 GB table at Qwen3-8B -- two passes for 128 sequences were 2.5 ms of a 14 ms
-        // round; the GEMM streams the table once.
+        // round; the GEMM streams the table once: 277 us at 32 rows, 290 at 64 (kernels_gemm_rows.hip; 385 / 391 with the 128 x 128 tiles,
+        // which keep the larger groups: 405 on both).
         launch_rmsnorm_rows(xb, norm, pXN_hi, pXN_lo, nb, H, cfg.eps, s);
         GemmArgs g{};
-        g.ws = pWS; g.ws_floats = gemm_ws_floats; g.wide256 = 0;
+        g.ws = pWS; g.ws_floats = gemm_ws_floats; g.wide256 = gemm256 == 1 ? 4 : 0;
         g.A_hi = pXN_hi; g.A_lo = pXN_lo; g.W = lm_head; g.C = logitsb + (size_t)rank * V_l; g.ldc = cfg.V; g.M = nb; g.N = v_eff; g.K = H;
         if (!launch_gemm(g, GEPI_STORE, s)) throw CmError(CM_ERR_UNSUPPORTED, "gemm shape");
         lmg = std::min(lm_gridb, 64);
