@@ -195,22 +195,17 @@ struct AttnPreArgs {
     const int32_t* block_table;
     const void* kpool;
     const void* vpool;
-    size_t kv_lo_off = 0;        // KV_BF16X2: element offset of the lo halves behind the hi halves in kpool / vpool
     uint16_t* out_hi;            // [Spad, Hq * D] bf16 hi (+lo) -> A operand of the o_proj GEMM
     uint16_t* out_lo;
     float* out_f32 = nullptr;    // causal kernels: write f32 rows [S, Hq * D] here INSTEAD of the bf16 planes (int8 prompt pass: the o_proj quantiser's input)
     const float* gate;           // [S, gate_stride] f32 (Qwen3.5 output gate) or null
     int gate_stride;
     int S, Hq, Hkv, nrep, page, start_pos;
-    int causal, kv_lo, kv_hi;    // causal = 0: bidirectional over tokens [kv_lo, kv_hi) (ViT frame)
     // several sequences in one causal launch: tiles[i] = {segment, query tile} ordered by ASCENDING key-tile count (walked from the
     // back: longest first); q / out / gate / block_table above are those of the whole pass
     const PrefillSegDev* segs = nullptr;
     const int2* tiles = nullptr;
     int ntiles = 0;
-    int ksplit = 1;              // bidirectional frames only: runs of key tiles per query tile (partials merged by a second kernel)
-    float* part_o = nullptr;     // [ksplit][S][Hq][D] un-normalised partial outputs
-    float* part_ml = nullptr;    // [ksplit][S][Hq][2] running max, running sum
 };
 
 void launch_embed_rows(const uint16_t* emb, const uint32_t* ids, float* x, int S, int H, int V, hipStream_t s);
@@ -229,7 +224,19 @@ int gemmw4_rows(bool split);               // rows of the one-wave-per-SIMD kern
 bool launch_gemmw4(const GemmArgs& a, int epi, int bn, hipStream_t s);    // same contract as launch_gemm256
 void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s);   // kvt: KV_BF16 | KV_F16 | KV_F32 (what the kernel reads)
 
-// ---- vision tower (kernels_vision.hip) ----
+// ---- vision tower (kernels_vision.hip, kernels_vision_attn.hip) ----
+// attention inside the frames of a pass of `rows` patches, head_dim 64: q / out [rows][heads][64], k / v [64 rows][heads][row][64] with the lo halves
+// `lo_off` elements behind the hi halves; tiles[i] = {first row, end row of the frame, first query row, 0}: 64 query rows each, 128 when `wide`
+struct VitAttnArgs {
+    const uint16_t *q_hi, *q_lo, *k, *v;
+    size_t lo_off;
+    uint16_t *out_hi, *out_lo;
+    const int4* tiles;
+    int ntiles, wide, heads, rows;
+    int runs;                    // of key tiles; more than one: partials part_o [runs][rows][heads][64], part_ml [..][2] and a merge launch
+    float *part_o, *part_ml;
+};
+void launch_vit_attn(const VitAttnArgs& a, hipStream_t s);
 void launch_layernorm_rows(const float* x, const float* w, const float* b, uint16_t* hi, uint16_t* lo, int N, int H, float eps,
                            hipStream_t s);
 void launch_pos_embed_add(float* x, const uint16_t* table, const int32_t* idx, const float* wts, int N, int H, hipStream_t s);

@@ -497,8 +497,7 @@ __global__ __launch_bounds__(BN * 2) void gemm_bf16_kernel(GemmArgs a) {
 // ---------------------------------------------------------------------------------------------
 // V tile row stride in LDS = D + 16 elements: the 4 key rows of a tr-read group land on disjoint banks
 // KVT: KV_BF16 pages (K rows / V^T fragments feed the bf16 MFMAs as cached), KV_F16 pages (the same on the f16 MFMAs; q_hi / q_lo
-// and P are then f16 hi + lo), KV_F32 (f32 rows split into bf16 hi + lo on load: the ViT scratch, f32 pages, the int8 / int4 shadow)
-// KV_BF16X2 (the ViT scratch): K/V rows arrive pre-split into bf16 hi + lo arrays -- the three-product arithmetic of KV_F32
+// and P are then f16 hi + lo), KV_F32 (f32 rows split into bf16 hi + lo on load: f32 pages, the int8 / int4 shadow)
 // without a conversion in the loop.
 // e^x for x <= 0 (softmax numerators after the running max): v_exp_f32 (2^x, 1 ulp) on x * log2(e) -- two instructions where
 // expf()'s range reduction and polynomial are ~20; 17 of them per lane and key tile were a quarter of the tile's VALU work
@@ -520,17 +519,16 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
         if (a.gate != nullptr) a.gate += (size_t)sg.row0 * a.gate_stride;
         qt_seg = tq.y;
     }
-    constexpr bool KVF32 = KVT == KV_F32, X2 = KVT == KV_BF16X2, THREE = KVF32 || X2;
+    constexpr bool THREE = KVT == KV_F32;
     constexpr int KT = 64, VLD = D + 16, NKS = D / 32, NNT = D / 16;
     __shared__ __attribute__((aligned(16))) uint16_t Vs[THREE ? 2 : 1][KT * VLD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sub = lane & 15, g = lane >> 4;
-    // causal: grid (Hq, query tiles) walked LONGEST TILE FIRST (a query tile of index i attends i + 1 key tiles): at 2048 rows the
+    // grid (Hq, query tiles) walked LONGEST TILE FIRST (a query tile of index i attends i + 1 key tiles): at 2048 rows the
     // 1024 workgroups do not fit at once, and in ascending order the last ones dispatched are the longest -- the launch ended
     // with a tail of up to 32 tile times; descending, a slot that finishes a long tile picks up a short one (LPT).
-    // bidirectional frames: grid (query tiles, Hq, key runs)
-    const int h = a.causal ? blockIdx.x : blockIdx.y, kvh = h / a.nrep;
-    const int qb = (qt_seg >= 0 ? qt_seg : a.causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.x) * 64;      // first query row of this block
+    const int h = blockIdx.x, kvh = h / a.nrep;
+    const int qb = (qt_seg >= 0 ? qt_seg : (int)(gridDim.y - 1 - blockIdx.y)) * 64;      // first query row of this block
     const int qrow = qb + wave * 16 + sub;          // this lane's query row (as Q^T column / stats owner)
     const int qrow_c = qrow < a.S ? qrow : a.S - 1; // clamp for loads
     const int qpos = a.start_pos + qrow;
@@ -549,18 +547,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
     float m_run = -INFINITY, l_run = 0.f;
 
     const int last_q = min(qb + 63, a.S - 1);
-    // causal: tokens [0, start_pos + last_q] ; window (ViT frame): tokens [kv_lo, kv_hi), bidirectional
-    const int kv_end = a.causal ? a.start_pos + last_q + 1 : a.kv_hi;
-    // bidirectional frames (ViT): blockIdx.z takes one of a.ksplit contiguous runs of key tiles and leaves an un-normalised
-    // partial (o, m, l) for attn_prefill_merge_kernel -- 13 x 16 blocks of 4 waves are one wave per SIMD on 208 of 256 CUs, each
-    // walking 13 tiles of VALU-bound softmax serially; four runs per query tile put 3 waves on every SIMD
-    int t_begin = a.causal ? 0 : a.kv_lo, t_end = kv_end;
-    if (a.ksplit > 1) {
-        const int ntile = (kv_end - t_begin + KT - 1) / KT, per = (ntile + a.ksplit - 1) / a.ksplit;
-        t_begin += (int)blockIdx.z * per * KT;
-        t_end = min(kv_end, t_begin + per * KT);
-    }
-    for (int t0 = t_begin; t0 < t_end; t0 += KT) {
+    const int kv_end = a.start_pos + last_q + 1;    // tokens [0, start_pos + last_q]
+    for (int t0 = 0; t0 < kv_end; t0 += KT) {
         __syncthreads();                                   // previous tile's V fully consumed
         // ---- stage V tile (64 tokens x D dims) into LDS, shared by the 4 waves ----
 #pragma unroll
@@ -569,7 +557,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
             const int t = min(t0 + tok, kv_end - 1);
             const int page = a.block_table[t / a.page];
             const size_t off = ((size_t)(page * a.Hkv + kvh) * a.page + (t % a.page)) * D + d8;
-            if (KVF32) {
+            if (THREE) {
                 const f32x4 v0 = *(const f32x4*)((const float*)a.vpool + off);
                 const f32x4 v1 = *(const f32x4*)((const float*)a.vpool + off + 4);
                 const float vv[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
@@ -582,9 +570,6 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
                 }
                 *(u32x4*)&Vs[0][tok * VLD + d8] = (u32x4){hi[0], hi[1], hi[2], hi[3]};
                 *(u32x4*)&Vs[THREE ? 1 : 0][tok * VLD + d8] = (u32x4){lo[0], lo[1], lo[2], lo[3]};
-            } else if (X2) {
-                *(u32x4*)&Vs[0][tok * VLD + d8] = ld16((const uint16_t*)a.vpool + off);
-                *(u32x4*)&Vs[THREE ? 1 : 0][tok * VLD + d8] = ld16((const uint16_t*)a.vpool + a.kv_lo_off + off);
             } else {
                 *(u32x4*)&Vs[0][tok * VLD + d8] = ld16((const uint16_t*)a.vpool + off);
             }
@@ -600,7 +585,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
                 bf16x8 kh, kl;
-                if (KVF32) {
+                if (THREE) {
                     const f32x4 k0 = *(const f32x4*)((const float*)a.kpool + kb + ks * 32);
                     const f32x4 k1 = *(const f32x4*)((const float*)a.kpool + kb + ks * 32 + 4);
                     const float kk[8] = {k0[0], k0[1], k0[2], k0[3], k1[0], k1[1], k1[2], k1[3]};
@@ -612,7 +597,6 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
                     }
                 } else {
                     kh = *(const bf16x8*)((const uint16_t*)a.kpool + kb + ks * 32);
-                    if (X2) kl = *(const bf16x8*)((const uint16_t*)a.kpool + a.kv_lo_off + kb + ks * 32);
                 }
                 s[tt] = mma_k32<KVT>(kh, qh[ks], s[tt]);
                 s[tt] = mma_k32<KVT>(kh, ql[ks], s[tt]);
@@ -626,7 +610,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int t = t0 + tt * 16 + g * 4 + r;
-                if (a.causal ? (t > qpos) : (t >= kv_end)) s[tt][r] = -INFINITY;
+                if (t > qpos) s[tt][r] = -INFINITY;
                 mt = fmaxf(mt, s[tt][r]);
             }
         mt = fmaxf(mt, __shfl_xor(mt, 16));
@@ -670,15 +654,6 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
     // ---- finalize: l over the 4 lane groups; O^T rows = dims nt*16 + g*4 + r, col = query `sub` ----
     l_run += __shfl_xor(l_run, 16);
     l_run += __shfl_xor(l_run, 32);
-    if (a.ksplit > 1) {
-        if (qrow < a.S) {
-            const size_t row = ((size_t)blockIdx.z * a.S + qrow) * a.Hq + h;
-#pragma unroll
-            for (int nt = 0; nt < NNT; ++nt) *(f32x4*)(a.part_o + row * D + nt * 16 + g * 4) = o[nt];
-            if (g == 0) { a.part_ml[row * 2] = m_run; a.part_ml[row * 2 + 1] = l_run; }
-        }
-        return;
-    }
     const float inv = 1.0f / l_run;
     if (qrow < a.S) {
 #pragma unroll
@@ -920,187 +895,6 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
             split_store4(a.out_hi, a.out_lo, ((size_t)qrow * a.Hq + h) * D + nt * 16 + g * 4, v);
         }
     }
-}
-
-// ---------------------------------------------------------------------------------------------
-// The same staging for the vision tower's frames (round 5): bidirectional attention inside a frame, head_dim 64, K / V scratch
-// pre-split into bf16 hi + lo planes (KV_BF16X2: s = kh.qh + kh.ql + kl.qh, o += vh.ph + vh.pl + vl.ph -- the general kernel's
-// three-product arithmetic), key runs over blockIdx.z with un-normalised partials for attn_prefill_merge_kernel.  Frames that
-// start on a 64-token boundary (every still image; page = 64): a key tile is one page.  All four planes of a tile go through LDS
-// once per workgroup, double-buffered, requested two tiles ahead.
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void attn_window_fast_kernel(AttnPreArgs a) {
-    constexpr int D = 64, KT = 64, KLD = D + 8, VLD = D + 16, NKS = D / 32, NNT = D / 16, NTT = KT / 16, CPR = D / 8, RPP = 256 / CPR;
-    constexpr float L2E = 1.4426950408889634f;
-    __shared__ __attribute__((aligned(16))) uint16_t Kh[2][KT * KLD], Kl[2][KT * KLD];
-    __shared__ __attribute__((aligned(16))) uint16_t Vh[2][KT * VLD], Vl[2][KT * VLD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int sub = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, kvh = h / a.nrep;
-    const int qb = (int)blockIdx.x * 64;
-    const int qrow = qb + wave * 16 + sub;
-    const int qrow_c = qrow < a.S ? qrow : a.S - 1;
-    bf16x8 qh[NKS], ql[NKS];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-        const size_t off = ((size_t)qrow_c * a.Hq + h) * D + ks * 32 + g * 8;
-        qh[ks] = *(const bf16x8*)(a.q_hi + off);
-        ql[ks] = *(const bf16x8*)(a.q_lo + off);
-    }
-    f32x4 o[NNT];
-#pragma unroll
-    for (int nt = 0; nt < NNT; ++nt) o[nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
-    const int kv_lo = a.kv_lo, kv_end = a.kv_hi;
-    const int ntile_all = (kv_end - kv_lo + KT - 1) / KT, nfull_all = (kv_end - kv_lo) / KT;
-    const int per = (ntile_all + a.ksplit - 1) / a.ksplit;
-    const int ti0 = (int)blockIdx.z * per, ti1 = min(ntile_all, ti0 + per);     // this workgroup's run of key tiles
-    const uint16_t* kpool = (const uint16_t*)a.kpool;
-    const uint16_t* vpool = (const uint16_t*)a.vpool;
-    const size_t lo_off = a.kv_lo_off;
-    const int pg0 = kv_lo / a.page, pglast = (kv_end - 1) / a.page;
-    int pgs_grp = ti0 >> 6;
-    int pgs = a.block_table[min(pg0 + pgs_grp * 64 + lane, pglast)];           // page ids of tiles 64 grp + lane of the frame (page = key tile)
-    auto tile_base = [&](int ti) __attribute__((always_inline)) -> size_t {
-        if ((ti >> 6) != pgs_grp) { pgs_grp = ti >> 6; pgs = a.block_table[min(pg0 + pgs_grp * 64 + lane, pglast)]; }
-        const int pg = __builtin_amdgcn_readlane(pgs, ti & 63);
-        return (size_t)(pg * a.Hkv + kvh) * a.page * D;
-    };
-    const int vtok = tid / CPR, vd8 = (tid % CPR) * 8;
-    struct KvRegs { u32x4 kh[2], kl[2], vh[2], vl[2]; };
-    auto kv_fetch = [&](int ti, KvRegs& rg) __attribute__((always_inline)) {
-        const int tf = min(ti, ntile_all - 1);               // (past the frame: its last tile again, parked into buffers nobody reads)
-        const size_t b = tile_base(tf);
-        const int t0 = kv_lo + tf * KT;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int tok = min(vtok + RPP * i, kv_end - 1 - t0);
-            const size_t off = b + (size_t)tok * D + vd8;
-            rg.kh[i] = ld16(kpool + off); rg.kl[i] = ld16(kpool + lo_off + off);
-            rg.vh[i] = ld16(vpool + off); rg.vl[i] = ld16(vpool + lo_off + off);
-        }
-    };
-    auto kv_park = [&](int buf, const KvRegs& rg) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            *(u32x4*)&Kh[buf][(vtok + RPP * i) * KLD + vd8] = rg.kh[i];
-            *(u32x4*)&Kl[buf][(vtok + RPP * i) * KLD + vd8] = rg.kl[i];
-            *(u32x4*)&Vh[buf][(vtok + RPP * i) * VLD + vd8] = rg.vh[i];
-            *(u32x4*)&Vl[buf][(vtok + RPP * i) * VLD + vd8] = rg.vl[i];
-        }
-    };
-    auto tile = [&](int ti, int buf, auto masked_c, KvRegs& rg_new, const KvRegs& rg_next) __attribute__((always_inline)) {
-        constexpr bool MASKED = decltype(masked_c)::value;
-        const int t0 = kv_lo + ti * KT;
-        kv_fetch(ti + 2, rg_new);
-        f32x4 s[NTT];
-#pragma unroll
-        for (int tt = 0; tt < NTT; ++tt) {
-            s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const bf16x8 kh = *(const bf16x8*)&Kh[buf][(tt * 16 + sub) * KLD + ks * 32 + g * 8];
-                const bf16x8 kl = *(const bf16x8*)&Kl[buf][(tt * 16 + sub) * KLD + ks * 32 + g * 8];
-                s[tt] = mma_k32<KV_BF16X2>(kh, qh[ks], s[tt]);
-                s[tt] = mma_k32<KV_BF16X2>(kh, ql[ks], s[tt]);
-                s[tt] = mma_k32<KV_BF16X2>(kl, qh[ks], s[tt]);
-            }
-        }
-        float mt = -INFINITY;
-#pragma unroll
-        for (int tt = 0; tt < NTT; ++tt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (MASKED) { if (t0 + tt * 16 + g * 4 + r >= kv_end) s[tt][r] = -INFINITY; }
-                mt = fmaxf(mt, s[tt][r]);
-            }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float m_new = fmaxf(m_run, mt);               // finite: every tile holds at least one token of the frame
-        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * L2E);
-        const float nm = -m_new * L2E;
-        float psum = 0.f;
-        bf16x4 ph[NTT], pl[NTT];
-#pragma unroll
-        for (int tt = 0; tt < NTT; ++tt) {
-            float p[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { p[r] = __builtin_amdgcn_exp2f(fmaf(s[tt][r], L2E, nm)); psum += p[r]; }
-            p_split4<KV_BF16X2>(p, ph[tt], pl[tt]);
-        }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-#pragma unroll
-        for (int nt = 0; nt < NNT; ++nt) { o[nt][0] *= alpha; o[nt][1] *= alpha; o[nt][2] *= alpha; o[nt][3] *= alpha; }
-#pragma unroll
-        for (int tt = 0; tt < NTT; ++tt) {
-#pragma unroll
-            for (int nt = 0; nt < NNT; ++nt) {
-                const int vo = (tt * 16 + g * 4 + (sub >> 2)) * VLD + nt * 16 + (sub & 3) * 4;
-                const bf16x4 vh = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)&Vh[buf][vo]);
-                const bf16x4 vl = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)&Vl[buf][vo]);
-                o[nt] = mma_k16<KV_BF16X2>(vh, ph[tt], o[nt]);
-                o[nt] = mma_k16<KV_BF16X2>(vh, pl[tt], o[nt]);
-                o[nt] = mma_k16<KV_BF16X2>(vl, ph[tt], o[nt]);
-            }
-        }
-        kv_park(buf ^ 1, rg_next);
-        lds_wg_barrier();
-    };
-    KvRegs rA, rB;
-    kv_fetch(ti0, rA);
-    kv_fetch(ti0 + 1, rB);
-    kv_park(0, rA);
-    __syncthreads();
-    for (int ti = ti0; ti < ti1; ti += 2) {
-        if (ti < nfull_all) tile(ti, 0, std::false_type{}, rA, rB); else tile(ti, 0, std::true_type{}, rA, rB);
-        if (ti + 1 < ti1) { if (ti + 1 < nfull_all) tile(ti + 1, 1, std::false_type{}, rB, rA); else tile(ti + 1, 1, std::true_type{}, rB, rA); }
-    }
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
-    if (a.ksplit > 1) {
-        if (qrow < a.S) {
-            const size_t row = ((size_t)blockIdx.z * a.S + qrow) * a.Hq + h;
-#pragma unroll
-            for (int nt = 0; nt < NNT; ++nt) *(f32x4*)(a.part_o + row * D + nt * 16 + g * 4) = o[nt];
-            if (g == 0) { a.part_ml[row * 2] = m_run; a.part_ml[row * 2 + 1] = l_run; }
-        }
-        return;
-    }
-    const float inv = 1.0f / l_run;
-    if (qrow < a.S) {
-#pragma unroll
-        for (int nt = 0; nt < NNT; ++nt) {
-            const float v[4] = {o[nt][0] * inv, o[nt][1] * inv, o[nt][2] * inv, o[nt][3] * inv};
-            split_store4(a.out_hi, a.out_lo, ((size_t)qrow * a.Hq + h) * D + nt * 16 + g * 4, v);
-        }
-    }
-}
-
-// merge of the ksplit partials of attn_prefill_kernel: out = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z, stored as bf16 hi + lo
-// (the A operand of the projection GEMM).  One thread per (query row, head, 4 dims).
-template <int D>
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnPreArgs a) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t n4 = (size_t)a.S * a.Hq * (D / 4);
-    if (i >= n4) return;
-    const size_t row = i / (D / 4);                       // qrow * Hq + h
-    const int d4 = (int)(i % (D / 4)) * 4;
-    const size_t zs = (size_t)a.S * a.Hq;
-    float M = -INFINITY;
-    for (int z = 0; z < a.ksplit; ++z) M = fmaxf(M, a.part_ml[(z * zs + row) * 2]);
-    float L = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < a.ksplit; ++z) {
-        const float mz = a.part_ml[(z * zs + row) * 2];
-        const float w = mz > -INFINITY ? expf(mz - M) : 0.f;
-        L += w * a.part_ml[(z * zs + row) * 2 + 1];
-        const f32x4 p = *(const f32x4*)(a.part_o + (z * zs + row) * D + d4);
-        acc[0] += w * p[0]; acc[1] += w * p[1]; acc[2] += w * p[2]; acc[3] += w * p[3];
-    }
-    const float inv = 1.0f / L;
-    float v[4] = {acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-    split_store4(a.out_hi, a.out_lo, row * D + d4, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1498,26 +1292,13 @@ static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
 #undef CM_GEMM
     return true;
 }
-// kvt: KV_BF16 | KV_F16 | KV_F32 (the element type the kernel READS: f32 for the ViT scratch and the int8 / int4 shadow)
-void launch_attn_prefill(const AttnPreArgs& a0, int D, int kvt, hipStream_t s) {
-    AttnPreArgs a = a0;
-    if (a.causal || a.part_o == nullptr || a.part_ml == nullptr || a.gate != nullptr || a.ksplit < 1) a.ksplit = 1;
-    dim3 grid((a.S + 63) / 64, a.Hq, a.ksplit);
-    if (a.causal) grid = dim3(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64, 1);
-    if (D == 64) {
-        static const int fastw_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
-        if (fastw_env != 0 && !a.causal && a.gate == nullptr && a.page == 64 && a.kv_lo % 64 == 0 && a.q_lo != nullptr && kvt == KV_BF16X2)
-            hipLaunchKernelGGL(attn_window_fast_kernel, grid, dim3(256), 0, s, a);
-        else
-        hipLaunchKernelGGL((attn_prefill_kernel<64, KV_BF16X2>), grid, dim3(256), 0, s, a);     // ViT: K/V scratch pre-split into bf16 hi + lo
-        if (a.ksplit > 1) {
-            const size_t n4 = (size_t)a.S * a.Hq * (64 / 4);
-            hipLaunchKernelGGL((attn_prefill_merge_kernel<64>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, a);
-        }
-    } else if (D == 128) {
+// kvt: KV_BF16 | KV_F16 | KV_F32 (the element type the kernel READS: f32 for the int8 / int4 shadow)
+void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
+    const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64);
+    if (D == 128) {
         // the dense family's causal prompts over 2-byte pages: the fast path (CM_ATTN_PREFILL_FAST=0: the general kernel, A/B)
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
-        if (fast_env != 0 && a.causal && a.gate == nullptr && a.ksplit == 1 && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 &&
+        if (fast_env != 0 && a.gate == nullptr && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 &&
             a.q_lo != nullptr) {
             if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<128, 64, KV_F16>), grid, dim3(256), 0, s, a);
             else hipLaunchKernelGGL((attn_prefill_fast_kernel<128, 64, KV_BF16>), grid, dim3(256), 0, s, a);
@@ -1529,7 +1310,7 @@ void launch_attn_prefill(const AttnPreArgs& a0, int D, int kvt, hipStream_t s) {
     } else {
         // the hybrid family's gated head_dim-256 attention: the same fast path on 32-token key tiles
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
-        if (fast_env != 0 && a.causal && a.ksplit == 1 && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 && a.q_lo != nullptr) {
+        if (fast_env != 0 && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 && a.q_lo != nullptr) {
             if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<256, 32, KV_F16>), grid, dim3(256), 0, s, a);
             else hipLaunchKernelGGL((attn_prefill_fast_kernel<256, 32, KV_BF16>), grid, dim3(256), 0, s, a);
             return;

@@ -1,6 +1,6 @@
 // Vision-tower (Qwen 3.5-VL ViT) row kernels; the projections reuse the MFMA GEMM of
-// kernels_prefill.hip (bias / GELU epilogues) and the bidirectional per-frame attention reuses
-// attn_prefill_kernel<64> in window mode.  Reference: crane-core/src/models/qwen3_5/vision.rs.
+// kernels_prefill.hip (bias / GELU epilogues) and the bidirectional per-frame attention is in
+// kernels_vision_attn.hip.  Reference: crane-core/src/models/qwen3_5/vision.rs.
 #include <cstdlib>
 
 #include "dev_common.h"

@@ -1410,7 +1410,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             at.kpool = kpool(li); at.vpool = vpool(li);
             at.out_hi = pAT_hi; at.out_lo = pAT_lo;
             at.S = S; at.Hq = Hq_l; at.Hkv = Hkv_l; at.nrep = nrep;
-            at.page = page; at.start_pos = 0; at.causal = 1;
+            at.page = page; at.start_pos = 0;
             at.gate = cfg.hybrid ? pQKV + (size_t)Hq_l * D : nullptr; at.gate_stride = qkv_rows;
             at.segs = d_segtab; at.tiles = d_tiles; at.ntiles = seg_ntiles;
             if (q8p) at.out_f32 = pATf;
@@ -1441,7 +1441,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
         at.kpool = kvq ? (void*)kshadow : kpool(li); at.vpool = kvq ? (void*)vshadow : vpool(li);
         at.out_hi = pAT_hi + (size_t)sg.row0 * Hq_l * D; at.out_lo = pAT_lo + (size_t)sg.row0 * Hq_l * D;
         at.S = sg.S; at.Hq = Hq_l; at.Hkv = Hkv_l; at.nrep = nrep;
-        at.page = page; at.start_pos = sp; at.causal = 1;
+        at.page = page; at.start_pos = sp;
         at.gate = cfg.hybrid ? pQKV + (size_t)sg.row0 * qkv_rows + (size_t)Hq_l * D : nullptr; at.gate_stride = qkv_rows;
         if (q8p) at.out_f32 = pATf + (size_t)sg.row0 * Hq_l * D;
         launch_attn_prefill(at, D, (kv_f32 || kvq) ? KV_F32 : kv_mode, s);

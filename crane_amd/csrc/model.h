@@ -184,8 +184,9 @@ struct Model {
     bool v_timed = false;
     float *vPartO = nullptr, *vPartML = nullptr;   // split-KV partials of the frame attention (VIT_KSPLIT runs of key tiles)
     int vit_ksplit = 2;                             // CM_VIT_KSPLIT
+    int4* vTiles = nullptr;                         // (frame, query rows) of every workgroup of the frame attention
     uint16_t *vA_hi = nullptr, *vA_lo = nullptr, *vB_hi = nullptr, *vB_lo = nullptr, *vQ_hi = nullptr, *vQ_lo = nullptr;
-    int32_t *vIdx = nullptr, *vBt = nullptr, *dMap = nullptr, *dPos3 = nullptr;
+    int32_t *vIdx = nullptr, *dMap = nullptr, *dPos3 = nullptr;
     const int32_t* pos3_dev = nullptr;   // set only while a VLM prefill runs
     const int32_t* splice_map_dev = nullptr;
     float* vDeep = nullptr;              // [n_deepstack][v_cap / merge^2 + 1][out_hidden] DeepStack feature maps of the last encode

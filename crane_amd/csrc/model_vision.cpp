@@ -33,7 +33,7 @@ void Model::ensure_vision_buffers(int n_patches) {
     vV = dalloc<uint16_t>(2 * vkv_lo_off);
     vW4 = dalloc<float>((size_t)4 * cap);
     vIdx = dalloc<int>((size_t)4 * cap);
-    vBt = dalloc<int>(pages);
+    vTiles = (int4*)dalloc<int>((size_t)cap * 4);                                    // (a frame has at least one row per tile)
     if (const char* e = getenv("CM_VIT_KSPLIT")) vit_ksplit = std::max(1, std::min(8, atoi(e)));
     if (vit_ksplit > 1) {
         vPartO = dalloc<float>((size_t)vit_ksplit * cap * VH);
@@ -43,9 +43,6 @@ void Model::ensure_vision_buffers(int n_patches) {
     vA_hi = z((size_t)pad * wide); vA_lo = z((size_t)pad * wide);
     vB_hi = z((size_t)pad * wide); vB_lo = z((size_t)pad * wide);
     vQ_hi = z((size_t)pad * VH); vQ_lo = z((size_t)pad * VH);
-    std::vector<int32_t> ident(pages);
-    for (size_t i = 0; i < pages; ++i) ident[i] = (int32_t)i;
-    CM_HIP(hipMemcpyAsync(vBt, ident.data(), pages * sizeof(int32_t), hipMemcpyHostToDevice, stream));
     CM_HIP(hipStreamSynchronize(stream));
     v_cap = cap;
 }
@@ -100,7 +97,21 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
                 }
         }
     }
+    VitAttnArgs at{};
+    at.q_hi = vQ_hi; at.q_lo = vQ_lo; at.k = vK; at.v = vV; at.lo_off = vkv_lo_off; at.out_hi = vB_hi; at.out_lo = vB_lo;
+    at.tiles = vTiles; at.heads = heads; at.rows = N; at.part_o = vPartO; at.part_ml = vPartML;
+    int longest = 0, wide_tiles = 0;
+    for (auto& fr : frames) { longest = std::max(longest, fr.second - fr.first); wide_tiles += (fr.second - fr.first + 127) / 128; }
+    // 128 query rows per workgroup where that gives every CU one (64 x 64 patches: tower 14.2 -> 13.2 ms), 64 below (28 x 28: 3.9 -> 3.8); the keys
+    // in runs of 8 tiles or more while the workgroups are fewer than two per CU (42 x 64 patches: 10.04 -> 9.85; full launches lose by the merge)
+    at.wide = wide_tiles * heads >= 256;
+    std::vector<int4> tiles;
+    for (auto& fr : frames)
+        for (int q = fr.first; q < fr.second; q += at.wide ? 128 : 64) tiles.push_back(int4{fr.first, fr.second, q, 0});
+    at.ntiles = (int)tiles.size();
+    at.runs = at.ntiles * heads < 512 ? std::max(1, std::min(vit_ksplit, longest / 512)) : 1;
     CM_HIP(hipStreamSynchronize(s));
+    CM_HIP(hipMemcpyAsync(vTiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     CM_HIP(hipMemcpyAsync(vIdx, idx.data(), idx.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
     CM_HIP(hipMemcpyAsync(vW4, wts.data(), wts.size() * sizeof(float), hipMemcpyHostToDevice, s));
     CM_HIP(hipMemcpyAsync(vCos, cs.data(), cs.size() * sizeof(float), hipMemcpyHostToDevice, s));
@@ -134,17 +145,7 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
         if (!n1_ready) launch_layernorm_rows(vX, b.n1w, b.n1b, vA_hi, vA_lo, N, VH, 1e-6f, s);
         gemm(vA_hi, vA_lo, b.qkv_w, b.qkv_b, N, 3 * VH, VH, GEPI_STORE, vQKV, nullptr, nullptr, 0);
         launch_vit_rope_kv(vQKV, vCos, vSin, vQ_hi, vQ_lo, vK, vV, vkv_lo_off, N, heads, scale, s);
-        for (auto& fr : frames) {                                  // full attention inside each frame (vision.rs:145-172)
-            AttnPreArgs at{};
-            at.q_hi = vQ_hi + (size_t)fr.first * VH; at.q_lo = vQ_lo + (size_t)fr.first * VH;
-            at.block_table = vBt; at.kpool = vK; at.vpool = vV; at.kv_lo_off = vkv_lo_off;
-            at.out_hi = vB_hi + (size_t)fr.first * VH; at.out_lo = vB_lo + (size_t)fr.first * VH;
-            at.S = fr.second - fr.first; at.Hq = heads; at.Hkv = heads; at.nrep = 1; at.page = 64;
-            at.start_pos = fr.first; at.causal = 0; at.kv_lo = fr.first; at.kv_hi = fr.second;
-            // enough (query tile, head, key run) blocks for ~3 waves per SIMD; a run is never shorter than two key tiles
-            at.ksplit = std::max(1, std::min(vit_ksplit, (at.S + 127) / 128)); at.part_o = vPartO; at.part_ml = vPartML;
-            launch_attn_prefill(at, 64, KV_BF16X2, s);
-        }
+        launch_vit_attn(at, s);                                    // full attention inside each frame (vision.rs:145-172)
         gemm(vB_hi, vB_lo, b.proj_w, b.proj_b, N, VH, VH, GEPI_RESADD, vX, nullptr, nullptr, 0, b.n2w, b.n2b);      // + norm2 -> vA
         gemm(vA_hi, vA_lo, b.fc1_w, b.fc1_b, N, vcfg.inter, VH, GEPI_ACT_SPLIT, nullptr, vB_hi, vB_lo, vcfg.act);
         // fc2 + the NEXT norm over vX rows (the next block's norm1, the merger's norm after the last block) -- unless a DeepStack
