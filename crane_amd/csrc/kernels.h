@@ -427,6 +427,7 @@ struct QGemmArgs {
 };
 void launch_quant_rows_q8(const float* x, int ldx, const float* nw, float eps, signed char* xq, float* xd, int M, int K, hipStream_t s, int xs = QGEMM_MAXM);
 bool gemm_q8_ok(const QWeight& w, int M);
+void launch_gemm_q8_rows(const QGemmArgs& a, int num_cu, hipStream_t s);      // kernels_quant_rows.hip: up to 64 rows, Q8_0 layout, groups of 4 blocks; set up by launch_gemm_q8
 // `next` (EPI_RESADD / EPI_SILUMUL): the rows this GEMM writes are the next projection's input -- the reduction launch also quantises
 // them (RMSNorm with next->nw first when set), exactly as launch_quant_rows_q8 would; *fused: 0 = not quantised, 1 = into next->xq / xd
 // (by the reduction launch), 2 = into next->xq2 / xd2 (by the unsplit gate|up GEMM itself, which cannot overwrite the codes it reads)

@@ -1142,7 +1142,7 @@ QGemmPlan plan_gemm_q8(int M, int N, int K, int epi, bool have_ws, size_t ws_flo
     // (more than 128 rows -- a prompt pass: geometry 4 = 8 waves x 4 m-tiles, 256 rows per workgroup, ceil(M / 256) m-panels per launch)
     const int geo = M > QGEMM_MAXM ? 4 : M > 64 ? (geo_env == 0 ? 1 : geo_env == 1 ? 2 : 3) : 0;
     p.geo = geo;
-    // (<= 64 rows, 4 waves: groups of 4 blocks = 52 / 61 KB of LDS, TWO workgroups per CU as `cap` below assumes; with groups of 8 -- 104 KB --
+    // (<= 64 rows, 4 waves: groups of 4 blocks -- Q8_0 layout: kernels_quant_rows.hip --, TWO workgroups per CU as `cap` below assumes; with groups of 8 -- 104 KB --
     // a CU held one 4-wave workgroup, one wave per SIMD.  CM_QGEMM_QG_SMALL = 8: A/B)
     static const int qg_small = getenv("CM_QGEMM_QG_SMALL") && atoi(getenv("CM_QGEMM_QG_SMALL")) == 8 ? 8 : 4;
     p.mh = geo == 1 || geo == 3 || geo == 4 ? 2 : 1; p.mt = geo == 2 || geo == 4 ? 4 : M > 32 ? 2 : 1; p.qg = geo >= 2 ? 4 : geo == 1 ? 8 : qg_small;
@@ -1219,8 +1219,6 @@ bool launch_gemm_q8(const QGemmArgs& a0, int epi, float* y, int ldy, float* ws, 
     static DevOnce attr;
     attr.run([&] {
         (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<1, 1, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<1, 2, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<1, 2, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<2, 2, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipFuncSetAttribute((const void*)gemm_q8_i8_kernel<1, 4, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -1248,13 +1246,12 @@ bool launch_gemm_q8(const QGemmArgs& a0, int epi, float* y, int ldy, float* ws, 
         else if (mt == 2) hipLaunchKernelGGL((gemm_q4k_i8_kernel<1, 2>), grid, block, lds, s, a);
         else hipLaunchKernelGGL((gemm_q4k_i8_kernel<1, 1>), grid, block, lds, s, a);
     }
+    else if (geo == 0 && pl.qg == 4) launch_gemm_q8_rows(a, num_cu, s);
     else if (geo == 4) hipLaunchKernelGGL((gemm_q8_i8_kernel<2, 4, 4>), grid, block, lds, s, a);
     else if (geo == 3) hipLaunchKernelGGL((gemm_q8_i8_kernel<2, 2, 4>), grid, block, lds, s, a);
     else if (geo == 2) hipLaunchKernelGGL((gemm_q8_i8_kernel<1, 4, 4>), grid, block, lds, s, a);
     else if (mh == 2) hipLaunchKernelGGL((gemm_q8_i8_kernel<2, 2, 8>), grid, block, lds, s, a);
-    else if (mt == 2 && pl.qg == 4) hipLaunchKernelGGL((gemm_q8_i8_kernel<1, 2, 4>), grid, block, lds, s, a);
     else if (mt == 2) hipLaunchKernelGGL((gemm_q8_i8_kernel<1, 2, 8>), grid, block, lds, s, a);
-    else if (pl.qg == 4) hipLaunchKernelGGL((gemm_q8_i8_kernel<1, 1, 4>), grid, block, lds, s, a);
     else hipLaunchKernelGGL((gemm_q8_i8_kernel<1, 1, 8>), grid, block, lds, s, a);
     if (direct) { if (fused && a.nxq) *fused = 2; return true; }
     if (epi == EPI_STORE && defer != nullptr && ks <= 4) { defer->ks = ks; defer->slice = a.slice; defer->ws = ws; return true; }      // (the consumer adds the slices)
