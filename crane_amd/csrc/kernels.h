@@ -67,12 +67,12 @@ struct AttnDecArgs {
     float* part_ml;              // [Hq][nsplit][2]
     float* out1 = nullptr;       // ONE token split per sequence (launch_attn_decode*: nsplit == 1): the kernel normalises (and gates) itself and
     int out1_stride = 0;         //   writes out1[seq * out1_stride + h * D + d] -- no partials, no combine launch
-    uint16_t* out1_hi = nullptr; //   ... or, when set (the caller asked attn_decode_single_split()), as bf16 hi + lo planes [seq][out1_cols]: the A
+    uint16_t* out1_hi = nullptr; //   ... or, when set by this kernel or, with several splits, by the combine kernel, as bf16 hi + lo planes [seq][out1_cols]: the A
     uint16_t* out1_lo = nullptr; //   operand of the o_proj GEMM of a large decode group (split_rows2d's arithmetic), instead of the f32 rows
     int out1_cols = 0;
     int qkv_ns = 1;              // qkv rows as qkv_ns f32 slices qkv_slice floats apart (the K-split partials of the int8 qkv GEMM, added in order by the
     size_t qkv_slice = 0;        //   matrix-core kernel's prologue: no reduction launch); 1 = plain rows
-    signed char* out1_q = nullptr;  // ... and ALSO (matrix-core kernel, single split) as Q8_0 blocks of the rows: codes [seq][out1_cols] + block scales
+    signed char* out1_q = nullptr;  // ... and ALSO (matrix-core kernel with a single split; combine kernel) as Q8_0 blocks of the rows: codes [seq][out1_cols] + block scales
     float* out1_qd = nullptr;       //   [out1_cols / 32][QGEMM_MAXM] -- quant_rows_q8_kernel's arithmetic: the int8 o_proj GEMM of a quantised group reads them
     int q_off, k_off, v_off;     // element offsets of q / k / v inside qkv
     int qkv_stride, bt_stride;   // batched step: per-sequence strides of qkv rows and block tables

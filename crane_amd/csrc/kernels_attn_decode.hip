@@ -299,12 +299,13 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(AttnDecArgs a) {
 // grid = Hq, block = 1024: out[h, d] = sum_s e^{m_s-M} o_s[d] / sum_s e^{m_s-M} l_s  (* sigmoid(gate)).
 // The kernel is pure latency (a few KB per head): 1024 / D thread groups split the `s` range so that every partial a
 // thread needs is requested in ONE batch, before the (m, l) weights it will be scaled by have even arrived.
+struct AttnRowOut { uint16_t *hi, *lo; signed char* q; float* qd; int cols; };      // AttnDecArgs::out1_*: what the o_proj GEMM reads
 template <int D>
 __global__ __launch_bounds__(1024) void attn_decode_combine_kernel(const float* __restrict__ part_o,
                                                                    const float* __restrict__ part_ml,
                                                                    const float* __restrict__ gate,
                                                                    float* __restrict__ out, int nsplit, int gate_stride,
-                                                                   int out_stride) {
+                                                                   int out_stride, AttnRowOut ro) {
     constexpr int NH = 1024 / D;                 // thread groups that split the `s` range
     constexpr int PER = 64 / NH;                 // nsplit <= 64
     __shared__ float w_s[64];
@@ -349,7 +350,23 @@ __global__ __launch_bounds__(1024) void attn_decode_combine_kernel(const float* 
     for (int g = 1; g < NH; ++g) O += grp_o[g][d];
     float v = O * inv_l;
     if (gate != nullptr) v *= 1.0f / (1.0f + expf(-gv));
-    out[(size_t)h * D + d] = v;
+    const int col = h * D + d;
+    if (ro.hi != nullptr) {                                      // the A operand of the o_proj GEMM instead of f32 rows (split_rows2d_kernel's arithmetic)
+        const uint16_t hh = f32_to_bf16(v);
+        ro.hi[(size_t)bq * ro.cols + col] = hh;
+        ro.lo[(size_t)bq * ro.cols + col] = f32_to_bf16(v - bf16_to_f32(hh));
+        return;
+    }
+    out[col] = v;
+    if (ro.q == nullptr) return;
+    // and the Q8_0 blocks of the row (32 lanes each, quant_rows_q8_kernel's arithmetic)
+    float am = fabsf(v);
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) am = fmaxf(am, __shfl_xor(am, o));
+    const float dq = am / 127.0f;
+    const float id = dq != 0.f ? 1.0f / dq : 0.f;
+    ro.q[(size_t)bq * ro.cols + col] = (signed char)(int)roundf(v * id);
+    if ((lane & 31) == 0) ro.qd[(size_t)(col >> 5) * QGEMM_MAXM + bq] = (float)(_Float16)dq;
 }
 
 
@@ -986,15 +1003,14 @@ bool launch_attn_decode_mfma(const AttnDecArgs& a, int D, int nrep, int nsplit, 
         b.out1 = out; b.out1_stride = out_stride;
         return D == 128 ? launch_mfma<128>(b, nrep, 1, kv_mode, n_seq, s) : launch_mfma<256>(b, nrep, 1, kv_mode, n_seq, s);
     }
-    if (a.out1_hi != nullptr || a.out1_q != nullptr) return false;       // (planes / codes are only written by the single-split form)
     if (D == 128) {
         if (!launch_mfma<128>(a, nrep, nsplit, kv_mode, n_seq, s)) return false;
         hipLaunchKernelGGL(attn_decode_combine_kernel<128>, dim3(a.Hkv * nrep, n_seq), dim3(1024), 0, s, a.part_o, a.part_ml,
-                           a.gate, out, nsplit, a.qkv_stride, out_stride);
+                           a.gate, out, nsplit, a.qkv_stride, out_stride, AttnRowOut{a.out1_hi, a.out1_lo, a.out1_q, a.out1_qd, a.out1_cols});
     } else if (D == 256) {
         if (!launch_mfma<256>(a, nrep, nsplit, kv_mode, n_seq, s)) return false;
         hipLaunchKernelGGL(attn_decode_combine_kernel<256>, dim3(a.Hkv * nrep, n_seq), dim3(1024), 0, s, a.part_o, a.part_ml,
-                           a.gate, out, nsplit, a.qkv_stride, out_stride);
+                           a.gate, out, nsplit, a.qkv_stride, out_stride, AttnRowOut{a.out1_hi, a.out1_lo, a.out1_q, a.out1_qd, a.out1_cols});
     } else {
         return false;
     }
@@ -1019,21 +1035,20 @@ static bool launch_split(const AttnDecArgs& a, int nrep, int nsplit, int kv_mode
 
 bool launch_attn_decode(const AttnDecArgs& a, int D, int nrep, int nsplit, int kv_mode, float* out, int out_stride, int n_seq,
                         hipStream_t s) {
-    if (a.out1_q != nullptr) return false;                       // (only the matrix-core kernel quantises its output rows)
     if (attn_decode_single_split(nsplit, D)) {                   // (see launch_attn_decode_mfma)
+        if (a.out1_q != nullptr) return false;                   // (this kernel itself does not quantise its rows)
         AttnDecArgs b = a;
         b.out1 = out; b.out1_stride = out_stride;
         return D == 128 ? launch_split<128>(b, nrep, 1, kv_mode, n_seq, s) : launch_split<256>(b, nrep, 1, kv_mode, n_seq, s);
     }
-    if (a.out1_hi != nullptr) return false;
     if (D == 128) {
         if (!launch_split<128>(a, nrep, nsplit, kv_mode, n_seq, s)) return false;
         hipLaunchKernelGGL(attn_decode_combine_kernel<128>, dim3(a.Hkv * nrep, n_seq), dim3(1024), 0, s, a.part_o, a.part_ml,
-                           a.gate, out, nsplit, a.qkv_stride, out_stride);
+                           a.gate, out, nsplit, a.qkv_stride, out_stride, AttnRowOut{a.out1_hi, a.out1_lo, a.out1_q, a.out1_qd, a.out1_cols});
     } else if (D == 256) {
         if (!launch_split<256>(a, nrep, nsplit, kv_mode, n_seq, s)) return false;
         hipLaunchKernelGGL(attn_decode_combine_kernel<256>, dim3(a.Hkv * nrep, n_seq), dim3(1024), 0, s, a.part_o, a.part_ml,
-                           a.gate, out, nsplit, a.qkv_stride, out_stride);
+                           a.gate, out, nsplit, a.qkv_stride, out_stride, AttnRowOut{a.out1_hi, a.out1_lo, a.out1_q, a.out1_qd, a.out1_cols});
     } else {
         return false;
     }

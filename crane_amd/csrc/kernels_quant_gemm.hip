@@ -958,36 +958,63 @@ __global__ __launch_bounds__(256) void q8_splitk_epilogue_kernel(const float* __
     }
 }
 
-// The reduction + the NEXT projection's quantiser in one launch: one 256-thread block per row, thread t owns the float4 chunks
-// k4 = t + 256 j + 1024 i of the OUTPUT row like quant_rows_q8_kernel, so codes and scales are bit-equal to the two launches.
-//   EPI_RESADD : y[m][n] += sum of the slices (N columns), then RMSNorm (NORM) + Q8_0 blocks of the row
-//   EPI_SILUMUL: y[m][k] = silu(gate_k) * up_k from the interleaved columns (2 k, 2 k + 1) (N / 2 outputs), then Q8_0 blocks
-template <int EPI, int KS, bool NORM>
+// Four consecutive columns of a row, slices in order (KS of them; 0: any number)
+template <int KS>
+__device__ __forceinline__ f32x4 q8_slices4(const float* p, size_t slice, int ksplit) {
+    f32x4 v;
+    if constexpr (KS > 0) {
+        f32x4 q[KS];
+#pragma unroll
+        for (int k = 0; k < KS; ++k) q[k] = *(const f32x4*)(p + (size_t)k * slice);
+        v = q[0];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) { v[0] += q[k][0]; v[1] += q[k][1]; v[2] += q[k][2]; v[3] += q[k][3]; }
+    } else {
+        v = *(const f32x4*)p;
+        for (int k = 1; k < ksplit; ++k) {
+            const f32x4 q = *(const f32x4*)(p + (size_t)k * slice);
+            v[0] += q[0]; v[1] += q[1]; v[2] += q[2]; v[3] += q[3];
+        }
+    }
+    return v;
+}
+// chunk k4 of a row -> its four codes, and the scale of the block its eight lanes hold (quant_rows_q8_kernel's arithmetic)
+__device__ __forceinline__ void q8_codes4(const f32x4& v, int k4, int m, uint32_t* row, float* xd, int xs) {
+    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    am = fmaxf(am, __shfl_xor(am, 1)); am = fmaxf(am, __shfl_xor(am, 2)); am = fmaxf(am, __shfl_xor(am, 4));
+    const float d = am / 127.0f;
+    const float id = d != 0.f ? 1.0f / d : 0.f;
+    uint32_t pk = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)roundf(v[e] * id) & 0xFFu) << (8 * e);
+    row[k4] = pk;
+    if ((threadIdx.x & 7) == 0) xd[(size_t)(k4 >> 3) * xs + m] = f16r(d);
+}
+
+// The reduction + the NEXT projection's quantiser in one launch: y[m][n] += sum of the slices (N columns), then RMSNorm + Q8_0 blocks of the row.  One
+// 256-thread block per row, thread t owns the float4 chunks k4 = t + 256 j + 1024 i of the row like quant_rows_q8_kernel, so codes and scales are
+// bit-equal to the two launches.
+template <int KS>
 __global__ __launch_bounds__(256) void q8_splitk_quant_kernel(const float* __restrict__ ws, int M, int N, int ksplit, float* __restrict__ y, int ldy,
                                                               const float* __restrict__ nw, float eps, signed char* __restrict__ xq, float* __restrict__ xd, int xs) {
     __shared__ float red[4];
     const int m = blockIdx.x, t2 = threadIdx.x, lane = t2 & 63, w2 = t2 >> 6;
-    const int Kout = EPI == EPI_SILUMUL ? N / 2 : N, n4 = Kout >> 2;
+    const int n4 = N >> 2;
     const size_t slice = (size_t)M * N;
     float* yr = y + (size_t)m * ldy;
-    auto reduce4 = [&](int col) -> f32x4 {                        // 4 consecutive columns of the row, slices in order
-        const float* p0 = ws + (size_t)m * N + col;
-        f32x4 v;
-        if (KS > 0) {
-            f32x4 p[KS > 0 ? KS : 1];
-#pragma unroll
-            for (int k = 0; k < KS; ++k) p[k] = *(const f32x4*)(p0 + (size_t)k * slice);
-            v = p[0];
-#pragma unroll
-            for (int k = 1; k < KS; ++k) { v[0] += p[k][0]; v[1] += p[k][1]; v[2] += p[k][2]; v[3] += p[k][3]; }
-        } else {
-            v = *(const f32x4*)p0;
-            for (int k = 1; k < ksplit; ++k) {
-                const f32x4 p = *(const f32x4*)(p0 + (size_t)k * slice);
-                v[0] += p[0]; v[1] += p[1]; v[2] += p[2]; v[3] += p[3];
-            }
-        }
-        return v;
+    uint32_t* xqr = (uint32_t*)(xq + (size_t)m * N);
+    auto summed = [&](int k4) -> f32x4 {
+        const f32x4 v = q8_slices4<KS>(ws + (size_t)m * N + 4 * k4, slice, ksplit), c = *(const f32x4*)(yr + 4 * k4);
+        return (f32x4){v[0] + c[0], v[1] + c[1], v[2] + c[2], v[3] + c[3]};
+    };
+    auto scale_of = [&](float ss) -> float {
+        const float t = wave_sum(ss);
+        if (lane == 0) red[w2] = t;
+        __syncthreads();
+        return 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)N + eps);
+    };
+    auto normed = [](f32x4 v, float r, const f32x4& w) -> f32x4 {
+        return (f32x4){__fmul_rn(__fmul_rn(v[0], r), w[0]), __fmul_rn(__fmul_rn(v[1], r), w[1]), __fmul_rn(__fmul_rn(v[2], r), w[2]), __fmul_rn(__fmul_rn(v[3], r), w[3])};
     };
     if (n4 <= 1024) {
         // rows of <= 4096 outputs (o_proj / down_proj of the 8B widths): a thread's four chunks stay in registers through the three passes
@@ -999,109 +1026,114 @@ __global__ __launch_bounds__(256) void q8_splitk_quant_kernel(const float* __res
             const int k4 = t2 + 256 * j;
             o[j] = (f32x4){0.f, 0.f, 0.f, 0.f}; wv[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
             if (k4 >= n4) continue;
-            if (NORM) wv[j] = *(const f32x4*)(nw + (k4 << 2));
-            if (EPI == EPI_SILUMUL) {
-                const f32x4 a0 = reduce4(8 * k4), a1 = reduce4(8 * k4 + 4);
-                o[j][0] = (a0[0] / (1.0f + expf(-a0[0]))) * a0[1]; o[j][1] = (a0[2] / (1.0f + expf(-a0[2]))) * a0[3];
-                o[j][2] = (a1[0] / (1.0f + expf(-a1[0]))) * a1[1]; o[j][3] = (a1[2] / (1.0f + expf(-a1[2]))) * a1[3];
-            } else {
-                const f32x4 v = reduce4(4 * k4), c = *(const f32x4*)(yr + 4 * k4);
-                o[j] = (f32x4){v[0] + c[0], v[1] + c[1], v[2] + c[2], v[3] + c[3]};
-            }
+            wv[j] = *(const f32x4*)(nw + (k4 << 2));
+            o[j] = summed(k4);
             *(f32x4*)(yr + 4 * k4) = o[j];
         }
-        float r = 1.f;
-        if (NORM) {
-            float ss = 0.f;
+        float ss = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (t2 + 256 * j < n4) ss = fmaf(o[j][3], o[j][3], fmaf(o[j][2], o[j][2], fmaf(o[j][1], o[j][1], fmaf(o[j][0], o[j][0], ss))));
-            const float t = wave_sum(ss);
-            if (lane == 0) red[w2] = t;
-            __syncthreads();
-            r = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)Kout + eps);
-        }
-        uint32_t* xqr = (uint32_t*)(xq + (size_t)m * Kout);
+        for (int j = 0; j < 4; ++j)
+            if (t2 + 256 * j < n4) ss = fmaf(o[j][3], o[j][3], fmaf(o[j][2], o[j][2], fmaf(o[j][1], o[j][1], fmaf(o[j][0], o[j][0], ss))));
+        const float r = scale_of(ss);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int k4 = t2 + 256 * j;
             if (k4 >= n4) break;
-            f32x4 xv = o[j];
-            if (NORM) {
-                xv[0] = __fmul_rn(__fmul_rn(xv[0], r), wv[j][0]); xv[1] = __fmul_rn(__fmul_rn(xv[1], r), wv[j][1]);
-                xv[2] = __fmul_rn(__fmul_rn(xv[2], r), wv[j][2]); xv[3] = __fmul_rn(__fmul_rn(xv[3], r), wv[j][3]);
-            }
-            float am = fmaxf(fmaxf(fabsf(xv[0]), fabsf(xv[1])), fmaxf(fabsf(xv[2]), fabsf(xv[3])));
-            am = fmaxf(am, __shfl_xor(am, 1)); am = fmaxf(am, __shfl_xor(am, 2)); am = fmaxf(am, __shfl_xor(am, 4));
-            const float d = am / 127.0f;
-            const float id = d != 0.f ? 1.0f / d : 0.f;
-            uint32_t pk = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)roundf(xv[e] * id) & 0xFFu) << (8 * e);
-            xqr[k4] = pk;
-            if ((t2 & 7) == 0) xd[(size_t)(k4 >> 3) * xs + m] = f16r(d);
+            q8_codes4(normed(o[j], r, wv[j]), k4, m, xqr, xd, xs);
         }
         return;
     }
     // pass 1: the row of y (what q8_splitk_epilogue_kernel writes)
-    for (int k4 = t2; k4 < n4; k4 += 256) {
-        f32x4 o;
-        if (EPI == EPI_SILUMUL) {
-            const f32x4 a0 = reduce4(8 * k4), a1 = reduce4(8 * k4 + 4);
-            o[0] = (a0[0] / (1.0f + expf(-a0[0]))) * a0[1]; o[1] = (a0[2] / (1.0f + expf(-a0[2]))) * a0[3];
-            o[2] = (a1[0] / (1.0f + expf(-a1[0]))) * a1[1]; o[3] = (a1[2] / (1.0f + expf(-a1[2]))) * a1[3];
-        } else {
-            const f32x4 v = reduce4(4 * k4), c = *(const f32x4*)(yr + 4 * k4);
-            o = (f32x4){v[0] + c[0], v[1] + c[1], v[2] + c[2], v[3] + c[3]};
-        }
-        *(f32x4*)(yr + 4 * k4) = o;
-    }
+    for (int k4 = t2; k4 < n4; k4 += 256) *(f32x4*)(yr + 4 * k4) = summed(k4);
     // pass 2 + 3: quant_rows_q8_kernel over this thread's own stores
-    float r = 1.f;
-    if (NORM) {
-        float ss = 0.f;
-        for (int kb = t2; kb < n4; kb += 1024) {
-            f32x4 v[4];
+    float ss = 0.f;
+    for (int kb = t2; kb < n4; kb += 1024) {
+        f32x4 v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = (kb + 256 * j < n4) ? *(const f32x4*)(yr + ((kb + 256 * j) << 2)) : (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 4; ++j) v[j] = (kb + 256 * j < n4) ? *(const f32x4*)(yr + ((kb + 256 * j) << 2)) : (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (kb + 256 * j < n4) ss = fmaf(v[j][3], v[j][3], fmaf(v[j][2], v[j][2], fmaf(v[j][1], v[j][1], fmaf(v[j][0], v[j][0], ss))));
-        }
-        const float t = wave_sum(ss);
-        if (lane == 0) red[w2] = t;
-        __syncthreads();
-        r = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)Kout + eps);
+        for (int j = 0; j < 4; ++j)
+            if (kb + 256 * j < n4) ss = fmaf(v[j][3], v[j][3], fmaf(v[j][2], v[j][2], fmaf(v[j][1], v[j][1], fmaf(v[j][0], v[j][0], ss))));
     }
-    uint32_t* xqr = (uint32_t*)(xq + (size_t)m * Kout);
+    const float r = scale_of(ss);
     for (int kb = t2; kb < n4; kb += 1024) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int k4 = kb + 256 * j;
             if (k4 >= n4) break;
-            f32x4 xv = *(const f32x4*)(yr + (k4 << 2));
-            if (NORM) {
-                const f32x4 w = *(const f32x4*)(nw + (k4 << 2));
-                xv[0] = __fmul_rn(__fmul_rn(xv[0], r), w[0]); xv[1] = __fmul_rn(__fmul_rn(xv[1], r), w[1]);
-                xv[2] = __fmul_rn(__fmul_rn(xv[2], r), w[2]); xv[3] = __fmul_rn(__fmul_rn(xv[3], r), w[3]);
-            }
-            float am = fmaxf(fmaxf(fabsf(xv[0]), fabsf(xv[1])), fmaxf(fabsf(xv[2]), fabsf(xv[3])));
-            am = fmaxf(am, __shfl_xor(am, 1)); am = fmaxf(am, __shfl_xor(am, 2)); am = fmaxf(am, __shfl_xor(am, 4));
-            const float d = am / 127.0f;
-            const float id = d != 0.f ? 1.0f / d : 0.f;
-            uint32_t pk = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pk |= ((uint32_t)(int)roundf(xv[e] * id) & 0xFFu) << (8 * e);
-            xqr[k4] = pk;
-            if ((t2 & 7) == 0) xd[(size_t)(k4 >> 3) * xs + m] = f16r(d);
+            q8_codes4(normed(*(const f32x4*)(yr + (k4 << 2)), r, *(const f32x4*)(nw + (k4 << 2))), k4, m, xqr, xd, xs);
         }
     }
 }
 
+// Reduction + quantiser without a norm: nothing couples the blocks of a row, so a thread takes ONE chunk and a row is spread over workgroups.  A
+// decode group has 8 .. 64 rows: one workgroup per row was latency on a tenth of the chip (20 rows of 12288 outputs, two slices: 14.4 -> 5.0 us)
+template <int EPI, int KS>
+__global__ __launch_bounds__(256) void q8_splitk_codes_kernel(const float* __restrict__ ws, int M, int N, int ksplit, float* __restrict__ y, int ldy,
+                                                              signed char* __restrict__ xq, float* __restrict__ xd, int xs) {
+    const int m = blockIdx.y, k4 = (int)(blockIdx.x * 256 + threadIdx.x), Kout = EPI == EPI_SILUMUL ? N / 2 : N;
+    if (k4 >= Kout >> 2) return;                                  // (Kout % 32 == 0: the eight lanes of a block leave together)
+    const size_t slice = (size_t)M * N;
+    const float* p = ws + (size_t)m * N;
+    float* yr = y + (size_t)m * ldy + 4 * k4;
+    f32x4 o;
+    if (EPI == EPI_SILUMUL) {
+        const f32x4 a0 = q8_slices4<KS>(p + 8 * k4, slice, ksplit), a1 = q8_slices4<KS>(p + 8 * k4 + 4, slice, ksplit);
+        o[0] = (a0[0] / (1.0f + expf(-a0[0]))) * a0[1]; o[1] = (a0[2] / (1.0f + expf(-a0[2]))) * a0[3];
+        o[2] = (a1[0] / (1.0f + expf(-a1[0]))) * a1[1]; o[3] = (a1[2] / (1.0f + expf(-a1[2]))) * a1[3];
+    } else {
+        const f32x4 v = q8_slices4<KS>(p + 4 * k4, slice, ksplit), c = *(const f32x4*)yr;
+        o = (f32x4){v[0] + c[0], v[1] + c[1], v[2] + c[2], v[3] + c[3]};
+    }
+    *(f32x4*)yr = o;
+    q8_codes4(o, k4, m, (uint32_t*)(xq + (size_t)m * Kout), xd, xs);
+}
+
+// Residual + RMSNorm + quantiser of a decode group's rows of up to 4096 columns: q8_splitk_quant_kernel with one chunk per thread of 1024 (every
+// slice of a thread's chunk in one batch of requests instead of four chunks' worth), the sum of squares over the row in LDS in that kernel's order
+template <int KS>
+__global__ __launch_bounds__(1024) void q8_splitk_norm_codes_kernel(const float* __restrict__ ws, int M, int N, int ksplit, float* __restrict__ y, int ldy,
+                                                                    const float* __restrict__ nw, float eps, signed char* __restrict__ xq, float* __restrict__ xd, int xs) {
+    __shared__ f32x4 row[1024];
+    __shared__ float red[4];
+    const int m = blockIdx.x, k4 = threadIdx.x, n4 = N >> 2;
+    const bool live = k4 < n4;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f}, w = o;
+    if (live) {
+        float* yr = y + (size_t)m * ldy + 4 * k4;
+        w = *(const f32x4*)(nw + 4 * k4);
+        const f32x4 c = *(const f32x4*)yr, v = q8_slices4<KS>(ws + (size_t)m * N + 4 * k4, (size_t)M * N, ksplit);
+        o = (f32x4){v[0] + c[0], v[1] + c[1], v[2] + c[2], v[3] + c[3]};
+        *(f32x4*)yr = o;
+    }
+    row[k4] = o;
+    __syncthreads();
+    if (k4 < 256) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4 v = row[k4 + 256 * j];
+            if (k4 + 256 * j < n4) ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], fmaf(v[0], v[0], ss))));
+        }
+        const float t = wave_sum(ss);
+        if ((k4 & 63) == 0) red[k4 >> 6] = t;
+    }
+    __syncthreads();
+    if (!live) return;
+    const float r = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)N + eps);
+    o[0] = __fmul_rn(__fmul_rn(o[0], r), w[0]); o[1] = __fmul_rn(__fmul_rn(o[1], r), w[1]);
+    o[2] = __fmul_rn(__fmul_rn(o[2], r), w[2]); o[3] = __fmul_rn(__fmul_rn(o[3], r), w[3]);
+    q8_codes4(o, k4, m, (uint32_t*)(xq + (size_t)m * N), xd, xs);
+}
+
 template <int EPI>
 static void launch_q8_epilogue_quant(const float* ws, int M, int N, int ks, float* y, int ldy, const QNext& nx, int xs, hipStream_t s) {
-#define CM_QQ(KS_) do { if (nx.nw) hipLaunchKernelGGL((q8_splitk_quant_kernel<EPI, KS_, true>), dim3(M), dim3(256), 0, s, ws, M, N, ks, y, ldy, nx.nw, nx.eps, nx.xq, nx.xd, xs); \
-                        else hipLaunchKernelGGL((q8_splitk_quant_kernel<EPI, KS_, false>), dim3(M), dim3(256), 0, s, ws, M, N, ks, y, ldy, nx.nw, nx.eps, nx.xq, nx.xd, xs); } while (0)
+    const int kout = EPI == EPI_SILUMUL ? N / 2 : N;
+    const dim3 spread((unsigned)((kout / 4 + 255) / 256), (unsigned)M);
+    const bool wide = EPI == EPI_RESADD && M <= QGEMM_MAXM && N <= 4096;
+#define CM_QQ(KS_) do { if (EPI == EPI_SILUMUL || nx.nw == nullptr) hipLaunchKernelGGL((q8_splitk_codes_kernel<EPI, KS_>), spread, dim3(256), 0, s, ws, M, N, ks, y, ldy, nx.xq, nx.xd, xs); \
+                        else if (wide) hipLaunchKernelGGL((q8_splitk_norm_codes_kernel<KS_>), dim3(M), dim3(1024), 0, s, ws, M, N, ks, y, ldy, nx.nw, nx.eps, nx.xq, nx.xd, xs); \
+                        else hipLaunchKernelGGL((q8_splitk_quant_kernel<KS_>), dim3(M), dim3(256), 0, s, ws, M, N, ks, y, ldy, nx.nw, nx.eps, nx.xq, nx.xd, xs); } while (0)
     switch (ks) {
         case 1: CM_QQ(1); break; case 2: CM_QQ(2); break; case 3: CM_QQ(3); break; case 4: CM_QQ(4); break; case 5: CM_QQ(5); break;
         case 6: CM_QQ(6); break; case 8: CM_QQ(8); break; case 10: CM_QQ(10); break; case 12: CM_QQ(12); break; case 16: CM_QQ(16); break;

@@ -2013,6 +2013,8 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 // reduction launch) and writes the Q8_0 blocks of its rows for the int8 o_proj GEMM (no quantiser launch)
                 const bool attn_q = attn_outq && mf && qgemm_ok && nb >= q_gemm_min && attn_decode_single_split(ns_b, D) && !cfg.hybrid &&
                                     !(heads_b && !quantized && !rccl);
+                const bool codes_ok = attn_outq && qgemm_ok && nb >= q_gemm_min && !cfg.hybrid && !(heads_b && !quantized && !rccl) &&
+                                      (mf || !attn_decode_single_split(ns_b, D));
                 QDefer qdef{1, 0, nullptr};
                 if (quantized) {
                     const bool defer_ok = attn_q && w.n_qkv == 1 && ldq == w.q_qkv[0].N && w.qkv_row0[0] == 0;
@@ -2040,12 +2042,13 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 // a group whose (kv head, sequence) pairs alone fill the chip twice takes ONE token split per sequence and the
                 // matrix-core kernel from 64 tokens on (the VALU kernel's 16-lane rows pay per token, not per tile): engine at
                 // max_running 128, contexts 128-256: 9567 -> 10264 tok/s
-                // one split per sequence: the kernel normalises itself (no combine launch) and, in front of the o_proj GEMM of a large
-                // group, writes the bf16 hi + lo planes the GEMM reads (no split_rows2d launch either)
-                const bool planes = gemm_b && !quantized && attn_decode_single_split(ns_b, D);
+                // one split per sequence: the kernel normalises itself (no combine launch); it, or the combine kernel, writes what the o_proj
+                // GEMM of a large group reads: the bf16 hi + lo planes (no split_rows2d launch)
+                const bool planes = gemm_b && !quantized;
                 if (planes) { a.out1_hi = pAT_hi; a.out1_lo = pAT_lo; a.out1_cols = Hq_l * D; }
-                // ... or, in front of the int8 o_proj GEMM of a quantised group, ALSO the Q8_0 blocks of the rows (no quantiser launch)
-                const bool codes = attn_q && gemm_q8_ok(w.q_o, nb) && w.q_o.fmt == QFMT_Q8_0 && (Hq_l * D) % 64 == 0;
+                // ... or, in front of the int8 o_proj GEMM of a quantised group, ALSO the Q8_0 blocks of the rows (no quantiser launch: the two
+                // 5.7 + 4.7 us at 20 sequences, 4.7 together)
+                const bool codes = codes_ok && gemm_q8_ok(w.q_o, nb) && w.q_o.fmt == QFMT_Q8_0 && (Hq_l * D) % 64 == 0;
                 if (codes) { a.out1_q = qx_codes; a.out1_qd = qx_scales; a.out1_cols = Hq_l * D; }
                 if (qdef.ks > 1) { a.qkv = qdef.ws; a.qkv_stride = w.q_qkv[0].N; a.qkv_ns = qdef.ks; a.qkv_slice = qdef.slice; }      // (the slices of the qkv GEMM, rows N floats apart)
                 if (mf) {
@@ -2054,7 +2057,6 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 if (codes) { qx_src = attnb; qx_nw = nullptr; qx_K = Hq_l * D; qx_kind = 0; if (q_capture) q_capture_rows(nb, Hq_l * D); }      // (the codes hold the attention rows)
                 if (quantized) qrp(w.q_o, attnb, (int)at_cols, w.ln2);
                 else if (gemm_b) {
-                    if (!planes) launch_split_rows2d(attnb, (int)at_cols, pAT_hi, pAT_lo, nb, Hq_l * D, s);
                     gmr(pAT_hi, pAT_lo, w.o, Hq_l * D, fuse_norm ? w.ln2 : nullptr);
                 } else rp(w.o, attnb, (int)at_cols, Hq_l * D);
                 }
