@@ -1244,8 +1244,21 @@ static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     if (ks > 1) launch_splitk(a, epi, s);
     return true;
 }
+static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s);
+// Prompt rows over a width that no tile of kernels_gemm256.hip divides because of its last 128 columns (the merged in_proj of a Gated-Delta-Net layer:
+// 8192 columns and 32 gate columns padded to 128): the wide part there, the last columns alone.  8320 x 2048, 2048 rows: 180 -> 137 us (a prompt of
+// 2048 / 1024 / 300 tokens 18.6 / 10.8 / 5.54 -> 17.8 / 10.2 / 5.49 ms; width 1024: 12.3 / 7.3 / 4.5 -> 12.0 / 7.2 / 4.5)
+static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {
+    if (epi != GEPI_STORE || a.norm_w != nullptr || a.M < 256 || a.N < 512 || a.N % 192 == 0 || a.N % 256 != 128) return false;
+    GemmArgs most = a, rest = a;
+    most.N = a.N - 128;
+    if (!try_gemm256(most, epi, s)) return false;
+    rest.W = a.W + (size_t)most.N * a.K; rest.C = a.C + most.N; rest.N = 128;
+    if (a.bias != nullptr) rest.bias = a.bias + most.N;
+    return launch_gemm_inner(rest, epi, s);
+}
 static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
-    if (try_gemm_rows(a, epi, s) || try_gemm256(a, epi, s)) return true;
+    if (try_gemm_tail(a, epi, s) || try_gemm_rows(a, epi, s) || try_gemm256(a, epi, s)) return true;
     const int tiles_m = (a.M + GBM - 1) / GBM;
     const bool split = a.A_lo != nullptr;
     // 256-wide tiles (one 8-wave block per CU) when they give every CU at least two blocks (1024-token gate||up: 428 -> ~370 us;
