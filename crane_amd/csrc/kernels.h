@@ -155,8 +155,8 @@ struct GemmArgs {
 
 // 9 .. 128 rows with hi + lo activations (kernels_gemm_rows.hip): K slices for these sizes (0: not taken) and the launch (a.ksplit set; more than
 // one slice: partial tiles in a.ws)
-int gemm_rows_split(int M, int N, int K, size_t ws_floats);
-bool launch_gemm_rows(const GemmArgs& a, int epi, hipStream_t s);
+bool gemm_rows_plan(int M, int N, int K, size_t ws_floats, int* bn, int* ks);
+bool launch_gemm_rows(const GemmArgs& a, int epi, int bn, hipStream_t s);
 
 // one sequence of a multi-sequence prompt pass (Model::prefill_multi): rows [row0, row0 + S) of the pass at positions start_pos...,
 // page table at block_table + bt_off

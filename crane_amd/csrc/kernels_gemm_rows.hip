@@ -2,15 +2,16 @@
 // activations as bf16 hi + lo planes, two MFMAs per product -- gemm256_kernel's arithmetic and epilogues on tiles made for a launch that waits
 // for its weights.
 //
-// What bounds it: the weight stream.  gemm256_kernel's tiles are 192 or 256 columns wide: 96 .. 128 workgroups for a 24576-column projection,
-// on half of the chip.  Here a workgroup of four waves owns 128 columns, one workgroup on each CU, with two (at 32 rows: three) weight tiles of
-// 16 KB in flight under the one it multiplies; the activations come out of the L2.  Tiles go from memory into LDS without passing registers
-// (8 rows x 128 bytes per wave instruction, the bank swizzle on the source address: slot p of a row holds its 16-byte chunk
-// p ^ ((row >> 1) & 7)), ST stages, one barrier per k-tile.  Narrow projections split K and leave f32 partial tiles for the fixed-order
+// What bounds it: the weight stream, and from 64 rows on what every column tile reads of the activations out of the L2 (128 rows, gate_up of width
+// 4096: 32 KB of them next to 12 KB of weights per tile and k-tile, 11 TB/s in all).  gemm256_kernel's tiles are 192 or 256 columns wide: 96 ..
+// 128 workgroups for a 24576-column projection, on half of the chip.  Here a workgroup owns 128 columns, or 96 where that fills the chip better,
+// one workgroup on each CU, with two (at 32 rows: three) weight tiles in flight under the one it multiplies.  Tiles go from memory into LDS
+// without passing registers (8 rows x 128 bytes per wave instruction, the bank swizzle on the source address: slot p of a row holds its 16-byte
+// chunk p ^ ((row >> 1) & 7)), ST stages, one barrier per k-tile.  Narrow projections split K and leave f32 partial tiles for the fixed-order
 // reduction kernels.  Measured (us per launch with its reduction, 32 rows, gemm256_kernel / gemm_bf16_kernel -> here):
-//   width 4096:  gate_up (24576 x 4096) 50.3 -> 46.6 (4.3 TB/s), down (4096 x 12288) 34.4 -> 24.8, qkv (6144 x 4096) 17.5 -> 14.9, o 15.0 -> 11.8;
-//                the whole layer at 16 / 32 / 64 / 128 rows 114 / 117 / 125 / 160 -> 95 / 98 / 113 / 149
-//   width 2048 (I 6144): layer 54 -> 40;  width 1024 (I 3072): 40 -> 31;  lm_head (151936 x 4096) 385 -> 277 (4.5 TB/s), 391 -> 290 at 64 rows
+//   width 4096:  gate_up (24576 x 4096) 50.3 -> 44.6 (4.5 TB/s), down (4096 x 12288) 34.4 -> 24.4, qkv (6144 x 4096) 17.5 -> 14.1, o 15.0 -> 11.6;
+//                the whole layer at 16 / 32 / 64 / 128 rows 114 / 117 / 125 / 160 -> 92 / 95 / 108 / 146
+//   width 2048 (I 6144): layer 58 -> 45;  width 1024 (I 3072): 40 -> 30;  lm_head (151936 x 4096) 385 -> 277 (4.5 TB/s), 391 -> 290 at 64 rows
 // Tiles of 64 columns, weight loads that bypass the caches, two workgroups per CU with fewer stages, a k start of its own per workgroup and
 // two k-tiles per barrier were all no faster.
 #include "dev_common.h"
@@ -20,7 +21,7 @@ namespace cm {
 
 namespace {
 
-constexpr int RBK = 64, RBN = 128;
+constexpr int RBK = 64;
 
 __device__ __forceinline__ void rows_load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
     uint32_t keep;
@@ -28,11 +29,11 @@ __device__ __forceinline__ void rows_load16(const void* gsrc, uint32_t lds_base)
                  : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
 }
 
-template <int BM, int ST, int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs a) {
-    constexpr int GM = BM == 32 ? 1 : 2, GN = 4 / GM, WM = BM / GM, WN = RBN / GN, NI = WM / 16, NJ = WN / 16;      // waves GM x GN, WM x WN outputs each
+template <int BM, int RBN, int ST, int EPI, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_rows_kernel(GemmArgs a) {
+    constexpr int GM = RBN == 96 ? NW / 2 : NW == 8 ? (BM == 128 ? 4 : 2) : BM == 32 ? 1 : 2, GN = NW / GM, WM = BM / GM, WN = RBN / GN, NI = WM / 16, NJ = WN / 16;      // NW waves GM x GN, WM x WN outputs each
     constexpr int PLANE = BM * RBK, STAGE = 2 * PLANE + RBN * RBK;
-    constexpr int APC = BM / 8, NL = (2 * APC + RBN / 8) / 4;                          // pieces per plane / requests per wave and k-tile
+    constexpr int APC = BM / 8, NP = 2 * APC + RBN / 8, NL = (NP + NW - 1) / NW;                          // pieces per plane / requests per wave and k-tile
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs a) {
     uint32_t dst[NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-        const int p = wave + 4 * i, plane = p / APC;                                   // 0: hi, 1: lo, 2 and up: weights
+        const int p = min(wave + NW * i, NP - 1), plane = p / APC;                                   // 0: hi, 1: lo, 2 and up: weights
         const int r0 = (plane < 2 ? p - plane * APC : p - 2 * APC) * 8, row = r0 + prow;
         const size_t kc = (size_t)kbeg * RBK + (size_t)((pslot ^ ((row >> 1) & 7)) << 3);
         const bool isw = plane >= 2;
@@ -127,43 +128,61 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(GemmArgs a) {
         }
 }
 
-template <int BM, int ST, int EPI>
+template <int BM, int RBN, int ST, int EPI, int NW>
 void go(const GemmArgs& a, hipStream_t s) {
     constexpr size_t lds = (size_t)ST * (2 * BM + RBN) * RBK * sizeof(uint16_t);
     static DevOnce attr;
-    attr.run([&] { (void)hipFuncSetAttribute((const void*)gemm_rows_kernel<BM, ST, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
-    hipLaunchKernelGGL((gemm_rows_kernel<BM, ST, EPI>), dim3((unsigned)(a.N / RBN * a.ksplit)), dim3(256), lds, s, a);
+    attr.run([&] { (void)hipFuncSetAttribute((const void*)gemm_rows_kernel<BM, RBN, ST, EPI, NW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+    hipLaunchKernelGGL((gemm_rows_kernel<BM, RBN, ST, EPI, NW>), dim3((unsigned)(a.N / RBN * a.ksplit)), dim3(64 * NW), lds, s, a);
 }
-template <int BM, int ST>
+template <int BM, int RBN, int ST, int NW>
 void go_epi(const GemmArgs& a, int epi, hipStream_t s) {
-    if (a.ksplit > 1) go<BM, ST, GEPI_PARTIAL>(a, s);
-    else if (epi == GEPI_STORE) go<BM, ST, GEPI_STORE>(a, s);
-    else if (epi == GEPI_RESADD) go<BM, ST, GEPI_RESADD>(a, s);
-    else go<BM, ST, GEPI_SILUMUL>(a, s);
+    if (a.ksplit > 1) go<BM, RBN, ST, GEPI_PARTIAL, NW>(a, s);
+    else if (epi == GEPI_STORE) go<BM, RBN, ST, GEPI_STORE, NW>(a, s);
+    else if (epi == GEPI_RESADD) go<BM, RBN, ST, GEPI_RESADD, NW>(a, s);
+    else go<BM, RBN, ST, GEPI_SILUMUL, NW>(a, s);
 }
 
 }  // namespace
 
 // Where the lines lie (both sides measured, old kernels / these, us): more than one round of workgroups pays only while the last round is well
-// filled -- 272 tiles (34816 x 5120, 64 rows) 98 / 124, 1187 tiles 391 / 290; above 64 rows a launch is bound by its MFMAs as much as by the
+// filled -- 272 tiles (34816 x 5120, 64 rows) 98 / 124, 1187 tiles 391 / 290; above 64 rows a launch is bound by its activations as much as by the
 // weights, and wide projections stay with the wider tiles -- 192 tiles at 128 rows 62 / 78, 1187 tiles 405 / 405, while 32 .. 48 tiles split 4
-// ways 46 / 40 and 28 / 27.  A slice of K keeps at least four k-tiles: the pipeline's fill costs two or three.
-int gemm_rows_split(int M, int N, int K, size_t ws_floats) {
-    if (M < 9 || M > 128 || N % RBN != 0 || K % RBK != 0) return 0;
-    const int tiles = N / RBN, nk = K / RBK, rounds = (tiles + 255) / 256;
-    if (tiles > 256 && tiles * 10 < rounds * 256 * 9) return 0;
-    if (M > 64 && tiles > 128) return 0;
+// ways 46 / 38 and 28 / 24.  A slice of K keeps at least four k-tiles: the pipeline's fill costs two or three.  96 columns where they fill more of
+// the last round (24576 columns: 256 workgroups for 192, 46.5 -> 44.6 at 32 rows, 53.5 -> 49.2 at 64; 6144: 4 x 64 for 4 x 48, 14.7 -> 14.1).
+static int rows_split(int M, int N, int K, int bn, size_t ws_floats) {
+    const int tiles = N / bn, nk = K / RBK;
     int ks = 1;
     while (ks < 8 && 2 * ks * tiles <= 256 && nk % (2 * ks) == 0 && nk / (2 * ks) >= 4 && (size_t)2 * ks * M * N <= ws_floats) ks *= 2;
     return ks;
 }
+bool gemm_rows_plan(int M, int N, int K, size_t ws_floats, int* bn, int* ks) {
+    if (M < 9 || M > 128 || K % RBK != 0) return false;
+    double best = 0.0;
+    for (int b : {128, 96}) {
+        if (N % b != 0) continue;
+        const int tiles = N / b, s = rows_split(M, N, K, b, ws_floats), rounds = (tiles * s + 255) / 256;
+        const double fill = (double)tiles * s / (rounds * 256);
+        if (tiles > 256 && fill < 0.9) continue;
+        if (M > 64 && tiles > 128) continue;
+        if (fill > best + 0.05) { best = fill; *bn = b; *ks = s; }
+    }
+    return best > 0.0;
+}
 
 // a.ksplit set by the caller (1: epilogue `epi`; > 1: partial tiles, the caller runs the reduction)
-bool launch_gemm_rows(const GemmArgs& a, int epi, hipStream_t s) {
-    if (a.M > 128 || a.A_lo == nullptr || a.N % RBN != 0 || a.K % (RBK * a.ksplit) != 0 || epi == GEPI_ACT_SPLIT) return false;
-    if (a.M <= 32) go_epi<32, 4>(a, epi, s);
-    else if (a.M <= 64) go_epi<64, 3>(a, epi, s);
-    else go_epi<128, 3>(a, epi, s);
+bool launch_gemm_rows(const GemmArgs& a, int epi, int bn, hipStream_t s) {
+    if (a.M > 128 || a.A_lo == nullptr || a.N % bn != 0 || a.K % (RBK * a.ksplit) != 0 || epi == GEPI_ACT_SPLIT) return false;
+    // (eight waves against four: 128 rows 153 -> 147 us for the layer of width 4096, 32 rows 98 -> 96; the 96-column tiles of up to 64 rows have no
+    // use for them: 17.9 / 16.8 us for the qkv of 64 rows)
+    if (bn == 96) {
+        if (a.M <= 32) go_epi<32, 96, 4, 4>(a, epi, s);
+        else if (a.M <= 64) go_epi<64, 96, 3, 4>(a, epi, s);
+        else go_epi<128, 96, 3, 8>(a, epi, s);
+    }
+    else if (a.M <= 32) go_epi<32, 128, 4, 8>(a, epi, s);
+    else if (a.M <= 64) go_epi<64, 128, 3, 8>(a, epi, s);
+    else go_epi<128, 128, 3, 8>(a, epi, s);
     return true;
 }
 

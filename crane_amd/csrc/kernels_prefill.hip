@@ -1237,10 +1237,10 @@ bool launch_gemm(const GemmArgs& a0, int epi, hipStream_t s) {
 static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     static const int env = getenv("CM_GEMM256") ? atoi(getenv("CM_GEMM256")) : 1;
     if (!env || (a.wide256 != 1 && a.wide256 != 4) || a.A_lo == nullptr || epi == GEPI_ACT_SPLIT) return false;
-    const int ks = gemm_rows_split(a.M, a.N, a.K, a.ws ? a.ws_floats : 0);
-    if (ks == 0) return false;
+    int bn = 0, ks = 0;
+    if (!gemm_rows_plan(a.M, a.N, a.K, a.ws ? a.ws_floats : 0, &bn, &ks)) return false;
     a.ksplit = ks;
-    if (!launch_gemm_rows(a, epi, s)) return false;
+    if (!launch_gemm_rows(a, epi, bn, s)) return false;
     if (ks > 1) launch_splitk(a, epi, s);
     return true;
 }
