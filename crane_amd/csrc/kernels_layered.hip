@@ -1457,7 +1457,9 @@ __global__ __launch_bounds__(256) void lay_attn_merge_kernel(LAttnArgs a, int ns
             acc = fmaf(a.part_o[pr * d + i], w, acc);
         }
         const float gate = a.gate == LGATE_NONE ? 1.f : a.gbuf[(size_t)row * a.ldg + (a.gate == LGATE_ELEM ? head * d + i : head)];
-        a.out[(size_t)row * a.ldo + head * d + i] = acc * gate / L * a.out_scale;
+        const float v = acc * gate / L * a.out_scale;
+        a.out[(size_t)row * a.ldo + head * d + i] = v;
+        if (a.out16 != nullptr) a.out16[(size_t)row * a.ldo + head * d + i] = f32_to_bf16(v);
     }
 }
 static size_t lay_attn_lds(int d, int e, bool own_v, int KT) {

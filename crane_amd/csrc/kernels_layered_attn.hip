@@ -194,6 +194,13 @@ __device__ __forceinline__ void put4(const LAttnArgs& a, int row, int head, int 
 #pragma unroll
         for (int r = 0; r < 4; ++r) out[r] = v[r];
     }
+    if (a.out16 == nullptr) return;
+    uint16_t* o16 = a.out16 + (size_t)row * a.ldo + head * a.e + c;
+    if (ovec) *(u32x2*)o16 = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o16[r] = f32_to_bf16(v[r]);
+    }
 }
 
 // ---- prompt passes.  DP / EP: key / value size the registers and LDS rows are laid out for (64 or 128).  A block

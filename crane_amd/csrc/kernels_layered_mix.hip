@@ -106,7 +106,7 @@ template <int VEC>
 __global__ __launch_bounds__(256) void lay_add_tanh_norm_kernel(float* __restrict__ x, const int32_t* __restrict__ rows, const float* __restrict__ y,
                                                                 int nsum, const float* __restrict__ wsel, float mult, float alpha,
                                                                 const float* __restrict__ w, const float* __restrict__ b,
-                                                                float* __restrict__ out, int W) {
+                                                                float* __restrict__ out, uint16_t* __restrict__ out16, int W) {
     typedef float vec __attribute__((ext_vector_type(VEC)));
     const int r = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * VEC;
     if (c >= W) return;
@@ -132,15 +132,18 @@ __global__ __launch_bounds__(256) void lay_add_tanh_norm_kernel(float* __restric
 #pragma unroll
     for (int i = 0; i < VEC; ++i) o[i] = fmaf(tanhf(alpha * v[i]), nw[i], nb[i]);
     *(vec*)(out + (size_t)r * W + c) = o;
+    if (out16 == nullptr) return;
+    if constexpr (VEC == 4) *(u32x2*)(out16 + (size_t)r * W + c) = (u32x2){pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+    else out16[(size_t)r * W + c] = f32_to_bf16(o[0]);
 }
 void launch_lay_add_tanh_norm(float* x, const int32_t* rows, const float* y, int nsum, const float* wsel, float mult, float alpha, const float* w,
-                              const float* b, float* out, int n_rows, int W, hipStream_t s) {
+                              const float* b, float* out, int n_rows, int W, hipStream_t s, uint16_t* out16) {
     if (n_rows <= 0 || (!y && !out)) return;
     // few rows (decode steps): narrow accesses, so that the row is spread over more threads
     const int vec = W % 4 == 0 && (n_rows > 32 || W > 8192) ? 4 : 1;
     const dim3 grid((unsigned)n_rows, (unsigned)((W / vec + 255) / 256));
-    if (vec == 4) hipLaunchKernelGGL(lay_add_tanh_norm_kernel<4>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, W);
-    else hipLaunchKernelGGL(lay_add_tanh_norm_kernel<1>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, W);
+    if (vec == 4) hipLaunchKernelGGL(lay_add_tanh_norm_kernel<4>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, out16, W);
+    else hipLaunchKernelGGL(lay_add_tanh_norm_kernel<1>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, out16, W);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

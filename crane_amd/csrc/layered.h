@@ -186,6 +186,7 @@ struct LaySegDev { int row0, n, start_pos, slot, bt_off, pad0, pad1, pad2; };
 
 struct LGemmArgs {
     const float* A = nullptr; int lda = 0;
+    const uint16_t* A16 = nullptr;                   // the same rows rounded to bfloat16, K apart, where the launch that made them left them so (or null)
     const int32_t* a_idx = nullptr; int a_div = 1;   // A row of output row p: a_idx ? a_idx[p] / a_div : p
     const uint16_t* W = nullptr;                     // [N][K] bf16
     const uint16_t* W2 = nullptr;                    // second matrix: C = act(A W^T) * (A W2^T)
@@ -276,6 +277,7 @@ struct LAttnArgs {
     const float* proj; int ldp, q_off, g_off;        // activated projection rows: q | k | gate
     const float* gbuf = nullptr; int ldg = 0;        // gates in rows of their own (null: proj + g_off, rows of ldp)
     float* out; int ldo;                             // [T][H d], gated
+    uint16_t* out16 = nullptr;                       // lay_attn_tile, lay_attn_few: the output rounded to bfloat16 as well, rows of ldo
     const void* kpool;                               // [n_pages][G][page][d]
     const int32_t* bt; const LaySegDev* segs; const int2* tiles; int ntiles;
     const float *r1, *r2;
@@ -366,9 +368,10 @@ void launch_lay_rms_gate(const float* o, const float* gate, int ldg, const float
 
 // ---- kernels_layered_mix.hip ----
 // norm without a statistic: x[r] += mult * sum_(k < nsum) y[(r nsum + k) W ..] (y null: nothing is added; wsel given: row k times
-// wsel[r nsum + k]), then out[r][c] = tanh(alpha x[rows ? rows[r] : r][c]) w[c] + b[c] (out null: the update alone).  rows and y exclude each other.
+// wsel[r nsum + k]), then out[r][c] = tanh(alpha x[rows ? rows[r] : r][c]) w[c] + b[c] (out null: the update alone; out16: rounded to bfloat16 as
+// well).  rows and y exclude each other.
 void launch_lay_add_tanh_norm(float* x, const int32_t* rows, const float* y, int nsum, const float* wsel, float mult, float alpha, const float* w,
-                              const float* b, float* out, int n_rows, int W, hipStream_t s);
+                              const float* b, float* out, int n_rows, int W, hipStream_t s, uint16_t* out16 = nullptr);
 // queries, keys and values of a pass between their projection and attention, one launch: causal convolution per channel (tails as in
 // LConvArgs), then on query and key heads the rotation by position and -- unit -- division by the head's root mean square; q -> rows of
 // their own, keys and values -> the sequence's pages.  G = 0: queries alone (keys and values are another layer's).

@@ -99,18 +99,18 @@ static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipSt
     // against 1955 (98 and 64 tiles, K 4096), but 128 rows 704 / 689 (52 and 32) and 2016 / 2022 (196 and 128), 700 rows 921 / 878, 2947 / 2916
     if (bf && L.shared_gemm && L.Abf && groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && !g.W2 && g.M > LAY_ROW_KERNEL_ROWS &&
         lay_tile_gemm_fits(g.N, g.K, 1) && (g.M < 32 || (size_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * 32 >= (size_t)g.K)) {
-        launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
+        if (!g.A16) launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
         LTileArgs t;
-        t.A = L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.N; t.K = g.K; t.bias = g.bias;
+        t.A = g.A16 ? g.A16 : L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.N; t.K = g.K; t.bias = g.bias;
         t.act = g.act; t.act2 = g.act2; t.act_split = g.act_split; t.act_param = g.act_param;
         launch_lay_tile_gemm(t, s);
         return;
     }
     if (bf && L.shared_gemm && L.Abf && groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && g.M >= 32 && g.N % 128 == 0 && g.K % 32 == 0 &&
         (!g.W2 || (g.ldc == g.N && L.G1 && L.G2))) {
-        launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
+        if (!g.A16) launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
         GemmArgs a{};
-        a.A_hi = L.Abf; a.A_lo = nullptr; a.W = g.W; a.bias = g.bias;
+        a.A_hi = g.A16 ? g.A16 : L.Abf; a.A_lo = nullptr; a.W = g.W; a.bias = g.bias;
         a.C = g.W2 ? L.G1 : g.C; a.ldc = g.W2 ? g.N : g.ldc;
         a.M = g.M; a.N = g.N; a.K = g.K; a.ws = m.pWS; a.ws_floats = m.pWS ? Model::gemm_ws_floats : 0; a.ksplit = 1; a.wide256 = m.gemm256;
         bool ok = launch_gemm(a, GEPI_STORE, s);
@@ -138,8 +138,9 @@ static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipSt
 
 // the experts of a pass over `T` rows of h (choices sorted by expert in L.srt / L.off, weights in L.wsel): their outputs, and those of the expert
 // that every token uses, into L.YS [token][slots][W].  bfloat16 format, more rows than the row kernel takes, sizes of whole k-tiles: the rows are
-// rounded once and everything runs on the tile kernel, the inner rows bfloat16 as the second product reads them
-static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const LayeredLayerW& w, const float* h, int T, int W, int slots, hipStream_t s) {
+// rounded once (h16: they are already) and everything runs on the tile kernel, the inner rows bfloat16 as the second product reads them
+static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const LayeredLayerW& w, const float* h, int T, int W, int slots, hipStream_t s,
+                        const uint16_t* h16 = nullptr) {
     LGemmArgs gu;
     gu.A = h; gu.lda = W; gu.a_idx = L.srt; gu.a_div = slots; gu.a_scale = sp.scale_input ? L.wsel : nullptr;
     gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
@@ -150,7 +151,7 @@ static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const Layered
     LGemmArgs su, sdn;
     const bool every = sp.shared_ff > 0 && slots > sp.top;
     if (every) {                           // row `top` of the token's rows
-        su.A = h; su.lda = W; su.W = w.sh_gate; su.W2 = w.sh_up; su.C = L.HS; su.ldc = sp.shared_ff; su.M = T; su.N = sp.shared_ff;
+        su.A = h; su.A16 = h16; su.lda = W; su.W = w.sh_gate; su.W2 = w.sh_up; su.C = L.HS; su.ldc = sp.shared_ff; su.M = T; su.N = sp.shared_ff;
         su.K = W; su.act = sp.expert_act; su.act_param = sp.shared_limit;
         sdn.A = L.HS; sdn.lda = sp.shared_ff; sdn.W = w.sh_down; sdn.C = L.YS + (size_t)sp.top * W; sdn.ldc = slots * W; sdn.M = T;
         sdn.N = W; sdn.K = sp.shared_ff;
@@ -166,14 +167,15 @@ static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const Layered
     };
     const bool routed = tiles && lay_tile_gemm_fits(sp.ff, W, sp.experts) && lay_tile_gemm_fits(W, sp.ff, sp.experts);
     const bool shared = tiles && every && lay_tile_gemm_fits(sp.shared_ff, W, 1) && lay_tile_gemm_fits(W, sp.shared_ff, 1);
-    if ((routed && !sp.scale_input) || shared) launch_lay_round_rows(h, W, L.Abf, T, W, s);
+    if (!h16 && ((routed && !sp.scale_input) || shared)) launch_lay_round_rows(h, W, L.Abf, T, W, s);
+    const uint16_t* A = h16 ? h16 : L.Abf;
     if (routed) {
         if (sp.scale_input) launch_lay_round_scaled(h, W, L.srt, slots, L.wsel, L.Asc, T * sp.top, W, s);
-        tile(gu, sp.scale_input ? L.Asc : L.Abf, !sp.scale_input);
+        tile(gu, sp.scale_input ? L.Asc : A, !sp.scale_input);
         tile(dn, (const uint16_t*)L.HH, false);
     }
     if (shared) {
-        tile(su, L.Abf, false);
+        tile(su, A, false);
         tile(sdn, (const uint16_t*)L.HS, false);
     }
     const bool beside = every && T <= LAY_ROW_KERNEL_ROWS;        // decode steps: the expert of every token rides in the same two launches
@@ -1727,10 +1729,15 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             launch_lay_canon(L.Hn, L.Hc, cw, conv_pool, conv_slot_elems, coff, d_segs, d_rowseg, T, W, L.taps, s);
             launch_lay_canon_tail(L.Hn, conv_pool, conv_slot_elems, coff, d_segs, nseg, W, L.taps, s);
         };
+        // the launches that make a product's input rows leave them in bfloat16 as well where the product would round them first (4 us a launch)
+        uint16_t* const rounded = !L.f32 && L.shared_gemm && T > LAY_ROW_KERNEL_ROWS ? L.Abf : nullptr;
+        const uint16_t *n16 = nullptr, *o16 = nullptr;                        // the last norm's and the last attention's rows, if they did
         // softmax attention of one layer over the pages: queries at qsrc[row ldq + q_off + head dk], output [T][H ev] into L.O
         auto run_attention = [&](const LayerSpec& sp, const LayeredLayerW& w, const float* qsrc, int ldq, int q_off, int g_off, int dk, int ev,
-                                 float* out = nullptr, int ldo = 0, float out_scale = 1.f, int v_div = 1, const float* gbuf = nullptr, int ldg = 0) {
+                                 float* out = nullptr, int ldo = 0, float out_scale = 1.f, int v_div = 1, const float* gbuf = nullptr, int ldg = 0,
+                                 uint16_t* out16 = nullptr) {
             LAttnArgs a;
+            o16 = nullptr;
             a.v_div = v_div; a.gbuf = gbuf; a.ldg = ldg;
             a.proj = qsrc; a.ldp = ldq; a.q_off = q_off; a.g_off = g_off;
             a.out = out ? out : L.O; a.ldo = out ? ldo : sp.heads * ev; a.out_scale = out_scale;
@@ -1757,10 +1764,11 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             if (L.attn_mfma && kv_mode == KV_BF16 && !all_decode && max_n >= 16 && lay_attn_mfma_fits(dk, ev, a.vpool != nullptr)) {
                 const auto& tm = tiles64[sp.heads / sp.kv_heads];
                 a.tiles = (const int2*)(L.d_tab + tm.first); a.ntiles = tm.second;
-                if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) launch_lay_attn_tile(a, s);
+                if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) { o16 = a.out16 = out16; launch_lay_attn_tile(a, s); }
                 else launch_lay_attn_mfma(a, s);
             } else if (L.attn_mfma && kv_mode == KV_BF16 && lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
                 a.nsplit = lay_attn_few_split(seen, a.ntiles * sp.kv_heads, Layered::ATT_PARTS);
+                o16 = a.out16 = out16;
                 launch_lay_attn_few(a, s);
             } else
                 launch_lay_attn(a, kv_mode, s);
@@ -1856,7 +1864,8 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         // pre-norm layers: the finished sublayer's rows (nsum per token, summed in order) join the residual inside the next norm's launch
         struct { const float* y = nullptr; int nsum = 1; const float* wsel = nullptr; } padd;
         auto add_norm = [&](const float* nw_, const float* off, float alpha, float* out) {
-            if (L.tanh_norm) launch_lay_add_tanh_norm(L.X, nullptr, padd.y, padd.nsum, padd.wsel, L.mult, alpha, nw_, off, out, T, W, s);
+            n16 = L.tanh_norm && out ? rounded : nullptr;
+            if (L.tanh_norm) launch_lay_add_tanh_norm(L.X, nullptr, padd.y, padd.nsum, padd.wsel, L.mult, alpha, nw_, off, out, T, W, s, out ? rounded : nullptr);
             else launch_lay_add_gnorm(L.X, nullptr, padd.y, padd.nsum, nw_, out, T, W, L.norm_groups, cfg.eps, s, padd.wsel);
             padd.y = nullptr; padd.wsel = nullptr;
         };
@@ -1931,11 +1940,12 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 // ---- x += mult mixer(norm1 x), x += mult ff(norm2 x); norms in equal parts, or of single elements
                 add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc);
                 LGemmArgs g;
-                g.A = L.Hc; g.lda = W; g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.K = W;
+                g.A = L.Hc; g.A16 = n16; g.lda = W; g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.K = W;
                 g.act_split = w.g_off; g.act = sp.mixer == LMIX_HGRN ? LACT_SILU : LACT_NONE;
                 g.act2 = sp.mixer == LMIX_ATTN && sp.gate != LGATE_NONE ? LACT_SIGMOID : LACT_NONE;
                 lay_gemm(*this, L, g, 1, s);
                 const float* oa = L.O;
+                const uint16_t* oa16 = nullptr;
                 int on = 0;
                 if (sp.mixer == LMIX_ATTN && sp.maps == 1) {
                     // convolution, rotation, unit heads and cache append in one launch (queries into rows of their own), then attention over
@@ -1955,8 +1965,8 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                         t.segs = d_segs; t.rowseg = d_rowseg;
                         launch_lay_conv_tail(t, nseg, s);
                     }
-                    run_attention(sp, w, L.XB, H * d, 0, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows);
-                    on = H * e;
+                    run_attention(sp, w, L.XB, H * d, 0, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows, rounded);
+                    on = H * e; oa16 = o16;
                 } else if (sp.mixer == LMIX_ATTN) {
                     // two maps per head as heads of their own (2 H query heads over 2 G key heads, pairs of key heads share a value head)
                     const int H = sp.heads, G = sp.kv_heads, d = sp.dim, e = sp.vdim;
@@ -2054,13 +2064,13 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     }
                 }
                 LGemmArgs go;
-                go.A = oa; go.lda = on; go.W = w.o_w; go.C = L.Y; go.ldc = W; go.M = T; go.N = W; go.K = on;
+                go.A = oa; go.A16 = oa16; go.lda = on; go.W = w.o_w; go.C = L.Y; go.ldc = W; go.M = T; go.N = W; go.K = on;
                 lay_gemm(*this, L, go, 1, s);
                 padd.y = L.Y; padd.nsum = 1;
                 if (sp.mlp == LMLP_DENSE) {
                     add_norm(w.norm2, w.norm2_off, w.norm2_alpha, L.Hc);
                     LGemmArgs gu;
-                    gu.A = L.Hc; gu.lda = W; gu.W = w.gate; gu.W2 = w.up; gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W;
+                    gu.A = L.Hc; gu.A16 = n16; gu.lda = W; gu.W = w.gate; gu.W2 = w.up; gu.C = L.HH; gu.ldc = sp.ff; gu.M = T; gu.N = sp.ff; gu.K = W;
                     gu.act = sp.ff_act; gu.act_param = sp.limit;
                     lay_gemm(*this, L, gu, 1, s);
                     LGemmArgs dn;
@@ -2073,7 +2083,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     // sum; otherwise the weights join in the combine
                     const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
                     route(L.Hc, w.router, sp.experts, sp.top, sp.router, nullptr, slots);
-                    lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s);
+                    lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s, n16);
                     padd.y = L.YS; padd.nsum = slots; padd.wsel = sp.scale_input ? nullptr : L.wsel;
                 }
                 if (L.capture || li + 1 == L.spec.size()) add_norm(nullptr, nullptr, 0.f, nullptr);
