@@ -432,8 +432,11 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a) {
 //     S_C = e^{G_C} S0 + K^T (e^{G_C - G} U)
 // gdn_chunk_prep_kernel (grid chunks x NV): A and P on v_mfma_f32_16x16x4_f32, (I + A)^-1 [.] by forward substitution (one
 // thread per column of [beta e^G K | beta V], its 64 unknowns in registers: no dependency between threads) -> W, U0, P, G.
-// gdn_chunk_scan_kernel (grid NV x V/16): the only sequential part -- three small matrix products per chunk over a 128 x 16
-// slice of the state (columns of S are independent).  Everything stays f32 (f32 MFMA: products and sums in f32), logs of the
+// gdn_chunk_scan_kernel (grid NV x V/16): the only sequential part -- U and the state's update, two small matrix products per chunk
+// over a 128 x 16 slice of the state (columns of S are independent); it leaves U and the state in front of every chunk to
+// gdn_chunk_out_kernel (grid chunks x NV), which forms Y and its gated norm for all chunks at once.  (Y inside the scan was half of
+// its products and most of its registers: 2048 + 2048 + 69 tokens, 16 heads, mean per launch: scan and norm 103.8 + 12.3 -> scan
+// 58.3, outputs 24.1 us.)  Everything stays f32 (f32 MFMA: products and sums in f32), logs of the
 // decays are summed, never multiplied (a decay of e^-80 per token underflows a running product after two tokens).
 // Same results as the sequential scan to f32 summation order (tests: prompts through both, logits < 1e-4).
 // ---------------------------------------------------------------------------------------------------------
@@ -458,7 +461,7 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& av, const f32x4& bv, f32x4 c
 }
 
 size_t gdn_chunk_prep_lds() { return (size_t)(2 * GDN_CK * CKP + GDN_CK * CTP + 2 * GDN_CK) * sizeof(float); }
-size_t gdn_chunk_scan_lds() { return (size_t)(16 * CKP + 2 * 16 * CTP + GDN_CK * CKP + GDN_CK) * sizeof(float); }
+size_t gdn_chunk_scan_lds() { return (size_t)(16 * CKP + 16 * CTP + GDN_CK * CKP + GDN_CK) * sizeof(float); }
 
 __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK;
@@ -594,10 +597,9 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK, VB = 16;
     extern __shared__ __attribute__((aligned(16))) float cl[];
     float (*St)[CKP] = (float (*)[CKP])cl;                              // state slice, transposed: [column][k]
-    float (*Ut)[CTP] = (float (*)[CTP])(cl + VB * CKP);                 // U of the chunk, transposed: [column][t]
-    float (*Vt)[CTP] = (float (*)[CTP])(cl + VB * CKP + VB * CTP);      // e^{G_C - G_t} U
-    float (*Ks)[CKP] = (float (*)[CKP])(cl + VB * CKP + 2 * VB * CTP);  // k^ rows of the chunk
-    float* lgs = cl + VB * CKP + 2 * VB * CTP + C * CKP;
+    float (*Vt)[CTP] = (float (*)[CTP])(cl + VB * CKP);                 // e^{G_C - G_t} U of the chunk, transposed: [column][t]
+    float (*Ks)[CKP] = (float (*)[CKP])(cl + VB * CKP + VB * CTP);      // k^ rows of the chunk
+    float* lgs = cl + VB * CKP + VB * CTP + C * CKP;
     const int h = blockIdx.x, cb = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, kq = lane >> 4;
     const int nk = a.NV / a.vpg, kh = a.chunked ? h % nk : h / a.vpg;
@@ -608,28 +610,20 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
         St[col][k] = Sg[k * V + VB * cb + col];
     }
     const int nchunks = (a.S + C - 1) / C;
-    // One wave per SIMD: nothing hides a load but the wave's own work, so the operands of chunk c + 1 (this wave's 16 rows of W,
-    // q^, P, its U0 values, its share of the k^ rows, the cumulative log decay) are requested into registers while chunk c is
-    // multiplied -- unconditionally (rows / chunks past the end are clamped and never consumed: DESIGN 3.13).
-    // Register sets: W / q^ rows (needed FIRST in a chunk) are requested TWO chunks ahead into two alternating sets, the rest
-    // (P rows, U0 values, k^ rows, cumulative log decay: needed later in the chunk) one chunk ahead.
-    f32x4 awA[8], aqA[8], awB[8], aqB[8], ap[4], kreg[8];
+    // One wave per SIMD: nothing hides a load but the wave's own work, so the operands of chunk c + 1 (this wave's 16 rows of W, its U0
+    // values, its share of the k^ rows, the cumulative log decay) are requested into registers while chunk c is multiplied --
+    // unconditionally (rows / chunks past the end are clamped and never consumed).
+    // Register sets: W rows (needed FIRST in a chunk) are requested TWO chunks ahead into two alternating sets, the rest one chunk ahead.
+    f32x4 awA[8], awB[8], kreg[8];
     float u0[4], glane = 0.f;
-    auto fetch_wq = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[8]) __attribute__((always_inline)) {
-        const int cc = min(c, nchunks - 1), t0 = cc * C;
-        const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
-        const int qrow = min(t0 + 16 * wave + r, a.S - 1);
+    auto fetch_w = [&](int c, f32x4 (&aw)[8]) __attribute__((always_inline)) {
+        const float* ck = a.ck + ((size_t)min(c, nchunks - 1) * a.NV + h) * GDN_CK_FLOATS;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            aw[j] = *(const f32x4*)(ck + (16 * wave + r) * 128 + 16 * j + 4 * kq);
-            aq[j] = *(const f32x4*)(a.pre_q + (size_t)qrow * a.key_dim + kh * K + 16 * j + 4 * kq);
-        }
+        for (int j = 0; j < 8; ++j) aw[j] = *(const f32x4*)(ck + (16 * wave + r) * 128 + 16 * j + 4 * kq);
     };
-    auto fetch_pu = [&](int c) __attribute__((always_inline)) {         // P rows + U0 values of chunk c (issued once the previous ones are consumed)
+    auto fetch_u = [&](int c) __attribute__((always_inline)) {          // U0 values of chunk c (issued once the previous ones are consumed)
         const int cc = min(c, nchunks - 1);
         const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ap[j] = *(const f32x4*)(ck + 2 * C * 128 + (16 * wave + r) * C + 16 * j + 4 * kq);
 #pragma unroll
         for (int i = 0; i < 4; ++i) u0[i] = ck[C * 128 + (16 * wave + 4 * kq + i) * 128 + VB * cb + r];
     };
@@ -652,47 +646,28 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
         }
         if (wave == 0) lgs[lane] = glane;
     };
-    auto chunk = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[8]) __attribute__((always_inline)) {
-        const int t0 = c * C, nt = min(C, a.S - t0);
+    auto chunk = [&](int c, f32x4 (&aw)[8]) __attribute__((always_inline)) {
+        float* ck = a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS;
         fetch_k(c + 1);
-        // ---- U = U0 - W S0 and Q S0 (same B operand): wave w owns token rows 16 w .. 16 w + 15 ----
-        f32x4 accU = {0.f, 0.f, 0.f, 0.f}, accQ = {0.f, 0.f, 0.f, 0.f};
+        // ---- U = U0 - W S0: wave w owns token rows 16 w .. 16 w + 15 ----
+        f32x4 accU = {0.f, 0.f, 0.f, 0.f}, accV = accU;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const f32x4 bs = *(const f32x4*)&St[r][16 * j + 4 * kq];
-            accU = mfma4(aw[j], bs, accU);
-            accQ = mfma4(aq[j], bs, accQ);
+        for (int j = 0; j < 8; j += 2) {
+            accU = mfma4(aw[j], *(const f32x4*)&St[r][16 * j + 4 * kq], accU);
+            accV = mfma4(aw[j + 1], *(const f32x4*)&St[r][16 * j + 16 + 4 * kq], accV);
         }
-        fetch_wq(c + 2, aw, aq);                       // this set is free again: the chunk after next
+        fetch_w(c + 2, aw);                            // this set is free again: the chunk after next
         const float gC = lgs[C - 1];
-        f32x4 u, ud, pc[4];
-        float eg[4];
+        f32x4 u, ud;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int t = 16 * wave + 4 * kq + i;
-            const float gt = lgs[t];
-            u[i] = u0[i] - accU[i];
-            ud[i] = u[i] * expf(gC - gt);
-            eg[i] = expf(gt);
+            u[i] = u0[i] - (accU[i] + accV[i]);
+            ud[i] = u[i] * expf(gC - lgs[16 * wave + 4 * kq + i]);
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) pc[j] = ap[j];
-        *(f32x4*)&Ut[r][16 * wave + 4 * kq] = u;
         *(f32x4*)&Vt[r][16 * wave + 4 * kq] = ud;
-        fetch_pu(c + 1);                               // (ap / u0 of this chunk are consumed or copied)
+        *(f32x4*)(ck + GDN_CK_UT + (VB * cb + r) * C + 16 * wave + 4 * kq) = u;
+        fetch_u(c + 1);                                // (u0 of this chunk is consumed)
         lds_barrier();
-        // ---- Y = e^G (Q S0) + P U ----
-        f32x4 accP = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f32x4 bu = *(const f32x4*)&Ut[r][16 * j + 4 * kq];
-            accP = mfma4(pc[j], bu, accP);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int t = 16 * wave + 4 * kq + i;
-            if (t < nt) a.out[(size_t)(t0 + t) * a.out_stride + h * V + VB * cb + r] = eg[i] * accQ[i] + accP[i];      // raw; gdn_post_kernel normalises
-        }
         // ---- S_C = e^{G_C} S0 + K^T (e^{G_C - G} U): wave w owns state rows k = 32 w .. 32 w + 31 ----
         f32x4 sn[2];
         const float eC = expf(gC);
@@ -712,26 +687,113 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) sn[mt][i] = eC * old[i] + accS[i];
         }
-        lds_barrier();                               // every read of St / Ut / Vt / Ks / lgs of this chunk is done
+        lds_barrier();                               // every read of St / Vt / Ks / lgs of this chunk is done
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) *(f32x4*)&St[r][32 * wave + 16 * mt + 4 * kq] = sn[mt];
+        for (int mt = 0; mt < 2; ++mt) {
+            *(f32x4*)&St[r][32 * wave + 16 * mt + 4 * kq] = sn[mt];
+            if (c + 1 < nchunks) *(f32x4*)(ck + (size_t)a.NV * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + r) * K + 32 * wave + 16 * mt + 4 * kq) = sn[mt];
+        }
         park_k(c + 1);
         lds_barrier();
     };
-    fetch_wq(0, awA, aqA);
-    fetch_pu(0);
+    fetch_w(0, awA);
+    fetch_u(0);
     fetch_k(0);
-    fetch_wq(1, awB, aqB);
+    fetch_w(1, awB);
     park_k(0);
     lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {                      // the state in front of chunk 0
+        const int e = (tid + 256 * i) * 4, col = e >> 7, k = e & 127;
+        *(f32x4*)(a.ck + (size_t)h * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + col) * K + k) = *(const f32x4*)&St[col][k];
+    }
     for (int c = 0; c < nchunks; c += 2) {
-        chunk(c, awA, aqA);
-        if (c + 1 < nchunks) chunk(c + 1, awB, aqB);
+        chunk(c, awA);
+        if (c + 1 < nchunks) chunk(c + 1, awB);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int e = tid + 256 * i, k = e >> 4, col = e & 15;
         Sg[k * V + VB * cb + col] = St[col][k];
+    }
+}
+
+// Y = e^G (Q S0) + P U of every chunk and the gated norm of its rows (gdn_post_kernel's), from the states and U rows the scan leaves.  Eight waves:
+// 16 token rows x 64 columns each.  Bound by its f32 matrix products (192 per wave, 32 cycles each) and the 150 KB a (chunk, head) reads; U and the
+// state share one LDS region, one after the other, so that two workgroups fit on a CU and one loads while the other multiplies (both at once: 29.2
+// for 24.1 us)
+constexpr size_t gdn_chunk_out_lds = (size_t)(128 * CKP + 128) * sizeof(float);
+__global__ __launch_bounds__(512, 4) void gdn_chunk_out_kernel(GdnArgs a) {
+    constexpr int K = 128, V = 128, C = GDN_CK;
+    extern __shared__ __attribute__((aligned(16))) float cl[];
+    float (*St)[CKP] = (float (*)[CKP])cl;                              // S0 transposed: [column][k]
+    float (*Ut)[CTP] = (float (*)[CTP])cl;                              // in front of it: U transposed: [column][t]
+    float (*red)[C] = (float (*)[C])(cl + 128 * CKP);                   // sums of squares of a row's two halves
+    const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, kq = lane >> 4, rt = wave & 3, hf = wave >> 2;
+    const int nk = a.NV / a.vpg, kh = a.chunked ? h % nk : h / a.vpg;
+    const int t0 = c * C, nt = min(C, a.S - t0);
+    const float* ck = a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS;
+    f32x4 p[4], q[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) { p[n] = (f32x4){0.f, 0.f, 0.f, 0.f}; q[n] = p[n]; }
+    f32x4 s[8];
+    {
+        f32x4 u[4], ap[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i] = *(const f32x4*)(ck + GDN_CK_UT + (tid + 512 * i) * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ap[j] = *(const f32x4*)(ck + 2 * C * 128 + (16 * rt + r) * C + 16 * j + 4 * kq);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = *(const f32x4*)(ck + GDN_CK_ST + (tid + 512 * i) * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { const int e = (tid + 512 * i) * 4; *(f32x4*)&Ut[e >> 6][e & 63] = u[i]; }
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) p[n] = mfma4(ap[j], *(const f32x4*)&Ut[64 * hf + 16 * n + r][16 * j + 4 * kq], p[n]);
+    }
+    f32x4 aq[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) aq[j] = *(const f32x4*)(a.pre_q + (size_t)min(t0 + 16 * rt + r, a.S - 1) * a.key_dim + kh * K + 16 * j + 4 * kq);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { const int e = (tid + 512 * i) * 4; *(f32x4*)&St[e >> 7][e & 127] = s[i]; }
+    lds_barrier();
+    // the gate's inputs, while the products run
+    const int conv_dim = 2 * a.key_dim + a.NV * V;
+    const f32x4 g = *(const f32x4*)(ck + 2 * C * 128 + C * C + 16 * rt + 4 * kq);
+    float z[4][4], gw[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const int v = 64 * hf + 16 * n + r;
+        gw[n] = a.gnorm_w[v];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[n][i] = a.proj[(size_t)min(t0 + 16 * rt + 4 * kq + i, a.S - 1) * a.proj_stride + conv_dim + h * V + v];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) q[n] = mfma4(aq[j], *(const f32x4*)&St[64 * hf + 16 * n + r][16 * j + 4 * kq], q[n]);
+    float y[4][4], ss[4] = {0.f, 0.f, 0.f, 0.f};                        // [row][column tile]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float eg = expf(g[i]);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) { y[i][n] = eg * q[n][i] + p[n][i]; ss[i] = fmaf(y[i][n], y[i][n], ss[i]); }
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) ss[i] += __shfl_xor(ss[i], o);
+        if (r == 0) red[hf][16 * rt + 4 * kq + i] = ss[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int t = 16 * rt + 4 * kq + i;
+        if (t >= nt) continue;
+        const float rms = 1.0f / sqrtf((red[0][t] + red[1][t]) / (float)V + a.eps);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) a.out[(size_t)(t0 + t) * a.out_stride + h * V + 64 * hf + 16 * n + r] = y[i][n] * rms * gw[n] * silu_f(z[n][i]);
     }
 }
 
@@ -762,10 +824,13 @@ void launch_gdn(const GdnArgs& a, hipStream_t s) {
             attr.run([&] {
                 (void)hipFuncSetAttribute((const void*)gdn_chunk_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_prep_lds());
                 (void)hipFuncSetAttribute((const void*)gdn_chunk_scan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_scan_lds());
+                (void)hipFuncSetAttribute((const void*)gdn_chunk_out_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_out_lds);
             });
             hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3((a.S + GDN_CK - 1) / GDN_CK, a.NV), dim3(256), gdn_chunk_prep_lds(), s, a);
             hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3(a.NV, 128 / 16), dim3(256), gdn_chunk_scan_lds(), s, a);
-        } else
+            hipLaunchKernelGGL(gdn_chunk_out_kernel, dim3((a.S + GDN_CK - 1) / GDN_CK, a.NV), dim3(512), gdn_chunk_out_lds, s, a);
+            return;
+        }
         hipLaunchKernelGGL(gdn_scan_kernel, dim3(a.NV, 4), dim3(512), 0, s, a);
         hipLaunchKernelGGL(gdn_post_kernel, dim3(a.S, a.NV), dim3(128), 0, s, a);
         return;
