@@ -69,6 +69,16 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
     const int quarter = hd / 4;
     std::vector<float> inv((size_t)quarter);
     for (int i = 0; i < quarter; ++i) inv[(size_t)i] = 1.0f / powf(10000.0f, (float)(2 * i) / (float)(hd / 2));   // vision.rs:285-297
+    // a row's angles depend on its grid row in the first half of a half head and on its grid column in the second: cosines and sines once per
+    // coordinate (3172 patches: 400 000 of them took as long as two blocks of the tower)
+    uint32_t coords = 0;
+    for (size_t g = 0; g < n_img; ++g) coords = std::max({coords, grid[3 * g + 1], grid[3 * g + 2]});
+    std::vector<float> tc((size_t)coords * quarter), ts((size_t)coords * quarter);
+    for (uint32_t x = 0; x < coords; ++x)
+        for (int i = 0; i < quarter; ++i) {
+            const float f = (float)(int)x * inv[(size_t)i];
+            tc[(size_t)x * quarter + i] = cosf(f); ts[(size_t)x * quarter + i] = sinf(f);
+        }
     std::vector<std::pair<int, int>> frames;      // [start, end) token ranges, one per temporal frame (vision.rs:543-556)
     int row = 0;
     for (size_t g = 0; g < n_img; ++g) {
@@ -88,10 +98,10 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
                     wts[0 * N + row] = (1.0f - dh) * (1.0f - dw); wts[1 * N + row] = (1.0f - dh) * dw;
                     wts[2 * N + row] = dh * (1.0f - dw); wts[3 * N + row] = dh * dw;
                     // (b) 2-D rotary: emb = cat(rot, rot), rot = [row freqs | col freqs] (vision.rs:491-541,565-569)
-                    for (int d = 0; d < hd; ++d) {
-                        const int e = d % (hd / 2);
-                        const float f = (e < quarter) ? (float)r * inv[(size_t)e] : (float)c * inv[(size_t)(e - quarter)];
-                        cs[(size_t)row * hd + d] = cosf(f); sn[(size_t)row * hd + d] = sinf(f);
+                    for (int part = 0; part < 4; ++part) {
+                        const size_t to = (size_t)row * hd + part * quarter, from = (size_t)(part % 2 ? c : r) * quarter;
+                        memcpy(&cs[to], &tc[from], quarter * sizeof(float));
+                        memcpy(&sn[to], &ts[from], quarter * sizeof(float));
                     }
                     ++row;
                 }
