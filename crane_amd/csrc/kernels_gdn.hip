@@ -287,61 +287,66 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs a) {
 // Prefill in three passes.  The fused kernel above walks a prompt with 4 barriers, two block reductions and a handful
 // of transcendental functions per token on ONE block per value head (~5 us per token and layer).  Everything except
 // the state recurrence is independent across tokens, so:
-//   gdn_pre_kernel  (grid S x (NK + NV)): conv + SiLU, L2 norms, q scale, beta, exp(g)  -> q^ k^ v beta decay per token
+//   gdn_pre_kernel  (a wave per head and 8 tokens): conv + SiLU, L2 norms, q scale, beta, exp(g)  -> q^ k^ v beta decay per token
 //   gdn_scan_kernel (grid NV x 4): the recurrence only; 16 lanes share a state column (8 of the 128 k each, partial
 //                   sums folded with one DPP row reduction), q^ / k^ of 8 tokens staged per barrier
 //   gdn_post_kernel (grid S x NV): gated RMSNorm of the raw y rows in place
 // Same per-token arithmetic as the fused kernel except for the association of the two 128-term sums over k.
 // ---------------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(128) void gdn_pre_kernel(GdnArgs a) {
-    constexpr int K = 128, V = 128, KER = 4;
-    __shared__ float red[4];
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// A wave takes one head (q, k or v; lane l its channels 2 l, 2 l + 1) over GDN_PT tokens: the convolution's window rolls in registers, a row is read
+// once instead of four times, norms need no other wave.  Bound by its traffic (a workgroup per token and head was bound by the 65 536 workgroups of a
+// 2048-token pass: mean per launch of a 4165-token prompt 31.7 -> 21.2 us).  The rolling window that the next call reads is written by the wave that read
+// the one of this call: both may be the same memory.
+constexpr int GDN_PT = 8;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__global__ __launch_bounds__(256) void gdn_pre_kernel(GdnArgs a) {
+    constexpr int K = 128, KER = 4;
+    const int lane = threadIdx.x & 63, item = (int)blockIdx.y * 4 + ((int)threadIdx.x >> 6), t0 = (int)blockIdx.x * GDN_PT;
     const int nk = a.NV / a.vpg;
-    const int conv_dim = 2 * a.key_dim + a.NV * V;
+    if (item >= 2 * nk + a.NV) return;
+    const int conv_dim = 2 * a.key_dim + a.NV * K;
+    const int c = item * K + 2 * lane;                   // channels: q heads, k heads, v heads
     const float* conv_state = a.conv_pool + ((size_t)a.slot * a.gdn_layers + a.layer_idx) * 2 * conv_dim * (KER - 1);
     const float* cs_in = conv_state + (size_t)(a.start_pos & 1) * conv_dim * (KER - 1);
-    float* cs_out = a.conv_pool + ((size_t)a.slot * a.gdn_layers + a.layer_idx) * 2 * conv_dim * (KER - 1) +
-                    (size_t)((a.start_pos + a.S) & 1) * conv_dim * (KER - 1);
-    // input of channel c at token tt (tt < 0: the rolling window left by the previous call, oldest first)
-    auto xin = [&](int c, int tt) -> float {
-        return tt >= 0 ? a.proj[(size_t)tt * a.proj_stride + c] : cs_in[c * (KER - 1) + (KER - 1) + tt];
-    };
-    auto conv = [&](int c) -> float {
-        const float x0 = xin(c, t - 3), x1 = xin(c, t - 2), x2 = xin(c, t - 1), x3 = xin(c, t);
-        const float* w = a.conv_w + c * KER;
-        return silu_f(x0 * w[0] + x1 * w[1] + x2 * w[2] + x3 * w[3]);
-    };
-    auto roll = [&](int c) {                         // the last token's block leaves the window for the next call
-        if (t == a.S - 1) {
+    const float* pc = a.proj + c;
+    f32x2 x[KER - 1 + GDN_PT];                           // inputs at tokens t0 - 3 ...
 #pragma unroll
-            for (int j = 0; j < KER - 1; ++j) cs_out[c * (KER - 1) + j] = xin(c, a.S - (KER - 1) + j);
+    for (int i = 0; i < KER - 1 + GDN_PT; ++i) x[i] = *(const f32x2*)(pc + (size_t)min(max(t0 + i - (KER - 1), 0), a.S - 1) * a.proj_stride);
+    const f32x4 w0 = *(const f32x4*)(a.conv_w + (size_t)c * KER), w1 = *(const f32x4*)(a.conv_w + (size_t)(c + 1) * KER);
+    if (t0 == 0) {
+#pragma unroll
+        for (int i = 0; i < KER - 1; ++i) x[i] = (f32x2){cs_in[c * (KER - 1) + i], cs_in[(c + 1) * (KER - 1) + i]};
+        float* cs_out = a.conv_pool + ((size_t)a.slot * a.gdn_layers + a.layer_idx) * 2 * conv_dim * (KER - 1) +
+                        (size_t)((a.start_pos + a.S) & 1) * conv_dim * (KER - 1);
+#pragma unroll
+        for (int i = 0; i < KER - 1; ++i) {              // (prompts of 16 tokens or more: the window lies in this pass)
+            const f32x2 v = *(const f32x2*)(pc + (size_t)(a.S - (KER - 1) + i) * a.proj_stride);
+            cs_out[c * (KER - 1) + i] = v[0]; cs_out[(c + 1) * (KER - 1) + i] = v[1];
         }
-    };
-    const float* pr = a.proj + (size_t)t * a.proj_stride;
-    if ((int)blockIdx.y < nk) {                      // q and k of key head kh
-        const int kh = blockIdx.y, cq = kh * K + tid, ck = a.key_dim + kh * K + tid;
-        float q = conv(cq), k = conv(ck);
-        const float sq = wave_sum(q * q), sk = wave_sum(k * k);
-        if (lane == 0) { red[wave] = sq; red[2 + wave] = sk; }
-        __syncthreads();
-        q = q / sqrtf(red[0] + red[1] + 1e-6f) * 0.08838834764831845f;      // 1/sqrt(128)
-        k = k / sqrtf(red[2] + red[3] + 1e-6f);
-        a.pre_q[(size_t)t * a.key_dim + cq] = q;
-        a.pre_k[(size_t)t * a.key_dim + kh * K + tid] = k;
-        roll(cq); roll(ck);
-    } else {                                         // v, beta, decay of value head h
-        const int h = blockIdx.y - nk, cv = 2 * a.key_dim + h * V + tid;
-        a.pre_v[((size_t)t * a.NV + h) * V + tid] = conv(cv);
-        if (tid == 0) {
-            const float beta = 1.0f / (1.0f + expf(-pr[conv_dim + a.NV * V + h]));
-            const float av = pr[conv_dim + a.NV * V + a.NV + h] + a.dt_bias[h];
-            const float g = -expf(a.A_log[h]) * logf(1.0f + expf(av));
-            a.pre_bd[((size_t)t * a.NV + h) * 2] = beta;
-            a.pre_bd[((size_t)t * a.NV + h) * 2 + 1] = expf(g);
-            if (a.pre_g != nullptr) a.pre_g[(size_t)t * a.NV + h] = g;
+    }
+    const int kind = item < nk ? 0 : item < 2 * nk ? 1 : 2;
+    float* dst = kind == 0 ? a.pre_q + c : kind == 1 ? a.pre_k + (c - a.key_dim) : a.pre_v + (c - 2 * a.key_dim);
+    const size_t ldd = kind == 2 ? (size_t)a.NV * K : (size_t)a.key_dim;
+#pragma unroll
+    for (int i = 0; i < GDN_PT; ++i) {
+        f32x2 y = {silu_f(x[i][0] * w0[0] + x[i + 1][0] * w0[1] + x[i + 2][0] * w0[2] + x[i + 3][0] * w0[3]),
+                   silu_f(x[i][1] * w1[0] + x[i + 1][1] * w1[1] + x[i + 2][1] * w1[2] + x[i + 3][1] * w1[3])};
+        if (kind < 2) {                                  // (a wave's own branch)
+            const float n = sqrtf(wave_sum(y[0] * y[0] + y[1] * y[1]) + 1e-6f);
+            y[0] = y[0] / n; y[1] = y[1] / n;
+            if (kind == 0) { y[0] *= 0.08838834764831845f; y[1] *= 0.08838834764831845f; }      // 1 / sqrt(128)
         }
-        roll(cv);
+        if (t0 + i < a.S) *(f32x2*)(dst + (size_t)(t0 + i) * ldd) = y;
+    }
+    if (kind == 2 && lane < GDN_PT && t0 + lane < a.S) { // beta and decay of the value head, a token per lane
+        const int h = item - 2 * nk, t = t0 + lane;
+        const float* pr = a.proj + (size_t)t * a.proj_stride;
+        const float beta = 1.0f / (1.0f + expf(-pr[conv_dim + a.NV * K + h]));
+        const float av = pr[conv_dim + a.NV * K + a.NV + h] + a.dt_bias[h];
+        const float g = -expf(a.A_log[h]) * logf(1.0f + expf(av));
+        a.pre_bd[((size_t)t * a.NV + h) * 2] = beta;
+        a.pre_bd[((size_t)t * a.NV + h) * 2 + 1] = expf(g);
+        if (a.pre_g != nullptr) a.pre_g[(size_t)t * a.NV + h] = g;
     }
 }
 
@@ -816,7 +821,7 @@ void launch_gdn(const GdnArgs& a, hipStream_t s) {
     // prompts: three passes (needs the scratch rows of ensure_prefill_buffers); decode steps and short tails: fused
     if (a.st == nullptr && a.pre_q != nullptr && a.S >= 16 && a.n_seq <= 1) {
         const int nk = a.NV / a.vpg;
-        hipLaunchKernelGGL(gdn_pre_kernel, dim3(a.S, nk + a.NV), dim3(128), 0, s, a);
+        hipLaunchKernelGGL(gdn_pre_kernel, dim3((a.S + GDN_PT - 1) / GDN_PT, (2 * nk + a.NV + 3) / 4), dim3(256), 0, s, a);
         // prompts of a chunk or more: the chunk-parallel scan on the f32 matrix cores (CM_GDN_CHUNKED=0: the sequential scan, A/B)
         static const int ck_env = getenv("CM_GDN_CHUNKED") ? atoi(getenv("CM_GDN_CHUNKED")) : 1;
         if (a.ck != nullptr && a.pre_g != nullptr && ck_env != 0 && a.S >= GDN_CK) {
