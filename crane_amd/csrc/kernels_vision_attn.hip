@@ -9,7 +9,7 @@
 // bank: 0 conflicts); a wave owns 32 rows where there are enough of them and uses every fragment twice; two 16-key groups of P^T go into one
 // 16 x 16 x 32 product, which takes as long as a 16 x 16 x 16 one (the order of the keys inside the product is the same permutation on both
 // operands).  All frames in one launch instead of one launch per frame with two runs of keys and a merge: 42 x 64 and 22 x 22 patches, 16 heads
-// 174 -> 127 us per block of the tower, six images of 22 x 22 patches: tower 10.6 -> 8.2 ms.  Measured and no better: the next tile's scores issued
+// 174 -> 114 us per block of the tower (two runs of keys and their merge; 127 in one run), six images of 22 x 22 patches: tower 10.6 -> 8.2 ms.  Measured and no better: the next tile's scores issued
 // between this tile's exponentials (registers), eight waves of 16 rows (registers).
 #include "dev_common.h"
 #include "kernels.h"
