@@ -40,7 +40,7 @@ __device__ __forceinline__ void store4(uint16_t* hi, uint16_t* lo, size_t at, co
     *(u32x2*)(lo + at) = (u32x2){l[0], l[1]};
 }
 
-// grid (heads, tiles, runs): the workgroups of a head follow each other by `heads`, so that its K / V stay in one XCD's L2 where heads % 8 == 0
+// grid (heads x tiles, runs), heads first: the workgroups of a head follow each other by `heads`, so that its K / V stay in one XCD's L2 where heads % 8 == 0
 template <int NQ>
 __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
     constexpr int PLANE = KT * D, STAGE = 4 * PLANE;                   // K hi, K lo, V hi, V lo
@@ -49,8 +49,8 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = lane & 15, g = lane >> 4;
-    const int h = blockIdx.x, heads = a.heads;
-    const int4 tl = a.tiles[blockIdx.y];                               // first and end row of the frame, first query row
+    const int heads = a.heads, h = (int)blockIdx.x % heads;
+    const int4 tl = a.tiles[(int)blockIdx.x / heads];                               // first and end row of the frame, first query row
     const int lo = tl.x, end = tl.y;
     bf16x8 qh[NQ][2], ql[NQ][2];
 #pragma unroll
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
         for (int nt = 0; nt < 4; ++nt) o[n][nt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     const int all = (end - lo + KT - 1) / KT, full = (end - lo) / KT, per = (all + a.runs - 1) / a.runs;
-    const int t0 = (int)blockIdx.z * per, t1 = min(all, t0 + per);     // this workgroup's run of key tiles (may be empty)
+    const int t0 = (int)blockIdx.y * per, t1 = min(all, t0 + per);     // this workgroup's run of key tiles (may be empty)
     // wave w brings plane w of a tile: eight requests of eight rows.  A row's address moves on by one 64-row block per tile
     const uint16_t* const plane = (wave < 2 ? a.k : a.v) + (wave & 1 ? a.lo_off : 0);
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds + (uint32_t)wave * PLANE * 2u;
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
         const int row = tl.z + (wave * NQ + n) * 16 + sub;
         if (row >= end) continue;
         if (a.runs > 1) {                                              // un-normalised; an empty run: maximum -inf, sum 0
-            const size_t at = ((size_t)blockIdx.z * a.rows + row) * heads + h;
+            const size_t at = ((size_t)blockIdx.y * a.rows + row) * heads + h;
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) *(f32x4*)(a.part_o + at * D + nt * 16 + g * 4) = o[n][nt];
             if (g == 0) { a.part_ml[at * 2] = m_run[n]; a.part_ml[at * 2 + 1] = l; }
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void vit_attn_merge_kernel(VitAttnArgs a) {
 }  // namespace
 
 void launch_vit_attn(const VitAttnArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)a.heads, (unsigned)a.ntiles, (unsigned)a.runs);
+    const dim3 grid((unsigned)a.heads * (unsigned)a.ntiles, (unsigned)a.runs);
     if (a.wide) hipLaunchKernelGGL(vit_attn_kernel<2>, grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL(vit_attn_kernel<1>, grid, dim3(256), 0, s, a);
     if (a.runs > 1) {
