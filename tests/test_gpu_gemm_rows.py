@@ -28,8 +28,9 @@ def _close(got, want):
 
 # prompts: rows below, at and above each tile height; K of an odd number of k-tiles (320 = 5), widths that split K 2, 4 and 8 ways, widths of more
 # than 256 column tiles that fill their last round (I 62208: 972 of 1024) and that do not (I 17408: 272 of 512)
+# rows of 1280 and 5120 columns: reductions with their norm in a part of a 1024-thread workgroup and in a loop of one;
 # (1024, 3072): qkv and gate_up of 6144 columns, 96 per workgroup; (128, 49152): 1024 workgroups of 96
-@pytest.mark.parametrize("H,I,heads,kv", [(640, 320, 4, 2), (1024, 2048, 8, 8), (384, 17408, 6, 2), (128, 62208, 2, 1), (1024, 3072, 24, 12), (128, 49152, 2, 1)])
+@pytest.mark.parametrize("H,I,heads,kv", [(640, 320, 4, 2), (1024, 2048, 8, 8), (384, 17408, 6, 2), (128, 62208, 2, 1), (1024, 3072, 24, 12), (128, 49152, 2, 1), (1280, 2048, 8, 2), (5120, 1024, 8, 2)])
 def test_prompts(H, I, heads, kv):
     m = _model(H, I, heads, kv, 512, max_seqs=2)
     rng = np.random.default_rng(1)
