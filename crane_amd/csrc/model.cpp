@@ -2004,11 +2004,7 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
             } else {
                 // (the attention path of this group, decided here because the qkv projection may leave its K-split slices to it)
                 const bool full_b = Hkv_l * nb >= 2 * num_cu;
-                // (f16 pages over bf16 weights: also where the group's tokens together are many -- q and p as f16 hi + lo carry the 22 bits that f16
-                // keys and values leave of a product.  Four rounds of Qwen3-8B, VALU / matrix cores: 32 sequences up to 700 tokens 23.0 / 20.9 ms, up to
-                // 200 20.2 / 19.7, 9 up to 700 18.4 / 17.8, 3 up to 700 16.9 / 16.8; even at 24 x 80 and 9 x 200, behind at 9 x 80)
-                const bool many_b = !quantized && kv_mode == KV_F16 && D == 128 && (int64_t)nb * longest >= 2048;
-                const int64_t mf_min = (full_b || many_b) && attn_mfma_min > 0 ? std::min<int64_t>(attn_mfma_min, attn_mfma_min_batch) : attn_mfma_min;
+                const int64_t mf_min = full_b && attn_mfma_min > 0 ? std::min<int64_t>(attn_mfma_min, attn_mfma_min_batch) : attn_mfma_min;
                 const bool mf = mf_min > 0 && longest >= mf_min && kv_mode != KV_F32 && (D == 128 || D == 256) && (page & (page - 1)) == 0;
                 // nb sequences already multiply the block count: fewer token splits per sequence keep ~2 blocks per CU
                 const int ns_b = mf ? std::max(attn_batch_ns_min, std::min(longest >= attn_mfma_wide_min ? nsplit_mfma : nsplit, 2 * num_cu / std::max(1, Hkv_l * nb)))

@@ -65,3 +65,16 @@ def test_planes(model, rows, ctx):
         assert np.isfinite(got).all() and np.abs(got - want).max() < 2e-3 * np.abs(want).max()
     finally:
         m.close()
+
+
+# groups that do not fill the chip, contexts below the matrix-core kernel's 768 tokens: queries, weights and their products in f32 like a single
+# sequence's (the matrix cores take f16 hi + lo pairs, 22 bits at most) -- the logits are those with that kernel switched off, bit for bit
+@pytest.mark.parametrize("rows,ctx", [(3, 700), (9, 300), (33, 70)])
+def test_short_contexts_keep_32_bit_queries_and_weights(rows, ctx):
+    from crane_amd.backend import Model
+    m = Model.synthetic(dict(configs.get_config("qwen3-0.6b"), vocab_size=512, num_hidden_layers=2), seed=3, max_seq_len=768, max_seqs=rows + 1)
+    try:
+        a, b = _logits(m, rows, ctx, [("attn_mfma_min", 768), ("attn_mfma_min", 0)])
+        assert np.isfinite(a).all() and (a == b).all()
+    finally:
+        m.close()
