@@ -77,8 +77,14 @@ __device__ __forceinline__ void query8(const float* src, int c, int d, bool ok, 
     }
 }
 
-// a lane's query (column lane % 16 of the transposed scores) and its running softmax.  PARTS: bfloat16 parts of a weight
+// a lane's query (column lane % 16 of the transposed scores) and its running softmax.  PARTS: bfloat16 parts of a weight.  Two parts (prompt
+// passes): scores in units of log 2, exp2 and log of the hardware units.  Three (decode steps): lay_attn_kernel's functions -- expf, and log1pf,
+// which keeps the low bits of a small r2 * distance that 1 + x drops (r1 = 1e6, r2 = 1e-7: weights 5 % off with the hardware's log of 1 + x)
+template <int PARTS>
 struct Query {
+    static constexpr bool EXACT = PARTS == 3;
+    static constexpr float UNIT = EXACT ? 1.f : L2E;
+    static __device__ __forceinline__ float ex(float x) { return EXACT ? expf(x) : __builtin_amdgcn_exp2f(x); }
     bool ok;
     int pos, head, row, clo;
     float r1, r2, m, l;
@@ -90,16 +96,16 @@ struct Query {
         row = sg.row0 + lp;
         pos = ok ? sg.start_pos + lp : -1;
         clo = chunk > 0 && ok ? pos / chunk * chunk : 0;
-        r1 = a.bias != LBIAS_NONE ? a.r1[head] * L2E : 0.f;
+        r1 = a.bias != LBIAS_NONE ? a.r1[head] * UNIT : 0.f;
         r2 = a.bias == LBIAS_LOG ? a.r2[head] : 0.f;
         m = -INFINITY; l = 0.f;
-        if (a.sink && ok && first) { m = a.sink[head] * L2E; l = lg == 0 ? 1.f : 0.f; }     // the four lane groups' sums meet at the end
+        if (a.sink && ok && first) { m = a.sink[head] * UNIT; l = lg == 0 ? 1.f : 0.f; }     // the four lane groups' sums meet at the end
     }
     // scores of tile t (products in s, keys 16 tt + 4 lg + r) -> weights in PARTS bfloat16 parts, the running pair moved on, o rescaled when a
     // new maximum appears in the wave.  p[..][h]: keys 16 (2 h) + 4 lg + 0 .. 3, then 16 (2 h + 1) + 4 lg + 0 .. 3
-    template <bool POOL, int PARTS, int NNT>
+    template <bool POOL, int NNT>
     __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int lg, f32x4 (&s)[4], bf16x8 (&p)[PARTS][2], f32x4 (&o)[NNT]) {
-        const float scale = a.scale * L2E;             // scores in units of log 2
+        const float scale = a.scale * UNIT;
         const int j0 = w.first(t);
         const bool blk = POOL && t < w.front;
         const bool full = t >= w.front && j0 >= w.vis_lo && j0 + KT - 1 <= w.pmin;
@@ -126,14 +132,17 @@ struct Query {
             const auto window = [&](int j, int dist) { return (bool)((dist >= 0) & (((dist < w.win) & (j >= clo)) | (j < w.keep))); };
             if (blk) each([](int) { return 0.f; }, [&](int j, int) { return (bool)((j < w.blocks) & ((j + 1) * w.pool <= pos - w.win + 1)); });
             else if (a.bias == LBIAS_NONE) each([](int) { return 0.f; }, window);
-            else if (a.bias == LBIAS_LOG) each([&](int dist) { return r1 * __logf(1.f + r2 * (float)max(dist, 0)); }, window);   // (absolute error 1e-7)
+            else if (a.bias == LBIAS_LOG) each([&](int dist) {
+                const float x = r2 * (float)max(dist, 0);
+                return r1 * (EXACT ? log1pf(x) : __logf(1.f + x));
+            }, window);
             else each([&](int dist) { return r1 * (float)dist; }, window);
         }
         mt = fmaxf(mt, __shfl_xor(mt, 16));
         mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.f : mn;    // nothing seen so far: every weight is exp2(-inf) = 0
+        const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.f : mn;    // nothing seen so far: every weight is exp(-inf) = 0
         if (__any(mn > m)) {
-            const float corr = __builtin_amdgcn_exp2f(m - ms);
+            const float corr = ex(m - ms);
             l *= corr;
 #pragma unroll
             for (int n = 0; n < NNT; ++n)
@@ -147,8 +156,8 @@ struct Query {
             u32x4 part[PARTS];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float p0 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1)] - ms);
-                float p1 = __builtin_amdgcn_exp2f(s[2 * h + (q >> 1)][2 * (q & 1) + 1] - ms);
+                float p0 = ex(s[2 * h + (q >> 1)][2 * (q & 1)] - ms);
+                float p1 = ex(s[2 * h + (q >> 1)][2 * (q & 1) + 1] - ms);
                 psum += p0 + p1;
 #pragma unroll
                 for (int k = 0; k < PARTS; ++k) {
@@ -222,7 +231,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     const int q0 = tile_id.y, nq = min(64, sg.n * nrep - q0);
     Walk w;
     w.init<POOL>(a, sg, q0, nq, nrep);
-    Query q;
+    Query<2> q;
     q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk, lg, grp == 0);
     bf16x8 qf[NKS];                                    // rounded once
 #pragma unroll
@@ -362,7 +371,7 @@ void go(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
 // fragments, values through a private LDS tile (no barrier inside the walk); a tile's keys are requested as soon as the one before has been
 // multiplied, its values as soon as the one before is in LDS.  The eight waves' sums meet in LDS once; gridDim.z > 1: they leave a partial
 // sum for lay_attn_merge_kernel instead.  Queries and weights keep their 24 bits, as in lay_attn_kernel: three bfloat16 parts each, three
-// products per tile (the launch waits for memory, not for the matrix cores).
+// products per tile (the launch waits for memory, not for the matrix cores), and its exponential and logarithm.
 constexpr int DW = 8;
 template <int DP, int EP, bool POOL>
 __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
@@ -381,7 +390,7 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
     Walk w;
     w.init<POOL>(a, sg, q0, nq, nrep);
     const int t_first = (int)blockIdx.z * DW + wave, t_step = DW * (int)gridDim.z;
-    Query q;
+    Query<3> q;
     q.init(a, sg, g, lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
     int pgs_grp = 0;                                   // lane i: page of this wave's tile 64 grp + i
     auto load_pages = [&](int grp) __attribute__((always_inline)) {
@@ -481,10 +490,10 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
     for (int k = 0; k < DW; ++k) M = fmaxf(M, pm[k][lr]);
     const float ms = M == -INFINITY ? 0.f : M;
 #pragma unroll
-    for (int k = 0; k < DW; ++k) { cw[k] = __builtin_amdgcn_exp2f(pm[k][lr] - ms); L = fmaf(pl_[k][lr], cw[k], L); }
+    for (int k = 0; k < DW; ++k) { cw[k] = expf(pm[k][lr] - ms); L = fmaf(pl_[k][lr], cw[k], L); }
     const int nsplit = (int)gridDim.z;
     const size_t pr = (((size_t)blockIdx.y * a.G + g) * nsplit + blockIdx.z) * 16 + lr;
-    if (nsplit > 1 && wave == 0 && lg == 0) { a.part_ml[pr * 2] = M * 0.6931471805599453f; a.part_ml[pr * 2 + 1] = L; }     // the merge works in e
+    if (nsplit > 1 && wave == 0 && lg == 0) { a.part_ml[pr * 2] = M; a.part_ml[pr * 2 + 1] = L; }
     for (int n = wave; n < NNT; n += DW) {
         const int c = n * 16 + lg * 4;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};

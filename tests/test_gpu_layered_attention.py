@@ -7,6 +7,8 @@ that moves a score by 2^-9 / sqrt(3) = 1.1e-3 in the mean square (d independent 
 same share and the largest logit by no more; everything else (weights as a 16-bit hi + lo pair, exp and log of the hardware units, the
 bfloat16 rounding of the attention rows on their way into the output projection, which tips 0.3 % of the elements over) is below 3e-4.
 8e-3 of the largest logit is seven times that."""
+import types
+
 import numpy as np
 import pytest
 
@@ -135,6 +137,19 @@ def test_decode_window_and_one_in_the_denominator(tmp_path, d, e, heads, kv, siz
 def test_decode_kept_first_tokens_and_distance_term(tmp_path, d, heads, kv, size, keep, contexts):
     mx = KO.attn(heads=heads, kv_heads=kv, dim=d, size=size, keep_first=keep)
     _few(tmp_path, KO, KO.config([KO.layer("attention", None, **mx)], vocab=96, width=64), contexts, (1, 1, 4), 15)
+
+
+# a steep distance term of small arguments, r1 log(1 + r2 dist) with r2 dist down to 1e-7: 1 + x in f32 is 6e-8 off, times r1 = 1e6 a score by 0.06 and
+# its weight by 6 %; log1p keeps both sides at 1e-7 of the term
+def test_decode_distance_term_of_small_arguments(tmp_path):
+    def weights(cfg, seed):
+        P = KO.random_weights(cfg, seed)
+        P["l0.mix.r1"][:] = KO.bf16_round(np.full_like(P["l0.mix.r1"], 1e6))
+        P["l0.mix.r2"][:] = KO.bf16_round(np.full_like(P["l0.mix.r2"], 1e-7))
+        return P
+    U = types.SimpleNamespace(random_weights=weights, tokens=KO.tokens, write_checkpoint=KO.write_checkpoint)
+    mx = KO.attn(heads=4, kv_heads=2, dim=32, size=1000, keep_first=3)
+    _few(tmp_path, U, KO.config([KO.layer("attention", None, **mx)], vocab=96, width=64), (5, 150, 400), (1, 1, 4), 21)
 
 
 @pytest.mark.parametrize("d,e,heads,kv,size,contexts", [(32, 16, 6, 2, 50, (49, 99, 100)), (128, 112, 4, 2, 64, (63, 64, 500)), (64, 64, 2, 2, 3000, (2999, 1, 2000))])
