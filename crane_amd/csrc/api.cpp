@@ -569,6 +569,14 @@ int cm_debug_qgemm_plan(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t w
     return CM_OK;
 }
 
+// test hook: the route of a decode step's router (pure host logic)
+int cm_debug_lay_router_plan(int32_t rows, int32_t width, int32_t outputs, int32_t top, int32_t shared_gate, int32_t offset) {
+    cm::RouterSpec rs;
+    rs.shared_gate = shared_gate != 0;
+    const uintptr_t at = (uintptr_t)4096 + (uintptr_t)offset;
+    return cm::lay_router_decode_fits((const float*)at, (const uint16_t*)at, rows, width, outputs, top, rs);
+}
+
 int cm_debug_set(cm_model* h, const char* key, int64_t value) {
     if (!h || !key) return CM_ERR_INVALID;
     return guard_all(h, [&](Model& mm, bool) {

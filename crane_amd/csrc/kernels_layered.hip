@@ -2167,8 +2167,9 @@ void launch_lay_moe_plan(const int32_t* sel, int32_t* off, int32_t* srt, int n, 
     hipLaunchKernelGGL(lay_moe_plan_kernel, dim3(1), dim3(1024), (size_t)E * sizeof(int), s, sel, off, srt, n, E, top, slots);
 }
 
-// decode steps: router logits, choice and plan in one block (three launches of 4.3, 5.6 and 2.6 us, each waiting for the one before, as one of
-// 7.9).  A wave per (token, logit) in lgemv_kernel's order of additions, a wave per token for the choice, the rows of an expert in token order
+// decode steps: router logits, choice and plan in one block, where three launches (streaming row kernel, choice, plan) wait for each other.  A wave per
+// (token, logit) in lgemv_kernel's order of additions, a wave per token for the choice, the rows of an expert in token order.  us, one block / three
+// launches, 4 of 14 + 1 logits: 1 row of 1024 7.3 / 11.0, 8 rows of 1024 14.3 / 18.6, 1 row of 4096 10.4 / 15.0
 __global__ __launch_bounds__(1024) void lay_router_decode_kernel(const float* __restrict__ h, const uint16_t* __restrict__ wr, int32_t* __restrict__ sel,
                                                                  float* __restrict__ wsel, int32_t* __restrict__ off, int32_t* __restrict__ srt, int T,
                                                                  int W, int E, int top, RouterSpec rs, const float* __restrict__ correction, int slots,
@@ -2214,9 +2215,15 @@ __global__ __launch_bounds__(1024) void lay_router_decode_kernel(const float* __
         off[e] = before;
     }
 }
-bool lay_router_decode_fits(int T, int W, int E, int top, const RouterSpec& rs) {
-    const size_t per_tok = (size_t)2 * E + (rs.shared_gate ? 1 : 0) + rs.groups + top;
-    return T <= LAY_ROW_KERNEL_ROWS && W % 8 == 0 && top <= 64 && (size_t)T * (per_tok + top) * sizeof(float) <= LDS_PLAIN;
+// One CU makes all T x n dot products of width W; the streaming kernel spreads the logits over the chip, eight to a block, and two launches more wait and
+// are waited for.  us a layer in steps of four-layer models, one launch / three, on both sides of the lines (W, n, T): up to 17 logits one is ahead
+// as far as measured (4096, 17, 1: 124.1 / 129.2; 8: 345.2 / 348.7), up to 33 to 2^18 products (1024, 25, 8: 122.4 / 124.5; 4096, 33, 1: 130.5 / 131.3 |
+// 2048, 33, 8: 193.7 / 188.0), more to 2^17 (512, 129, 1: 64.1 / 65.9; 2048, 49, 1: 82.7 / 85.3 | 1024, 129, 1: 73.8 / 73.5; 512, 49, 8: 107.3 /
+// 105.0; 4096, 65, 8: 467 / 413)
+bool lay_router_decode_fits(const float* h, const uint16_t* wr, int T, int W, int E, int top, const RouterSpec& rs) {
+    const size_t n = (size_t)E + (rs.shared_gate ? 1 : 0), per_tok = n + E + rs.groups + top;
+    return T <= LAY_ROW_KERNEL_ROWS && W % 8 == 0 && (((uintptr_t)h | (uintptr_t)wr) & 15) == 0 && top <= 64 &&
+           (size_t)T * (per_tok + top) * sizeof(float) <= LDS_PLAIN && (size_t)T * n * W <= (n <= 17 ? n << 15 : n <= 33 ? (size_t)1 << 18 : (size_t)1 << 17);
 }
 void launch_lay_router_decode(const float* h, const uint16_t* wr, int32_t* sel, float* wsel, int32_t* off, int32_t* srt, int T, int W, int E, int top,
                               hipStream_t s, const RouterSpec& rs, const float* correction, int slots) {

@@ -315,7 +315,7 @@ void launch_lay_qk_prep(float* proj, int ldp, int q_off, int k_off, int v_off, i
                         const LaySegDev* segs, const int32_t* rowseg, int T, int page, hipStream_t s, int pool = 0, int pool_rows = 0,
                         void* pk_pool = nullptr, void* pv_pool = nullptr, const LQkPrepExtra* extra = nullptr);
 // decode steps (at most LAY_ROW_KERNEL_ROWS rows): logits, choice and the rows sorted by expert in one launch (lay_router_decode_fits)
-bool lay_router_decode_fits(int T, int W, int E, int top, const RouterSpec& rs);
+bool lay_router_decode_fits(const float* h, const uint16_t* wr, int T, int W, int E, int top, const RouterSpec& rs);
 void launch_lay_router_decode(const float* h, const uint16_t* wr, int32_t* sel, float* wsel, int32_t* off, int32_t* srt, int T, int W, int E, int top,
                               hipStream_t s, const RouterSpec& rs, const float* correction, int slots);
 inline int lay_pool_rows(int page, long long pool) { return pool >= page ? 1 : (int)((page + pool - 1) / pool); }

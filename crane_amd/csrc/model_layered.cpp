@@ -1871,7 +1871,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         };
         // choices and weights of every row of h, and the rows sorted by expert
         auto route = [&](const float* h, const uint16_t* wr, int outs, int top, const RouterSpec& rs, const float* correction, int slots) {
-            if (lay_router_decode_fits(T, W, outs, top, rs)) {
+            if (lay_router_decode_fits(h, wr, T, W, outs, top, rs)) {
                 launch_lay_router_decode(h, wr, L.sel, L.wsel, L.off, L.srt, T, W, outs, top, s, rs, correction, slots);
                 return;
             }

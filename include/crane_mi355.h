@@ -517,6 +517,11 @@ long cm_debug_peer_selftest(int32_t n_ranks, int32_t device, int32_t iters, int3
  * rows per workgroup, 32-blocks per K group, K groups, K split, workgroups }.  Slice i of the split covers groups [i G / ks, (i + 1) G / ks). */
 int cm_debug_qgemm_plan(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats, int32_t num_cu, int64_t out[8]);
 
+/* Test hook (host logic only, no GPU): whether a step of `rows` tokens of a layer-list decoder makes its router's logits (`outputs`, and one more with
+ * `shared_gate`), the choice of `top` and the plan in one launch: 1, or in three: 0.  The rows and the matrix begin `offset` bytes behind a
+ * 16-byte boundary. */
+int cm_debug_lay_router_plan(int32_t rows, int32_t width, int32_t outputs, int32_t top, int32_t shared_gate, int32_t offset);
+
 /* Test hook: flips a path switch of a live model (the environment switches of the same names are read once, at
  * cm_create).  "no_prefill" = 1: prompts run token by token through the decode kernels; "quant_prefill" = 0: prompts over
  * quantised weights run through the integer-dot decode kernels instead of the dequantised MFMA GEMMs; "attn_outq" = 0 / 1: the single-split matrix-core

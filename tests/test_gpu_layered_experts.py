@@ -90,3 +90,20 @@ def test_router_rows(tmp_path, experts, shared, n):
     # for one position in a thousand
     off = np.abs(got - want).max(-1) / np.abs(want).max()
     assert np.quantile(off, 0.998) < 1e-4, (float(off.max()), int(off.argmax()))
+
+
+# 8 rows, 71 logits of width 256: more products than one CU is given (tests/test_lay_router_plan.py), logits by the streaming row kernel
+def test_router_of_eight_rows_on_the_whole_chip(tmp_path):
+    from crane_amd import _lib
+    from crane_amd.backend import Model
+    assert _lib.load().cm_debug_lay_router_plan(8, 256, 70, 3, 1, 0) == 0
+    cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=70, top=3, ff=24, shared=12))], vocab=61, width=256)
+    P = GZ.random_weights(cfg, 13)
+    toks = GZ.tokens(8, cfg["vocab"], 14)
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="float32", max_seqs=2, max_seq_len=64)
+    try:
+        got = m.step_batch([(m.seq_alloc(), toks, list(range(8)))])[0].astype(np.float64)
+    finally:
+        m.close()
+    want = O.forward(cfg, P, toks)
+    assert np.abs(got - want).max() < 1e-4 * np.abs(want).max()      # float32 sums against float64, as above
