@@ -442,7 +442,8 @@ class Model:
         self._check(self._lib.cm_vision_encode(self._h, pv.ctypes.data_as(C.POINTER(C.c_float)), pv.shape[0],
                                                g.ctypes.data_as(C.POINTER(C.c_uint32)), g.shape[0],
                                                out.ctypes.data_as(C.POINTER(C.c_float)), C.byref(rows)))
-        return out[: rows.value]
+        out.resize((rows.value, self.hidden_size), refcheck=False)              # in place: the caller's array owns its rows and no more memory
+        return out
 
     def vlm_forward(self, input_ids: Sequence[int], pixel_values: np.ndarray, grid_thw, start_pos: int = 0, seq: int = 0):
         """Qwen3_5VLModel::forward (vlm.rs:250-285): logits [V] of the last position and its arg-max."""
