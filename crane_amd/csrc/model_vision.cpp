@@ -51,11 +51,15 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
     if (!pix || !grid || n_img == 0 || n_patches == 0) throw CmError(CM_ERR_INVALID, "empty image input");
     const int VH = vcfg.hidden, heads = vcfg.heads, hd = VH / heads, m = vcfg.merge, M = m * m;
     size_t expect = 0;
+    bool beyond = false;
     for (size_t g = 0; g < n_img; ++g) {
         if (grid[3 * g + 1] % m || grid[3 * g + 2] % m) throw CmError(CM_ERR_INVALID, "grid_thw not divisible by spatial_merge_size");
-        expect += (size_t)grid[3 * g] * grid[3 * g + 1] * grid[3 * g + 2];
+        const size_t t = grid[3 * g], hw = (size_t)grid[3 * g + 1] * grid[3 * g + 2];
+        // (against what is left of the patches: a sum or product that wraps would pass for fewer rows than the loops below write)
+        if (t && hw && t > (n_patches - expect) / hw) beyond = true;
+        else expect += t * hw;
     }
-    if (expect != n_patches) throw CmError(CM_ERR_INVALID, "pixel_values rows != sum(t*h*w) of grid_thw");
+    if (beyond || expect != n_patches) throw CmError(CM_ERR_INVALID, "pixel_values rows != sum(t*h*w) of grid_thw");
     ensure_vision_buffers((int)n_patches);
     ensure_gemm_workspace();                   // (the split-K workspace of the GEMMs; not the text path's prompt buffers)
     const int N = (int)n_patches;
@@ -71,8 +75,9 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
     for (int i = 0; i < quarter; ++i) inv[(size_t)i] = 1.0f / powf(10000.0f, (float)(2 * i) / (float)(hd / 2));   // vision.rs:285-297
     // a row's angles depend on its grid row in the first half of a half head and on its grid column in the second: cosines and sines once per
     // coordinate (3172 patches: 400 000 of them took as long as two blocks of the tower)
-    uint32_t coords = 0;
-    for (size_t g = 0; g < n_img; ++g) coords = std::max({coords, grid[3 * g + 1], grid[3 * g + 2]});
+    uint32_t coords = 0;                          // (of images that have rows: at most N)
+    for (size_t g = 0; g < n_img; ++g)
+        if (grid[3 * g] && grid[3 * g + 1] && grid[3 * g + 2]) coords = std::max({coords, grid[3 * g + 1], grid[3 * g + 2]});
     std::vector<float> tc((size_t)coords * quarter), ts((size_t)coords * quarter);
     for (uint32_t x = 0; x < coords; ++x)
         for (int i = 0; i < quarter; ++i) {
@@ -83,6 +88,7 @@ int Model::vision_encode(const float* pix, size_t n_patches, const uint32_t* gri
     int row = 0;
     for (size_t g = 0; g < n_img; ++g) {
         const int t = (int)grid[3 * g], h = (int)grid[3 * g + 1], w = (int)grid[3 * g + 2];
+        if (h == 0 || w == 0) continue;
         auto lin = [&](int n, int i) { return n == 1 ? 0.0f : (float)i * ((float)(side - 1) / (float)(n - 1)); };
         for (int tt = 0; tt < t; ++tt) {
             frames.emplace_back(row, row + h * w);

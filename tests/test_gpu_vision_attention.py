@@ -41,3 +41,24 @@ def test_widths_and_runs_agree():
         assert rel(together, np.concatenate(alone)) < 3e-4
     finally:
         m.close()
+
+
+# entries of a grid without rows (no frames, or a side of 0) cost and change nothing, whatever their other numbers; numbers whose product wraps to 0 are
+# refused like any other that the patches do not match
+def test_images_without_rows():
+    from crane_amd import _lib
+    from crane_amd.backend import Model
+    g, cfg, w, text_w = _setup()
+    pix = np.random.default_rng(0).standard_normal((64, g["pixel_values"].shape[1])).astype(np.float32)
+    m = Model.synthetic(cfg, seed=0, max_seq_len=256, max_seqs=2)
+    try:
+        want = m.encode_images(pix, [[1, 8, 8]])
+        for empty in ([0, 2000000000, 2], [0, 8, 4000000000], [4000000000, 0, 4000000000]):
+            assert (m.encode_images(pix, [empty, [1, 8, 8]]) == want).all() and (m.encode_images(pix, [[1, 8, 8], empty]) == want).all()
+        for wrong in ([2 ** 22, 2 ** 21, 2 ** 21], [2 ** 31, 2 ** 31, 4], [1, 2, 2]):
+            for grid in ([wrong, [1, 8, 8]], [[1, 8, 8], wrong]):
+                with pytest.raises(_lib.CraneError):
+                    m.encode_images(pix, grid)
+        assert (m.encode_images(pix, [[1, 8, 8]]) == want).all()
+    finally:
+        m.close()
