@@ -107,3 +107,30 @@ def test_router_of_eight_rows_on_the_whole_chip(tmp_path):
         m.close()
     want = O.forward(cfg, P, toks)
     assert np.abs(got - want).max() < 1e-4 * np.abs(want).max()      # float32 sums against float64, as above
+
+
+# a sequence whose rows are NaN or infinite keeps them to itself: the others of the step have the same bits as beside a sound one (3 rows: the decode
+# kernels; 40: tiles, whose padding repeats the last row; portions of 30 rows: prompt attention)
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("seqs,portion", [(3, 1), (40, 1), (3, 30)])
+def test_rows_that_are_no_numbers(tmp_path, bad, seqs, portion):
+    from crane_amd.backend import Model
+    cfg = GZ.config([GZ.layer(GZ.attn(heads=4, kv_heads=2, dim=64, vdim=64), GZ.moe(experts=6, top=2, ff=128, shared=128)) for _ in range(2)], vocab=96,
+                    width=128)
+    P = GZ.random_weights(cfg, 17)
+    P["embed"][5] = bad
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=42, max_seq_len=128)
+    try:
+        got = []
+        for t in (5, 6):
+            ss = [m.seq_alloc() for _ in range(seqs)]
+            for i, s in enumerate(ss):
+                m.step_batch([(s, 7 + (np.arange(9 + i % 3) + i) % 80, [])], want_logits=False)
+            step = [np.full(portion, t) if i == seqs - 1 else 7 + (np.arange(portion) + 3 * i) % 80 for i in range(seqs)]
+            got.append(m.step_batch([(s, x, list(range(portion))) for s, x in zip(ss, step)])[0].reshape(seqs, portion, -1))
+            for s in ss:
+                m.seq_free(s)
+    finally:
+        m.close()
+    # (the norm's tanh takes infinities to one: their logits are finite)
+    assert np.isnan(got[0][-1]).all() == np.isnan(bad) and np.isfinite(got[1]).all() and (got[0][:-1] == got[1][:-1]).all()

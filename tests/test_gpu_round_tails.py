@@ -78,3 +78,37 @@ def test_short_contexts_keep_32_bit_queries_and_weights(rows, ctx):
         assert np.isfinite(a).all() and (a == b).all()
     finally:
         m.close()
+
+
+# a sequence whose rows are NaN or infinite keeps them to itself: the others of the group have the same bits as beside a sound one (products, the
+# reductions, norms and quantisers behind them, attention and its combine; rows that fill 32- and 64-row tiles in part)
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("isq", [None, "q8_0"])
+@pytest.mark.parametrize("rows,ctx", [(9, 9), (20, 70), (40, 70), (66, 20)])
+def test_rows_that_are_no_numbers(tmp_path, bad, isq, rows, ctx):
+    import json
+    import os
+
+    from crane_amd import synth
+    from crane_amd.backend import Model
+    cfg = dict(configs.get_config("qwen3-0.6b"), vocab_size=512, num_hidden_layers=2, tie_word_embeddings=False)
+    w = synth.synth_weights_f32(cfg, seed=3)
+    w["model.embed_tokens.weight"][5] = bad
+    path = str(tmp_path / "ckpt")
+    os.makedirs(path)
+    with open(os.path.join(path, "config.json"), "w") as f:
+        json.dump(cfg, f)
+    synth.write_safetensors_bf16(os.path.join(path, "model.safetensors"), [(k, v.shape, synth.f32_to_bf16_bits(v)) for k, v in w.items()])
+    m = Model.from_pretrained(path, max_seq_len=128, max_seqs=rows + 1, **({"isq": isq} if isq else {}))
+    try:
+        seqs = [m.seq_alloc() for _ in range(rows)]
+        for i, s in enumerate(seqs):
+            m.seq_forward(s, (6 + (np.arange(ctx + i % 3) + i) % 500).tolist(), 0)
+        toks, got = (6 + np.arange(rows) % 500).tolist(), []
+        for t in (5, 6):
+            got.append(np.asarray(m.step_batch_decode(seqs, toks[:-1] + [t])[0], np.float32).reshape(rows, -1))
+            for i, s in enumerate(seqs):
+                m.seq_truncate(s, ctx + i % 3)
+    finally:
+        m.close()
+    assert not np.isfinite(got[0][-1]).any() and np.isfinite(got[1]).all() and (got[0][:-1] == got[1][:-1]).all()
