@@ -42,6 +42,18 @@ __device__ __forceinline__ uint16_t f32_to_f16(float f) {
     const _Float16 h = (_Float16)fminf(fmaxf(f, -65504.f), 65504.f);
     return __builtin_bit_cast(uint16_t, h);
 }
+// from memory into LDS without passing registers: every lane's 16 (4) bytes at its gsrc land at lds_base + 16 (4) * lane.  M0 carries the LDS base and
+// belongs to the compiler: saved and restored around the instruction.  Counted by vmcnt like any load
+__device__ __forceinline__ void lds_load16(const void* gsrc, uint32_t lds_base) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
+}
+__device__ __forceinline__ void lds_load4(const void* gsrc, uint32_t lds_base) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
+}
 // internal KV-page element types (template parameter KVT of the attention kernels, Model::kv_mode)
 enum { KV_BF16 = 0, KV_F32 = 1, KV_INT8 = 2, KV_INT4 = 3, KV_F16 = 4 };
 // one cached 16-bit element pair -> f32 (bf16: bit shifts; f16: v_cvt_f32_f16)

@@ -33,16 +33,6 @@ namespace {
 constexpr int TBK = 64;              // k-tile depth (elements): one 128-byte line per operand row
 constexpr int TST = 2;               // LDS stages
 
-// one LDS-DMA piece: every lane's 16 bytes at `gsrc` land at lds_base + 16 * lane.  M0 carries the LDS base and belongs to the
-// compiler, so it is saved and restored around the instruction (cdna_hip_programming.md, inline-asm notes).
-__device__ __forceinline__ void glds16(const void* gsrc, uint32_t lds_base) {
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep)
-                 : "v"(gsrc), "s"(lds_base)
-                 : "memory");
-}
-
 }  // namespace
 
 // WST = 3 (round 4, decode groups: one m-tile, the weights come from HBM, not from a neighbour's L2 lines): a THIRD weight stage, the
@@ -154,8 +144,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
     // with three), each clamped to the last tile (past the end: into a stage nobody reads)
     auto piece = [&](int g, int ta, int tw) __attribute__((always_inline)) {
         const int tl = kpb - 1;
-        if (isw[g]) { const int tt = min(tw, tl); glds16(src[g] + (size_t)tt * TBK, dst[g] + (uint32_t)((tw % WST) * WSTAGE) * 2u); }
-        else { const int tt = min(ta, tl); glds16(src[g] + (size_t)tt * TBK, dst[g] + (uint32_t)((ta & 1) * ASTAGE) * 2u); }
+        if (isw[g]) { const int tt = min(tw, tl); lds_load16(src[g] + (size_t)tt * TBK, dst[g] + (uint32_t)((tw % WST) * WSTAGE) * 2u); }
+        else { const int tt = min(ta, tl); lds_load16(src[g] + (size_t)tt * TBK, dst[g] + (uint32_t)((ta & 1) * ASTAGE) * 2u); }
     };
     auto issue_all = [&](int ta, int tw) __attribute__((always_inline)) {
 #pragma unroll

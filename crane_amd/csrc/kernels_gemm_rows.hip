@@ -23,12 +23,6 @@ namespace {
 
 constexpr int RBK = 64;
 
-__device__ __forceinline__ void rows_load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
-}
-
 template <int BM, int RBN, int ST, int EPI, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_rows_kernel(GemmArgs a) {
     constexpr int GM = RBN == 96 ? NW / 2 : NW == 8 ? (BM == 128 ? 4 : 2) : BM == 32 ? 1 : 2, GN = NW / GM, WM = BM / GM, WN = RBN / GN, NI = WM / 16, NJ = WN / 16;      // NW waves GM x GN, WM x WN outputs each
@@ -58,7 +52,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_rows_kernel(Gem
         const size_t at = (size_t)min(t, kpb - 1) * RBK;
         const uint32_t stage = (uint32_t)((t % ST) * STAGE) * 2u;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) rows_load16(src[i] + at, dst[i] + stage);
+        for (int i = 0; i < NL; ++i) lds_load16(src[i] + at, dst[i] + stage);
     };
     f32x4 acc[NI][NJ];
 #pragma unroll

@@ -29,14 +29,6 @@ namespace {
 
 constexpr int BK = 64;
 
-__device__ __forceinline__ void lds_load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep)
-                 : "v"(gsrc), "s"(lds_base)
-                 : "memory");
-}
-
 template <int BM, int BN, int ST, bool DUAL>
 __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int mtiles, int ntiles) {
     constexpr int WM = BM / 2, WN = BN / 2, NI = WM / 16, NJ = WN / 16, APC = BM / 8, NL = (BM + BN) / 32;      // NL: loads per wave and k-tile

@@ -31,17 +31,6 @@ __device__ __forceinline__ float half_times(uint32_t w, float x) {
 }
 __device__ __forceinline__ float f16r(float v) { return (float)(_Float16)v; }
 
-__device__ __forceinline__ void dma16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
-}
-__device__ __forceinline__ void dma4(const void* gsrc, uint32_t lds_base) {       // every lane's 4 bytes land at lds_base + 4 * lane
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
-}
-
 constexpr int QG = 4, GB = QG * 32, ST = 2;                    // blocks and bytes of a row per group, stages
 
 // weight codes and scales, activation codes and scales of a stage
@@ -85,12 +74,12 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q8_rows_kernel(QGemmArgs a) {
     auto request = [&](int g) __attribute__((always_inline)) {
         const uint32_t st = lds0 + (uint32_t)((g % ST) * STAGE);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dma16(wsrc[i] + (size_t)g * GB, st + (uint32_t)((wave * 4 + i) * 1024));
+        for (int i = 0; i < 4; ++i) lds_load16(wsrc[i] + (size_t)g * GB, st + (uint32_t)((wave * 4 + i) * 1024));
 #pragma unroll
-        for (int i = 0; i < AI; ++i) dma16(xsrc[i] + (size_t)g * GB, st + (uint32_t)(WB + (wave * AI + i) * 1024));
-        dma4(ssrc + (size_t)g * (QG * 2), st + (uint32_t)(WB + PR * GB + wave * 256));
+        for (int i = 0; i < AI; ++i) lds_load16(xsrc[i] + (size_t)g * GB, st + (uint32_t)(WB + (wave * AI + i) * 1024));
+        lds_load4(ssrc + (size_t)g * (QG * 2), st + (uint32_t)(WB + PR * GB + wave * 256));
 #pragma unroll
-        for (int i = 0; i < XI; ++i) dma4(dsrc[i] + (size_t)g * QG * a.xs, st + (uint32_t)(WB + PR * GB + SB + (wave * XI + i) * 256));
+        for (int i = 0; i < XI; ++i) lds_load4(dsrc[i] + (size_t)g * QG * a.xs, st + (uint32_t)(WB + PR * GB + SB + (wave * XI + i) * 256));
     };
     float acc[MT][16];
 #pragma unroll

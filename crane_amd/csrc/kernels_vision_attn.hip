@@ -20,12 +20,6 @@ namespace {
 
 constexpr int D = 64, KT = 64;
 
-__device__ __forceinline__ void load16(const void* gsrc, uint32_t lds_base) {      // every lane's 16 bytes land at lds_base + 16 * lane
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(gsrc), "s"(lds_base) : "memory");
-}
-
 // four probabilities as bf16 hi and lo pairs
 __device__ __forceinline__ void split_p(const float (&p)[4], uint32_t* hi, uint32_t* lo) {
     hi[0] = pack_bf16x2(p[0], p[1]); hi[1] = pack_bf16x2(p[2], p[3]);
@@ -88,10 +82,10 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
         if (t < full) {
             const uint16_t* p = plane + (size_t)t * heads * (64 * D);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) load16(p + src[i], dst + i * 1024u);
+            for (int i = 0; i < 8; ++i) lds_load16(p + src[i], dst + i * 1024u);
         } else {                                                       // the ragged end: its last row again
 #pragma unroll
-            for (int i = 0; i < 8; ++i) load16(plane + source(min(lo + t * KT + 8 * i + prow, end - 1), i), dst + i * 1024u);
+            for (int i = 0; i < 8; ++i) lds_load16(plane + source(min(lo + t * KT + 8 * i + prow, end - 1), i), dst + i * 1024u);
         }
     };
     const int kf = (sub >> 1) & 7, vf = (2 * g + (sub >> 3)) & 3;
