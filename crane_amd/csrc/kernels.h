@@ -154,8 +154,8 @@ struct GemmArgs {
     float norm_eps = 0.f;
 };
 
-// 9 .. 128 rows with hi + lo activations (kernels_gemm_rows.hip): K slices for these sizes (0: not taken) and the launch (a.ksplit set; more than
-// one slice: partial tiles in a.ws)
+// 9 .. 128 rows with hi + lo activations (kernels_gemm_rows.hip): whether these sizes are taken, with the tile's columns *bn and the K slices *ks,
+// and the launch (a.ksplit set; more than one slice: partial tiles in a.ws)
 bool gemm_rows_plan(int M, int N, int K, size_t ws_floats, int* bn, int* ks);
 bool launch_gemm_rows(const GemmArgs& a, int epi, int bn, hipStream_t s);
 

@@ -1,4 +1,4 @@
-// Products of a decode group of 9 .. 64 rows (the narrow ones up to 128) and of prompts that short: C[M, N] (+)= A[M, K] . W[N, K]^T with the
+// Products of 9 .. 128 rows, decode groups and short prompts (from 65 rows on projections of up to 128 column tiles): C[M, N] (+)= A[M, K] . W[N, K]^T with the
 // activations as bf16 hi + lo planes, two MFMAs per product -- gemm256_kernel's arithmetic and epilogues on tiles made for a launch that waits
 // for its weights.
 //

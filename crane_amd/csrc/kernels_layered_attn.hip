@@ -372,6 +372,10 @@ void go(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
 // multiplied, its values as soon as the one before is in LDS.  The eight waves' sums meet in LDS once; gridDim.z > 1: they leave a partial
 // sum for lay_attn_merge_kernel instead.  Queries and weights keep their 24 bits, as in lay_attn_kernel: three bfloat16 parts each, three
 // products per tile (the launch waits for memory, not for the matrix cores), and its exponential and logarithm.
+// For 128 / 128 elements a block's 161 KB of LDS leave one block on a CU; it is ahead of lay_attn_kernel all the same, for any number of sequences.  us a
+// step of four layers, lay_attn_kernel / here: 8 heads on 2 of width 1024, 1 / 32 / 128 sequences behind 24 tokens 281 / 256, 514 / 460, 854 / 705,
+// behind 1000 tokens 296 / 280, 830 / 525, 2126 / 853; 32 heads on 8 of width 4096, 1 / 32 / 128 sequences behind 24 tokens 515 / 487, 1187 / 1068,
+// 1699 / 1552, behind 1000 tokens 536 / 522, 2523 / 1154, 4780 / 1927
 constexpr int DW = 8;
 template <int DP, int EP, bool POOL>
 __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {

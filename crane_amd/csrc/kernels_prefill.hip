@@ -493,12 +493,11 @@ __global__ __launch_bounds__(BN * 2) void gemm_bf16_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// causal flash attention over the paged cache.  grid (ceil(S/64), Hq), 4 waves x 16 query rows.
+// causal flash attention over the paged cache.  grid (Hq, query tiles of 64 rows), 4 waves x 16 query rows.
 // ---------------------------------------------------------------------------------------------
 // V tile row stride in LDS = D + 16 elements: the 4 key rows of a tr-read group land on disjoint banks
 // KVT: KV_BF16 pages (K rows / V^T fragments feed the bf16 MFMAs as cached), KV_F16 pages (the same on the f16 MFMAs; q_hi / q_lo
 // and P are then f16 hi + lo), KV_F32 (f32 rows split into bf16 hi + lo on load: f32 pages, the int8 / int4 shadow)
-// without a conversion in the loop.
 // e^x for x <= 0 (softmax numerators after the running max): v_exp_f32 (2^x, 1 ulp) on x * log2(e) -- two instructions where
 // expf()'s range reduction and polynomial are ~20; 17 of them per lane and key tile were a quarter of the tile's VALU work
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
@@ -1115,7 +1114,9 @@ static void launch_splitk_resadd_norm(const GemmArgs& a, hipStream_t s) {
     else if (a.ksplit == 8) hipLaunchKernelGGL((gemm_splitk_resadd_norm_kernel<8, LN>), dim3(a.M), dim3(256), 0, s, a); \
     else hipLaunchKernelGGL((gemm_splitk_resadd_norm_kernel<0, LN>), dim3(a.M), dim3(256), 0, s, a); } while (0)
     // up to 128 rows of more than 1024 columns: four times the threads per row (one workgroup per row leaves half of the chip idle either way).
-    // Rows of 4096, eight slices: 32 rows 5.8 -> 4.9, 117 rows 6.9 -> 5.9 us
+    // Rows of 4096, eight slices: 32 rows 5.8 -> 4.9, 117 rows 6.9 -> 5.9 us.  Product and reduction together, 256 / 1024 threads, 9 and 128 rows:
+    // 1152 columns, two slices 7.7 / 7.3 and 13.4 / 13.0; 1536, eight 8.7 / 8.0 and 15.5 / 14.6; 2048, eight 7.4 / 6.7 and 14.1 / 13.4; 5120, four
+    // 15.9 / 14.6 and 27.4 / 26.2
     if (a.norm_b == nullptr && a.M <= 128 && a.N > 1024 && (a.ksplit == 2 || a.ksplit == 4 || a.ksplit == 8)) {
         if (a.ksplit == 2) hipLaunchKernelGGL((gemm_splitk_resadd_norm_kernel<2, false, 1024>), dim3(a.M), dim3(1024), 0, s, a);
         else if (a.ksplit == 4) hipLaunchKernelGGL((gemm_splitk_resadd_norm_kernel<4, false, 1024>), dim3(a.M), dim3(1024), 0, s, a);

@@ -328,7 +328,7 @@ constexpr int LAY_ATTN_MFMA_ROWS = 64;
 void launch_lay_attn_mfma(const LAttnArgs& a, hipStream_t s);
 bool lay_attn_mfma_fits(int d, int e, bool own_v);         // sizes the matrix-core form takes
 // the same for sizes up to 128 over pages of whole 64-key tiles (kernels_layered_attn.hip): 2048 tokens of 32 query heads of 128 on 8 key
-// heads 106 us against 1590, 8 on 2 (a mixed batch of 24 tokens and 300 prompt rows) 27 against 174; the older form keeps other page sizes
+// heads 106 us against 1590, 8 on 2 (a mixed batch of 24 tokens and 300 prompt rows) 24 against 174; the older form keeps other page sizes
 // and long cached rows
 void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);

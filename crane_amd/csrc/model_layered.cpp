@@ -65,7 +65,7 @@ struct Layered {
     // bfloat16 format, products of 32 rows or more whose shape fits (N % 128 == 0, K % 32 == 0): the matrix-core GEMM the other
     // families' prompt passes use (kernels_prefill.hip / kernels_gemm256.hip), plain bf16 activations; cm_debug_set("lay_shared_gemm", 0): never
     bool shared_gemm = true;
-    bool attn_mfma = true;             // bfloat16 format, prompt passes: the matrix-core attention (cm_debug_set("lay_attn_mfma", 0): never)
+    bool attn_mfma = true;             // bfloat16 format: the matrix-core attention, prompt passes and decode steps (cm_debug_set("lay_attn_mfma", 0): never)
     bool fused_prep = true;            // query / key norm + rotation + cache append in one launch (cm_debug_set("lay_fused_prep", 0): single operations)
     uint16_t* Abf = nullptr;           // [cap rounded up to 256][widest K] bf16 A operand
     uint16_t* Asc = nullptr;           // [cap][top][W] bf16 rows times their expert's weight (scale_input)
