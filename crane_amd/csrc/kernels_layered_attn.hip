@@ -84,6 +84,10 @@ template <int PARTS>
 struct Query {
     static constexpr bool EXACT = PARTS == 3;
     static constexpr float UNIT = EXACT ? 1.f : L2E;
+    // the scores' loops take what lies in front and move the rest up: rolled where the functions are long.  A decode launch has about one key tile per
+    // wave and waits for its own code: with sixteen expf in a row it was 4 us longer than with sixteen v_exp_f32, with eight in a loop of two it is not
+    // (24 layers of width 1024, 8 tokens at 1000: 13.09 ms with v_exp_f32, 13.88 in a row, as long as with v_exp_f32 in the loop)
+    static constexpr int ROLL = EXACT ? 1 : 4;
     static __device__ __forceinline__ float ex(float x) { return EXACT ? expf(x) : __builtin_amdgcn_exp2f(x); }
     bool ok;
     int pos, head, row, clo;
@@ -118,15 +122,18 @@ struct Query {
         } else {
             // (the distance term and the kind of tile are settled outside the loops: a branch per score kept the vector units at a third)
             auto each = [&](auto penalty, auto visible) __attribute__((always_inline)) {
-#pragma unroll
-                for (int tt = 0; tt < 4; ++tt)
+#pragma unroll ROLL
+                for (int tt = 0; tt < 4; ++tt) {
+                    f32x4 v = s[0];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int j = j0 + tt * 16 + lg * 4 + r, dist = pos - j;
-                        const float sc = s[tt][r] * scale - penalty(dist);
-                        s[tt][r] = visible(j, dist) ? sc : -INFINITY;
-                        mt = fmaxf(mt, s[tt][r]);
+                        const float sc = v[r] * scale - penalty(dist);
+                        v[r] = visible(j, dist) ? sc : -INFINITY;
+                        mt = fmaxf(mt, v[r]);
                     }
+                    s[0] = s[1]; s[1] = s[2]; s[2] = s[3]; s[3] = v;
+                }
             };
             // bitwise: no short-circuit branches
             const auto window = [&](int j, int dist) { return (bool)((dist >= 0) & (((dist < w.win) & (j >= clo)) | (j < w.keep))); };
@@ -152,12 +159,14 @@ struct Query {
         }
         float psum = 0.f;
 #pragma unroll
+        for (int k = 0; k < PARTS; ++k) p[k][1] = __builtin_bit_cast(bf16x8, (u32x4){0u, 0u, 0u, 0u});
+#pragma unroll ROLL
         for (int h = 0; h < 2; ++h) {
             u32x4 part[PARTS];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float p0 = ex(s[2 * h + (q >> 1)][2 * (q & 1)] - ms);
-                float p1 = ex(s[2 * h + (q >> 1)][2 * (q & 1) + 1] - ms);
+                float p0 = ex(s[q >> 1][2 * (q & 1)] - ms);
+                float p1 = ex(s[q >> 1][2 * (q & 1) + 1] - ms);
                 psum += p0 + p1;
 #pragma unroll
                 for (int k = 0; k < PARTS; ++k) {
@@ -167,7 +176,8 @@ struct Query {
                 }
             }
 #pragma unroll
-            for (int k = 0; k < PARTS; ++k) p[k][h] = __builtin_bit_cast(bf16x8, part[k]);
+            for (int k = 0; k < PARTS; ++k) { p[k][0] = p[k][1]; p[k][1] = __builtin_bit_cast(bf16x8, part[k]); }
+            s[0] = s[2]; s[1] = s[3];
         }
         l += psum;
     }
