@@ -438,11 +438,11 @@ class Model:
         pv = np.ascontiguousarray(pixel_values, dtype=np.float32)
         g = np.ascontiguousarray(np.asarray(grid_thw, dtype=np.uint32).reshape(-1, 3))
         rows = C.c_size_t(0)
-        out = np.empty((pv.shape[0], self.hidden_size), dtype=np.float32)       # upper bound on rows
+        out = np.empty(int(self._lib.cm_vision_features(self._h, pv.shape[0])), dtype=np.float32)      # the caller's: exactly the features
         self._check(self._lib.cm_vision_encode(self._h, pv.ctypes.data_as(C.POINTER(C.c_float)), pv.shape[0],
                                                g.ctypes.data_as(C.POINTER(C.c_uint32)), g.shape[0],
                                                out.ctypes.data_as(C.POINTER(C.c_float)), C.byref(rows)))
-        out.resize((rows.value, self.hidden_size), refcheck=False)              # in place: the caller's array owns its rows and no more memory
+        out.shape = (rows.value, -1)
         return out
 
     def vlm_forward(self, input_ids: Sequence[int], pixel_values: np.ndarray, grid_thw, start_pos: int = 0, seq: int = 0):

@@ -376,6 +376,9 @@ int cm_step_batch(cm_model* h, const cm_step_item* items, size_t n, float* logit
     });
 }
 
+uint64_t cm_vision_features(const cm_model* h, size_t n_patches) {
+    return (h && h->m.vcfg.present && h->m.vcfg.merge > 0) ? (uint64_t)(n_patches / ((size_t)h->m.vcfg.merge * h->m.vcfg.merge)) * (uint64_t)h->m.vcfg.out_hidden : 0;
+}
 int64_t cm_image_token_id(const cm_model* h) { return (h && h->m.vcfg.present) ? (int64_t)h->m.vcfg.image_token : -1; }
 
 int cm_vision_encode(cm_model* h, const float* pixel_values, size_t n_patches, const uint32_t* grid_thw, size_t n_images,

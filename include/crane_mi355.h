@@ -349,6 +349,9 @@ int cm_prefill_batch(cm_model* m, const int32_t* seqs, const uint32_t* const* id
 /* image placeholder token of the checkpoint (config.json image_token_id), -1 when the model has no vision tower */
 int64_t cm_image_token_id(const cm_model* m);
 
+/* f32 values that cm_vision_encode writes to features_out for so many patches (0: the model has no vision tower) */
+uint64_t cm_vision_features(const cm_model* m, size_t n_patches);
+
 /* Qwen3_5VisionModel::forward (vision.rs:558-584).  pixel_values: host f32 [n_patches, C*T*P*P] exactly as
  * PreprocessorConfig::process emits them (processor.rs:114-210: merge-block-major rows, (channel, temporal, y, x)
  * inside a row); grid_thw: host u32 [n_images, 3].  Writes the merged image tokens

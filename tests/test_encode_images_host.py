@@ -13,6 +13,7 @@ class Lib:
     cm_vocab_size = staticmethod(lambda h: 16)
     cm_hidden_size = staticmethod(lambda h: 96)
     cm_destroy = staticmethod(lambda h: None)
+    cm_vision_features = staticmethod(lambda h, n: n // 4 * 96)
 
     @staticmethod
     def cm_vision_encode(h, pix, n, grid, images, out, rows):
