@@ -287,21 +287,22 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs a) {
 // Prefill in three passes.  The fused kernel above walks a prompt with 4 barriers, two block reductions and a handful
 // of transcendental functions per token on ONE block per value head (~5 us per token and layer).  Everything except
 // the state recurrence is independent across tokens, so:
-//   gdn_pre_kernel  (a wave per head and 8 tokens): conv + SiLU, L2 norms, q scale, beta, exp(g)  -> q^ k^ v beta decay per token
+//   gdn_pre_kernel  (a wave per head and 4 or 8 tokens): conv + SiLU, L2 norms, q scale, beta, exp(g)  -> q^ k^ v beta decay per token
 //   gdn_scan_kernel (grid NV x 4): the recurrence only; 16 lanes share a state column (8 of the 128 k each, partial
 //                   sums folded with one DPP row reduction), q^ / k^ of 8 tokens staged per barrier
 //   gdn_post_kernel (grid S x NV): gated RMSNorm of the raw y rows in place
 // Same per-token arithmetic as the fused kernel except for the association of the two 128-term sums over k.
 // ---------------------------------------------------------------------------------------------------------
-// A wave takes one head (q, k or v; lane l its channels 2 l, 2 l + 1) over GDN_PT tokens: the convolution's window rolls in registers, a row is read
+// A wave takes one head (q, k or v; lane l its channels 2 l, 2 l + 1) over PT tokens: the convolution's window rolls in registers, a row is read
 // once instead of four times, norms need no other wave.  Bound by its traffic (a workgroup per token and head was bound by the 65 536 workgroups of a
 // 2048-token pass: mean per launch of a 4165-token prompt 31.7 -> 21.2 us).  The rolling window that the next call reads is written by the wave that read
 // the one of this call: both may be the same memory.
-constexpr int GDN_PT = 8;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <int PT>
 __global__ __launch_bounds__(256) void gdn_pre_kernel(GdnArgs a) {
     constexpr int K = 128, KER = 4;
-    const int lane = threadIdx.x & 63, item = (int)blockIdx.y * 4 + ((int)threadIdx.x >> 6), t0 = (int)blockIdx.x * GDN_PT;
+    static_assert(PT >= KER - 1, "only the wave of token 0 reads the window of the call before");
+    const int lane = threadIdx.x & 63, item = (int)blockIdx.y * 4 + ((int)threadIdx.x >> 6), t0 = (int)blockIdx.x * PT;
     const int nk = a.NV / a.vpg;
     if (item >= 2 * nk + a.NV) return;
     const int conv_dim = 2 * a.key_dim + a.NV * K;
@@ -309,9 +310,9 @@ __global__ __launch_bounds__(256) void gdn_pre_kernel(GdnArgs a) {
     const float* conv_state = a.conv_pool + ((size_t)a.slot * a.gdn_layers + a.layer_idx) * 2 * conv_dim * (KER - 1);
     const float* cs_in = conv_state + (size_t)(a.start_pos & 1) * conv_dim * (KER - 1);
     const float* pc = a.proj + c;
-    f32x2 x[KER - 1 + GDN_PT];                           // inputs at tokens t0 - 3 ...
+    f32x2 x[KER - 1 + PT];                           // inputs at tokens t0 - 3 ...
 #pragma unroll
-    for (int i = 0; i < KER - 1 + GDN_PT; ++i) x[i] = *(const f32x2*)(pc + (size_t)min(max(t0 + i - (KER - 1), 0), a.S - 1) * a.proj_stride);
+    for (int i = 0; i < KER - 1 + PT; ++i) x[i] = *(const f32x2*)(pc + (size_t)min(max(t0 + i - (KER - 1), 0), a.S - 1) * a.proj_stride);
     const f32x4 w0 = *(const f32x4*)(a.conv_w + (size_t)c * KER), w1 = *(const f32x4*)(a.conv_w + (size_t)(c + 1) * KER);
     if (t0 == 0) {
 #pragma unroll
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(256) void gdn_pre_kernel(GdnArgs a) {
     float* dst = kind == 0 ? a.pre_q + c : kind == 1 ? a.pre_k + (c - a.key_dim) : a.pre_v + (c - 2 * a.key_dim);
     const size_t ldd = kind == 2 ? (size_t)a.NV * K : (size_t)a.key_dim;
 #pragma unroll
-    for (int i = 0; i < GDN_PT; ++i) {
+    for (int i = 0; i < PT; ++i) {
         f32x2 y = {silu_f(x[i][0] * w0[0] + x[i + 1][0] * w0[1] + x[i + 2][0] * w0[2] + x[i + 3][0] * w0[3]),
                    silu_f(x[i][1] * w1[0] + x[i + 1][1] * w1[1] + x[i + 2][1] * w1[2] + x[i + 3][1] * w1[3])};
         if (kind < 2) {                                  // (a wave's own branch)
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(256) void gdn_pre_kernel(GdnArgs a) {
         }
         if (t0 + i < a.S) *(f32x2*)(dst + (size_t)(t0 + i) * ldd) = y;
     }
-    if (kind == 2 && lane < GDN_PT && t0 + lane < a.S) { // beta and decay of the value head, a token per lane
+    if (kind == 2 && lane < PT && t0 + lane < a.S) { // beta and decay of the value head, a token per lane
         const int h = item - 2 * nk, t = t0 + lane;
         const float* pr = a.proj + (size_t)t * a.proj_stride;
         const float beta = 1.0f / (1.0f + expf(-pr[conv_dim + a.NV * K + h]));
@@ -438,7 +439,7 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a) {
 // gdn_chunk_prep_kernel (grid chunks x NV): A and P on v_mfma_f32_16x16x4_f32, (I + A)^-1 [.] by forward substitution (one
 // thread per column of [beta e^G K | beta V], its 64 unknowns in registers: no dependency between threads) -> W, U0, P, G.
 // gdn_chunk_scan_kernel (grid NV x V/16): the only sequential part -- U and the state's update, two small matrix products per chunk
-// over a 128 x 16 slice of the state (columns of S are independent); it leaves U and the state in front of every chunk to
+// over a 128 x 16 slice of the state (columns of S are independent); for prompts of more than a few chunks it leaves U and the state in front of every chunk to
 // gdn_chunk_out_kernel (grid chunks x NV), which forms Y and its gated norm for all chunks at once.  (Y inside the scan was half of
 // its products and most of its registers: 2048 + 2048 + 69 tokens, 16 heads, mean per launch: scan and norm 103.8 + 12.3 -> scan
 // 58.3, outputs 24.1 us.)  Everything stays f32 (f32 MFMA: products and sums in f32), logs of the
@@ -465,8 +466,14 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& av, const f32x4& bv, f32x4 c
     return c;
 }
 
+// Where Y is formed.  A launch for the outputs of all chunks costs its start and one chunk's chain of products whatever their number, Y inside the scan a
+// part of every chunk: short prompts, while the scan's NV x 8 workgroups fit on the chip at once, keep it inside.  us a layer, scan and outputs apart
+// minus together, prompts of 2 / 3 / 4 / 5 / 6 / 8 chunks: 16 heads 6.6 / 5.0 / 3.1 / 1.2 / -1.3 / -5.3, 32 heads 6.3 / 5.6 / 3.6 / 1.7 / -0.3 / -4.4, 48 heads (384
+// workgroups) 1.1 / -2.7 / -6.9 / -11.9 / -8.8 / -19.7
+static bool gdn_out_in_scan(int chunks, int NV) { return chunks <= 5 && NV * 8 <= 256; }
+
 size_t gdn_chunk_prep_lds() { return (size_t)(2 * GDN_CK * CKP + GDN_CK * CTP + 2 * GDN_CK) * sizeof(float); }
-size_t gdn_chunk_scan_lds() { return (size_t)(16 * CKP + 16 * CTP + GDN_CK * CKP + GDN_CK) * sizeof(float); }
+size_t gdn_chunk_scan_lds(bool out) { return (size_t)(16 * CKP + (out ? 2 : 1) * 16 * CTP + GDN_CK * CKP + GDN_CK) * sizeof(float); }
 
 __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK;
@@ -598,6 +605,8 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
     }
 }
 
+// OUT: Y of every chunk too (raw rows for gdn_post_kernel), nothing left for gdn_chunk_out_kernel
+template <bool OUT>
 __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK, VB = 16;
     extern __shared__ __attribute__((aligned(16))) float cl[];
@@ -605,6 +614,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
     float (*Vt)[CTP] = (float (*)[CTP])(cl + VB * CKP);                 // e^{G_C - G_t} U of the chunk, transposed: [column][t]
     float (*Ks)[CKP] = (float (*)[CKP])(cl + VB * CKP + VB * CTP);      // k^ rows of the chunk
     float* lgs = cl + VB * CKP + VB * CTP + C * CKP;
+    float (*Ut)[CTP] = (float (*)[CTP])(lgs + C);                       // OUT: U of the chunk, transposed: [column][t]
     const int h = blockIdx.x, cb = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, kq = lane >> 4;
     const int nk = a.NV / a.vpg, kh = a.chunked ? h % nk : h / a.vpg;
@@ -619,18 +629,27 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
     // values, its share of the k^ rows, the cumulative log decay) are requested into registers while chunk c is multiplied --
     // unconditionally (rows / chunks past the end are clamped and never consumed).
     // Register sets: W rows (needed FIRST in a chunk) are requested TWO chunks ahead into two alternating sets, the rest one chunk ahead.
-    f32x4 awA[8], awB[8], kreg[8];
+    // (OUT: q^ rows beside the W rows, P rows beside U0)
+    constexpr int NQ = OUT ? 8 : 1;
+    f32x4 awA[8], awB[8], aqA[NQ], aqB[NQ], ap[4], kreg[8];
     float u0[4], glane = 0.f;
-    auto fetch_w = [&](int c, f32x4 (&aw)[8]) __attribute__((always_inline)) {
-        const float* ck = a.ck + ((size_t)min(c, nchunks - 1) * a.NV + h) * GDN_CK_FLOATS;
+    auto fetch_w = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[NQ]) __attribute__((always_inline)) {
+        const int cc = min(c, nchunks - 1);
+        const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) aw[j] = *(const f32x4*)(ck + (16 * wave + r) * 128 + 16 * j + 4 * kq);
+        for (int j = 0; j < 8; ++j) {
+            aw[j] = *(const f32x4*)(ck + (16 * wave + r) * 128 + 16 * j + 4 * kq);
+            if constexpr (OUT) aq[j] = *(const f32x4*)(a.pre_q + (size_t)min(cc * C + 16 * wave + r, a.S - 1) * a.key_dim + kh * K + 16 * j + 4 * kq);
+        }
     };
     auto fetch_u = [&](int c) __attribute__((always_inline)) {          // U0 values of chunk c (issued once the previous ones are consumed)
         const int cc = min(c, nchunks - 1);
         const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u0[i] = ck[C * 128 + (16 * wave + 4 * kq + i) * 128 + VB * cb + r];
+        for (int i = 0; i < 4; ++i) {
+            u0[i] = ck[C * 128 + (16 * wave + 4 * kq + i) * 128 + VB * cb + r];
+            if constexpr (OUT) ap[i] = *(const f32x4*)(ck + 2 * C * 128 + (16 * wave + r) * C + 16 * i + 4 * kq);
+        }
     };
     auto fetch_k = [&](int c) __attribute__((always_inline)) {          // k^ rows + cumulative log decay of chunk c: parked in LDS at the END of
         const int cc = min(c, nchunks - 1), t0 = cc * C;                 //   chunk c - 1, so they are requested at its very beginning
@@ -651,28 +670,43 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
         }
         if (wave == 0) lgs[lane] = glane;
     };
-    auto chunk = [&](int c, f32x4 (&aw)[8]) __attribute__((always_inline)) {
+    auto chunk = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[NQ]) __attribute__((always_inline)) {
         float* ck = a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS;
         fetch_k(c + 1);
-        // ---- U = U0 - W S0: wave w owns token rows 16 w .. 16 w + 15 ----
-        f32x4 accU = {0.f, 0.f, 0.f, 0.f}, accV = accU;
+        // ---- U = U0 - W S0 (OUT: and Q S0): wave w owns token rows 16 w .. 16 w + 15 ----
+        f32x4 accU = {0.f, 0.f, 0.f, 0.f}, accV = accU, accQ = accU, accP = accU, pc[4];
+        float eg[4];
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
-            accU = mfma4(aw[j], *(const f32x4*)&St[r][16 * j + 4 * kq], accU);
-            accV = mfma4(aw[j + 1], *(const f32x4*)&St[r][16 * j + 16 + 4 * kq], accV);
+            const f32x4 s0 = *(const f32x4*)&St[r][16 * j + 4 * kq], s1 = *(const f32x4*)&St[r][16 * j + 16 + 4 * kq];
+            accU = mfma4(aw[j], s0, accU);
+            accV = mfma4(aw[j + 1], s1, accV);
+            if constexpr (OUT) { accQ = mfma4(aq[j], s0, accQ); accQ = mfma4(aq[j + 1], s1, accQ); }
         }
-        fetch_w(c + 2, aw);                            // this set is free again: the chunk after next
+        fetch_w(c + 2, aw, aq);                        // this set is free again: the chunk after next
         const float gC = lgs[C - 1];
         f32x4 u, ud;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            const float gt = lgs[16 * wave + 4 * kq + i];
             u[i] = u0[i] - (accU[i] + accV[i]);
-            ud[i] = u[i] * expf(gC - lgs[16 * wave + 4 * kq + i]);
+            ud[i] = u[i] * expf(gC - gt);
+            if constexpr (OUT) { eg[i] = expf(gt); pc[i] = ap[i]; }
         }
         *(f32x4*)&Vt[r][16 * wave + 4 * kq] = ud;
-        *(f32x4*)(ck + GDN_CK_UT + (VB * cb + r) * C + 16 * wave + 4 * kq) = u;
-        fetch_u(c + 1);                                // (u0 of this chunk is consumed)
+        if constexpr (OUT) *(f32x4*)&Ut[r][16 * wave + 4 * kq] = u;
+        else *(f32x4*)(ck + GDN_CK_UT + (VB * cb + r) * C + 16 * wave + 4 * kq) = u;
+        fetch_u(c + 1);                                // (u0 of this chunk is consumed, its P rows copied)
         lds_barrier();
+        if constexpr (OUT) {                           // ---- Y = e^G (Q S0) + P U ----
+#pragma unroll
+            for (int j = 0; j < 4; ++j) accP = mfma4(pc[j], *(const f32x4*)&Ut[r][16 * j + 4 * kq], accP);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = c * C + 16 * wave + 4 * kq + i;
+                if (t < a.S) a.out[(size_t)t * a.out_stride + h * V + VB * cb + r] = eg[i] * accQ[i] + accP[i];
+            }
+        }
         // ---- S_C = e^{G_C} S0 + K^T (e^{G_C - G} U): wave w owns state rows k = 32 w .. 32 w + 31 ----
         f32x4 sn[2];
         const float eC = expf(gC);
@@ -696,25 +730,25 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
             *(f32x4*)&St[r][32 * wave + 16 * mt + 4 * kq] = sn[mt];
-            if (c + 1 < nchunks) *(f32x4*)(ck + (size_t)a.NV * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + r) * K + 32 * wave + 16 * mt + 4 * kq) = sn[mt];
+            if (!OUT && c + 1 < nchunks) *(f32x4*)(ck + (size_t)a.NV * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + r) * K + 32 * wave + 16 * mt + 4 * kq) = sn[mt];
         }
         park_k(c + 1);
         lds_barrier();
     };
-    fetch_w(0, awA);
+    fetch_w(0, awA, aqA);
     fetch_u(0);
     fetch_k(0);
-    fetch_w(1, awB);
+    fetch_w(1, awB, aqB);
     park_k(0);
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {                      // the state in front of chunk 0
+    for (int i = 0; i < (OUT ? 0 : 2); ++i) {          // the state in front of chunk 0
         const int e = (tid + 256 * i) * 4, col = e >> 7, k = e & 127;
         *(f32x4*)(a.ck + (size_t)h * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + col) * K + k) = *(const f32x4*)&St[col][k];
     }
     for (int c = 0; c < nchunks; c += 2) {
-        chunk(c, awA);
-        if (c + 1 < nchunks) chunk(c + 1, awB);
+        chunk(c, awA, aqA);
+        if (c + 1 < nchunks) chunk(c + 1, awB, aqB);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -821,19 +855,29 @@ void launch_gdn(const GdnArgs& a, hipStream_t s) {
     // prompts: three passes (needs the scratch rows of ensure_prefill_buffers); decode steps and short tails: fused
     if (a.st == nullptr && a.pre_q != nullptr && a.S >= 16 && a.n_seq <= 1) {
         const int nk = a.NV / a.vpg;
-        hipLaunchKernelGGL(gdn_pre_kernel, dim3((a.S + GDN_PT - 1) / GDN_PT, (2 * nk + a.NV + 3) / 4), dim3(256), 0, s, a);
+        const unsigned heads = (unsigned)((2 * nk + a.NV + 3) / 4);
+        // (four tokens per wave where eight leave too few waves: 1.0 us a layer at 17 .. 449 tokens, none from 769 on)
+        if (a.S < 512) hipLaunchKernelGGL(gdn_pre_kernel<4>, dim3((unsigned)((a.S + 3) / 4), heads), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(gdn_pre_kernel<8>, dim3((unsigned)((a.S + 7) / 8), heads), dim3(256), 0, s, a);
         // prompts of a chunk or more: the chunk-parallel scan on the f32 matrix cores (CM_GDN_CHUNKED=0: the sequential scan, A/B)
         static const int ck_env = getenv("CM_GDN_CHUNKED") ? atoi(getenv("CM_GDN_CHUNKED")) : 1;
         if (a.ck != nullptr && a.pre_g != nullptr && ck_env != 0 && a.S >= GDN_CK) {
             static DevOnce attr;
             attr.run([&] {
                 (void)hipFuncSetAttribute((const void*)gdn_chunk_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_prep_lds());
-                (void)hipFuncSetAttribute((const void*)gdn_chunk_scan_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_scan_lds());
+                (void)hipFuncSetAttribute((const void*)gdn_chunk_scan_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_scan_lds(false));
+                (void)hipFuncSetAttribute((const void*)gdn_chunk_scan_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_scan_lds(true));
                 (void)hipFuncSetAttribute((const void*)gdn_chunk_out_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gdn_chunk_out_lds);
             });
-            hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3((a.S + GDN_CK - 1) / GDN_CK, a.NV), dim3(256), gdn_chunk_prep_lds(), s, a);
-            hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3(a.NV, 128 / 16), dim3(256), gdn_chunk_scan_lds(), s, a);
-            hipLaunchKernelGGL(gdn_chunk_out_kernel, dim3((a.S + GDN_CK - 1) / GDN_CK, a.NV), dim3(512), gdn_chunk_out_lds, s, a);
+            const int chunks = (a.S + GDN_CK - 1) / GDN_CK;
+            hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(chunks, a.NV), dim3(256), gdn_chunk_prep_lds(), s, a);
+            if (gdn_out_in_scan(chunks, a.NV)) {
+                hipLaunchKernelGGL(gdn_chunk_scan_kernel<true>, dim3(a.NV, 128 / 16), dim3(256), gdn_chunk_scan_lds(true), s, a);
+                hipLaunchKernelGGL(gdn_post_kernel, dim3(a.S, a.NV), dim3(128), 0, s, a);
+            } else {
+                hipLaunchKernelGGL(gdn_chunk_scan_kernel<false>, dim3(a.NV, 128 / 16), dim3(256), gdn_chunk_scan_lds(false), s, a);
+                hipLaunchKernelGGL(gdn_chunk_out_kernel, dim3(chunks, a.NV), dim3(512), gdn_chunk_out_lds, s, a);
+            }
             return;
         }
         hipLaunchKernelGGL(gdn_scan_kernel, dim3(a.NV, 4), dim3(512), 0, s, a);

@@ -1,5 +1,5 @@
-"""GPU: the chunk-parallel Gated-Delta-Net pass (scan over the states, outputs of all chunks at once) against the sequential scan, at the edges of its
-chunks of 64 tokens, from an empty state and from one that an earlier portion left, with one and two value heads per key head.
+"""GPU: the chunk-parallel Gated-Delta-Net pass (scan over the states, the outputs inside it for up to five chunks and 32 heads, else of all chunks at once) against the sequential scan, at the edges of its
+chunks of 64 tokens, from an empty state and from one that an earlier portion left, with one, two and three value heads per key head.
 
 Both are f32 throughout and differ in the order of their sums (and in decays as a sum of logarithms): 1e-4 of the largest logit, the bar of the prompt
 passes against the oracle."""
@@ -11,7 +11,7 @@ from crane_amd import configs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("values", [16, 32])
+@pytest.mark.parametrize("values", [16, 32, 48])
 def test_against_the_sequential_scan(values):
     from crane_amd.backend import Model
     cfg = dict(configs.get_config("qwen3.5-0.8b"), vocab_size=512, num_hidden_layers=4)
@@ -20,7 +20,7 @@ def test_against_the_sequential_scan(values):
     m = Model.synthetic(cfg, seed=5, max_seq_len=1024, max_seqs=2, kv_dtype="f32")
     rng = np.random.default_rng(values)
     try:
-        for n in (64, 65, 127, 128, 129, 200, 321):
+        for n in (64, 65, 127, 128, 129, 200, 320, 321, 512):
             ids, more = rng.integers(0, 512, n).tolist(), rng.integers(0, 512, 64 + n % 63).tolist()
             out = []
             for on in (1, 0):
