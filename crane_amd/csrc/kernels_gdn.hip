@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs a) {
 // ---------------------------------------------------------------------------------------------------------
 // A wave takes one head (q, k or v; lane l its channels 2 l, 2 l + 1) over PT tokens: the convolution's window rolls in registers, a row is read
 // once instead of four times, norms need no other wave.  Bound by its traffic (a workgroup per token and head was bound by the 65 536 workgroups of a
-// 2048-token pass: mean per launch of a 4165-token prompt 31.7 -> 21.2 us).  The rolling window that the next call reads is written by the wave that read
+// 2048-token pass: mean per launch of a 4165-token prompt 31.7 -> 20.2 us).  The rolling window that the next call reads is written by the wave that read
 // the one of this call: both may be the same memory.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <int PT>

@@ -85,8 +85,8 @@ struct Query {
     static constexpr bool EXACT = PARTS == 3;
     static constexpr float UNIT = EXACT ? 1.f : L2E;
     // the scores' loops take what lies in front and move the rest up: rolled where the functions are long.  A decode launch has about one key tile per
-    // wave and waits for its own code: with sixteen expf in a row it was 4 us longer than with sixteen v_exp_f32, with eight in a loop of two it is not
-    // (24 layers of width 1024, 8 tokens at 1000: 13.09 ms with v_exp_f32, 13.88 in a row, as long as with v_exp_f32 in the loop)
+    // wave and waits for its own code: with sixteen expf in a row it is 4 us longer than with sixteen v_exp_f32, with eight in a loop of two 0.9 (8 heads on
+    // 2 of 128, context 1000: 13.3 us against 12.4)
     static constexpr int ROLL = EXACT ? 1 : 4;
     static __device__ __forceinline__ float ex(float x) { return EXACT ? expf(x) : __builtin_amdgcn_exp2f(x); }
     bool ok;

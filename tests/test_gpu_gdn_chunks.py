@@ -1,5 +1,6 @@
-"""GPU: the chunk-parallel Gated-Delta-Net pass (scan over the states, the outputs inside it for up to five chunks and 32 heads, else of all chunks at once) against the sequential scan, at the edges of its
-chunks of 64 tokens, from an empty state and from one that an earlier portion left, with one, two and three value heads per key head.
+"""GPU: the chunk-parallel Gated-Delta-Net pass (the outputs inside the scan over the states for up to five chunks and 32 heads, else of all chunks
+at once) against the sequential scan, at the edges of its chunks of 64 tokens, from an empty state and from one that an earlier portion left, with
+one, two and three value heads per key head.
 
 Both are f32 throughout and differ in the order of their sums (and in decays as a sum of logarithms): 1e-4 of the largest logit, the bar of the prompt
 passes against the oracle."""
