@@ -9,13 +9,18 @@
 //
 // Which (row tile, expert) a block has follows from the group offsets in device memory: the tiles of all experts are numbered through and
 // every block finds its own with one scan over the offsets (at most 64 experts: a wave's lanes), so the grid is rows / BM + experts tiles
-// high whatever the router chose -- not experts x rows / BM, of which a 16-expert launch filled a quarter.  Tiles that share weight
-// columns have consecutive numbers on one XCD: its L2 serves them.
+// high whatever the router chose -- not experts x rows / BM, of which a 16-expert launch filled a quarter.  Numbered by expert, then column tile, then
+// row tile, each XCD a contiguous share of the real count: an XCD's 64 blocks share their expert's gathered rows as well as weight columns (row tiles
+// of all experts under one column tile: every XCD read all rows once per two column tiles, 1.6 GB a launch at the first size below, 4 TB/s;
+// 402 / 264 us there, 132 for 99 with 300 tokens).  The expert of every token rides in the same launches: its tiles
+// fill what the routed ones leave of the last round of blocks, and two launches less (a mixed step of 326 rows, 24 layers of width 1024: 54 us a layer
+// of the four products in four launches, 37 in two).  A wave whose rows lie behind a ragged tile's end loads its share and multiplies nothing.
 //
 // Bound: LDS.  A wave's k-step of 64 x 64 outputs reads 8 KB of fragments for 16 products (256 cycles); four waves of two blocks ask for the
 // LDS ports' full 128 bytes a cycle.  64 x 64 tiles: the latency of the weights' first touch and the L2's traffic per product.
 // Measured (us per launch, gate-and-up / down; the 64 x 64 kernel without a pipeline that this replaces in brackets): 8192 rows, 16 experts of
-// 2048 x 4096: 395 / 235 (2481 / 1566), 0.70 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 22.5 / 14.2 (60 / 50).
+// 2048 x 4096: 375 / 243 (2481 / 1566), 0.73 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 14.8 / 11.1 (60 / 50).  Tiles of 128 x 256 and 256 x 256
+// with eight waves: 388 and 396 at the first size (coarser shares of the last round), 70 for 75 on one matrix of 4096 x 4096; not kept.
 #include <algorithm>
 
 #include "dev_common.h"
@@ -29,34 +34,97 @@ namespace {
 
 constexpr int BK = 64;
 
+// a block's tile: sorted rows [p0, p0 + rows) of group g, column tile nt, of the launch's first product or (side) its second; false: a block behind
+// the last tile.  Every XCD takes a contiguous share of either product's tiles, numbered by group, then column tile, then row tile
+struct Tile { int g, p0, rows, nt; bool side; };
+template <int BM>
+__device__ __forceinline__ bool find_tile(const LTileArgs& a, const LTileArgs& b, int ntiles, int ntiles_b, int lane, Tile& t) {
+    int o0 = 0, o1 = a.M;
+    if (a.grp_off) {
+        o1 = 0;
+        if (lane < a.groups) { o0 = a.grp_off[lane]; o1 = a.grp_off[lane + 1]; }
+    }
+    const int mine = (o1 - o0 + BM - 1) / BM;
+    int incl = mine;
+    if (a.grp_off) {
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(incl, d); if (lane >= d) incl += v; }
+    }
+    const int total = __builtin_amdgcn_readlane(incl, 63) * ntiles, share = (total + 7) >> 3;
+    const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
+    t.side = slot >= share;
+    if (t.side) {
+        const int mb = (b.M + BM - 1) / BM, total_b = mb * ntiles_b, share_b = (total_b + 7) >> 3, at = xcd * share_b + slot - share;
+        if (slot - share >= share_b || at >= total_b) return false;
+        t.g = 0;
+        t.nt = at / mb;
+        t.p0 = (at - t.nt * mb) * BM;
+        t.rows = min(BM, b.M - t.p0);
+        return true;
+    }
+    const int at = xcd * share + slot;
+    if (at >= total) return false;
+    t.g = a.grp_off ? __builtin_ctzll(__ballot(at < incl * ntiles)) : 0;
+    const int m = __builtin_amdgcn_readlane(mine, t.g), local = at - (__builtin_amdgcn_readlane(incl, t.g) - m) * ntiles;
+    t.nt = local / m;
+    t.p0 = __builtin_amdgcn_readlane(o0, t.g) + (local - t.nt * m) * BM;
+    t.rows = min(BM, __builtin_amdgcn_readlane(o1, t.g) - t.p0);
+    return true;
+}
+
+// field by field: a choice between the two by reference puts them into scratch memory (6 us a launch)
+__device__ __forceinline__ void take(LTileArgs& a, const LTileArgs& b) {
+    a.A = b.A; a.lda = b.lda; a.a_idx = nullptr; a.W = b.W; a.W2 = b.W2; a.w_stride = 0; a.C = b.C; a.ldc = b.ldc; a.c_idx = nullptr;
+    a.M = b.M; a.N = b.N; a.K = b.K; a.grp_off = nullptr; a.bias = b.bias; a.act = b.act; a.act2 = b.act2; a.act_split = b.act_split; a.act_param = b.act_param;
+}
+
+// a wave's NI x NJ products to memory, rows mw .. and columns nw .. of the tile.  D of a product: column = lane % 16, rows 4 (lane / 16) + r.  DUAL: the
+// upper half of the NJ columns belongs to W2.  The outputs' function is chosen once per block
+template <int NI, int NJ, bool DUAL>
+__device__ __forceinline__ void store_tile(const LTileArgs& a, const f32x4 (&acc)[NI][NJ], int rows, int p0, int mw, int nw, int lane) {
+    constexpr int NC = DUAL ? NJ / 2 : NJ;
+    const int fr = lane & 15, lg = lane >> 4;
+    auto store = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = mw + i * 16 + lg * 4 + r;
+                if (m >= rows) continue;
+                const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
+#pragma unroll
+                for (int j = 0; j < NC; ++j) {
+                    const int n = nw + j * 16 + fr;
+                    if (n >= a.N) continue;
+                    if (DUAL) ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(f(acc[i][j][r], acc[i][j + (DUAL ? NC : 0)][r], n));
+                    else ((float*)a.C)[row * a.ldc + n] = f(acc[i][j][r], 0.f, n);
+                }
+            }
+    };
+    if (DUAL) {
+        if (a.act == LACT_SILU) store([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
+        else if (a.act == LACT_CAPGLU) store([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
+        else store([&](float v, float u, int) { return lay_act(v, a.act) * u; });
+    } else if (!a.bias && a.act == LACT_NONE && a.act2 == LACT_NONE) store([](float v, float, int) { return v; });
+    else store([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+}
+
 template <int BM, int BN, int ST, bool DUAL>
-__global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int mtiles, int ntiles) {
+__global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, LTileArgs second, int ntiles, int ntiles_b) {
     constexpr int WM = BM / 2, WN = BN / 2, NI = WM / 16, NJ = WN / 16, APC = BM / 8, NL = (BM + BN) / 32;      // NL: loads per wave and k-tile
     constexpr int NC = DUAL ? WN / 2 : WN;                                // output columns of a wave
     constexpr int STAGE = (BM + BN) * BK;
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
-    const int per = (int)gridDim.x >> 3, bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-    if (bid >= mtiles * ntiles) return;
-    const int nt = bid / mtiles, mt = bid - nt * mtiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    int g = 0, p0 = mt * BM, rows = min(BM, a.M - p0);
-    if (a.grp_off) {
-        int o0 = 0, o1 = 0;
-        if (lane < a.groups) { o0 = a.grp_off[lane]; o1 = a.grp_off[lane + 1]; }
-        const int mine = (o1 - o0 + BM - 1) / BM;
-        int incl = mine;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(incl, d); if (lane >= d) incl += v; }
-        const unsigned long long reach = __ballot(mt < incl);
-        if (reach == 0) return;                                           // behind the last expert's last tile
-        g = __builtin_ctzll(reach);
-        p0 = __builtin_amdgcn_readlane(o0, g) + (mt - __builtin_amdgcn_readlane(incl - mine, g)) * BM;
-        rows = min(BM, __builtin_amdgcn_readlane(o1, g) - p0);
-    }
-    const uint16_t* W = a.W + (size_t)g * a.w_stride;
-    const uint16_t* W2 = DUAL ? a.W2 + (size_t)g * a.w_stride : nullptr;
+    Tile at;
+    if (!find_tile<BM>(first, second, ntiles, ntiles_b, lane, at)) return;
+    LTileArgs a = first;
+    if (at.side) take(a, second);
+    const int p0 = at.p0, rows = at.rows, nt = at.nt;
+    const uint16_t* W = a.W + (size_t)at.g * a.w_stride;
+    const uint16_t* W2 = DUAL ? a.W2 + (size_t)at.g * a.w_stride : nullptr;
     const int n0 = nt * (DUAL ? BN / 2 : BN);
 
     // this lane's share of the loads: piece wave + 4 i covers 8 rows of A (pieces below APC) or of the weight tile.  Rows past the end repeat
@@ -95,12 +163,14 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int 
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int fr = lane & 15, lg = lane >> 4, sw = (fr >> 1) & 7;
+    const bool idle = wm * WM >= rows;                                    // a ragged tile's lower half: this wave loads, the matrix cores are the others'
 #pragma unroll
     for (int t = 0; t < ST - 1; ++t) request(t);
     for (int t = 0; t < nk; ++t) {
         // this wave's share of tile t has landed and its reads of tile t - 1 are done; behind the barrier that holds for every wave
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((ST - 2) * NL) : "memory");
         request(t + ST - 1);
+        if (idle) continue;
         const uint16_t* As = lds + (t % ST) * STAGE + wm * WM * BK;
         const uint16_t* Bs = lds + (t % ST) * STAGE + (BM + wn * WN) * BK;
 #pragma unroll
@@ -118,30 +188,7 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs a, int 
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail: none may land after the block is gone
-    // D of a product: column = lane % 16, rows 4 (lane / 16) + r.  f: the outputs' function, chosen once per block
-    auto store = [&](auto f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = wm * WM + i * 16 + lg * 4 + r;
-                if (m >= rows) continue;
-                const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
-#pragma unroll
-                for (int j = 0; j < NC / 16; ++j) {
-                    const int n = n0 + wn * NC + j * 16 + fr;
-                    if (n >= a.N) continue;
-                    if (DUAL) ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(f(acc[i][j][r], acc[i][j + (DUAL ? NJ / 2 : 0)][r], n));
-                    else ((float*)a.C)[row * a.ldc + n] = f(acc[i][j][r], 0.f, n);
-                }
-            }
-    };
-    if (DUAL) {
-        if (a.act == LACT_SILU) store([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
-        else if (a.act == LACT_CAPGLU) store([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
-        else store([&](float v, float u, int) { return lay_act(v, a.act) * u; });
-    } else if (!a.bias && a.act == LACT_NONE && a.act2 == LACT_NONE) store([](float v, float, int) { return v; });
-    else store([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+    store_tile<NI, NJ, DUAL>(a, acc, rows, p0, wm * WM, n0 + wn * NC, lane);
 }
 
 // row tiles of a launch; grouped: every expert ends in at most one ragged tile, and none has more than M rows
@@ -151,31 +198,33 @@ int mtiles(const LTileArgs& a) {
 }
 
 template <int BM, int BN, int ST, bool DUAL>
-void go(const LTileArgs& a, hipStream_t s) {
+void go(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
     constexpr size_t lds = (size_t)ST * (BM + BN) * BK * sizeof(uint16_t);
     static DevOnce attr;
     attr.run([&] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tile_gemm_kernel<BM, BN, ST, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    const int cols = DUAL ? BN / 2 : BN, mt = mtiles<BM>(a), nt = (a.N + cols - 1) / cols;
-    hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL>), dim3((unsigned)((mt * nt + 7) / 8 * 8)), dim3(256), lds, s, a, mt, nt);
+    const int cols = DUAL ? BN / 2 : BN, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
+    const int share = (mtiles<BM>(a) * nt + 7) / 8 + ((b.M + BM - 1) / BM * ntb + 7) / 8;
+    hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL>), dim3((unsigned)share * 8), dim3(256), lds, s, a, b, nt, ntb);
 }
 
 }  // namespace
 
 bool lay_tile_gemm_fits(int N, int K, int groups) { return N > 0 && K >= 2 * BK && K % BK == 0 && groups <= 64; }
 
-void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s) {
+void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s, const LTileArgs* beside) {
     if (a.M <= 0 || a.N <= 0) return;
+    const LTileArgs b = beside ? *beside : LTileArgs();
     // 128 x 128 tiles where they still give the chip 320 blocks and a group fills half a tile of rows; measured (us, gate-and-up, 128 / 64
-    // tiles): 16 experts of 2048 x 4096 -- 2048 tokens 395 / 685, 300 tokens (75 rows, 832 blocks) 156 / 168, 128 tokens (32 rows) 151 / 142;
-    // 14 of 768 x 1024 -- 2048 tokens 63 / 75, 700 tokens (432 blocks) 35 / 34; one matrix pair 2048 x 4096 -- 1200 rows (320 blocks) 66 / 79,
+    // tiles): 16 experts of 2048 x 4096 -- 2048 tokens 375 / 541, 300 tokens (75 rows, 832 blocks) 99 / 138, 128 tokens (32 rows) 151 / 142;
+    // 14 of 768 x 1024 -- 2048 tokens 49 / 55, 700 tokens (432 blocks) 25 / 24; one matrix pair 2048 x 4096 -- 1200 rows (320 blocks) 66 / 79,
     // 600 rows (160) 64 / 46
     const int total = a.grp_off ? a.total : a.M, groups = a.grp_off ? a.groups : 1;
     const int blocks = mtiles<128>(a) * ((a.N + (a.W2 ? 63 : 127)) / (a.W2 ? 64 : 128));
     const bool wide = blocks >= LAY_TILE_WIDE_BLOCKS && total >= 64 * groups;
-    if (a.W2) { if (wide) go<128, 128, 2, true>(a, s); else go<64, 64, 3, true>(a, s); }
-    else { if (wide) go<128, 128, 2, false>(a, s); else go<64, 64, 3, false>(a, s); }
+    if (a.W2) { if (wide) go<128, 128, 2, true>(a, b, s); else go<64, 64, 3, true>(a, b, s); }
+    else { if (wide) go<128, 128, 2, false>(a, b, s); else go<64, 64, 3, false>(a, b, s); }
 }
 
 // rows of f32, gathered and scaled -> bfloat16: out[p] = x[idx[p] / div] * scale[idx[p]]

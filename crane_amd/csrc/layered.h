@@ -233,7 +233,8 @@ struct LTileArgs {
 };
 constexpr int LAY_TILE_WIDE_BLOCKS = 320;       // 128 x 128 tiles from this many blocks on (launch_lay_tile_gemm)
 bool lay_tile_gemm_fits(int N, int K, int groups);
-void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s);
+// beside: a second product of as many matrices, not grouped, its rows neither gathered nor scattered, in the same launch
+void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s, const LTileArgs* beside = nullptr);
 void launch_lay_round_scaled(const float* x, int ldx, const int32_t* idx, int div, const float* scale, uint16_t* out, int P, int K, hipStream_t s);
 
 void launch_lay_act_cols(float* C, int ldc, int M, int N, int act, int act2, int split, hipStream_t s, float param = 1.f);

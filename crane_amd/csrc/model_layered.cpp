@@ -157,26 +157,28 @@ static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const Layered
         sdn.N = W; sdn.K = sp.shared_ff;
     }
     const bool tiles = !L.f32 && L.shared_gemm && L.Abf && T > LAY_ROW_KERNEL_ROWS && (!sp.scale_input || L.Asc);
-    auto tile = [&](const LGemmArgs& g, const uint16_t* A, bool gather) {
+    auto tile_args = [&](const LGemmArgs& g, const uint16_t* A, bool gather) {
         LTileArgs t;
         t.A = A; t.lda = g.K; t.W = g.W; t.W2 = g.W2; t.w_stride = g.w_stride; t.C = g.C; t.ldc = g.ldc; t.c_idx = g.c_idx;
         t.M = g.M; t.N = g.N; t.K = g.K; t.act = g.act; t.act_param = g.act_param;
         if (gather) { t.a_idx = g.a_idx; t.a_div = g.a_div; }
         if (g.grp_off) { t.grp_off = g.grp_off; t.groups = sp.experts; t.total = T * sp.top; }
-        launch_lay_tile_gemm(t, s);
+        return t;
     };
     const bool routed = tiles && lay_tile_gemm_fits(sp.ff, W, sp.experts) && lay_tile_gemm_fits(W, sp.ff, sp.experts);
     const bool shared = tiles && every && lay_tile_gemm_fits(sp.shared_ff, W, 1) && lay_tile_gemm_fits(W, sp.shared_ff, 1);
     if (!h16 && ((routed && !sp.scale_input) || shared)) launch_lay_round_rows(h, W, L.Abf, T, W, s);
     const uint16_t* A = h16 ? h16 : L.Abf;
+    // the expert of every token beside the routed ones, in their launches: its tiles fill what they leave of the last round of blocks
+    LTileArgs shu, shd;
+    if (shared) { shu = tile_args(su, A, false); shd = tile_args(sdn, (const uint16_t*)L.HS, false); }
     if (routed) {
         if (sp.scale_input) launch_lay_round_scaled(h, W, L.srt, slots, L.wsel, L.Asc, T * sp.top, W, s);
-        tile(gu, sp.scale_input ? L.Asc : A, !sp.scale_input);
-        tile(dn, (const uint16_t*)L.HH, false);
-    }
-    if (shared) {
-        tile(su, A, false);
-        tile(sdn, (const uint16_t*)L.HS, false);
+        launch_lay_tile_gemm(tile_args(gu, sp.scale_input ? L.Asc : A, !sp.scale_input), s, shared ? &shu : nullptr);
+        launch_lay_tile_gemm(tile_args(dn, (const uint16_t*)L.HH, false), s, shared ? &shd : nullptr);
+    } else if (shared) {
+        launch_lay_tile_gemm(shu, s);
+        launch_lay_tile_gemm(shd, s);
     }
     const bool beside = every && T <= LAY_ROW_KERNEL_ROWS;        // decode steps: the expert of every token rides in the same two launches
     if (beside) {

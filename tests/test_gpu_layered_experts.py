@@ -46,6 +46,13 @@ def test_softmax_routed_experts_and_a_shared_one(tmp_path, n, width, ff, shared,
     _check(tmp_path, GZ, cfg, n, 3)
 
 
+# the expert of every token in the routed ones' launches: deeper, wider and narrower than they are
+@pytest.mark.parametrize("ff,shared", [(128, 320), (320, 128)])
+def test_a_shared_expert_of_another_size(tmp_path, ff, shared):
+    cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=5, top=2, ff=ff, shared=shared))], vocab=96, width=192)
+    _check(tmp_path, GZ, cfg, 137, 9)
+
+
 # 128 x 128 tiles: enough rows and columns for 320 of them
 def test_wide_tiles(tmp_path):
     cfg = GZ.config([GZ.layer(GZ.attn(), GZ.moe(experts=8, top=4, ff=576, shared=192))], vocab=96, width=1216)
