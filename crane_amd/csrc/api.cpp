@@ -599,6 +599,7 @@ int cm_debug_set(cm_model* h, const char* key, int64_t value) {
         // which decode-attention kernel / persistent-kernel mode a step uses (tests and A/B runs; one hipGraph per variant, so
         // the thresholds switch live -- a switch that changes what a variant enqueues drops the captured graphs)
         else if (k == "attn_mfma_min") mm.attn_mfma_min = value;
+        else if (k == "attn_group") mm.attn_group = value != 0;
         else if (k == "attn_mfma_wide_min") mm.attn_mfma_wide_min = value;
         else if (k == "attn_heads_max") mm.attn_heads_max = value;
         else if (k == "attn_ns") { mm.attn_ns = (int)std::max<long long>(1, std::min<long long>(value, mm.nsplit)); mm.drop_graphs(); }

@@ -282,6 +282,11 @@ void launch_argmax_final(const float* pmax, const int* pidx, int n, StepState* s
                          int ring_mask, int advance, int n_seq, hipStream_t s, int slabs = 1, size_t slab_stride = 0);
 bool attn_decode_single_split(int nsplit, int D);     // launch_attn_decode(_mfma) will write the final output itself (AttnDecArgs::out1)
 bool launch_attn_decode_mfma(const AttnDecArgs& a, int D, int nrep, int nsplit, int kv_mode, float* out, int out_stride, int n_seq, hipStream_t s);
+// groups over 16-bit pages (kernels_attn_group.hip): 64 tokens per wave and step, queries and weights in 24 bits.  The rows leave finished (out1_*, as
+// launch_attn_decode_mfma with one split leaves them; out1 always set) for any nsplit; several: part_o / part_ml hold [heads][nsplit] sums in between
+bool attn_decode_group_fits(int head_dim, int nrep, int kv_mode, int page, int rot_dim);
+int attn_decode_group_split(int64_t longest, int pairs, int num_cu, int most);
+bool launch_attn_decode_group(const AttnDecArgs& a, int nrep, int kv_mode, int nsplit, int n_seq, hipStream_t s);
 bool launch_attn_decode_heads(const AttnDecArgs& a, int D, int nrep, int ns, bool kv_f32, int n_seq, hipStream_t s);
 bool launch_attn_decode(const AttnDecArgs& a, int D, int nrep, int nsplit, int kv_mode, float* out, int out_stride, int n_seq,
                         hipStream_t s);

@@ -2009,12 +2009,17 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 // nb sequences already multiply the block count: fewer token splits per sequence keep ~2 blocks per CU
                 const int ns_b = mf ? std::max(attn_batch_ns_min, std::min(longest >= attn_mfma_wide_min ? nsplit_mfma : nsplit, 2 * num_cu / std::max(1, Hkv_l * nb)))
                                     : (attn_splits_force ? attn_splits_force : std::max(attn_batch_ns_min, std::min(nsplit, 2 * num_cu / std::max(1, Hkv_l * nb))));
+                // 16-bit pages, head_dim 128: the group kernel, whole sequences or large shares of them per block.  A few sequences of some hundred tokens
+                // stay with the kernels above, whose many splits reach more CUs (3 up to 500 tokens: 11.0 us against 12.6; up to 200 10.3 against 9.2)
+                const bool grp = attn_group && !attn_splits_force && attn_decode_group_fits(D, nrep, kv_mode, page, cfg.rot_dim) &&
+                                 (Hkv_l * nb >= 48 || longest <= 256);
+                const int ns_g = grp ? attn_decode_group_split(longest, Hkv_l * nb, num_cu, std::max(nsplit, nsplit_mfma)) : 1;
                 // the single-split matrix-core kernel of a quantised group: adds the K-split slices of the int8 qkv GEMM in its prologue (no
                 // reduction launch) and writes the Q8_0 blocks of its rows for the int8 o_proj GEMM (no quantiser launch)
-                const bool attn_q = attn_outq && mf && qgemm_ok && nb >= q_gemm_min && attn_decode_single_split(ns_b, D) && !cfg.hybrid &&
+                const bool attn_q = attn_outq && qgemm_ok && nb >= q_gemm_min && (grp || (mf && attn_decode_single_split(ns_b, D))) && !cfg.hybrid &&
                                     !(heads_b && !quantized && !rccl);
                 const bool codes_ok = attn_outq && qgemm_ok && nb >= q_gemm_min && !cfg.hybrid && !(heads_b && !quantized && !rccl) &&
-                                      (mf || !attn_decode_single_split(ns_b, D));
+                                      (grp || mf || !attn_decode_single_split(ns_b, D));
                 QDefer qdef{1, 0, nullptr};
                 if (quantized) {
                     const bool defer_ok = attn_q && w.n_qkv == 1 && ldq == w.q_qkv[0].N && w.qkv_row0[0] == 0;
@@ -2051,7 +2056,10 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 const bool codes = codes_ok && gemm_q8_ok(w.q_o, nb) && w.q_o.fmt == QFMT_Q8_0 && (Hq_l * D) % 64 == 0;
                 if (codes) { a.out1_q = qx_codes; a.out1_qd = qx_scales; a.out1_cols = Hq_l * D; }
                 if (qdef.ks > 1) { a.qkv = qdef.ws; a.qkv_stride = w.q_qkv[0].N; a.qkv_ns = qdef.ks; a.qkv_slice = qdef.slice; }      // (the slices of the qkv GEMM, rows N floats apart)
-                if (mf) {
+                if (grp) {
+                    a.out1 = attnb; a.out1_stride = (int)at_cols;
+                    if (!launch_attn_decode_group(a, nrep, kv_mode, ns_g, nb, s)) throw CmError(CM_ERR_UNSUPPORTED, "GQA group size / head_dim");
+                } else if (mf) {
                     if (!launch_attn_decode_mfma(a, D, nrep, ns_b, kv_mode, attnb, (int)at_cols, nb, s)) throw CmError(CM_ERR_UNSUPPORTED, "GQA group size / head_dim");
                 } else if (!launch_attn_decode(a, D, nrep, ns_b, kv_mode, attnb, (int)at_cols, nb, s)) throw CmError(CM_ERR_UNSUPPORTED, "GQA group size / head_dim");
                 if (codes) { qx_src = attnb; qx_nw = nullptr; qx_K = Hq_l * D; qx_kind = 0; if (q_capture) q_capture_rows(nb, Hq_l * D); }      // (the codes hold the attention rows)

@@ -396,6 +396,7 @@ int prefill_lo_mask = 0;              // EXPERIMENT (cm_debug_set "prefill_lo_ma
     bool gdn_ba_fused = true;             // quantised hybrid decode: the GDN step computes its head's bf16 a / b projections itself (cm_debug_set("gdn_ba_fused"))
     bool gdn_defer_norm = true;           // CM_GDN_DEFER_NORM / cm_debug_set("gdn_defer_norm"): gated RMSNorm in out_proj's prologue
     int attn_batch_ns_min = 1;            // fewest token splits per sequence in the batched decode attention (CM_ATTN_BATCH_NS_MIN)
+    bool attn_group = true;                // groups over 16-bit pages: attn_decode_group_kernel where it fits (cm_debug_set("attn_group", 0): never)
     int64_t attn_mfma_min_batch = 64;     // matrix-core decode attention from this context on when the group fills the chip (CM_ATTN_MFMA_MIN_BATCH)
         int64_t attn_mfma_min = 768;   // contexts of at least this many tokens use the MFMA kernel (CM_ATTN_MFMA_MIN; 0 = never);
                                    // Qwen3-8B ms/token split vs MFMA(32 splits): 256: 3.056 / 3.068, 1 K: 3.11 / 3.085, 4 K: 3.44 / 3.26
