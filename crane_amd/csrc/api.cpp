@@ -339,7 +339,7 @@ int cm_prefill_batch(cm_model* h, const int32_t* seqs, const uint32_t* const* id
         m.prefill_multi(seqs, ids, lens, n, out_or(primary, greedy_out, tg, n));
         if (logits_out && primary) {
             m.ensure_batch_buffers();
-            CM_HIP(hipMemcpy(logits_out, m.logitsb, n * (size_t)m.cfg.V * sizeof(float), hipMemcpyDeviceToHost));
+            m.read_back(logits_out, m.logitsb, n * (size_t)m.cfg.V * sizeof(float));
         }
     });
 }
@@ -388,10 +388,7 @@ int cm_vision_encode(cm_model* h, const float* pixel_values, size_t n_patches, c
         const int rows = m.vision_encode(pixel_values, n_patches, grid_thw, n_images);
         if (!primary) return;
         if (rows_out) *rows_out = (size_t)rows;
-        if (features_out) {
-            CM_HIP(hipStreamSynchronize(m.stream));
-            CM_HIP(hipMemcpy(features_out, m.vFeat, (size_t)rows * m.vcfg.out_hidden * sizeof(float), hipMemcpyDeviceToHost));
-        }
+        if (features_out) m.read_back(features_out, m.vFeat, (size_t)rows * m.vcfg.out_hidden * sizeof(float));
     });
 }
 

@@ -230,7 +230,11 @@ struct Model {
     uint32_t ring_count = 0;           // host mirror of StepState.pad
     StepState* h_st = nullptr;         // pinned
     uint32_t* h_ring = nullptr;        // pinned
-    float* h_logits = nullptr;         // pinned [V]
+    // pinned ring in front of the caller's memory (read_back): the copy out of it of one piece runs beside the transfer of the next
+    static constexpr size_t STAGE_PIECE = 4u << 20;
+    static constexpr int STAGES = 4;
+    char* h_stage = nullptr;
+    hipEvent_t ev_stage[STAGES] = {};
 
     // prefill scratch (allocated on first use; sized for one chunk)
     int chunk = 2048, chunk_pad = 2048;
@@ -273,7 +277,6 @@ struct Model {
     int32_t* h_btb = nullptr;          // pinned
     float *xb = nullptr, *qkvb = nullptr, *attnb = nullptr, *hbb = nullptr, *logitsb = nullptr, *part_ob = nullptr, *part_mlb = nullptr, *pmaxb = nullptr;
     int* pidxb = nullptr;
-    float* h_logitsb = nullptr;
     int ldq = 0;
     void ensure_batch_buffers();
     // after_group(g0, nb): called once per <= MAXB group after the stream is idle; logitsb[b * V] (b < nb) is valid
@@ -473,6 +476,8 @@ int prefill_lo_mask = 0;              // EXPERIMENT (cm_debug_set "prefill_lo_ma
     void bench_kernel(const std::string& which, size_t iters, float* ms, uint64_t* bytes);
     uint64_t decode_bytes_per_token(size_t ctx) const;
     void fetch_logits(float* out);
+    void ensure_stage();
+    void read_back(void* out, const void* dev, size_t bytes);      // behind what the stream holds; waits
 };
 
 // loaders (loader.cpp)

@@ -58,7 +58,7 @@ struct Layered {
           *wsel = nullptr, *Xw = nullptr;
     int32_t *sel = nullptr, *srt = nullptr, *off = nullptr;
     uint32_t *d_greedy = nullptr, *h_greedy = nullptr;
-    float* h_rows = nullptr;           // pinned staging of logits rows
+    bool keep_row = false;             // layered_forward: the pass leaves its last row in Model::logits as well
     int32_t *d_tab = nullptr, *h_tab = nullptr;
     size_t tab_ints = 0;
     static constexpr int LOGIT_ROWS = 256;
@@ -83,7 +83,6 @@ struct Layered {
     std::vector<float> captured;
     ~Layered() {
         if (h_greedy) (void)hipHostFree(h_greedy);
-        if (h_rows) (void)hipHostFree(h_rows);
         if (h_tab) (void)hipHostFree(h_tab);
     }
 };
@@ -1519,8 +1518,7 @@ void Model::alloc_runtime_layered() {
     logitsb = dalloc<float>((size_t)Layered::LOGIT_ROWS * cfg.V);
     logits = dalloc<float>((size_t)cfg.V);
     V_l = cfg.V;
-    CM_HIP(hipHostMalloc((void**)&h_logits, (size_t)cfg.V * sizeof(float)));
-    CM_HIP(hipHostMalloc((void**)&L.h_rows, (size_t)Layered::LOGIT_ROWS * cfg.V * sizeof(float)));
+    ensure_stage();
     L.d_greedy = dalloc<uint32_t>(Layered::LOGIT_ROWS);
     CM_HIP(hipHostMalloc((void**)&L.h_greedy, Layered::LOGIT_ROWS * sizeof(uint32_t)));
     // one table upload per pass: ids | rowseg | wanted rows | segments | page tables | attention tiles per group size
@@ -2221,10 +2219,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 launch_lay_argmax_rows(logitsb, V, V, L.d_greedy, nr, L.am_pv, L.am_pi, s);
                 CM_HIP(hipMemcpyAsync(L.h_greedy, L.d_greedy, (size_t)nr * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
             }
-            if (logits_out) CM_HIP(hipMemcpyAsync(L.h_rows, logitsb, (size_t)nr * V * sizeof(float), hipMemcpyDeviceToHost, s));
-            if (greedy_out || logits_out || w0 + nr < nw) CM_HIP(hipStreamSynchronize(s));
+            if (L.keep_row) CM_HIP(hipMemcpyAsync(logits, logitsb, (size_t)V * sizeof(float), hipMemcpyDeviceToDevice, s));
+            if (logits_out) read_back(logits_out + out_row * (size_t)V, logitsb, (size_t)nr * V * sizeof(float));
+            else if (greedy_out || w0 + nr < nw) CM_HIP(hipStreamSynchronize(s));
             if (greedy_out) memcpy(greedy_out + out_row, L.h_greedy, (size_t)nr * sizeof(uint32_t));
-            if (logits_out) memcpy(logits_out + out_row * (size_t)V, L.h_rows, (size_t)nr * V * sizeof(float));
             out_row += (size_t)nr;
         }
     }
@@ -2239,11 +2237,11 @@ void Model::layered_forward(int sq, const uint32_t* ids, size_t n, size_t start_
     if ((int64_t)start_pos < q.len) seq_truncate(sq, start_pos);     // only to 0: the recurrent state cannot be rewound
     StepItem it{sq, ids, n, nullptr, -1};
     uint32_t g = 0;
-    step_batch(&it, 1, logits_out, &g);
-    if (greedy_out) *greedy_out = g;
     // the last row's logits are also what cm_sample / cm_read_logits look at
-    CM_HIP(hipMemcpyAsync(logits, logitsb, (size_t)cfg.V * sizeof(float), hipMemcpyDeviceToDevice, stream));
-    CM_HIP(hipStreamSynchronize(stream));
+    lay->keep_row = true;
+    try { step_batch(&it, 1, logits_out, &g); } catch (...) { lay->keep_row = false; throw; }
+    lay->keep_row = false;
+    if (greedy_out) *greedy_out = g;
 }
 
 uint64_t Model::layered_decode_bytes(size_t ctx) const {
