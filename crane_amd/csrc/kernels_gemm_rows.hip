@@ -9,11 +9,10 @@
 // without passing registers (8 rows x 128 bytes per wave instruction, the bank swizzle on the source address: slot p of a row holds its 16-byte
 // chunk p ^ ((row >> 1) & 7)), ST stages, one barrier per k-tile.  Narrow projections split K and leave f32 partial tiles for the fixed-order
 // reduction kernels.  Measured (us per launch with its reduction, 32 rows, gemm256_kernel / gemm_bf16_kernel -> here):
-//   width 4096:  gate_up (24576 x 4096) 50.3 -> 44.6 (4.5 TB/s), down (4096 x 12288) 34.4 -> 24.4, qkv (6144 x 4096) 17.5 -> 14.1, o 15.0 -> 11.6;
-//                the whole layer at 16 / 32 / 64 / 128 rows 114 / 117 / 125 / 160 -> 92 / 95 / 108 / 146
-//   width 2048 (I 6144): layer 58 -> 45;  width 1024 (I 3072): 40 -> 30;  lm_head (151936 x 4096) 385 -> 277 (4.5 TB/s), 391 -> 290 at 64 rows
-// Tiles of 64 columns, weight loads that bypass the caches, two workgroups per CU with fewer stages, a k start of its own per workgroup and
-// two k-tiles per barrier were all no faster.
+//   width 4096:  gate_up (24576 x 4096) 50.3 -> 38.0 (5.3 TB/s; 45.0 with all workgroups in step along K), down (4096 x 12288) 34.4 -> 24.4, qkv (6144 x
+//                4096) 17.5 -> 14.1, o 15.0 -> 11.6
+//   width 2048 (I 6144): layer 58 -> 45;  width 1024 (I 3072): 40 -> 30;  lm_head (151936 x 4096) 385 -> 226 (5.5 TB/s; 275 in step)
+// Tiles of 64 columns, weight loads that bypass the caches, two workgroups per CU with fewer stages and two k-tiles per barrier were all no faster.
 #include "dev_common.h"
 #include "kernels.h"
 
@@ -22,6 +21,10 @@ namespace cm {
 namespace {
 
 constexpr int RBK = 64;
+// k-tiles between the starts of neighbouring workgroups of an XCD.  In step, all workgroups ask for the same columns of all rows, and those reach a part
+// of the memory channels.  Rows of 8 KB read by 256 workgroups as here: 42 us for 201 MB (36.5 for the 8 matrices of 36 that happen to lie well), 36.0 with
+// four starts 2 KB apart, 37 .. 39 with as many as there are workgroups, 43 with two
+constexpr int K_TURN = 16;
 
 template <int BM, int RBN, int ST, int EPI, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_rows_kernel(GemmArgs a) {
@@ -48,8 +51,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void gemm_rows_kernel(Gem
         src[i] = isw ? a.W + (size_t)(n0 + row) * K + kc : (plane ? a.A_lo : a.A_hi) + (size_t)min(row, a.M - 1) * K + kc;
         dst[i] = lds0 + (uint32_t)((isw ? 2 * PLANE : plane * PLANE) + r0 * RBK) * 2u;
     }
+    // (slices of K start apart by themselves: 16.0 / 16.3 us with a turn on top; so do the 128-row tiles, which all have slices)
+    const int turn = EPI != GEPI_PARTIAL && BM < 128 ? ((int)blockIdx.x >> 3 & 3) * K_TURN % kpb : 0;
     auto request = [&](int t) __attribute__((always_inline)) {                          // past the end: the last tile again, into a stage nobody reads
-        const size_t at = (size_t)min(t, kpb - 1) * RBK;
+        const int k = min(t, kpb - 1) + turn;
+        const size_t at = (size_t)(k < kpb ? k : k - kpb) * RBK;
         const uint32_t stage = (uint32_t)((t % ST) * STAGE) * 2u;
 #pragma unroll
         for (int i = 0; i < NL; ++i) lds_load16(src[i] + at, dst[i] + stage);
