@@ -1950,89 +1950,6 @@ void launch_lay_memory_out(const float* o, const float* mrun, const float* gate,
 // ------------------------------------------------------------------------------------------------------------------
 // mixture of experts: router + counting sort
 // ------------------------------------------------------------------------------------------------------------------
-// One wave turns the E logits of token t in zs into choices and weights.  zs: [E] logits, then choice scores (shared_gate: one more
-// logit behind them); sc: [E] scores, [groups], [top].
-__device__ __forceinline__ void lay_router_choose(float* zs, int t, int lane, int32_t* __restrict__ sel, float* __restrict__ wsel, int E, int top,
-                                                  const RouterSpec& rs, const float* __restrict__ correction, int slots) {
-    float* sc = zs + E + (rs.shared_gate ? 1 : 0);
-    // wave 0: lane l owns outputs l, l + 64, ...; maxima, sums and the arg-max (lowest index among equals) are wave reductions
-    auto arg_best = [&](bool want_max, int lo, int hi, float& bv) {      // over the live (not -inf) entries of zs[lo, hi)
-        float v = 0.f; int at = 0x7fffffff;
-        for (int ex = lo + lane; ex < hi; ex += 64) {
-            const float z = zs[ex];
-            if (z == -INFINITY) continue;
-            if (at == 0x7fffffff || (want_max ? z > v : z < v)) { v = z; at = ex; }
-        }
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(v, off); const int oa = __shfl_xor(at, off);
-            if (oa != 0x7fffffff && (at == 0x7fffffff || (want_max ? ov > v : ov < v) || (ov == v && oa < at))) { v = ov; at = oa; }
-        }
-        bv = v;
-        return at;
-    };
-    // scores; the choice goes by score + correction (plain sigmoid scores: by the logits themselves, the same order -- unless groups are
-    // compared by sums of scores)
-    if (rs.softmax) {
-        float mx = -INFINITY;
-        for (int ex = lane; ex < E; ex += 64) mx = fmaxf(mx, zs[ex]);
-        mx = wave_max(mx);
-        float sum = 0.f;
-        for (int ex = lane; ex < E; ex += 64) { const float p = expf(zs[ex] - mx); sc[ex] = p; sum += p; }
-        sum = wave_sum(sum);
-        for (int ex = lane; ex < E; ex += 64) sc[ex] /= sum;
-    } else
-        for (int ex = lane; ex < E; ex += 64) sc[ex] = 1.f / (1.f + expf(-zs[ex]));
-    if (rs.softmax || correction || (rs.groups > 1 && rs.group_top > 1))
-        for (int ex = lane; ex < E; ex += 64) zs[ex] = sc[ex] + (correction ? correction[ex] : 0.f);
-    __builtin_amdgcn_wave_barrier();
-    if (rs.groups > 1) {                   // keep the best groups: every pass removes the worst remaining one
-        const int per = E / rs.groups;
-        float* gb = sc + E;                // [groups] a group's score: its largest choice score, or the sum of its two largest (-inf: removed)
-        for (int g = lane; g < rs.groups; g += 64) {
-            float best = -INFINITY, second = -INFINITY;
-            for (int j = 0; j < per; ++j) {
-                const float v = zs[g * per + j];
-                second = fmaxf(second, fminf(best, v));
-                best = fmaxf(best, v);
-            }
-            gb[g] = rs.group_top > 1 && per > 1 ? best + second : best;
-        }
-        for (int drop = 0; drop < rs.groups - rs.keep_groups; ++drop) {
-            // the worst live group, among equals the last one
-            float v = 0.f; int at = -1;
-            for (int g = lane; g < rs.groups; g += 64) {
-                const float b = gb[g];
-                if (b == -INFINITY) continue;
-                if (at < 0 || b <= v) { v = b; at = g; }
-            }
-            for (int off = 32; off > 0; off >>= 1) {
-                const float ov = __shfl_xor(v, off); const int oa = __shfl_xor(at, off);
-                if (oa >= 0 && (at < 0 || ov < v || (ov == v && oa > at))) { v = ov; at = oa; }
-            }
-            if (at < 0) break;
-            if (lane == 0) gb[at] = -INFINITY;
-            for (int j = lane; j < per; j += 64) zs[at * per + j] = -INFINITY;
-            __builtin_amdgcn_wave_barrier();      // LDS accesses of one wave complete in order; this keeps the compiler from moving them
-        }
-    }
-    float* wl = sc + E + rs.groups;        // [top] the chosen scores
-    float wsum = 0.f;
-    for (int k = 0; k < top; ++k) {
-        float bz;
-        int best = arg_best(true, 0, E, bz);
-        if (best == 0x7fffffff) best = 0;
-        const float w = sc[best];
-        wsum += w;
-        if (lane == 0) {
-            sel[(size_t)t * top + k] = best;
-            wl[k] = w;
-            zs[best] = -INFINITY;
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    for (int k = lane; k < top; k += 64) wsel[(size_t)t * slots + k] = (rs.normalise ? wl[k] / (wsum + 1e-20f) : wl[k]) * rs.scale;
-    for (int k = top + lane; k < slots; k += 64) wsel[(size_t)t * slots + k] = rs.shared_gate ? 1.f / (1.f + expf(-zs[E])) : 1.f;
-}
 // logits and choice in one launch, one block per token
 __global__ __launch_bounds__(256) void lay_router_kernel(const float* __restrict__ h, const uint16_t* __restrict__ wr, int32_t* __restrict__ sel,
                                                          float* __restrict__ wsel, int W, int E, int top, RouterSpec rs,

@@ -315,6 +315,21 @@ void launch_lay_qk_prep(float* proj, int ldp, int q_off, int k_off, int v_off, i
                         float eps, int dims, bool half, const float* freq, float mag, void* kpool, void* vpool, int kvt, const int32_t* bt,
                         const LaySegDev* segs, const int32_t* rowseg, int T, int page, hipStream_t s, int pool = 0, int pool_rows = 0,
                         void* pk_pool = nullptr, void* pv_pool = nullptr, const LQkPrepExtra* extra = nullptr);
+// steps of one row, tanh norms, bfloat16 format (kernels_layered_step.hip).  The row in front of a product: x + mult (sum of nsum rows y, times wsel where given),
+// written to xout, through tanh(alpha .) w + b.  xout is no buffer that the launch reads; y null: xout = x
+struct LStepNorm { const float *x, *y, *wsel, *w, *b; float* xout; int nsum; float mult, alpha; };
+struct LStepProj { const uint16_t* W; const float* bias; float* C; int N, act, act2, act_split; float act_param; };
+struct LStepMoe {
+    const uint16_t *router, *gate, *up, *down, *sh_gate, *sh_up, *sh_down;
+    float *hh, *hs, *wsel;             // inner rows of the choices [top][ff] and of the expert of every token [sh_ff]; weights [slots]
+    int32_t* sel;                      // choices [top]
+    int experts, top, slots, ff, sh_ff, act;
+    float limit, sh_limit;
+    RouterSpec rs;
+};
+bool lay_step_fits(int W, const LayerSpec& sp);
+void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream_t s);
+void launch_lay_step_moe(const LStepNorm& a, const LStepMoe& m, float* ys, int W, hipStream_t s);       // both products: ys [slots][W]
 // decode steps (at most LAY_ROW_KERNEL_ROWS rows): logits, choice and the rows sorted by expert in one launch (lay_router_decode_fits)
 bool lay_router_decode_fits(const float* h, const uint16_t* wr, int T, int W, int E, int top, const RouterSpec& rs);
 void launch_lay_router_decode(const float* h, const uint16_t* wr, int32_t* sel, float* wsel, int32_t* off, int32_t* srt, int T, int W, int E, int top,

@@ -73,6 +73,7 @@ struct Layered {
     float* U = nullptr;                // lightning attention, chunk-parallel form: [chunks of a pass][widest H d e] f32
     size_t u_stride = 0;
     float* Dch = nullptr;              // gated linear attention, chunk-parallel form: [chunks of a pass][widest H d] decay of a chunk
+    float* X2 = nullptr;               // [W] the residual between the two halves of a layer, steps of one row
     float *H2 = nullptr, *Y2 = nullptr;                  // parallel layers: second norm's rows, feed-forward output
     float *CQ = nullptr, *Q = nullptr, *Qa = nullptr;    // latent attention: query latent, queries, queries against the cached latent
     float* LD = nullptr;               // gated linear attention: logarithm of the decay per token and key channel
@@ -1473,6 +1474,7 @@ void Model::alloc_runtime_layered() {
     if (L.max_conv) L.XB = dalloc<float>(cap * (size_t)L.max_conv);
     if (L.max_E > 1 || L.max_top > 1 || std::any_of(L.spec.begin(), L.spec.end(), [](const LayerSpec& s) { return s.mlp == LMLP_MOE; })) {
         L.YS = dalloc<float>(cap * (size_t)L.max_slots * W);
+        if (L.tanh_norm) L.X2 = dalloc<float>((size_t)W);
         L.wsel = dalloc<float>(cap * (size_t)L.max_slots);
         L.sel = dalloc<int32_t>(cap * (size_t)L.max_top);
         L.srt = dalloc<int32_t>(cap * (size_t)L.max_top);
@@ -1938,12 +1940,21 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 }
             } else if (L.pre_norm) {
                 // ---- x += mult mixer(norm1 x), x += mult ff(norm2 x); norms in equal parts, or of single elements
-                add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc);
+                // one row: the norms inside the launches of the products behind them, the router inside the experts' (x -> X2 -> x)
+                const bool one_row = T == 1 && L.tanh_norm && !L.f32 && L.fused_prep && lay_step_fits(W, sp);
                 LGemmArgs g;
-                g.A = L.Hc; g.A16 = n16; g.lda = W; g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.K = W;
+                g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.K = W;
                 g.act_split = w.g_off; g.act = sp.mixer == LMIX_HGRN ? LACT_SILU : LACT_NONE;
                 g.act2 = sp.mixer == LMIX_ATTN && sp.gate != LGATE_NONE ? LACT_SIGMOID : LACT_NONE;
-                lay_gemm(*this, L, g, 1, s);
+                if (one_row) {
+                    launch_lay_step_in({L.X, padd.y, padd.wsel, w.norm1, w.norm1_off, L.X2, padd.nsum, L.mult, w.norm1_alpha},
+                                       {g.W, g.bias, g.C, g.N, g.act, g.act2, g.act_split, g.act_param}, W, s);
+                    padd.y = nullptr; padd.wsel = nullptr;
+                } else {
+                    add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc);
+                    g.A = L.Hc; g.A16 = n16; g.lda = W;
+                    lay_gemm(*this, L, g, 1, s);
+                }
                 const float* oa = L.O;
                 const uint16_t* oa16 = nullptr;
                 int on = 0;
@@ -2077,6 +2088,12 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     dn.A = L.HH; dn.lda = sp.ff; dn.W = w.down; dn.C = L.Y; dn.ldc = W; dn.M = T; dn.N = W; dn.K = sp.ff;
                     lay_gemm(*this, L, dn, 1, s);
                     padd.y = L.Y; padd.nsum = 1;
+                } else if (one_row) {
+                    const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
+                    const LStepMoe m{w.router, w.gate, w.up, w.down, w.sh_gate, w.sh_up, w.sh_down, L.HH, L.HS, L.wsel, L.sel, sp.experts, sp.top, slots, sp.ff,
+                                     sp.shared_ff, sp.expert_act, sp.limit, sp.shared_limit, sp.router};
+                    launch_lay_step_moe({L.X2, padd.y, nullptr, w.norm2, w.norm2_off, L.X, 1, L.mult, w.norm2_alpha}, m, L.YS, W, s);
+                    padd.y = L.YS; padd.nsum = slots; padd.wsel = L.wsel;
                 } else if (sp.mlp == LMLP_MOE) {
                     add_norm(w.norm2, w.norm2_off, w.norm2_alpha, L.Hc);
                     // scale_input: an expert's weight multiplies its INPUT, the rows of the grouped product are w h and the combine is a plain
