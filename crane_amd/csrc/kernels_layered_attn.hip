@@ -28,6 +28,13 @@ namespace cm {
 namespace {
 
 constexpr int KT = 64;
+// a decode step whose queries' parts fit side by side (lay_attn_few_kernel)
+bool lay_attn_packed(const LAttnArgs& a) { return a.single && a.H <= 4 * a.G; }
+// over the four columns of a row of sixteen lanes that are four apart; each of them gets the same sum
+__device__ __forceinline__ float parts_sum(float v) {
+    v += dpp_mov<0x128>(v);        // row_ror 8
+    return v + dpp_mov<0x124>(v);  // row_ror 4
+}
 constexpr float L2E = 1.4426950408889634f;
 
 __device__ __forceinline__ void lds_barrier() {        // LDS hand-off only: requests for later tiles stay in flight
@@ -80,9 +87,12 @@ __device__ __forceinline__ void query8(const float* src, int c, int d, bool ok, 
 // a lane's query (column lane % 16 of the transposed scores) and its running softmax.  PARTS: bfloat16 parts of a weight.  Two parts (prompt
 // passes): scores in units of log 2, exp2 and log of the hardware units.  Three (decode steps): lay_attn_kernel's functions -- expf, and log1pf,
 // which keeps the low bits of a small r2 * distance that 1 + x drops (r1 = 1e6, r2 = 1e-7: weights 5 % off with the hardware's log of 1 + x)
-template <int PARTS>
+// PACK: column lane % 16 holds part (lane % 16) / 4 (the fourth: nothing) of query min(lane % 4, ..); the scores come as sums over the parts, a lane keeps its
+// own part of the weights
+template <int PARTS, bool PACK = false>
 struct Query {
     static constexpr bool EXACT = PARTS == 3;
+    static constexpr int KEPT = PACK ? 1 : PARTS;
     static constexpr float UNIT = EXACT ? 1.f : L2E;
     // the scores' loops take what lies in front and move the rest up: rolled where the functions are long.  A decode launch has about one key tile per
     // wave and waits for its own code: with sixteen expf in a row it is 4 us longer than with sixteen v_exp_f32, with eight in a loop of two 0.9 (8 heads on
@@ -108,7 +118,7 @@ struct Query {
     // scores of tile t (products in s, keys 16 tt + 4 lg + r) -> weights in PARTS bfloat16 parts, the running pair moved on, o rescaled when a
     // new maximum appears in the wave.  p[..][h]: keys 16 (2 h) + 4 lg + 0 .. 3, then 16 (2 h + 1) + 4 lg + 0 .. 3
     template <bool POOL, int NNT>
-    __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int lg, f32x4 (&s)[4], bf16x8 (&p)[PARTS][2], f32x4 (&o)[NNT]) {
+    __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int lg, f32x4 (&s)[4], bf16x8 (&p)[KEPT][2], f32x4 (&o)[NNT], int part_of = 0) {
         const float scale = a.scale * UNIT;
         const int j0 = w.first(t);
         const bool blk = POOL && t < w.front;
@@ -159,24 +169,33 @@ struct Query {
         }
         float psum = 0.f;
 #pragma unroll
-        for (int k = 0; k < PARTS; ++k) p[k][1] = __builtin_bit_cast(bf16x8, (u32x4){0u, 0u, 0u, 0u});
+        for (int k = 0; k < KEPT; ++k) p[k][1] = __builtin_bit_cast(bf16x8, (u32x4){0u, 0u, 0u, 0u});
 #pragma unroll ROLL
         for (int h = 0; h < 2; ++h) {
-            u32x4 part[PARTS];
+            u32x4 part[KEPT];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 float p0 = ex(s[q >> 1][2 * (q & 1)] - ms);
                 float p1 = ex(s[q >> 1][2 * (q & 1) + 1] - ms);
                 psum += p0 + p1;
+                if (PACK) {
 #pragma unroll
-                for (int k = 0; k < PARTS; ++k) {
-                    const uint32_t pk = pack_bf16x2(p0, p1);
-                    part[k][q] = pk;
-                    p0 -= bf16_lo(pk); p1 -= bf16_hi(pk);
+                    for (int k = 0; k < PARTS - 1; ++k) {          // what the parts in front of this lane's leave
+                        const uint32_t pk = pack_bf16x2(p0, p1);
+                        p0 -= part_of > k ? bf16_lo(pk) : 0.f; p1 -= part_of > k ? bf16_hi(pk) : 0.f;
+                    }
+                    part[0][q] = part_of < PARTS ? pack_bf16x2(p0, p1) : 0u;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < KEPT; ++k) {
+                        const uint32_t pk = pack_bf16x2(p0, p1);
+                        part[k][q] = pk;
+                        p0 -= bf16_lo(pk); p1 -= bf16_hi(pk);
+                    }
                 }
             }
 #pragma unroll
-            for (int k = 0; k < PARTS; ++k) { p[k][0] = p[k][1]; p[k][1] = __builtin_bit_cast(bf16x8, part[k]); }
+            for (int k = 0; k < KEPT; ++k) { p[k][0] = p[k][1]; p[k][1] = __builtin_bit_cast(bf16x8, part[k]); }
             s[0] = s[2]; s[1] = s[3];
         }
         l += psum;
@@ -386,26 +405,32 @@ void go(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
 // step of four layers, lay_attn_kernel / here: 8 heads on 2 of width 1024, 1 / 32 / 128 sequences behind 24 tokens 281 / 256, 514 / 460, 854 / 705,
 // behind 1000 tokens 296 / 280, 830 / 525, 2126 / 853; 32 heads on 8 of width 4096, 1 / 32 / 128 sequences behind 24 tokens 515 / 487, 1187 / 1068,
 // 1699 / 1552, behind 1000 tokens 536 / 522, 2523 / 1154, 4780 / 1927
-constexpr int DW = 8;
-template <int DP, int EP, bool POOL>
-__global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
+// PACK: every sequence has one row and a key head at most four query heads: their parts are columns side by side of one product, as in
+// attn_decode_group_kernel, and blocks of four waves fit a CU twice: one sequence behind 1000 tokens, 8 heads on 2, 13.1 -> 10.7 us.
+template <int DP, int EP, bool POOL, bool PACK>
+__global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
+    constexpr int DW = PACK ? 4 : 8, QR = PACK ? 4 : 16;          // waves, query rows of the tile
     constexpr int QLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16, VC = EP / 8, VPL = KT * VC / 64;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
     __shared__ float pm[DW][16], pl_[DW][16];
-    uint16_t* const Qs = smem + DW * KT * VLD;         // [3 parts][16][QLD]
+    uint16_t* const Qs = smem + DW * KT * VLD;         // [3 parts][QR][QLD]
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     uint16_t* const Vw = smem + wave * KT * VLD;       // [64][VLD] of this wave
     const int g = blockIdx.x;
-    const int2 tile_id = a.tiles[blockIdx.y];
+    const int2 tile_id = PACK ? make_int2((int)blockIdx.y, 0) : a.tiles[blockIdx.y];
     const LaySegDev sg = a.segs[tile_id.x];
     const int nrep = a.H / a.G, d = a.d, e = a.e;
     const int q0 = tile_id.y, nq = min(16, sg.n * nrep - q0);
     Walk w;
     w.init<POOL>(a, sg, q0, nq, nrep);
     const int t_first = (int)blockIdx.z * DW + wave, t_step = DW * (int)gridDim.z;
-    Query<3> q;
-    q.init(a, sg, g, lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
+    const int part_of = PACK ? lr >> 2 : 0;
+    Query<3, PACK> q;
+    q.init(a, sg, g, PACK ? min(lr & 3, nq - 1) : lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
+    // requested in front of the first tile: answers come in order
+    float x[8];
+    if (wave < NKS) query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, wave * 32 + lg * 8, d, q.ok, qvec, x);
     int pgs_grp = 0;                                   // lane i: page of this wave's tile 64 grp + i
     auto load_pages = [&](int grp) __attribute__((always_inline)) {
         const int j = min(w.first(min(t_first + (grp * 64 + lane) * t_step, w.ntile - 1)), w.pmax);
@@ -454,9 +479,7 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
     for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
     fetch_k(0);
     fetch_v(0);
-    for (int ks = wave; ks < NKS; ks += DW) {
-        float x[8];
-        query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, ks * 32 + lg * 8, d, q.ok, qvec, x);
+    if (wave < NKS) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             u32x4 pk;
@@ -465,7 +488,7 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
                 pk[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
                 x[2 * i] -= bf16_lo(pk[i]); x[2 * i + 1] -= bf16_hi(pk[i]);
             }
-            *(u32x4*)&Qs[(k * 16 + lr) * QLD + ks * 32 + lg * 8] = pk;
+            if (lr < QR) *(u32x4*)&Qs[(k * QR + lr) * QLD + wave * 32 + lg * 8] = pk;
         }
     }
     lds_barrier();
@@ -476,17 +499,25 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-            for (int k = 2; k >= 0; --k) {             // the smallest part first
-                const bf16x8 qf = *(const bf16x8*)&Qs[(k * 16 + lr) * QLD + ks * 32 + lg * 8];
+            for (int k = PACK ? 0 : 2; k >= 0; --k) {  // the smallest part first
+                u32x4 qv = *(const u32x4*)&Qs[(PACK ? min(part_of, 2) * QR + (lr & 3) : k * 16 + lr) * QLD + ks * 32 + lg * 8];
+                if (PACK && part_of == 3) qv = (u32x4){0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int tt = 0; tt < 4; ++tt) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[tt][ks]), qf, s[tt], 0, 0, 0);
+                for (int tt = 0; tt < 4; ++tt)
+                    s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[tt][ks]), __builtin_bit_cast(bf16x8, qv), s[tt], 0, 0, 0);
             }
+        if (PACK) {
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[tt][r] = parts_sum(s[tt][r]);
+        }
         fetch_k(i + 1);
 #pragma unroll
         for (int k = 0; k < VPL; ++k) *(u32x4*)&Vw[(lane / VC + k * (64 / VC)) * VLD + (lane % VC) * 8] = vr[k];
         fetch_v(i + 1);
-        bf16x8 p[3][2];
-        q.template weights<POOL>(a, w, t, lg, s, p, o);
+        bf16x8 p[PACK ? 1 : 3][2];
+        q.template weights<POOL>(a, w, t, lg, s, p, o, part_of);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the wave's own tile is in LDS
         values<VLD>(Vw, lr, lg, p, o);
     }
@@ -496,9 +527,16 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
     if (lg == 0) { pm[wave][lr] = q.m; pl_[wave][lr] = l; }
     __syncthreads();                                   // every wave's value tile has been read: its place holds the sums
     float* po = (float*)smem;                          // [wave][NNT][64 lanes][4]
+    if (PACK) {
+#pragma unroll
+        for (int n = 0; n < NNT; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[n][r] = parts_sum(o[n][r]);
+    }
 #pragma unroll
     for (int n = 0; n < NNT; ++n) *(f32x4*)&po[((wave * NNT + n) * 64 + lane) * 4] = o[n];
     __syncthreads();
+    if (PACK && lr >= nq) return;
     float M = -INFINITY, L = 0.f, cw[DW];
 #pragma unroll
     for (int k = 0; k < DW; ++k) M = fmaxf(M, pm[k][lr]);
@@ -524,15 +562,21 @@ __global__ __launch_bounds__(DW * 64, 1) void lay_attn_few_kernel(LAttnArgs a, b
         } else if (q.ok) put4(a, q.row, q.head, c, v, L, ovec);
     }
 }
-template <int DP, int EP, bool POOL>
+template <int DP, int EP, bool POOL, bool PACK>
 void go_few(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
-    constexpr size_t lds = ((size_t)DW * KT * (EP + 16) + 3 * 16 * (DP + 8)) * sizeof(uint16_t);
+    constexpr int DW = PACK ? 4 : 8, QR = PACK ? 4 : 16;
+    constexpr size_t lds = ((size_t)DW * KT * (EP + 16) + 3 * QR * (DP + 8)) * sizeof(uint16_t);
     static_assert(lds >= (size_t)DW * (EP / 16) * 64 * 4 * sizeof(float), "the waves' sums");
+    static_assert(DP / 32 <= DW, "a wave per 32 elements of the queries");
     static DevOnce attr;
     attr.run([&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_few_kernel<DP, EP, POOL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_few_kernel<DP, EP, POOL, PACK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    hipLaunchKernelGGL((lay_attn_few_kernel<DP, EP, POOL>), dim3((unsigned)a.G, (unsigned)a.ntiles, (unsigned)nsplit), dim3(DW * 64), lds, s, a, qvec, ovec);
+    hipLaunchKernelGGL((lay_attn_few_kernel<DP, EP, POOL, PACK>), dim3((unsigned)a.G, (unsigned)a.ntiles, (unsigned)nsplit), dim3(DW * 64), lds, s, a, qvec, ovec);
+}
+template <int DP, int EP, bool POOL>
+void go_few(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
+    if (lay_attn_packed(a)) go_few<DP, EP, POOL, true>(a, nsplit, qvec, ovec, s); else go_few<DP, EP, POOL, false>(a, nsplit, qvec, ovec, s);
 }
 // nsplit 0: the prompt kernel
 template <int DP, int EP>
@@ -565,20 +609,21 @@ void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s) {
     if (a.ntiles > 0) launch(a, 0, s);
 }
 
-int lay_attn_few_split(long long visible, int blocks, int parts) {
+int lay_attn_few_split(long long visible, int blocks, int parts, bool packed) {
     // one key tile per wave, then more blocks and a merge: a further tile in the same wave costs about 4 us (its keys and values are two trips to
     // memory), the merge 6.  Eight tokens of four layers of width 4096, 32 heads on 8: context 3500 5.02 - 5.20 ms with one, 5.17 - 5.23 with two
     // tiles per wave; context 100 (no split) 4.96
+    const int DW = packed ? 4 : 8;
     const long long tiles = (visible + KT - 1) / KT + 1;
     if (tiles <= DW) return 1;
-    return (int)std::max(1ll, std::min({(tiles + DW - 1) / DW, 256ll / std::max(1, blocks), (long long)parts / std::max(1, blocks)}));
+    return (int)std::max(1ll, std::min({(tiles + DW - 1) / DW, (packed ? 512ll : 256ll) / std::max(1, blocks), (long long)parts / std::max(1, blocks)}));
 }
 
-void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s) {
+void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s, bool merge) {
     if (a.ntiles <= 0) return;
     const int nsplit = a.part_o && a.part_ml && a.nsplit > 1 ? a.nsplit : 1;
     launch(a, nsplit, s);
-    if (nsplit > 1) launch_lay_attn_merge(a, nsplit, s);
+    if (nsplit > 1 && merge) launch_lay_attn_merge(a, nsplit, s);
 }
 
 }  // namespace cm

@@ -5,9 +5,11 @@
 // few operations per element, so every block of the next product makes the whole row for itself (rows of 1024 .. 4096 elements out of the L2) while its
 // weights are on their way; so is a router of some tens of logits.  What leaves a launch besides its product is written by one block, into a buffer that
 // no other block of the launch reads: the residual goes from x to x2 in front of the mixer and back in front of the experts.
-// Every sum is made in the order of the launches that these replace (lay_add_tanh_norm_kernel, lgemv_kernel, lay_router_decode_kernel): the same bits.
-// Measured (us, width 1024, 14 experts of 768, 4 per token, and one of 512): norm + router + gate-and-up 18.9 in three launches, 11.5 here; norm and input
-// projection 7.8 in two, 4.1 here; the second product 5.3, 4.1 (its matrices follow from the choices, not from the sorted rows).
+// Every sum is made in the order of the launches that these replace (lay_add_tanh_norm_kernel, lgemv_kernel, lay_router_decode_kernel, lay_attn_merge_kernel): the
+// same bits.
+// Measured (us, width 1024, 14 experts of 768, 4 per token, and one of 512): norm + router + gate-and-up 18.9 in three launches, 9.1 here; norm and input
+// projection 7.8 in two, 4.1 here; the second product 5.3, 4.2 (its matrices follow from the choices, not from the sorted rows); output projection behind
+// five attention shares 9.0 with a merging launch, 5.5 here.
 #include <algorithm>
 
 #include "dev_common.h"
@@ -96,6 +98,67 @@ __global__ __launch_bounds__(256) void lay_step_in_kernel(LStepNorm a, LStepProj
         if (p.bias) v += p.bias[n];
         p.C[n] = lay_act(v, n < p.act_split ? p.act : p.act2, p.act_param);
     }
+}
+
+// C = (attention rows merged from their shares) W^T, two columns per wave: lay_attn_merge_kernel's sums in every block
+template <int NIT>
+__global__ __launch_bounds__(256) void lay_step_out_kernel(LAttnArgs a, int nsplit, const uint16_t* __restrict__ W, float* __restrict__ C, int N) {
+    constexpr int K = NIT * 512;
+    __shared__ __attribute__((aligned(16))) float h[K];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n0 = min((int)(blockIdx.x * 4 + wave) * 2, N - 1), n1 = min(n0 + 1, N - 1);
+    u32x4 w0[NIT], w1[NIT];
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+        w0[i] = ld_nt16(W + (size_t)n0 * K + lane * 8 + i * 512);
+        w1[i] = ld_nt16(W + (size_t)n1 * K + lane * 8 + i * 512);
+    }
+    const int nrep = a.H / a.G, e = a.e;
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+        const int k = (int)threadIdx.x * 2 + i * 512, head = k / e, c = k - head * e, g = head / nrep;      // (e is even)
+        const size_t p0 = (size_t)g * nsplit * 16 + (head - g * nrep);
+        const float2 gate = a.gate == LGATE_NONE ? make_float2(1.f, 1.f) : a.gate == LGATE_ELEM ? *(const float2*)(a.gbuf + k) : make_float2(a.gbuf[head], a.gbuf[head]);
+        // eight shares requested at once (a loop over their number would wait for each): past the last one it again, with weight 0
+        constexpr int AT = 8;
+        float2 ml[AT], po[AT];
+        auto request = [&](int z0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int z = 0; z < AT; ++z) {
+                const size_t pr = p0 + (size_t)min(z0 + z, nsplit - 1) * 16;
+                ml[z] = *(const float2*)(a.part_ml + pr * 2); po[z] = *(const float2*)(a.part_o + pr * e + c);
+            }
+        };
+        request(0);
+        float M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int z = 0; z < AT; ++z) M = fmaxf(M, ml[z].x);
+        for (int z = AT; z < nsplit; ++z) M = fmaxf(M, a.part_ml[(p0 + (size_t)z * 16) * 2]);
+        float2 acc = make_float2(0.f, 0.f);
+        for (int z0 = 0; z0 < nsplit; z0 += AT) {
+            if (z0 > 0) request(z0);
+#pragma unroll
+            for (int z = 0; z < AT; ++z) {
+                const float w = ml[z].x == -INFINITY || z0 + z >= nsplit ? 0.f : expf(ml[z].x - M);
+                L = z0 + z < nsplit ? fmaf(ml[z].y, w, L) : L;
+                acc.x = z0 + z < nsplit ? fmaf(po[z].x, w, acc.x) : acc.x;
+                acc.y = z0 + z < nsplit ? fmaf(po[z].y, w, acc.y) : acc.y;
+            }
+        }
+        *(float2*)(h + k) = make_float2(bf16_round(acc.x * gate.x / L * a.out_scale), bf16_round(acc.y * gate.y / L * a.out_scale));
+    }
+    __syncthreads();
+    float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+        float x[8];
+        step_row(h, lane * 8 + i * 512, x);
+        acc0 = step_dot(acc0, w0[i], x);
+        acc1 = step_dot(acc1, w1[i], x);
+    }
+    acc0 = wave_sum(acc0); acc1 = wave_sum(acc1);
+    const int n = (int)(blockIdx.x * 4 + wave) * 2 + lane;
+    if (lane < 2 && n < N) C[n] = lane ? acc1 : acc0;
 }
 
 // norm, router, choice, and act(h W_e^T) * (h W2_e^T) of the chosen experts and the one of every token.  blockIdx.y: the choice, the last the expert of every token
@@ -217,6 +280,16 @@ bool lay_step_fits(int W, const LayerSpec& sp) {
 #define CM_STEP_W(CALL) switch (W) { case 512: CALL(1); break; case 1024: CALL(2); break; case 2048: CALL(4); break; default: CALL(8); }
 void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream_t s) {
 #define CM_CALL(I) hipLaunchKernelGGL(lay_step_in_kernel<I>, dim3((unsigned)((p.N + 7) / 8)), dim3(256), 0, s, a, p)
+    CM_STEP_W(CM_CALL)
+#undef CM_CALL
+}
+bool lay_step_out_fits(const LAttnArgs& a) {
+    const int K = a.H * a.e;
+    return (K == 512 || K == 1024 || K == 2048 || K == 4096) && a.e % 2 == 0 && (a.gate != LGATE_ELEM || ((uintptr_t)a.gbuf & 7) == 0);
+}
+void launch_lay_step_out(const LAttnArgs& a, const uint16_t* Wm, float* C, int N, hipStream_t s) {
+    const int W = a.H * a.e;
+#define CM_CALL(I) hipLaunchKernelGGL(lay_step_out_kernel<I>, dim3((unsigned)((N + 7) / 8)), dim3(256), 0, s, a, a.nsplit, Wm, C, N)
     CM_STEP_W(CM_CALL)
 #undef CM_CALL
 }

@@ -295,6 +295,7 @@ struct LAttnArgs {
     // b pool + pool - 1 <= i - win; rows [n_pages][G][pool_rows][d] / [e] (lay_pool_append), in front of the window in the key walk
     long long pool = 0; const void* pk_pool = nullptr; const void* pv_pool = nullptr; int pool_rows = 0;
     float out_scale = 1.f;                           // factor on the output
+    bool single = false;                             // lay_attn_few: every segment is one row (tile i: segment i)
     int v_div = 1;                                   // v_div consecutive key heads share one value head: value pages [n_pages][G / v_div][page][e]
 };
 void launch_lay_k_append(const float* proj, int ldp, int k_off, void* kpool, int kvt, const int32_t* bt, const LaySegDev* segs,
@@ -329,6 +330,9 @@ struct LStepMoe {
 };
 bool lay_step_fits(int W, const LayerSpec& sp);
 void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream_t s);
+// the output projection behind an attention of one row whose nsplit > 1 shares have not been merged (a: its arguments, e and gbuf filled in)
+bool lay_step_out_fits(const LAttnArgs& a);
+void launch_lay_step_out(const LAttnArgs& a, const uint16_t* W, float* C, int N, hipStream_t s);
 void launch_lay_step_moe(const LStepNorm& a, const LStepMoe& m, float* ys, int W, hipStream_t s);       // both products: ys [slots][W]
 // decode steps (at most LAY_ROW_KERNEL_ROWS rows): logits, choice and the rows sorted by expert in one launch (lay_router_decode_fits)
 bool lay_router_decode_fits(const float* h, const uint16_t* wr, int T, int W, int E, int top, const RouterSpec& rs);
@@ -350,8 +354,8 @@ void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
 // the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can
 // see, blocks of an unsplit launch, scratch parts)
-void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s);
-int lay_attn_few_split(long long visible, int blocks, int parts);
+void launch_lay_attn_few(const LAttnArgs& a, hipStream_t s, bool merge = true);      // merge false: several shares stay in part_o, part_ml
+int lay_attn_few_split(long long visible, int blocks, int parts, bool packed);
 void launch_lay_attn_merge(const LAttnArgs& a, int nsplit, hipStream_t s);
 
 struct LLightArgs {

@@ -1735,6 +1735,8 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         uint16_t* const rounded = !L.f32 && L.shared_gemm && T > LAY_ROW_KERNEL_ROWS ? L.Abf : nullptr;
         const uint16_t *n16 = nullptr, *o16 = nullptr;                        // the last norm's and the last attention's rows, if they did
         // softmax attention of one layer over the pages: queries at qsrc[row ldq + q_off + head dk], output [T][H ev] into L.O
+        bool keep_shares = false;              // the next attention may leave its shares (in `left`) to the output projection
+        LAttnArgs left;
         auto run_attention = [&](const LayerSpec& sp, const LayeredLayerW& w, const float* qsrc, int ldq, int q_off, int g_off, int dk, int ev,
                                  float* out = nullptr, int ldo = 0, float out_scale = 1.f, int v_div = 1, const float* gbuf = nullptr, int ldg = 0,
                                  uint16_t* out16 = nullptr) {
@@ -1769,9 +1771,13 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) { o16 = a.out16 = out16; launch_lay_attn_tile(a, s); }
                 else launch_lay_attn_mfma(a, s);
             } else if (L.attn_mfma && kv_mode == KV_BF16 && lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
-                a.nsplit = lay_attn_few_split(seen, a.ntiles * sp.kv_heads, Layered::ATT_PARTS);
+                a.single = all_decode;
+                a.nsplit = lay_attn_few_split(seen, a.ntiles * sp.kv_heads, Layered::ATT_PARTS, all_decode && sp.heads <= 4 * sp.kv_heads);
                 o16 = a.out16 = out16;
-                launch_lay_attn_few(a, s);
+                const bool leave = keep_shares && a.nsplit > 1 && a.gbuf && lay_step_out_fits(a);
+                launch_lay_attn_few(a, s, !leave);
+                left = a;
+                if (!leave) left.nsplit = 1;
             } else
                 launch_lay_attn(a, kv_mode, s);
         };
@@ -1976,7 +1982,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                         t.segs = d_segs; t.rowseg = d_rowseg;
                         launch_lay_conv_tail(t, nseg, s);
                     }
+                    keep_shares = one_row;
+                    left.nsplit = 1;
                     run_attention(sp, w, L.XB, H * d, 0, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows, rounded);
+                    keep_shares = false;
                     on = H * e; oa16 = o16;
                 } else if (sp.mixer == LMIX_ATTN) {
                     // two maps per head as heads of their own (2 H query heads over 2 G key heads, pairs of key heads share a value head)
@@ -2076,7 +2085,9 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 }
                 LGemmArgs go;
                 go.A = oa; go.A16 = oa16; go.lda = on; go.W = w.o_w; go.C = L.Y; go.ldc = W; go.M = T; go.N = W; go.K = on;
-                lay_gemm(*this, L, go, 1, s);
+                if (one_row && left.nsplit > 1) launch_lay_step_out(left, w.o_w, L.Y, W, s);
+                else lay_gemm(*this, L, go, 1, s);
+                left.nsplit = 1;
                 padd.y = L.Y; padd.nsum = 1;
                 if (sp.mlp == LMLP_DENSE) {
                     add_norm(w.norm2, w.norm2_off, w.norm2_alpha, L.Hc);

@@ -1,0 +1,37 @@
+"""GPU: steps of one row (kernels_layered_step.hip: norms, router and the merging of attention shares inside the products behind them) against the launches
+they stand for.  Every sum is made in the same order, so the logits are the same bits."""
+import numpy as np
+import pytest
+
+from tests import gizezen_util as GZ
+
+pytestmark = pytest.mark.gpu
+
+
+# every width; router logits of less and more than one batch of a wave's requests, up to a wave's lanes; inner sizes below and above one piece of 512 and no
+# multiple of it, the expert of every token narrower, wider and absent; attention rows of 512 and 1024 from no, few and more shares than one batch, and of a
+# width that the merging launch keeps
+@pytest.mark.parametrize("width,heads,kv_heads,dim,window,experts,top,ff,shared", [
+    (512, 8, 2, 64, 4096, 5, 2, 136, 72), (1024, 8, 2, 128, 1024, 14, 4, 776, 512), (2048, 8, 8, 64, 700, 64, 6, 64, 0), (4096, 16, 4, 64, 300, 63, 1, 72, 1032),
+    (512, 4, 2, 48, 900, 20, 3, 520, 520)])
+@pytest.mark.parametrize("context", [3, 300, 2900])
+def test_against_single_launches(tmp_path, width, heads, kv_heads, dim, window, experts, top, ff, shared, context):
+    from crane_amd.backend import Model
+    mixer = dict(heads=heads, kv_heads=kv_heads, dim=dim, vdim=dim, conv=4, size=window, rot_dims=dim)
+    cfg = GZ.config([GZ.layer(GZ.attn(**mixer), GZ.moe(experts=experts, top=top, ff=ff, shared=shared)),
+                     GZ.layer(GZ.attn(**mixer, kv_from=0), None),
+                     GZ.layer(GZ.attn(**mixer), GZ.moe(experts=experts, top=top, ff=ff, shared=shared))], vocab=96, width=width)
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, GZ.random_weights(cfg, 3)), compute_dtype="bfloat16", max_seqs=4, max_seq_len=3072)
+    toks = GZ.tokens(context + 3, cfg["vocab"], 4)
+    out = []
+    try:
+        s = m.seq_alloc()
+        m.step_batch([(s, toks[:context], [])], want_logits=False)
+        for on in (1, 0):
+            m.debug_set("lay_fused_prep", on)
+            f = m.seq_fork(s)
+            out.append(np.stack([m.step_batch([(f, toks[context + i:context + i + 1], None)])[0] for i in range(3)]))
+            m.seq_free(f)
+    finally:
+        m.close()
+    assert np.isfinite(out[0]).all() and (out[0] == out[1]).all()
