@@ -33,6 +33,11 @@ namespace cm {
 namespace {
 
 constexpr int BK = 64;
+// experts: k-tiles between the starts of neighbouring column tiles (2 KB).  Few rows per expert read matrices out of memory, and blocks in step along K ask
+// for the same columns of all their rows, a part of the memory channels: 40 tokens, 16 experts of 2048 x 4096: gate-and-up 126 -> 102 us (5.3 TB/s), down 70 ->
+// 51; 700 tokens (175 rows each) 165 / 107 -> 165 / 98.  Not where a matrix is read by many row tiles, whose rows then come from several places: 2048 tokens, four
+// layers, 4.85 -> 4.95 ms; one matrix alone 77 -> 91 us
+constexpr int K_TURN = 16;
 
 // a block's tile: sorted rows [p0, p0 + rows) of group g, column tile nt, of the launch's first product or (side) its second; false: a block behind
 // the last tile.  Every XCD takes a contiguous share of either product's tiles, numbered by group, then column tile, then row tile
@@ -151,8 +156,10 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
         dst[i] = lds0 + (uint32_t)((isA ? p * 8 : BM + (p - APC) * 8) * BK) * 2u;
     }
     const int nk = a.K / BK;
+    const int turn = a.grp_off && a.total < 256 * a.groups ? (nt & 3) * K_TURN % nk : 0;
     auto request = [&](int t) __attribute__((always_inline)) {            // past the end: the last tile again, into a stage nobody reads
-        const int tc = min(t, nk - 1);
+        int tc = min(t, nk - 1) + turn;
+        tc = tc < nk ? tc : tc - nk;
         const uint32_t at = (uint32_t)((t % ST) * STAGE) * 2u;
 #pragma unroll
         for (int i = 0; i < NL; ++i) lds_load16(src[i] + (size_t)tc * BK, dst[i] + at);
@@ -222,7 +229,8 @@ void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s, const LTileArgs* be
     // 600 rows (160) 64 / 46
     const int total = a.grp_off ? a.total : a.M, groups = a.grp_off ? a.groups : 1;
     const int blocks = mtiles<128>(a) * ((a.N + (a.W2 ? 63 : 127)) / (a.W2 ? 64 : 128));
-    const bool wide = blocks >= LAY_TILE_WIDE_BLOCKS && total >= 64 * groups;
+    // (the second product of 16 experts of 2048 x 4096: 100 tokens, 25 rows each, 54 / 66 -- twice the columns per block count there)
+    const bool wide = blocks >= LAY_TILE_WIDE_BLOCKS && (total >= 64 * groups || (a.grp_off && !a.W2));
     if (a.W2) { if (wide) go<128, 128, 2, true>(a, b, s); else go<64, 64, 3, true>(a, b, s); }
     else { if (wide) go<128, 128, 2, false>(a, b, s); else go<64, 64, 3, false>(a, b, s); }
 }
