@@ -207,6 +207,11 @@ struct AttnPreArgs {
     const PrefillSegDev* segs = nullptr;
     const int2* tiles = nullptr;
     int ntiles = 0;
+    // few queries behind many keys (one sequence): scratch that launch_attn_prefill may share the keys of a query tile among blocks with: nsplit shares of
+    // [S][Hq][D] sums and [S][Hq][2] maxima and denominators
+    float* ws = nullptr;
+    size_t ws_floats = 0;
+    int nsplit = 1;              // (set by launch_attn_prefill)
 };
 
 void launch_embed_rows(const uint16_t* emb, const uint32_t* ids, float* x, int S, int H, int V, hipStream_t s);

@@ -681,7 +681,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
 //     K rows and V rows at compile-time offsets from one base -- no per-row division, clamp and 64-bit address chain;
 //   * only the tiles that touch the diagonal (or the end of the context) are masked and clamped: two loop bodies;
 //   * the softmax runs in the exp2 domain (one FMA + v_exp_f32 per score), P is split with packed conversions;
-//   * K AND V go through LDS once per workgroup, double-buffered (comment at kv_fetch): one workgroup barrier per tile.
+//   * K AND V go through LDS once per workgroup, double-buffered (comment at kv_fetch): one workgroup barrier per tile;
+//   * the products of a tile are all 32 keys deep (126 -> 109 us for 2048 tokens of 32 heads, 78 -> 66 for 452 behind them, when the second product
+//     took 16 at a time).
+// A launch of few query tiles behind many keys leaves the chip idle and walks the keys one after the other: there several blocks share a query tile's keys and
+// attn_prefill_merge_kernel adds the shares (69 queries behind 4096 keys, 8 heads of 256: 232 us for 16 blocks -> 30 for 256 and 9; 452 behind 2048, 32
+// heads of 128: 66 -> 55 and 7).
 // ---------------------------------------------------------------------------------------------
 // workgroup barrier for LDS hand-offs only: waits for this wave's LDS operations, not for its outstanding global loads
 // (__syncthreads() drains vmcnt as well and would retire the two-tiles-ahead requests at every tile)
@@ -760,6 +765,8 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
     const int kv_end = a.start_pos + last_q + 1;
     const int ntile = (kv_end + KT - 1) / KT;
     const int nfull = (a.start_pos + qb + 1) / KT;          // tiles every query of the block sees completely (and that end before kv_end)
+    const int tps = a.nsplit > 1 ? ((ntile + a.nsplit - 1) / a.nsplit + 1) / 2 * 2 : ntile;        // tiles of a share (even: the buffers alternate)
+    const int tbeg = (int)blockIdx.z * tps, tend = min(ntile, tbeg + tps);
     const uint16_t* kpool = (const uint16_t*)a.kpool;
     const uint16_t* vpool = (const uint16_t*)a.vpool;
     // element offset of the first row of key tile t inside the pool (one page per tile).  The page ids of 64 consecutive tiles sit
@@ -834,9 +841,10 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
             }
         mt = fmaxf(mt, __shfl_xor(mt, 16));
         mt = fmaxf(mt, __shfl_xor(mt, 32));
-        const float m_new = fmaxf(m_run, mt);               // finite: token 0 is visible to every query
-        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * L2E);
-        const float nm = -m_new * L2E;
+        const float m_new = fmaxf(m_run, mt);               // finite: token 0 is visible to every query (the first share; in others nothing may be so far)
+        const float m_use = MASKED && m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * L2E);
+        const float nm = -m_use * L2E;
         float psum = 0.f;
         bf16x4 ph[NTT], pl[NTT];
 #pragma unroll
@@ -850,34 +858,51 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
         m_run = m_new;
 #pragma unroll
         for (int nt = 0; nt < NNT; ++nt) { o[nt][0] *= alpha; o[nt][1] *= alpha; o[nt][2] *= alpha; o[nt][3] *= alpha; }
-        // ---- O^T += V^T . P^T : A = V^T fragment (tr-read from this tile's LDS buffer), B = P^T fragment ----
+        // ---- O^T += V^T . P^T : A = V^T fragment (tr-read from this tile's LDS buffer), B = P^T fragment.  The 32 keys of a product are two score tiles side
+        // by side (the k index of a product is any order its operands agree on): a 16-deep product takes the matrix unit as long ----
         const uint16_t* Vb = Vs[t & 1];
 #pragma unroll
-        for (int tt = 0; tt < NTT; ++tt) {
+        for (int tt = 0; tt < NTT; tt += 2) {
+            const bf16x8 p8h = __builtin_shufflevector(ph[tt], ph[tt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+            const bf16x8 p8l = __builtin_shufflevector(pl[tt], pl[tt + 1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
             for (int nt = 0; nt < NNT; ++nt) {
-                const uint16_t* vp = &Vb[(tt * 16 + g * 4 + (sub >> 2)) * VLD + nt * 16 + (sub & 3) * 4];
-                const bf16x4 vh = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)vp);
-                o[nt] = mma_k16<KVT>(vh, ph[tt], o[nt]);
-                o[nt] = mma_k16<KVT>(vh, pl[tt], o[nt]);
+                bf16x4 v2[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const uint16_t* vp = &Vb[((tt + k) * 16 + g * 4 + (sub >> 2)) * VLD + nt * 16 + (sub & 3) * 4];
+                    v2[k] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)vp);
+                }
+                const bf16x8 vh = __builtin_shufflevector(v2[0], v2[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                o[nt] = mma_k32<KVT>(vh, p8h, o[nt]);
+                o[nt] = mma_k32<KVT>(vh, p8l, o[nt]);
             }
         }
         kv_park((t + 1) & 1, rg_next);                      // the other buffers: last read one iteration ago, behind that iteration's barrier
         lds_wg_barrier();
     };
     KvRegs rA, rB;
-    kv_fetch(0, rA);
-    kv_fetch(1, rB);
+    kv_fetch(tbeg, rA);
+    kv_fetch(tbeg + 1, rB);
     kv_park(0, rA);
     __syncthreads();
     // (a tile is "full" when every query of the block sees all of it; the diagonal / ragged tiles are masked)
-    for (int t = 0; t < ntile; t += 2) {
+    for (int t = tbeg; t < tend; t += 2) {
         if (t < nfull) tile(t, std::false_type{}, rA, rB); else tile(t, std::true_type{}, rA, rB);
-        if (t + 1 < ntile) { if (t + 1 < nfull) tile(t + 1, std::false_type{}, rB, rA); else tile(t + 1, std::true_type{}, rB, rA); }
+        if (t + 1 < tend) { if (t + 1 < nfull) tile(t + 1, std::false_type{}, rB, rA); else tile(t + 1, std::true_type{}, rB, rA); }
     }
     // ---- finalize: l over the 4 lane groups; O^T rows = dims nt*16 + g*4 + r, col = query `sub` ----
     l_run += __shfl_xor(l_run, 16);
     l_run += __shfl_xor(l_run, 32);
+    if (a.nsplit > 1) {                                     // attn_prefill_merge_kernel takes it from here
+        if (qrow >= a.S) return;
+        const size_t at = ((size_t)blockIdx.z * a.S + qrow) * a.Hq + h;
+#pragma unroll
+        for (int nt = 0; nt < NNT; ++nt) *(f32x4*)(a.ws + at * D + nt * 16 + g * 4) = o[nt];
+        float* ml = a.ws + (size_t)a.nsplit * a.S * a.Hq * D + at * 2;
+        if (g == 0) { ml[0] = m_run; ml[1] = l_run; }
+        return;
+    }
     const float inv = 1.0f / l_run;
     if (qrow < a.S) {
 #pragma unroll
@@ -894,6 +919,38 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
             split_store4(a.out_hi, a.out_lo, ((size_t)qrow * a.Hq + h) * D + nt * 16 + g * 4, v);
         }
     }
+}
+
+// the shares of attn_prefill_fast_kernel's keys merged, four columns per thread
+template <int D>
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnPreArgs a) {
+    constexpr float L2E = 1.4426950408889634f;
+    const size_t n = (size_t)a.S * a.Hq, i = (size_t)blockIdx.x * (1024 / D) + threadIdx.x / (D / 4);      // (row, head)
+    if (i >= n) return;
+    const int c = (int)(threadIdx.x % (D / 4)) * 4, row = (int)(i / a.Hq), h = (int)(i % a.Hq);
+    const float* ml = a.ws + (size_t)a.nsplit * n * D;
+    float M = -INFINITY, L = 0.f;
+#pragma unroll 4
+    for (int z = 0; z < a.nsplit; ++z) M = fmaxf(M, ml[((size_t)z * n + i) * 2]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int z = 0; z < a.nsplit; ++z) {
+        const float2 p = *(const float2*)(ml + ((size_t)z * n + i) * 2);
+        const f32x4 v = *(const f32x4*)(a.ws + ((size_t)z * n + i) * D + c);
+        const float w = __builtin_amdgcn_exp2f((p.x - M) * L2E);          // (the first share sees token 0: M is finite; a share that saw nothing: 0)
+        L = fmaf(p.y, w, L);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = fmaf(v[r], w, o[r]);
+    }
+    const float inv = 1.0f / L;
+    float v[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+    if (a.gate != nullptr) {
+        const f32x4 gv = *(const f32x4*)(a.gate + (size_t)row * a.gate_stride + h * D + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + expf(-gv[r]));
+    }
+    if (a.out_f32 != nullptr) *(f32x4*)(a.out_f32 + i * D + c) = (f32x4){v[0], v[1], v[2], v[3]};
+    else split_store4(a.out_hi, a.out_lo, i * D + c, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1329,6 +1386,23 @@ static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
     return true;
 }
 // kvt: KV_BF16 | KV_F16 | KV_F32 (the element type the kernel READS: f32 for the int8 / int4 shadow)
+// shares of the keys for a launch of the fast path: `fill` blocks keep the chip busy (two on a CU at head_dim 128, one at 256); a share of fewer than eight
+// key tiles is not worth the merging launch
+static int prefill_split(const AttnPreArgs& a, int D, int kt, int fill) {
+    if (a.tiles != nullptr || a.ws == nullptr) return 1;
+    const int blocks = a.Hq * ((a.S + 63) / 64), tiles = (a.start_pos + a.S + kt - 1) / kt;
+    int n = std::min(std::min(fill / std::max(1, blocks), tiles / 8), 16);
+    while (n > 1 && (size_t)n * a.S * a.Hq * (D + 2) > a.ws_floats) --n;
+    return std::max(1, n);
+}
+template <int D, int KT>
+static void launch_prefill_fast(AttnPreArgs a, int kvt, int fill, hipStream_t s) {
+    a.nsplit = prefill_split(a, D, KT, fill);
+    const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64, a.nsplit);
+    if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_F16>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_BF16>), grid, dim3(256), 0, s, a);
+    if (a.nsplit > 1) hipLaunchKernelGGL(attn_prefill_merge_kernel<D>, dim3((unsigned)(((size_t)a.S * a.Hq + 1024 / D - 1) / (1024 / D))), dim3(256), 0, s, a);
+}
 void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
     const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64);
     if (D == 128) {
@@ -1336,8 +1410,7 @@ void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
         if (fast_env != 0 && a.gate == nullptr && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 &&
             a.q_lo != nullptr) {
-            if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<128, 64, KV_F16>), grid, dim3(256), 0, s, a);
-            else hipLaunchKernelGGL((attn_prefill_fast_kernel<128, 64, KV_BF16>), grid, dim3(256), 0, s, a);
+            launch_prefill_fast<128, 64>(a, kvt, 512, s);
             return;
         }
         if (kvt == KV_F32) hipLaunchKernelGGL((attn_prefill_kernel<128, KV_F32>), grid, dim3(256), 0, s, a);
@@ -1347,8 +1420,7 @@ void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
         // the hybrid family's gated head_dim-256 attention: the same fast path on 32-token key tiles
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
         if (fast_env != 0 && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 && a.q_lo != nullptr) {
-            if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<256, 32, KV_F16>), grid, dim3(256), 0, s, a);
-            else hipLaunchKernelGGL((attn_prefill_fast_kernel<256, 32, KV_BF16>), grid, dim3(256), 0, s, a);
+            launch_prefill_fast<256, 32>(a, kvt, 256, s);
             return;
         }
         if (kvt == KV_F32) hipLaunchKernelGGL((attn_prefill_kernel<256, KV_F32>), grid, dim3(256), 0, s, a);

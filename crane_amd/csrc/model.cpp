@@ -1444,6 +1444,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
         at.page = page; at.start_pos = sp;
         at.gate = cfg.hybrid ? pQKV + (size_t)sg.row0 * qkv_rows + (size_t)Hq_l * D : nullptr; at.gate_stride = qkv_rows;
         if (q8p) at.out_f32 = pATf + (size_t)sg.row0 * Hq_l * D;
+        at.ws = pWS; at.ws_floats = pWS ? gemm_ws_floats : 0;
         launch_attn_prefill(at, D, (kv_f32 || kvq) ? KV_F32 : kv_mode, s);
         }
         if (q8p) { q8_tail(w, w.q_o, pATf, Hq_l * D, li); continue; }
