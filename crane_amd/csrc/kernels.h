@@ -70,8 +70,8 @@ struct AttnDecArgs {
     uint16_t* out1_hi = nullptr; //   ... or, when set by this kernel or, with several splits, by the combine kernel, as bf16 hi + lo planes [seq][out1_cols]: the A
     uint16_t* out1_lo = nullptr; //   operand of the o_proj GEMM of a large decode group (split_rows2d's arithmetic), instead of the f32 rows
     int out1_cols = 0;
-    int qkv_ns = 1;              // qkv rows as qkv_ns f32 slices qkv_slice floats apart (the K-split partials of the int8 qkv GEMM, added in order by the
-    size_t qkv_slice = 0;        //   matrix-core kernel's prologue: no reduction launch); 1 = plain rows
+    int qkv_ns = 1;              // qkv rows as qkv_ns f32 slices qkv_slice floats apart (the K-split partials of the qkv GEMM, added in order by the prologue of
+    size_t qkv_slice = 0;        //   attn_decode_mfma_kernel (up to 4) or attn_decode_group_kernel (up to 8): no reduction launch); 1 = plain rows
     signed char* out1_q = nullptr;  // ... and ALSO (matrix-core kernel with a single split; combine kernel) as Q8_0 blocks of the rows: codes [seq][out1_cols] + block scales
     float* out1_qd = nullptr;       //   [out1_cols / 32][QGEMM_MAXM] -- quant_rows_q8_kernel's arithmetic: the int8 o_proj GEMM of a quantised group reads them
     int q_off, k_off, v_off;     // element offsets of q / k / v inside qkv
@@ -152,6 +152,9 @@ struct GemmArgs {
     uint16_t* norm_hi = nullptr;
     uint16_t* norm_lo = nullptr;
     float norm_eps = 0.f;
+    // GEPI_STORE of 9 .. 128 rows with a consumer that adds the slices of K itself (attn_decode_group_kernel): no reduction is launched where K is split, *defer_ks
+    // slices of M x N stay in ws; 1: C holds the rows as usual
+    int* defer_ks = nullptr;
 };
 
 // 9 .. 128 rows with hi + lo activations (kernels_gemm_rows.hip): whether these sizes are taken, with the tile's columns *bn and the K slices *ks,
@@ -444,8 +447,8 @@ void launch_gemm_q8_rows(const QGemmArgs& a, int num_cu, hipStream_t s);      //
 // (by the reduction launch), 2 = into next->xq2 / xd2 (by the unsplit gate|up GEMM itself, which cannot overwrite the codes it reads)
 struct QNext { const float* nw; float eps; signed char* xq; float* xd; signed char* xq2; float* xd2; };      // (xq2 / xd2: a second pair, or null)
 // EPI_STORE with a consumer that adds the K-split slices itself (the decode attention's prologue): when `defer` is given and the launch
-// splits K into 2 .. 4 slices, no reduction is launched -- ks slices of `slice` floats at ws, rows N floats apart; ks = 1: y holds the rows as usual
-struct QDefer { int ks; size_t slice; const float* ws; };
+// splits K into 2 .. `most` slices (<= 8), no reduction is launched -- ks slices of `slice` floats at ws, rows N floats apart; ks = 1: y holds the rows as usual
+struct QDefer { int ks; size_t slice; const float* ws; int most = 4; };
 // what launch_gemm_q8 will do for a shape (host logic only): ok = false -> the caller's GEMV fallback
 struct QGemmPlan { bool ok, direct; int geo, mh, mt, qg, groups, ks, grid; size_t lds; int mpan; };
 QGemmPlan plan_gemm_q8(int M, int N, int K, int epi, bool have_ws, size_t ws_floats, int num_cu, int fmt = QFMT_Q8_0);

@@ -116,15 +116,16 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
         const float* nw = item < NREP ? a.qnw : item == NREP ? a.knw : nullptr;
         x0[k] = src[lane]; x1[k] = src[lane + 64];
         n0[k] = nw ? nw[lane] : 1.f; n1[k] = nw ? nw[lane + 64] : 1.f;
-        if (a.qkv_ns > 1) {                                       // slices of a product whose depth is split (2 .. 4), added in their order; all loads first
-            float p0[3], p1[3];
+        if (a.qkv_ns > 1) {                                       // slices of a product whose depth is split (2 .. 8), added in their order; all loads first
+            float p0[7], p1[7];
 #pragma unroll
-            for (int sl = 1; sl < 4; ++sl) {
+            for (int sl = 1; sl < 8; ++sl) {
                 const float* ps = src + (size_t)(sl < a.qkv_ns ? sl : 0) * a.qkv_slice;
                 p0[sl - 1] = ps[lane]; p1[sl - 1] = ps[lane + 64];
             }
 #pragma unroll
-            for (int sl = 1; sl < 4; ++sl) { x0[k] += sl < a.qkv_ns ? p0[sl - 1] : 0.f; x1[k] += sl < a.qkv_ns ? p1[sl - 1] : 0.f; }
+            for (int sl = 1; sl < 8; ++sl)
+                if (sl < a.qkv_ns) { x0[k] += p0[sl - 1]; x1[k] += p1[sl - 1]; }
         }
     }
     fetch_k(0);

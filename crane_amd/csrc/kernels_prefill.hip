@@ -1321,7 +1321,8 @@ static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     if (!gemm_rows_plan(a.M, a.N, a.K, a.ws ? a.ws_floats : 0, &bn, &ks)) return false;
     a.ksplit = ks;
     if (!launch_gemm_rows(a, epi, bn, s)) return false;
-    if (ks > 1) launch_splitk(a, epi, s);
+    if (ks > 1 && a.defer_ks != nullptr && epi == GEPI_STORE && a.bias == nullptr) *a.defer_ks = ks;
+    else if (ks > 1) launch_splitk(a, epi, s);
     return true;
 }
 static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s);

@@ -1847,9 +1847,9 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
         // y[nb, N] (+)= A[nb, K] . W^T through launch_gemm; A = the bf16 hi + lo rows produced by rows_in
         // next_norm (GEPI_RESADD into xb only): RMSNorm(xb) * next_norm -> pXN_hi / pXN_lo, the A operand of the NEXT projection,
         // written by the GEMM's split-K reduction launch (GemmArgs::norm_w) instead of a rmsnorm_rows launch of its own
-        auto gm = [&](int epi, const uint16_t* A_hi, const uint16_t* A_lo, const uint16_t* W, float* C, int ldc, int N, int K, const float* next_norm = nullptr) {
+        auto gm = [&](int epi, const uint16_t* A_hi, const uint16_t* A_lo, const uint16_t* W, float* C, int ldc, int N, int K, const float* next_norm = nullptr, int* defer_ks = nullptr) {
             GemmArgs g{};
-            g.ws = pWS; g.ws_floats = gemm_ws_floats; g.wide256 = gemm256;
+            g.ws = pWS; g.ws_floats = gemm_ws_floats; g.wide256 = gemm256; g.defer_ks = defer_ks;
             g.A_hi = A_hi; g.A_lo = A_lo; g.W = W; g.C = C; g.ldc = ldc; g.M = nb; g.N = N; g.K = K;
             g.H_hi = pHH_hi; g.H_lo = pHH_lo;
             if (next_norm) { g.norm_w = next_norm; g.norm_hi = pXN_hi; g.norm_lo = pXN_lo; g.norm_eps = cfg.eps; }
@@ -2044,14 +2044,16 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                                     !(heads_b && !quantized && !rccl);
                 const bool codes_ok = attn_outq && qgemm_ok && nb >= q_gemm_min && !cfg.hybrid && !(heads_b && !quantized && !rccl) &&
                                       (grp || mf || !attn_decode_single_split(ns_b, D));
-                QDefer qdef{1, 0, nullptr};
+                QDefer qdef{1, 0, nullptr, grp ? 8 : 4};
                 if (quantized) {
                     const bool defer_ok = attn_q && w.n_qkv == 1 && ldq == w.q_qkv[0].N && w.qkv_row0[0] == 0;
                     for (int i = 0; i < w.n_qkv; ++i) qb(PRO_RMSNORM, EPI_STORE, w.q_qkv[i], xb, H, w.ln1, qkvb + w.qkv_row0[i], ldq, nullptr, false, defer_ok ? &qdef : nullptr);
                 }
                 else if (gemm_b) {
                     if (!xn_ready) launch_rmsnorm_rows(xb, w.ln1, pXN_hi, pXN_lo, nb, H, cfg.eps, s);
-                    gm(GEPI_STORE, pXN_hi, pXN_lo, w.qkv, qkvb, ldq, qkv_rows, H);
+                    // (the group attention adds the slices of a split product itself)
+                    gm(GEPI_STORE, pXN_hi, pXN_lo, w.qkv, qkvb, ldq, qkv_rows, H, nullptr, grp && !cfg.hybrid ? &qdef.ks : nullptr);
+                    if (qdef.ks > 1) { qdef.ws = pWS; qdef.slice = (size_t)nb * qkv_rows; }
                 } else gb(PRO_RMSNORM, EPI_STORE, w.qkv, xb, H, w.ln1, qkvb, ldq, qkv_rows, H);
                 AttnDecArgs a{};
                 a.qkv = qkvb; a.qnw = w.qn; a.knw = w.kn; a.cos = cos; a.sin = sin; a.st = stb; a.block_table = d_btb;
@@ -2079,7 +2081,7 @@ void Model::decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, floa
                 // 5.7 + 4.7 us at 20 sequences, 4.7 together)
                 const bool codes = codes_ok && gemm_q8_ok(w.q_o, nb) && w.q_o.fmt == QFMT_Q8_0 && (Hq_l * D) % 64 == 0;
                 if (codes) { a.out1_q = qx_codes; a.out1_qd = qx_scales; a.out1_cols = Hq_l * D; }
-                if (qdef.ks > 1) { a.qkv = qdef.ws; a.qkv_stride = w.q_qkv[0].N; a.qkv_ns = qdef.ks; a.qkv_slice = qdef.slice; }      // (the slices of the qkv GEMM, rows N floats apart)
+                if (qdef.ks > 1) { a.qkv = qdef.ws; a.qkv_stride = quantized ? w.q_qkv[0].N : qkv_rows; a.qkv_ns = qdef.ks; a.qkv_slice = qdef.slice; }      // (the slices of the qkv GEMM, rows N floats apart)
                 if (grp) {
                     a.out1 = attnb; a.out1_stride = (int)at_cols;
                     if (!launch_attn_decode_group(a, nrep, kv_mode, ns_g, nb, s)) throw CmError(CM_ERR_UNSUPPORTED, "GQA group size / head_dim");
