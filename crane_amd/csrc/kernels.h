@@ -103,7 +103,7 @@ struct GdnArgs {
     float* pre_v = nullptr;
     float* pre_bd = nullptr;
     float* pre_g = nullptr;      //   g = log(decay) [S][NV] (the chunk-parallel scan works in log space); null: not written
-    float* ck = nullptr;         // chunk-parallel scan scratch: [chunks][NV][GDN_CK_FLOATS] (W | U0 | P | cumulative g | U and the state in front of the chunk, transposed); null: sequential scan
+    float* ck = nullptr;         // chunk-parallel scan scratch: [chunks][NV][GDN_CK_FLOATS] (W | U0 | P | cumulative g | U and the state in front of the chunk; all but P and g in pieces of 64 lanes x 4 floats, as the scan's waves hold them); null: sequential scan
     float* gdn_scratch = nullptr;   // decode step on 4 workgroups per head: [n_seq][NV][V + 4] raw y + partial sums of squares
     int* gdn_ticket = nullptr;      //   and [n_seq][NV] arrival tickets (zero between launches); null: one workgroup per head
     int defer_norm = 0;         // decode step: out = RAW y, the gated RMSNorm is the out_proj GEMV's prologue (PRO_GDNNORM) -- no

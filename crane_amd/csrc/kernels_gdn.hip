@@ -426,7 +426,7 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a) {
 
 
 // ---------------------------------------------------------------------------------------------------------
-// Chunk-parallel prompt scan (round 5): the gated delta rule in its WY / UT-transform form on the f32 matrix cores.
+// Chunk-parallel prompt scan: the gated delta rule in its WY / UT-transform form on the f32 matrix cores.
 // The sequential scan above is bound by two dependent 16-lane reductions per token on 64 workgroups (240 us per layer and
 // 1024 tokens on Qwen3.5-0.8B: 43 % of its prompt pass).  The reference names the chunked form as the prompt-path algorithm
 // (ops/gdn/backend.rs:100-104); HF's torch_chunk_gated_delta_rule is the same algebra.  Per value head and chunk of C = 64
@@ -440,9 +440,8 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a) {
 // thread per column of [beta e^G K | beta V], its 64 unknowns in registers: no dependency between threads) -> W, U0, P, G.
 // gdn_chunk_scan_kernel (grid NV x V/16): the only sequential part -- U and the state's update, two small matrix products per chunk
 // over a 128 x 16 slice of the state (columns of S are independent); for prompts of more than a few chunks it leaves U and the state in front of every chunk to
-// gdn_chunk_out_kernel (grid chunks x NV), which forms Y and its gated norm for all chunks at once.  (Y inside the scan was half of
-// its products and most of its registers: 2048 + 2048 + 69 tokens, 16 heads, mean per launch: scan and norm 103.8 + 12.3 -> scan
-// 58.3, outputs 24.1 us.)  Everything stays f32 (f32 MFMA: products and sums in f32), logs of the
+// gdn_chunk_out_kernel (grid chunks x NV), which forms Y and its gated norm for all chunks at once.  (Y inside the scan is half of
+// its products and most of its registers: 2048 tokens, 16 heads, all kernels but gdn_pre_kernel: 145.2 us with it there, 118.3 apart.)  Everything stays f32 (f32 MFMA: products and sums in f32), logs of the
 // decays are summed, never multiplied (a decay of e^-80 per token underflows a running product after two tokens).
 // Same results as the sequential scan to f32 summation order (tests: prompts through both, logits < 1e-4).
 // ---------------------------------------------------------------------------------------------------------
@@ -468,71 +467,98 @@ __device__ __forceinline__ f32x4 mfma4(const f32x4& av, const f32x4& bv, f32x4 c
 
 // Where Y is formed.  A launch for the outputs of all chunks costs its start and one chunk's chain of products whatever their number, Y inside the scan a
 // part of every chunk: short prompts, while the scan's NV x 8 workgroups fit on the chip at once, keep it inside.  us a layer, scan and outputs apart
-// minus together, prompts of 2 / 3 / 4 / 5 / 6 / 8 chunks: 16 heads 6.6 / 5.0 / 3.1 / 1.2 / -1.3 / -5.3, 32 heads 6.3 / 5.6 / 3.6 / 1.7 / -0.3 / -4.4, 48 heads (384
-// workgroups) 1.1 / -2.7 / -6.9 / -11.9 / -8.8 / -19.7
+// minus together, prompts of 2 / 3 / 4 / 5 / 6 / 8 chunks: 16 heads 5.4 / 4.3 / 3.5 / 1.5 / -0.2 / -3.8, 32 heads 6.4 / 2.8 / 0.9 / 0.0 / -1.5 / -4.1, 48 heads (384
+// workgroups) -1.7 / -5.2 / -8.4 / -11.0 / -6.2 / -14.3
 static bool gdn_out_in_scan(int chunks, int NV) { return chunks <= 5 && NV * 8 <= 256; }
 
-size_t gdn_chunk_prep_lds() { return (size_t)(2 * GDN_CK * CKP + GDN_CK * CTP + 2 * GDN_CK) * sizeof(float); }
-size_t gdn_chunk_scan_lds(bool out) { return (size_t)(16 * CKP + (out ? 2 : 1) * 16 * CTP + GDN_CK * CKP + GDN_CK) * sizeof(float); }
+constexpr int ATP = 20;           // ... of a row of a 16 x 16 tile of A
+size_t gdn_chunk_prep_lds() { return (size_t)(2 * GDN_CK * CKP + 10 * 16 * ATP + 3 * GDN_CK) * sizeof(float); }
+size_t gdn_chunk_scan_lds(bool out) { return (size_t)(16 * CKP + (out ? 2 : 1) * 16 * CTP) * sizeof(float); }
 
-__global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
+// A keeps the tiles on and under its diagonal only, 81 152 bytes in all: two workgroups fit on a CU and one's products run under the other's chains (the whole of A,
+// one workgroup, V requested after the products, a row's decay exponentiated by every column: 50.1 us a launch of 32 chunks and 16 heads, 33.2 now; 48 heads 146.3, 83.9).
+// The waves' shares of the triangle are five tiles of A or of P each.
+__global__ __launch_bounds__(256, 2) void gdn_chunk_prep_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK;
     extern __shared__ __attribute__((aligned(16))) float cl[];
     float (*Ks)[CKP] = (float (*)[CKP])cl;
     float (*Qs)[CKP] = (float (*)[CKP])(cl + C * CKP);
-    float (*Am)[CTP] = (float (*)[CTP])(cl + 2 * C * CKP);
-    float* lg = cl + 2 * C * CKP + C * CTP;
+    float (*Am)[16][ATP] = (float (*)[16][ATP])(cl + 2 * C * CKP);      // tile (I, L), L <= I, at I (I + 1) / 2 + L
+    float* lg = cl + 2 * C * CKP + 10 * 16 * ATP;
     float* bt = lg + C;
+    float* be = bt + C;                                                 // beta e^G
     const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nk = a.NV / a.vpg, kh = a.chunked ? h % nk : h / a.vpg;
     const int t0 = c * C, nt = min(C, a.S - t0);
+    const bool isk = tid < K;
     float* ck = a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS;
     float* Wg = ck, *U0g = ck + C * 128, *Pg = ck + 2 * C * 128, *Gg = ck + 2 * C * 128 + C * C;
-    if (wave == 0) {                                   // cumulative log decay of the chunk (inclusive), beta
-        float g = lane < nt ? a.pre_g[(size_t)(t0 + lane) * a.NV + h] : 0.f;
+    float b[C];                                        // this thread's column of [beta e^G K | beta V]
+    {
+        f32x4 kv[8], qv[8];                            // k^ and q^ rows of the chunk (rows past the prompt: zero)
+        float g = a.pre_g[(size_t)(t0 + min(lane, nt - 1)) * a.NV + h], beta = a.pre_bd[((size_t)(t0 + min(lane, nt - 1)) * a.NV + h) * 2];
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) { const float o = __shfl_up(g, d); if (lane >= d) g += o; }
-        lg[lane] = g;
-        bt[lane] = lane < nt ? a.pre_bd[((size_t)(t0 + lane) * a.NV + h) * 2] : 0.f;
-        Gg[lane] = g;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {                      // k^ and q^ rows of the chunk (rows past the prompt: zero)
-        const int e = tid + 256 * i, row = e >> 5, c4 = (e & 31) << 2;
-        f32x4 kv = {0.f, 0.f, 0.f, 0.f}, qv = {0.f, 0.f, 0.f, 0.f};
-        if (row < nt) {
-            kv = *(const f32x4*)(a.pre_k + (size_t)(t0 + row) * a.key_dim + kh * K + c4);
-            qv = *(const f32x4*)(a.pre_q + (size_t)(t0 + row) * a.key_dim + kh * K + c4);
+        for (int i = 0; i < 8; ++i) {
+            const int e = tid + 256 * i, row = min(e >> 5, nt - 1), c4 = (e & 31) << 2;
+            kv[i] = *(const f32x4*)(a.pre_k + (size_t)(t0 + row) * a.key_dim + kh * K + c4);
+            qv[i] = *(const f32x4*)(a.pre_q + (size_t)(t0 + row) * a.key_dim + kh * K + c4);
         }
-        *(f32x4*)&Ks[row][c4] = kv;
-        *(f32x4*)&Qs[row][c4] = qv;
-    }
-    __syncthreads();
-    {   // A = tril(beta e^{G_t - G_s} K K^T, -1) -> LDS; P = tril(e^{G_t - G_s} Q K^T) -> scratch.  Wave w: token rows 16 w ..
-        const int r = lane & 15, kq = lane >> 4;
-        f32x4 accA[4], accP[4];
+        if (!isk) {                                    // (requested behind the rows that are needed first)
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc) { accA[tc] = (f32x4){0.f, 0.f, 0.f, 0.f}; accP[tc] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
+            for (int t = 0; t < C; ++t) b[t] = a.pre_v[((size_t)min(t0 + t, a.S - 1) * a.NV + h) * V + (tid - K)];
+        }
+        if (wave == 0) {                               // cumulative log decay of the chunk (inclusive), beta
+            if (lane >= nt) { g = 0.f; beta = 0.f; }
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) { const float o = __shfl_up(g, d); if (lane >= d) g += o; }
+            lg[lane] = g;
+            bt[lane] = beta;
+            be[lane] = beta * expf(g);
+            Gg[lane] = g;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int e = tid + 256 * i, row = e >> 5, c4 = (e & 31) << 2;
+            *(f32x4*)&Ks[row][c4] = row < nt ? kv[i] : (f32x4){0.f, 0.f, 0.f, 0.f};
+            *(f32x4*)&Qs[row][c4] = row < nt ? qv[i] : (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    lds_barrier();
+    {   // A = tril(beta e^{G_t - G_s} K K^T, -1) -> LDS; P = tril(e^{G_t - G_s} Q K^T) -> scratch.  Even waves A, odd ones P; waves 0 and 1 the rows of
+        // tiles 3 and 0, waves 2 and 3 those of 2 and 1: tile n of a wave's five is (hi, n) or (lo, n - n0)
+        const int r = lane & 15, kq = lane >> 4;
+        const bool isp = wave & 1;
+        const int hi = wave < 2 ? 3 : 2, lo = 3 - hi, n0 = hi + 1;
+        const float (*As)[CKP] = isp ? Qs : Ks;
+        f32x4 acc[5];
+#pragma unroll
+        for (int n = 0; n < 5; ++n) acc[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const f32x4 ak = *(const f32x4*)&Ks[16 * wave + r][16 * j + 4 * kq];
-            const f32x4 aq = *(const f32x4*)&Qs[16 * wave + r][16 * j + 4 * kq];
+            const f32x4 ah = *(const f32x4*)&As[16 * hi + r][16 * j + 4 * kq], al = *(const f32x4*)&As[16 * lo + r][16 * j + 4 * kq];
 #pragma unroll
-            for (int tc = 0; tc < 4; ++tc) {
-                if (tc > wave) continue;               // (s > t everywhere in the tile)
-                const f32x4 b = *(const f32x4*)&Ks[16 * tc + r][16 * j + 4 * kq];
-                accA[tc] = mfma4(ak, b, accA[tc]);
-                accP[tc] = mfma4(aq, b, accP[tc]);
+            for (int n = 0; n < 5; ++n) {
+                const bool up = n < n0;
+                acc[n] = mfma4(up ? ah : al, *(const f32x4*)&Ks[16 * (up ? n : n - n0) + r][16 * j + 4 * kq], acc[n]);
             }
         }
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc)
+        for (int n = 0; n < 5; ++n) {
+            const int I = n < n0 ? hi : lo, L = n < n0 ? n : n - n0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int t = 16 * wave + 4 * kq + i, s2 = 16 * tc + r;
+                const int t = 16 * I + 4 * kq + i, s2 = 16 * L + r;
                 const float e = s2 <= t ? expf(lg[t] - lg[s2]) : 0.f;
-                Am[t][s2] = s2 < t ? bt[t] * e * accA[tc][i] : 0.f;
-                Pg[t * C + s2] = e * accP[tc][i];
+                if (isp) Pg[t * C + s2] = e * acc[n][i];
+                else Am[I * (I + 1) / 2 + L][4 * kq + i][r] = s2 < t ? bt[t] * e * acc[n][i] : 0.f;
+            }
+        }
+        if (isp)
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {              // P over its diagonal: the tiles that neither row of the wave multiplies
+                const int I = n < 3 - hi ? hi : lo, L = n < 3 - hi ? n0 + n : lo + 1 + n - (3 - hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) Pg[(16 * I + 4 * kq + i) * C + 16 * L + r] = 0.f;
             }
     }
     lds_barrier();
@@ -541,14 +567,10 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
     // (All 64 rows per thread as scalar FMAs were LDS-bound: every thread reads every A[t][s] -- 512 broadcast reads per thread.)
     // X lives in LDS where k^ / q^ were ([64][264] = the same floats): every thread first forms its column of B in registers.
     {
-        const bool isk = tid < K;
-        float b[C];
         if (isk) {
 #pragma unroll
-            for (int t = 0; t < C; ++t) b[t] = bt[t] * expf(lg[t]) * Ks[t][tid];
+            for (int t = 0; t < C; ++t) b[t] = be[t] * Ks[t][tid];
         } else {
-#pragma unroll
-            for (int t = 0; t < C; ++t) b[t] = a.pre_v[((size_t)min(t0 + t, a.S - 1) * a.NV + h) * V + (tid - K)];
 #pragma unroll
             for (int t = 0; t < C; ++t) b[t] = t < nt ? bt[t] * b[t] : 0.f;
         }
@@ -557,18 +579,29 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
         float (*X)[XP] = (float (*)[XP])cl;
 #pragma unroll
         for (int t = 0; t < C; ++t) X[t][tid] = b[t];
-        float* dst = (isk ? Wg : U0g) + (isk ? tid : tid - K);
         const int r = lane & 15, kq = lane >> 4;
+        auto store = [&](int I) __attribute__((always_inline)) {        // 16 rows of W and of U0, a lane of the scan's own values in one piece
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int j = wave + 4 * i;
+                f32x4 u;
+#pragma unroll
+                for (int n = 0; n < 4; ++n) u[n] = X[16 * I + 4 * kq + n][128 + 16 * j + r];
+                *(f32x4*)(Wg + (I * 8 + j) * 256 + lane * 4) = *(const f32x4*)&X[16 * I + r][16 * j + 4 * kq];
+                *(f32x4*)(U0g + (I * 8 + j) * 256 + lane * 4) = u;
+            }
+        };
 #pragma unroll
         for (int I = 0; I < 4; ++I) {
             lds_barrier();
+            if (I > 0) store(I - 1);
             if (I > 0) {                               // R_I: wave w owns column tiles 4 w .. 4 w + 3
                 f32x4 acc[4];
 #pragma unroll
                 for (int n = 0; n < 4; ++n) acc[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int L = 0; L < I; ++L) {
-                    const f32x4 av = *(const f32x4*)&Am[16 * I + r][16 * L + 4 * kq];
+                    const f32x4 av = *(const f32x4*)&Am[I * (I + 1) / 2 + L][r][4 * kq];
 #pragma unroll
                     for (int n = 0; n < 4; ++n) {
                         f32x4 bv;
@@ -591,7 +624,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
                 float p0 = 0.f, p1 = 0.f;
 #pragma unroll
                 for (int s4 = 0; s4 < t; s4 += 4) {
-                    const f32x4 av = *(const f32x4*)&Am[16 * I + t][16 * I + s4];
+                    const f32x4 av = *(const f32x4*)&Am[I * (I + 3) / 2][t][s4];
                     p0 += av[0] * x[s4];
                     if (s4 + 1 < t) p1 += av[1] * x[s4 + 1];
                     if (s4 + 2 < t) p0 += av[2] * x[s4 + 2];
@@ -600,104 +633,106 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(GdnArgs a) {
                 x[t] -= p0 + p1;
             }
 #pragma unroll
-            for (int t = 0; t < 16; ++t) { X[16 * I + t][tid] = x[t]; dst[(16 * I + t) * 128] = x[t]; }
+            for (int t = 0; t < 16; ++t) X[16 * I + t][tid] = x[t];
         }
+        lds_barrier();
+        store(3);
     }
 }
 
 // OUT: Y of every chunk too (raw rows for gdn_post_kernel), nothing left for gdn_chunk_out_kernel
 template <bool OUT>
-__global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
+__global__ __launch_bounds__(256, OUT ? 1 : 2) void gdn_chunk_scan_kernel(GdnArgs a) {
     constexpr int K = 128, V = 128, C = GDN_CK, VB = 16;
     extern __shared__ __attribute__((aligned(16))) float cl[];
     float (*St)[CKP] = (float (*)[CKP])cl;                              // state slice, transposed: [column][k]
     float (*Vt)[CTP] = (float (*)[CTP])(cl + VB * CKP);                 // e^{G_C - G_t} U of the chunk, transposed: [column][t]
-    float (*Ks)[CKP] = (float (*)[CKP])(cl + VB * CKP + VB * CTP);      // k^ rows of the chunk
-    float* lgs = cl + VB * CKP + VB * CTP + C * CKP;
-    float (*Ut)[CTP] = (float (*)[CTP])(lgs + C);                       // OUT: U of the chunk, transposed: [column][t]
-    const int h = blockIdx.x, cb = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float (*Ut)[CTP] = (float (*)[CTP])(cl + VB * CKP + VB * CTP);      // OUT: U of the chunk, transposed: [column][t]
+    const int h = blockIdx.x, cb = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
     const int nk = a.NV / a.vpg, kh = a.chunked ? h % nk : h / a.vpg;
     float* Sg = a.state_pool + (((size_t)a.slot * a.gdn_layers + a.layer_idx) * a.NV + h) * K * V;
+    float s0[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int e = tid + 256 * i, k = e >> 4, col = e & 15;
-        St[col][k] = Sg[k * V + VB * cb + col];
+        s0[i] = Sg[k * V + VB * cb + col];
     }
+    asm volatile("" ::: "memory");
     const int nchunks = (a.S + C - 1) / C;
-    // One wave per SIMD: nothing hides a load but the wave's own work, so the operands of chunk c + 1 (this wave's 16 rows of W, its U0
-    // values, its share of the k^ rows, the cumulative log decay) are requested into registers while chunk c is multiplied --
-    // unconditionally (rows / chunks past the end are clamped and never consumed).
-    // Register sets: W rows (needed FIRST in a chunk) are requested TWO chunks ahead into two alternating sets, the rest one chunk ahead.
-    // (OUT: q^ rows beside the W rows, P rows beside U0)
+    // One or two waves per SIMD: little hides a load but the wave's own work, so the operands of a chunk are requested two chunks ahead into two alternating
+    // register sets, each where the one before it in the set is consumed -- unconditionally (rows / chunks past the end are clamped and never
+    // consumed, or multiplied by U rows that are zero); each request stands under the products that follow it.  The k^ rows go to registers too: a wave multiplies its own 32 of their columns only, lane r
+    // columns 2 r, 2 r + 1 of them, so the two state tiles hold even and odd rows and a lane's eight new state values are neighbours.  Bound by its f32 products
+    // (64 a wave and chunk, 14.3 ns each: 0.92 us) and the two hand-offs through LDS.  Us per chunk of 64 tokens: 2.4 with k^ rows staged in LDS one chunk
+    // ahead and three barriers; 2.4 from registers with the requests bunched behind the products; 1.8 with them between; 1.66 with W, U0, U and the state
+    // stored in the order of the scan's lanes, a request 1 KB in one piece.  32 chunks, 16 heads 80.4 -> 56.6 us, 48 heads 141.1 -> 106.6.
     constexpr int NQ = OUT ? 8 : 1;
-    f32x4 awA[8], awB[8], aqA[NQ], aqB[NQ], ap[4], kreg[8];
-    float u0[4], glane = 0.f;
-    auto fetch_w = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[NQ]) __attribute__((always_inline)) {
-        const int cc = min(c, nchunks - 1);
-        const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            aw[j] = *(const f32x4*)(ck + (16 * wave + r) * 128 + 16 * j + 4 * kq);
-            if constexpr (OUT) aq[j] = *(const f32x4*)(a.pre_q + (size_t)min(cc * C + 16 * wave + r, a.S - 1) * a.key_dim + kh * K + 16 * j + 4 * kq);
-        }
+    struct Set { f32x4 w[8], q[NQ], p[4], g, u0; f32x2 k[16]; float gC; } sa, sb;
+    auto part = [&](int c) __attribute__((always_inline)) { return (const char*)(a.ck + ((size_t)(min(c, nchunks - 1)) * a.NV + h) * GDN_CK_FLOATS); };
+    const uint32_t wof = (uint32_t)(wave * 2048 + lane * 4) * 4, kof = (uint32_t)(32 * wave + 2 * r) * 4;
+    auto fetch_w = [&](int c, int j, Set& o) __attribute__((always_inline)) {       // 16 columns of the W rows (OUT: and of the q^ rows)
+        o.w[j] = *(const f32x4*)(part(c) + wof + 1024 * j);
+        if constexpr (OUT) o.q[j] = *(const f32x4*)(a.pre_q + (size_t)min(min(c, nchunks - 1) * C + 16 * wave + r, a.S - 1) * a.key_dim + kh * K + 16 * j + 4 * kq);
     };
-    auto fetch_u = [&](int c) __attribute__((always_inline)) {          // U0 values of chunk c (issued once the previous ones are consumed)
-        const int cc = min(c, nchunks - 1);
-        const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
+    auto fetch_u = [&](int c, Set& o) __attribute__((always_inline)) {  // U0 values and cumulative log decays (OUT: and P rows)
+        const char* ck = part(c);
+        o.g = *(const f32x4*)(ck + (uint32_t)(2 * C * 128 + C * C + 16 * wave + 4 * kq) * 4);
+        o.u0 = *(const f32x4*)(ck + (uint32_t)(C * 128 + (wave * 8 + cb) * 256 + lane * 4) * 4);
+        o.gC = *(const float*)(ck + (2 * C * 128 + C * C + C - 1) * 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            u0[i] = ck[C * 128 + (16 * wave + 4 * kq + i) * 128 + VB * cb + r];
-            if constexpr (OUT) ap[i] = *(const f32x4*)(ck + 2 * C * 128 + (16 * wave + r) * C + 16 * i + 4 * kq);
+            if constexpr (OUT) o.p[i] = *(const f32x4*)(ck + (uint32_t)(2 * C * 128 + (16 * wave + r) * C + 16 * i + 4 * kq) * 4);
         }
     };
-    auto fetch_k = [&](int c) __attribute__((always_inline)) {          // k^ rows + cumulative log decay of chunk c: parked in LDS at the END of
-        const int cc = min(c, nchunks - 1), t0 = cc * C;                 //   chunk c - 1, so they are requested at its very beginning
-        const float* ck = a.ck + ((size_t)cc * a.NV + h) * GDN_CK_FLOATS;
+    auto fetch_k = [&](int c, int j, Set& o) __attribute__((always_inline)) {       // this wave's columns of four of every 16 k^ rows
+        const int t0 = (min(c, nchunks - 1)) * C, last = a.S - 1 - t0;
+        const char* kr = (const char*)(a.pre_k + (size_t)t0 * a.key_dim + kh * K);
+        int q4 = 4 * kq;
+        asm volatile("" : "+v"(q4));                   // (row numbers are added up here, not kept in 16 registers over the whole scan: those spilled)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = tid + 256 * i, row = min(t0 + (e >> 5), a.S - 1), c4 = (e & 31) << 2;
-            kreg[i] = *(const f32x4*)(a.pre_k + (size_t)row * a.key_dim + kh * K + c4);
-        }
-        glane = ck[2 * C * 128 + C * C + lane];
+        for (int i = 0; i < 4; ++i)                    // (24-bit products: 64 rows of a few thousand floats)
+            o.k[4 * j + i] = *(const f32x2*)(kr + (__umul24(min(q4 + (16 * j + i), last), 4 * a.key_dim) + kof));
     };
-    auto park_k = [&](int c) __attribute__((always_inline)) {          // k^ rows + cumulative log decay of chunk c -> LDS
-        const int nt = min(C, a.S - c * C);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = tid + 256 * i, row = e >> 5, c4 = (e & 31) << 2;
-            *(f32x4*)&Ks[row][c4] = row < nt ? kreg[i] : (f32x4){0.f, 0.f, 0.f, 0.f};
-        }
-        if (wave == 0) lgs[lane] = glane;
-    };
-    auto chunk = [&](int c, f32x4 (&aw)[8], f32x4 (&aq)[NQ]) __attribute__((always_inline)) {
-        float* ck = a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS;
-        fetch_k(c + 1);
+    f32x4 st[2];                                       // this lane's state values: column r, rows k = 32 wave + 8 kq + 2 i + m in st[m][i]
+    auto chunk = [&](int c, Set& o) __attribute__((always_inline)) {
+        char* ck = (char*)(a.ck + ((size_t)c * a.NV + h) * GDN_CK_FLOATS);
         // ---- U = U0 - W S0 (OUT: and Q S0): wave w owns token rows 16 w .. 16 w + 15 ----
         f32x4 accU = {0.f, 0.f, 0.f, 0.f}, accV = accU, accQ = accU, accP = accU, pc[4];
-        float eg[4];
+        float eg[4], ed[4];
+        const float eC = expf(o.gC);
+        f32x4 s[8];                                    // (all of them requested before the first product waits for one, here and below)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] = *(const f32x4*)&St[r][16 * j + 4 * kq];
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
-            const f32x4 s0 = *(const f32x4*)&St[r][16 * j + 4 * kq], s1 = *(const f32x4*)&St[r][16 * j + 16 + 4 * kq];
-            accU = mfma4(aw[j], s0, accU);
-            accV = mfma4(aw[j + 1], s1, accV);
-            if constexpr (OUT) { accQ = mfma4(aq[j], s0, accQ); accQ = mfma4(aq[j + 1], s1, accQ); }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                accU = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[j][i], s[j][i], accU, 0, 0, 0);
+                accV = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[j + 1][i], s[j + 1][i], accV, 0, 0, 0);
+                if constexpr (OUT) accQ = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[j + i / 2][2 * (i & 1)], s[j + i / 2][2 * (i & 1)], accQ, 0, 0, 0);
+                if constexpr (OUT) accQ = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[j + i / 2][2 * (i & 1) + 1], s[j + i / 2][2 * (i & 1) + 1], accQ, 0, 0, 0);
+            }
+            if (!OUT && j == 0) {                        // (stores and requests lie under products: bunched in front of a barrier they hold it up)
+                char* sd = ck + (uint32_t)(GDN_CK_ST + (cb * 8 + 2 * wave) * 256 + lane * 4) * 4;
+                *(f32x4*)sd = (f32x4){st[0][0], st[1][0], st[0][1], st[1][1]};
+                *(f32x4*)(sd + 1024) = (f32x4){st[0][2], st[1][2], st[0][3], st[1][3]};
+            }
+            ed[j / 2] = expf(o.gC - o.g[j / 2]);
+            fetch_w(c + 2, j, o);
+            fetch_w(c + 2, j + 1, o);
         }
-        fetch_w(c + 2, aw, aq);                        // this set is free again: the chunk after next
-        const float gC = lgs[C - 1];
         f32x4 u, ud;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float gt = lgs[16 * wave + 4 * kq + i];
-            u[i] = u0[i] - (accU[i] + accV[i]);
-            ud[i] = u[i] * expf(gC - gt);
-            if constexpr (OUT) { eg[i] = expf(gt); pc[i] = ap[i]; }
+            u[i] = o.u0[i] - (accU[i] + accV[i]);
+            ud[i] = u[i] * ed[i];
+            if constexpr (OUT) { eg[i] = expf(o.g[i]); pc[i] = o.p[i]; }
         }
         *(f32x4*)&Vt[r][16 * wave + 4 * kq] = ud;
         if constexpr (OUT) *(f32x4*)&Ut[r][16 * wave + 4 * kq] = u;
-        else *(f32x4*)(ck + GDN_CK_UT + (VB * cb + r) * C + 16 * wave + 4 * kq) = u;
-        fetch_u(c + 1);                                // (u0 of this chunk is consumed, its P rows copied)
-        lds_barrier();
+        lds_barrier();                                 // Vt is whole, every read of St is done
         if constexpr (OUT) {                           // ---- Y = e^G (Q S0) + P U ----
 #pragma unroll
             for (int j = 0; j < 4; ++j) accP = mfma4(pc[j], *(const f32x4*)&Ut[r][16 * j + 4 * kq], accP);
@@ -708,48 +743,61 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan_kernel(GdnArgs a) {
             }
         }
         // ---- S_C = e^{G_C} S0 + K^T (e^{G_C - G} U): wave w owns state rows k = 32 w .. 32 w + 31 ----
-        f32x4 sn[2];
-        const float eC = expf(gC);
+        f32x4 accS[2], bv[4];
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            f32x4 accS = {0.f, 0.f, 0.f, 0.f};
-            const int kr = 32 * wave + 16 * mt;
+        for (int m = 0; m < 2; ++m) accS[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const f32x4 bv = *(const f32x4*)&Vt[r][16 * j + 4 * kq];
-                f32x4 ak;
+        for (int j = 0; j < 4; ++j) bv[j] = *(const f32x4*)&Vt[r][16 * j + 4 * kq];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ak[i] = Ks[16 * j + 4 * kq + i][kr + r];
-                accS = mfma4(ak, bv, accS);
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) accS[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[4 * j + i][m], bv[j][i], accS[m], 0, 0, 0);
+            if (j == 0) {
+                if constexpr (!OUT) *(f32x4*)(ck + (uint32_t)(GDN_CK_UT + (cb * 4 + wave) * 256 + lane * 4) * 4) = u;
+                fetch_u(c + 2, o);
             }
-            const f32x4 old = *(const f32x4*)&St[r][kr + 4 * kq];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sn[mt][i] = eC * old[i] + accS[i];
+            fetch_k(c + 2, j, o);
         }
-        lds_barrier();                               // every read of St / Vt / Ks / lgs of this chunk is done
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            *(f32x4*)&St[r][32 * wave + 16 * mt + 4 * kq] = sn[mt];
-            if (!OUT && c + 1 < nchunks) *(f32x4*)(ck + (size_t)a.NV * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + r) * K + 32 * wave + 16 * mt + 4 * kq) = sn[mt];
-        }
-        park_k(c + 1);
-        lds_barrier();
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st[m][i] = eC * st[m][i] + accS[m][i];
+        *(f32x4*)&St[r][32 * wave + 8 * kq] = (f32x4){st[0][0], st[1][0], st[0][1], st[1][1]};
+        *(f32x4*)&St[r][32 * wave + 8 * kq + 4] = (f32x4){st[0][2], st[1][2], st[0][3], st[1][3]};
+        lds_barrier();                                 // St is whole, every read of Vt is done
     };
-    fetch_w(0, awA, aqA);
-    fetch_u(0);
-    fetch_k(0);
-    fetch_w(1, awB, aqB);
-    park_k(0);
+    // (in the loop's order: its waits count the loads behind the one they wait for, over both ways into it)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        Set& o = i ? sb : sa;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) fetch_w(i, j, o);
+        asm volatile("" ::: "memory");
+        fetch_u(i, o);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < 4; ++j) fetch_k(i, j, o);
+        asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int e = tid + 256 * i, k = e >> 4, col = e & 15;
+        St[col][k] = s0[i];
+    }
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < (OUT ? 0 : 2); ++i) {          // the state in front of chunk 0
-        const int e = (tid + 256 * i) * 4, col = e >> 7, k = e & 127;
-        *(f32x4*)(a.ck + (size_t)h * GDN_CK_FLOATS + GDN_CK_ST + (VB * cb + col) * K + k) = *(const f32x4*)&St[col][k];
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st[m][i] = St[r][32 * wave + 8 * kq + 2 * i + m];
+    int c = 0;
+    for (; c + 1 < nchunks; c += 2) {
+        chunk(c, sa);
+        chunk(c + 1, sb);
     }
-    for (int c = 0; c < nchunks; c += 2) {
-        chunk(c, awA, aqA);
-        if (c + 1 < nchunks) chunk(c + 1, awB, aqB);
-    }
+    if (c < nchunks) chunk(c, sa);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int e = tid + 256 * i, k = e >> 4, col = e & 15;
@@ -786,7 +834,7 @@ __global__ __launch_bounds__(512, 4) void gdn_chunk_out_kernel(GdnArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i] = *(const f32x4*)(ck + GDN_CK_ST + (tid + 512 * i) * 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { const int e = (tid + 512 * i) * 4; *(f32x4*)&Ut[e >> 6][e & 63] = u[i]; }
+        for (int i = 0; i < 4; ++i) { const int e = tid + 512 * i, l = e & 63; *(f32x4*)&Ut[(e >> 8) * 16 + (l & 15)][((e >> 6) & 3) * 16 + (l >> 4) * 4] = u[i]; }
         lds_barrier();
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -798,7 +846,10 @@ __global__ __launch_bounds__(512, 4) void gdn_chunk_out_kernel(GdnArgs a) {
     for (int j = 0; j < 8; ++j) aq[j] = *(const f32x4*)(a.pre_q + (size_t)min(t0 + 16 * rt + r, a.S - 1) * a.key_dim + kh * K + 16 * j + 4 * kq);
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { const int e = (tid + 512 * i) * 4; *(f32x4*)&St[e >> 7][e & 127] = s[i]; }
+    for (int i = 0; i < 8; ++i) {
+        const int e = tid + 512 * i, l = e & 63;
+        *(f32x4*)&St[(e >> 9) * 16 + (l & 15)][((e >> 7) & 3) * 32 + (l >> 4) * 8 + ((e >> 6) & 1) * 4] = s[i];
+    }
     lds_barrier();
     // the gate's inputs, while the products run
     const int conv_dim = 2 * a.key_dim + a.NV * V;
