@@ -285,7 +285,8 @@ void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream
 }
 bool lay_step_out_fits(const LAttnArgs& a) {
     const int K = a.H * a.e;
-    return (K == 512 || K == 1024 || K == 2048 || K == 4096) && a.e % 2 == 0 && (a.gate != LGATE_ELEM || ((uintptr_t)a.gbuf & 7) == 0);
+    // (a key head's queries in one tile of 16: the kernel finds a head's shares by its place in the first)
+    return a.H <= 16 * a.G && (K == 512 || K == 1024 || K == 2048 || K == 4096) && a.e % 2 == 0 && (a.gate != LGATE_ELEM || ((uintptr_t)a.gbuf & 7) == 0);
 }
 void launch_lay_step_out(const LAttnArgs& a, const uint16_t* Wm, float* C, int N, hipStream_t s) {
     const int W = a.H * a.e;

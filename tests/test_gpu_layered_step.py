@@ -10,10 +10,10 @@ pytestmark = pytest.mark.gpu
 
 # every width; router logits of less and more than one batch of a wave's requests, up to a wave's lanes; inner sizes below and above one piece of 512 and no
 # multiple of it, the expert of every token narrower, wider and absent; attention rows of 512 and 1024 from no, few and more shares than one batch, and of a
-# width that the merging launch keeps
+# width or with queries in two tiles that the merging launch keeps
 @pytest.mark.parametrize("width,heads,kv_heads,dim,window,experts,top,ff,shared", [
     (512, 8, 2, 64, 4096, 5, 2, 136, 72), (1024, 8, 2, 128, 1024, 14, 4, 776, 512), (2048, 8, 8, 64, 700, 64, 6, 64, 0), (4096, 16, 4, 64, 300, 63, 1, 72, 1032),
-    (512, 4, 2, 48, 900, 20, 3, 520, 520)])
+    (512, 4, 2, 48, 900, 20, 3, 520, 520), (512, 32, 1, 64, 4096, 5, 2, 136, 72)])
 @pytest.mark.parametrize("context", [3, 300, 2900])
 def test_against_single_launches(tmp_path, width, heads, kv_heads, dim, window, experts, top, ff, shared, context):
     from crane_amd.backend import Model
