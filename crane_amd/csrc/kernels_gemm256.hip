@@ -33,6 +33,21 @@ namespace {
 constexpr int TBK = 64;              // k-tile depth (elements): one 128-byte line per operand row
 constexpr int TST = 2;               // LDS stages
 
+// NW words of a plane: 16 bytes at a time where the 4 or 8 words of 256-column tiles are aligned to it, the 3 or 6 of 192-column ones in units that are
+template <int NW>
+__device__ __forceinline__ void put_words(uint16_t* p, const uint32_t (&w)[NW]) {
+    if constexpr (NW % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < NW; i += 4) *(u32x4*)(p + 2 * i) = (u32x4){w[i], w[i + 1], w[i + 2], w[i + 3]};
+    } else if constexpr (NW % 2 == 0) {
+#pragma unroll
+        for (int i = 0; i < NW; i += 2) *(u32x2*)(p + 2 * i) = (u32x2){w[i], w[i + 1]};
+    } else {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) *(uint32_t*)(p + 2 * i) = w[i];
+    }
+}
+
 }  // namespace
 
 // WST = 3 (round 4, decode groups: one m-tile, the weights come from HBM, not from a neighbour's L2 lines): a THIRD weight stage, the
@@ -45,6 +60,13 @@ template <int SPLIT, int EPI, int BN, int WST = 2, int BMX = 0>
 __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
     constexpr int BM = BMX ? BMX : (SPLIT == 2 ? 128 : 256);              // rows of a tile (two planes double the activation bytes)
     constexpr int NI = BM / 32, NJ = BN / 64, WM = BM / 2, WN = BN / 4;  // per wave: NI x NJ tiles of 16 x 16
+    // SWAP: the weight is the first operand of a product, so that a lane has four neighbouring columns of one row in the place of one column of four rows, 16 bytes
+    // per store or load of f32 outputs: 8192 x 2048, 2048 rows 123 -> 117 us; 3072 x 1024, 3172 rows 62 -> 57.  Not the slices of a split K, nor decode groups: no
+    // gain, and the gate_up of 117 rows took 1.3 us of 57 longer.
+    // NEAR (16-bit outputs): row 4 g + r of weight fragment j is column 4 NJ g + 4 j + r of the wave's, so that a lane's 4 NJ columns are neighbours (f32
+    // outputs in that order: pieces of a 64-byte row in four instructions, 130 us in the place of 117).  A workgroup that walks over several tiles, the next one's
+    // first requests in front of this one's stores, was slower by what its registers cost the loop: 2500 tokens of the 8B model 66.5 -> 73.3 ms
+    constexpr bool NEAR = EPI == GEPI_ACT_SPLIT || EPI == GEPI_SILUMUL, SWAP = NEAR || (WST == 2 && EPI != GEPI_PARTIAL);
     constexpr int PLANE = BM * TBK;                                       // elements of one activation plane of a stage
     constexpr int ASTAGE = SPLIT * PLANE, WSTAGE = BN * TBK;             // elements of an activation / a weight stage
     constexpr int WBASE = TST * ASTAGE;                                   // LDS image: [TST activation stages][WST weight stages]
@@ -86,7 +108,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
         if (p >= NPC) p = wave;
         const int plane = p < SPLIT * APC ? p / APC : SPLIT;              // SPLIT: the weight tile
         const int r0 = (plane < SPLIT ? p - plane * APC : p - SPLIT * APC) * 8, row = r0 + prow;
-        const size_t kc = (size_t)kbeg * TBK + (size_t)((pslot ^ ((row >> 1) & 7)) << 3);
+        const int turn = plane < SPLIT || !NEAR ? (row >> 1) & 7 : row % WN / (4 * NJ) * 2 + ((row >> 1) & 1);      // = fr / 2 of the lane that reads the row
+        const size_t kc = (size_t)kbeg * TBK + (size_t)((pslot ^ turn) << 3);
         if (plane < SPLIT) {
             const uint16_t* base = (SPLIT == 2 && plane == 1) ? a.A_lo : a.A_hi;
             src[i] = base + (size_t)min(m0 + row, a.M - 1) * K + kc;
@@ -100,7 +123,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
     constexpr int NWP = (BN / 8) / 8;
     static_assert(WST == 2 || ((SPLIT * APC) % 8 == 0 && (BN / 8) % 8 == 0), "counted waits need whole piece rows per wave");
 
-    const int fr = lane & 15, sw = (fr >> 1) & 7;
+    const int fr = lane & 15, sw = fr >> 1, wrow = wc * WN + (NEAR ? (fr >> 2) * 4 * NJ + (fr & 3) : fr);
     const int fk0 = ((0 + (lane >> 4)) ^ sw) << 3, fk1 = ((4 + (lane >> 4)) ^ sw) << 3;      // element offsets of the lane's chunk, k-steps 0 / 1
     bf16x8 ah[2][NI], al[2][NI], bfr[2][NJ];
     auto fetch = [&](int t) __attribute__((always_inline)) {
@@ -110,13 +133,16 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
         for (int s = 0; s < 2; ++s) {
             const int fk = s ? fk1 : fk0;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) bfr[s][j] = *(const bf16x8*)&Bs[(wc * WN + j * 16 + fr) * TBK + fk];
+            for (int j = 0; j < NJ; ++j) bfr[s][j] = *(const bf16x8*)&Bs[(wrow + j * (NEAR ? 4 : 16)) * TBK + fk];
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
                 ah[s][i] = *(const bf16x8*)&S[(wr * WM + i * 16 + fr) * TBK + fk];
                 if (SPLIT == 2) al[s][i] = *(const bf16x8*)&S[PLANE + (wr * WM + i * 16 + fr) * TBK + fk];
             }
         }
+    };
+    auto product = [](const bf16x8& x, const bf16x8& w, const f32x4& c) __attribute__((always_inline)) {
+        return SWAP ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, w, c, 0, 0, 0);
     };
     // ---- schedule: the two wave rows (waves 0-3 / 4-7; every SIMD hosts one wave of either) run half a tile apart.  A tile is two
     // phases per row, each closed by the workgroup barrier: FETCH (all fragments of tile t: LDS -> registers) and MULTIPLY (the
@@ -133,10 +159,10 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[s][i], bfr[s][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j) acc[i][j] = product(ah[s][i], bfr[s][j], acc[i][j]);
                 if (SPLIT == 2) {
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[s][i], bfr[s][j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < NJ; ++j) acc[i][j] = product(al[s][i], bfr[s][j], acc[i][j]);
                 }
             }
     };
@@ -159,10 +185,10 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[s][i], bfr[s][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j) acc[i][j] = product(ah[s][i], bfr[s][j], acc[i][j]);
                 if (SPLIT == 2) {
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[s][i], bfr[s][j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < NJ; ++j) acc[i][j] = product(al[s][i], bfr[s][j], acc[i][j]);
                 }
                 constexpr int PER = (NLOAD + 2 * NI - 1) / (2 * NI);         // requests per band (1 with 128-row tiles; 2 with 64-row tiles)
                 const int g = (s * NI + i) * PER;
@@ -220,6 +246,98 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
 
     // ---- epilogue (gemm_bf16_kernel's): C layout of mfma 16x16: col = lane & 15 (n), row = (lane >> 4) * 4 + reg (m) ----
     const int mw = m0 + wr * WM, nw = n0 + wc * WN;
+    if constexpr (NEAR) {                                                 // columns n .. n + 4 NJ - 1 of rows mw + 16 i + fr: 16 bytes per store
+        // (A column per lane, planes in 2-byte stores, tanhf: the tanh-gelu product of 3172 rows, 4096 x 1024, 100 us -> 70; gate_up of 2048 rows, 12288 x
+        // 2048, 193 -> 181)
+        const int n = nw + (lane >> 4) * 4 * NJ;
+        f32x4 bv[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bv[j][r] = a.bias != nullptr ? a.bias[n + j * 4 + r] : 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int m = mw + i * 16 + fr;
+            if (m >= a.M) continue;
+            f32x4 v[NJ];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                v[j] = acc[i][j];
+                if (a.bias != nullptr) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[j][r] += bv[j][r];
+                }
+            }
+            if (EPI == GEPI_ACT_SPLIT) {
+                if (a.act == 1) {                                             // 0.5 v (1 + tanh u) = v / (1 + e^-2u)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float x = v[j][r], u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+                            v[j][r] = x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.8853900817779268f * u));
+                        }
+                } else if (a.act == 2) {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[j][r] = 0.5f * v[j][r] * (1.0f + erff(v[j][r] * 0.7071067811865476f));
+                }
+                uint32_t hi[2 * NJ], lo[2 * NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2) {
+                        const uint32_t h = pack_bf16x2(v[j][r], v[j][r + 1]);
+                        hi[j * 2 + r / 2] = h;
+                        lo[j * 2 + r / 2] = pack_bf16x2(v[j][r] - bf16_lo(h), v[j][r + 1] - bf16_hi(h));
+                    }
+                put_words<2 * NJ>(a.H_hi + (size_t)m * a.N + n, hi);
+                if (a.H_lo) put_words<2 * NJ>(a.H_lo + (size_t)m * a.N + n, lo);
+            } else {                                                      // GEPI_SILUMUL: even column = gate_j, odd column = up_j
+                uint32_t hi[NJ], lo[NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const float x = (v[j][0] / (1.0f + expf(-v[j][0]))) * v[j][1], y = (v[j][2] / (1.0f + expf(-v[j][2]))) * v[j][3];
+                    hi[j] = pack_bf16x2(x, y);
+                    lo[j] = pack_bf16x2(x - bf16_lo(hi[j]), y - bf16_hi(hi[j]));
+                }
+                put_words<NJ>(a.H_hi + (size_t)m * (a.N / 2) + (n >> 1), hi);
+                if (a.H_lo) put_words<NJ>(a.H_lo + (size_t)m * (a.N / 2) + (n >> 1), lo);
+            }
+        }
+        return;
+    }
+    if constexpr (SWAP) {
+        const int n = nw + (lane >> 4) * 4;
+        f32x4 bv[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bv[j][r] = a.bias != nullptr ? a.bias[n + j * 16 + r] : 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int m = mw + i * 16 + fr;
+            float* c = a.C + (size_t)min(m, a.M - 1) * a.ldc + n;
+            f32x4 cold[NJ];
+            if (EPI == GEPI_RESADD) {                                     // one batch of clamped loads per row band
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) cold[j] = *(const f32x4*)(c + j * 16);
+            }
+            if (m >= a.M) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                f32x4 v = acc[i][j];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (a.bias != nullptr) v[r] += bv[j][r];
+                    if (EPI == GEPI_RESADD) v[r] = cold[j][r] + v[r];
+                }
+                *(f32x4*)(c + j * 16) = v;
+            }
+        }
+        return;
+    }
     if (EPI == GEPI_PARTIAL) {
         float* P = a.ws + (size_t)ks * a.M * a.N;
 #pragma unroll
@@ -258,28 +376,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
                 if (a.bias != nullptr) v += bv[j];
                 if (EPI == GEPI_STORE) {
                     if (m < a.M) a.C[(size_t)m * a.ldc + n] = v;
-                } else if (EPI == GEPI_RESADD) {
-                    if (m < a.M) a.C[(size_t)m * a.ldc + n] = cold[j][r] + v;
-                } else if (EPI == GEPI_ACT_SPLIT) {
-                    if (m < a.M) {
-                        float h = v;
-                        if (a.act == 1) h = 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
-                        else if (a.act == 2) h = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
-                        const size_t off = (size_t)m * a.N + n;
-                        const uint16_t hh = f32_to_bf16(h);
-                        a.H_hi[off] = hh;
-                        if (a.H_lo) a.H_lo[off] = f32_to_bf16(h - bf16_to_f32(hh));
-                    }
-                } else {                                                  // GEPI_SILUMUL: even column = gate_j, odd column = up_j
-                    const float up = dpp_mov<0xB1>(v);                    // lane ^ 1
-                    if (((lane & 1) == 0) && m < a.M) {
-                        const float h = (v / (1.0f + expf(-v))) * up;
-                        const size_t off = (size_t)m * (a.N / 2) + (n >> 1);
-                        const uint16_t hh = f32_to_bf16(h);
-                        a.H_hi[off] = hh;
-                        if (a.H_lo) a.H_lo[off] = f32_to_bf16(h - bf16_to_f32(hh));
-                    }
-                }
+                } else if (m < a.M) a.C[(size_t)m * a.ldc + n] = cold[j][r] + v;
             }
         }
     }
@@ -304,6 +401,8 @@ static void launch_one(const GemmArgs& a, int blocks, hipStream_t s) {
 // a.ksplit set by the caller (1: epilogue `epi`; > 1: GEPI_PARTIAL tiles, the caller runs gemm_splitk_epilogue_kernel)
 bool launch_gemm256(const GemmArgs& a, int epi, int bn, hipStream_t s) {
     if ((bn != 256 && bn != 192) || a.N % bn != 0 || a.K % TBK != 0 || (a.K / TBK) % a.ksplit != 0) return false;
+    const bool near = epi == GEPI_ACT_SPLIT || epi == GEPI_SILUMUL;
+    if (near ? (((uintptr_t)a.H_hi | (uintptr_t)a.H_lo) & 15) != 0 : ((uintptr_t)a.C & 15) != 0 || a.ldc % 4 != 0) return false;      // (16 bytes at a time)
     const bool split = a.A_lo != nullptr;
     const int bm = gemm256_rows(split, a.M);
     const int blocks = ((a.M + bm - 1) / bm) * (a.N / bn) * a.ksplit;
