@@ -19,7 +19,7 @@
 // Bound: LDS.  A wave's k-step of 64 x 64 outputs reads 8 KB of fragments for 16 products (256 cycles); four waves of two blocks ask for the
 // LDS ports' full 128 bytes a cycle.  64 x 64 tiles: the latency of the weights' first touch and the L2's traffic per product.
 // Measured (us per launch, gate-and-up / down; the 64 x 64 kernel without a pipeline that this replaces in brackets): 8192 rows, 16 experts of
-// 2048 x 4096: 375 / 243 (2481 / 1566), 0.73 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 14.8 / 11.1 (60 / 50).  Tiles of 128 x 256 and 256 x 256
+// 2048 x 4096: 375 / 243 (2481 / 1566), 0.73 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 14.8 / 11.1 (60 / 50); before 16-byte stores.  Tiles of 128 x 256 and 256 x 256
 // with eight waves: 388 and 396 at the first size (coarser shares of the last round), 70 for 75 on one matrix of 4096 x 4096; not kept.
 #include <algorithm>
 
@@ -83,35 +83,55 @@ __device__ __forceinline__ void take(LTileArgs& a, const LTileArgs& b) {
     a.M = b.M; a.N = b.N; a.K = b.K; a.grp_off = nullptr; a.bias = b.bias; a.act = b.act; a.act2 = b.act2; a.act_split = b.act_split; a.act_param = b.act_param;
 }
 
-// a wave's NI x NJ products to memory, rows mw .. and columns nw .. of the tile.  D of a product: column = lane % 16, rows 4 (lane / 16) + r.  DUAL: the
-// upper half of the NJ columns belongs to W2.  The outputs' function is chosen once per block
+// a wave's NI x NJ products to memory, rows mw .. and columns nw .. of the tile.  The weight is a product's first operand: a lane has columns 4 (lane / 16) + r of row
+// lane % 16, one store of 8 or 16 bytes per product and one look at c_idx per band (a column of four rows each: 54 us for 46 and 49 for 37, gate-and-up and
+// down of 1200 tokens, 14 experts of 768 x 1024; 417 and 174 for 409 and 163, 2048 tokens, 16 of 2048 x 4096 and the projections beside them).  DUAL: the upper half of the NJ
+// columns belongs to W2.  The outputs' function is chosen once per block
 template <int NI, int NJ, bool DUAL>
-__device__ __forceinline__ void store_tile(const LTileArgs& a, const f32x4 (&acc)[NI][NJ], int rows, int p0, int mw, int nw, int lane) {
+__device__ __forceinline__ void store_tile(const LTileArgs& a, f32x4 (&acc)[NI][NJ], int rows, int p0, int mw, int nw, int lane) {
     constexpr int NC = DUAL ? NJ / 2 : NJ;
     const int fr = lane & 15, lg = lane >> 4;
-    auto store = [&](auto f) __attribute__((always_inline)) {
+    const bool vec = a.ldc % 4 == 0 && ((uintptr_t)a.C & (DUAL ? 7 : 15)) == 0;
+    size_t row[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int p = p0 + min(mw + i * 16 + fr, rows - 1);
+        row[i] = a.c_idx ? (size_t)a.c_idx[p] : (size_t)p;
+    }
+    auto apply = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = mw + i * 16 + lg * 4 + r;
-                if (m >= rows) continue;
-                const size_t row = a.c_idx ? (size_t)a.c_idx[p0 + m] : (size_t)(p0 + m);
+            for (int j = 0; j < NC; ++j)
 #pragma unroll
-                for (int j = 0; j < NC; ++j) {
-                    const int n = nw + j * 16 + fr;
-                    if (n >= a.N) continue;
-                    if (DUAL) ((uint16_t*)a.C)[row * a.ldc + n] = f32_to_bf16(f(acc[i][j][r], acc[i][j + (DUAL ? NC : 0)][r], n));
-                    else ((float*)a.C)[row * a.ldc + n] = f(acc[i][j][r], 0.f, n);
-                }
-            }
+                for (int r = 0; r < 4; ++r) acc[i][j][r] = f(acc[i][j][r], acc[i][j + (DUAL ? NC : 0)][r], min(nw + j * 16 + lg * 4 + r, a.N - 1));
     };
     if (DUAL) {
-        if (a.act == LACT_SILU) store([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
-        else if (a.act == LACT_CAPGLU) store([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
-        else store([&](float v, float u, int) { return lay_act(v, a.act) * u; });
-    } else if (!a.bias && a.act == LACT_NONE && a.act2 == LACT_NONE) store([](float v, float, int) { return v; });
-    else store([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+        if (a.act == LACT_SILU) apply([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
+        else if (a.act == LACT_CAPGLU) apply([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
+        else apply([&](float v, float u, int) { return lay_act(v, a.act) * u; });
+    } else if (a.bias || a.act != LACT_NONE || a.act2 != LACT_NONE)
+        apply([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        if (mw + i * 16 + fr >= rows) continue;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int n = nw + j * 16 + lg * 4;
+            const f32x4 v = acc[i][j];
+            const size_t at = row[i] * a.ldc + n;
+            if (vec && n + 4 <= a.N) {
+                if (DUAL) *(u32x2*)((uint16_t*)a.C + at) = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                else *(f32x4*)((float*)a.C + at) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (n + r >= a.N) continue;
+                    if (DUAL) ((uint16_t*)a.C)[at + r] = f32_to_bf16(v[r]); else ((float*)a.C)[at + r] = v[r];
+                }
+            }
+        }
+    }
 }
 
 template <int BM, int BN, int ST, bool DUAL>
@@ -191,7 +211,7 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
 #pragma unroll
             for (int i = 0; i < NI; ++i)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail: none may land after the block is gone
