@@ -141,3 +141,10 @@ def test_rows_that_are_no_numbers(tmp_path, bad, seqs, portion):
         m.close()
     # (the norm's tanh takes infinities to one: their logits are finite)
     assert np.isnan(got[0][-1]).all() == np.isnan(bad) and np.isfinite(got[1]).all() and (got[0][:-1] == got[1][:-1]).all()
+
+
+# outputs of a number of columns that four does not divide (a gate per head, three heads): rows that are not 16-byte aligned
+@pytest.mark.parametrize("n", [33, 130])
+def test_columns_that_four_does_not_divide(tmp_path, n):
+    cfg = GZ.config([GZ.layer(GZ.attn(heads=3, kv_heads=3), GZ.moe(experts=4, top=2, ff=128, shared=128))], vocab=97, width=128)
+    _check(tmp_path, GZ, cfg, n, 11)
