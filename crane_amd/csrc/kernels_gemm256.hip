@@ -1,7 +1,7 @@
 // Prompt-pass GEMM for LARGE M fed by LDS-DMA in FULL cache lines:  C[M, N] (+)= A[M, K] . W[N, K]^T, bf16 operands, f32
 // accumulate, the activation operand as one bf16 plane (SPLIT = 1) or as bf16 hi + lo planes (SPLIT = 2, the parity mode: two
 // MFMAs per product).  Same epilogues and, per accumulator, the same sequence of MFMAs (k ascending; hi then lo) as
-// gemm_bf16_kernel (kernels_prefill.hip): an un-split launch is bit-equal to that kernel's.
+// gemm_bf16_kernel (kernels_prefill.hip): an un-split launch of several row tiles is bit-equal to that kernel's, but for tanh-gelu (one row tile: another k start per column tile).
 //
 // Why a second kernel -- what the round-2 profile's 47 % MFMA-busy was waiting for.  gemm_bf16_kernel walks K in 32-element
 // k-tiles: every operand row contributes a 64-byte segment per tile, i.e. HALF of a 128-byte cache line, and the other half is
