@@ -597,6 +597,22 @@ int cm_debug_lay_tile_plan(int32_t tokens, int32_t columns, int32_t experts, int
     return cm::lay_tile_wide(a, beside != 0);
 }
 
+int cm_debug_lay_tile_shape(int32_t tokens, int32_t columns, int32_t inner, int32_t experts, int32_t top, int32_t pair, int32_t beside, int32_t function) {
+    cm::LTileArgs a, b;
+    a.M = tokens; a.N = columns; a.K = inner;
+    const uint16_t w = 0;
+    const int32_t off = 0;
+    if (pair) a.W2 = &w;
+    if (experts > 0) { a.grp_off = &off; a.groups = experts; a.total = tokens * top; }
+    if (function) { a.act = cm::LACT_SILU; a.act_split = columns; }
+    if (beside > 0) { b.M = tokens; b.N = beside; b.K = inner; b.W2 = a.W2; }
+    const bool tail = cm::lay_tile_tail(a, beside > 0);
+    if (tail) a.N -= a.N % 128;
+    static const int sizes[] = {64064, 128128, 192128, 128192, 256256};
+    const int size = sizes[cm::lay_tile_shape(a, b)];
+    return tail ? -size : size;
+}
+
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim) { return cm::attn_prefill_shares(rows, start, heads, head_dim); }
 
 int cm_debug_set(cm_model* h, const char* key, int64_t value) {

@@ -19,9 +19,12 @@
 // Bound: LDS.  A wave's k-step of 64 x 64 outputs reads 8 KB of fragments for 16 products (256 cycles); four waves of two blocks ask for the
 // LDS ports' full 128 bytes a cycle.  64 x 64 tiles: the latency of the weights' first touch and the L2's traffic per product.
 // Measured (us per launch, gate-and-up / down; the 64 x 64 kernel without a pipeline that this replaces in brackets): 8192 rows, 16 experts of
-// 2048 x 4096: 375 / 243 (2481 / 1566), 0.73 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 14.8 / 11.1 (60 / 50); before 16-byte stores.  Tiles of 128 x 256 and 256 x 256
-// with eight waves: 388 and 396 at the first size (coarser shares of the last round), 70 for 75 on one matrix of 4096 x 4096; not kept.
+// 2048 x 4096: 375 / 243 (2481 / 1566), 0.73 PFLOP/s; 1200 rows, 14 experts of 768 x 1024: 14.8 / 11.1 (60 / 50); before 16-byte stores.  Larger tiles read fewer
+// fragments per product: 192 x 128 and 128 x 192 on the same kernel (two blocks still share a CU: 160 KB of LDS), 256 x 256 with eight waves in two phases
+// (lay_tall_gemm_kernel; with this kernel's one barrier per k-tile it was no faster); lay_tile_shape says which a product takes, with the figures.
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 #include "dev_common.h"
 #include "kernels.h"
@@ -87,7 +90,7 @@ __device__ __forceinline__ void take(LTileArgs& a, const LTileArgs& b) {
 // lane % 16, one store of 8 or 16 bytes per product and one look at c_idx per band (a column of four rows each: 54 us for 46 and 49 for 37, gate-and-up and
 // down of 1200 tokens, 14 experts of 768 x 1024; 417 and 174 for 409 and 163, 2048 tokens, 16 of 2048 x 4096 and the projections beside them).  DUAL: the upper half of the NJ
 // columns belongs to W2.  The outputs' function is chosen once per block
-template <int NI, int NJ, bool DUAL>
+template <int NI, int NJ, bool DUAL, bool FN = true>
 __device__ __forceinline__ void store_tile(const LTileArgs& a, f32x4 (&acc)[NI][NJ], int rows, int p0, int mw, int nw, int lane) {
     constexpr int NC = DUAL ? NJ / 2 : NJ;
     const int fr = lane & 15, lg = lane >> 4;
@@ -110,8 +113,12 @@ __device__ __forceinline__ void store_tile(const LTileArgs& a, f32x4 (&acc)[NI][
         if (a.act == LACT_SILU) apply([](float v, float u, int) { return lay_act(v, LACT_SILU) * u; });
         else if (a.act == LACT_CAPGLU) apply([&](float v, float u, int) { return lay_capglu(v, u, a.act_param); });
         else apply([&](float v, float u, int) { return lay_act(v, a.act) * u; });
-    } else if (a.bias || a.act != LACT_NONE || a.act2 != LACT_NONE)
-        apply([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+    } else if (FN && (a.bias || (nw < a.act_split && a.act != LACT_NONE) || (nw + NC * 16 > a.act_split && a.act2 != LACT_NONE))) {
+        // (columns that have a function; a sigmoid behind the rest by itself, lay_act for every element is 10 KB of code and more: the projection of 326 rows of 1024
+        // 13.3 us, 8.2 here)
+        if (!a.bias && a.act == LACT_NONE && a.act2 == LACT_SIGMOID) apply([&](float v, float, int n) { const float g = lay_act(v, LACT_SIGMOID); return n < a.act_split ? v : g; });
+        else apply([&](float v, float, int n) { return lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param); });
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         if (mw + i * 16 + fr >= rows) continue;
@@ -134,7 +141,7 @@ __device__ __forceinline__ void store_tile(const LTileArgs& a, f32x4 (&acc)[NI][
     }
 }
 
-template <int BM, int BN, int ST, bool DUAL>
+template <int BM, int BN, int ST, bool DUAL, bool FN>
 __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, LTileArgs second, int ntiles, int ntiles_b) {
     constexpr int WM = BM / 2, WN = BN / 2, NI = WM / 16, NJ = WN / 16, APC = BM / 8, NL = (BM + BN) / 32;      // NL: loads per wave and k-tile
     constexpr int NC = DUAL ? WN / 2 : WN;                                // output columns of a wave
@@ -215,7 +222,123 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail: none may land after the block is gone
-    store_tile<NI, NJ, DUAL>(a, acc, rows, p0, wm * WM, n0 + wn * NC, lane);
+    store_tile<NI, NJ, DUAL, FN>(a, acc, rows, p0, wm * WM, n0 + wn * NC, lane);
+}
+
+// 256 x 256 tiles, eight waves as 2 x 4, a wave 128 x 64 outputs: 24 KB of fragments for 64 products a k-tile, three quarters of what the 64 x 64 of the
+// kernel above ask the LDS for per product.  The schedule of gemm256_kernel (kernels_gemm256.hip): the two wave rows run half a tile apart, one multiplies a tile
+// from registers while the other fetches its fragments of the next and requests the tile behind it, a request between two bands of products.  A band of 16 rows
+// behind a ragged tile's end multiplies nothing.  8192 rows, 4096 columns, K 4096: 359 us on 128 x 128 tiles, 228 - 305 here by what the clock allows (183 with
+// operands of zeros: 1.5 PFLOP/s)
+template <bool DUAL>
+__global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTileArgs second, int ntiles, int ntiles_b) {
+    constexpr int BM = 256, BN = 256, WM = 128, WN = 64, NI = 8, NJ = 4, NL = 8, NC = DUAL ? WN / 2 : WN, APC = BM / 8, STAGE = (BM + BN) * BK;
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3;
+    Tile at;
+    if (!find_tile<BM>(first, second, ntiles, ntiles_b, lane, at)) return;
+    LTileArgs a = first;
+    if (at.side) take(a, second);
+    const int p0 = at.p0, rows = at.rows;
+    const uint16_t* W = a.W + (size_t)at.g * a.w_stride;
+    const uint16_t* W2 = DUAL ? a.W2 + (size_t)at.g * a.w_stride : nullptr;
+    const int n0 = at.nt * (DUAL ? BN / 2 : BN);
+
+    // loads as above: piece wave + 8 i covers 8 rows of A (i < 4) or of the weight tile
+    const int prow = lane >> 3, pslot = lane & 7;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+    const uint16_t* src[NL];
+    uint32_t dst[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int p = wave + 8 * i;
+        const bool isA = p < APC;
+        const int row = (isA ? p : p - APC) * 8 + prow;
+        const int kc = (pslot ^ ((row >> 1) & 7)) << 3;
+        if (isA) {
+            const int r = p0 + min(row, rows - 1);
+            src[i] = a.A + (size_t)(a.a_idx ? a.a_idx[r] / a.a_div : r) * a.lda + kc;
+        } else {
+            const int c = row / WN, q = row - c * WN;
+            const bool up = DUAL && q >= NC;
+            src[i] = (up ? W2 : W) + (size_t)min(n0 + c * NC + (up ? q - NC : q), a.N - 1) * a.K + kc;
+        }
+        dst[i] = lds0 + (uint32_t)(p * 8 * BK) * 2u;
+    }
+    const int nk = a.K / BK;
+    auto piece = [&](int i, int t) __attribute__((always_inline)) {       // past the end: the last tile again, into a stage nobody reads
+        lds_load16(src[i] + (size_t)min(t, nk - 1) * BK, dst[i] + (uint32_t)((t & 1) * STAGE) * 2u);
+    };
+    auto request = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) piece(i, t);
+    };
+    f32x4 acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, lg = lane >> 4, sw = (fr >> 1) & 7;
+    const int bands = min(NI, (rows - wm * WM + 15) >> 4);                // bands of this wave that have rows (none: 0 or less)
+    bf16x8 af[2][NI], bf[2][NJ];
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+        const uint16_t* As = lds + (t & 1) * STAGE + wm * WM * BK;
+        const uint16_t* Bs = lds + (t & 1) * STAGE + (BM + wn * WN) * BK;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int fk = ((s * 4 + lg) ^ sw) << 3;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) bf[s][j] = *(const bf16x8*)&Bs[(j * 16 + fr) * BK + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) af[s][i] = *(const bf16x8*)&As[(i * 16 + fr) * BK + fk];
+        }
+    };
+    auto band = [&](int s, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[s][j], af[s][i], acc[i][j], 0, 0, 0);
+    };
+    // every wave runs 2 nk + 2 barriers
+    request(0);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (wm == 0) {
+        for (int t = 0; t < nk; ++t) {
+            request(t + 1);
+            fetch(t);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (i < bands) { band(0, i); band(1, i); }
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        asm volatile("s_barrier" ::: "memory");
+    } else {
+        request(1);                                                       // in the slot in which row 0 fetches tile 0
+        asm volatile("s_barrier" ::: "memory");
+        for (int t = 0; t < nk; ++t) {
+            fetch(t);
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                if (i < bands) { band(0, i); band(1, i); }
+                __builtin_amdgcn_sched_barrier(0);
+                piece(i, t + 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_barrier" ::: "memory");
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // the repeated loads of the tail
+    store_tile<NI, NJ, DUAL, DUAL>(a, acc, rows, p0, wm * WM, n0 + wn * NC, lane);
 }
 
 // row tiles of a launch; grouped: every expert ends in at most one ragged tile, and none has more than M rows
@@ -224,17 +347,87 @@ int mtiles(const LTileArgs& a) {
     return a.grp_off ? std::min((a.total + BM - 1) / BM + a.groups, a.groups * ((a.M + BM - 1) / BM)) : (a.M + BM - 1) / BM;
 }
 
-template <int BM, int BN, int ST, bool DUAL>
+template <int BM, int BN, int ST, bool DUAL, bool FN = true>
 void go(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
     constexpr size_t lds = (size_t)ST * (BM + BN) * BK * sizeof(uint16_t);
     static DevOnce attr;
     attr.run([&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tile_gemm_kernel<BM, BN, ST, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tile_gemm_kernel<BM, BN, ST, DUAL, FN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
     const int cols = DUAL ? BN / 2 : BN, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
     const int share = (mtiles<BM>(a) * nt + 7) / 8 + ((b.M + BM - 1) / BM * ntb + 7) / 8;
-    hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL>), dim3((unsigned)share * 8), dim3(256), lds, s, a, b, nt, ntb);
+    hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL, FN>), dim3((unsigned)share * 8), dim3(256), lds, s, a, b, nt, ntb);
 }
+template <bool DUAL>
+void go_tall(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
+    constexpr size_t lds = (size_t)2 * 512 * BK * sizeof(uint16_t);
+    static DevOnce attr;
+    attr.run([&] { (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tall_gemm_kernel<DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+    const int cols = DUAL ? 128 : 256, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
+    const int share = (mtiles<256>(a) * nt + 7) / 8 + ((b.M + 255) / 256 * ntb + 7) / 8;
+    hipLaunchKernelGGL((lay_tall_gemm_kernel<DUAL>), dim3((unsigned)share * 8), dim3(512), lds, s, a, b, nt, ntb);
+}
+
+// The last columns of one matrix, [n0, N), at most 64 of them: 16 rows per block, the k-tiles dealt to its eight waves, operands from memory straight into fragments.
+// What it saves: 32 gate columns behind 4096 others were a column tile of their own, 16 blocks behind the 512 that fill the chip (2048 rows, K 4096: 116 us in
+// the place of 76; here 76 + 14, four tiles requested together no less)
+template <int NJ>
+__global__ __launch_bounds__(512) void lay_few_cols_kernel(LTileArgs a, int n0) {
+    constexpr int NW = 8;
+    __shared__ __attribute__((aligned(16))) float part[NW][NJ][64][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, lg = lane >> 4, m0 = (int)blockIdx.x * 16;
+    const uint16_t* A = a.A + (size_t)min(m0 + fr, a.M - 1) * a.lda + lg * 8;
+    const uint16_t* W[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) W[j] = a.W + (size_t)min(n0 + j * 16 + fr, a.N - 1) * a.K + lg * 8;
+    f32x4 acc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // (a row's stride is a multiple of the memory channels' turn where K is a power of two: blocks start at different tiles, or all ask the same channels at once: 16 us)
+    const int cnt = (a.K / BK - wave + NW - 1) / NW;
+    int at = cnt > 0 ? (int)blockIdx.x % cnt : 0;
+#pragma unroll 4
+    for (int i = 0; i < cnt; ++i, at = at + 1 < cnt ? at + 1 : 0) {
+        const int k = (at * NW + wave) * BK;
+        bf16x8 x[2], w[2][NJ];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            x[h] = *(const bf16x8*)(A + k + h * 32);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) w[h][j] = *(const bf16x8*)(W[j] + k + h * 32);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h][j], x[h], acc[j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) *(f32x4*)part[wave][j][lane] = acc[j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < NJ * 256; i += 512) {                   // element i: fragment i / 256, row i / 16 % 16, column i % 16
+        const int j = i >> 8, m = (i >> 4) & 15, c = i & 15, l = (c >> 2) * 16 + m, n = n0 + j * 16 + c;
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) v += part[w][j][l][c & 3];
+        if (m0 + m < a.M && n < a.N) ((float*)a.C)[(size_t)(m0 + m) * a.ldc + n] = lay_act(a.bias ? v + a.bias[n] : v, n < a.act_split ? a.act : a.act2, a.act_param);
+    }
+}
+void go_few_cols(const LTileArgs& a, int n0, hipStream_t s) {
+    const dim3 grid((unsigned)((a.M + 15) / 16));
+    if (a.N - n0 <= 16) hipLaunchKernelGGL(lay_few_cols_kernel<1>, grid, dim3(512), 0, s, a, n0);
+    else if (a.N - n0 <= 32) hipLaunchKernelGGL(lay_few_cols_kernel<2>, grid, dim3(512), 0, s, a, n0);
+    else hipLaunchKernelGGL(lay_few_cols_kernel<4>, grid, dim3(512), 0, s, a, n0);
+}
+
+// row tiles that a launch will have: of n rows an expert has on average, spread by their root
+float row_tiles(const LTileArgs& a, int bm) {
+    if (!a.grp_off) return (float)((a.M + bm - 1) / bm);
+    const float avg = (float)a.total / a.groups, sd = std::sqrt(avg) + 1e-3f;
+    float t = 1.f;
+    for (int k = 1; k * bm < a.M; ++k) t += std::min(1.f, std::max(0.f, 0.5f + (avg - (float)(k * bm)) / (3.f * sd)));
+    return t * a.groups;
+}
+bool plain_out(const LTileArgs& a) { return !a.bias && (a.act == LACT_NONE || a.act_split <= 0) && (a.act2 == LACT_NONE || a.act_split >= a.N); }
 
 }  // namespace
 
@@ -252,12 +445,65 @@ bool lay_tile_wide(const LTileArgs& a, bool beside) {
     return blocks >= LAY_TILE_WIDE_BLOCKS && (total >= 64 * groups || (a.grp_off && !a.W2 && !beside));
 }
 
-void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s, const LTileArgs* beside) {
-    if (a.M <= 0 || a.N <= 0) return;
-    const LTileArgs b = beside ? *beside : LTileArgs();
+// Larger tiles than those two have fewer blocks, and a launch takes as many rounds of blocks as do not fit the chip at once (512 of four waves, 256 of eight): the shape
+// whose rounds take the least.  A round in quarters of one of 128 x 128 tiles, measured: 192 x 128 5, 128 x 192 5.4, 256 x 256 6.2; 64 x 64 tiles, three blocks on a CU and
+// short ones, 2.6 and half a round for the ends.  us a launch, the two above / the shape taken, experts of 2048 x 4096 as above, weights out of memory:
+// gate-and-up 2048 tokens 465 / 397 (256 x 256), 1200 310 / 289 (192 x 128), 700 231 / 198 (192 x 128), 450 185 / 130 (128 x 192), 300 177 / 119, 200 126 / 113, 100 115 / 115 (64);
+// down 250 / 219, 167 / 156, 124 / 110, 92 / 83, 87 / 73, 69 / 62, 62 / 62.  14 experts of 768 x 1024, one of 512: 2048 tokens 47, 38 / 30 (192 x 128), 1300 43 / 33, 22, 500 24, 15.
+// One matrix, K 4096: 2048 rows, 6144 columns 135 / 111 (256 x 256), 4096 columns 76 (128)
+static LayTileShape lay_tile_least(const LTileArgs& a, const LTileArgs& b, float& least) {
+    struct { LayTileShape shape; int bm, bn, slots; float round; } const all[] = {
+        {LTILE_128, 128, 128, 512, 4.f}, {LTILE_192_128, 192, 128, 512, 5.f}, {LTILE_128_192, 128, 192, 512, 5.4f}, {LTILE_256, 256, 256, 256, 6.2f}};
+    auto blocks = [&](int bm, int bn) {
+        const int cols = a.W2 ? bn / 2 : bn;
+        return row_tiles(a, bm) * (float)((a.N + cols - 1) / cols) + (b.M > 0 ? row_tiles(b, bm) * (float)((b.N + cols - 1) / cols) : 0.f);
+    };
     const bool wide = lay_tile_wide(a, b.M > 0);
-    if (a.W2) { if (wide) go<128, 128, 2, true>(a, b, s); else go<64, 64, 3, true>(a, b, s); }
-    else { if (wide) go<128, 128, 2, false>(a, b, s); else go<64, 64, 3, false>(a, b, s); }
+    LayTileShape best = wide ? LTILE_128 : LTILE_64;
+    least = wide ? 4.f * std::ceil(blocks(128, 128) / 512.f) : 2.6f * (blocks(64, 64) / 768.f + 0.5f);
+    if (!a.W2 && !(plain_out(a) && (b.M <= 0 || plain_out(b)))) return best;      // (the large tiles' stores know no bias and no function)
+    for (const auto& c : all) {
+        const float t = c.round * std::ceil(blocks(c.bm, c.bn) / (float)c.slots);
+        if (t < least) { least = t; best = c.shape; }
+    }
+    return best;
+}
+
+LayTileShape lay_tile_shape(const LTileArgs& a, const LTileArgs& b) { float t; return lay_tile_least(a, b, t); }
+
+// One matrix whose last 1 .. 64 columns reach into a further column tile: a launch of their own (5 us at K 1024, 14 at 4096) where it saves more rounds' time than that, a quarter of a round of 128 x 128
+// tiles being about 5 us per 1024 of K.  2048 rows, K 4096: 4128 columns 116 us in one launch, 76 + 14 in two; 6176 145, 109 + 14; K 1024, 1032 columns: 14 in one, 11 + 5
+bool lay_tile_tail(const LTileArgs& a, bool beside) {
+    const int rest = a.N % 128;
+    if (a.grp_off || a.W2 || a.a_idx || a.c_idx || beside || rest == 0 || rest > 64 || a.N < 256) return false;
+    LTileArgs m = a;
+    m.N -= rest;
+    float all, main;
+    lay_tile_least(a, LTileArgs(), all);
+    lay_tile_least(m, LTileArgs(), main);
+    return (all - main) * (float)a.K > 4096.f * 0.8f;
+}
+
+void launch_lay_tile_gemm(const LTileArgs& a0, hipStream_t s, const LTileArgs* beside) {
+    if (a0.M <= 0 || a0.N <= 0) return;
+    LTileArgs a = a0;
+    const LTileArgs b = beside ? *beside : LTileArgs();
+    const int rest = a.N % 128;
+    if (lay_tile_tail(a, b.M > 0)) {                                      // the last columns in a launch of their own
+        go_few_cols(a, a.N - rest, s);
+        a.N -= rest;
+    }
+    auto launch = [&](auto dual) {
+        constexpr bool DUAL = decltype(dual)::value;
+        switch (lay_tile_shape(a, b)) {
+            case LTILE_64: go<64, 64, 3, DUAL>(a, b, s); break;
+            case LTILE_128: go<128, 128, 2, DUAL>(a, b, s); break;
+            case LTILE_192_128: go<192, 128, 2, DUAL, DUAL>(a, b, s); break;
+            case LTILE_128_192: go<128, 192, 2, DUAL, DUAL>(a, b, s); break;
+            case LTILE_256: go_tall<DUAL>(a, b, s); break;
+        }
+    };
+    if (a.W2) launch(std::true_type()); else launch(std::false_type());
 }
 
 // rows of f32, gathered and scaled -> bfloat16: out[p] = x[idx[p] / div] * scale[idx[p]]

@@ -138,7 +138,7 @@ struct LayeredLayerW {
     //   chunk attention: q (H d) | k (G d) | v (G e) | g (H e) (k, v absent when borrowed);  latent: dq (q_rank) | dkv (kv_rank + rot) | g (H e)
     //   gated linear attention: q (H d) | k (H d) | v (H e) | a1 (rank) | g (H e)
     float* in_b = nullptr;                           // [rows] (zeros where the checkpoint has no bias) or null
-    int in_rows = 0, q_off = 0, k_off = 0, v_off = 0, g_off = 0, a_off = 0;
+    int in_rows = 0, in_used = 0 /* in front of rows of zeros; 0: all */, q_off = 0, k_off = 0, v_off = 0, g_off = 0, a_off = 0;
     float* shift = nullptr;                          // token shift as a two-tap convolution: [W][2] = {s, -s}
     float *sink = nullptr;                           // attention: [H]
     float *dq_norm = nullptr, *dkv_norm = nullptr;   // latent attention: plain norm weights of the two latents
@@ -195,6 +195,7 @@ struct LGemmArgs {
     float* C = nullptr; int ldc = 0;
     const int32_t* c_idx = nullptr;                  // output row of p: c_idx ? c_idx[p] : p
     int M = 0, N = 0, K = 0;
+    int n_used = 0;                                  // columns from here on are padding that nobody reads: rows of zeros (0: none)
     const int32_t* grp_off = nullptr;                // grouped: rows [grp_off[g], grp_off[g + 1]) use matrix g; M bounds a group's rows
     int act = LACT_NONE, act2 = LACT_NONE, act_split = 0;   // columns < act_split: act, the others act2 (W2: act on the first product)
     float act_param = 1.f;                           // LACT_LOGSIG: the factor
@@ -234,6 +235,9 @@ struct LTileArgs {
 constexpr int LAY_TILE_WIDE_BLOCKS = 320;       // 128 x 128 tiles from this many blocks on (launch_lay_tile_gemm)
 bool lay_tile_gemm_fits(int N, int K, int groups);
 bool lay_tile_wide(const LTileArgs& a, bool beside);      // 128 x 128 tiles (else 64 x 64)
+enum LayTileShape { LTILE_64, LTILE_128, LTILE_192_128, LTILE_128_192, LTILE_256 };      // rows x columns of a block's tile
+LayTileShape lay_tile_shape(const LTileArgs& a, const LTileArgs& b);                     // b.M = 0: nothing beside
+bool lay_tile_tail(const LTileArgs& a, bool beside);      // the columns behind the last whole 128 in a launch of their own
 // beside: a second product of as many matrices, not grouped, its rows neither gathered nor scattered, in the same launch
 void launch_lay_tile_gemm(const LTileArgs& a, hipStream_t s, const LTileArgs* beside = nullptr);
 void launch_lay_round_scaled(const float* x, int ldx, const int32_t* idx, int div, const float* scale, uint16_t* out, int P, int K, hipStream_t s);

@@ -101,7 +101,7 @@ static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipSt
         lay_tile_gemm_fits(g.N, g.K, 1) && (g.M < 32 || (size_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * 32 >= (size_t)g.K)) {
         if (!g.A16) launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
         LTileArgs t;
-        t.A = g.A16 ? g.A16 : L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.N; t.K = g.K; t.bias = g.bias;
+        t.A = g.A16 ? g.A16 : L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.n_used ? g.n_used : g.N; t.K = g.K; t.bias = g.bias;
         t.act = g.act; t.act2 = g.act2; t.act_split = g.act_split; t.act_param = g.act_param;
         launch_lay_tile_gemm(t, s);
         return;
@@ -1273,6 +1273,7 @@ static void build_gizezen(Model& m, LaySource& src) {
         // whole tiles for the projection's kernels: rows of zeros behind the last one (their products are not read)
         const size_t rows = in.size() / W, unit = rows >= 1024 ? 128 : 8;
         w.in_rows = (int)((rows + unit - 1) / unit * unit);
+        w.in_used = (int)rows;
         in.resize((size_t)w.in_rows * W, 0.f);
         w.in_w = up_bf16(m, in);
         w.o_w = up_bf16(m, src.get(q + "o", W * H * e, 1.0f / std::sqrt((float)(H * e)), 0.f));
@@ -1949,12 +1950,12 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 // one row: the norms inside the launches of the products behind them, the router inside the experts' (x -> X2 -> x)
                 const bool one_row = T == 1 && L.tanh_norm && !L.f32 && L.fused_prep && lay_step_fits(W, sp);
                 LGemmArgs g;
-                g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.K = W;
+                g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.n_used = w.in_used; g.K = W;
                 g.act_split = w.g_off; g.act = sp.mixer == LMIX_HGRN ? LACT_SILU : LACT_NONE;
                 g.act2 = sp.mixer == LMIX_ATTN && sp.gate != LGATE_NONE ? LACT_SIGMOID : LACT_NONE;
                 if (one_row) {
                     launch_lay_step_in({L.X, padd.y, padd.wsel, w.norm1, w.norm1_off, L.X2, padd.nsum, L.mult, w.norm1_alpha},
-                                       {g.W, g.bias, g.C, g.N, g.act, g.act2, g.act_split, g.act_param}, W, s);
+                                       {g.W, g.bias, g.C, g.n_used ? g.n_used : g.N, g.act, g.act2, g.act_split, g.act_param}, W, s);
                     padd.y = nullptr; padd.wsel = nullptr;
                 } else {
                     add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc);

@@ -537,6 +537,10 @@ int cm_debug_lay_step_out_plan(int32_t heads, int32_t kv_heads, int32_t vdim, in
  * `experts` matrices of `columns` (experts 0: one matrix); `pair`: gate and up together; `beside`: the expert of every token in the same launch. */
 int cm_debug_lay_tile_plan(int32_t tokens, int32_t columns, int32_t experts, int32_t top, int32_t pair, int32_t beside);
 
+/* Test hook (host logic only, no GPU): rows * 1000 + columns of the tiles of such a product where its inner size is `inner` and the expert of every token beside it, if any,
+ * has `beside` columns (0: none); negative: the columns behind the last whole 128 are a launch of their own.  `function`: an activation behind a single matrix's product. */
+int cm_debug_lay_tile_shape(int32_t tokens, int32_t columns, int32_t inner, int32_t experts, int32_t top, int32_t pair, int32_t beside, int32_t function);
+
 /* Test hook (host logic only, no GPU): among how many blocks the prompt attention shares the keys of a query tile: `rows` queries behind `start` cached
  * tokens, `heads` query heads of 128 or 256. */
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim);
