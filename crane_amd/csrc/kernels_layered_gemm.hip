@@ -44,27 +44,30 @@ constexpr int K_TURN = 16;
 
 // a block's tile: sorted rows [p0, p0 + rows) of group g, column tile nt, of the launch's first product or (side) its second; false: a block behind
 // the last tile.  Every XCD takes a contiguous share of either product's tiles, numbered by group, then column tile, then row tile
-struct Tile { int g, p0, rows, nt; bool side; };
+struct Tile { int g, p0, rows, nt, shift; bool side; };      // shift: from a sorted row to its place among the indices
 template <int BM>
 __device__ __forceinline__ bool find_tile(const LTileArgs& a, const LTileArgs& b, int ntiles, int ntiles_b, int lane, Tile& t) {
-    int o0 = 0, o1 = a.M;
-    if (a.grp_off) {
-        o1 = 0;
-        if (lane < a.groups) { o0 = a.grp_off[lane]; o1 = a.grp_off[lane + 1]; }
-    }
-    const int mine = (o1 - o0 + BM - 1) / BM;
-    int incl = mine;
-    if (a.grp_off) {
+    int o0 = 0, n = a.M;
+    auto running = [&](int v) __attribute__((always_inline)) {
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) { const int v = __shfl_up(incl, d); if (lane >= d) incl += v; }
+        for (int d = 1; d < 64; d <<= 1) { const int u = __shfl_up(v, d); if (lane >= d) v += u; }
+        return v;
+    };
+    if (a.grp_off) {
+        n = 0;
+        if (a.bucket > 0) {
+            if (lane < a.groups) n = a.grp_off[lane * LAY_COUNT_STRIDE];
+            o0 = running(n) - n;
+        } else if (lane < a.groups) { o0 = a.grp_off[lane]; n = a.grp_off[lane + 1] - o0; }
     }
+    const int mine = (n + BM - 1) / BM, incl = a.grp_off ? running(mine) : mine;
     const int total = __builtin_amdgcn_readlane(incl, 63) * ntiles, share = (total + 7) >> 3;
     const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
     t.side = slot >= share;
     if (t.side) {
         const int mb = (b.M + BM - 1) / BM, total_b = mb * ntiles_b, share_b = (total_b + 7) >> 3, at = xcd * share_b + slot - share;
         if (slot - share >= share_b || at >= total_b) return false;
-        t.g = 0;
+        t.g = 0; t.shift = 0;
         t.nt = at / mb;
         t.p0 = (at - t.nt * mb) * BM;
         t.rows = min(BM, b.M - t.p0);
@@ -74,16 +77,17 @@ __device__ __forceinline__ bool find_tile(const LTileArgs& a, const LTileArgs& b
     if (at >= total) return false;
     t.g = a.grp_off ? __builtin_ctzll(__ballot(at < incl * ntiles)) : 0;
     const int m = __builtin_amdgcn_readlane(mine, t.g), local = at - (__builtin_amdgcn_readlane(incl, t.g) - m) * ntiles;
-    t.nt = local / m;
-    t.p0 = __builtin_amdgcn_readlane(o0, t.g) + (local - t.nt * m) * BM;
-    t.rows = min(BM, __builtin_amdgcn_readlane(o1, t.g) - t.p0);
+    const int first = __builtin_amdgcn_readlane(o0, t.g), row = (local - (t.nt = local / m) * m) * BM;
+    t.p0 = first + row;
+    t.rows = min(BM, __builtin_amdgcn_readlane(n, t.g) - row);
+    t.shift = a.bucket > 0 ? t.g * a.bucket - first : 0;
     return true;
 }
 
 // field by field: a choice between the two by reference puts them into scratch memory (6 us a launch)
 __device__ __forceinline__ void take(LTileArgs& a, const LTileArgs& b) {
     a.A = b.A; a.lda = b.lda; a.a_idx = nullptr; a.W = b.W; a.W2 = b.W2; a.w_stride = 0; a.C = b.C; a.ldc = b.ldc; a.c_idx = nullptr;
-    a.M = b.M; a.N = b.N; a.K = b.K; a.grp_off = nullptr; a.bias = b.bias; a.act = b.act; a.act2 = b.act2; a.act_split = b.act_split; a.act_param = b.act_param;
+    a.M = b.M; a.N = b.N; a.K = b.K; a.grp_off = nullptr; a.bucket = 0; a.bias = b.bias; a.act = b.act; a.act2 = b.act2; a.act_split = b.act_split; a.act_param = b.act_param;
 }
 
 // a wave's NI x NJ products to memory, rows mw .. and columns nw .. of the tile.  The weight is a product's first operand: a lane has columns 4 (lane / 16) + r of row
@@ -154,6 +158,8 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
     if (!find_tile<BM>(first, second, ntiles, ntiles_b, lane, at)) return;
     LTileArgs a = first;
     if (at.side) take(a, second);
+    if (a.a_idx) a.a_idx += at.shift;
+    if (a.c_idx) a.c_idx += at.shift;
     const int p0 = at.p0, rows = at.rows, nt = at.nt;
     const uint16_t* W = a.W + (size_t)at.g * a.w_stride;
     const uint16_t* W2 = DUAL ? a.W2 + (size_t)at.g * a.w_stride : nullptr;
@@ -241,6 +247,8 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
     if (!find_tile<BM>(first, second, ntiles, ntiles_b, lane, at)) return;
     LTileArgs a = first;
     if (at.side) take(a, second);
+    if (a.a_idx) a.a_idx += at.shift;
+    if (a.c_idx) a.c_idx += at.shift;
     const int p0 = at.p0, rows = at.rows;
     const uint16_t* W = a.W + (size_t)at.g * a.w_stride;
     const uint16_t* W2 = DUAL ? a.W2 + (size_t)at.g * a.w_stride : nullptr;
@@ -370,7 +378,7 @@ void go_tall(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
 
 // The last columns of one matrix, [n0, N), at most 64 of them: 16 rows per block, the k-tiles dealt to its eight waves, operands from memory straight into fragments.
 // What it saves: 32 gate columns behind 4096 others were a column tile of their own, 16 blocks behind the 512 that fill the chip (2048 rows, K 4096: 116 us in
-// the place of 76; here 76 + 14, four tiles requested together no less)
+// the place of 76; here 76 + 14; four tiles requested together 13, but 7 for 5 at K 1024)
 template <int NJ>
 __global__ __launch_bounds__(512) void lay_few_cols_kernel(LTileArgs a, int n0) {
     constexpr int NW = 8;
@@ -385,10 +393,9 @@ __global__ __launch_bounds__(512) void lay_few_cols_kernel(LTileArgs a, int n0) 
     for (int j = 0; j < NJ; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     // (a row's stride is a multiple of the memory channels' turn where K is a power of two: blocks start at different tiles, or all ask the same channels at once: 16 us)
     const int cnt = (a.K / BK - wave + NW - 1) / NW;
-    int at = cnt > 0 ? (int)blockIdx.x % cnt : 0;
-#pragma unroll 4
-    for (int i = 0; i < cnt; ++i, at = at + 1 < cnt ? at + 1 : 0) {
-        const int k = (at * NW + wave) * BK;
+    const int first = cnt > 0 ? (int)blockIdx.x % cnt : 0;
+    for (int i = 0; i < cnt; ++i) {
+        const int k = ((i + first < cnt ? i + first : i + first - cnt) * NW + wave) * BK;
         bf16x8 x[2], w[2][NJ];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {

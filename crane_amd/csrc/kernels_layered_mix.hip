@@ -10,6 +10,7 @@
 
 #include "dev_common.h"
 #include "layered.h"
+#include "layered_dev.h"
 
 namespace cm {
 
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(256) void lay_add_tanh_norm_kernel(float* __restric
     float* xr = x + (size_t)(rows ? rows[r] : r) * W + c;
     vec v = *(const vec*)xr;
     vec nw = 0.f, nb = 0.f;
-    if (out) { nw = *(const vec*)(w + c); nb = *(const vec*)(b + c); }
+    if (out || out16) { nw = *(const vec*)(w + c); nb = *(const vec*)(b + c); }
     if (y) {
         vec sum = 0.f;
 #pragma unroll 4
@@ -126,24 +127,238 @@ __global__ __launch_bounds__(256) void lay_add_tanh_norm_kernel(float* __restric
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[i] = fmaf(mult, sum[i], v[i]);
         *(vec*)xr = v;
-        if (!out) return;
+        if (!out && !out16) return;
     }
     vec o;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) o[i] = fmaf(tanhf(alpha * v[i]), nw[i], nb[i]);
-    *(vec*)(out + (size_t)r * W + c) = o;
+    if (out) *(vec*)(out + (size_t)r * W + c) = o;
     if (out16 == nullptr) return;
     if constexpr (VEC == 4) *(u32x2*)(out16 + (size_t)r * W + c) = (u32x2){pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
     else out16[(size_t)r * W + c] = f32_to_bf16(o[0]);
 }
 void launch_lay_add_tanh_norm(float* x, const int32_t* rows, const float* y, int nsum, const float* wsel, float mult, float alpha, const float* w,
                               const float* b, float* out, int n_rows, int W, hipStream_t s, uint16_t* out16) {
-    if (n_rows <= 0 || (!y && !out)) return;
+    if (n_rows <= 0 || (!y && !out && !out16)) return;
     // few rows (decode steps): narrow accesses, so that the row is spread over more threads
     const int vec = W % 4 == 0 && (n_rows > 32 || W > 8192) ? 4 : 1;
     const dim3 grid((unsigned)n_rows, (unsigned)((W / vec + 255) / 256));
     if (vec == 4) hipLaunchKernelGGL(lay_add_tanh_norm_kernel<4>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, out16, W);
     else hipLaunchKernelGGL(lay_add_tanh_norm_kernel<1>, grid, dim3(256), 0, s, x, rows, y, nsum, wsel, mult, alpha, w, b, out, out16, W);
+}
+
+// the new tail of channel c of a segment: the last taps - 1 entries of (old tail ++ the portion's inputs).  In place: entry k reads entry n + k > k of the old
+// tail, and a thread touches its own channel only
+__device__ __forceinline__ void conv_tail(const LConvArgs& a, const LaySegDev& sg, int c) {
+    float* tail = a.conv_pool + (size_t)sg.slot * a.slot_stride + a.cv_off;
+    for (int k = 0; k < a.taps - 1; ++k) {
+        const int idx = sg.n + k;
+        tail[(size_t)k * a.C + c] = idx < a.taps - 1 ? tail[(size_t)idx * a.C + c]
+                                                      : a.src[(size_t)(sg.row0 + idx - (a.taps - 1)) * a.lds + a.off + c];
+    }
+}
+
+// v[j] summed over the wave: lane l gets the sum of v[l % 16].  A pair of lanes exchanges half of what is left at every step (16 sums one by one are four
+// times the instructions)
+__device__ __forceinline__ float wave_sum16(float (&v)[16], int lane) {
+#define CM_HALVE(N, CTRL, BIT) \
+    _Pragma("unroll") for (int i = 0; i < N; ++i) { \
+        const float keep = (lane & BIT) ? v[i + N] : v[i], send = (lane & BIT) ? v[i] : v[i + N]; \
+        v[i] = keep + dpp_mov<CTRL>(send); \
+    }
+    CM_HALVE(8, 0x128, 8)      // row_ror 8: lane ^ 8
+    float s4[4];               // lane ^ 4 is no row operation: through the lanes
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float keep = (lane & 4) ? v[i + 4] : v[i], send = (lane & 4) ? v[i] : v[i + 4];
+        s4[i] = keep + __shfl_xor(send, 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = s4[i];
+    CM_HALVE(2, 0x4E, 2)       // quad_perm [2, 3, 0, 1]
+    CM_HALVE(1, 0xB1, 1)       // quad_perm [1, 0, 3, 2]
+#undef CM_HALVE
+    float r = v[0];
+    r += __shfl_xor(r, 16);
+    r += __shfl_xor(r, 32);
+    return r;
+}
+__device__ __forceinline__ void late_tail(const LNormRouter& a, int i) {
+    const int per = (a.tail.C + (int)blockDim.x - 1) / (int)blockDim.x, sn = i / per, c = (i - sn * per) * (int)blockDim.x + (int)threadIdx.x;
+    if (c < a.tail.C) conv_tail(a.tail, a.tail.segs[sn], c);
+}
+
+// Update, norm, router, choice and the experts' lists of a row per block: the row is in registers where the router's products want it, a choice joins its expert's rows
+// by one atomic addition, and the tails of the layer's convolution, which wait for every reader of the old ones, ride along.  NE >= logits, a multiple of 16.
+// What bounds it: the chain of first loads, products, sums over lanes, choice and addition.  326 rows of 1024, 15 logits: 8.1 us where norm,
+// router, plan and tails took 4.7, 12.0, 3.4 and 3.2 and the gaps between four launches
+template <int NE>
+__global__ __launch_bounds__(256) void lay_norm_router_kernel(LNormRouter a, int per_tok) {
+    extern __shared__ float zs[];              // [per_tok + top] of the choice, then [4 waves][NE]
+    if ((int)blockIdx.x >= a.T) { late_tail(a, (int)blockIdx.x - a.T); return; }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x, n = a.E + (a.rs.shared_gate ? 1 : 0), W = a.W;
+    float acc[NE];
+#pragma unroll
+    for (int ex = 0; ex < NE; ++ex) acc[ex] = 0.f;
+    for (int i = (int)threadIdx.x * 4; i < W; i += 1024) {
+        const size_t at = (size_t)t * W + i;
+        f32x4 v = *(const f32x4*)(a.x + at);
+        const f32x4 y = *(const f32x4*)(a.y + at), nw = *(const f32x4*)(a.w + i), nb = *(const f32x4*)(a.b + i);
+        u32x2 w[NE];
+#pragma unroll
+        for (int ex = 0; ex < NE; ++ex) w[ex] = *(const u32x2*)(a.wr + (size_t)min(ex, n - 1) * W + i);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = fmaf(a.mult, y[c], v[c]);
+        *(f32x4*)(a.x + at) = v;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = fmaf(tanhf(a.alpha * v[c]), nw[c], nb[c]);
+        *(u32x2*)(a.out16 + at) = (u32x2){pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+#pragma unroll
+        for (int ex = 0; ex < NE; ++ex)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                acc[ex] = fmaf(v[2 * c], bf16_lo(w[ex][c]), acc[ex]);
+                acc[ex] = fmaf(v[2 * c + 1], bf16_hi(w[ex][c]), acc[ex]);
+            }
+    }
+    float* part = zs + per_tok + a.top;
+#pragma unroll
+    for (int g = 0; g < NE / 16; ++g) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = acc[g * 16 + j];
+        const float s = wave_sum16(v, lane);
+        if (lane < 16) part[wave * NE + g * 16 + lane] = s;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane < n) zs[lane] = (part[lane] + part[NE + lane]) + (part[2 * NE + lane] + part[3 * NE + lane]);
+    __builtin_amdgcn_wave_barrier();
+    int32_t* chosen = (int32_t*)(zs + per_tok);
+    lay_router_choose(zs, 0, lane, chosen, a.wsel + (size_t)t * a.slots, a.E, a.top, a.rs, nullptr, a.slots);
+    __builtin_amdgcn_wave_barrier();
+    for (int j = lane; j < a.top; j += 64) {
+        const int e = chosen[j];
+        a.srt[(size_t)e * a.bucket + atomicAdd(&a.cnt[e * LAY_COUNT_STRIDE], 1)] = t * a.slots + j;
+    }
+}
+
+// The same of eight rows per block, for prompts: reading the router's matrix once per row out of the L2 would take longer than the rows.  Eight waves share the
+// row's 64-element pieces; a lane has eight elements of one row, as the operand of a matrix instruction wants them, in three bfloat16 parts (24 bits: the row is
+// not rounded).  Columns 0 .. 7 of that operand are the rows' first 32 elements, 8 .. 15 their last: a product for either half, of which half the columns count, so that all
+// lanes have elements of their own and 2048 rows are 256 blocks.  Bound: memory and tanhf.  2048 rows of
+// 4096, 17 logits: 36.5 us (sixteen rows per block 52; the single launches 33.1, 25.6, 7.4, 4.6), 1892 of 1024 15.5 (18.6; 10.1, 12.3, 5.0, 3.2)
+template <int NG>
+__global__ __launch_bounds__(512) void lay_norm_router_tile_kernel(LNormRouter a, int row_blocks, int per_tok) {
+    extern __shared__ float zs[];              // [8 waves][per_tok] of a choice, [8 waves][NG][16 columns][17] logits, [8][top] choices
+    __shared__ int32_t rows_of[32], base_of[32];           // of an expert in this block; their place among all
+    if ((int)blockIdx.x >= row_blocks) { late_tail(a, (int)blockIdx.x - row_blocks); return; }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, lg = lane >> 4, t0 = (int)blockIdx.x * 8;
+    const int n = a.E + (a.rs.shared_gate ? 1 : 0), W = a.W, t = min(t0 + (fr & 7), a.T - 1), i0 = wave * 64 + lg * 8, half = fr >= 8 ? 32 : 0;
+    const bool own = t0 + (fr & 7) < a.T;
+    f32x4 acc[2][NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) acc[0][g] = acc[1][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    struct Piece { f32x4 x[2], y[2], nw[2], nb[2]; bf16x8 w[2][NG]; };
+    auto load = [&](int i) __attribute__((always_inline)) {
+        Piece p;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = i + half + 4 * h;
+            p.x[h] = *(const f32x4*)(a.x + (size_t)t * W + c); p.y[h] = *(const f32x4*)(a.y + (size_t)t * W + c);
+            p.nw[h] = *(const f32x4*)(a.w + c); p.nb[h] = *(const f32x4*)(a.b + c);
+        }
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const uint16_t* wr = a.wr + (size_t)min(g * 16 + fr, n - 1) * W + i;
+            p.w[0][g] = *(const bf16x8*)wr; p.w[1][g] = *(const bf16x8*)(wr + 32);
+        }
+        return p;
+    };
+    const int pieces = (W - wave * 64 + 511) / 512;        // (W is a multiple of 64)
+    Piece next;
+    if (pieces > 0) next = load(i0);
+    for (int k0 = 0; k0 < pieces; ++k0) {
+        Piece p = next;
+        const int i = i0 + k0 * 512;
+        next = load(k0 + 1 < pieces ? i + 512 : i);        // requested in front of this piece's work
+        const size_t at = (size_t)t * W + i + half;
+        f32x4 (&x)[2] = p.x; f32x4 (&y)[2] = p.y; f32x4 (&nw)[2] = p.nw; f32x4 (&nb)[2] = p.nb;
+        u32x4 part[3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[h][c] = fmaf(a.mult, y[h][c], x[h][c]);
+            if (own) *(f32x4*)(a.x + at + 4 * h) = x[h];
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = fmaf(tanhf(a.alpha * x[h][c]), nw[h][c], nb[h][c]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const uint32_t pk = pack_bf16x2(v[2 * c], v[2 * c + 1]);
+                    part[k][2 * h + c] = pk;
+                    v[2 * c] -= bf16_lo(pk); v[2 * c + 1] -= bf16_hi(pk);
+                }
+        }
+        if (own) *(u32x4*)(a.out16 + at) = part[0];
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+#pragma unroll
+            for (int g = 0; g < NG; ++g)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) acc[h][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p.w[h][g], __builtin_bit_cast(bf16x8, part[k]), acc[h][g], 0, 0, 0);
+    }
+    float* sums = zs + 8 * per_tok;                        // of a wave: column fr's share of logits 16 g + 4 lg + r
+    int32_t* chosen = (int32_t*)(sums + 8 * NG * 16 * 17);
+    if (threadIdx.x < 32) rows_of[threadIdx.x] = 0;
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[((wave * NG + g) * 16 + fr) * 17 + lg * 4 + r] = fr < 8 ? acc[0][g][r] : acc[1][g][r];
+    __syncthreads();
+    float* mine = zs + wave * per_tok;
+    const int rows = min(8, a.T - t0), row = wave;
+    if (row < rows) {
+        if (lane < n) {
+            float z = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float* at = sums + ((k * NG + (lane >> 4)) * 16 + row) * 17 + (lane & 15);
+                z += at[0] + at[8 * 17];
+            }
+            mine[lane] = z;
+        }
+        __builtin_amdgcn_wave_barrier();
+        lay_router_choose(mine, 0, lane, chosen + row * a.top, a.wsel + (size_t)(t0 + row) * a.slots, a.E, a.top, a.rs, nullptr, a.slots);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    const int i = (int)threadIdx.x, e = i < rows * a.top ? chosen[i] : -1;       // (at most 32 choices of a row)
+    const int at = e >= 0 ? atomicAdd(&rows_of[e], 1) : 0;
+    __syncthreads();
+    if (i < a.E && rows_of[i] > 0) base_of[i] = atomicAdd(&a.cnt[i * LAY_COUNT_STRIDE], rows_of[i]);
+    __syncthreads();
+    if (e >= 0) a.srt[(size_t)e * a.bucket + base_of[e] + at] = (t0 + i / a.top) * a.slots + i % a.top;
+}
+// choices of up to 32 logits, rows of whole 64-element pieces (the addresses are the scratch's and the weights', 16-byte aligned)
+bool lay_norm_router_fits(int W, int E, const RouterSpec& rs) {
+    return W % 64 == 0 && E + (rs.shared_gate ? 1 : 0) <= 32 && rs.identity == 0 && !rs.correction;
+}
+void launch_lay_norm_router(const LNormRouter& a, hipStream_t s) {
+    if (a.T <= 0) return;
+    const int logits = a.E + (a.rs.shared_gate ? 1 : 0), per_tok = logits + a.E + a.rs.groups + a.top;
+    const bool tile = a.T >= 1024;
+    const int threads = tile ? 512 : 256, row_blocks = tile ? (a.T + 7) / 8 : a.T;
+    const int tails = a.tail_segs > 0 && a.tail.taps > 1 ? a.tail_segs * ((a.tail.C + threads - 1) / threads) : 0;
+    const dim3 grid((unsigned)(row_blocks + tails));
+    const size_t own = (size_t)(per_tok + a.top) * sizeof(float), lds = (size_t)(8 * per_tok + 8 * a.top) * sizeof(float);
+    if (tile) {
+        if (logits <= 16) hipLaunchKernelGGL(lay_norm_router_tile_kernel<1>, grid, dim3(threads), lds + 8 * 16 * 17 * sizeof(float), s, a, row_blocks, per_tok);
+        else hipLaunchKernelGGL(lay_norm_router_tile_kernel<2>, grid, dim3(threads), lds + 16 * 16 * 17 * sizeof(float), s, a, row_blocks, per_tok);
+    } else if (logits <= 16) hipLaunchKernelGGL(lay_norm_router_kernel<16>, grid, dim3(threads), own + 4 * 16 * sizeof(float), s, a, per_tok);
+    else hipLaunchKernelGGL(lay_norm_router_kernel<32>, grid, dim3(threads), own + 4 * 32 * sizeof(float), s, a, per_tok);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -419,18 +634,9 @@ void launch_lay_conv_act(const LConvArgs& a, int T, hipStream_t s) {
     if (T <= 0) return;
     hipLaunchKernelGGL(lay_conv_act_kernel, dim3((unsigned)T, (unsigned)((a.C + a.H + 255) / 256)), dim3(256), 0, s, a);
 }
-// new tail = last taps - 1 entries of (old tail ++ the portion's inputs).  In place: entry k reads entry n + k > k of the old tail, and a
-// thread touches its own channel only.
 __global__ __launch_bounds__(256) void lay_conv_tail_kernel(LConvArgs a) {
-    const LaySegDev sg = a.segs[blockIdx.x];
     const int c = blockIdx.y * 256 + threadIdx.x;
-    if (c >= a.C) return;
-    float* tail = a.conv_pool + (size_t)sg.slot * a.slot_stride + a.cv_off;
-    for (int k = 0; k < a.taps - 1; ++k) {
-        const int idx = sg.n + k;
-        tail[(size_t)k * a.C + c] = idx < a.taps - 1 ? tail[(size_t)idx * a.C + c]
-                                                      : a.src[(size_t)(sg.row0 + idx - (a.taps - 1)) * a.lds + a.off + c];
-    }
+    if (c < a.C) conv_tail(a, a.segs[blockIdx.x], c);
 }
 void launch_lay_conv_tail(const LConvArgs& a, int nseg, hipStream_t s) {
     if (nseg <= 0 || a.taps <= 1) return;

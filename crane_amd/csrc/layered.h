@@ -221,6 +221,8 @@ void launch_lgemm(const LGemmArgs& a, bool bf16, int groups, hipStream_t s);
 // products over bfloat16 rows on matrix-core tiles (kernels_layered_gemm.hip).  W2 given: C (bfloat16) = act(A W^T) * (A W2^T); else C (f32) =
 // A W^T + bias, columns below act_split through act, the others through act2.  grp_off: rows [grp_off[g], grp_off[g + 1]) use matrix g; `total` rows in all groups, at most M in one.  A row of output row p:
 // a_idx ? a_idx[p] / a_div : p; output row: c_idx ? c_idx[p] : p.  K a multiple of 64, at most 64 groups; A, W, W2 and their rows 16-byte aligned
+// counters a cache line apart: additions to one line wait for each other, 12 ns each (1304 of 326 rows to 14 counters: 5.3 us on one line, 2.6 on one each; 8192 25 and 8)
+constexpr int LAY_COUNT_STRIDE = 32;
 struct LTileArgs {
     const uint16_t* A = nullptr; int lda = 0;
     const int32_t* a_idx = nullptr; int a_div = 1;
@@ -229,6 +231,7 @@ struct LTileArgs {
     const int32_t* c_idx = nullptr;
     int M = 0, N = 0, K = 0;
     const int32_t* grp_off = nullptr; int groups = 1, total = 0;
+    int bucket = 0;                                  // > 0: grp_off[g * LAY_COUNT_STRIDE] is group g's row count, its indices start at g * bucket
     const float* bias = nullptr;
     int act = LACT_NONE, act2 = LACT_NONE, act_split = 0; float act_param = 1.f;
 };
@@ -495,6 +498,16 @@ void launch_lay_router(const float* h, const uint16_t* wr, int32_t* sel, float* 
                        const RouterSpec* rs = nullptr, const float* correction = nullptr, int slots = 0, float* zbuf = nullptr);
 // counting sort of the T top (token, choice) pairs by expert: off [E + 1], srt [T top] = token * slots + choice
 void launch_lay_moe_plan(const int32_t* sel, int32_t* off, int32_t* srt, int n, int E, hipStream_t s, int top = 1, int slots = 1);
+// residual update, tanh norm, router, choice and every expert's rows in one launch (kernels_layered_mix.hip): x += mult y, out16 = norm(x) in bfloat16, weights of
+// a token's choices in wsel [T][slots], srt[e bucket + i] = t slots + k for choice k of token t, cnt[e LAY_COUNT_STRIDE] of them (in any order; zero before).  tail_segs: the
+// convolution tails of that many segments beside it
+struct LNormRouter {
+    float* x; const float* y; float mult, alpha; const float *w, *b; uint16_t* out16;
+    const uint16_t* wr; float* wsel; int32_t *cnt, *srt; int bucket, T, W, E, top, slots; RouterSpec rs;
+    LConvArgs tail; int tail_segs = 0;
+};
+bool lay_norm_router_fits(int W, int E, const RouterSpec& rs);
+void launch_lay_norm_router(const LNormRouter& a, hipStream_t s);
 
 // matrix memory, gates: per (sequence, head) over the portion's tokens, from the pre-activations zi, zf at proj[t ldp + i_off / f_off + head]
 //   li = cap tanh(zi / cap), lf = ln sigmoid(cap tanh(zf / cap)), m' = max(lf + m, li)  (m: per-sequence state at mstate, [H])

@@ -90,15 +90,19 @@ struct Layered {
 
 void LayeredDeleter::operator()(Layered* p) const { delete p; }
 
+// one matrix of N x K over M rows runs on the tile kernel.  Below 32 rows the alternative is the plain kernel (24 rows, four layers: 840 -> 632 us at width 1024, 2747 -> 1890 at
+// 4096); from there on the shared GEMM, whose split sums win while the tiles are few for the depth: 64 rows 644 against 663 us (26 and 16 tiles, K 1024) and 1884
+// against 1955 (98 and 64 tiles, K 4096), but 128 rows 704 / 689 (52 and 32) and 2016 / 2022 (196 and 128), 700 rows 921 / 878, 2947 / 2916
+static bool lay_on_tiles(const Layered& L, int M, int N, int K) {
+    return !L.f32 && L.shared_gemm && L.Abf && M > LAY_ROW_KERNEL_ROWS && lay_tile_gemm_fits(N, K, 1) &&
+           (M < 32 || (size_t)((M + 63) / 64) * ((N + 63) / 64) * 32 >= (size_t)K);
+}
+
 // one projection of a pass: the shared matrix-core GEMM where it applies, else the kernels of kernels_layered.hip
 static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipStream_t s) {
     const bool bf = !L.f32;
-    // the tile kernel with bias and activation in its epilogue, instead of (split sums, their reduction,) a product and an activation sweep.  Below
-    // 32 rows the alternative is the plain kernel (24 rows, four layers: 840 -> 632 us at width 1024, 2747 -> 1890 at 4096); from there on the
-    // shared GEMM, whose split sums win while the tiles are few for the depth: 64 rows 644 against 663 us (26 and 16 tiles, K 1024) and 1884
-    // against 1955 (98 and 64 tiles, K 4096), but 128 rows 704 / 689 (52 and 32) and 2016 / 2022 (196 and 128), 700 rows 921 / 878, 2947 / 2916
-    if (bf && L.shared_gemm && L.Abf && groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && !g.W2 && g.M > LAY_ROW_KERNEL_ROWS &&
-        lay_tile_gemm_fits(g.N, g.K, 1) && (g.M < 32 || (size_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * 32 >= (size_t)g.K)) {
+    // the tile kernel with bias and activation in its epilogue, instead of (split sums, their reduction,) a product and an activation sweep
+    if (groups == 1 && !g.a_idx && !g.c_idx && !g.grp_off && !g.mul && !g.W2 && lay_on_tiles(L, g.M, g.N, g.K)) {
         if (!g.A16) launch_lay_round_rows(g.A, g.lda, L.Abf, g.M, g.K, s);
         LTileArgs t;
         t.A = g.A16 ? g.A16 : L.Abf; t.lda = g.K; t.W = g.W; t.C = g.C; t.ldc = g.ldc; t.M = g.M; t.N = g.n_used ? g.n_used : g.N; t.K = g.K; t.bias = g.bias;
@@ -139,8 +143,13 @@ static void lay_gemm(Model& m, Layered& L, const LGemmArgs& g, int groups, hipSt
 // the experts of a pass over `T` rows of h (choices sorted by expert in L.srt / L.off, weights in L.wsel): their outputs, and those of the expert
 // that every token uses, into L.YS [token][slots][W].  bfloat16 format, more rows than the row kernel takes, sizes of whole k-tiles: the rows are
 // rounded once (h16: they are already) and everything runs on the tile kernel, the inner rows bfloat16 as the second product reads them
+// cnt: the choices are counted there and listed in buckets of T rows (lay_norm_router_kernel)
+static bool lay_experts_on_tiles(const Layered& L, const LayerSpec& sp, int T, int W) {
+    return !L.f32 && L.shared_gemm && L.Abf && T > LAY_ROW_KERNEL_ROWS && (!sp.scale_input || L.Asc) && lay_tile_gemm_fits(sp.ff, W, sp.experts) &&
+           lay_tile_gemm_fits(W, sp.ff, sp.experts);
+}
 static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const LayeredLayerW& w, const float* h, int T, int W, int slots, hipStream_t s,
-                        const uint16_t* h16 = nullptr) {
+                        const uint16_t* h16 = nullptr, const int32_t* cnt = nullptr) {
     LGemmArgs gu;
     gu.A = h; gu.lda = W; gu.a_idx = L.srt; gu.a_div = slots; gu.a_scale = sp.scale_input ? L.wsel : nullptr;
     gu.W = w.gate; gu.W2 = w.up; gu.w_stride = (size_t)sp.ff * W;
@@ -162,10 +171,10 @@ static void lay_experts(Model& m, Layered& L, const LayerSpec& sp, const Layered
         t.A = A; t.lda = g.K; t.W = g.W; t.W2 = g.W2; t.w_stride = g.w_stride; t.C = g.C; t.ldc = g.ldc; t.c_idx = g.c_idx;
         t.M = g.M; t.N = g.N; t.K = g.K; t.act = g.act; t.act_param = g.act_param;
         if (gather) { t.a_idx = g.a_idx; t.a_div = g.a_div; }
-        if (g.grp_off) { t.grp_off = g.grp_off; t.groups = sp.experts; t.total = T * sp.top; }
+        if (g.grp_off) { t.grp_off = cnt ? cnt : g.grp_off; t.bucket = cnt ? T : 0; t.groups = sp.experts; t.total = T * sp.top; }
         return t;
     };
-    const bool routed = tiles && lay_tile_gemm_fits(sp.ff, W, sp.experts) && lay_tile_gemm_fits(W, sp.ff, sp.experts);
+    const bool routed = lay_experts_on_tiles(L, sp, T, W);
     const bool shared = tiles && every && lay_tile_gemm_fits(sp.shared_ff, W, 1) && lay_tile_gemm_fits(W, sp.shared_ff, 1);
     if (!h16 && ((routed && !sp.scale_input) || shared)) launch_lay_round_rows(h, W, L.Abf, T, W, s);
     const uint16_t* A = h16 ? h16 : L.Abf;
@@ -1478,7 +1487,7 @@ void Model::alloc_runtime_layered() {
         if (L.tanh_norm) L.X2 = dalloc<float>((size_t)W);
         L.wsel = dalloc<float>(cap * (size_t)L.max_slots);
         L.sel = dalloc<int32_t>(cap * (size_t)L.max_top);
-        L.srt = dalloc<int32_t>(cap * (size_t)L.max_top);
+        L.srt = dalloc<int32_t>(cap * (size_t)std::max(L.max_top, std::min(L.max_E, 64)));      // sorted choices, or a bucket of a pass per expert
         L.off = dalloc<int32_t>((size_t)L.max_E + 1);
         L.Z = dalloc<float>(cap * (size_t)L.max_E);
     }
@@ -1529,7 +1538,7 @@ void Model::alloc_runtime_layered() {
     for (int nrep : L.nreps) tiles += 2 * (cap * (size_t)nrep / 16 + (size_t)MAXB + 1) + 2 * (cap * (size_t)nrep / LAY_ATTN_MFMA_ROWS + (size_t)MAXB + 1);
     tiles += 2 * (cap / LAY_LIGHT_CHUNK + (size_t)MAXB + 1);      // lightning chunks
     tiles += 2 * ((size_t)L.ds_chunks + 1);                       // delta-rule chunks
-    L.tab_ints = 3 * cap + (size_t)MAXB * (sizeof(LaySegDev) / 4) + (size_t)MAXB * max_pages_per_seq + tiles + 64;
+    L.tab_ints = 3 * cap + (size_t)MAXB * (sizeof(LaySegDev) / 4) + (size_t)MAXB * max_pages_per_seq + tiles + L.spec.size() * (size_t)std::min(L.max_E, 32) * LAY_COUNT_STRIDE + 64;
     L.d_tab = dalloc<int32_t>(L.tab_ints);
     CM_HIP(hipHostMalloc((void**)&L.h_tab, L.tab_ints * sizeof(int32_t)));
     CM_HIP(hipStreamSynchronize(stream));
@@ -1690,6 +1699,9 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             for (int k = 0; k < nseg; ++k)
                 if (t_segs[k].n > LAY_DELTA_SEQ)
                     for (int t0 = 0; t0 < t_segs[k].n; t0 += LAY_DELTA_CHUNK) { tab[o++] = k; tab[o++] = t0; }
+        const bool rows_listed = L.tanh_norm && !L.f32 && L.shared_gemm && T > LAY_ROW_KERNEL_ROWS;
+        const size_t o_cnt = o, n_cnt = (size_t)std::min(L.max_E, 32) * LAY_COUNT_STRIDE;       // every layer's rows per expert, counted in place
+        if (rows_listed) { memset(tab + o, 0, L.spec.size() * n_cnt * sizeof(int32_t)); o += L.spec.size() * n_cnt; }
         if (o > L.tab_ints) throw CmError(CM_ERR_INVALID, "step tables overflow");
         CM_HIP(hipMemcpyAsync(L.d_tab, tab, o * sizeof(int32_t), hipMemcpyHostToDevice, s));
         const uint32_t* d_ids = (const uint32_t*)(L.d_tab + o_ids);
@@ -1872,9 +1884,9 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         };
         // pre-norm layers: the finished sublayer's rows (nsum per token, summed in order) join the residual inside the next norm's launch
         struct { const float* y = nullptr; int nsum = 1; const float* wsel = nullptr; } padd;
-        auto add_norm = [&](const float* nw_, const float* off, float alpha, float* out) {
+        auto add_norm = [&](const float* nw_, const float* off, float alpha, float* out, bool only16 = false) {       // only16: the reader takes the bfloat16 rows
             n16 = L.tanh_norm && out ? rounded : nullptr;
-            if (L.tanh_norm) launch_lay_add_tanh_norm(L.X, nullptr, padd.y, padd.nsum, padd.wsel, L.mult, alpha, nw_, off, out, T, W, s, out ? rounded : nullptr);
+            if (L.tanh_norm) launch_lay_add_tanh_norm(L.X, nullptr, padd.y, padd.nsum, padd.wsel, L.mult, alpha, nw_, off, only16 && n16 ? nullptr : out, T, W, s, out ? rounded : nullptr);
             else launch_lay_add_gnorm(L.X, nullptr, padd.y, padd.nsum, nw_, out, T, W, L.norm_groups, cfg.eps, s, padd.wsel);
             padd.y = nullptr; padd.wsel = nullptr;
         };
@@ -1949,6 +1961,12 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 // ---- x += mult mixer(norm1 x), x += mult ff(norm2 x); norms in equal parts, or of single elements
                 // one row: the norms inside the launches of the products behind them, the router inside the experts' (x -> X2 -> x)
                 const bool one_row = T == 1 && L.tanh_norm && !L.f32 && L.fused_prep && lay_step_fits(W, sp);
+                // the norm in front of the experts, their router and lists and this layer's convolution tails in one launch
+                const bool joined = L.tanh_norm && rounded && sp.mlp == LMLP_MOE && !sp.scale_input && lay_norm_router_fits(W, sp.experts, sp.router) &&
+                                    lay_experts_on_tiles(L, sp, T, W) &&
+                                    (sp.shared_ff == 0 || (lay_tile_gemm_fits(sp.shared_ff, W, 1) && lay_tile_gemm_fits(W, sp.shared_ff, 1)));
+                LConvArgs late_tail{};
+                int late_segs = 0;
                 LGemmArgs g;
                 g.W = w.in_w; g.bias = w.in_b; g.C = L.P; g.ldc = w.in_rows; g.M = T; g.N = w.in_rows; g.n_used = w.in_used; g.K = W;
                 g.act_split = w.g_off; g.act = sp.mixer == LMIX_HGRN ? LACT_SILU : LACT_NONE;
@@ -1958,7 +1976,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                                        {g.W, g.bias, g.C, g.n_used ? g.n_used : g.N, g.act, g.act2, g.act_split, g.act_param}, W, s);
                     padd.y = nullptr; padd.wsel = nullptr;
                 } else {
-                    add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc);
+                    add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc, lay_on_tiles(L, T, g.N, W));
                     g.A = L.Hc; g.A16 = n16; g.lda = W;
                     lay_gemm(*this, L, g, 1, s);
                 }
@@ -1977,11 +1995,12 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     c.bt = d_bt; c.segs = d_segs; c.rowseg = d_rowseg; c.page = page; c.T = T; c.tail_too = all_decode;
                     launch_lay_conv_qkv(c, kv_mode, s);
                     if (!all_decode && sp.conv > 1) {
-                        LConvArgs t;
+                        LConvArgs& t = late_tail;
                         t.src = L.P; t.lds = w.in_rows; t.off = w.q_off; t.C = w.g_off; t.dst = nullptr; t.ldd = 0; t.cw = nullptr; t.cb = nullptr;
                         t.taps = sp.conv; t.act = LACT_NONE; t.conv_pool = conv_pool; t.slot_stride = conv_slot_elems; t.cv_off = w.cv_off;
                         t.segs = d_segs; t.rowseg = d_rowseg;
-                        launch_lay_conv_tail(t, nseg, s);
+                        if (!joined) launch_lay_conv_tail(t, nseg, s);
+                        else late_segs = nseg;
                     }
                     keep_shares = one_row;
                     left.nsplit = 1;
@@ -2107,12 +2126,21 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     launch_lay_step_moe({L.X2, padd.y, nullptr, w.norm2, w.norm2_off, L.X, 1, L.mult, w.norm2_alpha}, m, L.YS, W, s);
                     padd.y = L.YS; padd.nsum = slots; padd.wsel = L.wsel;
                 } else if (sp.mlp == LMLP_MOE) {
-                    add_norm(w.norm2, w.norm2_off, w.norm2_alpha, L.Hc);
+                    const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
+                    int32_t* cnt = nullptr;
+                    if (joined) {
+                        cnt = L.d_tab + o_cnt + li * n_cnt;
+                        launch_lay_norm_router({L.X, padd.y, L.mult, w.norm2_alpha, w.norm2, w.norm2_off, rounded, w.router, L.wsel, cnt, L.srt, T, T, W, sp.experts,
+                                                sp.top, slots, sp.router, late_tail, late_segs}, s);
+                        n16 = rounded;
+                        padd.y = nullptr;
+                    } else {
+                        add_norm(w.norm2, w.norm2_off, w.norm2_alpha, L.Hc);
+                        route(L.Hc, w.router, sp.experts, sp.top, sp.router, nullptr, slots);
+                    }
                     // scale_input: an expert's weight multiplies its INPUT, the rows of the grouped product are w h and the combine is a plain
                     // sum; otherwise the weights join in the combine
-                    const int slots = sp.top + (sp.shared_ff > 0 ? 1 : 0);
-                    route(L.Hc, w.router, sp.experts, sp.top, sp.router, nullptr, slots);
-                    lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s, n16);
+                    lay_experts(*this, L, sp, w, L.Hc, T, W, slots, s, n16, cnt);
                     padd.y = L.YS; padd.nsum = slots; padd.wsel = sp.scale_input ? nullptr : L.wsel;
                 }
                 if (L.capture || li + 1 == L.spec.size()) add_norm(nullptr, nullptr, 0.f, nullptr);
