@@ -219,10 +219,11 @@ __device__ __forceinline__ void values(const uint16_t* Vb, int lr, int lg, const
             for (int k = 0; k < PARTS; ++k) o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p[k][h], o[n], 0, 0, 0);
         }
 }
-// four output elements c .. c + 3 of a query: v times inv times the gate
-__device__ __forceinline__ void put4(const LAttnArgs& a, int row, int head, int c, const f32x4& o, float l, bool ovec) {
-    const float* gp = a.gbuf + (size_t)row * a.ldg + (a.gate == LGATE_ELEM ? head * a.e : head);
-    const float inv = (a.gate == LGATE_HEAD ? gp[0] : 1.f) / l * a.out_scale;
+__device__ __forceinline__ const float* gate_of(const LAttnArgs& a, int row, int head) { return a.gbuf + (size_t)row * a.ldg + (a.gate == LGATE_ELEM ? head * a.e : head); }
+// four output elements c .. c + 3 of a query: v times inv times the gate; head_gate: the gate of the whole head (LGATE_HEAD)
+__device__ __forceinline__ void put4(const LAttnArgs& a, int row, int head, int c, const f32x4& o, float l, bool ovec, float head_gate) {
+    const float* gp = gate_of(a, row, head);
+    const float inv = (a.gate == LGATE_HEAD ? head_gate : 1.f) / l * a.out_scale;
     float* out = a.out + (size_t)row * a.ldo + head * a.e + c;
     f32x4 v;
 #pragma unroll
@@ -255,13 +256,17 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     uint16_t* const Vs = Ks + 2 * KT * KLD;                       // [2][64][VLD]
     const int g = blockIdx.x;
     const int2 tile_id = a.tiles[blockIdx.y];
-    const LaySegDev sg = a.segs[tile_id.x];
+    const LaySegDev sg = a.segs[KS == 2 ? tile_id.x & 0xffff : tile_id.x];
+    const int share = KS == 2 ? (tile_id.x >> 16) & 255 : 0, shares = KS == 2 ? max(1, tile_id.x >> 24) : 1;
     const int nrep = a.H / a.G, d = a.d, e = a.e;
     const int q0 = tile_id.y, nq = min(64, sg.n * nrep - q0);
     Walk w;
     w.init<POOL>(a, sg, q0, nq, nrep);
+    // this block's key tiles [t0, t1)
+    const int per = (w.ntile + shares - 1) / shares, t0 = share * per, t1 = min(w.ntile, t0 + per), t_last = min(max(t0, t1 - 1), w.ntile - 1);      // (a share may be empty)
     Query<2> q;
-    q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk, lg, grp == 0);
+    q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk, lg, grp == 0 && share == 0);
+    const float head_gate = a.gate == LGATE_HEAD ? *gate_of(a, q.row, q.head) : 1.f;       // (here, not behind the walk: a trip to memory less)
     bf16x8 qf[NKS];                                    // rounded once
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -279,7 +284,8 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
         const int j = min(w.first(min(grp64 * 64 + lane, w.ntile - 1)), w.pmax);
         return a.bt[sg.bt_off + j / a.page];
     };
-    int pgs = load_pages(0);
+    pgs_grp = t0 >> 6;
+    int pgs = load_pages(pgs_grp);
     struct Rows { u32x4 k[KPT], v[VPT]; };
     const int Gv = a.v_div > 1 ? a.G / a.v_div : a.G, gv = a.v_div > 1 ? g / a.v_div : g, ldv = a.vpool ? e : d;
     // this thread's rows and 16-byte column of a tile.  Columns of the padding hold column 0 (their queries' are zero): no load under a branch
@@ -287,7 +293,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     const int kr0 = tid / KC, vr0 = tid / VC;
     const int kc = (tid % KC) * 8 < d ? (tid % KC) * 8 : 0, vc = (tid % VC) * 8 < e ? (tid % VC) * 8 : 0;
     auto fetch = [&](int t_, Rows& rg) __attribute__((always_inline)) {
-        const int t = min(t_, w.ntile - 1);            // past the end: the last tile again, parked into a buffer nobody reads
+        const int t = min(t_, t_last);                 // past the end: the last tile again, parked into a buffer nobody reads
         const int j0 = w.first(t);
         if ((t >> 6) != pgs_grp) { pgs_grp = t >> 6; pgs = load_pages(pgs_grp); }      // (uniform)
         if (POOL && t < w.front) {
@@ -320,9 +326,9 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
     // step i: tile KS i + grp of this group; the rows of step i + 2 are requested at its top, those of step i + 1 parked at its bottom
     auto step = [&](int i, Rows& rg_new, const Rows& rg_next) __attribute__((always_inline)) {
-        const int t = KS * i + grp;
+        const int t = t0 + KS * i + grp;
         fetch(t + 2 * KS, rg_new);
-        if (KS == 1 || t < w.ntile) {                  // (uniform) the last step of an odd walk: the other group's only
+        if (KS == 1 || t < t1) {                  // (uniform) the last step of an odd walk: the other group's only
             const uint16_t* Kb = Ks + (i & 1) * KT * KLD;
             f32x4 s[4];
 #pragma unroll
@@ -342,11 +348,11 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
         lds_barrier();
     };
     Rows ra, rb;
-    fetch(grp, ra);
-    fetch(grp + KS, rb);
+    fetch(t0 + grp, ra);
+    fetch(t0 + grp + KS, rb);
     park(0, ra);
     lds_barrier();
-    const int steps = (w.ntile + KS - 1) / KS;
+    const int steps = (max(0, t1 - t0) + KS - 1) / KS;
     for (int i = 0; i < steps; i += 2) {
         step(i, ra, rb);
         if (i + 1 < steps) step(i + 1, rb, ra);
@@ -364,7 +370,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
             pm[256 + wave * 64 + lane] = l;
         }
         lds_barrier();
-        if (grp == 1) return;
+        if (grp == 1 && shares == 1) return;
         const float m1 = pm[wave * 64 + lane], l1 = pm[256 + wave * 64 + lane];
         const float mn = fmaxf(q.m, m1), ms = mn == -INFINITY ? 0.f : mn;
         const float c1 = __builtin_amdgcn_exp2f(m1 - ms);
@@ -376,12 +382,64 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[n][r] = o[n][r] * c0 + p[r] * c1;
         }
+        if (shares > 1) {                              // (uniform) the last share to arrive adds all of them up, in their order
+            __shared__ int last;
+            float* const po2 = a.part_o + (size_t)((int)blockIdx.y * a.G + g) * (4 * NNT * 256);
+            float* const pm2 = a.part_ml + (size_t)((int)blockIdx.y * a.G + g) * 512;
+            // written through to where every XCD reads, and read from there: the counter needs no fence (fences write back and drop whole L2s: 18 us a launch became 52)
+            auto put = [](float* p, float x, float y) __attribute__((always_inline)) {
+                __hip_atomic_store((unsigned long long*)p, (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            };
+            if (grp == 0) {
+#pragma unroll
+                for (int n = 0; n < NNT; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2) put(&po2[((wave * NNT + n) * 64 + lane) * 4 + r], o[n][r], o[n][r + 1]);
+                put(&pm2[(wave * 64 + lane) * 2], mn, l);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            int32_t* const done = a.done + ((int)blockIdx.y - share) * a.G + g;
+            if (threadIdx.x == 0) last = atomicAdd(done, 1) == shares - 1;
+            __syncthreads();
+            if (!last || grp == 1) return;
+            if (threadIdx.x == 0) *done = 0;
+            auto get = [](const float* p) __attribute__((always_inline)) {
+                const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+            };
+            const size_t stride = (size_t)a.G * (4 * NNT * 256);
+            const float* p0 = po2 - share * stride, *m0 = pm2 - (size_t)share * a.G * 512;
+            float M = -INFINITY;
+            for (int k = 0; k < shares; ++k) M = fmaxf(M, get(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]).x);
+            const float Ms = M == -INFINITY ? 0.f : M;
+            l = 0.f;
+#pragma unroll
+            for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k < shares; ++k) {
+                const float2 ml = get(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]);
+                f32x4 p[NNT];
+#pragma unroll
+                for (int n = 0; n < NNT; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; r += 2) {
+                        const float2 v = get(&p0[k * stride + ((wave * NNT + n) * 64 + lane) * 4 + r]);
+                        p[n][r] = v.x; p[n][r + 1] = v.y;
+                    }
+                const float c = __builtin_amdgcn_exp2f(ml.x - Ms);
+                l = fmaf(ml.y, c, l);
+#pragma unroll
+                for (int n = 0; n < NNT; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[n][r] = fmaf(p[n][r], c, o[n][r]);
+            }
+        }
     }
     if (!q.ok) return;
 #pragma unroll
     for (int n = 0; n < NNT; ++n) {
         const int c = n * 16 + lg * 4;
-        if (c < e) put4(a, q.row, q.head, c, o[n], l, ovec);
+        if (c < e) put4(a, q.row, q.head, c, o[n], l, ovec, head_gate);
     }
 }
 
@@ -428,6 +486,7 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
     const int part_of = PACK ? lr >> 2 : 0;
     Query<3, PACK> q;
     q.init(a, sg, g, PACK ? min(lr & 3, nq - 1) : lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
+    const float head_gate = a.gate == LGATE_HEAD ? *gate_of(a, q.row, q.head) : 1.f;
     // requested in front of the first tile: answers come in order
     float x[8];
     if (wave < NKS) query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, wave * 32 + lg * 8, d, q.ok, qvec, x);
@@ -559,7 +618,7 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
         if (nsplit > 1) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) a.part_o[pr * e + c + r] = v[r];
-        } else if (q.ok) put4(a, q.row, q.head, c, v, L, ovec);
+        } else if (q.ok) put4(a, q.row, q.head, c, v, L, ovec, head_gate);
     }
 }
 template <int DP, int EP, bool POOL, bool PACK>
@@ -590,6 +649,11 @@ void go_sizes(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t 
 }
 
 }  // namespace
+
+// A walk of more than six tiles in shares of `each`.  A mixed step of 24 single tokens and 302 prompt rows behind up to 900 others, 8 heads on 2, leaves two thirds of the chip
+// idle while its longest blocks walk 19 tiles in ten steps: 18, 25, 29 and 33 us a layer behind 0, 302, 605 and 907 tokens, 16, 20, 21 and 21 with shares of six (of four 16, 20,
+// 20, 22; of two 17, 20, 20, 22): what is left of a launch is its start, first loads and end
+int lay_attn_tile_shares(int tiles, int each) { return tiles > 6 ? std::min(127, (tiles + each - 1) / each) : 1; }
 
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page) {
     return d > 0 && e > 0 && d % 16 == 0 && e % 16 == 0 && d <= 128 && e <= 128 && (own_v || e <= d) && page % KT == 0;

@@ -299,6 +299,9 @@ struct LAttnArgs {
     // few query tiles, many keys (decode steps): nsplit blocks per tile share its key tiles and a merge launch follows;
     // part_o [ntiles][G][nsplit][16][d], part_ml [ntiles][G][nsplit][16][2].  nsplit <= 1 or null scratch: one block per tile
     int nsplit = 1; float* part_o = nullptr; float* part_ml = nullptr;
+    // lay_attn_tile: a tile's keys shared among blocks.  tiles[i].x = segment + (share << 16) + (shares << 24), the shares of a tile side by side; sums in part_o [ntiles][G][64 e],
+    // part_ml [ntiles][G][64][2], the last one to arrive (done [ntiles][G], zero before and after) adds them up.  null: no tile is shared
+    int32_t* done = nullptr;
     // pool > 0: block b of `pool` positions is seen by position i through one mean key and one mean value when its last position
     // b pool + pool - 1 <= i - win; rows [n_pages][G][pool_rows][d] / [e] (lay_pool_append), in front of the window in the key walk
     long long pool = 0; const void* pk_pool = nullptr; const void* pv_pool = nullptr; int pool_rows = 0;
@@ -358,6 +361,9 @@ bool lay_attn_mfma_fits(int d, int e, bool own_v);         // sizes the matrix-c
 // heads 106 us against 1590, 8 on 2 (a mixed batch of 24 tokens and 300 prompt rows) 24 against 174; the older form keeps other page sizes
 // and long cached rows
 void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
+// among how many blocks a tile of `tiles` key tiles is shared when `each` are enough for a block; launches of at most LAY_ATTN_TILE_BLOCKS blocks
+constexpr int LAY_ATTN_TILE_BLOCKS = 256;
+int lay_attn_tile_shares(int tiles, int each);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
 // the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can
 // see, blocks of an unsplit launch, scratch parts)

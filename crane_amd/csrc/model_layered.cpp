@@ -1520,9 +1520,9 @@ void Model::alloc_runtime_layered() {
     }
     if (hde) { L.u_stride = hde; L.U = dalloc<float>((cap / LAY_LIGHT_CHUNK + (size_t)MAXB + 1) * hde); }
     if (hd) L.Dch = dalloc<float>((cap / LAY_LIGHT_CHUNK + (size_t)MAXB + 1) * hd);
-    if (L.max_e) {
-        L.att_po = dalloc<float>((size_t)Layered::ATT_PARTS * 16 * L.max_e);
-        L.att_pml = dalloc<float>((size_t)Layered::ATT_PARTS * 16 * 2);
+    if (L.max_e) {                     // shares of 16 query rows, or of 64 in the layout of 128 columns and 64 lanes (lay_attn_tile_kernel)
+        L.att_po = dalloc<float>(std::max((size_t)Layered::ATT_PARTS * 16 * L.max_e, (size_t)LAY_ATTN_TILE_BLOCKS * 64 * 128));
+        L.att_pml = dalloc<float>(std::max((size_t)Layered::ATT_PARTS * 16 * 2, (size_t)LAY_ATTN_TILE_BLOCKS * 512));
     }
     L.am_pv = dalloc<float>((size_t)Layered::LOGIT_ROWS * LAY_ARGMAX_PARTS);
     L.am_pi = dalloc<int>((size_t)Layered::LOGIT_ROWS * LAY_ARGMAX_PARTS);
@@ -1536,6 +1536,7 @@ void Model::alloc_runtime_layered() {
     // one table upload per pass: ids | rowseg | wanted rows | segments | page tables | attention tiles per group size
     size_t tiles = 0;
     for (int nrep : L.nreps) tiles += 2 * (cap * (size_t)nrep / 16 + (size_t)MAXB + 1) + 2 * (cap * (size_t)nrep / LAY_ATTN_MFMA_ROWS + (size_t)MAXB + 1);
+    tiles += (2 * L.nreps.size() + 1) * LAY_ATTN_TILE_BLOCKS;     // shared tiles, and their counters
     tiles += 2 * (cap / LAY_LIGHT_CHUNK + (size_t)MAXB + 1);      // lightning chunks
     tiles += 2 * ((size_t)L.ds_chunks + 1);                       // delta-rule chunks
     L.tab_ints = 3 * cap + (size_t)MAXB * (sizeof(LaySegDev) / 4) + (size_t)MAXB * max_pages_per_seq + tiles + L.spec.size() * (size_t)std::min(L.max_E, 32) * LAY_COUNT_STRIDE + 64;
@@ -1669,7 +1670,8 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             row += n;
             q.len += n;                        // the cache holds these positions once the pass has run
         }
-        std::map<int, std::pair<size_t, int>> tiles, tiles64;      // nrep -> (offset, count): 16 / 64 query rows per tile
+        int shared_heads = 0;
+        std::map<int, std::pair<size_t, int>> tiles, tiles64, shared64;      // nrep -> (offset, count): 16 / 64 query rows per tile
         for (int nrep : L.nreps) {
             if (o & 1) ++o;                    // int2 entries
             const size_t o_t = o; int cnt = 0;
@@ -1686,7 +1688,33 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     return t_segs[x.x].start_pos + x.y / nrep > t_segs[y.x].start_pos + y.y / nrep; });
             }
             tiles64[nrep] = {o_m, cnt};
+            // the same with the keys of long walks shared among blocks (lay_attn_tile_kernel), where blocks are few.  The walk: the longest window of the layers
+            int G = 0;
+            long long win = 0;
+            for (const LayerSpec& sp : L.spec)
+                if (sp.mixer == LMIX_ATTN && sp.kv_heads > 0 && sp.heads / sp.kv_heads == nrep && sp.pool == 0) { G = std::max(G, sp.kv_heads); win = std::max(win, sp.win + sp.keep); }
+            if (L.f32 || all_decode || G == 0 || cnt * G > LAY_ATTN_TILE_BLOCKS / 2) continue;
+            const int2* tl = (const int2*)(tab + o_m);
+            auto walk = [&](const int2& t) {
+                const LaySegDev& sg = t_segs[t.x];
+                const long long first = sg.start_pos + t.y / nrep, newest = sg.start_pos + (std::min(t.y + LAY_ATTN_MFMA_ROWS, sg.n * nrep) - 1) / nrep;
+                return (int)(newest / 64 - std::max(0ll, first - win + 1) / 64 + 1);
+            };
+            int each = 6, total = 0;
+            for (;; each += 2) {
+                total = 0;
+                for (int i = 0; i < cnt; ++i) total += lay_attn_tile_shares(walk(tl[i]), each);
+                if (total * G <= LAY_ATTN_TILE_BLOCKS) break;
+            }
+            if (total == cnt) continue;
+            const size_t o_s = o;
+            for (int i = 0; i < cnt; ++i)
+                for (int k = 0, n = lay_attn_tile_shares(walk(tl[i]), each); k < n; ++k) { tab[o++] = tl[i].x + (n > 1 ? (k << 16) + (n << 24) : 0); tab[o++] = tl[i].y; }
+            shared64[nrep] = {o_s, total};
+            shared_heads = std::max(shared_heads, G);
         }
+        const size_t o_done = o;               // blocks of every shared tile that have arrived
+        if (!shared64.empty()) { memset(tab + o, 0, LAY_ATTN_TILE_BLOCKS * sizeof(int32_t)); o += LAY_ATTN_TILE_BLOCKS; }
         if (o & 1) ++o;
         const size_t o_chunks = o;
         if (L.U && max_n > LAY_LIGHT_CHUNK)
@@ -1781,7 +1809,15 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
             if (L.attn_mfma && kv_mode == KV_BF16 && !all_decode && max_n >= 16 && lay_attn_mfma_fits(dk, ev, a.vpool != nullptr)) {
                 const auto& tm = tiles64[sp.heads / sp.kv_heads];
                 a.tiles = (const int2*)(L.d_tab + tm.first); a.ntiles = tm.second;
-                if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) { o16 = a.out16 = out16; launch_lay_attn_tile(a, s); }
+                if (lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
+                    const auto sh = shared64.find(sp.heads / sp.kv_heads);
+                    if (sh != shared64.end() && sp.pool == 0 && sp.kv_heads <= shared_heads && sh->second.second * sp.kv_heads <= LAY_ATTN_TILE_BLOCKS) {
+                        a.tiles = (const int2*)(L.d_tab + sh->second.first); a.ntiles = sh->second.second;
+                        a.done = L.d_tab + o_done;
+                    }
+                    o16 = a.out16 = out16;
+                    launch_lay_attn_tile(a, s);
+                }
                 else launch_lay_attn_mfma(a, s);
             } else if (L.attn_mfma && kv_mode == KV_BF16 && lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
                 a.single = all_decode;
