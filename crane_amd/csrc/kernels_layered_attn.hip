@@ -22,6 +22,7 @@
 #include "dev_common.h"
 #include "kernels.h"
 #include "layered.h"
+#include "layered_dev.h"
 
 namespace cm {
 
@@ -45,21 +46,22 @@ __device__ __forceinline__ void lds_barrier() {        // LDS hand-off only: req
 
 // The key walk of query rows [q0, q0 + nq) of a portion: `front` tiles of block rows (POOL) or of the kept first tokens that lie in front of the
 // window's first tile, then the window from a multiple of 64 on.
-struct Walk {
-    int pmin, pmax, main0, front, ntile, blocks, vis_lo;      // everybody sees [vis_lo, pmin]
-    int win, keep, chunk, pool;
+struct Walk : LAttnWalk {                                     // (everybody sees [vis_lo, pmin])
     template <bool POOL>
-    __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int q0, int nq, int nrep) {
-        win = (int)min(a.win, 1ll << 30); keep = (int)min(a.keep, 1ll << 30); chunk = (int)min(a.chunk, 1ll << 30);
-        pool = POOL ? (int)min(a.pool, 1ll << 30) : 0;
+    __host__ __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int q0, int nq, int nrep) {
+        auto word = [](long long v) { return (int)(v < (1ll << 30) ? v : 1ll << 30); };
+        auto lower = [](int x, int y) { return x < y ? x : y; };
+        auto upper = [](int x, int y) { return x > y ? x : y; };
+        win = word(a.win); keep = word(a.keep); chunk = word(a.chunk);
+        pool = POOL ? word(a.pool) : 0;
         pmin = sg.start_pos + q0 / nrep; pmax = sg.start_pos + (q0 + nq - 1) / nrep;
-        int main_lo = max(0, pmin - win + 1);
-        if (chunk > 0) main_lo = max(main_lo, pmin / chunk * chunk);
+        int main_lo = upper(0, pmin - win + 1);
+        if (chunk > 0) main_lo = upper(main_lo, pmin / chunk * chunk);
         main0 = main_lo / KT * KT;
-        blocks = POOL ? max(0, (pmax - win + 1) / pool) : 0;
-        front = POOL ? (blocks + KT - 1) / KT : min((keep + KT - 1) / KT, main0 / KT);
+        blocks = POOL ? upper(0, (pmax - win + 1) / pool) : 0;
+        front = POOL ? (blocks + KT - 1) / KT : lower((keep + KT - 1) / KT, main0 / KT);
         ntile = front + (pmax - main0) / KT + 1;
-        vis_lo = max(pmax - win + 1, chunk > 0 ? pmax / chunk * chunk : 0);
+        vis_lo = upper(pmax - win + 1, chunk > 0 ? pmax / chunk * chunk : 0);
     }
     __device__ __forceinline__ int first(int t) const { return t < front ? t * KT : main0 + (t - front) * KT; }
 };
@@ -102,38 +104,50 @@ struct Query {
     bool ok;
     int pos, head, row, clo;
     float r1, r2, m, l;
-    // pos -1: sees nothing where masks are applied.  first: this wave starts the running pair from the sink
-    __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int g, int qr, int q0, int nq, int nrep, int chunk, int lg, bool first) {
+    // pos -1: sees nothing where masks are applied
+    __device__ __forceinline__ void init(const LAttnArgs& a, const LaySegDev& sg, int g, int qr, int q0, int nq, int nrep, int chunk) {
         ok = qr < nq;
         const int qi = q0 + (ok ? qr : 0), lp = qi / nrep;
         head = g * nrep + (qi - lp * nrep);
         row = sg.row0 + lp;
         pos = ok ? sg.start_pos + lp : -1;
         clo = chunk > 0 && ok ? pos / chunk * chunk : 0;
+        begin(a);
+    }
+    // queries of one row in all (LAttnPrep)
+    __device__ __forceinline__ void init_alone(const LAttnArgs& a, int g, int j) {
+        ok = true; head = g * a.prep.nrep + j; row = 0; pos = a.prep.walk.pmax; clo = a.prep.clo;
+        begin(a);
+    }
+    __device__ __forceinline__ void begin(const LAttnArgs& a) {
         r1 = a.bias != LBIAS_NONE ? a.r1[head] * UNIT : 0.f;
         r2 = a.bias == LBIAS_LOG ? a.r2[head] : 0.f;
         m = -INFINITY; l = 0.f;
-        if (a.sink && ok && first) { m = a.sink[head] * UNIT; l = lg == 0 ? 1.f : 0.f; }     // the four lane groups' sums meet at the end
+    }
+    // the wave that starts the running pair from the sink (behind its first requests: the sink's arrival is no reason to hold them back)
+    __device__ __forceinline__ void start(const LAttnArgs& a, float sink, int lg, bool first) {
+        if (a.sink && ok && first) { m = sink * UNIT; l = lg == 0 ? 1.f : 0.f; }     // the four lane groups' sums meet at the end
     }
     // scores of tile t (products in s, keys 16 tt + 4 lg + r) -> weights in PARTS bfloat16 parts, the running pair moved on, o rescaled when a
     // new maximum appears in the wave.  p[..][h]: keys 16 (2 h) + 4 lg + 0 .. 3, then 16 (2 h + 1) + 4 lg + 0 .. 3
-    template <bool POOL, int NNT>
-    __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int lg, f32x4 (&s)[4], bf16x8 (&p)[KEPT][2], f32x4 (&o)[NNT], int part_of = 0) {
+    // TT groups of 16 keys from j0 on, in tile t of the walk
+    template <bool POOL, int NNT, int TT>
+    __device__ __forceinline__ void weights(const LAttnArgs& a, const Walk& w, int t, int j0, int lg, f32x4 (&s)[TT], bf16x8 (&p)[KEPT][TT / 2], f32x4 (&o)[NNT],
+                                            int part_of = 0) {
         const float scale = a.scale * UNIT;
-        const int j0 = w.first(t);
         const bool blk = POOL && t < w.front;
-        const bool full = t >= w.front && j0 >= w.vis_lo && j0 + KT - 1 <= w.pmin;
+        const bool full = t >= w.front && j0 >= w.vis_lo && j0 + 16 * TT - 1 <= w.pmin;
         float mt = -INFINITY;
         if (full && a.bias == LBIAS_NONE) {
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) { s[tt][r] *= scale; mt = fmaxf(mt, s[tt][r]); }
         } else {
             // (the distance term and the kind of tile are settled outside the loops: a branch per score kept the vector units at a third)
             auto each = [&](auto penalty, auto visible) __attribute__((always_inline)) {
 #pragma unroll ROLL
-                for (int tt = 0; tt < 4; ++tt) {
+                for (int tt = 0; tt < TT; ++tt) {
                     f32x4 v = s[0];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -142,7 +156,9 @@ struct Query {
                         v[r] = visible(j, dist) ? sc : -INFINITY;
                         mt = fmaxf(mt, v[r]);
                     }
-                    s[0] = s[1]; s[1] = s[2]; s[2] = s[3]; s[3] = v;
+#pragma unroll
+                    for (int k = 0; k + 1 < TT; ++k) s[k] = s[k + 1];
+                    s[TT - 1] = v;
                 }
             };
             // bitwise: no short-circuit branches
@@ -169,9 +185,9 @@ struct Query {
         }
         float psum = 0.f;
 #pragma unroll
-        for (int k = 0; k < KEPT; ++k) p[k][1] = __builtin_bit_cast(bf16x8, (u32x4){0u, 0u, 0u, 0u});
+        for (int k = 0; k < KEPT; ++k) p[k][TT / 2 - 1] = __builtin_bit_cast(bf16x8, (u32x4){0u, 0u, 0u, 0u});
 #pragma unroll ROLL
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < TT / 2; ++h) {
             u32x4 part[KEPT];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -195,17 +211,17 @@ struct Query {
                 }
             }
 #pragma unroll
-            for (int k = 0; k < KEPT; ++k) { p[k][0] = p[k][1]; p[k][1] = __builtin_bit_cast(bf16x8, part[k]); }
-            s[0] = s[2]; s[1] = s[3];
+            for (int k = 0; k < KEPT; ++k) { p[k][0] = p[k][TT / 2 - 1]; p[k][TT / 2 - 1] = __builtin_bit_cast(bf16x8, part[k]); }
+            if constexpr (TT == 4) { s[0] = s[2]; s[1] = s[3]; }
         }
         l += psum;
     }
 };
 // O^T += V^T P^T of one tile from its rows in LDS
-template <int VLD, int PARTS, int NNT>
-__device__ __forceinline__ void values(const uint16_t* Vb, int lr, int lg, const bf16x8 (&p)[PARTS][2], f32x4 (&o)[NNT]) {
+template <int VLD, int PARTS, int NNT, int NH>
+__device__ __forceinline__ void values(const uint16_t* Vb, int lr, int lg, const bf16x8 (&p)[PARTS][NH], f32x4 (&o)[NNT]) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < NH; ++h)
 #pragma unroll
         for (int n = 0; n < NNT; ++n) {
             bf16x4 v2[2];
@@ -265,7 +281,8 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     // this block's key tiles [t0, t1)
     const int per = (w.ntile + shares - 1) / shares, t0 = share * per, t1 = min(w.ntile, t0 + per), t_last = min(max(t0, t1 - 1), w.ntile - 1);      // (a share may be empty)
     Query<2> q;
-    q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk, lg, grp == 0 && share == 0);
+    q.init(a, sg, g, wave * 16 + lr, q0, nq, nrep, w.chunk);
+    const float sink = a.sink ? a.sink[q.head] : 0.f;
     const float head_gate = a.gate == LGATE_HEAD ? *gate_of(a, q.row, q.head) : 1.f;       // (here, not behind the walk: a trip to memory less)
     bf16x8 qf[NKS];                                    // rounded once
 #pragma unroll
@@ -341,7 +358,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
                 }
             }
             bf16x8 p[2][2];
-            q.template weights<POOL>(a, w, t, lg, s, p, o);
+            q.template weights<POOL>(a, w, t, w.first(t), lg, s, p, o);
             values<VLD>(Vs + (i & 1) * KT * VLD, lr, lg, p, o);
         }
         park((i + 1) & 1, rg_next);                    // that buffer was last read one step ago, behind that step's barrier
@@ -352,6 +369,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     fetch(t0 + grp + KS, rb);
     park(0, ra);
     lds_barrier();
+    q.start(a, sink, lg, grp == 0 && share == 0);
     const int steps = (max(0, t1 - t0) + KS - 1) / KS;
     for (int i = 0; i < steps; i += 2) {
         step(i, ra, rb);
@@ -465,50 +483,79 @@ void go(const LAttnArgs& a, bool qvec, bool ovec, hipStream_t s) {
 // 1699 / 1552, behind 1000 tokens 536 / 522, 2523 / 1154, 4780 / 1927
 // PACK: every sequence has one row and a key head at most four query heads: their parts are columns side by side of one product, as in
 // attn_decode_group_kernel, and blocks of four waves fit a CU twice: one sequence behind 1000 tokens, 8 heads on 2, 13.1 -> 10.7 us.
-template <int DP, int EP, bool POOL, bool PACK>
-__global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
-    constexpr int DW = PACK ? 4 : 8, QR = PACK ? 4 : 16;          // waves, query rows of the tile
-    constexpr int QLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16, VC = EP / 8, VPL = KT * VC / 64;
+// HALF (one sequence in all): eight waves on halves of tiles, since a wave's chain of requests, scores, weights and sums over a whole one is what the launch takes.
+// PREP (HALF, and its projection convolved): convolved q | k | v come from the projection; a wave rotates and scales a query head, and the wave that has the newest tile the key.  That key and
+// value take their rows' places in the wave's registers and go to the pages for the next step.
+// 8 heads on 2 of 128 behind 1000 tokens, with the convolution's launch: 5.1 + 10.5 us, 10.3 in one (whole tiles 11.3; the walk's divisions on the host, single-byte flags made words and the
+// sink's first use behind the first requests: 2.6 us of its chain)
+template <int DP, int EP, bool POOL, bool PACK, bool HALF, bool PREP>
+__global__ __launch_bounds__(PACK && !HALF ? 256 : 512, PACK && !HALF ? 2 : 1) void lay_attn_few_kernel(LAttnArgs a, bool qvec, bool ovec) {
+    constexpr int DW = PACK && !HALF ? 4 : 8, QR = PACK ? 4 : 16, TT = HALF ? 2 : 4, KW = 16 * TT;          // waves, query rows of the tile, keys of a wave's step
+    constexpr int QLD = DP + 8, VLD = EP + 16, NKS = DP / 32, NNT = EP / 16, VC = EP / 8, VPL = KW * VC / 64;
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
     __shared__ float pm[DW][16], pl_[DW][16];
-    uint16_t* const Qs = smem + DW * KT * VLD;         // [3 parts][QR][QLD]
+    __shared__ __attribute__((aligned(16))) uint16_t newest[PREP ? DP + EP : 8];
+    uint16_t* const Qs = smem + DW * KW * VLD;         // [3 parts][QR][QLD]
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    uint16_t* const Vw = smem + wave * KT * VLD;       // [64][VLD] of this wave
+    uint16_t* const Vw = smem + wave * KW * VLD;       // [KW][VLD] of this wave
     const int g = blockIdx.x;
     const int2 tile_id = PACK ? make_int2((int)blockIdx.y, 0) : a.tiles[blockIdx.y];
-    const LaySegDev sg = a.segs[tile_id.x];
-    const int nrep = a.H / a.G, d = a.d, e = a.e;
-    const int q0 = tile_id.y, nq = min(16, sg.n * nrep - q0);
+    const LaySegDev sg = PREP ? a.prep.seg : a.segs[tile_id.x];
+    const int nrep = PREP ? a.prep.nrep : a.H / a.G, d = a.d, e = a.e;
+    const int q0 = PREP ? 0 : tile_id.y, nq = PREP ? nrep : min(16, sg.n * nrep - q0);
     Walk w;
-    w.init<POOL>(a, sg, q0, nq, nrep);
+    if (PREP) static_cast<LAttnWalk&>(w) = a.prep.walk; else w.init<POOL>(a, sg, q0, nq, nrep);
+    auto page_no = [&](int j) __attribute__((always_inline)) { return PREP ? j >> a.prep.page_shift : j / a.page; };
+    auto in_page = [&](int j) __attribute__((always_inline)) { return PREP ? j & (a.page - 1) : j % a.page; };
+    // steps of KW keys: tile u of the walk, or (HALF) half u & 1 of tile u / 2
     const int t_first = (int)blockIdx.z * DW + wave, t_step = DW * (int)gridDim.z;
+    const int steps = HALF ? 2 * w.ntile - (w.pmax - w.first(w.ntile - 1) < 32 ? 1 : 0) : w.ntile;
+    auto tile_of = [&](int u) __attribute__((always_inline)) { return HALF ? u >> 1 : u; };
+    auto first_of = [&](int u) __attribute__((always_inline)) { return HALF ? w.first(u >> 1) + 32 * (u & 1) : w.first(u); };
     const int part_of = PACK ? lr >> 2 : 0;
     Query<3, PACK> q;
-    q.init(a, sg, g, PACK ? min(lr & 3, nq - 1) : lr, q0, nq, nrep, w.chunk, lg, t_first == 0);
+    if (PREP) q.init_alone(a, g, min(lr & 3, nq - 1)); else q.init(a, sg, g, PACK ? min(lr & 3, nq - 1) : lr, q0, nq, nrep, w.chunk);
+    const float sink = a.sink ? a.sink[q.head] : 0.f;
     const float head_gate = a.gate == LGATE_HEAD ? *gate_of(a, q.row, q.head) : 1.f;
     // requested in front of the first tile: answers come in order
     float x[8];
-    if (wave < NKS) query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, wave * 32 + lg * 8, d, q.ok, qvec, x);
+    const int t_new = steps - 1;
+    const bool has_new = PREP && a.prep.own && t_new >= t_first && (t_new - t_first) % t_step == 0;       // (uniform in the wave)
+    float2 qp = make_float2(0.f, 0.f), kp2 = qp, vp2 = qp;
+    int e0 = -1, e1 = -1, pg_new = 0;
+    float turn = 0.f;
+    if (PREP) {                                        // a rotated pair per lane, or two neighbours behind the rotated part
+        const int hd = a.prep.dims / 2;
+        if (lane < hd) { e0 = a.prep.half ? lane : 2 * lane; e1 = a.prep.half ? lane + hd : 2 * lane + 1; turn = a.prep.freq[lane]; }
+        else if (a.prep.dims + 2 * (lane - hd) < d) { e0 = a.prep.dims + 2 * (lane - hd); e1 = e0 + 1; }          // (d is even)
+        const float* qs = a.proj + a.q_off + (g * nrep + min(wave, nq - 1)) * d, *ks = a.proj + a.prep.k_off + g * d, *vs = a.proj + a.prep.v_off + g * e;
+        if (e0 >= 0 && wave < QR) qp = make_float2(qs[e0], qs[e1]);
+        if (has_new) {
+            if (e0 >= 0) kp2 = make_float2(ks[e0], ks[e1]);
+            if (2 * lane < e) vp2 = *(const float2*)(vs + 2 * lane);
+            pg_new = a.bt[sg.bt_off + page_no(w.pmax)];
+        }
+    } else if (wave < NKS) query8(a.proj + (size_t)q.row * a.ldp + a.q_off + q.head * d, wave * 32 + lg * 8, d, q.ok, qvec, x);
     int pgs_grp = 0;                                   // lane i: page of this wave's tile 64 grp + i
     auto load_pages = [&](int grp) __attribute__((always_inline)) {
-        const int j = min(w.first(min(t_first + (grp * 64 + lane) * t_step, w.ntile - 1)), w.pmax);
-        return a.bt[sg.bt_off + j / a.page];
+        const int j = min(first_of(min(t_first + (grp * 64 + lane) * t_step, steps - 1)), w.pmax);
+        return a.bt[sg.bt_off + page_no(j)];
     };
     int pgs = load_pages(0);
     const int Gv = a.v_div > 1 ? a.G / a.v_div : a.G, gv = a.v_div > 1 ? g / a.v_div : g;
-    u32x4 kr[4][NKS], vr[VPL];
+    u32x4 kr[TT][NKS], vr[VPL];
     auto page_of = [&](int i) __attribute__((always_inline)) {
         if ((i >> 6) != pgs_grp) { pgs_grp = i >> 6; pgs = load_pages(pgs_grp); }      // (uniform)
         return __builtin_amdgcn_readlane(pgs, i & 63);
     };
     auto fetch_k = [&](int i) __attribute__((always_inline)) {
-        const int t = t_first + i * t_step;
-        if (t >= w.ntile) return;                      // (uniform)
-        const int j0 = w.first(t), pg = page_of(i), last = w.pmax - j0;
-        const uint16_t* kp = (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + j0 % a.page) * d;
+        const int u = t_first + i * t_step, t = tile_of(u);
+        if (u >= steps) return;                        // (uniform)
+        const int j0 = first_of(u), pg = page_of(i), last = w.pmax - j0;
+        const uint16_t* kp = (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + in_page(j0)) * d;
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
+        for (int tt = 0; tt < TT; ++tt) {
             const uint16_t* row = kp + min(tt * 16 + lr, last) * d;
             if (POOL && t < w.front) row = (const uint16_t*)a.pk_pool + block_row(a, sg, g, min(j0 + tt * 16 + lr, w.blocks - 1), w.pool) * d;
 #pragma unroll
@@ -516,9 +563,9 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
         }
     };
     auto fetch_v = [&](int i) __attribute__((always_inline)) {
-        const int t = t_first + i * t_step;
-        if (t >= w.ntile) return;
-        const int j0 = w.first(t), pg = page_of(i), last = w.pmax - j0, r0 = j0 % a.page;
+        const int u = t_first + i * t_step, t = tile_of(u);
+        if (u >= steps) return;
+        const int j0 = first_of(u), pg = page_of(i), last = w.pmax - j0, r0 = in_page(j0);
         const uint16_t* vp = a.vpool ? (const uint16_t*)a.vpool + (((size_t)pg * Gv + gv) * a.page + r0) * e
                                      : (const uint16_t*)a.kpool + (((size_t)pg * a.G + g) * a.page + r0) * d;
         const int ldv = a.vpool ? e : d, c = (lane % VC) * 8 < e ? (lane % VC) * 8 : 0;
@@ -538,7 +585,45 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
     for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
     fetch_k(0);
     fetch_v(0);
-    if (wave < NKS) {
+    if (PREP) {
+        float sn = 0.f, cs = 1.f;
+        const int hd = a.prep.dims / 2;
+        if ((wave < QR || has_new) && lane < hd) { sincosf((float)w.pmax * turn, &sn, &cs); sn *= a.prep.mag; cs *= a.prep.mag; }
+        auto ready = [&](float2 v) __attribute__((always_inline)) {
+#pragma clang fp contract(off)                         // (a head times its factor is rounded before it is split)
+            if (lane < hd) v = lay_turn(v, cs, sn);
+            if (a.prep.unit) {
+                float ss = fmaf(v.x, v.x, 0.f);
+                ss = fmaf(v.y, v.y, ss);
+                for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+                const float rs = 1.f / sqrtf(ss / (float)d + a.prep.eps);
+                v.x *= rs; v.y *= rs;
+            }
+            return v;
+        };
+        if (wave < QR) qp = ready(qp);
+#pragma unroll
+        for (int k = 0; k < 3 && wave < QR; ++k) {
+            uint16_t* qd = &Qs[(k * QR + wave) * QLD];
+            const uint32_t pk = pack_bf16x2(qp.x, qp.y);
+            if (e0 >= 0) { qd[e0] = (uint16_t)pk; qd[e1] = (uint16_t)(pk >> 16); }
+            if (d + lane < DP) qd[d + lane] = 0;
+            qp.x -= bf16_lo(pk); qp.y -= bf16_hi(pk);
+        }
+        if (has_new) {                                 // (read back by this wave alone)
+            kp2 = ready(kp2);
+            const uint32_t kk = pack_bf16x2(kp2.x, kp2.y), vv = pack_bf16x2(vp2.x, vp2.y);
+            const size_t row = ((size_t)pg_new * a.G + g) * a.page + (size_t)in_page(w.pmax);
+            if (e0 >= 0) {
+                newest[e0] = (uint16_t)kk; newest[e1] = (uint16_t)(kk >> 16);
+                uint16_t* to = (uint16_t*)a.kpool + row * d;
+                to[e0] = (uint16_t)kk; to[e1] = (uint16_t)(kk >> 16);
+            }
+            if (d + lane < DP) newest[d + lane] = 0;
+            if (2 * lane < EP) *(uint32_t*)&newest[DP + 2 * lane] = 2 * lane < e ? vv : 0u;
+            if (2 * lane < e) *(uint32_t*)((uint16_t*)a.vpool + row * e + 2 * lane) = vv;
+        }
+    } else if (wave < NKS) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             u32x4 pk;
@@ -550,11 +635,27 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
             if (lr < QR) *(u32x4*)&Qs[(k * QR + lr) * QLD + wave * 32 + lg * 8] = pk;
         }
     }
+    q.start(a, sink, lg, t_first == 0);
     lds_barrier();
-    for (int i = 0, t = t_first; t < w.ntile; ++i, t += t_step) {
-        f32x4 s[4];
+    for (int i = 0, u = t_first; u < steps; ++i, u += t_step) {
+        const int t = tile_of(u), j0 = first_of(u);
+        if (PREP && has_new && u == t_new) {           // rows from the newest position on (those behind it are masked)
+            const int from = w.pmax - j0;
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int ks = 0; ks < NKS; ++ks) {
+                    const u32x4 nk = *(const u32x4*)&newest[ks * 32 + lg * 8];
+                    if (tt * 16 + lr >= from) kr[tt][ks] = nk;
+                }
+            const u32x4 nv = *(const u32x4*)&newest[DP + (lane % VC) * 8];
+#pragma unroll
+            for (int k = 0; k < VPL; ++k)
+                if (lane / VC + k * (64 / VC) >= from) vr[k] = nv;
+        }
+        f32x4 s[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) s[tt] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
@@ -562,12 +663,12 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
                 u32x4 qv = *(const u32x4*)&Qs[(PACK ? min(part_of, 2) * QR + (lr & 3) : k * 16 + lr) * QLD + ks * 32 + lg * 8];
                 if (PACK && part_of == 3) qv = (u32x4){0u, 0u, 0u, 0u};
 #pragma unroll
-                for (int tt = 0; tt < 4; ++tt)
+                for (int tt = 0; tt < TT; ++tt)
                     s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[tt][ks]), __builtin_bit_cast(bf16x8, qv), s[tt], 0, 0, 0);
             }
         if (PACK) {
 #pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
+            for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) s[tt][r] = parts_sum(s[tt][r]);
         }
@@ -575,8 +676,8 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
 #pragma unroll
         for (int k = 0; k < VPL; ++k) *(u32x4*)&Vw[(lane / VC + k * (64 / VC)) * VLD + (lane % VC) * 8] = vr[k];
         fetch_v(i + 1);
-        bf16x8 p[PACK ? 1 : 3][2];
-        q.template weights<POOL>(a, w, t, lg, s, p, o, part_of);
+        bf16x8 p[PACK ? 1 : 3][TT / 2];
+        q.template weights<POOL>(a, w, t, j0, lg, s, p, o, part_of);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the wave's own tile is in LDS
         values<VLD>(Vw, lr, lg, p, o);
     }
@@ -616,26 +717,28 @@ __global__ __launch_bounds__(PACK ? 256 : 512, PACK ? 2 : 1) void lay_attn_few_k
         }
         if (c >= e) continue;
         if (nsplit > 1) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) a.part_o[pr * e + c + r] = v[r];
+            *(f32x4*)(a.part_o + pr * e + c) = v;      // (e and c: multiples of 16 and 4)
         } else if (q.ok) put4(a, q.row, q.head, c, v, L, ovec, head_gate);
     }
 }
-template <int DP, int EP, bool POOL, bool PACK>
+template <int DP, int EP, bool POOL, bool PACK, bool HALF, bool PREP>
 void go_few(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
-    constexpr int DW = PACK ? 4 : 8, QR = PACK ? 4 : 16;
-    constexpr size_t lds = ((size_t)DW * KT * (EP + 16) + 3 * QR * (DP + 8)) * sizeof(uint16_t);
+    constexpr int DW = PACK && !HALF ? 4 : 8, QR = PACK ? 4 : 16;
+    constexpr size_t lds = ((size_t)DW * (HALF ? 32 : KT) * (EP + 16) + 3 * QR * (DP + 8)) * sizeof(uint16_t);
     static_assert(lds >= (size_t)DW * (EP / 16) * 64 * 4 * sizeof(float), "the waves' sums");
     static_assert(DP / 32 <= DW, "a wave per 32 elements of the queries");
     static DevOnce attr;
     attr.run([&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_few_kernel<DP, EP, POOL, PACK>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_attn_few_kernel<DP, EP, POOL, PACK, HALF, PREP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     });
-    hipLaunchKernelGGL((lay_attn_few_kernel<DP, EP, POOL, PACK>), dim3((unsigned)a.G, (unsigned)a.ntiles, (unsigned)nsplit), dim3(DW * 64), lds, s, a, qvec, ovec);
+    hipLaunchKernelGGL((lay_attn_few_kernel<DP, EP, POOL, PACK, HALF, PREP>), dim3((unsigned)a.G, (unsigned)a.ntiles, (unsigned)nsplit), dim3(DW * 64), lds, s, a, qvec, ovec);
 }
 template <int DP, int EP, bool POOL>
 void go_few(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
-    if (lay_attn_packed(a)) go_few<DP, EP, POOL, true>(a, nsplit, qvec, ovec, s); else go_few<DP, EP, POOL, false>(a, nsplit, qvec, ovec, s);
+    if (a.prep.on) go_few<DP, EP, false, true, true, true>(a, nsplit, qvec, ovec, s);      // (lay_attn_prep_fits)
+    else if (lay_attn_packed(a) && a.ntiles == 1) go_few<DP, EP, POOL, true, true, false>(a, nsplit, qvec, ovec, s);
+    else if (lay_attn_packed(a)) go_few<DP, EP, POOL, true, false, false>(a, nsplit, qvec, ovec, s);
+    else go_few<DP, EP, POOL, false, false, false>(a, nsplit, qvec, ovec, s);
 }
 // nsplit 0: the prompt kernel
 template <int DP, int EP>
@@ -659,10 +762,23 @@ bool lay_attn_tile_fits(int d, int e, bool own_v, int page) {
     return d > 0 && e > 0 && d % 16 == 0 && e % 16 == 0 && d <= 128 && e <= 128 && (own_v || e <= d) && page % KT == 0;
 }
 
+// queries of one row on their way through lay_attn_few_kernel: a wave per query head, a pair of elements per lane, values in pages of their own
+bool lay_attn_prep_fits(int H, int G, int d, int e, int dims, int page, bool pooled) {
+    return lay_attn_tile_fits(d, e, true, page) && H <= 4 * G && H % G == 0 && dims % 2 == 0 && dims <= d && !pooled && (page & (page - 1)) == 0;
+}
+
 static void launch(const LAttnArgs& a0, int nsplit, hipStream_t s) {
     LAttnArgs a = a0;
     if (!a.gbuf) { a.gbuf = a.proj + a.g_off; a.ldg = a.ldp; }
     if (a.e <= 0) a.e = a.d;
+    if (a.prep.on) {
+        Walk w;
+        a.prep.nrep = a.H / a.G;
+        w.init<false>(a, a.prep.seg, 0, a.prep.nrep, a.prep.nrep);
+        a.prep.walk = w;
+        a.prep.clo = w.chunk > 0 ? w.pmax / w.chunk * w.chunk : 0;
+        for (a.prep.page_shift = 0; (1 << a.prep.page_shift) < a.page;) ++a.prep.page_shift;
+    }
     const bool qvec = a.ldp % 4 == 0 && a.q_off % 4 == 0 && ((uintptr_t)a.proj & 15) == 0;
     const bool ovec = a.ldo % 4 == 0 && ((uintptr_t)a.out & 15) == 0;
     if (a.d <= 64) { if (a.e <= 64) go_sizes<64, 64>(a, nsplit, qvec, ovec, s); else go_sizes<64, 128>(a, nsplit, qvec, ovec, s); }

@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int n
                 float sn_, cs;
                 sincosf((float)pos * fr[p], &sn_, &cs);
                 sn_ *= a.mag; cs *= a.mag;
-                v[p] = make_float2(v[p].x * cs - v[p].y * sn_, v[p].y * cs + v[p].x * sn_);
+                v[p] = lay_turn(v[p], cs, sn_);
             }
             ss = fmaf(v[p].x, v[p].x, ss); ss = fmaf(v[p].y, v[p].y, ss);
         }

@@ -7,7 +7,7 @@
 // no other block of the launch reads: the residual goes from x to x2 in front of the mixer and back in front of the experts.
 // Every sum is made in the order of the launches that these replace (lay_add_tanh_norm_kernel, lgemv_kernel, lay_router_decode_kernel, lay_attn_merge_kernel): the
 // same bits.
-// Measured (us, width 1024, 14 experts of 768, 4 per token, and one of 512): norm + router + gate-and-up 18.9 in three launches, 9.1 here; norm and input
+// Measured (us, width 1024, 14 experts of 768, 4 per token, and one of 512): norm + router + gate-and-up 18.9 in three launches, 8.3 here; norm and input
 // projection 7.8 in two, 4.1 here; the second product 5.3, 4.2 (its matrices follow from the choices, not from the sorted rows); output projection behind
 // five attention shares 9.0 with a merging launch, 4.3 here.
 #include <algorithm>
@@ -66,9 +66,9 @@ __device__ __forceinline__ float step_dot(float acc, const u32x4& w, const float
     return acc;
 }
 
-// C = act(norm(x) W^T + bias), two columns per wave
+// C = act(norm(x) W^T + bias), two columns per wave; columns of queries, keys and values through their convolution, whose inputs and weights are on their way meanwhile
 template <int NIT>
-__global__ __launch_bounds__(256) void lay_step_in_kernel(LStepNorm a, LStepProj p) {
+__global__ __launch_bounds__(256) void lay_step_in_kernel(LStepNorm a, LStepProj p, LStepConv cv) {
     constexpr int K = NIT * 512;
     __shared__ __attribute__((aligned(16))) float h[K];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -78,6 +78,15 @@ __global__ __launch_bounds__(256) void lay_step_in_kernel(LStepNorm a, LStepProj
     for (int i = 0; i < NIT; ++i) {
         w0[i] = ld_nt16(p.W + (size_t)n0 * K + lane * 8 + i * 512);
         w1[i] = ld_nt16(p.W + (size_t)n1 * K + lane * 8 + i * 512);
+    }
+    const int n = (int)(blockIdx.x * 4 + wave) * 2 + lane;
+    const bool conv = lane < 2 && n < cv.C;
+    float in[LAY_STEP_TAPS], cw[LAY_STEP_TAPS];            // taps in front of the first one: weight 0
+#pragma unroll
+    for (int j = 0; j < LAY_STEP_TAPS; ++j) {
+        const int t = j - (LAY_STEP_TAPS - cv.taps);
+        cw[j] = conv && t >= 0 ? cv.cw[(size_t)t * cv.C + n] : 0.f;
+        in[j] = conv && t >= 0 && t < cv.taps - 1 ? cv.tail[(size_t)t * cv.C + n] : 0.f;
     }
     step_norm<NIT>(a, h, blockIdx.x == 0);
     __syncthreads();
@@ -92,11 +101,22 @@ __global__ __launch_bounds__(256) void lay_step_in_kernel(LStepNorm a, LStepProj
         acc1 = step_dot(acc1, w1[i], x);
     }
     acc0 = wave_sum(acc0); acc1 = wave_sum(acc1);
-    const int n = (int)(blockIdx.x * 4 + wave) * 2 + lane;
     if (lane < 2 && n < p.N) {
         float v = lane ? acc1 : acc0;
         if (p.bias) v += p.bias[n];
-        p.C[n] = lay_act(v, n < p.act_split ? p.act : p.act2, p.act_param);
+        v = lay_act(v, n < p.act_split ? p.act : p.act2, p.act_param);
+        if (conv) {
+            in[LAY_STEP_TAPS - 1] = v;
+            v = 0.f;
+#pragma unroll
+            for (int j = 0; j < LAY_STEP_TAPS; ++j) v = fmaf(cw[j], in[j], v);
+#pragma unroll
+            for (int j = 1; j < LAY_STEP_TAPS; ++j) {
+                const int t = j - 1 - (LAY_STEP_TAPS - cv.taps);
+                if (t >= 0) cv.tail[(size_t)t * cv.C + n] = in[j];
+            }
+        }
+        p.C[n] = v;
     }
 }
 
@@ -161,7 +181,27 @@ __global__ __launch_bounds__(256) void lay_step_out_kernel(LAttnArgs a, int nspl
     if (lane < 2 && n < N) C[n] = lane ? acc1 : acc0;
 }
 
-// norm, router, choice, and act(h W_e^T) * (h W2_e^T) of the chosen experts and the one of every token.  blockIdx.y: the choice, the last the expert of every token
+// the expert of choice `slot` by what lay_router_choose chooses by, in every wave for itself: the lane with `slot` better ones (equals: the lower lane first).  -1: not by numbers
+__device__ __forceinline__ int step_choice(const float* zs, int lane, int slot, int E, const RouterSpec& rs) {
+    const float z = lane < E ? zs[lane] : -INFINITY;
+    float own = z;
+    if (rs.softmax) {
+        const float mx = wave_max(z), p = lane < E ? expf(z - mx) : 0.f;
+        own = p / wave_sum(p);
+    }
+    if (__any(lane < E && own != own)) return -1;
+    int better = 0;
+    for (int j = 0; j < E; ++j) {
+        const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), j));
+        better += v > own || (v == own && j < lane);
+    }
+    const unsigned long long at = __ballot(lane < E && better == slot);
+    return at ? __builtin_ctzll(at) : -1;
+}
+
+// norm, router, choice, and act(h W_e^T) * (h W2_e^T) of the chosen experts and the one of every token.  blockIdx.y: the choice, the last the expert of every token.  A last block
+// of the first choice writes the choices and their weights, which the others do not wait for (one wave's choice for
+// the block and all of them through it 9.3 us a launch, each its own 8.3)
 template <int NIT>
 __global__ __launch_bounds__(256) void lay_step_moe_kernel(LStepNorm a, LStepMoe m) {
     constexpr int K = NIT * 512, NR = NIT <= 2 ? 4 : NIT == 4 ? 2 : 1;     // router outputs of a wave whose weights are requested together
@@ -169,9 +209,9 @@ __global__ __launch_bounds__(256) void lay_step_moe_kernel(LStepNorm a, LStepMoe
     __shared__ float zs[2 * 64 + 2 + 64], swt[65];            // lay_router_choose: logits, scores, one group, choices
     __shared__ int32_t ss[64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slot = blockIdx.y;
-    const bool every = slot == m.top, first = blockIdx.x == 0 && slot == 0;
+    const bool every = slot == m.top, first = blockIdx.x == 0 && slot == 0, writes = blockIdx.x == gridDim.x - 1;
     const int N = every ? m.sh_ff : m.ff;
-    if ((int)blockIdx.x * 8 >= N) return;
+    if (writes ? slot != 0 : (int)blockIdx.x * 8 >= N) return;
     const int logits = m.experts + (m.rs.shared_gate ? 1 : 0);
     u32x4 rw[NR][NIT];
     auto request = [&](int e0) __attribute__((always_inline)) {
@@ -204,13 +244,18 @@ __global__ __launch_bounds__(256) void lay_step_moe_kernel(LStepNorm a, LStepMoe
             }
         }
         __syncthreads();
-        if (wave == 0) lay_router_choose(zs, 0, lane, ss, swt, m.experts, m.top, m.rs, nullptr, m.slots);
-        __syncthreads();
-        e = __builtin_amdgcn_readfirstlane(ss[slot]);
-        if (first) {
-            for (int k = threadIdx.x; k < m.top; k += 256) m.sel[k] = ss[k];
-            for (int k = threadIdx.x; k < m.slots; k += 256) m.wsel[k] = swt[k];
+        e = writes ? -1 : step_choice(zs, lane, slot, m.experts, m.rs);
+        if (e < 0) {                           // (uniform in the block)
+            if (wave == 0) lay_router_choose(zs, 0, lane, ss, swt, m.experts, m.top, m.rs, nullptr, m.slots);
+            __syncthreads();
+            e = ss[slot];
+            if (writes) {
+                for (int k = threadIdx.x; k < m.top; k += 256) m.sel[k] = ss[k];
+                for (int k = threadIdx.x; k < m.slots; k += 256) m.wsel[k] = swt[k];
+                return;
+            }
         }
+        e = __builtin_amdgcn_readfirstlane(e);
     }
     const uint16_t* W = every ? m.sh_gate : m.gate + (size_t)e * m.ff * K;
     const uint16_t* W2 = every ? m.sh_up : m.up + (size_t)e * m.ff * K;
@@ -281,8 +326,8 @@ bool lay_step_fits(int W, const LayerSpec& sp) {
            !sp.router.correction && sp.expert_act == LACT_SILU && logits <= 64 && sp.top <= 63 && sp.ff % 8 == 0 && sp.shared_ff % 8 == 0;
 }
 #define CM_STEP_W(CALL) switch (W) { case 512: CALL(1); break; case 1024: CALL(2); break; case 2048: CALL(4); break; default: CALL(8); }
-void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream_t s) {
-#define CM_CALL(I) hipLaunchKernelGGL(lay_step_in_kernel<I>, dim3((unsigned)((p.N + 7) / 8)), dim3(256), 0, s, a, p)
+void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, const LStepConv& c, int W, hipStream_t s) {
+#define CM_CALL(I) hipLaunchKernelGGL(lay_step_in_kernel<I>, dim3((unsigned)((p.N + 7) / 8)), dim3(256), 0, s, a, p, c)
     CM_STEP_W(CM_CALL)
 #undef CM_CALL
 }
@@ -305,7 +350,7 @@ void launch_lay_step_out(const LAttnArgs& a, const uint16_t* Wm, float* C, int N
 }
 void launch_lay_step_moe(const LStepNorm& a, const LStepMoe& m, float* ys, int W, hipStream_t s) {
     const unsigned slots = (unsigned)(m.top + (m.sh_ff > 0 ? 1 : 0));
-    const dim3 grid((unsigned)((std::max(m.ff, m.sh_ff) + 7) / 8), slots);
+    const dim3 grid((unsigned)((std::max(m.ff, m.sh_ff) + 7) / 8 + 1), slots);
 #define CM_CALL(I) hipLaunchKernelGGL(lay_step_moe_kernel<I>, grid, dim3(256), 0, s, a, m)
     CM_STEP_W(CM_CALL)
 #undef CM_CALL

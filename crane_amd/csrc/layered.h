@@ -72,15 +72,16 @@ struct RotSpec {
     double low = 1.0, high = 4.0;
 };
 // how a router turns its logits into choices and weights
+// (kernels take this and the structures below by value: flags are words, since a byte there is a vector load and a wait of its own, about 1 us)
 struct RouterSpec {
-    bool softmax = false;              // scores: softmax over all outputs (false: sigmoid of each)
-    bool correction = false;           // a learned vector joins the scores for the choice only
+    int softmax = 0;              // scores: softmax over all outputs (false: sigmoid of each)
+    int correction = 0;           // a learned vector joins the scores for the choice only
     int groups = 1, keep_groups = 1;   // outputs form `groups` equal groups of neighbours; only the keep_groups best can be chosen
     int group_top = 1;                 // a group's score: the sum of its group_top (1 or 2) largest choice scores
-    bool normalise = false;            // weights divided by their sum
+    int normalise = 0;            // weights divided by their sum
     float scale = 1.f;                 // ... then times this
     int identity = 0;                  // the last `identity` outputs pass the input through (no matrices)
-    bool shared_gate = false;          // one more logit behind the outputs': its sigmoid is the weight of the expert every token uses
+    int shared_gate = 0;          // one more logit behind the outputs': its sigmoid is the weight of the expert every token uses
 };
 
 // one entry of config "layers"
@@ -282,6 +283,13 @@ void launch_lay_post_norm_canon_decode(float* x, const float* y, const float* pw
 void launch_lay_post_norm(float* x, const float* y, const float* w, float mult, float eps, int T, int W, const float* wsel, int top,
                           hipStream_t s, const int32_t* sel = nullptr, int sel_top = 0, int n_real = -1, const float* hin = nullptr);
 
+// a step of one row whose projection has left convolved q | k | v (LStepConv): the attention rotates and scales its queries itself, and the block that has the newest tile the
+// key, which goes to the pages with the value from there.  own: the layer has keys of its own
+struct LAttnWalk { int pmin, pmax, main0, front, ntile, blocks, vis_lo, win, keep, chunk, pool; };      // the key walk of a query tile (kernels_layered_attn.hip)
+struct LAttnPrep {
+    int on = 0, own = 0, half = 0, unit = 0, k_off = 0, v_off = 0, dims = 0; const float* freq = nullptr; float mag = 1.f, eps = 0.f; LaySegDev seg{};
+    LAttnWalk walk{}; int clo = 0, nrep = 0, page_shift = 0;      // filled in by the launch: what a block would divide for
+};
 struct LAttnArgs {
     const float* proj; int ldp, q_off, g_off;        // activated projection rows: q | k | gate
     const float* gbuf = nullptr; int ldg = 0;        // gates in rows of their own (null: proj + g_off, rows of ldp)
@@ -302,11 +310,12 @@ struct LAttnArgs {
     // lay_attn_tile: a tile's keys shared among blocks.  tiles[i].x = segment + (share << 16) + (shares << 24), the shares of a tile side by side; sums in part_o [ntiles][G][64 e],
     // part_ml [ntiles][G][64][2], the last one to arrive (done [ntiles][G], zero before and after) adds them up.  null: no tile is shared
     int32_t* done = nullptr;
+    LAttnPrep prep;                                  // lay_attn_few, single rows
     // pool > 0: block b of `pool` positions is seen by position i through one mean key and one mean value when its last position
     // b pool + pool - 1 <= i - win; rows [n_pages][G][pool_rows][d] / [e] (lay_pool_append), in front of the window in the key walk
     long long pool = 0; const void* pk_pool = nullptr; const void* pv_pool = nullptr; int pool_rows = 0;
     float out_scale = 1.f;                           // factor on the output
-    bool single = false;                             // lay_attn_few: every segment is one row (tile i: segment i)
+    int single = 0;                                  // lay_attn_few: every segment is one row (tile i: segment i)
     int v_div = 1;                                   // v_div consecutive key heads share one value head: value pages [n_pages][G / v_div][page][e]
 };
 void launch_lay_k_append(const float* proj, int ldp, int k_off, void* kpool, int kvt, const int32_t* bt, const LaySegDev* segs,
@@ -331,6 +340,9 @@ void launch_lay_qk_prep(float* proj, int ldp, int q_off, int k_off, int v_off, i
 // written to xout, through tanh(alpha .) w + b.  xout is no buffer that the launch reads; y null: xout = x
 struct LStepNorm { const float *x, *y, *wsel, *w, *b; float* xout; int nsum; float mult, alpha; };
 struct LStepProj { const uint16_t* W; const float* bias; float* C; int N, act, act2, act_split; float act_param; };
+// columns below C through their causal convolution (at most LAY_STEP_TAPS taps, as LConvQkvArgs), their tail moved on
+constexpr int LAY_STEP_TAPS = 4;
+struct LStepConv { int C = 0, taps = 0; const float* cw = nullptr; float* tail = nullptr; };
 struct LStepMoe {
     const uint16_t *router, *gate, *up, *down, *sh_gate, *sh_up, *sh_down;
     float *hh, *hs, *wsel;             // inner rows of the choices [top][ff] and of the expert of every token [sh_ff]; weights [slots]
@@ -339,7 +351,7 @@ struct LStepMoe {
     RouterSpec rs;
 };
 bool lay_step_fits(int W, const LayerSpec& sp);
-void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, int W, hipStream_t s);
+void launch_lay_step_in(const LStepNorm& a, const LStepProj& p, const LStepConv& c, int W, hipStream_t s);
 // the output projection behind an attention of one row whose nsplit > 1 shares have not been merged (a: its arguments, e and gbuf filled in; a gate per head)
 bool lay_step_out_fits(const LAttnArgs& a);
 void launch_lay_step_out(const LAttnArgs& a, const uint16_t* W, float* C, int N, hipStream_t s);
@@ -364,6 +376,7 @@ void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
 // among how many blocks a tile of `tiles` key tiles is shared when `each` are enough for a block; launches of at most LAY_ATTN_TILE_BLOCKS blocks
 constexpr int LAY_ATTN_TILE_BLOCKS = 256;
 int lay_attn_tile_shares(int tiles, int each);
+bool lay_attn_prep_fits(int H, int G, int d, int e, int dims, int page, bool pooled);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
 // the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can
 // see, blocks of an unsplit launch, scratch parts)
@@ -381,7 +394,7 @@ struct LLightArgs {
     // chunk-parallel form (long portions; head size up to 128): chunk table {segment, first token}, segs[].pad0 = a segment's first
     // chunk, U = [nchunks][H][d][e] f32 scratch.  Null / 0: one block per (sequence, head, value slice) walks the portion.
     float* U = nullptr; const int2* chunks = nullptr; int nchunks = 0;
-    bool all_single = false;     // every portion of the pass is one token (decode steps): the state is updated in place in HBM
+    int all_single = 0;          // every portion of the pass is one token (decode steps): the state is updated in place in HBM
     // gated form: the decay of key channel i at token t is exp(ldec[t ldd + head d + i]) instead of decay[head]
     const float* ldec = nullptr; int ldd = 0;
     float qscale = 1.f;          // q is multiplied by this
@@ -389,7 +402,7 @@ struct LLightArgs {
     // one decay per head and token instead of one per key channel: ldec[t ldd + head] (head_decay), and a factor on the key:
     // k_t * kmul[t ldd + head].  ones_col: the last of the e value columns is the constant 1 (the projection row holds e - 1 per
     // head), so that the state's last column carries sum_s decay(s..t) k_s -- the normaliser of a matrix memory
-    bool head_decay = false; const float* kmul = nullptr; bool ones_col = false;
+    int head_decay = 0; const float* kmul = nullptr; int ones_col = 0;
     int qk_rep = 1;              // qk_rep consecutive heads share one query / key vector: q and k hold H / qk_rep vectors of d
 };
 constexpr int LAY_LIGHT_CHUNK = 32;
@@ -413,12 +426,12 @@ struct LConvQkvArgs {
     int H, G, d, e;
     const float* cw; int taps;                       // [taps][channels], the last row the current token's
     float* conv_pool; size_t slot_stride, cv_off;    // tails [taps - 1][channels], oldest first
-    int dims; bool half; const float* freq; float mag;   // rotation (freq null: none), as lay_rope
-    bool unit; float eps;
+    int dims; int half; const float* freq; float mag;    // rotation (freq null: none), as lay_rope
+    int unit; float eps;
     float* q; int ldq;                               // [T][H d]
     void *kpool, *vpool;                             // [n_pages][G][page][d] / [e]
     const int32_t* bt; const LaySegDev* segs; const int32_t* rowseg; int page, T;
-    bool tail_too = false;                           // every portion of the pass is one token: a channel's tail is shifted by its thread
+    int tail_too = 0;                                // every portion of the pass is one token: a channel's tail is shifted by its thread
                                                      // (otherwise launch_lay_conv_tail follows)
 };
 constexpr int LAY_CONV_QKV_MAX_DIM = 1024;           // largest d
@@ -441,7 +454,7 @@ struct LConvArgs {
     const float* src; int lds, off, C; float* dst; int ldd; const float *cw, *cb; int taps, act;
     float* conv_pool; size_t slot_stride, cv_off; const LaySegDev* segs; const int32_t* rowseg;
     int H = 0, dt_off = 0; const float *dt_bias = nullptr, *a_neg = nullptr; float *ldec = nullptr, *kmul = nullptr;
-    bool tail_too = false;
+    int tail_too = 0;
 };
 void launch_lay_conv_act(const LConvArgs& a, int T, hipStream_t s);
 void launch_lay_conv_tail(const LConvArgs& a, int nseg, hipStream_t s);
@@ -476,14 +489,14 @@ struct LDeltaArgs {
     const float *dt_bias, *a_neg;                    // head form: ln g = a_neg[h] softplus(a + dt_bias[h]);  channel: ln g = a_neg[h] softplus(ldec)
     float* xb;                                       // [T][2 G d + H e]: convolved q (unit length, times d^(-1/2)) | k (unit length) | v
     float* beta;                                     // [T][H]
-    float* ldec; bool channel;                       // [T][H] (written by the preparation: ln g), or [T][H d] (channel: the argument of the softplus)
+    float* ldec; int channel;                        // [T][H] (written by the preparation: ln g), or [T][H d] (channel: the argument of the softplus)
     float* state_pool; size_t slot_stride, st_off;
     const LaySegDev* segs; const int32_t* rowseg; int nseg, T;
     const float* gate; int ldg, gate_act;            // output gate [T][H e] before its activation (LACT_SILU, LACT_SIGMOID)
     const float* norm_w; float eps;
     float* o_raw;                                    // [T][H e] scratch (token-by-token form)
     float* out;                                      // [T][H e]
-    bool all_single;                                 // every portion of the pass is one token
+    int all_single;                                  // every portion of the pass is one token
     int min_n;                                       // the shortest portion
     // chunk-parallel form for portions of more than LAY_DELTA_SEQ tokens: table {segment, first token}, segs[].pad1 = a segment's first
     // chunk; scratch of lay_delta_chunk_floats per (chunk, head).  Null / 0: every portion token by token.

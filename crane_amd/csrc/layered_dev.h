@@ -26,6 +26,9 @@ __device__ __forceinline__ float lay_capglu(float g, float u, float cap) {
     return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
 }
 
+// a pair turned by an angle; spelled out, so that every kernel rounds it alike
+__device__ __forceinline__ float2 lay_turn(float2 v, float cs, float sn) { return make_float2(fmaf(v.x, cs, -(v.y * sn)), fmaf(v.y, cs, v.x * sn)); }
+
 // One wave turns the E logits of token t in zs into choices and weights.  zs: [E] logits, then choice scores (shared_gate: one more
 // logit behind them); sc: [E] scores, [groups], [top].
 __device__ __forceinline__ void lay_router_choose(float* zs, int t, int lane, int32_t* __restrict__ sel, float* __restrict__ wsel, int E, int top,

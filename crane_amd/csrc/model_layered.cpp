@@ -1778,6 +1778,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         // softmax attention of one layer over the pages: queries at qsrc[row ldq + q_off + head dk], output [T][H ev] into L.O
         bool keep_shares = false;              // the next attention may leave its shares (in `left`) to the output projection
         LAttnArgs left;
+        LAttnPrep prep;                        // the next attention's own preparation
         auto run_attention = [&](const LayerSpec& sp, const LayeredLayerW& w, const float* qsrc, int ldq, int q_off, int g_off, int dk, int ev,
                                  float* out = nullptr, int ldo = 0, float out_scale = 1.f, int v_div = 1, const float* gbuf = nullptr, int ldg = 0,
                                  uint16_t* out16 = nullptr) {
@@ -1821,6 +1822,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 else launch_lay_attn_mfma(a, s);
             } else if (L.attn_mfma && kv_mode == KV_BF16 && lay_attn_tile_fits(dk, ev, a.vpool != nullptr, page)) {
                 a.single = all_decode;
+                a.prep = prep;
                 a.nsplit = lay_attn_few_split(seen, a.ntiles * sp.kv_heads, Layered::ATT_PARTS, all_decode && sp.heads <= 4 * sp.kv_heads);
                 o16 = a.out16 = out16;
                 const bool leave = keep_shares && lay_step_out_fits(a);
@@ -1997,6 +1999,9 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 // ---- x += mult mixer(norm1 x), x += mult ff(norm2 x); norms in equal parts, or of single elements
                 // one row: the norms inside the launches of the products behind them, the router inside the experts' (x -> X2 -> x)
                 const bool one_row = T == 1 && L.tanh_norm && !L.f32 && L.fused_prep && lay_step_fits(W, sp);
+                // ... the convolutions behind the projection's sums, rotation, unit heads and cache append inside the attention
+                const bool prepared = one_row && sp.mixer == LMIX_ATTN && sp.maps == 1 && L.attn_mfma && kv_mode == KV_BF16 && sp.conv <= LAY_STEP_TAPS && w.v_page_bytes != 0 &&
+                                      lay_attn_prep_fits(sp.heads, sp.kv_heads, sp.dim, sp.vdim, w.rot_freq ? sp.rot.dims : 0, page, sp.pool > 0);
                 // the norm in front of the experts, their router and lists and this layer's convolution tails in one launch
                 const bool joined = L.tanh_norm && rounded && sp.mlp == LMLP_MOE && !sp.scale_input && lay_norm_router_fits(W, sp.experts, sp.router) &&
                                     lay_experts_on_tiles(L, sp, T, W) &&
@@ -2008,8 +2013,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 g.act_split = w.g_off; g.act = sp.mixer == LMIX_HGRN ? LACT_SILU : LACT_NONE;
                 g.act2 = sp.mixer == LMIX_ATTN && sp.gate != LGATE_NONE ? LACT_SIGMOID : LACT_NONE;
                 if (one_row) {
+                    LStepConv c;
+                    if (prepared) { c.C = w.g_off; c.taps = sp.conv; c.cw = w.conv_wt; c.tail = conv_pool + (size_t)t_segs[0].slot * conv_slot_elems + w.cv_off; }
                     launch_lay_step_in({L.X, padd.y, padd.wsel, w.norm1, w.norm1_off, L.X2, padd.nsum, L.mult, w.norm1_alpha},
-                                       {g.W, g.bias, g.C, g.n_used ? g.n_used : g.N, g.act, g.act2, g.act_split, g.act_param}, W, s);
+                                       {g.W, g.bias, g.C, g.n_used ? g.n_used : g.N, g.act, g.act2, g.act_split, g.act_param}, c, W, s);
                     padd.y = nullptr; padd.wsel = nullptr;
                 } else {
                     add_norm(w.norm1, w.norm1_off, w.norm1_alpha, L.Hc, lay_on_tiles(L, T, g.N, W));
@@ -2029,7 +2036,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     c.dims = sp.rot.dims; c.half = sp.rot.half; c.freq = w.rot_freq; c.mag = w.rot_mag; c.unit = sp.unit_qk; c.eps = cfg.eps;
                     c.q = L.XB; c.ldq = H * d; c.kpool = kv_pool + w.k_pool_off; c.vpool = kv_pool + w.v_pool_off;
                     c.bt = d_bt; c.segs = d_segs; c.rowseg = d_rowseg; c.page = page; c.T = T; c.tail_too = all_decode;
-                    launch_lay_conv_qkv(c, kv_mode, s);
+                    if (prepared) {
+                        prep.on = true; prep.own = sp.kv_from < 0; prep.half = c.half; prep.unit = c.unit; prep.k_off = w.k_off; prep.v_off = w.v_off;
+                        prep.dims = c.freq ? c.dims : 0; prep.freq = c.freq; prep.mag = c.mag; prep.eps = c.eps; prep.seg = t_segs[0];
+                    } else launch_lay_conv_qkv(c, kv_mode, s);
                     if (!all_decode && sp.conv > 1) {
                         LConvArgs& t = late_tail;
                         t.src = L.P; t.lds = w.in_rows; t.off = w.q_off; t.C = w.g_off; t.dst = nullptr; t.ldd = 0; t.cw = nullptr; t.cb = nullptr;
@@ -2040,8 +2050,10 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     }
                     keep_shares = one_row;
                     left.nsplit = 1;
-                    run_attention(sp, w, L.XB, H * d, 0, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows, rounded);
+                    if (prepared) run_attention(sp, w, L.P, w.in_rows, w.q_off, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows, rounded);
+                    else run_attention(sp, w, L.XB, H * d, 0, 0, d, e, nullptr, 0, 1.f, 1, L.P + w.g_off, w.in_rows, rounded);
                     keep_shares = false;
+                    prep.on = false;
                     on = H * e; oa16 = o16;
                 } else if (sp.mixer == LMIX_ATTN) {
                     // two maps per head as heads of their own (2 H query heads over 2 G key heads, pairs of key heads share a value head)
