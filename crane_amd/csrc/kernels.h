@@ -65,6 +65,7 @@ struct AttnDecArgs {
     void* vpool;
     float* part_o;               // [Hq][nsplit][D]
     float* part_ml;              // [Hq][nsplit][2]
+    int32_t* done = nullptr;     // attn_decode_group_kernel: [sequences][Hkv] shares that have arrived, zero before and after
     float* out1 = nullptr;       // ONE token split per sequence (launch_attn_decode*: nsplit == 1): the kernel normalises (and gates) itself and
     int out1_stride = 0;         //   writes out1[seq * out1_stride + h * D + d] -- no partials, no combine launch
     uint16_t* out1_hi = nullptr; //   ... or, when set by this kernel or, with several splits, by the combine kernel, as bf16 hi + lo planes [seq][out1_cols]: the A

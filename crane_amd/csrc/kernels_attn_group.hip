@@ -11,10 +11,10 @@
 //
 // What bounds it: the chain of one wave -- page number, keys, scores, exponentials, weights, values -- and not the bytes.  So a wave takes 64 tokens at a time
 // (16 in attn_decode_mfma_kernel: four times the chains), requests the next tile's keys as soon as this one's are multiplied, and every wave of
-// the block has tiles of its own; they meet in LDS once.  A sequence whole in a block needs no partial sums in memory and no launch that merges
-// them.  The loops over the scores are rolled: unrolled, sixteen expf are longer to fetch than to run.  The key head is the fastest grid dimension: with the
+// the block has tiles of its own; they meet in LDS once.  A sequence whole in a block needs no partial sums in memory; the shares
+// of one are merged by the block that arrives last (a launch for that: 4.2 us and its gap; 20 sequences up to 700 tokens, three shares: 19.5 us a layer, 15.9 in one).  The loops over the scores are rolled: unrolled, sixteen expf are longer to fetch than to run.  The key head is the fastest grid dimension: with the
 // share there, the shares that short sequences don't have fall on the same XCDs (20 sequences up to 700 tokens, 4 shares: 22.1 us for 17.1).
-// Measured (us, with merging launches; attn_decode_split_kernel / attn_decode_mfma_kernel / here; 32 query heads on 8, lengths spread up to the longest; error
+// Measured (us, with the merging launches there were; attn_decode_split_kernel / attn_decode_mfma_kernel / here; 32 query heads on 8, lengths spread up to the longest; error
 // against 64 bits 2.0e-7 / 3.2e-7 / 2.1e-7): 8 sequences up to 1000 tokens 16.9 / 14.7 / 12.6; 20 up to 700 30.8 / 20.1 / 17.1; 32 up to 1000 50.4 / 28.1 /
 // 24.0; 64 up to 500 48.7 / 25.6 / 23.0; 128 up to 4000 443 / 249 / 213 (4.9 TB/s).  Three products per tile instead of one with the parts side by side: 20.2
 // and 27.4 at the second and third; blocks of eight waves: 17.4 and 24.5, 212 and more at the last.
@@ -53,6 +53,52 @@ __device__ __forceinline__ float q8_scale(float am, float& id) {
     const float dq = am / 127.0f;
     id = dq != 0.f ? 1.0f / dq : 0.f;
     return (float)(_Float16)dq;
+}
+
+// sums that another XCD's block reads: written through to where all of them read, and read from there, so that their counter needs no fence (a fence writes back
+// and drops a whole L2)
+__device__ __forceinline__ void put_through(float* p, float x, float y) {
+    __hip_atomic_store((unsigned long long*)p, (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 get_through(const float* p) {
+    const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
+}
+// the shares of a sequence's head merged by one wave, two columns per lane, always in their order
+__device__ __forceinline__ void merge_head(const AttnDecArgs& a, int bq, int h, int nh, int nsplit, int shares, int lane) {
+    constexpr int AT = 8;                                         // shares requested at once
+    const size_t p0 = ((size_t)bq * nh + h) * nsplit;
+    const float* po = a.part_o + p0 * D + 2 * lane;
+    float2 v[AT];
+#pragma unroll
+    for (int k = 0; k < AT; ++k) v[k] = get_through(po + (size_t)min(k, shares - 1) * D);
+    const float2 ml = get_through(a.part_ml + (p0 + min(lane, shares - 1)) * 2);      // (at most 64 shares)
+    const float M = wave_max(ml.x), w = lane < shares ? expf(ml.x - M) : 0.f;
+    const float inv = 1.0f / wave_sum(w * ml.y);
+    float x = 0.f, y = 0.f;
+    for (int k0 = 0; k0 < shares; k0 += AT) {
+#pragma unroll
+        for (int k = 0; k < AT; ++k) {
+            const float wk = __shfl(w, min(k0 + k, 63));          // 0 behind the last share
+            x = fmaf(wk, v[k].x, x); y = fmaf(wk, v[k].y, y);
+        }
+        if (k0 + AT < shares) {
+#pragma unroll
+            for (int k = 0; k < AT; ++k) v[k] = get_through(po + (size_t)min(k0 + AT + k, shares - 1) * D);
+        }
+    }
+    x *= inv; y *= inv;
+    const int col = h * D + 2 * lane;
+    if (a.gate) {
+        const float2 g = *(const float2*)(a.gate + (size_t)bq * a.qkv_stride + col);
+        x *= 1.0f / (1.0f + expf(-g.x)); y *= 1.0f / (1.0f + expf(-g.y));
+    }
+    put_pair(a, bq, col, x, y);
+    if (!a.out1_q) return;
+    float id;
+    const float dq = q8_scale(row16_max(fmaxf(fabsf(x), fabsf(y))), id);      // 16 lanes: 32 columns
+    *(uint16_t*)(a.out1_q + (size_t)bq * a.out1_cols + col) = (uint16_t)(((uint32_t)(int)roundf(x * id) & 0xFFu) | (((uint32_t)(int)roundf(y * id) & 0xFFu) << 8));
+    if ((lane & 15) == 0) a.out1_qd[(size_t)(col >> 5) * QGEMM_MAXM + bq] = dq;
 }
 
 template <int NREP, int KVT>
@@ -107,29 +153,38 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
     // ---- the heads' queries (norm, rotation, 1 / sqrt(D), three parts), this step's key and value (the owner appends them).  Everything they need is
     // requested in front of the first tile: answers come in order, so none of it waits for the tile
     constexpr int IT = (NREP + 2 + DW - 1) / DW;
-    float x0[IT], x1[IT], n0[IT], n1[IT];
+    float x0[IT], x1[IT], n0[IT], n1[IT], p0[IT][7], p1[IT][7];
     const float c = a.cos[(size_t)rpos * 64 + lane], sn = a.sin[(size_t)rpos * 64 + lane];
+    auto source = [&](int item) __attribute__((always_inline)) { return qkv + (item < NREP ? a.q_off + (kvh * NREP + item) * D : (item == NREP ? a.k_off : a.v_off) + kvh * D); };
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
         const int item = min(wave + k * DW, NREP + 1);
-        const float* src = qkv + (item < NREP ? a.q_off + (kvh * NREP + item) * D : (item == NREP ? a.k_off : a.v_off) + kvh * D);
+        const float* src = source(item);
         const float* nw = item < NREP ? a.qnw : item == NREP ? a.knw : nullptr;
         x0[k] = src[lane]; x1[k] = src[lane + 64];
         n0[k] = nw ? nw[lane] : 1.f; n1[k] = nw ? nw[lane + 64] : 1.f;
-        if (a.qkv_ns > 1) {                                       // slices of a product whose depth is split (2 .. 8), added in their order; all loads first
-            float p0[7], p1[7];
+    }
+    if (a.qkv_ns > 1) {                                           // slices of a product whose depth is split (2 .. 8), added in their order below
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            const float* src = source(min(wave + k * DW, NREP + 1));
 #pragma unroll
             for (int sl = 1; sl < 8; ++sl) {
                 const float* ps = src + (size_t)(sl < a.qkv_ns ? sl : 0) * a.qkv_slice;
-                p0[sl - 1] = ps[lane]; p1[sl - 1] = ps[lane + 64];
+                p0[k][sl - 1] = ps[lane]; p1[k][sl - 1] = ps[lane + 64];
             }
-#pragma unroll
-            for (int sl = 1; sl < 8; ++sl)
-                if (sl < a.qkv_ns) { x0[k] += p0[sl - 1]; x1[k] += p1[sl - 1]; }
         }
     }
     fetch_k(0);
     fetch_v(0);
+    // (the sums behind every request: with an item's in front of the next one's the first keys were asked for two trips to memory later)
+    if (a.qkv_ns > 1) {
+#pragma unroll
+        for (int k = 0; k < IT; ++k)
+#pragma unroll
+            for (int sl = 1; sl < 8; ++sl)
+                if (sl < a.qkv_ns) { x0[k] += p0[k][sl - 1]; x1[k] += p1[k][sl - 1]; }
+    }
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
         const int item = wave + k * DW;
@@ -283,12 +338,12 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
         red_w[wave][lr] = w; red_l[wave][lr] = w * l;
     }
     __syncthreads();
-    if (lr >= NREP) return;
+    if (shares == 1 && lr >= NREP) return;
 #pragma unroll
     for (int k = 0; k < DW; ++k) { cw[k] = red_w[k][lr]; L += red_l[k][lr]; }
     const int hq = kvh * NREP + lr;
     const float inv = shares == 1 ? 1.0f / L : 1.f;
-    for (int b = wave; b < NNT / 2; b += DW) {                    // 32 columns: two tiles of sixteen
+    for (int b = wave; b < NNT / 2 && lr < NREP; b += DW) {       // 32 columns: two tiles of sixteen
         f32x4 v[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -305,8 +360,10 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
         if (shares > 1) {
             const size_t ph = ((size_t)bq * a.Hkv * NREP + hq) * nsplit + split;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) *(f32x4*)(a.part_o + ph * D + (b * 2 + j) * 16 + lg * 4) = v[j];
-            if (b == 0 && lg == 0) { a.part_ml[ph * 2] = M; a.part_ml[ph * 2 + 1] = L; }
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) put_through(a.part_o + ph * D + (b * 2 + j) * 16 + lg * 4 + r, v[j][r], v[j][r + 1]);
+            if (b == 0 && lg == 0) put_through(a.part_ml + ph * 2, M, L);
             continue;
         }
         float am = 0.f;
@@ -336,46 +393,17 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
         }
         if (lg == 0) a.out1_qd[(size_t)(hq * (D / 32) + b) * QGEMM_MAXM + bq] = dq;
     }
-}
-
-// the shares of a sequence merged: a wave per (sequence, head), two columns per lane.  Sequences whole in one block are done already
-__global__ __launch_bounds__(256) void attn_group_merge_kernel(AttnDecArgs a, int nsplit, int nh) {
-    constexpr int AT = 8;                                         // shares requested at once
-    const int lane = threadIdx.x & 63, h = blockIdx.x * 4 + (int)(threadIdx.x >> 6), bq = blockIdx.y;
-    const int shares = min(nsplit, (a.st[bq].pos / KT + DW) / DW);
-    if (h >= nh || shares == 1) return;
-    const size_t p0 = ((size_t)bq * nh + h) * nsplit;
-    const float* po = a.part_o + p0 * D + 2 * lane;
-    float2 v[AT];
-#pragma unroll
-    for (int k = 0; k < AT; ++k) v[k] = *(const float2*)(po + (size_t)min(k, shares - 1) * D);
-    const float2 ml = *(const float2*)(a.part_ml + (p0 + min(lane, shares - 1)) * 2);      // (at most 64 shares)
-    const float M = wave_max(ml.x), w = lane < shares ? expf(ml.x - M) : 0.f;
-    const float inv = 1.0f / wave_sum(w * ml.y);
-    float x = 0.f, y = 0.f;
-    for (int k0 = 0; k0 < shares; k0 += AT) {
-#pragma unroll
-        for (int k = 0; k < AT; ++k) {
-            const float wk = __shfl(w, min(k0 + k, 63));          // 0 behind the last share
-            x = fmaf(wk, v[k].x, x); y = fmaf(wk, v[k].y, y);
-        }
-        if (k0 + AT < shares) {
-#pragma unroll
-            for (int k = 0; k < AT; ++k) v[k] = *(const float2*)(po + (size_t)min(k0 + AT + k, shares - 1) * D);
-        }
-    }
-    x *= inv; y *= inv;
-    const int col = h * D + 2 * lane;
-    if (a.gate) {
-        const float2 g = *(const float2*)(a.gate + (size_t)bq * a.qkv_stride + col);
-        x *= 1.0f / (1.0f + expf(-g.x)); y *= 1.0f / (1.0f + expf(-g.y));
-    }
-    put_pair(a, bq, col, x, y);
-    if (!a.out1_q) return;
-    float id;
-    const float dq = q8_scale(row16_max(fmaxf(fabsf(x), fabsf(y))), id);      // 16 lanes: 32 columns
-    *(uint16_t*)(a.out1_q + (size_t)bq * a.out1_cols + col) = (uint16_t)(((uint32_t)(int)roundf(x * id) & 0xFFu) | (((uint32_t)(int)roundf(y * id) & 0xFFu) << 8));
-    if ((lane & 15) == 0) a.out1_qd[(size_t)(col >> 5) * QGEMM_MAXM + bq] = dq;
+    if (shares == 1) return;
+    // the last share to arrive merges them (a launch for it: 4 us and the gap in front of it)
+    __shared__ int last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int32_t* done = a.done + (size_t)bq * a.Hkv + kvh;
+    if (threadIdx.x == 0) last = atomicAdd(done, 1) == shares - 1;
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) *done = 0;
+    for (int k = wave; k < NREP; k += DW) merge_head(a, bq, kvh * NREP + k, a.Hkv * NREP, nsplit, shares, lane);
 }
 
 template <int NREP, int KVT>
@@ -385,7 +413,6 @@ void go(const AttnDecArgs& a, int nsplit, int n_seq, hipStream_t s) {
     static DevOnce attr;
     attr.run([&] { (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_decode_group_kernel<NREP, KVT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
     hipLaunchKernelGGL((attn_decode_group_kernel<NREP, KVT>), dim3((unsigned)a.Hkv, (unsigned)n_seq, (unsigned)nsplit), dim3(DW * 64), lds, s, a);
-    if (nsplit > 1) hipLaunchKernelGGL(attn_group_merge_kernel, dim3((unsigned)((a.Hkv * NREP + 3) / 4), (unsigned)n_seq), dim3(256), 0, s, a, nsplit, a.Hkv * NREP);
 }
 }  // namespace
 
@@ -395,7 +422,8 @@ bool attn_decode_group_fits(int head_dim, int nrep, int kv_mode, int page, int r
 }
 
 // Whether a group is this kernel's.  For it: every wave has 64 tokens, so few launches' blocks are short of work; the slices of a split qkv product are added here, a
-// launch less.  Against it: parts for four heads whatever NREP is, and a merging launch (4 us) where a sequence is more than four tiles.  us a layer (width 1024, 32 query
+// launch less.  Against it: parts for four heads whatever NREP is, and the merging (a launch of 4 us when these were measured, about 2 inside the
+// kernel now) where a sequence is more than four tiles.  us a layer (width 1024, 32 query
 // heads on 8 unless said; qkv product, attention, o_proj, feed-forward), older kernels / this one, lengths spread up to the longest:
 //   slices to add: 9 sequences up to 300 / 700 / 4000 tokens 50.4 / 48.2, 54.9 / 47.9, 64.2 / 59.5; 16 up to 400 54.5 / 48.5; 8 heads on 2, 9 up to 200 / 1000 / 4000
 //     42.2 / 38.4, 44.7 / 43.7, 48.6 / 47.9, 16 up to 300 45.0 / 44.2; 4 on 1, 33 up to 300 45.1 / 45.2; 16 on 8, 9 up to 200 / 300 / 400 44.0 / 42.2, 45.1 / 46.0, 45.7 / 45.7,
@@ -412,7 +440,8 @@ bool attn_decode_group_pays(int pairs, int nrep, int64_t longest, bool slices, i
 }
 
 // shares of a sequence, given the tokens of the longest and the (sequence, key head) pairs: a tile per wave, as far as that makes two blocks per CU; pairs that
-// fill the chip by themselves are taken whole, and half as many where two shares would do (a launch that merges is 4 us).  us, 1 / 2 / 3 / 4 / 8 shares:
+// fill the chip by themselves are taken whole, and half as many where two shares would do (32 sequences up to 1000 tokens in 1 / 2 / 4 shares merged by the last: 24.6 / 25.6 / 27.3 us:
+// all blocks ask for their first tiles at once, and the memory takes as long for them either way).  us with merging launches, 1 / 2 / 3 / 4 / 8 shares:
 // 8 sequences up to 1000 tokens 19.6 / 16.3 / 16.5 / 12.6 / -, up to 4000 58.7 / 37.7 / 31.1 / 26.0 / 25.8; 20 up to 500 14.4 / 15.3, up to 700 17.8 / 17.7 /
 // 17.1, up to 1000 22.2 / 24.5 / 21.8 / 19.6, up to 4000 61.7 / 63.1 / 50.8 / 53.5 / 51.1; 32 up to 2000 38.7 / 43.3 / 43.0 / 42.2 / 41.8 -- lengths spread evenly.
 // One long context beside short ones (100 tokens) would like more: us a layer, the kernels that single sequences use / 1 / 2 / 4 / 8 / 16 shares, 32 sequences with one of 1000

@@ -276,6 +276,7 @@ struct Model {
     int32_t* d_btb = nullptr;          // device [MAXB][max_pages_per_seq]
     int32_t* h_btb = nullptr;          // pinned
     float *xb = nullptr, *qkvb = nullptr, *attnb = nullptr, *hbb = nullptr, *logitsb = nullptr, *part_ob = nullptr, *part_mlb = nullptr, *pmaxb = nullptr;
+    int32_t* attn_done = nullptr;      // [MAXB][Hkv_l] shares of a decode group's attention that have arrived (attn_decode_group_kernel leaves zeros)
     int* pidxb = nullptr;
     int ldq = 0;
     void ensure_batch_buffers();
