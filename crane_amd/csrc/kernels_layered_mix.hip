@@ -401,10 +401,9 @@ struct LcqPair {
         }
     }
     // fresh: the first row of this thread's walk or of a portion
-    __device__ __forceinline__ float2 row(const LConvQkvArgs& a, const LaySegDev& sg, int local, bool fresh) {
+    __device__ __forceinline__ float2 row(const LConvQkvArgs& a, const LaySegDev& sg, int local, bool fresh, float2 now) {
         float2 acc = make_float2(0.f, 0.f);
         if (ROLL) {
-            const float2 now = fetch(a, sg, local);
             if (fresh) {
 #pragma unroll
                 for (int j = 0; j < LCQ_TAPS - 1; ++j) win[j] = j >= LCQ_TAPS - a.taps ? fetch(a, sg, local - (LCQ_TAPS - 1) + j) : make_float2(0.f, 0.f);
@@ -453,26 +452,48 @@ __device__ __forceinline__ void lcq_store(void* pool, size_t at, int i0, int i1,
         else { p[i0] = f32_to_bf16(v0); if (i1 >= 0) p[i1] = f32_to_bf16(v1); }
     }
 }
-// PPL: pairs per lane.  wide: d, e and every offset and stride are even
-template <int KVT, int PPL, bool ROLL>
-__global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int nqk, int L, int rpb, bool wide) {
-    const int tid = threadIdx.x, r0 = blockIdx.x * rpb, r1 = min(r0 + rpb, a.T);
+// cosine and sine, times the layer's factor, of every row's position and rotated pair: once per pass, for all layers and heads that turn alike
+__global__ __launch_bounds__(256) void lay_angles_kernel(const float* __restrict__ freq, float mag, int pairs, const LaySegDev* __restrict__ segs,
+                                                         const int32_t* __restrict__ rowseg, float2* __restrict__ out, int T) {
+    const int i = blockIdx.x * 256 + threadIdx.x, r = i / pairs, p = i - r * pairs;
+    if (r >= T) return;
+    const LaySegDev sg = segs[rowseg[r]];
+    float sn, cs;
+    sincosf((float)(sg.start_pos + r - sg.row0) * freq[p], &sn, &cs);
+    out[i] = make_float2(cs * mag, sn * mag);
+}
+void launch_lay_angles(const float* freq, float mag, int pairs, const LaySegDev* segs, const int32_t* rowseg, float2* out, int T, hipStream_t s) {
+    if (T <= 0 || pairs <= 0) return;
+    hipLaunchKernelGGL(lay_angles_kernel, dim3((unsigned)(((size_t)T * pairs + 255) / 256)), dim3(256), 0, s, freq, mag, pairs, segs, rowseg, out, T);
+}
+// PPL: pairs per lane.  RPB: rows of a block, whose inputs are requested together.  wide: d, e and every offset and stride are even
+template <int KVT, int PPL, bool ROLL, int RPB>
+__global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int nqk, int L, bool wide) {
+    const int tid = threadIdx.x, r0 = blockIdx.x * RPB;
     const int C = (a.H + a.G) * a.d + a.G * a.e;
-    int seg = -1;
-    LaySegDev sg{};
+    int sn[RPB];
+    LaySegDev sgs[RPB];
+#pragma unroll
+    for (int k = 0; k < RPB; ++k) sn[k] = a.rowseg[min(r0 + k, a.T - 1)];
+#pragma unroll
+    for (int k = 0; k < RPB; ++k) sgs[k] = a.segs[sn[k]];
     if ((int)blockIdx.y >= nqk) {          // values
         const int i0 = (((int)blockIdx.y - nqk) * 256 + tid) * 2, n = a.G * a.e;
         if (i0 >= n) return;
         const int i1 = i0 + 1 < n ? i0 + 1 : -1, base = (a.H + a.G) * a.d;
         LcqPair<ROLL> pr;
         pr.init(a, base + i0, i1 >= 0 ? base + i1 : -1, C, wide);
+        float2 now[RPB];
+#pragma unroll
+        for (int k = 0; k < RPB; ++k) now[k] = ROLL ? pr.fetch(a, sgs[k], min(r0 + k, a.T - 1) - sgs[k].row0) : make_float2(0.f, 0.f);
         const int g0 = i0 / a.e, g1 = i1 >= 0 ? i1 / a.e : g0;
-        for (int r = r0; r < r1; ++r) {
-            const int sn = a.rowseg[r];
-            const bool fresh = sn != seg;
-            if (fresh) { sg = a.segs[sn]; seg = sn; }
+#pragma unroll
+        for (int k = 0; k < RPB; ++k) {
+            const int r = r0 + k;
+            if (r >= a.T) break;
+            const LaySegDev& sg = sgs[k];
             const int local = r - sg.row0, pos = sg.start_pos + local;
-            const float2 v = pr.row(a, sg, local, fresh);
+            const float2 v = pr.row(a, sg, local, k == 0 || sn[k] != sn[k > 0 ? k - 1 : 0], now[k]);
             if (a.tail_too) pr.shift_tail(a, sg);
             const size_t row = (size_t)a.bt[sg.bt_off + pos / a.page] * a.G * a.page + (size_t)(pos % a.page);
             const size_t at0 = (row + (size_t)g0 * a.page) * a.e;
@@ -490,31 +511,41 @@ __global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int n
     const int hd = a.dims / 2, np = hd + (a.d - a.dims + 1) / 2;
     LcqPair<ROLL> pr[PPL];
     int e0[PPL], e1[PPL]; float fr[PPL];
+    float2 now[PPL][RPB], turn[PPL][RPB];
 #pragma unroll
     for (int p = 0; p < PPL; ++p) {        // a rotated pair, or two neighbours behind the rotated part (the last one may be alone)
         const int i = ln + p * L;
         e0[p] = e1[p] = -1; fr[p] = 0.f;
         if (live && i < np) {
-            if (i < hd) { e0[p] = a.half ? i : 2 * i; e1[p] = a.half ? i + hd : 2 * i + 1; fr[p] = a.freq[i]; }
+            if (i < hd) { e0[p] = a.half ? i : 2 * i; e1[p] = a.half ? i + hd : 2 * i + 1; if (!a.angles) fr[p] = a.freq[i]; }
             else { e0[p] = a.dims + 2 * (i - hd); e1[p] = e0[p] + 1 < a.d ? e0[p] + 1 : -1; }
         }
         pr[p].init(a, e0[p] >= 0 ? hv * a.d + e0[p] : -1, e1[p] >= 0 ? hv * a.d + e1[p] : -1, C, wide);
+#pragma unroll
+        for (int k = 0; k < RPB; ++k) {
+            const int r = min(r0 + k, a.T - 1);
+            now[p][k] = ROLL ? pr[p].fetch(a, sgs[k], r - sgs[k].row0) : make_float2(0.f, 0.f);
+            turn[p][k] = a.angles && i < hd ? a.angles[(size_t)r * hd + i] : make_float2(1.f, 0.f);
+        }
     }
-    for (int r = r0; r < r1; ++r) {
-        const int sn = a.rowseg[r];
-        const bool fresh = sn != seg;
-        if (fresh) { sg = a.segs[sn]; seg = sn; }
+#pragma unroll
+    for (int k = 0; k < RPB; ++k) {
+        const int r = r0 + k;
+        if (r >= a.T) break;
+        const LaySegDev& sg = sgs[k];
         const int local = r - sg.row0, pos = sg.start_pos + local;
         float2 v[PPL];
         float ss = 0.f;
 #pragma unroll
         for (int p = 0; p < PPL; ++p) {
-            v[p] = pr[p].row(a, sg, local, fresh);
+            v[p] = pr[p].row(a, sg, local, k == 0 || sn[k] != sn[k > 0 ? k - 1 : 0], now[p][k]);
             if (a.tail_too) pr[p].shift_tail(a, sg);
             if (ln + p * L < hd) {
-                float sn_, cs;
-                sincosf((float)pos * fr[p], &sn_, &cs);
-                sn_ *= a.mag; cs *= a.mag;
+                float cs = turn[p][k].x, sn_ = turn[p][k].y;
+                if (!a.angles) {
+                    sincosf((float)pos * fr[p], &sn_, &cs);
+                    sn_ *= a.mag; cs *= a.mag;
+                }
                 v[p] = lay_turn(v[p], cs, sn_);
             }
             ss = fmaf(v[p].x, v[p].x, ss); ss = fmaf(v[p].y, v[p].y, ss);
@@ -536,18 +567,17 @@ __global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int n
 template <int KVT>
 static void lay_conv_qkv_go(const LConvQkvArgs& a, dim3 grid, int nqk, int L, int ppl, int rpb, bool wide, hipStream_t s) {
     const bool roll = a.taps <= LCQ_TAPS;
-    if (ppl <= 1) {
-        if (roll) hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 1, true>), grid, dim3(256), 0, s, a, nqk, L, rpb, wide);
-        else hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 1, false>), grid, dim3(256), 0, s, a, nqk, L, rpb, wide);
-    } else if (ppl <= 2) {
-        if (roll) hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 2, true>), grid, dim3(256), 0, s, a, nqk, L, rpb, wide);
-        else hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 2, false>), grid, dim3(256), 0, s, a, nqk, L, rpb, wide);
-    } else hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 8, false>), grid, dim3(256), 0, s, a, nqk, L, rpb, wide);
+#define CM_LCQ(PPL, ROLL) do { if (rpb == 1) hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, PPL, ROLL, 1>), grid, dim3(256), 0, s, a, nqk, L, wide); \
+                               else hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, PPL, ROLL, 4>), grid, dim3(256), 0, s, a, nqk, L, wide); } while (0)
+    if (ppl <= 1) { if (roll) CM_LCQ(1, true); else CM_LCQ(1, false); }
+    else if (ppl <= 2) { if (roll) CM_LCQ(2, true); else CM_LCQ(2, false); }
+    else hipLaunchKernelGGL((lay_conv_qkv_kernel<KVT, 8, false, 1>), grid, dim3(256), 0, s, a, nqk, L, wide);
+#undef CM_LCQ
 }
 void launch_lay_conv_qkv(const LConvQkvArgs& a0, int kvt, hipStream_t s) {
     if (a0.T <= 0 || a0.H <= 0 || a0.d > LAY_CONV_QKV_MAX_DIM || a0.taps < 1) return;      // the configuration reader has refused these
     LConvQkvArgs a = a0;
-    if (!a.freq) a.dims = 0;
+    if (!a.freq) { a.dims = 0; a.angles = nullptr; }
     const int np = a.dims / 2 + (a.d - a.dims + 1) / 2;
     int L = 1;
     while (L < np && L < 64) L <<= 1;
@@ -555,7 +585,7 @@ void launch_lay_conv_qkv(const LConvQkvArgs& a0, int kvt, hipStream_t s) {
     const int nqk = ((a.H + a.G) * L + 255) / 256, nv = (a.G * a.e + 511) / 512;
     // a block per row while all rows fit on the chip at once (2048 blocks of 256 threads; 300 rows of 12 heads of 128: 8.8 us against 15.5); more rows: the
     // window rolls over four
-    const int rpb = a.tail_too || a.T * (nqk + (a.G > 0 ? nv : 0)) <= 2048 ? 1 : 4;
+    const int rpb = a.tail_too || ppl > 2 || a.T * (nqk + (a.G > 0 ? nv : 0)) <= 2048 ? 1 : 4;
     const bool wide = !((size_t)a.d & 1) && !((size_t)a.e & 1) && !(((size_t)a.lds | (size_t)a.off | (size_t)a.ldq | a.slot_stride | a.cv_off) & 1);
     const dim3 grid((unsigned)((a.T + rpb - 1) / rpb), (unsigned)(nqk + (a.G > 0 ? nv : 0)));
     if (kvt == KV_F32) lay_conv_qkv_go<KV_F32>(a, grid, nqk, L, ppl, rpb, wide, s);

@@ -145,6 +145,7 @@ struct LayeredLayerW {
     float *dq_norm = nullptr, *dkv_norm = nullptr;   // latent attention: plain norm weights of the two latents
     uint16_t *uq = nullptr, *uk_t = nullptr, *uv = nullptr;   // [H (d + rot)][q_rank]; per head [kv_rank][d] (transposed); [H e][kv_rank]
     float* rot_freq = nullptr; float rot_mag = 1.f;  // [rot.dims / 2] angle per position; factor on cos and sin
+    int rot_id = -1;                                 // which of the model's angle tables (Layered::rots), if any
     uint16_t* a2 = nullptr; float* a2_b = nullptr;   // gated linear attention: [H d][rank], [H d]
     size_t v_pool_off = 0, v_page_bytes = 0;         // value pages (layers whose values are not their keys)
     size_t sh_off = 0;                               // the shift's previous input inside a slot of the conv pool (floats)
@@ -427,6 +428,7 @@ struct LConvQkvArgs {
     const float* cw; int taps;                       // [taps][channels], the last row the current token's
     float* conv_pool; size_t slot_stride, cv_off;    // tails [taps - 1][channels], oldest first
     int dims; int half; const float* freq; float mag;    // rotation (freq null: none), as lay_rope
+    const float2* angles = nullptr;                  // [T][dims / 2] cosine and sine times mag of this pass's rows (launch_lay_angles); null: made here
     int unit; float eps;
     float* q; int ldq;                               // [T][H d]
     void *kpool, *vpool;                             // [n_pages][G][page][d] / [e]
@@ -436,6 +438,7 @@ struct LConvQkvArgs {
 };
 constexpr int LAY_CONV_QKV_MAX_DIM = 1024;           // largest d
 void launch_lay_conv_qkv(const LConvQkvArgs& a, int kvt, hipStream_t s);
+void launch_lay_angles(const float* freq, float mag, int pairs, const LaySegDev* segs, const int32_t* rowseg, float2* out, int T, hipStream_t s);
 // x[r] += sum_(k < nsum) y[(r nsum + k) W ..] (y null: nothing is added; wsel given: row k times wsel[r nsum + k]), then out[r] =
 // x[rows ? rows[r] : r] in `groups` equal consecutive parts, each over its own root mean square, times w (out null: the update alone).
 // rows and y exclude each other.

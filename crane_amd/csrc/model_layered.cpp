@@ -80,6 +80,10 @@ struct Layered {
     static constexpr int ATT_PARTS = 512;   // (query tile, key head, split) blocks of a split-key attention launch
     float *att_po = nullptr, *att_pml = nullptr;
     float* am_pv = nullptr; int* am_pi = nullptr;   // arg-max partials of the logits rows
+    // tables of a pass's cosines and sines, one for each distinct rotation of the layers (up to ROTS; the others make their own in every launch)
+    static constexpr size_t ROTS = 4;
+    std::vector<std::pair<std::vector<float>, float>> rots;      // frequencies and factor
+    float2* angles = nullptr; int rot_pairs = 0;                 // [table][cap][rot_pairs]
     bool capture = false;              // cm_debug_set("lay_capture"): keep the residual stream after every layer of every pass
     std::vector<float> captured;
     ~Layered() {
@@ -1287,7 +1291,13 @@ static void build_gizezen(Model& m, LaySource& src) {
         w.in_w = up_bf16(m, in);
         w.o_w = up_bf16(m, src.get(q + "o", W * H * e, 1.0f / std::sqrt((float)(H * e)), 0.f));
         w.sink = up_f32(m, std::vector<float>(H, 0.f));       // one in the denominator: exp(0)
-        if (sp.rot.dims > 0) w.rot_freq = up_f32(m, rot_frequencies(sp.rot, &w.rot_mag));
+        if (sp.rot.dims > 0) {
+            const std::vector<float> f = rot_frequencies(sp.rot, &w.rot_mag);
+            w.rot_freq = up_f32(m, f);
+            const std::pair<std::vector<float>, float> key(f, w.rot_mag);
+            w.rot_id = (int)(std::find(L.rots.begin(), L.rots.end(), key) - L.rots.begin());
+            if ((size_t)w.rot_id == L.rots.size()) { if (L.rots.size() < Layered::ROTS) L.rots.push_back(key); else w.rot_id = -1; }
+        }
         if (sp.mlp == LMLP_NONE) continue;
         norm(p + "norm2", w.norm2, w.norm2_off, w.norm2_alpha);
         build_experts(m, src, p, sp, w);
@@ -1463,6 +1473,8 @@ void Model::alloc_runtime_layered() {
     L.Hn = dalloc<float>(cap * W);
     L.Hc = dalloc<float>(cap * W);
     L.Y = dalloc<float>(cap * W);
+    for (const auto& r : L.rots) L.rot_pairs = std::max(L.rot_pairs, (int)r.first.size());
+    if (!L.rots.empty()) L.angles = (float2*)dalloc<float>(L.rots.size() * cap * (size_t)L.rot_pairs * 2);
     L.P = dalloc<float>(cap * (size_t)L.max_in);
     L.O = dalloc<float>(cap * (size_t)L.max_o);
     L.O2 = dalloc<float>(cap * (size_t)L.max_o);
@@ -1779,6 +1791,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
         bool keep_shares = false;              // the next attention may leave its shares (in `left`) to the output projection
         LAttnArgs left;
         LAttnPrep prep;                        // the next attention's own preparation
+        bool turned[Layered::ROTS] = {};       // angle tables of this pass that are there
         auto run_attention = [&](const LayerSpec& sp, const LayeredLayerW& w, const float* qsrc, int ldq, int q_off, int g_off, int dk, int ev,
                                  float* out = nullptr, int ldo = 0, float out_scale = 1.f, int v_div = 1, const float* gbuf = nullptr, int ldg = 0,
                                  uint16_t* out16 = nullptr) {
@@ -2039,7 +2052,15 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     if (prepared) {
                         prep.on = true; prep.own = sp.kv_from < 0; prep.half = c.half; prep.unit = c.unit; prep.k_off = w.k_off; prep.v_off = w.v_off;
                         prep.dims = c.freq ? c.dims : 0; prep.freq = c.freq; prep.mag = c.mag; prep.eps = c.eps; prep.seg = t_segs[0];
-                    } else launch_lay_conv_qkv(c, kv_mode, s);
+                    } else {
+                        if (T > 1 && w.rot_id >= 0) {      // (a single row: a launch more than it saves)
+                            float2* at = L.angles + (size_t)w.rot_id * L.cap * L.rot_pairs;
+                            if (!turned[w.rot_id]) launch_lay_angles(w.rot_freq, w.rot_mag, sp.rot.dims / 2, d_segs, d_rowseg, at, T, s);
+                            turned[w.rot_id] = true;
+                            c.angles = at;
+                        }
+                        launch_lay_conv_qkv(c, kv_mode, s);
+                    }
                     if (!all_decode && sp.conv > 1) {
                         LConvArgs& t = late_tail;
                         t.src = L.P; t.lds = w.in_rows; t.off = w.q_off; t.C = w.g_off; t.dst = nullptr; t.ldd = 0; t.cw = nullptr; t.cb = nullptr;
