@@ -577,6 +577,8 @@ int cm_debug_lay_router_plan(int32_t rows, int32_t width, int32_t outputs, int32
     return cm::lay_router_decode_fits((const float*)at, (const uint16_t*)at, rows, width, outputs, top, rs);
 }
 
+int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats) { return cm::gemm_band(m, n, k, epi, (size_t)ws_floats, 0); }
+
 int cm_debug_attn_group_plan(int32_t pairs, int32_t nrep, int64_t longest, int32_t slices, int32_t num_cu, int32_t most) {
     return cm::attn_decode_group_pays(pairs, nrep, longest, slices != 0, num_cu) ? cm::attn_decode_group_split(longest, pairs, num_cu, most) : 0;
 }

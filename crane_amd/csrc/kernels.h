@@ -162,6 +162,8 @@ struct GemmArgs {
 // and the launch (a.ksplit set; more than one slice: partial tiles in a.ws)
 bool gemm_rows_plan(int M, int N, int K, size_t ws_floats, int* bn, int* ks);
 bool launch_gemm_rows(const GemmArgs& a, int epi, int bn, hipStream_t s);
+// prompt rows with hi + lo activations: how many of them a first launch takes where two cost less than one, 0 where they don't (host rule)
+int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap);
 
 // one sequence of a multi-sequence prompt pass (Model::prefill_multi): rows [row0, row0 + S) of the pass at positions start_pos...,
 // page table at block_table + bt_off

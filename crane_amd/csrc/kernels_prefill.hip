@@ -1222,51 +1222,58 @@ static void launch_splitk(GemmArgs& a, int epi, hipStream_t s) {
 // 256-row tiles with plain bf16) where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost
 // model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
 // register-staged kernel should run.
-static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
-    static const int env = getenv("CM_GEMM256") ? atoi(getenv("CM_GEMM256")) : 1;
+// the column tile and the K slices of such a product; false: not for that kernel
+static bool gemm256_plan(int M, int N, int K, bool lo, size_t ws_floats, bool w4, int* bn_out, int* ks_out) {
     static const int force_bn = getenv("CM_GEMM256_BN") ? atoi(getenv("CM_GEMM256_BN")) : 0;     // tuning
     static const int force_ks = getenv("CM_GEMM256_KS") ? atoi(getenv("CM_GEMM256_KS")) : 0;
-    // hi + lo: 128-row tiles, 64-row tiles up to 64 rows.  From 9 rows on (not 33): a decode round of 16 / 32 sequences 5.87 / 6.25 ->
-    // 5.41 / 5.82 ms against the 128-wide kernel + split-K (profiles/r06_small_group_gemm_ab.log); a 32-row tile variant measured no faster
-    // than the 64-row one (the launch is not bound by its MFMAs), 8 rows run on the batched GEMVs
-    static const int min_m2 = getenv("CM_GEMM256_MIN_M") ? atoi(getenv("CM_GEMM256_MIN_M")) : 9;
     static const int min_blocks = getenv("CM_GEMM256_MIN_BLOCKS") ? atoi(getenv("CM_GEMM256_MIN_BLOCKS")) : 128;
-    if (!env || !a.wide256 || a.wide256 == 4 || a.M < (a.A_lo ? min_m2 : 512) || a.K % 64 != 0) return false;
-    // the one-wave-per-SIMD kernel (kernels_gemmw4.hip) -- built, bit-compatible, measured 0 .. 4 % SLOWER than the ping-pong kernel
-    // on every prompt shape, so it is opt-in: CM_GEMMW4 = 1 from `w4_min` rows on, GemmArgs::wide256 = 2 (cm_debug_set "gemm256" = 2) always
-    static const int w4_env = getenv("CM_GEMMW4") ? atoi(getenv("CM_GEMMW4")) : 0;
-    static const int w4_min = getenv("CM_GEMMW4_MIN_M") ? atoi(getenv("CM_GEMMW4_MIN_M")) : 65;
-    const bool w4 = a.wide256 == 2 || (a.wide256 == 1 && w4_env != 0 && a.M >= w4_min);
-    const int bm = w4 ? gemmw4_rows(a.A_lo != nullptr) : gemm256_rows(a.A_lo != nullptr, a.M);
-    const int tiles_m = (a.M + bm - 1) / bm, nk = a.K / 64;
-    const double terms = a.A_lo ? 2.0 : 1.0;
+    const int bm = w4 ? gemmw4_rows(lo) : gemm256_rows(lo, M);
+    const int tiles_m = (M + bm - 1) / bm, nk = K / 64;
+    const double terms = lo ? 2.0 : 1.0;
     double best = 1e30;
     int best_bn = 0, best_ks = 1;
     for (int bn : {256, 192}) {
-        if (a.N % bn != 0 || (force_bn && bn != force_bn)) continue;
-        const int tiles = tiles_m * (a.N / bn);
+        if (N % bn != 0 || (force_bn && bn != force_bn)) continue;
+        const int tiles = tiles_m * (N / bn);
         for (int ks = 1; ks <= 8; ks *= 2) {
             if (force_ks && ks != force_ks) continue;
             if (nk % ks != 0 || nk / ks < 8) break;
-            if (ks > 1 && (a.ws == nullptr || (size_t)ks * a.M * a.N > a.ws_floats)) break;
+            if (ks > 1 && (size_t)ks * M * N > ws_floats) break;
             const int blocks = tiles * ks, rounds = (blocks + 255) / 256;
-            const double t_blk = (double)bm * bn * (double)(a.K / ks) * 2.0 * terms / 6.0e12;                   // ~60 % of a CU's MFMA peak
-            const double t_split = ks > 1 ? ((double)(2 * ks + 1) * a.M * a.N * 4.0) / 3.0e12 + 6e-6 : 0.0;   // partial tiles out and back + a launch
+            const double t_blk = (double)bm * bn * (double)(K / ks) * 2.0 * terms / 6.0e12;                   // ~60 % of a CU's MFMA peak
+            const double t_split = ks > 1 ? ((double)(2 * ks + 1) * M * N * 4.0) / 3.0e12 + 6e-6 : 0.0;   // partial tiles out and back + a launch
             const double t = rounds * t_blk + t_split;
             if (t < best) { best = t; best_bn = bn; best_ks = ks; }
         }
     }
     if (best_bn == 0) return false;
     // the chip must be reasonably full: otherwise the 128-row kernel's own split-K heuristics do better
-    const int blocks = tiles_m * (a.N / best_bn) * best_ks;
+    const int blocks = tiles_m * (N / best_bn) * best_ks;
     // (64-row tiles, measured at 48 / 64 rows: gate||up 60 -> 51 us, QKV 25 -> 22, but o_proj 16.3 -> 17.7 and down_proj equal -- the
     // projections of fewer than 24 column tiles stay on the 128-wide kernel)
-    if (bm == 64 && tiles_m * (a.N / best_bn) < 24 && !force_bn) return false;
-    if (blocks < (a.M >= 512 ? 192 : min_blocks) && !force_bn) return false;
-    a.ksplit = best_ks;
-    if (w4) { if (!launch_gemmw4(a, epi, best_bn, s)) return false; }
-    else if (!launch_gemm256(a, epi, best_bn, s)) return false;
-    if (best_ks > 1) launch_splitk(a, epi, s);
+    if (bm == 64 && tiles_m * (N / best_bn) < 24 && !force_bn) return false;
+    if (blocks < (M >= 512 ? 192 : min_blocks) && !force_bn) return false;
+    *bn_out = best_bn; *ks_out = best_ks;
+    return true;
+}
+static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
+    static const int env = getenv("CM_GEMM256") ? atoi(getenv("CM_GEMM256")) : 1;
+    // hi + lo: 128-row tiles, 64-row tiles up to 64 rows.  From 9 rows on (not 33): a decode round of 16 / 32 sequences 5.87 / 6.25 ->
+    // 5.41 / 5.82 ms against the 128-wide kernel + split-K (profiles/r06_small_group_gemm_ab.log); a 32-row tile variant measured no faster
+    // than the 64-row one (the launch is not bound by its MFMAs), 8 rows run on the batched GEMVs
+    static const int min_m2 = getenv("CM_GEMM256_MIN_M") ? atoi(getenv("CM_GEMM256_MIN_M")) : 9;
+    if (!env || !a.wide256 || a.wide256 == 4 || a.M < (a.A_lo ? min_m2 : 512) || a.K % 64 != 0) return false;
+    // the one-wave-per-SIMD kernel (kernels_gemmw4.hip) -- built, bit-compatible, measured 0 .. 4 % SLOWER than the ping-pong kernel
+    // on every prompt shape, so it is opt-in: CM_GEMMW4 = 1 from `w4_min` rows on, GemmArgs::wide256 = 2 (cm_debug_set "gemm256" = 2) always
+    static const int w4_env = getenv("CM_GEMMW4") ? atoi(getenv("CM_GEMMW4")) : 0;
+    static const int w4_min = getenv("CM_GEMMW4_MIN_M") ? atoi(getenv("CM_GEMMW4_MIN_M")) : 65;
+    const bool w4 = a.wide256 == 2 || (a.wide256 == 1 && w4_env != 0 && a.M >= w4_min);
+    int bn = 0, ks = 1;
+    if (!gemm256_plan(a.M, a.N, a.K, a.A_lo != nullptr, a.ws ? a.ws_floats : 0, w4, &bn, &ks)) return false;
+    a.ksplit = ks;
+    if (w4) { if (!launch_gemmw4(a, epi, bn, s)) return false; }
+    else if (!launch_gemm256(a, epi, bn, s)) return false;
+    if (ks > 1) launch_splitk(a, epi, s);
     return true;
 }
 
@@ -1284,6 +1291,12 @@ __global__ void silu_mul_split_kernel(const float* __restrict__ gu, uint16_t* __
 }
 
 static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s);
+static bool launch_gemm_once(GemmArgs& a, int epi, hipStream_t s);
+// the planes of a.norm_w's norm of C, where no reduction wrote them
+static void launch_gemm_norm(const GemmArgs& a, hipStream_t s) {
+    if (a.norm_b != nullptr) launch_layernorm_rows(a.C, a.norm_w, a.norm_b, a.norm_hi, a.norm_lo, a.M, a.N, a.norm_eps, s);
+    else launch_rmsnorm_rows(a.C, a.norm_w, a.norm_hi, a.norm_lo, a.M, a.N, a.norm_eps, s);
+}
 bool launch_gemm(const GemmArgs& a0, int epi, hipStream_t s) {
     if (a0.N % 128 != 0 || a0.K % GBK != 0) return false;
     GemmArgs a = a0;
@@ -1306,10 +1319,7 @@ bool launch_gemm(const GemmArgs& a0, int epi, hipStream_t s) {
     } else
     if (!launch_gemm_inner(a, epi, s)) return false;
     // the planes of RMSNorm(C) were not written by the split-K reduction (no split, or switched off): the row kernel
-    if (a.norm_w != nullptr) {
-        if (a.norm_b != nullptr) launch_layernorm_rows(a.C, a.norm_w, a.norm_b, a.norm_hi, a.norm_lo, a.M, a.N, a.norm_eps, s);
-        else launch_rmsnorm_rows(a.C, a.norm_w, a.norm_hi, a.norm_lo, a.M, a.N, a.norm_eps, s);
-    }
+    if (a.norm_w != nullptr) launch_gemm_norm(a, s);
     return true;
 }
 
@@ -1325,20 +1335,77 @@ static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     else if (ks > 1) launch_splitk(a, epi, s);
     return true;
 }
-static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s);
+static bool gemm_tail_columns(int M, int N) { return M >= 256 && N >= 512 && N % 192 != 0 && N % 256 == 128; }
 // Prompt rows over a width that no tile of kernels_gemm256.hip divides because of its last 128 columns (the merged in_proj of a Gated-Delta-Net layer:
 // 8192 columns and 32 gate columns padded to 128): the wide part there, the last columns alone.  8320 x 2048, 2048 rows: 180 -> 137 us (a prompt of
 // 2048 / 1024 / 300 tokens 18.6 / 10.8 / 5.54 -> 17.8 / 10.2 / 5.49 ms; width 1024: 12.3 / 7.3 / 4.5 -> 12.0 / 7.2 / 4.5)
 static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {
-    if (epi != GEPI_STORE || a.norm_w != nullptr || a.M < 256 || a.N < 512 || a.N % 192 == 0 || a.N % 256 != 128) return false;
+    if (epi != GEPI_STORE || a.norm_w != nullptr || !gemm_tail_columns(a.M, a.N)) return false;
     GemmArgs most = a, rest = a;
     most.N = a.N - 128;
     if (!try_gemm256(most, epi, s)) return false;
     rest.W = a.W + (size_t)most.N * a.K; rest.C = a.C + most.N; rest.N = 128;
     if (a.bias != nullptr) rest.bias = a.bias + most.N;
-    return launch_gemm_inner(rest, epi, s);
+    return launch_gemm_once(rest, epi, s);
 }
-static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) {
+// What M rows of a product with hi + lo activations take on the kernel that launch_gemm_once finds for them, in seconds: rounds of blocks, a 64-deep k-tile of 128 x 256 outputs
+// 1.44 us and about 13 us a block around them (measured / so: 24576 x 4096 at 300, 650, 1000, 1400 rows 164 / 164, 248 / 246, 313 / 315, 502 / 493 us); two blocks
+// of 128 x 128 on a CU 1.6 and 10; products of at most 128 rows by their weights
+static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
+    int bn = 0, ks = 0;
+    const auto split = [&](int cols) { return ks > 1 ? (double)(2 * ks + 1) * M * cols * 4.0 / 5e12 + 4e-6 : 0.0; };
+    if (epi != GEPI_ACT_SPLIT && gemm_rows_plan(M, N, K, ws_floats, &bn, &ks)) {
+        const int blocks = N / bn * ks;
+        return (double)N * K * 2.0 / (M <= 64 ? 4.6e12 : 3.4e12) * ((blocks + 255) / 256 * 256) / blocks + (ks > 1 ? 9e-6 : 4e-6);
+    }
+    const int tiles_m = (M + 127) / 128;
+    const bool tail = epi == GEPI_STORE && gemm_tail_columns(M, N);
+    const int cols = N - (tail ? 128 : 0);
+    if (gemm256_plan(M, cols, K, true, ws_floats, false, &bn, &ks))
+        return (tiles_m * (cols / bn) * ks + 255) / 256 * (K / 64 / ks * 1.44e-6 * bn / 256 + 13e-6) + split(cols) + (tail ? 15e-6 : 0.0);
+    ks = gemm_ksplit(M, N, tiles_m * (N / 128), K / GBK, ws_floats, ksplit_cap);
+    return (tiles_m * (N / 128) * ks + 511) / 512 * (K / 64 / ks * 1.6e-6 + 10e-6) + split(N);
+}
+// the rows of the first of two bands that take less time than all rows at once; 0: all at once
+int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
+    if (M <= 256 || N % 128 != 0 || K % 64 != 0 || epi == GEPI_ACT_SPLIT) return 0;
+    const double whole = gemm_seconds(M, N, K, epi, ws_floats, ksplit_cap);
+    double least = std::min(0.95 * whole, whole - 8e-6);
+    int rows = 0;
+    for (int m = (M - 9) / 128 * 128; m >= 128 && M - m <= 1024; m -= 128) {
+        const double t = gemm_seconds(m, N, K, epi, ws_floats, ksplit_cap) + gemm_seconds(M - m, N, K, epi, ws_floats, ksplit_cap) + 2e-6;
+        if (t < least) { least = t; rows = m; }
+    }
+    return rows;
+}
+// A round of blocks that the last tiles fill to a part takes as long as a full one: a band of rows whose tiles fill their rounds first, the rows behind it on
+// the kernel that suits so few.  What bounds either band is what bounded the whole; the second reads the weights again (24576 x 4096: 44 us of the memory's time
+// against a round of 105).  One launch / two, prompts on width 4096 with 36 layers: 300 tokens 12.8 / 11.8 ms, 520 20.0 / 18.2, 1200 38.1 / 33.6, 1400 44.2 / 37.6;
+// width 2048, 650: 7.5 / 7.1.  The line is a gain of 5 % and 8 us by the figures above: with 5 % alone the products of width 1024 lost (300 tokens 3.32 / 3.45
+// ms, 560 4.30 / 4.41: a launch and a reduction more for a round of 30 us).  Rows of products with an activation behind them and the vision tower's norm stay in one launch (not measured).
+static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
+    if (a.A_lo == nullptr || a.defer_ks != nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
+    const int m = gemm_band(a.M, a.N, a.K, epi, a.ws ? a.ws_floats : 0, a.ksplit_cap);
+    if (m == 0) return false;
+    const size_t hcols = epi == GEPI_SILUMUL ? (size_t)a.N / 2 : (size_t)a.N;
+    for (int part = 0; part < 2; ++part) {
+        const size_t r0 = part ? (size_t)m : 0;
+        GemmArgs b = a;
+        b.M = part ? a.M - m : m;
+        b.A_hi += r0 * a.K; b.A_lo += r0 * a.K;
+        if (a.C) b.C += r0 * a.ldc;
+        if (a.H_hi) b.H_hi += r0 * hcols;
+        if (a.H_lo) b.H_lo += r0 * hcols;
+        if (a.norm_hi) b.norm_hi += r0 * a.N;
+        if (a.norm_lo) b.norm_lo += r0 * a.N;
+        if (!launch_gemm_once(b, epi, s)) return false;
+        if (b.norm_w != nullptr) launch_gemm_norm(b, s);
+    }
+    a.norm_w = nullptr;
+    return true;
+}
+static bool launch_gemm_inner(GemmArgs& a, int epi, hipStream_t s) { return try_gemm_bands(a, epi, s) || launch_gemm_once(a, epi, s); }
+static bool launch_gemm_once(GemmArgs& a, int epi, hipStream_t s) {
     if (try_gemm_tail(a, epi, s) || try_gemm_rows(a, epi, s) || try_gemm256(a, epi, s)) return true;
     const int tiles_m = (a.M + GBM - 1) / GBM;
     const bool split = a.A_lo != nullptr;

@@ -541,6 +541,9 @@ int cm_debug_lay_tile_plan(int32_t tokens, int32_t columns, int32_t experts, int
  * has `beside` columns (0: none); negative: the columns behind the last whole 128 are a launch of their own.  `function`: an activation behind a single matrix's product. */
 int cm_debug_lay_tile_shape(int32_t tokens, int32_t columns, int32_t inner, int32_t experts, int32_t top, int32_t pair, int32_t beside, int32_t function);
 
+/* Test hook: how many of m prompt rows the first of two launches of an m x k by k x n product takes (epi: 0 store, 1 add, 2 SiLU product, 3 activation); 0: one launch. */
+int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats);
+
 /* Test hook (host logic only, no GPU): among how many blocks the prompt attention shares the keys of a query tile: `rows` queries behind `start` cached
  * tokens, `heads` query heads of 128 or 256. */
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim);
