@@ -304,6 +304,7 @@ bool launch_attn_decode_heads(const AttnDecArgs& a, int D, int nrep, int ns, boo
 bool launch_attn_decode(const AttnDecArgs& a, int D, int nrep, int nsplit, int kv_mode, float* out, int out_stride, int n_seq,
                         hipStream_t s);
 void launch_gdn(const GdnArgs& a, hipStream_t s);
+bool gdn_in_passes(const GdnArgs& a);      // whether launch_gdn takes its passes over all rows: any S, where the fused kernels need an odd one (the two windows of conv_pool)
 void launch_bf16_to_f32(const uint16_t* src, float* dst, size_t n, float add, hipStream_t s);
 
 // ---- persistent decode kernel (kernels_engine.hip): the row-streaming projections of MANY layers in one launch ----

@@ -908,9 +908,11 @@ __global__ __launch_bounds__(128) void gdn_post_kernel(GdnArgs a) {
     *o = y * rms * a.gnorm_w[tid] * silu_f(z);
 }
 
+// prompts: three passes (needs the scratch rows of ensure_prefill_buffers); decode steps and short tails: fused
+bool gdn_in_passes(const GdnArgs& a) { return a.st == nullptr && a.pre_q != nullptr && a.S >= 16 && a.n_seq <= 1; }
+
 void launch_gdn(const GdnArgs& a, hipStream_t s) {
-    // prompts: three passes (needs the scratch rows of ensure_prefill_buffers); decode steps and short tails: fused
-    if (a.st == nullptr && a.pre_q != nullptr && a.S >= 16 && a.n_seq <= 1) {
+    if (gdn_in_passes(a)) {
         const int nk = a.NV / a.vpg;
         const unsigned heads = (unsigned)((2 * nk + a.NV + 3) / 4);
         // (four tokens per wave where eight leave too few waves: 1.0 us a layer at 17 .. 449 tokens, none from 769 on)

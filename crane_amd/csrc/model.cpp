@@ -1350,18 +1350,20 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             ga.key_dim = cfg.key_dim(); ga.layer_idx = w.gdn_idx; ga.gdn_layers = gdn_layers; ga.eps = cfg.eps;
             ga.n_seq = 1;
             ga.pre_q = gdn_pre_q; ga.pre_k = gdn_pre_k; ga.pre_v = gdn_pre_v; ga.pre_bd = gdn_pre_bd; ga.pre_g = gdn_pre_g; ga.ck = gdn_ck_on ? gdn_ck : nullptr;
-            // the conv windows are double-buffered by position parity: every launch must advance an ODD
-            // number of positions, so an even chunk is scanned as (S-1) + 1.  One scan per sequence of the pass (its own state slot).
+            // the conv windows are double-buffered by position parity: a launch of the fused kernel must advance an ODD
+            // number of positions, so an even one is scanned as (S-1) + 1; the passes over all rows (16 rows or more) read a channel's window in the wave that
+            // writes it and take any number -- the last token of an even prompt alone was 10 us a layer of one workgroup per head (a prompt of 200 tokens
+            // on 18 such layers 4.77 -> 4.62 ms).  One scan per sequence of the pass (its own state slot).
             for (int gi = 0; gi < nseg; ++gi) {
                 const PrefillSeg& sg = segs[gi];
                 ga.slot = sg.seq;
                 int done = 0;
                 while (done < sg.S) {
-                    const int part = ((sg.S - done) % 2 == 1) ? (sg.S - done) : (sg.S - done - 1);
                     ga.proj = pQKV + (size_t)(sg.row0 + done) * in_proj_pad; ga.out = pGY + (size_t)(sg.row0 + done) * cfg.value_dim();
-                    ga.start_pos = sg.start_pos + done; ga.S = part;
+                    ga.start_pos = sg.start_pos + done; ga.S = sg.S - done;
+                    if (ga.S % 2 == 0 && !gdn_in_passes(ga)) --ga.S;
                     launch_gdn(ga, s);
-                    done += part;
+                    done += ga.S;
                 }
             }
             if (q8p) { q8_tail(w, w.q_out_proj, pGY, cfg.value_dim(), li); continue; }

@@ -1,0 +1,38 @@
+"""GPU: prompts and portions of an even number of tokens through the Gated-Delta-Net passes -- the convolution's window is then written where it is read --
+against the same tokens with the last of each alone.
+
+All f32, the last token's sums in another order (the fused kernel instead of the chunk-parallel or the sequential scan): 1e-4 of the largest logit, the bar of the
+prompt passes against the oracle.  A window that is stale or mixed up moves the next token's channels by their own size."""
+import numpy as np
+import pytest
+
+from crane_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+
+# around the smallest number of rows that the passes take, the chunk of 64 and the wider tiles of 512; two even portions, then an odd one, then steps of one token
+@pytest.mark.parametrize("values", [16, 32])
+def test_even_portions(values):
+    from crane_amd.backend import Model
+    cfg = dict(configs.get_config("qwen3.5-0.8b"), vocab_size=512, num_hidden_layers=4, linear_num_value_heads=values)
+    m = Model.synthetic(cfg, seed=6, max_seq_len=1300, max_seqs=2, kv_dtype="f32")
+    rng = np.random.default_rng(values)
+    try:
+        for n, more in ((14, 16), (16, 18), (18, 64), (62, 2), (64, 66), (66, 128), (510, 512), (512, 514)):
+            ids = rng.integers(0, 512, n + more + 17 + 2).tolist()
+            ends = [n, n + more, n + more + 17, n + more + 18, n + more + 19]
+            out = []
+            for alone in (False, True):
+                s, at, rows = m.seq_alloc(), 0, []
+                for end in ends:
+                    if alone and end - at > 1:
+                        m.seq_forward(s, ids[at:end - 1], at)
+                        at = end - 1
+                    rows.append(np.asarray(m.seq_forward(s, ids[at:end], at)[0], np.float64))
+                    at = end
+                m.seq_free(s)
+                out.append(np.stack(rows))
+            assert np.isfinite(out[0]).all() and np.abs(out[0] - out[1]).max() < 1e-4 * np.abs(out[1]).max(), (n, more)
+    finally:
+        m.close()
