@@ -94,7 +94,9 @@ struct GdnArgs {
     const float* A_log;          // [NV]
     const float* dt_bias;        // [NV]
     const float* gnorm_w;        // [V] plain RMSNormGated weight
-    float* out;                  // [S, out_stride] f32 gated-normed y
+    float* out;                  // [S, out_stride] f32 gated-normed y (prompts with out_hi: scratch of the passes)
+    uint16_t* out_hi = nullptr;  // prompts: the rows as bf16 hi + lo planes instead, the A operand of the out_proj GEMM (split_rows_kernel's arithmetic; out_lo null: hi alone).
+    uint16_t* out_lo = nullptr;  //   Even addresses: out_stride and the rows' starts are multiples of 128
     const StepState* st;         // decode: start_pos and slot are read from device state
     int proj_stride, out_stride;
     int start_pos, slot;         // used when st == nullptr (prefill)

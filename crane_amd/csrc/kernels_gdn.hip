@@ -25,6 +25,15 @@
 
 namespace cm {
 
+// a gated, normalised value of a prompt row: f32, or the two bfloat16 terms that the projection behind multiplies (a launch that split the f32 rows was 6.7 us
+// a layer of 2048 tokens and 2048 values; the stores of the terms in their place cost 1.2)
+__device__ __forceinline__ void gdn_put(const GdnArgs& a, size_t at, float v) {
+    if (a.out_hi == nullptr) { a.out[at] = v; return; }
+    const uint16_t h = f32_to_bf16(v);
+    a.out_hi[at] = h;
+    if (a.out_lo != nullptr) a.out_lo[at] = f32_to_bf16(v - bf16_to_f32(h));
+}
+
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 
 // grid = NV value heads, block = 128 threads.  Processes S tokens sequentially (S = 1 at decode).
@@ -105,7 +114,7 @@ __global__ __launch_bounds__(128) void gdn_kernel(GdnArgs a) {
         __syncthreads();
         const float rms = 1.0f / sqrtf((red[4] + red[5]) / (float)V + a.eps);
         const float z = pr[conv_dim + h * V + tid];
-        a.out[(size_t)bq * a.batch_out_stride + (size_t)t * a.out_stride + h * V + tid] = y * rms * gw * silu_f(z);
+        gdn_put(a, (size_t)bq * a.batch_out_stride + (size_t)t * a.out_stride + h * V + tid, y * rms * gw * silu_f(z));
     }
     // ---- write back state and conv windows (other parity buffer) ----
 #pragma unroll
@@ -889,7 +898,16 @@ __global__ __launch_bounds__(512, 4) void gdn_chunk_out_kernel(GdnArgs a) {
         if (t >= nt) continue;
         const float rms = 1.0f / sqrtf((red[0][t] + red[1][t]) / (float)V + a.eps);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) a.out[(size_t)(t0 + t) * a.out_stride + h * V + 64 * hf + 16 * n + r] = y[i][n] * rms * gw[n] * silu_f(z[n][i]);
+        for (int n = 0; n < 4; ++n) {
+            const float v = y[i][n] * rms * gw[n] * silu_f(z[n][i]);
+            const size_t at = (size_t)(t0 + t) * a.out_stride + h * V + 64 * hf + 16 * n + r;
+            if (a.out_hi == nullptr) { a.out[at] = v; continue; }
+            // neighbouring columns make a word: the even lane stores the first terms of both, the odd one the second
+            const float o = __shfl_xor(v, 1), e0 = r & 1 ? o : v, e1 = r & 1 ? v : o;
+            const uint32_t hi = pack_bf16x2(e0, e1);
+            if (!(r & 1)) *(uint32_t*)(a.out_hi + at) = hi;
+            else if (a.out_lo != nullptr) *(uint32_t*)(a.out_lo + at - 1) = pack_bf16x2(e0 - bf16_lo(hi), e1 - bf16_hi(hi));
+        }
     }
 }
 
@@ -898,14 +916,13 @@ __global__ __launch_bounds__(128) void gdn_post_kernel(GdnArgs a) {
     __shared__ float red[2];
     const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int conv_dim = 2 * a.key_dim + a.NV * V;
-    float* o = a.out + (size_t)t * a.out_stride + h * V + tid;
-    const float y = *o;
+    const float y = a.out[(size_t)t * a.out_stride + h * V + tid];
     const float sy = wave_sum(y * y);
     if (lane == 0) red[wave] = sy;
     __syncthreads();
     const float rms = 1.0f / sqrtf((red[0] + red[1]) / (float)V + a.eps);
     const float z = a.proj[(size_t)t * a.proj_stride + conv_dim + h * V + tid];
-    *o = y * rms * a.gnorm_w[tid] * silu_f(z);
+    gdn_put(a, (size_t)t * a.out_stride + h * V + tid, y * rms * a.gnorm_w[tid] * silu_f(z));
 }
 
 // prompts: three passes (needs the scratch rows of ensure_prefill_buffers); decode steps and short tails: fused

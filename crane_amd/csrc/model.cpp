@@ -1360,6 +1360,10 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
                 int done = 0;
                 while (done < sg.S) {
                     ga.proj = pQKV + (size_t)(sg.row0 + done) * in_proj_pad; ga.out = pGY + (size_t)(sg.row0 + done) * cfg.value_dim();
+                    if (!q8p) {
+                        ga.out_hi = pAT_hi + (size_t)(sg.row0 + done) * cfg.value_dim();
+                        ga.out_lo = sp2 ? pAT_lo + (size_t)(sg.row0 + done) * cfg.value_dim() : nullptr;
+                    }
                     ga.start_pos = sg.start_pos + done; ga.S = sg.S - done;
                     if (ga.S % 2 == 0 && !gdn_in_passes(ga)) --ga.S;
                     launch_gdn(ga, s);
@@ -1367,7 +1371,6 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
                 }
             }
             if (q8p) { q8_tail(w, w.q_out_proj, pGY, cfg.value_dim(), li); continue; }
-            launch_split_rows(pGY, pAT_hi, sp2 ? pAT_lo : nullptr, (size_t)S * cfg.value_dim(), s);
             g = GemmArgs{}; g.ws = pWS; g.ws_floats = gemm_ws_floats; g.wide256 = gemm256;
             g.A_hi = pAT_hi; g.A_lo = sp2 ? pAT_lo : nullptr; g.W = w.out_proj; g.M = S; g.N = H; g.K = cfg.value_dim(); g.ldc = H;
             if (quantized) set_w(g, deq_w(w, 1, (size_t)w.q_out_proj.N * w.q_out_proj.K, [&](uint16_t* dst, uint16_t* lo) { launch_dequant_bf16(w.q_out_proj, dst, 1, 0, s, lo); }));
