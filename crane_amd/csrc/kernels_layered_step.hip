@@ -181,24 +181,6 @@ __global__ __launch_bounds__(256) void lay_step_out_kernel(LAttnArgs a, int nspl
     if (lane < 2 && n < N) C[n] = lane ? acc1 : acc0;
 }
 
-// the expert of choice `slot` by what lay_router_choose chooses by, in every wave for itself: the lane with `slot` better ones (equals: the lower lane first).  -1: not by numbers
-__device__ __forceinline__ int step_choice(const float* zs, int lane, int slot, int E, const RouterSpec& rs) {
-    const float z = lane < E ? zs[lane] : -INFINITY;
-    float own = z;
-    if (rs.softmax) {
-        const float mx = wave_max(z), p = lane < E ? expf(z - mx) : 0.f;
-        own = p / wave_sum(p);
-    }
-    if (__any(lane < E && own != own)) return -1;
-    int better = 0;
-    for (int j = 0; j < E; ++j) {
-        const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), j));
-        better += v > own || (v == own && j < lane);
-    }
-    const unsigned long long at = __ballot(lane < E && better == slot);
-    return at ? __builtin_ctzll(at) : -1;
-}
-
 // norm, router, choice, and act(h W_e^T) * (h W2_e^T) of the chosen experts and the one of every token.  blockIdx.y: the choice, the last the expert of every token.  A last block
 // of the first choice writes the choices and their weights, which the others do not wait for (one wave's choice for
 // the block and all of them through it 9.3 us a launch, each its own 8.3)
@@ -244,8 +226,9 @@ __global__ __launch_bounds__(256) void lay_step_moe_kernel(LStepNorm a, LStepMoe
             }
         }
         __syncthreads();
-        e = writes ? -1 : step_choice(zs, lane, slot, m.experts, m.rs);
-        if (e < 0) {                           // (uniform in the block)
+        e = writes ? -1 : lay_router_choice(zs, lane, slot, m.experts, m.rs);
+        if (e < 0) {                           // (every wave has it from the same logits: uniform in the block)
+            __syncthreads();                   // lay_router_choose writes over logits that a slower wave may still read
             if (wave == 0) lay_router_choose(zs, 0, lane, ss, swt, m.experts, m.top, m.rs, nullptr, m.slots);
             __syncthreads();
             e = ss[slot];

@@ -125,4 +125,24 @@ __device__ __forceinline__ void lay_router_choose(float* zs, int t, int lane, in
     for (int k = top + lane; k < slots; k += 64) wsel[(size_t)t * slots + k] = rs.shared_gate ? 1.f / (1.f + expf(-zs[E])) : 1.f;
 }
 
+// Choice `slot` of lay_router_choose by itself, for at most 64 outputs without correction or groups, in every wave that calls it and with nothing written: the lane with `slot` better
+// scores, equal ones in the lanes' order, as that function's maxima come one after another.  -1: it goes by another rule there (scores that are no numbers, a choice of none).  Scores
+// are made and compared here as they are there; a change to one is a change to the other
+__device__ __forceinline__ int lay_router_choice(const float* zs, int lane, int slot, int E, const RouterSpec& rs) {
+    const float z = lane < E ? zs[lane] : -INFINITY;
+    float own = z;
+    if (rs.softmax) {
+        const float mx = wave_max(z), p = lane < E ? expf(z - mx) : 0.f;
+        own = p / wave_sum(p);
+    }
+    if (__any(lane < E && !(own > -INFINITY))) return -1;
+    int better = 0;
+    for (int j = 0; j < E; ++j) {
+        const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), j));
+        better += v > own || (v == own && j < lane);
+    }
+    const unsigned long long at = __ballot(lane < E && better == slot);
+    return at ? __builtin_ctzll(at) : -1;
+}
+
 }  // namespace cm

@@ -36,3 +36,41 @@ def test_against_single_launches(tmp_path, width, heads, kv_heads, dim, window, 
     finally:
         m.close()
     assert np.isfinite(out[0]).all() and (out[0] == out[1]).all()
+
+
+def _bits(tmp_path, cfg, P, context, steps=4, **kw):
+    """Logits of `steps` single rows behind `context` tokens: in the launches of this file's subject, then in single ones."""
+    from crane_amd.backend import Model
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=4, max_seq_len=768, **kw)
+    toks = GZ.tokens(context + steps, cfg["vocab"], 4)
+    out = []
+    try:
+        s = m.seq_alloc()
+        m.step_batch([(s, toks[:context], [])], want_logits=False)
+        for on in (1, 0):
+            m.debug_set("lay_fused_prep", on)
+            f = m.seq_fork(s)
+            out.append(np.stack([m.step_batch([(f, toks[context + i:context + i + 1], None)])[0] for i in range(steps)]))
+            m.seq_free(f)
+    finally:
+        m.close()
+    return out
+
+
+# the choice that every block makes for itself against the one whose weights are written: equal logits (the lower output first), and scores that are no numbers
+@pytest.mark.parametrize("kind", ["equal", "pairs", "nan"])
+@pytest.mark.parametrize("experts,top,shared", [(6, 2, 72), (14, 4, 0), (63, 5, 72)])
+def test_choices_of_equal_scores_and_of_none(tmp_path, kind, experts, top, shared):
+    cfg = GZ.config([GZ.layer(GZ.attn(heads=4, kv_heads=2, dim=64, vdim=64, conv=4, rot_dims=64), GZ.moe(experts=experts, top=top, ff=136, shared=shared)) for _ in range(2)],
+                    vocab=96, width=512)
+    P = GZ.random_weights(cfg, 6)
+    router = P["l0.mlp.router"]
+    if kind == "equal":
+        router[:] = router[0]
+    elif kind == "pairs":
+        router[1::2] = router[0:experts - experts % 2:2]
+    else:
+        router[experts // 2] = np.nan
+    a, b = _bits(tmp_path, cfg, P, 40)
+    assert np.isfinite(a).all() != (kind == "nan")
+    np.testing.assert_array_equal(a, b)
