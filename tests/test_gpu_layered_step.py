@@ -57,6 +57,21 @@ def _bits(tmp_path, cfg, P, context, steps=4, **kw):
     return out
 
 
+# the row's own convolution, rotation and append: layers on borrowed keys (queries alone are convolved, nothing is appended), one to four taps on either side of a loan, five that the
+# single launches keep, rotated parts of no, some and all elements, keys narrower and wider than values with padding behind either, one to four query heads on a key head; steps across a
+# tile of 64 keys and a page, in one block and in shares; a page that is no power of two (divisions instead of shifts: the single launches)
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,taps,rot", [
+    (4, 2, 64, 96, (1, 4, 2), (0, 32, 64)), (8, 2, 112, 64, (3, 2, 4), (56, 0, 112)), (3, 1, 48, 128, (2, 1, 3), (48, 48, 16)), (6, 6, 128, 16, (4, 3, 1), (128, 64, 0)),
+    (8, 2, 80, 80, (4, 5, 4), (80, 8, 80))])
+@pytest.mark.parametrize("context,page", [(1, 64), (62, 64), (317, 64), (317, 128), (190, 192)])
+def test_rows_on_their_way_into_the_attention(tmp_path, heads, kv_heads, dim, vdim, taps, rot, context, page):
+    mk = lambda i, **kw: GZ.layer(GZ.attn(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, conv=taps[i], size=4096 if i < 2 else 200, rot_dims=rot[i], **kw),
+                                  GZ.moe(experts=5, top=2, ff=136, shared=72))
+    cfg = GZ.config([mk(0), mk(1, kv_from=0), mk(2), mk(1, kv_from=2)], vocab=96, width=512)
+    a, b = _bits(tmp_path, cfg, GZ.random_weights(cfg, 5), context, kv_block_size=page)
+    assert np.isfinite(a).all() and (a == b).all()
+
+
 # the choice that every block makes for itself against the one whose weights are written: equal logits (the lower output first), and scores that are no numbers
 @pytest.mark.parametrize("kind", ["equal", "pairs", "nan"])
 @pytest.mark.parametrize("experts,top,shared", [(6, 2, 72), (14, 4, 0), (63, 5, 72)])
