@@ -615,6 +615,28 @@ int cm_debug_lay_tile_shape(int32_t tokens, int32_t columns, int32_t inner, int3
     return tail ? -size : size;
 }
 
+int cm_debug_lay_attn_shares(const int32_t* starts, const int32_t* rows, int32_t n, int32_t heads, int32_t kv_heads, int64_t window, int32_t* out) {
+    if (!starts || !rows || !out || n < 0 || kv_heads <= 0 || heads < kv_heads) return -1;
+    int total = -1;
+    guard(nullptr, [&] {
+        const int nrep = heads / kv_heads;
+        std::vector<cm::LaySegDev> segs((size_t)n);
+        std::vector<int2> tiles, list((size_t)cm::LAY_ATTN_TILE_BLOCKS);
+        for (int i = 0; i < n; ++i) {
+            segs[(size_t)i] = cm::LaySegDev{};
+            segs[(size_t)i].n = rows[i]; segs[(size_t)i].start_pos = starts[i];
+            for (int q0 = 0; q0 < rows[i] * nrep; q0 += cm::LAY_ATTN_MFMA_ROWS) tiles.push_back(make_int2(i, q0));
+        }
+        const int blocks = cm::lay_attn_tile_shared(tiles.data(), (int)tiles.size(), segs.data(), nrep, kv_heads, window, list.data());
+        for (int i = 0; i < blocks; ++i) {
+            const int2 t = list[(size_t)i];
+            out[4 * i] = cm::lay_share_seg(t.x); out[4 * i + 1] = t.y; out[4 * i + 2] = cm::lay_share_no(t.x); out[4 * i + 3] = cm::lay_shares(t.x);
+        }
+        total = blocks;
+    });
+    return total;
+}
+
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim) { return cm::attn_prefill_shares(rows, start, heads, head_dim); }
 
 int cm_debug_set(cm_model* h, const char* key, int64_t value) {

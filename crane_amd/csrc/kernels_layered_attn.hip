@@ -272,8 +272,8 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
     uint16_t* const Vs = Ks + 2 * KT * KLD;                       // [2][64][VLD]
     const int g = blockIdx.x;
     const int2 tile_id = a.tiles[blockIdx.y];
-    const LaySegDev sg = a.segs[KS == 2 ? tile_id.x & 0xffff : tile_id.x];
-    const int share = KS == 2 ? (tile_id.x >> 16) & 255 : 0, shares = KS == 2 ? max(1, tile_id.x >> 24) : 1;
+    const LaySegDev sg = a.segs[KS == 2 ? lay_share_seg(tile_id.x) : tile_id.x];
+    const int share = KS == 2 ? lay_share_no(tile_id.x) : 0, shares = KS == 2 ? lay_shares(tile_id.x) : 1;
     const int nrep = a.H / a.G, d = a.d, e = a.e;
     const int q0 = tile_id.y, nq = min(64, sg.n * nrep - q0);
     Walk w;
@@ -745,7 +745,7 @@ template <int DP, int EP>
 void go_sizes(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t s) {
     // one block per CU at most: two groups of waves share the key tiles (a mixed batch of 24 single tokens and 300 prompt rows on 8 heads:
     // 24 us against 27); more blocks share the CUs by themselves
-    const bool two = (long long)a.ntiles * a.G <= 256;
+    const bool two = a.done != nullptr || (long long)a.ntiles * a.G <= LAY_ATTN_TILE_BLOCKS;      // (shared tiles: this form alone)
     if (nsplit > 0) { if (a.pool > 0) go_few<DP, EP, true>(a, nsplit, qvec, ovec, s); else go_few<DP, EP, false>(a, nsplit, qvec, ovec, s); }
     else if (a.pool > 0) { if (two) go<DP, EP, true, 2>(a, qvec, ovec, s); else go<DP, EP, true, 1>(a, qvec, ovec, s); }
     else { if (two) go<DP, EP, false, 2>(a, qvec, ovec, s); else go<DP, EP, false, 1>(a, qvec, ovec, s); }
@@ -756,7 +756,25 @@ void go_sizes(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t 
 // A walk of more than six tiles in shares of `each`.  A mixed step of 24 single tokens and 302 prompt rows behind up to 900 others, 8 heads on 2, leaves two thirds of the chip
 // idle while its longest blocks walk 19 tiles in ten steps: 18, 25, 29 and 33 us a layer behind 0, 302, 605 and 907 tokens, 16, 20, 21 and 21 with shares of six (of four 16, 20,
 // 20, 22; of two 17, 20, 20, 22): what is left of a launch is its start, first loads and end
-int lay_attn_tile_shares(int tiles, int each) { return tiles > 6 ? std::min(127, (tiles + each - 1) / each) : 1; }
+static int lay_attn_tile_shares(int tiles, int each) { return tiles > 6 ? std::min(127, (tiles + each - 1) / each) : 1; }
+int lay_attn_tile_shared(const int2* tiles, int n, const LaySegDev* segs, int nrep, int heads, long long win, int2* out) {
+    if (heads <= 0 || (long long)n * heads > LAY_ATTN_TILE_BLOCKS / 2) return 0;
+    auto walk = [&](const int2& t) {                   // (of a window alone: first tokens that are kept count as if they lay in front of it)
+        const LaySegDev& sg = segs[t.x];
+        const long long first = sg.start_pos + t.y / nrep, newest = sg.start_pos + (std::min(t.y + LAY_ATTN_MFMA_ROWS, sg.n * nrep) - 1) / nrep;
+        return (int)(newest / KT - std::max(0ll, first - win + 1) / KT + 1);
+    };
+    int each = 6, total;
+    for (;; each += 2) {
+        total = 0;
+        for (int i = 0; i < n; ++i) total += lay_attn_tile_shares(walk(tiles[i]), each);
+        if (total * heads <= LAY_ATTN_TILE_BLOCKS) break;
+    }
+    if (total == n) return 0;
+    for (int i = 0, at = 0; i < n; ++i)
+        for (int k = 0, shares = lay_attn_tile_shares(walk(tiles[i]), each); k < shares; ++k) out[at++] = make_int2(lay_share(tiles[i].x, k, shares), tiles[i].y);
+    return total;
+}
 
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page) {
     return d > 0 && e > 0 && d % 16 == 0 && e % 16 == 0 && d <= 128 && e <= 128 && (own_v || e <= d) && page % KT == 0;

@@ -308,7 +308,7 @@ struct LAttnArgs {
     // few query tiles, many keys (decode steps): nsplit blocks per tile share its key tiles and a merge launch follows;
     // part_o [ntiles][G][nsplit][16][d], part_ml [ntiles][G][nsplit][16][2].  nsplit <= 1 or null scratch: one block per tile
     int nsplit = 1; float* part_o = nullptr; float* part_ml = nullptr;
-    // lay_attn_tile: a tile's keys shared among blocks.  tiles[i].x = segment + (share << 16) + (shares << 24), the shares of a tile side by side; sums in part_o [ntiles][G][64 e],
+    // lay_attn_tile: a tile's keys shared among blocks (tiles: lay_attn_tile_shared); sums in part_o [ntiles][G][64 e],
     // part_ml [ntiles][G][64][2], the last one to arrive (done [ntiles][G], zero before and after) adds them up.  null: no tile is shared
     int32_t* done = nullptr;
     LAttnPrep prep;                                  // lay_attn_few, single rows
@@ -374,9 +374,15 @@ bool lay_attn_mfma_fits(int d, int e, bool own_v);         // sizes the matrix-c
 // heads 106 us against 1590, 8 on 2 (a mixed batch of 24 tokens and 300 prompt rows) 24 against 174; the older form keeps other page sizes
 // and long cached rows
 void launch_lay_attn_tile(const LAttnArgs& a, hipStream_t s);
-// among how many blocks a tile of `tiles` key tiles is shared when `each` are enough for a block; launches of at most LAY_ATTN_TILE_BLOCKS blocks
+// Launches of few query tiles share the keys of long walks among blocks: at most LAY_ATTN_TILE_BLOCKS blocks, all of them of the kernel's form with two groups of waves, which alone knows shares.
+// A shared tile's entries stand side by side, x = lay_share(segment, share, shares).  lay_attn_tile_shared: the list of n tiles over segs, `heads` key heads and a window of `win` keys in
+// out (LAY_ATTN_TILE_BLOCKS / heads entries at most); 0: no tile is shared
 constexpr int LAY_ATTN_TILE_BLOCKS = 256;
-int lay_attn_tile_shares(int tiles, int each);
+__host__ __device__ constexpr int lay_share(int seg, int share, int shares) { return shares > 1 ? seg + (share << 16) + (shares << 24) : seg; }
+__host__ __device__ constexpr int lay_share_seg(int x) { return x & 0xffff; }
+__host__ __device__ constexpr int lay_share_no(int x) { return (x >> 16) & 0xff; }
+__host__ __device__ constexpr int lay_shares(int x) { return x >> 24 > 1 ? x >> 24 : 1; }
+int lay_attn_tile_shared(const int2* tiles, int n, const LaySegDev* segs, int nrep, int heads, long long win, int2* out);
 bool lay_attn_prep_fits(int H, int G, int d, int e, int dims, int page, bool pooled);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
 // the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can

@@ -1700,29 +1700,17 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     return t_segs[x.x].start_pos + x.y / nrep > t_segs[y.x].start_pos + y.y / nrep; });
             }
             tiles64[nrep] = {o_m, cnt};
-            // the same with the keys of long walks shared among blocks (lay_attn_tile_kernel), where blocks are few.  The walk: the longest window of the layers
+            // the same with the keys of long walks shared among blocks, where blocks are few.  The walk: the longest window of the layers
             int G = 0;
             long long win = 0;
             for (const LayerSpec& sp : L.spec)
                 if (sp.mixer == LMIX_ATTN && sp.kv_heads > 0 && sp.heads / sp.kv_heads == nrep && sp.pool == 0) { G = std::max(G, sp.kv_heads); win = std::max(win, sp.win + sp.keep); }
-            if (L.f32 || all_decode || G == 0 || cnt * G > LAY_ATTN_TILE_BLOCKS / 2) continue;
-            const int2* tl = (const int2*)(tab + o_m);
-            auto walk = [&](const int2& t) {
-                const LaySegDev& sg = t_segs[t.x];
-                const long long first = sg.start_pos + t.y / nrep, newest = sg.start_pos + (std::min(t.y + LAY_ATTN_MFMA_ROWS, sg.n * nrep) - 1) / nrep;
-                return (int)(newest / 64 - std::max(0ll, first - win + 1) / 64 + 1);
-            };
-            int each = 6, total = 0;
-            for (;; each += 2) {
-                total = 0;
-                for (int i = 0; i < cnt; ++i) total += lay_attn_tile_shares(walk(tl[i]), each);
-                if (total * G <= LAY_ATTN_TILE_BLOCKS) break;
-            }
-            if (total == cnt) continue;
-            const size_t o_s = o;
-            for (int i = 0; i < cnt; ++i)
-                for (int k = 0, n = lay_attn_tile_shares(walk(tl[i]), each); k < n; ++k) { tab[o++] = tl[i].x + (n > 1 ? (k << 16) + (n << 24) : 0); tab[o++] = tl[i].y; }
-            shared64[nrep] = {o_s, total};
+            if (L.f32 || all_decode || G == 0) continue;
+            static_assert(MAXB <= 1 << 16, "lay_share: the segment's bits");
+            const int total = lay_attn_tile_shared((const int2*)(tab + o_m), cnt, t_segs, nrep, G, win, (int2*)(tab + o));
+            if (total == 0) continue;
+            shared64[nrep] = {o, total};
+            o += 2 * (size_t)total;
             shared_heads = std::max(shared_heads, G);
         }
         const size_t o_done = o;               // blocks of every shared tile that have arrived

@@ -541,6 +541,10 @@ int cm_debug_lay_tile_plan(int32_t tokens, int32_t columns, int32_t experts, int
  * has `beside` columns (0: none); negative: the columns behind the last whole 128 are a launch of their own.  `function`: an activation behind a single matrix's product. */
 int cm_debug_lay_tile_shape(int32_t tokens, int32_t columns, int32_t inner, int32_t experts, int32_t top, int32_t pair, int32_t beside, int32_t function);
 
+/* Test hook (host logic only, no GPU): the blocks of a prompt attention whose key walks are shared: n portions of rows[i] tokens behind starts[i] cached ones, `heads` query heads on `kv_heads`, at
+ * most `window` keys.  out: 4 numbers a block (portion, first query row, share, shares), 256 blocks at most; returns how many for each key head, 0: no walk is shared. */
+int cm_debug_lay_attn_shares(const int32_t* starts, const int32_t* rows, int32_t n, int32_t heads, int32_t kv_heads, int64_t window, int32_t* out);
+
 /* Test hook: how many of m prompt rows the first of two launches of an m x k by k x n product takes (epi: 0 store, 1 add, 2 SiLU product, 3 activation); 0: one launch. */
 int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats);
 
