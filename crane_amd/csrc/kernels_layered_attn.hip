@@ -753,19 +753,23 @@ void go_sizes(const LAttnArgs& a, int nsplit, bool qvec, bool ovec, hipStream_t 
 
 }  // namespace
 
-// A walk of more than six tiles in shares of `each`.  A mixed step of 24 single tokens and 302 prompt rows behind up to 900 others, 8 heads on 2, leaves two thirds of the chip
-// idle while its longest blocks walk 19 tiles in ten steps: 18, 25, 29 and 33 us a layer behind 0, 302, 605 and 907 tokens, 16, 20, 21 and 21 with shares of six (of four 16, 20,
-// 20, 22; of two 17, 20, 20, 22): what is left of a launch is its start, first loads and end
+// A walk of more than six tiles in shares of `each`, six or what fits the blocks.  A launch of few blocks leaves the chip idle while its longest walk 19 tiles in ten steps; what is left
+// with shares is its start, first loads and end.  us a launch, whole / shares of 4 / 6 / 10 (more than 3, 6 and 12 tiles shared: within 3 us of those of 6, either way):
+// 24 single tokens and 302 rows behind 0, 302, 605, 907 and 2000 tokens, 8 heads of 128 on 2 20.6 / 17.8 / 19.1 / 19.8, 21.9 / 19.7 / 21.5 / 21.9, 28.1 / 21.6 / 22.9 / 23.2, 32.8 / 23.3 / 23.0 /
+// 26.1, 50.2 / 27.8 / 27.7 / 28.4; 64 rows alone behind 500, 1000 and 4000 21.7 / 19.2 / 19.3 / 21.6, 30.0 / 20.8 / 21.0 / 23.5, 79.3 / 31.7 / 28.8 / 29.2; 512 rows behind 1000 and 4000 38.2 / 26.2 / 26.0 /
+// 27.2, 88.7 / 39.4 / 39.4 / 39.5; 4 on 1, 32 on 8 and heads of 64 (16 on 4, 16 on 16) alike.  They are looked at while the tiles as a whole fit one round of blocks: up to half of them, as
+// long as it was, 60 single tokens and 128 rows behind 1000 on 2 key heads (136 blocks) took 30.8, now 23.2, 24 and 302 on 4 heads of 64 (172) behind 302, 605, 907 and 2000 16.2, 20.1,
+// 23.4, 34.5, now 16.6, 18.0, 19.8, 25.5
 static int lay_attn_tile_shares(int tiles, int each) { return tiles > 6 ? std::min(127, (tiles + each - 1) / each) : 1; }
 int lay_attn_tile_shared(const int2* tiles, int n, const LaySegDev* segs, int nrep, int heads, long long win, int2* out) {
-    if (heads <= 0 || (long long)n * heads > LAY_ATTN_TILE_BLOCKS / 2) return 0;
+    if (heads <= 0 || (long long)n * heads > LAY_ATTN_TILE_BLOCKS) return 0;
     auto walk = [&](const int2& t) {                   // (of a window alone: first tokens that are kept count as if they lay in front of it)
         const LaySegDev& sg = segs[t.x];
         const long long first = sg.start_pos + t.y / nrep, newest = sg.start_pos + (std::min(t.y + LAY_ATTN_MFMA_ROWS, sg.n * nrep) - 1) / nrep;
         return (int)(newest / KT - std::max(0ll, first - win + 1) / KT + 1);
     };
     int each = 6, total;
-    for (;; each += 2) {
+    for (;; each += std::max(2, each / 8)) {           // (an eighth at a time where walks are thousands of tiles)
         total = 0;
         for (int i = 0; i < n; ++i) total += lay_attn_tile_shares(walk(tiles[i]), each);
         if (total * heads <= LAY_ATTN_TILE_BLOCKS) break;

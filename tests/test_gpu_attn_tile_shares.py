@@ -29,12 +29,13 @@ def _shares(portions, heads, kv_heads, window):
     return [tuple(out[4 * i:4 * i + 4]) for i in range(total)]
 
 
-# seven key tiles of 64 are the first walk that is shared; half the chip's blocks are the most that are looked at
+# seven key tiles of 64 are the first walk that is shared; walks are looked at while the tiles leave blocks of one round free
 @pytest.mark.parametrize("start,shares", [(300, 1), (383 - 29, 1), (383 - 28, 2), (1000, 3)])
 def test_walks_of_more_than_six_tiles(start, shares):
     got = _shares([(start, 30), (5, 1)], 4, 2, 1 << 40)
     assert max([s[3] for s in got], default=1) == shares
-    assert not _shares([(start, 30)] * 65, 4, 2, 1 << 40)
+    # long walks among short ones on two key heads: more than half a round of blocks, as many as a round has, more
+    assert [bool(_shares([(start, 30)] * n + [(5, 1)] * 70, 4, 2, 1 << 40)) for n in (10, 58, 59)] == [shares > 1, False, False]
 
 
 def test_lists_are_whole_and_fit_one_round_of_blocks():
