@@ -807,7 +807,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnDecArgs a) {
                 q_hi[item * D + lane + 64 * j] = h;
                 q_lo[item * D + lane + 64 * j] = kv16_from_f32<KVT>(x - kv16_to_f32<KVT>(h));
             }
-        } else {
+        } else {                                                 // (the owner's block alone comes here)
             uint16_t* dst = (item == NREP) ? knew : vnew;
             if (KVQ) {
                 // quantize_per_token (qwen3_5/kv_cache.rs:253-268); LDS keeps code - offset as a bf16 integer
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnDecArgs a) {
                 amax = wave_max(amax);
                 const float scale = __fadd_rn(__fmul_rn(amax, (float)(1.0 / (double)QMAX)), 1e-8f);
                 uint8_t* pb = (uint8_t*)((item == NREP) ? a.kpool : a.vpool);
-                const size_t pbase = owner ? (size_t)block_table[pos / a.page] * a.page_bytes : 0;
+                const size_t pbase = (size_t)block_table[pos / a.page] * a.page_bytes;
                 const size_t roff = pbase + (size_t)(kvh * a.page + (pos % a.page)) * ROWB;
 #pragma unroll
                 for (int j = 0; j < EPL; ++j) {
@@ -825,25 +825,25 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnDecArgs a) {
                     const float code = roundf(__fdiv_rn(xv[j], scale)) + OFFS;
                     dst[d] = f32_to_bf16(code - OFFS);
                     const uint32_t ci = (uint32_t)(int)code;
-                    if (KVT == 2) { if (owner) pb[roff + d] = (uint8_t)ci; }
+                    if (KVT == 2) pb[roff + d] = (uint8_t)ci;
                     else {
                         const uint32_t hi = (uint32_t)__shfl_down((int)ci, 1);
-                        if (owner && !(lane & 1)) pb[roff + (d >> 1)] = (uint8_t)(ci | (hi << 4));
+                        if (!(lane & 1)) pb[roff + (d >> 1)] = (uint8_t)(ci | (hi << 4));
                     }
                 }
                 if (lane == 0) {
                     new_scale[item - NREP] = scale;
-                    if (owner) *(float*)(pb + pbase + (size_t)a.Hkv * a.page * ROWB + (size_t)(kvh * a.page + (pos % a.page)) * 4) = scale;
+                    *(float*)(pb + pbase + (size_t)a.Hkv * a.page * ROWB + (size_t)(kvh * a.page + (pos % a.page)) * 4) = scale;
                 }
             } else {
             uint16_t* pool = (uint16_t*)((item == NREP) ? a.kpool : a.vpool);
-            const size_t eoff = owner ? ((size_t)(block_table[pos / a.page] * a.Hkv + kvh) * a.page + (pos % a.page)) * D : 0;
+            const size_t eoff = ((size_t)(block_table[pos / a.page] * a.Hkv + kvh) * a.page + (pos % a.page)) * D;
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
                 const int d = lane + 64 * j;
                 const uint16_t b = kv16_from_f32<KVT>(xv[j]);
                 dst[d] = b;
-                if (owner) pool[eoff + d] = b;
+                pool[eoff + d] = b;
             }
             }
         }
