@@ -527,7 +527,7 @@ __global__ __launch_bounds__(PACK && !HALF ? 256 : 512, PACK && !HALF ? 2 : 1) v
     float turn = 0.f;
     if (PREP) {                                        // a rotated pair per lane, or two neighbours behind the rotated part
         const int hd = a.prep.dims / 2;
-        if (lane < hd) { e0 = a.prep.half ? lane : 2 * lane; e1 = a.prep.half ? lane + hd : 2 * lane + 1; turn = a.prep.freq[lane]; }
+        if (lane < hd) { e0 = 2 * lane; e1 = e0 + 1; turn = a.prep.freq[lane]; }
         else if (a.prep.dims + 2 * (lane - hd) < d) { e0 = a.prep.dims + 2 * (lane - hd); e1 = e0 + 1; }          // (d is even)
         const float* qs = a.proj + a.q_off + (g * nrep + min(wave, nq - 1)) * d, *ks = a.proj + a.prep.k_off + g * d, *vs = a.proj + a.prep.v_off + g * e;
         if (e0 >= 0 && wave < QR) qp = make_float2(qs[e0], qs[e1]);
@@ -592,13 +592,11 @@ __global__ __launch_bounds__(PACK && !HALF ? 256 : 512, PACK && !HALF ? 2 : 1) v
         auto ready = [&](float2 v) __attribute__((always_inline)) {
 #pragma clang fp contract(off)                         // (a head times its factor is rounded before it is split)
             if (lane < hd) v = lay_turn(v, cs, sn);
-            if (a.prep.unit) {
-                float ss = fmaf(v.x, v.x, 0.f);
-                ss = fmaf(v.y, v.y, ss);
-                for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-                const float rs = 1.f / sqrtf(ss / (float)d + a.prep.eps);
-                v.x *= rs; v.y *= rs;
-            }
+            float ss = fmaf(v.x, v.x, 0.f);
+            ss = fmaf(v.y, v.y, ss);
+            for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+            const float rs = 1.f / sqrtf(ss / (float)d + a.prep.eps);
+            v.x *= rs; v.y *= rs;
             return v;
         };
         if (wave < QR) qp = ready(qp);
@@ -784,9 +782,10 @@ bool lay_attn_tile_fits(int d, int e, bool own_v, int page) {
     return d > 0 && e > 0 && d % 16 == 0 && e % 16 == 0 && d <= 128 && e <= 128 && (own_v || e <= d) && page % KT == 0;
 }
 
-// queries of one row on their way through lay_attn_few_kernel: a wave per query head, a pair of elements per lane, values in pages of their own
-bool lay_attn_prep_fits(int H, int G, int d, int e, int dims, int page, bool pooled) {
-    return lay_attn_tile_fits(d, e, true, page) && H <= 4 * G && H % G == 0 && dims % 2 == 0 && dims <= d && !pooled && (page & (page - 1)) == 0;
+// queries of one row on their way through lay_attn_few_kernel: a wave per query head, a pair of neighbouring elements per lane, heads of unit root mean square, values in pages of their own
+bool lay_attn_prep_fits(const LayerSpec& sp, int dims, int page) {
+    return sp.unit_qk && !(dims > 0 && sp.rot.half) && sp.pool == 0 && lay_attn_tile_fits(sp.dim, sp.vdim, true, page) && sp.heads <= 4 * sp.kv_heads && sp.heads % sp.kv_heads == 0 &&
+           dims % 2 == 0 && dims <= sp.dim && (page & (page - 1)) == 0;
 }
 
 static void launch(const LAttnArgs& a0, int nsplit, hipStream_t s) {

@@ -288,7 +288,7 @@ void launch_lay_post_norm(float* x, const float* y, const float* w, float mult, 
 // key, which goes to the pages with the value from there.  own: the layer has keys of its own
 struct LAttnWalk { int pmin, pmax, main0, front, ntile, blocks, vis_lo, win, keep, chunk, pool; };      // the key walk of a query tile (kernels_layered_attn.hip)
 struct LAttnPrep {
-    int on = 0, own = 0, half = 0, unit = 0, k_off = 0, v_off = 0, dims = 0; const float* freq = nullptr; float mag = 1.f, eps = 0.f; LaySegDev seg{};
+    int on = 0, own = 0, k_off = 0, v_off = 0, dims = 0; const float* freq = nullptr; float mag = 1.f, eps = 0.f; LaySegDev seg{};
     LAttnWalk walk{}; int clo = 0, nrep = 0, page_shift = 0;      // filled in by the launch: what a block would divide for
 };
 struct LAttnArgs {
@@ -383,7 +383,7 @@ __host__ __device__ constexpr int lay_share_seg(int x) { return x & 0xffff; }
 __host__ __device__ constexpr int lay_share_no(int x) { return (x >> 16) & 0xff; }
 __host__ __device__ constexpr int lay_shares(int x) { return x >> 24 > 1 ? x >> 24 : 1; }
 int lay_attn_tile_shared(const int2* tiles, int n, const LaySegDev* segs, int nrep, int heads, long long win, int2* out);
-bool lay_attn_prep_fits(int H, int G, int d, int e, int dims, int page, bool pooled);
+bool lay_attn_prep_fits(const LayerSpec& sp, int dims, int page);
 bool lay_attn_tile_fits(int d, int e, bool own_v, int page);
 // the same sizes, few query rows (decode steps): a.tiles in steps of 16 rows, as lay_attn_kernel; nsplit from lay_attn_few_split (keys a query can
 // see, blocks of an unsplit launch, scratch parts)

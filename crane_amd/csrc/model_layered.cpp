@@ -2002,7 +2002,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                 const bool one_row = T == 1 && L.tanh_norm && !L.f32 && L.fused_prep && lay_step_fits(W, sp);
                 // ... the convolutions behind the projection's sums, rotation, unit heads and cache append inside the attention
                 const bool prepared = one_row && sp.mixer == LMIX_ATTN && sp.maps == 1 && L.attn_mfma && kv_mode == KV_BF16 && sp.conv <= LAY_STEP_TAPS && w.v_page_bytes != 0 &&
-                                      lay_attn_prep_fits(sp.heads, sp.kv_heads, sp.dim, sp.vdim, w.rot_freq ? sp.rot.dims : 0, page, sp.pool > 0);
+                                      lay_attn_prep_fits(sp, w.rot_freq ? sp.rot.dims : 0, page);
                 // the norm in front of the experts, their router and lists and this layer's convolution tails in one launch
                 const bool joined = L.tanh_norm && rounded && sp.mlp == LMLP_MOE && !sp.scale_input && lay_norm_router_fits(W, sp.experts, sp.router) &&
                                     lay_experts_on_tiles(L, sp, T, W) &&
@@ -2038,7 +2038,7 @@ void Model::step_batch(const StepItem* items, size_t n_items, float* logits_out,
                     c.q = L.XB; c.ldq = H * d; c.kpool = kv_pool + w.k_pool_off; c.vpool = kv_pool + w.v_pool_off;
                     c.bt = d_bt; c.segs = d_segs; c.rowseg = d_rowseg; c.page = page; c.T = T; c.tail_too = all_decode;
                     if (prepared) {
-                        prep.on = true; prep.own = sp.kv_from < 0; prep.half = c.half; prep.unit = c.unit; prep.k_off = w.k_off; prep.v_off = w.v_off;
+                        prep.on = true; prep.own = sp.kv_from < 0; prep.k_off = w.k_off; prep.v_off = w.v_off;
                         prep.dims = c.freq ? c.dims : 0; prep.freq = c.freq; prep.mag = c.mag; prep.eps = c.eps; prep.seg = t_segs[0];
                     } else {
                         if (T > 1 && w.rot_id >= 0) {      // (a single row: a launch more than it saves)
