@@ -55,15 +55,6 @@ __device__ __forceinline__ float q8_scale(float am, float& id) {
     return (float)(_Float16)dq;
 }
 
-// sums that another XCD's block reads: written through to where all of them read, and read from there, so that their counter needs no fence (a fence writes back
-// and drops a whole L2)
-__device__ __forceinline__ void put_through(float* p, float x, float y) {
-    __hip_atomic_store((unsigned long long*)p, (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float2 get_through(const float* p) {
-    const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
-}
 // the shares of a sequence's head merged by one wave, two columns per lane, always in their order
 __device__ __forceinline__ void merge_head(const AttnDecArgs& a, int bq, int h, int nh, int nsplit, int shares, int lane) {
     constexpr int AT = 8;                                         // shares requested at once
@@ -402,7 +393,7 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
     if (threadIdx.x == 0) last = atomicAdd(done, 1) == shares - 1;
     __syncthreads();
     if (!last) return;
-    if (threadIdx.x == 0) *done = 0;
+    if (threadIdx.x == 0) __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int k = wave; k < NREP; k += DW) merge_head(a, bq, kvh * NREP + k, a.Hkv * NREP, nsplit, shares, lane);
 }
 

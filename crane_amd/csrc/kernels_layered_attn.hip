@@ -404,16 +404,12 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
             __shared__ int last;
             float* const po2 = a.part_o + (size_t)((int)blockIdx.y * a.G + g) * (4 * NNT * 256);
             float* const pm2 = a.part_ml + (size_t)((int)blockIdx.y * a.G + g) * 512;
-            // written through to where every XCD reads, and read from there: the counter needs no fence (fences write back and drop whole L2s: 18 us a launch became 52)
-            auto put = [](float* p, float x, float y) __attribute__((always_inline)) {
-                __hip_atomic_store((unsigned long long*)p, (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            };
             if (grp == 0) {
 #pragma unroll
                 for (int n = 0; n < NNT; ++n)
 #pragma unroll
-                    for (int r = 0; r < 4; r += 2) put(&po2[((wave * NNT + n) * 64 + lane) * 4 + r], o[n][r], o[n][r + 1]);
-                put(&pm2[(wave * 64 + lane) * 2], mn, l);
+                    for (int r = 0; r < 4; r += 2) put_through(&po2[((wave * NNT + n) * 64 + lane) * 4 + r], o[n][r], o[n][r + 1]);
+                put_through(&pm2[(wave * 64 + lane) * 2], mn, l);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
@@ -421,27 +417,23 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
             if (threadIdx.x == 0) last = atomicAdd(done, 1) == shares - 1;
             __syncthreads();
             if (!last || grp == 1) return;
-            if (threadIdx.x == 0) *done = 0;
-            auto get = [](const float* p) __attribute__((always_inline)) {
-                const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return make_float2(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)));
-            };
+            if (threadIdx.x == 0) __hip_atomic_store(done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const size_t stride = (size_t)a.G * (4 * NNT * 256);
             const float* p0 = po2 - share * stride, *m0 = pm2 - (size_t)share * a.G * 512;
             float M = -INFINITY;
-            for (int k = 0; k < shares; ++k) M = fmaxf(M, get(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]).x);
+            for (int k = 0; k < shares; ++k) M = fmaxf(M, get_through(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]).x);
             const float Ms = M == -INFINITY ? 0.f : M;
             l = 0.f;
 #pragma unroll
             for (int n = 0; n < NNT; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
             for (int k = 0; k < shares; ++k) {
-                const float2 ml = get(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]);
+                const float2 ml = get_through(&m0[(size_t)k * a.G * 512 + (wave * 64 + lane) * 2]);
                 f32x4 p[NNT];
 #pragma unroll
                 for (int n = 0; n < NNT; ++n)
 #pragma unroll
                     for (int r = 0; r < 4; r += 2) {
-                        const float2 v = get(&p0[k * stride + ((wave * NNT + n) * 64 + lane) * 4 + r]);
+                        const float2 v = get_through(&p0[k * stride + ((wave * NNT + n) * 64 + lane) * 4 + r]);
                         p[n][r] = v.x; p[n][r + 1] = v.y;
                     }
                 const float c = __builtin_amdgcn_exp2f(ml.x - Ms);
