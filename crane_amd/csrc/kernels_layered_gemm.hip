@@ -457,7 +457,8 @@ bool lay_tile_wide(const LTileArgs& a, bool beside) {
 // short ones, 2.6 and half a round for the ends.  us a launch, the two above / the shape taken, experts of 2048 x 4096 as above, weights out of memory:
 // gate-and-up 2048 tokens 465 / 397 (256 x 256), 1200 310 / 289 (192 x 128), 700 231 / 198 (192 x 128), 450 185 / 130 (128 x 192), 300 177 / 119, 200 126 / 113, 100 115 / 115 (64);
 // down 250 / 219, 167 / 156, 124 / 110, 92 / 83, 87 / 73, 69 / 62, 62 / 62.  14 experts of 768 x 1024, one of 512: 2048 tokens 47, 38 / 30 (192 x 128), 1300 43 / 33, 22, 500 24, 15.
-// One matrix, K 4096: 2048 rows, 6144 columns 135 / 111 (256 x 256), 4096 columns 76 (128)
+// One matrix, K 4096: 2048 rows, 6144 columns 136 / 100 (128 x 192; 256 x 256 109, 192 x 128 140), 8192 columns 155 / 114 (256 x 256; 192 x 128 149, 128 x 192 154), 4096 columns 79 (128; the others 89 to
+// 102); 1536 rows, 8192 columns 128 / 98 (192 x 128; 256 x 256 107)
 static LayTileShape lay_tile_least(const LTileArgs& a, const LTileArgs& b, float& least) {
     struct { LayTileShape shape; int bm, bn, slots; float round; } const all[] = {
         {LTILE_128, 128, 128, 512, 4.f}, {LTILE_192_128, 192, 128, 512, 5.f}, {LTILE_128_192, 128, 192, 512, 5.4f}, {LTILE_256, 256, 256, 256, 6.2f}};

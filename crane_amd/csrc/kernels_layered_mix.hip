@@ -349,6 +349,9 @@ bool lay_norm_router_fits(int W, int E, const RouterSpec& rs) {
 void launch_lay_norm_router(const LNormRouter& a, hipStream_t s) {
     if (a.T <= 0) return;
     const int logits = a.E + (a.rs.shared_gate ? 1 : 0), per_tok = logits + a.E + a.rs.groups + a.top;
+    // us, a row per block / eight, at 512, 768, 1024, 1280 and 2048 rows: width 512, 8 logits 8.1 / 9.1, 10.9 / 10.5, 11.1 / 9.8, 13.6 / 11.6, 17.5 / 14.5; 1024, 15 10.7 / 13.4, 12.2 / 14.7, 13.3 / 14.8, 15.9 /
+    // 15.7, 21.8 / 15.0, 32 11.5 / 14.6, 12.7 / 15.7, 14.9 / 16.5, 17.5 / 17.8, 23.2 / 16.6; 2048, 17 14.2 / 17.7, 16.4 / 17.2, 20.3 / 19.1, 23.7 / 20.0, 33.1 / 22.0; 4096, 17 20.4 / 25.6, 25.1 / 26.1, 31.0 / 26.6,
+    // 36.5 / 27.6, 53.2 / 34.0, 32 19.8 / 28.3, 25.0 / 29.0, 31.3 / 30.1, 37.4 / 31.3, 53.9 / 36.2: the two cross between 750 and 1350 rows, by no rule of width or logits
     const bool tile = a.T >= 1024;
     const int threads = tile ? 512 : 256, row_blocks = tile ? (a.T + 7) / 8 : a.T;
     const int tails = a.tail_segs > 0 && a.tail.taps > 1 ? a.tail_segs * ((a.tail.C + threads - 1) / threads) : 0;
