@@ -114,3 +114,26 @@ def test_position_blocks_and_sink(tmp_path, dim, vdim, heads, kv_heads, size, st
     assert _shares([(start, 30), (50, 1)], heads, kv_heads, 1 << 40)
     layers = [MO.layer("attention", None, **MO.attn(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, size=s)) for s in (size, None)]
     _run(tmp_path, MO, MO.config(layers, vocab=96, width=256), start)
+
+
+# a long walk of rows that are NaN beside a sound one, both shared: the sound rows keep the bits that they have beside other sound ones, and so does the next pass on the same counters
+@pytest.mark.gpu
+def test_rows_that_are_no_numbers(tmp_path):
+    from crane_amd.backend import Model
+    cfg = GZ.config([GZ.layer(GZ.attn(heads=4, kv_heads=2, dim=64, vdim=64, size=1024), None) for _ in range(2)], vocab=96, width=256)
+    assert len(_shares([(600, 30), (500, 30)], 4, 2, 1024)) == 4
+    P = GZ.random_weights(cfg, 8)
+    P["embed"][5] = np.nan
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=4, max_seq_len=768)
+    toks, got = 7 + np.array(GZ.tokens(660, 80, 9)), []
+    try:
+        for t in (5, 6):
+            a, b = m.seq_alloc(), m.seq_alloc()
+            m.step_batch([(a, toks[:600], []), (b, np.full(500, t), [])], want_logits=False)
+            rows = [m.step_batch([(a, toks[600 + 30 * k:630 + 30 * k], list(range(30))), (b, np.full(30, t), list(range(30)))])[0] for k in range(2)]
+            got.append(np.stack(rows))
+            m.seq_free(a)
+            m.seq_free(b)
+    finally:
+        m.close()
+    assert np.isnan(got[0][:, 30:]).all() and np.isfinite(got[1]).all() and (got[0][:, :30] == got[1][:, :30]).all()

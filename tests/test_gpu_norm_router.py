@@ -43,3 +43,28 @@ def test_tails_of_mixed_steps(tmp_path):
     finally:
         m.close()
     assert np.isfinite(got[0]).all() and np.abs(got[0] - got[1]).max() < 1e-3 * np.abs(got[1]).max()
+
+
+# rows that are NaN beside sound ones, in blocks of eight rows as in blocks of one: the sound rows keep the bits that they have beside other sound ones
+@pytest.mark.parametrize("n", [130, 1027])
+def test_rows_that_are_no_numbers(tmp_path, n):
+    import numpy as np
+
+    from crane_amd.backend import Model
+    cfg = GZ.config([GZ.layer(GZ.attn(heads=4, kv_heads=2, dim=64, vdim=64), GZ.moe(experts=15, top=4, ff=128, shared=128)) for _ in range(2)], vocab=96, width=192)
+    P = GZ.random_weights(cfg, 17)
+    P["embed"][5] = np.nan
+    m = Model.from_pretrained(GZ.write_checkpoint(str(tmp_path / "ckpt"), cfg, P), compute_dtype="bfloat16", max_seqs=4, max_seq_len=1280, prefill_chunk=2560)
+    toks, got = 7 + np.array(GZ.tokens(n, 80, 18)), []
+    try:
+        for t in (5, 6):
+            ss = [m.seq_alloc() for _ in range(3)]
+            step = [toks[:n - 16], np.full(3, t), toks[:13]]
+            got.append(m.step_batch([(s, x, list(range(len(x)))) for s, x in zip(ss, step)])[0])
+            for s in ss:
+                m.seq_free(s)
+    finally:
+        m.close()
+    bad = slice(n - 16, n - 13)
+    assert np.isnan(got[0][bad]).all() and np.isfinite(got[1]).all()
+    assert (np.delete(got[0], np.r_[bad], 0) == np.delete(got[1], np.r_[bad], 0)).all()
