@@ -579,6 +579,11 @@ int cm_debug_lay_router_plan(int32_t rows, int32_t width, int32_t outputs, int32
 
 int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats) { return cm::gemm_band(m, n, k, epi, (size_t)ws_floats, 0); }
 
+int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats) {
+    int bm = 0, bn = 0, ks = 0;
+    return cm::gemm_tile_plan(m, n, k, (size_t)ws_floats, norm != 0, &bm, &bn, &ks, nullptr) ? bm * 10000 + bn * 10 + ks : 0;
+}
+
 int cm_debug_attn_group_plan(int32_t pairs, int32_t nrep, int64_t longest, int32_t slices, int32_t num_cu, int32_t most) {
     return cm::attn_decode_group_pays(pairs, nrep, longest, slices != 0, num_cu) ? cm::attn_decode_group_split(longest, pairs, num_cu, most) : 0;
 }

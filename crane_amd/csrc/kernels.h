@@ -164,6 +164,10 @@ struct GemmArgs {
 // and the launch (a.ksplit set; more than one slice: partial tiles in a.ws)
 bool gemm_rows_plan(int M, int N, int K, size_t ws_floats, int* bn, int* ks);
 bool launch_gemm_rows(const GemmArgs& a, int epi, int bn, hipStream_t s);
+// more than 128 rows with hi + lo activations (kernels_gemm_tile.hip): what a tile shape takes, in seconds (host rule), the shape and K slices that take least, the launch
+double gemm_tile_seconds(int M, int N, int K, int bm, int bn, int ks, bool norm);
+bool gemm_tile_plan(int M, int N, int K, size_t ws_floats, bool norm, int* bm, int* bn, int* ks, double* seconds);
+bool launch_gemm_tile(const GemmArgs& a, int epi, int bm, int bn, hipStream_t s);
 // prompt rows with hi + lo activations: how many of them a first launch takes where two cost less than one, 0 where they don't (host rule)
 int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap);
 

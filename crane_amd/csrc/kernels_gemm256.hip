@@ -1,7 +1,7 @@
 // Prompt-pass GEMM for LARGE M fed by LDS-DMA in FULL cache lines:  C[M, N] (+)= A[M, K] . W[N, K]^T, bf16 operands, f32
 // accumulate, the activation operand as one bf16 plane (SPLIT = 1) or as bf16 hi + lo planes (SPLIT = 2, the parity mode: two
-// MFMAs per product).  Same epilogues and, per accumulator, the same sequence of MFMAs (k ascending; hi then lo) as
-// gemm_bf16_kernel (kernels_prefill.hip): an un-split launch of several row tiles is bit-equal to that kernel's, but for tanh-gelu (one row tile: another k start per column tile).
+// MFMAs per product; up to 128 rows, more are kernels_gemm_tile.hip's).  Same epilogues and, per accumulator, the same sequence of MFMAs (k ascending; hi then lo) as
+// gemm_bf16_kernel (kernels_prefill.hip): an un-split launch of plain bf16 rows is bit-equal to that kernel's, but for tanh-gelu (hi + lo: another k start per column tile).
 //
 // Why a second kernel -- what that kernel's 47 % MFMA-busy was waiting for.  gemm_bf16_kernel walks K in 32-element
 // k-tiles: every operand row contributes a 64-byte segment per tile, i.e. HALF of a 128-byte cache line, and the other half is
@@ -19,7 +19,7 @@
 //   * two LDS stages + the register file as the third, and the two wave rows of the workgroup half a tile apart: one row
 //     multiplies from registers while the other fetches the next tile's fragments (schedule comment in the kernel).  The DMA
 //     is issued from inline asm: the compiler's own wait-count pass would make every ds_read wait for ALL outstanding LDS-DMA;
-//   * parity mode: 128 x BN x 64 tiles (two activation planes: 64 KB per stage at BN = 256); plain bf16: 256 x BN x 64;
+//   * parity mode: one tile of 128 (or 64) rows x BN x 64; plain bf16: 256 x BN x 64;
 //     8 waves as 2 (M) x 4 (N); BN = 256 or 192 (whole rounds of 256 CUs: N = 24576 at M = 1024).
 #include <cstdlib>
 
@@ -50,13 +50,13 @@ __device__ __forceinline__ void put_words(uint16_t* p, const uint32_t (&w)[NW]) 
 
 }  // namespace
 
-// WST = 3 (decode groups: one m-tile, the weights come from HBM, not from a neighbour's L2 lines): a THIRD weight stage, the
+// WST = 3 (parity mode: one m-tile, the weights come from HBM, not from a neighbour's L2 lines): a THIRD weight stage, the
 // weight requests running two k-tiles ahead (the activation stages stay at two).  With two stages a workgroup has one 32 KB weight
 // tile in flight; 96-192 workgroups of a 128-row launch are then 3-6 MB in flight chip-wide -- about 3 TB/s at the ~2 us of a loaded
 // HBM round trip, which is what the launch measured.  The waits become counted: the newest weight requests may stay outstanding.
 // BMX = 64 (parity mode): 64-row tiles for decode groups of <= 64 sequences -- half the activation bytes and half the MFMAs
 // of a 128-row tile whose upper half would be padding.
-template <int SPLIT, int EPI, int BN, int WST = 2, int BMX = 0>
+template <int SPLIT, int EPI, int BN, int BMX = 0>
 __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
     constexpr int BM = BMX ? BMX : (SPLIT == 2 ? 128 : 256);              // rows of a tile (two planes double the activation bytes)
     constexpr int NI = BM / 32, NJ = BN / 64, WM = BM / 2, WN = BN / 4;  // per wave: NI x NJ tiles of 16 x 16
@@ -66,7 +66,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmArgs a) {
     // NEAR (16-bit outputs): row 4 g + r of weight fragment j is column 4 NJ g + 4 j + r of the wave's, so that a lane's 4 NJ columns are neighbours (f32
     // outputs in that order: pieces of a 64-byte row in four instructions, 130 us in the place of 117).  A workgroup that walks over several tiles, the next one's
     // first requests in front of this one's stores, was slower by what its registers cost the loop: 2500 tokens of the 8B model 66.5 -> 73.3 ms
-    constexpr bool NEAR = EPI == GEPI_ACT_SPLIT || EPI == GEPI_SILUMUL, SWAP = NEAR || (WST == 2 && EPI != GEPI_PARTIAL);
+    constexpr bool NEAR = EPI == GEPI_ACT_SPLIT || EPI == GEPI_SILUMUL, SWAP = NEAR || (SPLIT == 1 && EPI != GEPI_PARTIAL);
+    constexpr int WST = SPLIT == 2 ? 3 : 2;
     constexpr int PLANE = BM * TBK;                                       // elements of one activation plane of a stage
     constexpr int ASTAGE = SPLIT * PLANE, WSTAGE = BN * TBK;             // elements of an activation / a weight stage
     constexpr int WBASE = TST * ASTAGE;                                   // LDS image: [TST activation stages][WST weight stages]
@@ -394,14 +395,14 @@ int gemm256_rows(bool split, int M) {
     static const int bm64 = getenv("CM_GEMM256_BM64") ? atoi(getenv("CM_GEMM256_BM64")) : 1;
     return split ? ((M <= 64 && bm64) ? 64 : 128) : 256;
 }
-static size_t gemm256_lds(int split, int bm, int bn, int wst = 2) { return ((size_t)TST * split * bm * TBK + (size_t)wst * bn * TBK) * 2; }
+static size_t gemm256_lds(int split, int bm, int bn) { return ((size_t)TST * split * bm * TBK + (size_t)(split + 1) * bn * TBK) * 2; }
 
-template <int SPLIT, int EPI, int BN, int WST = 2, int BMX = 0>
+template <int SPLIT, int EPI, int BN, int BMX = 0>
 static void launch_one(const GemmArgs& a, int blocks, hipStream_t s) {
     static DevOnce attr;
-    const size_t lds = gemm256_lds(SPLIT, BMX ? BMX : (SPLIT == 2 ? 128 : 256), BN, WST);
-    attr.run([&] { (void)hipFuncSetAttribute((const void*)gemm256_kernel<SPLIT, EPI, BN, WST, BMX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
-    hipLaunchKernelGGL((gemm256_kernel<SPLIT, EPI, BN, WST, BMX>), dim3(blocks), dim3(512), lds, s, a);
+    const size_t lds = gemm256_lds(SPLIT, BMX ? BMX : (SPLIT == 2 ? 128 : 256), BN);
+    attr.run([&] { (void)hipFuncSetAttribute((const void*)gemm256_kernel<SPLIT, EPI, BN, BMX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+    hipLaunchKernelGGL((gemm256_kernel<SPLIT, EPI, BN, BMX>), dim3(blocks), dim3(512), lds, s, a);
 }
 
 // a.ksplit set by the caller (1: epilogue `epi`; > 1: GEPI_PARTIAL tiles, the caller runs gemm_splitk_epilogue_kernel)
@@ -413,13 +414,9 @@ bool launch_gemm256(const GemmArgs& a, int epi, int bn, hipStream_t s) {
     const int bm = gemm256_rows(split, a.M);
     const int blocks = ((a.M + bm - 1) / bm) * (a.N / bn) * a.ksplit;
     const int e = a.ksplit > 1 ? (int)GEPI_PARTIAL : epi;
-    // three weight stages (WST = 3): parity-mode tiles (160 KB of LDS at 256 columns, 136 KB at 192); by default for one-m-tile launches (decode
-    // groups: the weights stream from HBM), CM_GEMM256_WST = 2 never, 3 always (A/B)
-    static const int wst_env = getenv("CM_GEMM256_WST") ? atoi(getenv("CM_GEMM256_WST")) : 0;
-    const bool w3 = split && (wst_env == 3 || (wst_env == 0 && a.M <= bm)) && a.K / TBK / a.ksplit >= 3;
-#define CM_G256(SP, EP) do { if (SP == 2 && bm == 64) { if (bn == 256) launch_one<2, EP, 256, 3, 64>(a, blocks, s); else launch_one<2, EP, 192, 3, 64>(a, blocks, s); } \
-                             else if (bn == 256) { if (SP == 2 && w3) launch_one<2, EP, 256, 3>(a, blocks, s); else launch_one<SP, EP, 256>(a, blocks, s); } \
-                             else { if (SP == 2 && w3) launch_one<2, EP, 192, 3>(a, blocks, s); else launch_one<SP, EP, 192>(a, blocks, s); } } while (0)
+    if (split && (a.M > bm || a.K / TBK / a.ksplit < 3)) return false;     // (one row tile: three weight stages; more rows: kernels_gemm_tile.hip)
+#define CM_G256(SP, EP) do { if (SP == 2 && bm == 64) { if (bn == 256) launch_one<2, EP, 256, 64>(a, blocks, s); else launch_one<2, EP, 192, 64>(a, blocks, s); } \
+                             else if (bn == 256) launch_one<SP, EP, 256>(a, blocks, s); else launch_one<SP, EP, 192>(a, blocks, s); } while (0)
 #define CM_G256_EPI(SP) do { if (e == GEPI_STORE) CM_G256(SP, GEPI_STORE); else if (e == GEPI_RESADD) CM_G256(SP, GEPI_RESADD); \
         else if (e == GEPI_ACT_SPLIT) CM_G256(SP, GEPI_ACT_SPLIT); else if (e == GEPI_SILUMUL) CM_G256(SP, GEPI_SILUMUL); \
         else CM_G256(SP, GEPI_PARTIAL); } while (0)

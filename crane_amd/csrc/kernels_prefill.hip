@@ -1218,9 +1218,8 @@ static void launch_splitk(GemmArgs& a, int epi, hipStream_t s) {
     else launch_splitk_epilogue<GEPI_SILUMUL>(a, eb, s);
 }
 
-// Large M (>= 512 rows): the LDS-DMA kernel on full cache lines (kernels_gemm256.hip; 128-row tiles with hi + lo activations,
-// 256-row tiles with plain bf16) where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost
-// model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
+// The LDS-DMA kernel on full cache lines (kernels_gemm256.hip; one tile of up to 128 rows with hi + lo activations, 256-row tiles with plain bf16 from 512 rows on)
+// where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
 // register-staged kernel should run.
 // the column tile and the K slices of such a product; false: not for that kernel
 static bool gemm256_plan(int M, int N, int K, bool lo, size_t ws_floats, bool w4, int* bn_out, int* ks_out) {
@@ -1268,7 +1267,14 @@ static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
     static const int w4_env = getenv("CM_GEMMW4") ? atoi(getenv("CM_GEMMW4")) : 0;
     static const int w4_min = getenv("CM_GEMMW4_MIN_M") ? atoi(getenv("CM_GEMMW4_MIN_M")) : 65;
     const bool w4 = a.wide256 == 2 || (a.wide256 == 1 && w4_env != 0 && a.M >= w4_min);
-    int bn = 0, ks = 1;
+    int bm = 0, bn = 0, ks = 1;
+    if (!w4 && a.A_lo != nullptr && a.M > 128) {                 // hi + lo prompts: kernels_gemm_tile.hip
+        if (!gemm_tile_plan(a.M, a.N, a.K, a.ws ? a.ws_floats : 0, a.norm_w != nullptr, &bm, &bn, &ks, nullptr)) return false;
+        a.ksplit = ks;
+        if (!launch_gemm_tile(a, epi, bm, bn, s)) return false;
+        if (ks > 1) launch_splitk(a, epi, s);
+        return true;
+    }
     if (!gemm256_plan(a.M, a.N, a.K, a.A_lo != nullptr, a.ws ? a.ws_floats : 0, w4, &bn, &ks)) return false;
     a.ksplit = ks;
     if (w4) { if (!launch_gemmw4(a, epi, bn, s)) return false; }
@@ -1348,10 +1354,10 @@ static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {
     if (a.bias != nullptr) rest.bias = a.bias + most.N;
     return launch_gemm_once(rest, epi, s);
 }
-// What M rows of a product with hi + lo activations take on the kernel that launch_gemm_once finds for them, in seconds: rounds of blocks, a 64-deep k-tile of 128 x 256 outputs
-// 1.44 us and about 13 us a block around them (measured / so: 24576 x 4096 at 300, 650, 1000, 1400 rows 164 / 164, 248 / 246, 313 / 315, 502 / 493 us); two blocks
+// What M rows of a product with hi + lo activations take, in seconds.  On tiles of 128 rows (tall: on those of kernels_gemm_tile.hip by their own figures): rounds of blocks, a 64-deep
+// k-tile of 128 x 256 outputs 1.44 us and about 13 us a block around them (measured / so: 24576 x 4096 at 300, 650, 1000, 1400 rows 164 / 164, 248 / 246, 313 / 315, 502 / 493 us); two blocks
 // of 128 x 128 on a CU 1.6 and 10; products of at most 128 rows by their weights
-static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
+static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap, bool tall) {
     int bn = 0, ks = 0;
     const auto split = [&](int cols) { return ks > 1 ? (double)(2 * ks + 1) * M * cols * 4.0 / 5e12 + 4e-6 : 0.0; };
     if (epi != GEPI_ACT_SPLIT && gemm_rows_plan(M, N, K, ws_floats, &bn, &ks)) {
@@ -1361,19 +1367,22 @@ static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int k
     const int tiles_m = (M + 127) / 128;
     const bool tail = epi == GEPI_STORE && gemm_tail_columns(M, N);
     const int cols = N - (tail ? 128 : 0);
-    if (gemm256_plan(M, cols, K, true, ws_floats, false, &bn, &ks))
+    int bm = 0;
+    double best = 0.0;
+    if (tall && gemm_tile_plan(M, cols, K, ws_floats, epi == GEPI_RESADD, &bm, &bn, &ks, &best)) return best + (tail ? 15e-6 : 0.0);
+    if ((!tall || M <= 128) && gemm256_plan(M, cols, K, true, ws_floats, false, &bn, &ks))
         return (tiles_m * (cols / bn) * ks + 255) / 256 * (K / 64 / ks * 1.44e-6 * bn / 256 + 13e-6) + split(cols) + (tail ? 15e-6 : 0.0);
     ks = gemm_ksplit(M, N, tiles_m * (N / 128), K / GBK, ws_floats, ksplit_cap);
     return (tiles_m * (N / 128) * ks + 511) / 512 * (K / 64 / ks * 1.6e-6 + 10e-6) + split(N);
 }
-// the rows of the first of two bands that take less time than all rows at once; 0: all at once
+// the rows of the first of two bands that take less time than all rows at once on tiles of 128; 0: all at once
 int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
     if (M <= 256 || N % 128 != 0 || K % 64 != 0 || epi == GEPI_ACT_SPLIT) return 0;
-    const double whole = gemm_seconds(M, N, K, epi, ws_floats, ksplit_cap);
+    const double whole = gemm_seconds(M, N, K, epi, ws_floats, ksplit_cap, false);
     double least = std::min(0.95 * whole, whole - 8e-6);
     int rows = 0;
     for (int m = (M - 9) / 128 * 128; m >= 128 && M - m <= 1024; m -= 128) {
-        const double t = gemm_seconds(m, N, K, epi, ws_floats, ksplit_cap) + gemm_seconds(M - m, N, K, epi, ws_floats, ksplit_cap) + 2e-6;
+        const double t = gemm_seconds(m, N, K, epi, ws_floats, ksplit_cap, false) + gemm_seconds(M - m, N, K, epi, ws_floats, ksplit_cap, false) + 2e-6;
         if (t < least) { least = t; rows = m; }
     }
     return rows;
@@ -1385,8 +1394,13 @@ int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
 // ms, 560 4.30 / 4.41: a launch and a reduction more for a round of 30 us).  Rows of products with an activation behind them and the vision tower's norm stay in one launch (not measured).
 static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
     if (a.A_lo == nullptr || a.defer_ks != nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
-    const int m = gemm_band(a.M, a.N, a.K, epi, a.ws ? a.ws_floats : 0, a.ksplit_cap);
+    const size_t ws = a.ws ? a.ws_floats : 0;
+    const int m = gemm_band(a.M, a.N, a.K, epi, ws, a.ksplit_cap);
     if (m == 0) return false;
+    // larger tiles and wider ones leave fewer rounds nearly empty: 300 rows of 24576 x 4096 123 us in one launch, 44 more for 44 rows behind 256
+    const double whole = gemm_seconds(a.M, a.N, a.K, epi, ws, a.ksplit_cap, true);
+    const double two = gemm_seconds(m, a.N, a.K, epi, ws, a.ksplit_cap, true) + gemm_seconds(a.M - m, a.N, a.K, epi, ws, a.ksplit_cap, true) + 2e-6;
+    if (two >= std::min(0.95 * whole, whole - 8e-6)) return false;
     const size_t hcols = epi == GEPI_SILUMUL ? (size_t)a.N / 2 : (size_t)a.N;
     for (int part = 0; part < 2; ++part) {
         const size_t r0 = part ? (size_t)m : 0;

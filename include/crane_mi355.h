@@ -548,6 +548,9 @@ int cm_debug_lay_attn_shares(const int32_t* starts, const int32_t* rows, int32_t
 /* Test hook: how many of m prompt rows the first of two launches of an m x k by k x n product takes (epi: 0 store, 1 add, 2 SiLU product, 3 activation); 0: one launch. */
 int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws_floats);
 
+/* Test hook (host logic only, no GPU): rows * 10000 + columns * 10 + K slices of the tiles that m prompt rows of such a product run on (norm: one of the rows behind it); 0: another kernel. */
+int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats);
+
 /* Test hook (host logic only, no GPU): among how many blocks the prompt attention shares the keys of a query tile: `rows` queries behind `start` cached
  * tokens, `heads` query heads of 128 or 256. */
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim);
