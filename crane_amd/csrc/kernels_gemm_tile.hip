@@ -23,12 +23,6 @@ namespace cm {
 
 namespace {
 
-// 16 bytes per lane from base + off to lds_base + 16 lane (lds_load16 with the base in scalar registers)
-__device__ __forceinline__ void lds_load16_at(const char* base, uint32_t off, uint32_t lds_base) {
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_base) : "memory");
-}
 // silu(g) u as g / (1 + e^-g) with the hardware's exponential and reciprocal (expf and a division: 11 us of a 256 x 256 tile's 190)
 __device__ __forceinline__ float silu_mul(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u; }
 template <int NW>

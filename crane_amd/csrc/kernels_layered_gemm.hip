@@ -232,13 +232,14 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
 }
 
 // 256 x 256 tiles, eight waves as 2 x 4, a wave 128 x 64 outputs: 24 KB of fragments for 64 products a k-tile, three quarters of what the 64 x 64 of the
-// kernel above ask the LDS for per product.  The schedule of gemm256_kernel (kernels_gemm256.hip): the two wave rows run half a tile apart, one multiplies a tile
-// from registers while the other fetches its fragments of the next and requests the tile behind it, a request between two bands of products.  A band of 16 rows
+// kernel above ask the LDS for per product.  The two wave rows run half a tile apart: in one slot a row fetches its fragments of a tile, in the next it multiplies, the other row the other way
+// round.  The first slot of tile t asks for the rows of tile t + 1, the second for the weights of tile t + 2 (three stages of those: 160 KB), a request between two bands of products: 32 requests
+// of 16 cycles each per slot of 1024 (both for t + 1 in the first slot, which they filled: 8192 rows, 16 experts of 2048 x 4096 and one of every token, gate-and-up / down 350 / 212 us, here 337 / 202).  A band of 16 rows
 // behind a ragged tile's end multiplies nothing.  8192 rows, 4096 columns, K 4096: 359 us on 128 x 128 tiles, 228 - 305 here by what the clock allows (183 with
 // operands of zeros: 1.5 PFLOP/s)
 template <bool DUAL>
 __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTileArgs second, int ntiles, int ntiles_b) {
-    constexpr int BM = 256, BN = 256, WM = 128, WN = 64, NI = 8, NJ = 4, NL = 8, NC = DUAL ? WN / 2 : WN, APC = BM / 8, STAGE = (BM + BN) * BK;
+    constexpr int BM = 256, BN = 256, WM = 128, WN = 64, NI = 8, NJ = 4, NL = 4, NC = DUAL ? WN / 2 : WN, STAGE = 256 * BK, WBASE = 2 * STAGE;
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -250,39 +251,26 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
     if (a.a_idx) a.a_idx += at.shift;
     if (a.c_idx) a.c_idx += at.shift;
     const int p0 = at.p0, rows = at.rows;
-    const uint16_t* W = a.W + (size_t)at.g * a.w_stride;
-    const uint16_t* W2 = DUAL ? a.W2 + (size_t)at.g * a.w_stride : nullptr;
     const int n0 = at.nt * (DUAL ? BN / 2 : BN);
 
-    // loads as above: piece wave + 8 i covers 8 rows of A (i < 4) or of the weight tile
-    const int prow = lane >> 3, pslot = lane & 7;
+    // loads as above: piece wave + 8 i covers 8 rows of A, and as many of the weight tile, a wave's all in W or all in W2.  32-bit offsets from bases in scalar registers: 16
+    // vector registers for pointers are 8 too many (launch_lay_tile_gemm: the rows of A are within reach)
+    const int r0 = wave * 8 + (lane >> 3), slot = lane & 7;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
-    const uint16_t* src[NL];
-    uint32_t dst[NL];
+    const char* const A0 = (const char*)a.A;
+    const char* const W0 = (const char*)((DUAL && (wave & 4) ? a.W2 : a.W) + (size_t)at.g * a.w_stride + (size_t)n0 * a.K);
+    uint32_t aoff[NL], woff[NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-        const int p = wave + 8 * i;
-        const bool isA = p < APC;
-        const int row = (isA ? p : p - APC) * 8 + prow;
-        const int kc = (pslot ^ ((row >> 1) & 7)) << 3;
-        if (isA) {
-            const int r = p0 + min(row, rows - 1);
-            src[i] = a.A + (size_t)(a.a_idx ? a.a_idx[r] / a.a_div : r) * a.lda + kc;
-        } else {
-            const int c = row / WN, q = row - c * WN;
-            const bool up = DUAL && q >= NC;
-            src[i] = (up ? W2 : W) + (size_t)min(n0 + c * NC + (up ? q - NC : q), a.N - 1) * a.K + kc;
-        }
-        dst[i] = lds0 + (uint32_t)(p * 8 * BK) * 2u;
+        const int r = p0 + min(i * 64 + r0, rows - 1);
+        const uint32_t kc = (uint32_t)(slot ^ ((r0 >> 1) & 7)) << 4;
+        aoff[i] = (uint32_t)(a.a_idx ? a.a_idx[r] / a.a_div : r) * (uint32_t)(a.lda * 2) + kc;
+        woff[i] = (uint32_t)min(i * NC + (DUAL ? r0 & 31 : r0), a.N - 1 - n0) * (uint32_t)(a.K * 2) + kc;
     }
     const int nk = a.K / BK;
-    auto piece = [&](int i, int t) __attribute__((always_inline)) {       // past the end: the last tile again, into a stage nobody reads
-        lds_load16(src[i] + (size_t)min(t, nk - 1) * BK, dst[i] + (uint32_t)((t & 1) * STAGE) * 2u);
-    };
-    auto request = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NL; ++i) piece(i, t);
-    };
+    // (past the end: the last tile again, into a stage nobody reads)
+    auto ask_a = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(A0 + (size_t)min(t, nk - 1) * (BK * 2), aoff[i], lds0 + (uint32_t)((t & 1) * STAGE + (wave + 8 * i) * 8 * BK) * 2u); };
+    auto ask_w = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(W0 + (size_t)min(t, nk - 1) * (BK * 2), woff[i], lds0 + (uint32_t)(WBASE + t % 3 * STAGE + (wave + 8 * i) * 8 * BK) * 2u); };
     f32x4 acc[NI][NJ];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -293,7 +281,7 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
     bf16x8 af[2][NI], bf[2][NJ];
     auto fetch = [&](int t) __attribute__((always_inline)) {
         const uint16_t* As = lds + (t & 1) * STAGE + wm * WM * BK;
-        const uint16_t* Bs = lds + (t & 1) * STAGE + (BM + wn * WN) * BK;
+        const uint16_t* Bs = lds + WBASE + t % 3 * STAGE + wn * WN * BK;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int fk = ((s * 4 + lg) ^ sw) << 3;
@@ -307,41 +295,46 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[s][j], af[s][i], acc[i][j], 0, 0, 0);
     };
-    // every wave runs 2 nk + 2 barriers
-    request(0);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // a slot's products with its requests between the bands
+    auto multiply = [&](auto ask) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if (i < bands) { band(0, i); band(1, i); }
+            __builtin_amdgcn_sched_barrier(0);
+            if (i < NL) ask(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // every wave runs 2 nk + 2 barriers.  What is asked for in the second slot of a tile, the newest NL requests, may stay in flight at its end
+#pragma unroll
+    for (int i = 0; i < NL; ++i) { ask_a(i, 0); ask_w(i, 0); }
+#pragma unroll
+    for (int i = 0; i < NL; ++i) ask_w(i, 1);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NL) : "memory");
     if (wm == 0) {
         for (int t = 0; t < nk; ++t) {
-            request(t + 1);
+#pragma unroll
+            for (int i = 0; i < NL; ++i) ask_a(i, t + 1);
             fetch(t);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-                if (i < bands) { band(0, i); band(1, i); }
-            __builtin_amdgcn_s_setprio(0);
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+            multiply([&](int i) __attribute__((always_inline)) { ask_w(i, t + 2); });
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NL) : "memory");
         }
         asm volatile("s_barrier" ::: "memory");
     } else {
-        request(1);                                                       // in the slot in which row 0 fetches tile 0
+#pragma unroll
+        for (int i = 0; i < NL; ++i) ask_a(i, 1);                         // in the slot in which row 0 fetches tile 0
         asm volatile("s_barrier" ::: "memory");
         for (int t = 0; t < nk; ++t) {
-            fetch(t);
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                if (i < bands) { band(0, i); band(1, i); }
-                __builtin_amdgcn_sched_barrier(0);
-                piece(i, t + 2);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            __builtin_amdgcn_s_setprio(0);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < NL; ++i) ask_w(i, t + 2);
+            fetch(t);
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NL) : "memory");
+            multiply([&](int i) __attribute__((always_inline)) { ask_a(i, t + 2); });
             asm volatile("s_barrier" ::: "memory");
         }
     }
@@ -368,7 +361,7 @@ void go(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
 }
 template <bool DUAL>
 void go_tall(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
-    constexpr size_t lds = (size_t)2 * 512 * BK * sizeof(uint16_t);
+    constexpr size_t lds = (size_t)5 * 256 * BK * sizeof(uint16_t);
     static DevOnce attr;
     attr.run([&] { (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tall_gemm_kernel<DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
     const int cols = DUAL ? 128 : 256, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
@@ -470,7 +463,9 @@ static LayTileShape lay_tile_least(const LTileArgs& a, const LTileArgs& b, float
     LayTileShape best = wide ? LTILE_128 : LTILE_64;
     least = wide ? 4.f * std::ceil(blocks(128, 128) / 512.f) : 2.6f * (blocks(64, 64) / 768.f + 0.5f);
     if (!a.W2 && !(plain_out(a) && (b.M <= 0 || plain_out(b)))) return best;      // (the large tiles' stores know no bias and no function)
+    auto near = [](const LTileArgs& x) { return (uint64_t)std::max(x.total, x.M) * x.lda * 2 + (uint64_t)x.K * 2 < 1ull << 32; };      // (lay_tall_gemm_kernel's offsets)
     for (const auto& c : all) {
+        if (c.shape == LTILE_256 && !(near(a) && near(b))) continue;
         const float t = c.round * std::ceil(blocks(c.bm, c.bn) / (float)c.slots);
         if (t < least) { least = t; best = c.shape; }
     }
