@@ -81,6 +81,36 @@ __device__ __forceinline__ f32x4 mma_k16(const bf16x4& a, const bf16x4& b, const
     else return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
+// four f32 as bf16 hi + lo planes; four weights as two terms of the pages' type
+__device__ __forceinline__ void split_store4(uint16_t* hi, uint16_t* lo, size_t off, const float v[4]) {
+    uint16_t h[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = f32_to_bf16(v[i]);
+        l[i] = f32_to_bf16(v[i] - bf16_to_f32(h[i]));
+    }
+    *(u32x2*)(hi + off) = (u32x2){(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
+    if (lo) *(u32x2*)(lo + off) = (u32x2){(uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16)};
+}
+template <int KVT>
+__device__ __forceinline__ void p_split4(const float (&p)[4], bf16x4& hi, bf16x4& lo) {
+    if constexpr (KVT == KV_F16) {
+        typedef __attribute__((ext_vector_type(2))) _Float16 h2;
+        const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[0], p[1]));
+        const h2 b = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[2], p[3]));
+        const h2 c = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[0] - (float)a[0], p[1] - (float)a[1]));
+        const h2 d = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[2] - (float)b[0], p[3] - (float)b[1]));
+        const u32x2 hv = {__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)};
+        const u32x2 lv = {__builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)};
+        hi = __builtin_bit_cast(bf16x4, hv); lo = __builtin_bit_cast(bf16x4, lv);
+    } else {
+        const uint32_t a = pack_bf16x2(p[0], p[1]), b = pack_bf16x2(p[2], p[3]);
+        const uint32_t c = pack_bf16x2(p[0] - bf16_lo(a), p[1] - bf16_hi(a)), d = pack_bf16x2(p[2] - bf16_lo(b), p[3] - bf16_hi(b));
+        const u32x2 hv = {a, b}, lv = {c, d};
+        hi = __builtin_bit_cast(bf16x4, hv); lo = __builtin_bit_cast(bf16x4, lv);
+    }
+}
+
 // ---- streaming (non-temporal) 16-byte load: weights are read once ----------
 __device__ __forceinline__ u32x4 ld_nt16(const void* p) {
     return __builtin_nontemporal_load((const u32x4*)p);
@@ -91,6 +121,43 @@ __device__ __forceinline__ u32x4 ld16(const void* p) { return *(const u32x4*)p; 
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+// The value of lane l ^ 1, 2, 4, 8, 16 without the LDS (a __shfl_xor is a ds_bpermute, about 100 cycles in a chain that waits for it; these are 4 .. 8).  Both lanes of a pair active.
+// permlane16_swap(v, v): {rows 0 0 2 2, rows 1 1 3 3} of 16 lanes; permlane32_swap(v, v): {lower half twice, upper half twice}
+typedef __attribute__((ext_vector_type(2))) unsigned int cm_u32x2;
+__device__ __forceinline__ cm_u32x2 rows16(float v) { return __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false); }
+__device__ __forceinline__ cm_u32x2 rows32(float v) { return __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false); }
+template <int X>
+__device__ __forceinline__ float lane_xor(float v) {
+    static_assert(X == 1 || X == 2 || X == 4 || X == 8 || X == 16, "");
+    if constexpr (X == 1) return dpp_mov<0xB1>(v);                    // quad_perm [1,0,3,2]
+    else if constexpr (X == 2) return dpp_mov<0x4E>(v);               // quad_perm [2,3,0,1]
+    else if constexpr (X == 4) return dpp_mov<0x141>(dpp_mov<0x1B>(v));   // row_half_mirror (l ^ 7) of quad_perm [3,2,1,0] (l ^ 3)
+    else if constexpr (X == 8) return dpp_mov<0x128>(v);              // row_ror 8
+    else { const cm_u32x2 r = rows16(v); return __uint_as_float(threadIdx.x & 16 ? r[0] : r[1]); }
+}
+// v summed, or its maximum taken, over lanes l, l ^ 16 and then l ^ 32
+__device__ __forceinline__ float rows_sum(float v) {
+    cm_u32x2 r = rows16(v);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = rows32(v);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float rows_max(float v) {
+    cm_u32x2 r = rows16(v);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = rows32(v);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// sum over an aligned group of L lanes (a power of two), partners L / 2 apart first
+__device__ __forceinline__ float group_sum(float v, int L) {
+    if (L > 32) { const cm_u32x2 r = rows32(v); v = __uint_as_float(r[0]) + __uint_as_float(r[1]); }
+    if (L > 16) { const cm_u32x2 r = rows16(v); v = __uint_as_float(r[0]) + __uint_as_float(r[1]); }
+    if (L > 8) v += lane_xor<8>(v);
+    if (L > 4) v += lane_xor<4>(v);
+    if (L > 2) v += lane_xor<2>(v);
+    if (L > 1) v += lane_xor<1>(v);
+    return v;
 }
 // sum over each aligned group of 16 lanes ("row"); every lane of the row gets it
 __device__ __forceinline__ float row16_sum(float v) {

@@ -883,8 +883,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnDecArgs a) {
             if (tb + g * 4 + r >= limit) sc[r] = -INFINITY;
             mt = fmaxf(mt, sc[r]);
         }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = rows_max(mt);
         const float m_new = fmaxf(m_run, mt);                    // finite: token tb < limit is in this tile
         const float alpha = expf(m_run - m_new);
         float psum = 0.f;
@@ -948,8 +947,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(AttnDecArgs a) {
             step(kA, vA, ksA, vsA, pos, pos + 1);
         }
     }
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
+    l_run = rows_sum(l_run);
 
     // ---- merge the 4 waves: O^T rows = dims nt*16 + g*4 + r, column = head `sub` ----
     __syncthreads();

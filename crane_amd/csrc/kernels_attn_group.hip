@@ -263,8 +263,7 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
                 s[tt][r] = tt * 16 + lg * 4 + r <= own ? sc : -INFINITY;
                 mt = fmaxf(mt, s[tt][r]);
             }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = rows_max(mt);
         const float mn = fmaxf(m, mt);
         const float corr = expf(m - mn);
         l *= corr;
@@ -308,8 +307,7 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
                 o[n] = mma_k32<KVT>(vf, p[h], o[n]);
             }
     }
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = rows_sum(l);
     if (lg == 0) red_m[wave][lr] = m;
     __syncthreads();                                              // every wave's tile has been read: its place holds the sums
 #pragma unroll
@@ -371,8 +369,7 @@ __global__ __launch_bounds__(DW * 64, 2) void attn_decode_group_kernel(AttnDecAr
             for (int r = 0; r < 4; ++r) am = fmaxf(am, fabsf(v[j][r]));
         }
         if (!a.out1_q) continue;
-        am = fmaxf(am, __shfl_xor(am, 16));
-        am = fmaxf(am, __shfl_xor(am, 32));
+        am = rows_max(am);
         float id;
         const float dq = q8_scale(am, id);
 #pragma unroll

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? (PIPE ? 3 : 4) : 2) void gemv_bf
             // multiples of 32, so a half-wave is active as a whole): sum of squares over the head with five xor steps
             f32x4 v = *(const f32x4*)(a.x + (k4i << 2));
             float ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-            ss += __shfl_xor(ss, 1); ss += __shfl_xor(ss, 2); ss += __shfl_xor(ss, 4); ss += __shfl_xor(ss, 8); ss += __shfl_xor(ss, 16);
+            ss += lane_xor<1>(ss); ss += lane_xor<2>(ss); ss += lane_xor<4>(ss); ss += lane_xor<8>(ss); ss += lane_xor<16>(ss);
             const float rms = 1.0f / sqrtf(ss / 128.0f + a.eps);
             const f32x4 z = *(const f32x4*)(a.gdn_z + (k4i << 2));
             const f32x4 w = *(const f32x4*)(a.gdn_w + ((k4i & 31) << 2));

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs a) {
         for (int j = 0; j < KS; ++j) y += part[j][tid];
         __hip_atomic_store(&yraw[cb * CB + tid], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         float sy = y * y;
-        sy += __shfl_xor(sy, 16); sy += __shfl_xor(sy, 8); sy += __shfl_xor(sy, 4); sy += __shfl_xor(sy, 2); sy += __shfl_xor(sy, 1);
+        sy = group_sum(sy, 32);
         if (tid == 0) __hip_atomic_store(&yraw[V + cb], sy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // every storing wave drains its write-through stores

@@ -171,8 +171,7 @@ struct Query {
             }, window);
             else each([&](int dist) { return r1 * (float)dist; }, window);
         }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = rows_max(mt);
         const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.f : mn;    // nothing seen so far: every weight is exp(-inf) = 0
         if (__any(mn > m)) {
             const float corr = ex(m - ms);
@@ -376,8 +375,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void lay_attn_tile_kerne
         if (i + 1 < steps) step(i + 1, rb, ra);
     }
     float l = q.l, c0 = 1.f;
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = rows_sum(l);
     if (KS == 2) {                                     // group 1 leaves its sums, group 0 takes them in
         float* po = (float*)smem;                      // [4 waves][NNT][64 lanes][4], then [4 waves][64 lanes] maxima and sums
         float* pm = po + 4 * NNT * 64 * 4;
@@ -586,7 +584,7 @@ __global__ __launch_bounds__(PACK && !HALF ? 256 : 512, PACK && !HALF ? 2 : 1) v
             if (lane < hd) v = lay_turn(v, cs, sn);
             float ss = fmaf(v.x, v.x, 0.f);
             ss = fmaf(v.y, v.y, ss);
-            for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+            ss = group_sum(ss, 64);
             const float rs = 1.f / sqrtf(ss / (float)d + a.prep.eps);
             v.x *= rs; v.y *= rs;
             return v;
@@ -672,8 +670,7 @@ __global__ __launch_bounds__(PACK && !HALF ? 256 : 512, PACK && !HALF ? 2 : 1) v
         values<VLD>(Vw, lr, lg, p, o);
     }
     float l = q.l;
-    l += __shfl_xor(l, 16);
-    l += __shfl_xor(l, 32);
+    l = rows_sum(l);
     if (lg == 0) { pm[wave][lr] = q.m; pl_[wave][lr] = l; }
     __syncthreads();                                   // every wave's value tile has been read: its place holds the sums
     float* po = (float*)smem;                          // [wave][NNT][64 lanes][4]

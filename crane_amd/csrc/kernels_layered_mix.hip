@@ -167,21 +167,18 @@ __device__ __forceinline__ float wave_sum16(float (&v)[16], int lane) {
         v[i] = keep + dpp_mov<CTRL>(send); \
     }
     CM_HALVE(8, 0x128, 8)      // row_ror 8: lane ^ 8
-    float s4[4];               // lane ^ 4 is no row operation: through the lanes
+    float s4[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float keep = (lane & 4) ? v[i + 4] : v[i], send = (lane & 4) ? v[i] : v[i + 4];
-        s4[i] = keep + __shfl_xor(send, 4);
+        s4[i] = keep + lane_xor<4>(send);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = s4[i];
     CM_HALVE(2, 0x4E, 2)       // quad_perm [2, 3, 0, 1]
     CM_HALVE(1, 0xB1, 1)       // quad_perm [1, 0, 3, 2]
 #undef CM_HALVE
-    float r = v[0];
-    r += __shfl_xor(r, 16);
-    r += __shfl_xor(r, 32);
-    return r;
+    return rows_sum(v[0]);
 }
 __device__ __forceinline__ void late_tail(const LNormRouter& a, int i) {
     const int per = (a.tail.C + (int)blockDim.x - 1) / (int)blockDim.x, sn = i / per, c = (i - sn * per) * (int)blockDim.x + (int)threadIdx.x;
@@ -555,7 +552,7 @@ __global__ __launch_bounds__(256) void lay_conv_qkv_kernel(LConvQkvArgs a, int n
         }
         float rs = 1.f;
         if (a.unit) {
-            for (int o = L >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+            ss = group_sum(ss, L);
             rs = 1.f / sqrtf(ss / (float)a.d + a.eps);
         }
         const size_t krow = isq ? 0 : (((size_t)a.bt[sg.bt_off + pos / a.page] * a.G + (hv - a.H)) * a.page + (size_t)(pos % a.page)) * a.d;

@@ -34,16 +34,6 @@ __global__ void embed_rows_kernel(const uint16_t* __restrict__ emb, const uint32
     }
 }
 
-__device__ __forceinline__ void split_store4(uint16_t* hi, uint16_t* lo, size_t off, const float v[4]) {
-    uint16_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        h[i] = f32_to_bf16(v[i]);
-        l[i] = f32_to_bf16(v[i] - bf16_to_f32(h[i]));
-    }
-    *(u32x2*)(hi + off) = (u32x2){(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)};
-    if (lo) *(u32x2*)(lo + off) = (u32x2){(uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16)};
-}
 
 // one block per token row: out = x * w / sqrt(mean(x^2)+eps) -> bf16 hi (+ lo)
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -202,7 +192,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv4_kernel(QkRopeArgs a_in) {
         const float* nw = is_q ? a.qnw : a.knw;
         if (nw) {
             float ss = xv[0] * xv[0] + xv[1] * xv[1] + xv[2] * xv[2] + xv[3] * xv[3];
-            ss += __shfl_xor(ss, 1); ss += __shfl_xor(ss, 2); ss += __shfl_xor(ss, 4); ss += __shfl_xor(ss, 8); ss += __shfl_xor(ss, 16);
+            ss += lane_xor<1>(ss); ss += lane_xor<2>(ss); ss += lane_xor<4>(ss); ss += lane_xor<8>(ss); ss += lane_xor<16>(ss);
             const float r = 1.0f / sqrtf(ss / (float)D + a.eps);
             const f32x4 w4 = *(const f32x4*)(nw + d0);
 #pragma unroll
@@ -212,7 +202,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv4_kernel(QkRopeArgs a_in) {
         const f32x4 c4 = *(const f32x4*)(a.cos + (size_t)rp * 64 + i0), s4 = *(const f32x4*)(a.sin + (size_t)rp * 64 + i0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float other = __shfl_xor(xv[e], 16);         // d < 64: x[d + 64], else x[d - 64]
+            const float other = lane_xor<16>(xv[e]);           // d < 64: x[d + 64], else x[d - 64]
             const float lo = d0 < 64 ? xv[e] : other, hi = d0 < 64 ? other : xv[e];
             xv[e] = d0 < 64 ? lo * c4[e] - hi * s4[e] : lo * s4[e] + hi * c4[e];
         }
@@ -612,8 +602,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
                 if (t > qpos) s[tt][r] = -INFINITY;
                 mt = fmaxf(mt, s[tt][r]);
             }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = rows_max(mt);
         const float m_new = fmaxf(m_run, mt);               // finite: token 0 is visible to every query
         const float alpha = fast_exp(m_run - m_new);
         float psum = 0.f;
@@ -651,8 +640,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
         }
     }
     // ---- finalize: l over the 4 lane groups; O^T rows = dims nt*16 + g*4 + r, col = query `sub` ----
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
+    l_run = rows_sum(l_run);
     const float inv = 1.0f / l_run;
     if (qrow < a.S) {
 #pragma unroll
@@ -694,25 +682,6 @@ __device__ __forceinline__ void lds_wg_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-}
-
-template <int KVT>
-__device__ __forceinline__ void p_split4(const float (&p)[4], bf16x4& hi, bf16x4& lo) {
-    if constexpr (KVT == KV_F16) {
-        typedef __attribute__((ext_vector_type(2))) _Float16 h2;
-        const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[0], p[1]));
-        const h2 b = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[2], p[3]));
-        const h2 c = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[0] - (float)a[0], p[1] - (float)a[1]));
-        const h2 d = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p[2] - (float)b[0], p[3] - (float)b[1]));
-        const u32x2 hv = {__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b)};
-        const u32x2 lv = {__builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, d)};
-        hi = __builtin_bit_cast(bf16x4, hv); lo = __builtin_bit_cast(bf16x4, lv);
-    } else {
-        const uint32_t a = pack_bf16x2(p[0], p[1]), b = pack_bf16x2(p[2], p[3]);
-        const uint32_t c = pack_bf16x2(p[0] - bf16_lo(a), p[1] - bf16_hi(a)), d = pack_bf16x2(p[2] - bf16_lo(b), p[3] - bf16_hi(b));
-        const u32x2 hv = {a, b}, lv = {c, d};
-        hi = __builtin_bit_cast(bf16x4, hv); lo = __builtin_bit_cast(bf16x4, lv);
-    }
 }
 
 // D = 128: 64-token key tiles; D = 256 (the hybrid family's gated attention): 32-token tiles, so that both double-buffered tiles of two
@@ -839,8 +808,7 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
                 if (MASKED) { if (t0 + tt * 16 + g * 4 + r > qpos) s[tt][r] = -INFINITY; }
                 mt = fmaxf(mt, s[tt][r]);
             }
-        mt = fmaxf(mt, __shfl_xor(mt, 16));
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        mt = rows_max(mt);
         const float m_new = fmaxf(m_run, mt);               // finite: token 0 is visible to every query (the first share; in others nothing may be so far)
         const float m_use = MASKED && m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * L2E);
@@ -892,8 +860,7 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
         if (t + 1 < tend) { if (t + 1 < nfull) tile(t + 1, std::false_type{}, rB, rA); else tile(t + 1, std::true_type{}, rB, rA); }
     }
     // ---- finalize: l over the 4 lane groups; O^T rows = dims nt*16 + g*4 + r, col = query `sub` ----
-    l_run += __shfl_xor(l_run, 16);
-    l_run += __shfl_xor(l_run, 32);
+    l_run = rows_sum(l_run);
     if (a.nsplit > 1) {                                     // attn_prefill_merge_kernel takes it from here
         if (qrow >= a.S) return;
         const size_t at = ((size_t)blockIdx.z * a.S + qrow) * a.Hq + h;

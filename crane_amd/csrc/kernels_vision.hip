@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256) void vit_rope_kv4_kernel(const float* __restri
         const f32x4 c4 = *(const f32x4*)(cs + (size_t)n * HD + d0), s4 = *(const f32x4*)(sn + (size_t)n * HD + d0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float partner = __shfl_xor(x[e], 8);                   // rotate_half: d < 32 -> -x[d+32], else x[d-32]
+            const float partner = lane_xor<8>(x[e]);                     // rotate_half: d < 32 -> -x[d+32], else x[d-32]
             const float rh = d0 < 32 ? -partner : partner;
             o[e] = x[e] * c4[e] + rh * s4[e];
         }

@@ -125,8 +125,7 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
                     if (MASKED) { if (lo + t * KT + tt * 16 + g * 4 + r >= end) s[n][tt][r] = -INFINITY; }
                     mt = fmaxf(mt, s[n][tt][r]);
                 }
-            mt = fmaxf(mt, __shfl_xor(mt, 16));
-            mt = fmaxf(mt, __shfl_xor(mt, 32));
+            mt = rows_max(mt);
             const float m_new = fmaxf(m_run[n], mt);                   // finite: every tile holds a patch of the frame
             const float alpha = __builtin_amdgcn_exp2f((m_run[n] - m_new) * L2E), nm = -m_new * L2E;
             float psum = 0.f;
@@ -179,8 +178,7 @@ __global__ __launch_bounds__(256, 2) void vit_attn_kernel(VitAttnArgs a) {
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
         float l = l_run[n];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
+        l = rows_sum(l);
         const int row = tl.z + (wave * NQ + n) * 16 + sub;
         if (row >= end) continue;
         if (a.runs > 1) {                                              // un-normalised; an empty run: maximum -inf, sum 0
