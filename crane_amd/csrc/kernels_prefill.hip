@@ -1454,6 +1454,8 @@ template <int D, int KT>
 static void launch_prefill_fast(AttnPreArgs a, int kvt, hipStream_t s) {
     a.nsplit = prefill_split(a, D);
     const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64, a.nsplit);
+    // more than two workgroups on every CU: half as many with twice the waves (figures beside that kernel)
+    if (D == 128 && a.nrep % 2 == 0 && a.nsplit == 1 && grid.x * grid.y > 512) { launch_attn_prompt_pair(a, kvt, s); return; }
     if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_F16>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_BF16>), grid, dim3(256), 0, s, a);
     if (a.nsplit > 1) hipLaunchKernelGGL(attn_prefill_merge_kernel<D>, dim3((unsigned)(((size_t)a.S * a.Hq + 1024 / D - 1) / (1024 / D))), dim3(256), 0, s, a);

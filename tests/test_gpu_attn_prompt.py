@@ -1,0 +1,56 @@
+"""GPU: prompt attention of many query tiles (kernels_attn_prompt.hip) against the same prompt in portions, whose launches are small enough for attn_prefill_fast_kernel, and several
+prompts in one pass against each by itself.
+
+One layer: the cached rows and the weights are the same, and so is the order of every sum of the attention; the products around it add up in other tiles (1e-7 of a row), attention rows
+travel as bfloat16 hi + lo planes, 2^-17 of an element where the two land on both sides of a boundary: 2e-5 of the largest logit, as in tests/test_gpu_prefill_shares.py."""
+import numpy as np
+import pytest
+
+from crane_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-5
+
+
+def _model(heads, kv, chunk, page=64, dtype="f16", seqs=2):
+    from crane_amd.backend import Model
+    cfg = dict(configs.get_config("qwen3-0.6b"), vocab_size=512, num_hidden_layers=1, hidden_size=512, intermediate_size=1024, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128)
+    return Model.synthetic(cfg, seed=3, max_seq_len=2304, max_seqs=seqs, prefill_chunk=chunk, kv_block_size=page, kv_dtype=dtype)
+
+
+def _last(m, ids):
+    s = m.seq_alloc()
+    row = np.asarray(m.seq_forward(s, ids, 0)[0], np.float64).ravel()
+    m.seq_free(s)
+    return row
+
+
+# a query tile of one row behind whole ones, whole tiles only, a ragged one; two, four and eight query heads per key head; pages of one tile and of two; both page types; a second pass behind 2048 rows
+@pytest.mark.parametrize("heads,kv,page,dtype,tokens", [(32, 8, 64, "f16", (1025, 1088, 2048, 2300)), (32, 16, 128, "bf16", (1087, 1500)), (32, 4, 128, "f16", (1100,)), (40, 20, 64, "bf16", (833, 900))])
+def test_against_portions(heads, kv, page, dtype, tokens):
+    ids = np.random.default_rng(heads + kv).integers(0, 512, 2300).tolist()
+    rows = []
+    for chunk in (2048, 512 if heads == 32 else 384):
+        m = _model(heads, kv, chunk, page, dtype)
+        try:
+            rows.append([_last(m, ids[:n]) for n in tokens])
+        finally:
+            m.close()
+    for a, b in zip(*rows):
+        assert np.isfinite(a).all() and np.abs(a - b).max() < TOL * np.abs(b).max()
+
+
+# several sequences in one launch: tiles of every length, sequences of one row and of a tile and one
+def test_several_prompts():
+    rng = np.random.default_rng(1)
+    prompts = [rng.integers(0, 512, n).tolist() for n in (1, 65, 700, 64, 310, 900)]
+    m = _model(32, 8, 2048, seqs=8)
+    try:
+        alone = [_last(m, p) for p in prompts]
+        seqs = [m.seq_alloc() for _ in prompts]
+        together = np.asarray(m.prefill_batch(seqs, prompts)[0], np.float64)
+    finally:
+        m.close()
+    for a, b in zip(together, alone):
+        assert np.isfinite(a).all() and np.abs(a.ravel() - b).max() < TOL * np.abs(b).max()
