@@ -237,9 +237,17 @@ __global__ __launch_bounds__(256, 2) void lay_tile_gemm_kernel(LTileArgs first, 
 // of 16 cycles each per slot of 1024 (both for t + 1 in the first slot, which they filled: 8192 rows, 16 experts of 2048 x 4096 and one of every token, gate-and-up / down 350 / 212 us, here 337 / 202).  A band of 16 rows
 // behind a ragged tile's end multiplies nothing.  8192 rows, 4096 columns, K 4096: 359 us on 128 x 128 tiles, 228 - 305 here by what the clock allows (183 with
 // operands of zeros: 1.5 PFLOP/s)
-template <bool DUAL>
+//
+// 128 x 256 and 128 x 384 are two tiles of 128 x 128 or 128 x 192 side by side, of one matrix: the same schedule over half the rows, which the two tiles read once.  A block of 128 x 128 asks for
+// 32 KB per k-tile of 512 MFMA cycles, which is all that the address path takes in that time; two together 48 KB per 1024.  384 columns leave LDS for two stages of weights and three of rows:
+// there the weights are the near operand.  Bound by the LDS: 16 fragments per 32 products of a wave and the 48 KB that come in are 1400 cycles of its port per 1024 of the matrix cores.  2048 rows, K 4096,
+// single tiles / in pairs: 4096 columns 79 / 69 us, 6144 109 / 100; a prompt of four layers 3.70 -> 3.64 ms, 1200 tokens 2.88 -> 2.84, 650 2.25 -> 2.22; width 1024 equal.
+template <bool DUAL, int BM, int BN>
 __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTileArgs second, int ntiles, int ntiles_b) {
-    constexpr int BM = 256, BN = 256, WM = 128, WN = 64, NI = 8, NJ = 4, NL = 4, NC = DUAL ? WN / 2 : WN, STAGE = 256 * BK, WBASE = 2 * STAGE;
+    constexpr int WM = BM / 2, WN = BN / 4, NI = WM / 16, NJ = WN / 16, NA = BM / 64, NW = BN / 64, NC = DUAL ? WN / 2 : WN;
+    constexpr bool WFAR = BN == 256;                                      // the operand with three stages, asked for two tiles ahead: weights, or rows
+    constexpr int AST = WFAR ? 2 : 3, WST = WFAR ? 3 : 2, ASTAGE = BM * BK, WSTAGE = BN * BK, WBASE = AST * ASTAGE, NEAR = WFAR ? NA : NW, FAR = WFAR ? NW : NA;
+    static_assert(!DUAL || BN == 256, "a wave's pieces are all of W or all of W2");
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -259,18 +267,21 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
     const char* const A0 = (const char*)a.A;
     const char* const W0 = (const char*)((DUAL && (wave & 4) ? a.W2 : a.W) + (size_t)at.g * a.w_stride + (size_t)n0 * a.K);
-    uint32_t aoff[NL], woff[NL];
+    uint32_t aoff[NA], woff[NW];
+    const uint32_t kc = (uint32_t)(slot ^ ((r0 >> 1) & 7)) << 4;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
+    for (int i = 0; i < NA; ++i) {
         const int r = p0 + min(i * 64 + r0, rows - 1);
-        const uint32_t kc = (uint32_t)(slot ^ ((r0 >> 1) & 7)) << 4;
         aoff[i] = (uint32_t)(a.a_idx ? a.a_idx[r] / a.a_div : r) * (uint32_t)(a.lda * 2) + kc;
-        woff[i] = (uint32_t)min(i * NC + (DUAL ? r0 & 31 : r0), a.N - 1 - n0) * (uint32_t)(a.K * 2) + kc;
     }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) woff[i] = (uint32_t)min(DUAL ? i * NC + (r0 & 31) : i * 64 + r0, a.N - 1 - n0) * (uint32_t)(a.K * 2) + kc;
     const int nk = a.K / BK;
     // (past the end: the last tile again, into a stage nobody reads)
-    auto ask_a = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(A0 + (size_t)min(t, nk - 1) * (BK * 2), aoff[i], lds0 + (uint32_t)((t & 1) * STAGE + (wave + 8 * i) * 8 * BK) * 2u); };
-    auto ask_w = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(W0 + (size_t)min(t, nk - 1) * (BK * 2), woff[i], lds0 + (uint32_t)(WBASE + t % 3 * STAGE + (wave + 8 * i) * 8 * BK) * 2u); };
+    auto ask_a = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(A0 + (size_t)min(t, nk - 1) * (BK * 2), aoff[i], lds0 + (uint32_t)(t % AST * ASTAGE + (wave + 8 * i) * 8 * BK) * 2u); };
+    auto ask_w = [&](int i, int t) __attribute__((always_inline)) { lds_load16_at(W0 + (size_t)min(t, nk - 1) * (BK * 2), woff[i], lds0 + (uint32_t)(WBASE + t % WST * WSTAGE + (wave + 8 * i) * 8 * BK) * 2u); };
+    auto ask_near = [&](int i, int t) __attribute__((always_inline)) { if (i < NEAR) { if (WFAR) ask_a(i, t); else ask_w(i, t); } };
+    auto ask_far = [&](int i, int t) __attribute__((always_inline)) { if (i < FAR) { if (WFAR) ask_w(i, t); else ask_a(i, t); } };
     f32x4 acc[NI][NJ];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -280,8 +291,8 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
     const int bands = min(NI, (rows - wm * WM + 15) >> 4);                // bands of this wave that have rows (none: 0 or less)
     bf16x8 af[2][NI], bf[2][NJ];
     auto fetch = [&](int t) __attribute__((always_inline)) {
-        const uint16_t* As = lds + (t & 1) * STAGE + wm * WM * BK;
-        const uint16_t* Bs = lds + WBASE + t % 3 * STAGE + wn * WN * BK;
+        const uint16_t* As = lds + t % AST * ASTAGE + wm * WM * BK;
+        const uint16_t* Bs = lds + WBASE + t % WST * WSTAGE + wn * WN * BK;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int fk = ((s * 4 + lg) ^ sw) << 3;
@@ -296,6 +307,7 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
         for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[s][j], af[s][i], acc[i][j], 0, 0, 0);
     };
     // a slot's products with its requests between the bands
+    constexpr int PER = (std::max(NEAR, FAR) + NI - 1) / NI;
     auto multiply = [&](auto ask) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
@@ -303,38 +315,39 @@ __global__ __launch_bounds__(512) void lay_tall_gemm_kernel(LTileArgs first, LTi
         for (int i = 0; i < NI; ++i) {
             if (i < bands) { band(0, i); band(1, i); }
             __builtin_amdgcn_sched_barrier(0);
-            if (i < NL) ask(i);
+#pragma unroll
+            for (int k = 0; k < PER; ++k) ask(i * PER + k);
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // every wave runs 2 nk + 2 barriers.  What is asked for in the second slot of a tile, the newest NL requests, may stay in flight at its end
+    // every wave runs 2 nk + 2 barriers.  What is asked for in the second slot of a tile, the newest FAR requests, may stay in flight at its end
 #pragma unroll
-    for (int i = 0; i < NL; ++i) { ask_a(i, 0); ask_w(i, 0); }
+    for (int i = 0; i < std::max(NEAR, FAR); ++i) { ask_near(i, 0); ask_far(i, 0); }
 #pragma unroll
-    for (int i = 0; i < NL; ++i) ask_w(i, 1);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NL) : "memory");
+    for (int i = 0; i < FAR; ++i) ask_far(i, 1);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(FAR) : "memory");
     if (wm == 0) {
         for (int t = 0; t < nk; ++t) {
 #pragma unroll
-            for (int i = 0; i < NL; ++i) ask_a(i, t + 1);
+            for (int i = 0; i < NEAR; ++i) ask_near(i, t + 1);
             fetch(t);
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            multiply([&](int i) __attribute__((always_inline)) { ask_w(i, t + 2); });
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NL) : "memory");
+            multiply([&](int i) __attribute__((always_inline)) { ask_far(i, t + 2); });
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(FAR) : "memory");
         }
         asm volatile("s_barrier" ::: "memory");
     } else {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) ask_a(i, 1);                         // in the slot in which row 0 fetches tile 0
+        for (int i = 0; i < NEAR; ++i) ask_near(i, 1);                    // in the slot in which row 0 fetches tile 0
         asm volatile("s_barrier" ::: "memory");
         for (int t = 0; t < nk; ++t) {
 #pragma unroll
-            for (int i = 0; i < NL; ++i) ask_w(i, t + 2);
+            for (int i = 0; i < FAR; ++i) ask_far(i, t + 2);
             fetch(t);
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NL) : "memory");
-            multiply([&](int i) __attribute__((always_inline)) { ask_a(i, t + 2); });
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(FAR) : "memory");
+            multiply([&](int i) __attribute__((always_inline)) { ask_near(i, t + 2); });
             asm volatile("s_barrier" ::: "memory");
         }
     }
@@ -359,14 +372,14 @@ void go(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
     const int share = (mtiles<BM>(a) * nt + 7) / 8 + ((b.M + BM - 1) / BM * ntb + 7) / 8;
     hipLaunchKernelGGL((lay_tile_gemm_kernel<BM, BN, ST, DUAL, FN>), dim3((unsigned)share * 8), dim3(256), lds, s, a, b, nt, ntb);
 }
-template <bool DUAL>
+template <bool DUAL, int BM = 256, int BN = 256>
 void go_tall(const LTileArgs& a, const LTileArgs& b, hipStream_t s) {
-    constexpr size_t lds = (size_t)5 * 256 * BK * sizeof(uint16_t);
+    constexpr size_t lds = (size_t)(BN == 256 ? 2 * BM + 3 * BN : 3 * BM + 2 * BN) * BK * sizeof(uint16_t);
     static DevOnce attr;
-    attr.run([&] { (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tall_gemm_kernel<DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
-    const int cols = DUAL ? 128 : 256, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
-    const int share = (mtiles<256>(a) * nt + 7) / 8 + ((b.M + 255) / 256 * ntb + 7) / 8;
-    hipLaunchKernelGGL((lay_tall_gemm_kernel<DUAL>), dim3((unsigned)share * 8), dim3(512), lds, s, a, b, nt, ntb);
+    attr.run([&] { (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&lay_tall_gemm_kernel<DUAL, BM, BN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); });
+    const int cols = DUAL ? BN / 2 : BN, nt = (a.N + cols - 1) / cols, ntb = (b.N + cols - 1) / cols;
+    const int share = (mtiles<BM>(a) * nt + 7) / 8 + ((b.M + BM - 1) / BM * ntb + 7) / 8;
+    hipLaunchKernelGGL((lay_tall_gemm_kernel<DUAL, BM, BN>), dim3((unsigned)share * 8), dim3(512), lds, s, a, b, nt, ntb);
 }
 
 // The last columns of one matrix, [n0, N), at most 64 of them: 16 rows per block, the k-tiles dealt to its eight waves, operands from memory straight into fragments.
@@ -427,6 +440,8 @@ float row_tiles(const LTileArgs& a, int bm) {
     for (int k = 1; k * bm < a.M; ++k) t += std::min(1.f, std::max(0.f, 0.5f + (avg - (float)(k * bm)) / (3.f * sd)));
     return t * a.groups;
 }
+// every row of A within lay_tall_gemm_kernel's 32-bit offsets
+bool lay_near(const LTileArgs& x) { return (uint64_t)std::max(x.total, x.M) * x.lda * 2 + (uint64_t)x.K * 2 < 1ull << 32; }
 bool plain_out(const LTileArgs& a) { return !a.bias && (a.act == LACT_NONE || a.act_split <= 0) && (a.act2 == LACT_NONE || a.act_split >= a.N); }
 
 }  // namespace
@@ -463,9 +478,8 @@ static LayTileShape lay_tile_least(const LTileArgs& a, const LTileArgs& b, float
     LayTileShape best = wide ? LTILE_128 : LTILE_64;
     least = wide ? 4.f * std::ceil(blocks(128, 128) / 512.f) : 2.6f * (blocks(64, 64) / 768.f + 0.5f);
     if (!a.W2 && !(plain_out(a) && (b.M <= 0 || plain_out(b)))) return best;      // (the large tiles' stores know no bias and no function)
-    auto near = [](const LTileArgs& x) { return (uint64_t)std::max(x.total, x.M) * x.lda * 2 + (uint64_t)x.K * 2 < 1ull << 32; };      // (lay_tall_gemm_kernel's offsets)
     for (const auto& c : all) {
-        if (c.shape == LTILE_256 && !(near(a) && near(b))) continue;
+        if (c.shape == LTILE_256 && !(lay_near(a) && lay_near(b))) continue;
         const float t = c.round * std::ceil(blocks(c.bm, c.bn) / (float)c.slots);
         if (t < least) { least = t; best = c.shape; }
     }
@@ -496,9 +510,16 @@ void launch_lay_tile_gemm(const LTileArgs& a0, hipStream_t s, const LTileArgs* b
         go_few_cols(a, a.N - rest, s);
         a.N -= rest;
     }
+    // (one matrix: the tiles of a shape in pairs, rows by rows, where their number is even)
+    auto pairs = [&](int bn) { return !a.grp_off && !a.W2 && b.M <= 0 && plain_out(a) && lay_near(a) && a.N % (2 * bn) == 0; };
     auto launch = [&](auto dual) {
         constexpr bool DUAL = decltype(dual)::value;
-        switch (lay_tile_shape(a, b)) {
+        const LayTileShape shape = lay_tile_shape(a, b);
+        if constexpr (!DUAL) {
+            if (shape == LTILE_128 && pairs(128)) return go_tall<false, 128, 256>(a, b, s);
+            if (shape == LTILE_128_192 && pairs(192)) return go_tall<false, 128, 384>(a, b, s);
+        }
+        switch (shape) {
             case LTILE_64: go<64, 64, 3, DUAL>(a, b, s); break;
             case LTILE_128: go<128, 128, 2, DUAL>(a, b, s); break;
             case LTILE_192_128: go<192, 128, 2, DUAL, DUAL>(a, b, s); break;

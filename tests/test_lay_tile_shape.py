@@ -43,3 +43,11 @@ def test_last_columns(tmp_path, n, width, heads, kv_heads, tail):
     cols = (heads + 2 * kv_heads) * 64 + heads
     assert (_lib.load().cm_debug_lay_tile_shape(n, cols, width, 0, 0, 0, 0, 0) < 0) == tail
     _check(tmp_path, GZ, GZ.config([GZ.layer(mixer, None)], vocab=96, width=width), n, 5)
+
+
+# one matrix on tiles in pairs (an even number of 128- or 192-wide ones): a projection of 5 k-tiles, ragged rows, a last row tile of 4 rows and none
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,width,shape", [(1300, 3072, 128128), (1028, 4096, 128128), (2000, 6144, 128192), (2048, 6144, 128192)])
+def test_tiles_in_pairs(tmp_path, n, width, shape):
+    assert _lib.load().cm_debug_lay_tile_shape(n, width, 320, 0, 0, 0, 0, 0) == shape
+    _check(tmp_path, GZ, GZ.config([GZ.layer(GZ.attn(heads=5, kv_heads=5, dim=64, vdim=64), None)], vocab=96, width=width), n, 7)
