@@ -155,8 +155,8 @@ struct GemmArgs {
     uint16_t* norm_hi = nullptr;
     uint16_t* norm_lo = nullptr;
     float norm_eps = 0.f;
-    // GEPI_STORE of 9 .. 128 rows with a consumer that adds the slices of K itself (attn_decode_group_kernel): no reduction is launched where K is split, *defer_ks
-    // slices of M x N stay in ws; 1: C holds the rows as usual
+    // GEPI_STORE without a bias, of 9 .. 128 rows or of a prompt, with a consumer that adds the slices of K itself (attn_decode_group_kernel, qknorm_rope_kv4_kernel): no reduction is
+    // launched where K is split, *defer_ks slices of M x N stay in ws; 1: C holds the rows as usual
     int* defer_ks = nullptr;
 };
 
@@ -200,6 +200,9 @@ struct QkRopeArgs {
     // several sequences in one launch: row s of the pass belongs to segs[rowseg[s]] (null: one sequence, start_pos / block_table above)
     const PrefillSegDev* segs = nullptr;
     const int32_t* rowseg = nullptr;
+    // the projection's K slices, `part` floats apart from qkv on, to be added in their order (qknorm_rope_adds_slices; GemmArgs::defer_ks)
+    int parts = 1;
+    size_t part = 0;
 };
 
 struct AttnPreArgs {
@@ -230,6 +233,7 @@ void launch_embed_rows(const uint16_t* emb, const uint32_t* ids, float* x, int S
 void launch_rmsnorm_rows(const float* x, const float* w, uint16_t* hi, uint16_t* lo, int S, int H, float eps,
                          hipStream_t s);
 void launch_qknorm_rope_kv(const QkRopeArgs& a, int D, int S, int kv_mode, hipStream_t s);
+bool qknorm_rope_adds_slices(const QkRopeArgs& a, int D, int kv_mode);    // whether that launch's kernel takes a.parts > 1
 void launch_kvq_dequant_prefix(const void* kpool, const void* vpool, const int32_t* block_table, float* kshadow, float* vshadow,
                                int tokens, int Hkv, int page, int D, int kv_mode, size_t page_bytes, hipStream_t s);
 void launch_split_rows(const float* x, uint16_t* hi, uint16_t* lo, size_t n, hipStream_t s);

@@ -188,6 +188,13 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv4_kernel(QkRopeArgs a_in) {
     const int kvh = is_k ? item - Hq : item - Hq - Hkv;
     const float* src = a.qkv + (size_t)s * a.row_stride + (is_q ? a.q_off + item * D : (is_k ? a.k_off + kvh * D : a.v_off + kvh * D));
     f32x4 xv = *(const f32x4*)(src + d0);
+    // a split projection's slices, as gemm_splitk_epilogue_kernel adds them (its launch in front of this one: 5.4 + 5.2 us for 117 rows of 6144 columns in four slices, 5.3 here alone;
+    // 117 tokens of the 8B model 5.98 -> 5.89 ms, of the 0.6B model 2.03 -> 1.95)
+    for (int k = 1; k < a.parts; ++k) {
+        const f32x4 p = *(const f32x4*)(src + (size_t)k * a.part + d0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xv[e] += p[e];
+    }
     if (is_q || is_k) {
         const float* nw = is_q ? a.qnw : a.knw;
         if (nw) {
@@ -930,10 +937,13 @@ void launch_rmsnorm_rows(const float* x, const float* w, uint16_t* hi, uint16_t*
                          hipStream_t s) {
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(S), dim3(256), 0, s, x, w, hi, lo, H, eps);
 }
-void launch_qknorm_rope_kv(const QkRopeArgs& a, int D, int S, int kv_mode, hipStream_t s) {
+bool qknorm_rope_adds_slices(const QkRopeArgs& a, int D, int kv_mode) {
     static const int v4 = getenv("CM_ROPE_KV4") ? atoi(getenv("CM_ROPE_KV4")) : 1;          // 0: always the one-wave-per-head kernel (A/B)
-    if (v4 && D == 128 && a.rot_dim == 128 && a.pos3 == nullptr && (kv_mode == 0 || kv_mode == 1 || kv_mode == KV_F16) &&
-        a.q_off % 4 == 0 && a.k_off % 4 == 0 && a.v_off % 4 == 0 && a.row_stride % 4 == 0) {
+    return v4 && D == 128 && a.rot_dim == 128 && a.pos3 == nullptr && (kv_mode == 0 || kv_mode == 1 || kv_mode == KV_F16) &&
+           a.q_off % 4 == 0 && a.k_off % 4 == 0 && a.v_off % 4 == 0 && a.row_stride % 4 == 0;
+}
+void launch_qknorm_rope_kv(const QkRopeArgs& a, int D, int S, int kv_mode, hipStream_t s) {
+    if (qknorm_rope_adds_slices(a, D, kv_mode)) {
         dim3 g4(S, (a.Hq + 2 * a.Hkv + 7) / 8);
         if (kv_mode == 1) hipLaunchKernelGGL((qknorm_rope_kv4_kernel<1>), g4, dim3(256), 0, s, a);
         else if (kv_mode == KV_F16) hipLaunchKernelGGL((qknorm_rope_kv4_kernel<KV_F16>), g4, dim3(256), 0, s, a);
@@ -1185,6 +1195,12 @@ static void launch_splitk(GemmArgs& a, int epi, hipStream_t s) {
     else launch_splitk_epilogue<GEPI_SILUMUL>(a, eb, s);
 }
 
+// ... or left to a consumer that adds the slices itself
+static void leave_slices(GemmArgs& a, int epi, hipStream_t s) {
+    if (a.defer_ks != nullptr && epi == GEPI_STORE && a.bias == nullptr) *a.defer_ks = a.ksplit;
+    else launch_splitk(a, epi, s);
+}
+
 // The LDS-DMA kernel on full cache lines (kernels_gemm256.hip; one tile of up to 128 rows with hi + lo activations, 256-row tiles with plain bf16 from 512 rows on)
 // where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
 // register-staged kernel should run.
@@ -1239,7 +1255,7 @@ static bool try_gemm256(GemmArgs& a, int epi, hipStream_t s) {
         if (!gemm_tile_plan(a.M, a.N, a.K, a.ws ? a.ws_floats : 0, a.norm_w != nullptr, &bm, &bn, &ks, nullptr)) return false;
         a.ksplit = ks;
         if (!launch_gemm_tile(a, epi, bm, bn, s)) return false;
-        if (ks > 1) launch_splitk(a, epi, s);
+        if (ks > 1) leave_slices(a, epi, s);
         return true;
     }
     if (!gemm256_plan(a.M, a.N, a.K, a.A_lo != nullptr, a.ws ? a.ws_floats : 0, w4, &bn, &ks)) return false;
@@ -1280,7 +1296,7 @@ bool launch_gemm(const GemmArgs& a0, int epi, hipStream_t s) {
         if (epi != GEPI_STORE && epi != GEPI_RESADD && epi != GEPI_SILUMUL) return false;
         if (epi == GEPI_SILUMUL && a.gu_tmp == nullptr) return false;
         GemmArgs p1 = a, p2 = a;
-        p1.W_lo = nullptr; p1.norm_w = nullptr;
+        p1.W_lo = nullptr; p1.norm_w = nullptr; p1.defer_ks = p2.defer_ks = nullptr;
         p2.W = a.W_lo; p2.W_lo = nullptr; p2.A_lo = nullptr; p2.norm_w = nullptr;
         if (epi == GEPI_SILUMUL) { p1.C = a.gu_tmp; p1.ldc = a.N; p2.C = a.gu_tmp; p2.ldc = a.N; }
         if (!launch_gemm_inner(p1, epi == GEPI_RESADD ? GEPI_RESADD : GEPI_STORE, s)) return false;
@@ -1304,8 +1320,7 @@ static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     if (!gemm_rows_plan(a.M, a.N, a.K, a.ws ? a.ws_floats : 0, &bn, &ks)) return false;
     a.ksplit = ks;
     if (!launch_gemm_rows(a, epi, bn, s)) return false;
-    if (ks > 1 && a.defer_ks != nullptr && epi == GEPI_STORE && a.bias == nullptr) *a.defer_ks = ks;
-    else if (ks > 1) launch_splitk(a, epi, s);
+    if (ks > 1) leave_slices(a, epi, s);
     return true;
 }
 static bool gemm_tail_columns(int M, int N) { return M >= 256 && N >= 512 && N % 192 != 0 && N % 256 == 128; }
@@ -1315,6 +1330,7 @@ static bool gemm_tail_columns(int M, int N) { return M >= 256 && N >= 512 && N %
 static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {
     if (epi != GEPI_STORE || a.norm_w != nullptr || !gemm_tail_columns(a.M, a.N)) return false;
     GemmArgs most = a, rest = a;
+    most.defer_ks = rest.defer_ks = nullptr;
     most.N = a.N - 128;
     if (!try_gemm256(most, epi, s)) return false;
     rest.W = a.W + (size_t)most.N * a.K; rest.C = a.C + most.N; rest.N = 128;
@@ -1360,7 +1376,7 @@ int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
 // width 2048, 650: 7.5 / 7.1.  The line is a gain of 5 % and 8 us by the figures above: with 5 % alone the products of width 1024 lost (300 tokens 3.32 / 3.45
 // ms, 560 4.30 / 4.41: a launch and a reduction more for a round of 30 us).  Rows of products with an activation behind them and the vision tower's norm stay in one launch (not measured).
 static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
-    if (a.A_lo == nullptr || a.defer_ks != nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
+    if (a.A_lo == nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
     const size_t ws = a.ws ? a.ws_floats : 0;
     const int m = gemm_band(a.M, a.N, a.K, epi, ws, a.ksplit_cap);
     if (m == 0) return false;
@@ -1372,6 +1388,7 @@ static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
     for (int part = 0; part < 2; ++part) {
         const size_t r0 = part ? (size_t)m : 0;
         GemmArgs b = a;
+        b.defer_ks = nullptr;                                      // (slices of either band's rows)
         b.M = part ? a.M - m : m;
         b.A_hi += r0 * a.K; b.A_lo += r0 * a.K;
         if (a.C) b.C += r0 * a.ldc;

@@ -1381,6 +1381,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
                 launch_add_rows(pX, pY, (size_t)S * H, s);
             }
         } else {
+        int qkv_parts = 1;
         if (q8p) {
             for (int i = 0; i < w.n_qkv; ++i) q8_mm(w.q_qkv[i], pX, H, w.ln1, EPI_STORE, pQKV + w.qkv_row0[i], qkv_rows, S, nullptr, false);
         } else {
@@ -1392,6 +1393,11 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             }));
         }
         g.M = S; g.N = qkv_rows; g.K = H;
+        // K slices are added by the rotation (dense decoders: nobody else reads the rows), where it is one launch over all of them
+        QkRopeArgs shape{};
+        shape.rot_dim = cfg.rot_dim; shape.pos3 = pos3_dev; shape.row_stride = qkv_rows; shape.k_off = Hq_l * D; shape.v_off = shape.k_off + Hkv_l * D;
+        const bool one_rope = nseg == 1 || (seg_batch && seg_tables_ok);
+        if (!cfg.hybrid && !quantized && !this->kvq() && one_rope && qknorm_rope_adds_slices(shape, D, kv_mode)) g.defer_ks = &qkv_parts;
         if (!launch_gemm(g, GEPI_STORE, s)) throw CmError(CM_ERR_UNSUPPORTED, "gemm shape");
         }
         // QK-norm + RoPE + KV append and the causal attention run once per sequence of the pass (its own pages and positions)
@@ -1409,6 +1415,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             q.sec_h = cfg.mrope_sec[1]; q.sec_w = cfg.mrope_sec[2];
             q.scale = (float)(1.0 / std::sqrt((double)D));
             q.segs = d_segtab; q.rowseg = d_rowseg;
+            if (qkv_parts > 1) { q.qkv = pWS; q.parts = qkv_parts; q.part = (size_t)S * qkv_rows; }
             launch_qknorm_rope_kv(q, D, S, kv_mode, s);
             AttnPreArgs at{};
             at.q_hi = pQ_hi; at.q_lo = pQ_lo; at.block_table = d_btb;
@@ -1440,6 +1447,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             q.page_bytes = page_bytes; q.kshadow = kshadow; q.vshadow = vshadow;
             launch_kvq_dequant_prefix(kpool(li), vpool(li), sg.bt, kshadow, vshadow, sp, Hkv_l, page, D, kv_mode, page_bytes, s);
         }
+        if (qkv_parts > 1) { q.qkv = pWS; q.parts = qkv_parts; q.part = (size_t)S * qkv_rows; }      // (one sequence: sg.row0 is 0)
         launch_qknorm_rope_kv(q, D, sg.S, kv_mode, s);
         AttnPreArgs at{};
         at.q_hi = q.q_hi; at.q_lo = q.q_lo; at.block_table = kvq ? d_ident_bt : sg.bt;

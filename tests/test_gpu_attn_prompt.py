@@ -41,10 +41,11 @@ def test_against_portions(heads, kv, page, dtype, tokens):
         assert np.isfinite(a).all() and np.abs(a - b).max() < TOL * np.abs(b).max()
 
 
-# several sequences in one launch: tiles of every length, sequences of one row and of a tile and one
-def test_several_prompts():
+# several sequences in one launch: tiles of every length, sequences of one row and of a tile and one; few rows, whose projection is split and added up by the rotation
+@pytest.mark.parametrize("lengths", [(1, 65, 700, 64, 310, 900), (3, 40, 17, 60), (9, 1), (150, 120, 30)])
+def test_several_prompts(lengths):
     rng = np.random.default_rng(1)
-    prompts = [rng.integers(0, 512, n).tolist() for n in (1, 65, 700, 64, 310, 900)]
+    prompts = [rng.integers(0, 512, n).tolist() for n in lengths]
     m = _model(32, 8, 2048, seqs=8)
     try:
         alone = [_last(m, p) for p in prompts]
