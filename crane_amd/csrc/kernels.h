@@ -246,6 +246,7 @@ int gemmw4_rows(bool split);               // rows of the one-wave-per-SIMD kern
 bool launch_gemmw4(const GemmArgs& a, int epi, int bn, hipStream_t s);    // same contract as launch_gemm256
 int attn_prefill_shares(int rows, int start, int heads, int D);      // blocks that share the keys of a query tile, scratch permitting
 void launch_attn_prompt_pair(const AttnPreArgs& a, int kvt, hipStream_t s);      // kernels_attn_prompt.hip: head_dim 128, an even number of query heads per key head, keys not shared
+void launch_attn_prompt_wide(const AttnPreArgs& a, int kvt, hipStream_t s);      // head_dim 256; a.nsplit shares of the keys
 void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s);   // kvt: KV_BF16 | KV_F16 | KV_F32 (what the kernel reads)
 
 // ---- vision tower (kernels_vision.hip, kernels_vision_attn.hip) ----

@@ -680,8 +680,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnPreArgs a_in) {
 //   * the products of a tile are all 32 keys deep (126 -> 109 us for 2048 tokens of 32 heads, 78 -> 66 for 452 behind them, when the second product
 //     took 16 at a time).
 // A launch of few query tiles behind many keys leaves the chip idle and walks the keys one after the other: there several blocks share a query tile's keys and
-// attn_prefill_merge_kernel adds the shares (69 queries behind 4096 keys, 8 heads of 256: 232 us for 16 blocks -> 30 for 256 and 9; 452 behind 2048, 32
-// heads of 128: 66 -> 55 and 7).
+// attn_prefill_merge_kernel adds the shares (452 queries behind 2048 keys, 32 heads: 66 -> 55 us and 7).
 // ---------------------------------------------------------------------------------------------
 // workgroup barrier for LDS hand-offs only: waits for this wave's LDS operations, not for its outstanding global loads
 // (__syncthreads() drains vmcnt as well and would retire the two-tiles-ahead requests at every tile)
@@ -691,11 +690,10 @@ __device__ __forceinline__ void lds_wg_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// D = 128: 64-token key tiles; D = 256 (the hybrid family's gated attention): 32-token tiles, so that both double-buffered tiles of two
-// workgroups still fit a CU's LDS (69 KB per workgroup either way)
-template <int D, int KT, int KVT>
+// (69 KB of LDS per workgroup: two on a CU)
+template <int KVT>
 __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in) {
-    constexpr int VLD = D + 16, NKS = D / 32, NNT = D / 16, NTT = KT / 16, CPR = D / 8, RPP = 256 / CPR;      // chunks per row, rows per staging pass
+    constexpr int D = 128, KT = 64, VLD = D + 16, NKS = D / 32, NNT = D / 16, NTT = KT / 16, CPR = D / 8, RPP = 256 / CPR;      // chunks per row, rows per staging pass
     static_assert(KT * CPR == 4 * 256, "four 16-byte chunks per thread and tile");
     constexpr float L2E = 1.4426950408889634f;
     AttnPreArgs a = a_in;
@@ -709,7 +707,6 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
         if (a.q_lo != nullptr) a.q_lo += r0;
         if (a.out_lo != nullptr) a.out_lo += r0;
         if (a.out_f32 != nullptr) a.out_f32 += r0;
-        if (a.gate != nullptr) a.gate += (size_t)sg.row0 * a.gate_stride;
         qt_seg = tq.y;
     }
     __shared__ __attribute__((aligned(16))) uint16_t Vs[2][KT * VLD];
@@ -881,12 +878,7 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
     if (qrow < a.S) {
 #pragma unroll
         for (int nt = 0; nt < NNT; ++nt) {
-            float v[4] = {o[nt][0] * inv, o[nt][1] * inv, o[nt][2] * inv, o[nt][3] * inv};
-            if (a.gate != nullptr) {        // Qwen3.5: y * sigmoid(gate) (qwen3_5/modeling.rs:556-561)
-                const f32x4 gv = *(const f32x4*)(a.gate + (size_t)qrow * a.gate_stride + h * D + nt * 16 + g * 4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + expf(-gv[r]));
-            }
+            const float v[4] = {o[nt][0] * inv, o[nt][1] * inv, o[nt][2] * inv, o[nt][3] * inv};
             // (f32 rows: the input of the int8 o_proj GEMM's quantiser -- prompts over Q8_0-layout weights)
             if (a.out_f32 != nullptr) *(f32x4*)(a.out_f32 + ((size_t)qrow * a.Hq + h) * D + nt * 16 + g * 4) = (f32x4){v[0], v[1], v[2], v[3]};
             else
@@ -895,7 +887,7 @@ __global__ __launch_bounds__(256) void attn_prefill_fast_kernel(AttnPreArgs a_in
     }
 }
 
-// the shares of attn_prefill_fast_kernel's keys merged, four columns per thread
+// the shares of attn_prefill_fast_kernel's and attn_prompt_wide_kernel's keys merged, four columns per thread
 template <int D>
 __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(AttnPreArgs a) {
     constexpr float L2E = 1.4426950408889634f;
@@ -1452,7 +1444,7 @@ static bool launch_gemm_once(GemmArgs& a, int epi, hipStream_t s) {
     return true;
 }
 // kvt: KV_BF16 | KV_F16 | KV_F32 (the element type the kernel READS: f32 for the int8 / int4 shadow)
-// shares of the keys for a launch of the fast path (key tiles of 64 tokens at head_dim 128, of 32 at 256): `fill` blocks keep the chip busy (two on a CU, one); a share of fewer than eight
+// shares of the keys for a launch of the fast path (key tiles of 64 tokens; at head_dim 256, whose waves take halves of them, counted in those): `fill` blocks keep the chip busy (two on a CU, one); a share of fewer than eight
 // key tiles is not worth the merging launch, which costs more the more rows there are: at least a tile for every nine of the blocks that there are without shares.  us a layer of
 // width 1024, whole / shared: 500 rows (256 blocks) behind 512 / 1024 / 2048 / 3584 tokens, 32 heads of 128: 132.5 / 135.9, 144.2 / 145.2, 167.3 / 163.5, 201.6 / 191.5; 384 rows (192)
 // behind 1024 145.4 / 144.1; 256 rows (128) behind 1024 123.5 / 115.1; 64 rows behind 1024 / 3584 79.2 / 73.1, 136.7 / 78.4; 16 heads, 500 rows (128) behind 512 123.4 / 118.4;
@@ -1467,15 +1459,19 @@ static int prefill_split(const AttnPreArgs& a, int D) {
     while (n > 1 && (size_t)n * a.S * a.Hq * (D + 2) > a.ws_floats) --n;
     return n;
 }
-template <int D, int KT>
-static void launch_prefill_fast(AttnPreArgs a, int kvt, hipStream_t s) {
+// causal prompts over 2-byte pages
+static void launch_prefill_fast(AttnPreArgs a, int D, int kvt, hipStream_t s) {
     a.nsplit = prefill_split(a, D);
     const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64, a.nsplit);
-    // more than two workgroups on every CU: half as many with twice the waves (figures beside that kernel)
-    if (D == 128 && a.nrep % 2 == 0 && a.nsplit == 1 && grid.x * grid.y > 512) { launch_attn_prompt_pair(a, kvt, s); return; }
-    if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_F16>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((attn_prefill_fast_kernel<D, KT, KV_BF16>), grid, dim3(256), 0, s, a);
-    if (a.nsplit > 1) hipLaunchKernelGGL(attn_prefill_merge_kernel<D>, dim3((unsigned)(((size_t)a.S * a.Hq + 1024 / D - 1) / (1024 / D))), dim3(256), 0, s, a);
+    // head_dim 128, more than two workgroups on every CU: half as many with twice the waves (figures beside these kernels)
+    if (D == 256) launch_attn_prompt_wide(a, kvt, s);
+    else if (a.nrep % 2 == 0 && a.nsplit == 1 && grid.x * grid.y > 512) launch_attn_prompt_pair(a, kvt, s);
+    else if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<KV_F16>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_prefill_fast_kernel<KV_BF16>), grid, dim3(256), 0, s, a);
+    if (a.nsplit == 1) return;
+    const dim3 rows((unsigned)(((size_t)a.S * a.Hq + 1024 / D - 1) / (1024 / D)));
+    if (D == 256) hipLaunchKernelGGL(attn_prefill_merge_kernel<256>, rows, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(attn_prefill_merge_kernel<128>, rows, dim3(256), 0, s, a);
 }
 void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
     const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64);
@@ -1484,17 +1480,17 @@ void launch_attn_prefill(const AttnPreArgs& a, int D, int kvt, hipStream_t s) {
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
         if (fast_env != 0 && a.gate == nullptr && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 &&
             a.q_lo != nullptr) {
-            launch_prefill_fast<128, 64>(a, kvt, s);
+            launch_prefill_fast(a, D, kvt, s);
             return;
         }
         if (kvt == KV_F32) hipLaunchKernelGGL((attn_prefill_kernel<128, KV_F32>), grid, dim3(256), 0, s, a);
         else if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_kernel<128, KV_F16>), grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL((attn_prefill_kernel<128, KV_BF16>), grid, dim3(256), 0, s, a);
     } else {
-        // the hybrid family's gated head_dim-256 attention: the same fast path on 32-token key tiles
+        // the hybrid family's gated head_dim-256 attention: attn_prompt_wide_kernel
         static const int fast_env = getenv("CM_ATTN_PREFILL_FAST") ? atoi(getenv("CM_ATTN_PREFILL_FAST")) : 1;
         if (fast_env != 0 && (kvt == KV_F16 || kvt == KV_BF16) && a.page % 64 == 0 && a.q_lo != nullptr) {
-            launch_prefill_fast<256, 32>(a, kvt, s);
+            launch_prefill_fast(a, D, kvt, s);
             return;
         }
         if (kvt == KV_F32) hipLaunchKernelGGL((attn_prefill_kernel<256, KV_F32>), grid, dim3(256), 0, s, a);

@@ -1,4 +1,4 @@
-"""GPU: prompt attention of many query tiles (kernels_attn_prompt.hip) against the same prompt in portions, whose launches are small enough for attn_prefill_fast_kernel, and several
+"""GPU: prompt attention (kernels_attn_prompt.hip): many query tiles against the same prompt in portions, whose launches are small enough for attn_prefill_fast_kernel, and several
 prompts in one pass against each by itself.
 
 One layer: the cached rows and the weights are the same, and so is the order of every sum of the attention; the products around it add up in other tiles (1e-7 of a row), attention rows
@@ -55,3 +55,29 @@ def test_several_prompts(lengths):
         m.close()
     for a, b in zip(together, alone):
         assert np.isfinite(a).all() and np.abs(a.ravel() - b).max() < TOL * np.abs(b).max()
+
+
+# head_dim 256 with an output gate (attn_prompt_wide_kernel) against the general kernel, which pages of 32 tokens take: last rows at both ends of a tile's halves and of the query groups, several
+# sequences in a launch; a second pass whose keys are shared (37 and 200 rows behind 320 and 1024: shares of one tile, and of none, to eight).  The same rows and cache as above: 2e-5.
+@pytest.mark.parametrize("heads,kv,dtype", [(8, 2, "f16"), (4, 4, "bf16"), (16, 4, "f16")])
+def test_wide_heads(heads, kv, dtype):
+    from crane_amd.backend import Model
+    cfg = dict(configs.get_config("qwen3.5-0.8b"), vocab_size=512, num_hidden_layers=1, full_attention_interval=1, num_attention_heads=heads, num_key_value_heads=kv)
+    cfg.pop("layer_types", None)
+    rng = np.random.default_rng(heads)
+    prompts = [rng.integers(0, 512, n).tolist() for n in (1, 16, 31, 32, 33, 63, 64, 65, 97, 128, 193)]
+    long = rng.integers(0, 512, 1224).tolist()
+    rows = []
+    for page in (64, 128, 32):
+        got = []
+        for chunk in (1024, 320):
+            m = Model.synthetic(cfg, seed=3, max_seq_len=1280, max_seqs=16, prefill_chunk=chunk, kv_block_size=page, kv_dtype=dtype)
+            try:
+                got += [_last(m, long[:n]) for n in (357, 640, 1224)]
+                if chunk == 1024:
+                    got += [r.ravel() for r in np.asarray(m.prefill_batch([m.seq_alloc() for _ in prompts], prompts)[0], np.float64)]
+            finally:
+                m.close()
+        rows.append(got)
+    for a, b, c in zip(*rows):
+        assert np.isfinite(a).all() and np.abs(a - c).max() < TOL * np.abs(c).max() and np.abs(b - c).max() < TOL * np.abs(c).max()
