@@ -81,6 +81,9 @@ __device__ __forceinline__ f32x4 mma_k16(const bf16x4& a, const bf16x4& b, const
     else return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
+// Workgroups go round the eight XCDs: the place of workgroup `id` of `all` where those of an XCD are neighbours
+__device__ __forceinline__ int xcd_neighbours(int id, int all) { return (id & 7) * (all >> 3) + min(id & 7, all & 7) + (id >> 3); }
+
 // four f32 as bf16 hi + lo planes; four weights as two terms of the pages' type
 __device__ __forceinline__ void split_store4(uint16_t* hi, uint16_t* lo, size_t off, const float v[4]) {
     uint16_t h[4], l[4];

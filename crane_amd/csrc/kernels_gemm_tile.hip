@@ -9,7 +9,7 @@
 //   * the walk is in slots of 32 elements of K, and the requests for a later tile are spread over two or three of the four slots that a tile of activations lasts;
 //   * a request's address is a scalar base, advanced with K, and one 32-bit offset per lane and row band: no 64-bit pointers in vector registers (256 x 256: 230 of 256 registers).
 // Measured (us a launch, real operands back to back, before / here): 24576 x 4096 at 2048 rows 674 / 560, at 452 180 / 145, at 300 158 / 123; 6144 x 4096 at 2048 193 / 162;
-// 4096 x 12288 at 2048 330 / 312 (one round of 128 x 256 either way); 12288 x 2048 at 2048 196 / 171; 4096 x 1024 with gelu at 3172 72 / 60.
+// 4096 x 12288 at 2048 330 / 288 (one round of 128 x 256 either way); 12288 x 2048 at 2048 196 / 171; 4096 x 1024 with gelu at 3172 72 / 60.
 //
 // LDS: two stages of activations, 64 deep (an operand row is one whole 128-byte line per stage), and two of weights, 64 deep, or 32 where 256 rows of activations leave 32 KB
 // for them (their lines are fetched twice, which the L1's fill path has room for: 64 KB of lines per 2048 cycles of MFMA at 64 bytes a cycle).  Slot p of a row holds its 16-byte
@@ -55,10 +55,12 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(GemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % GM, wn = wave / GM;
     const int tiles_m = (a.M + BM - 1) / BM, nb = tiles_m * (a.N / BN);
-    const int ks = (int)blockIdx.x / nb;
-    int bid = (int)blockIdx.x - ks * nb;
-    bid = (bid & 7) * (nb >> 3) + min(bid & 7, nb & 7) + (bid >> 3);      // neighbouring tiles, which share a weight tile, on one XCD
-    const int tn = bid / tiles_m, m0 = (bid - tn * tiles_m) * BM, n0 = tn * BN;
+    const int ks = (int)blockIdx.x / nb, bid = xcd_neighbours((int)blockIdx.x - ks * nb, nb);
+    // The tiles of an XCD are a patch of four row tiles and the columns beside them, which its L2 fetches once for all: a whole column of 16 row tiles and the next one was the
+    // activations of every row, 8 times over the chip.  us, columns first / patches (of eight rows in brackets): 4096 x 12288 at 2048 rows 304 / 288 (291), at 1400 245 / 237 (245), at 1000
+    // 165 / 160 (165); 4096 x 4096 at 2048 110 / 103 (104); 2048 x 6144 at 2048 89.4 / 86.0 (87.0); products of one or two row patches as before
+    const int tiles_n = a.N / BN, patches = (tiles_m + 3) / 4, high = (tiles_m + patches - 1) / patches, patch = bid / (high * tiles_n), in = bid - patch * high * tiles_n;
+    const int rows = min(high, tiles_m - patch * high), tn = in / rows, m0 = (patch * high + in - tn * rows) * BM, n0 = tn * BN;
     const int K = a.K, nt = K / 64 / a.ksplit;                            // tiles of 64 of this block, from ks * nt on
 
     f32x4 acc[NI][NJ];
