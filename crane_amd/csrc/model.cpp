@@ -1144,11 +1144,29 @@ int Model::prefill_chunk_rows() const {
     return c < 1 ? 1 : c;
 }
 
+// Rows of one pass over ONE sequence's prompt where the caller left the chunk open: 4096 for hybrid decoders, and 128 more where those are the last.  Their projections are 1024 .. 5120 wide: at 2048
+// rows the tiles of a product fill the chip only with K in slices, whose sums cost a launch and three times the output's bytes; every launch of a pass has a start and an end, and the last rows
+// of a prompt have passes of their own over all weights.  ms, passes of 2048 / so: Qwen3.5-2B 2100 tokens 15.1 / 14.7, 2500 18.0 / 16.8, 4000 25.5 / 23.2, 4165 28.5 / 25.5 (in passes of 4096 26.2), 4500 30.8 /
+// 28.4 (in 4224 30.4); 0.8B 2049 9.7 / 9.3, 3000 13.1 / 11.7, 4165 18.4 / 15.9; 27B 2100 194 / 182, 3000 275 / 246, 4165 379 / 366.  Dense decoders, 8B: 2500 57.6 / 57.3, 3000 69.3 / 71.8: 2048.
+// Several prompts in a pass, images and explicit positions keep the chunk as their limit.  Scratch that the card has no room for twice over is not asked for.
+constexpr int PASS_ROWS = 4096, PASS_TAIL = 128;
+int Model::prefill_pass_rows() const {
+    const int c = prefill_chunk_rows();
+    if (!cfg.hybrid || quantized || rccl || opts.prefill_chunk != 0 || max_seq <= c) return c;
+    const int rows = std::min<long>(max_seq, PASS_ROWS + PASS_TAIL);
+    const int qkv_rows = (2 * Hq_l + 2 * Hkv_l) * cfg.D;
+    const size_t per_row = 4 * ((size_t)2 * cfg.H + std::max(qkv_rows, in_proj_pad) + 3 * (size_t)std::max(cfg.value_dim(), Hq_l * cfg.D) + 2 * (size_t)cfg.key_dim() + I_l + 3 * (size_t)cfg.NV +
+                                (size_t)cfg.NV * GDN_CK_FLOATS / GDN_CK);
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) == hipSuccess && (size_t)(rows - c) * per_row * 2 <= free ? rows : c;
+}
+
 void Model::ensure_prefill_buffers() {
     if (pX || layered) return;
     const int H = cfg.H, D = cfg.D;
     chunk = prefill_chunk_rows();
-    chunk_pad = (chunk + 127) / 128 * 128;
+    pass_rows = prefill_pass_rows();
+    const int rows = pass_rows, rows_pad = (rows + 127) / 128 * 128;
     // prompt activations as bf16 hi + lo (two products per GEMM: what the 1e-3 bound of a bf16 checkpoint needs) unless the caller asked
     // for plain bf16 -- or left the choice open (0) on QUANTISED weights: their scratch copy for the GEMMs is already rounded to bf16
     // (2^-9 per weight, tests: 1e-2 of the oracle on the dequantised weights), the activations' low halves would refine past that
@@ -1157,30 +1175,30 @@ void Model::ensure_prefill_buffers() {
     prefill_ok = (qkv_rows % 128 == 0) && (H % 128 == 0) && ((2 * I_l) % 128 == 0) && (H % 32 == 0) && (I_l % 32 == 0) &&
                  (!cfg.hybrid || cfg.value_dim() % 32 == 0);
     if (!prefill_ok) return;
-    pX = dalloc<float>((size_t)chunk * H);
+    pX = dalloc<float>((size_t)rows * H);
     ensure_gemm_workspace();
-    if (rccl) pY = dalloc<float>((size_t)chunk * H);
-    pQKV = dalloc<float>((size_t)chunk * std::max(qkv_rows, in_proj_pad));
+    if (rccl) pY = dalloc<float>((size_t)rows * H);
+    pQKV = dalloc<float>((size_t)rows * std::max(qkv_rows, in_proj_pad));
     if (cfg.hybrid) {
-        pGY = dalloc<float>((size_t)chunk * cfg.value_dim());
-        gdn_pre_q = dalloc<float>((size_t)chunk * cfg.key_dim());      // three-pass Gated-Delta-Net prefill (kernels_gdn.hip)
-        gdn_pre_k = dalloc<float>((size_t)chunk * cfg.key_dim());
-        gdn_pre_v = dalloc<float>((size_t)chunk * cfg.value_dim());
-        gdn_pre_bd = dalloc<float>((size_t)chunk * cfg.NV * 2);
-        gdn_pre_g = dalloc<float>((size_t)chunk * cfg.NV);
+        pGY = dalloc<float>((size_t)rows * cfg.value_dim());
+        gdn_pre_q = dalloc<float>((size_t)rows * cfg.key_dim());      // three-pass Gated-Delta-Net prefill (kernels_gdn.hip)
+        gdn_pre_k = dalloc<float>((size_t)rows * cfg.key_dim());
+        gdn_pre_v = dalloc<float>((size_t)rows * cfg.value_dim());
+        gdn_pre_bd = dalloc<float>((size_t)rows * cfg.NV * 2);
+        gdn_pre_g = dalloc<float>((size_t)rows * cfg.NV);
         if (cfg.Kd == 128 && cfg.Vd == 128)           // chunk-parallel scan scratch: W | U0 | P | G per (64-token chunk, value head)
-            gdn_ck = dalloc<float>((size_t)((chunk + GDN_CK - 1) / GDN_CK) * cfg.NV * GDN_CK_FLOATS);
+            gdn_ck = dalloc<float>((size_t)((rows + GDN_CK - 1) / GDN_CK) * cfg.NV * GDN_CK_FLOATS);
     }
     auto z = [&](size_t n) {
         uint16_t* p = dalloc<uint16_t>(n);
         CM_HIP(hipMemsetAsync(p, 0, n * sizeof(uint16_t), stream));
         return p;
     };
-    pXN_hi = z((size_t)chunk_pad * H); pXN_lo = z((size_t)chunk_pad * H);
-    pQ_hi = z((size_t)chunk_pad * Hq_l * D); pQ_lo = z((size_t)chunk_pad * Hq_l * D);
+    pXN_hi = z((size_t)rows_pad * H); pXN_lo = z((size_t)rows_pad * H);
+    pQ_hi = z((size_t)rows_pad * Hq_l * D); pQ_lo = z((size_t)rows_pad * Hq_l * D);
     const size_t at_cols = std::max((size_t)Hq_l * D, (size_t)(cfg.hybrid ? cfg.value_dim() : 0));
-    pAT_hi = z((size_t)chunk_pad * at_cols); pAT_lo = z((size_t)chunk_pad * at_cols);
-    pHH_hi = z((size_t)chunk_pad * I_l); pHH_lo = z((size_t)chunk_pad * I_l);
+    pAT_hi = z((size_t)rows_pad * at_cols); pAT_lo = z((size_t)rows_pad * at_cols);
+    pHH_hi = z((size_t)rows_pad * I_l); pHH_lo = z((size_t)rows_pad * I_l);
     if (kvq()) {
         const size_t shadow = (size_t)max_pages_per_seq * Hkv_l * page * D;
         kshadow = dalloc<float>(shadow);
@@ -1196,8 +1214,8 @@ void Model::ensure_prefill_buffers() {
     q8_prefill = q8_prefill_want && q8_prefill_eligible();
     if (q8_prefill) {
         ensure_batch_buffers();                                    // qx_codes / qx_scales pairs (sized for a whole pass there)
-        pATf = dalloc<float>((size_t)chunk * Hq_l * D);
-        pHf = dalloc<float>((size_t)chunk * I_l);                  // silu(gate) * up of the pass, f32 (the down projection's quantiser input)
+        pATf = dalloc<float>((size_t)rows * Hq_l * D);
+        pHf = dalloc<float>((size_t)rows * I_l);                  // silu(gate) * up of the pass, f32 (the down projection's quantiser input)
         for (LayerW& w : layers) {
             if (w.full) continue;
             w.ba_pad = dalloc<uint16_t>((size_t)128 * H);          // the a / b rows as one zero-padded 128-row GEMM tile
@@ -1209,7 +1227,7 @@ void Model::ensure_prefill_buffers() {
         // one dequantised matrix at a time: bf16 hi plane + lo plane (parity mode), and the f32 gate|up sums of the two-pass GEMM
         wq_scratch_elems = std::max(std::max((size_t)2 * I_l * H, (size_t)qkv_rows * H), (size_t)in_proj_pad * H);
         wq_scratch = dalloc<uint16_t>(2 * wq_scratch_elems);
-        pGU = dalloc<float>((size_t)chunk * 2 * I_l);
+        pGU = dalloc<float>((size_t)rows * 2 * I_l);
         // CM_QUANT_PREFILL_CACHE=1 (opt-in): keep every
         // dequantised matrix (hi + lo: 4 bytes per weight -- more than the bf16 checkpoint) instead of dequantising it again per pass
         // (4.5 % of a Q8_0 serving run, before Q8_0-layout models moved to the int8 prompt pass).  An allocation that fails mid-pass
@@ -1217,8 +1235,8 @@ void Model::ensure_prefill_buffers() {
         wq_cache = false;
         if (const char* e = getenv("CM_QUANT_PREFILL_CACHE")) wq_cache = atoi(e) != 0;
     }
-    d_ids = (uint32_t*)dalloc<int>(chunk);
-    CM_HIP(hipHostMalloc((void**)&h_ids, (size_t)chunk * sizeof(uint32_t)));
+    d_ids = (uint32_t*)dalloc<int>(rows);
+    CM_HIP(hipHostMalloc((void**)&h_ids, (size_t)rows * sizeof(uint32_t)));
 }
 
 // the decoder layers over the S rows of pX.  The row-wise work (norms, every GEMM) runs once over all rows; what mixes tokens --
@@ -1595,8 +1613,8 @@ void Model::prefill_multi(const int32_t* sq, const uint32_t* const* ids, const s
 void Model::prefill(const uint32_t* ids, size_t n, size_t start_pos) {
     const int H = cfg.H;
     hipStream_t s = stream;
-    for (size_t off = 0; off < n; off += (size_t)chunk) {
-        const int S = (int)std::min<size_t>((size_t)chunk, n - off);
+    for (size_t off = 0; off < n;) {
+        const int S = (int)(n - off <= (size_t)pass_rows ? n - off : (size_t)std::min(pass_rows, std::max(chunk, PASS_ROWS)));
         const int sp = (int)(start_pos + off);
         CM_HIP(hipStreamSynchronize(s));                       // h_ids reuse
         if (embeds_host != nullptr) {                          // forward_embeds: the caller's hidden rows ARE the layer-0 input
@@ -1616,6 +1634,7 @@ void Model::prefill(const uint32_t* ids, size_t n, size_t start_pos) {
             ++ring_count;
             enqueue_lm_head(true);
         }
+        off += (size_t)S;
     }
 }
 

@@ -236,20 +236,21 @@ struct Model {
     char* h_stage = nullptr;
     hipEvent_t ev_stage[STAGES] = {};
 
-    // prefill scratch (allocated on first use; sized for one chunk)
-    int chunk = 2048, chunk_pad = 2048;
+    // prefill scratch (allocated on first use; sized for pass_rows)
+    int chunk = 2048;           // tokens of several prompts in a pass, of a prompt with images
+    int pass_rows = 2048;       // rows of a pass over one prompt: the chunk or more (prefill_pass_rows)
     bool prefill_ok = false, prefill_split2 = true;
     int gemm256 = 1;           // prompt-pass / decode-group GEMMs: 0 = never an LDS-DMA kernel, 1 = automatic, 2 = always kernels_gemmw4.hip, 3 = kernels_gemm256.hip only (cm_debug_set("gemm256"))
-    float* pX = nullptr;        // [chunk, H] f32 residual stream
+    float* pX = nullptr;        // [pass_rows, H] f32 residual stream
     float* pWS = nullptr;       // split-K workspace of the prefill GEMMs: at most 1024 partial tiles of 128 x 128 f32
     static constexpr size_t gemm_ws_floats = (size_t)1024 * 128 * 128;
-    float* pY = nullptr;        // [chunk, H] TP partial
-    float* pQKV = nullptr;      // [chunk, qkv_rows] f32
-    uint16_t *pXN_hi = nullptr, *pXN_lo = nullptr;     // [chunk_pad, H]
-    uint16_t *pQ_hi = nullptr, *pQ_lo = nullptr;       // [chunk_pad, Hq_l D]
-    uint16_t *pAT_hi = nullptr, *pAT_lo = nullptr;     // [chunk_pad, Hq_l D]
-    uint16_t *pHH_hi = nullptr, *pHH_lo = nullptr;     // [chunk_pad, I_l]
-    float* pGY = nullptr;       // [chunk, value_dim] f32 GDN output (Qwen3.5)
+    float* pY = nullptr;        // [pass_rows, H] TP partial
+    float* pQKV = nullptr;      // [pass_rows, qkv_rows] f32
+    uint16_t *pXN_hi = nullptr, *pXN_lo = nullptr;     // [pass_rows, H]
+    uint16_t *pQ_hi = nullptr, *pQ_lo = nullptr;       // [pass_rows, Hq_l D]
+    uint16_t *pAT_hi = nullptr, *pAT_lo = nullptr;     // [pass_rows, Hq_l D]
+    uint16_t *pHH_hi = nullptr, *pHH_lo = nullptr;     // [pass_rows, I_l]
+    float* pGY = nullptr;       // [pass_rows, value_dim] f32 GDN output (Qwen3.5)
     uint32_t* d_ids = nullptr;
     uint32_t* h_ids = nullptr;
 
@@ -322,14 +323,15 @@ struct Model {
     // prompts over Q8_0-layout weights on the int8 matrix cores (default where every projection of the dense family qualifies;
     // CM_QUANT_PREFILL_INT8=0 / cm_debug_set("prefill_q8", 0) before the first prompt: the dequantised-to-bf16 GEMMs)
     bool q8_prefill_want = true, q8_prefill = false;
-    float* pATf = nullptr;             // [chunk][Hq_l D] f32 attention rows of the pass (the o_proj quantiser's input)
-    float* pHf = nullptr;              // [chunk][I_l] f32 silu(gate) * up rows of the pass
+    float* pATf = nullptr;             // [pass_rows][Hq_l D] f32 attention rows of the pass (the o_proj quantiser's input)
+    float* pHf = nullptr;              // [pass_rows][I_l] f32 silu(gate) * up rows of the pass
     int q8_xs = QGEMM_MAXM;            // floats between the scale rows of the code buffers in a prompt pass of more than 128 rows
     int prefill_chunk_rows() const;
+    int prefill_pass_rows() const;
     bool q8_prefill_eligible() const;
     uint16_t* wq_scratch = nullptr;    // [2][max N*K] bf16 hi | lo planes: one dequantised matrix at a time for the prefill GEMMs
     size_t wq_scratch_elems = 0;
-    float* pGU = nullptr;              // [chunk][2 I_l] f32 gate|up sums of the two-pass (hi + lo operand) GEMM
+    float* pGU = nullptr;              // [pass_rows][2 I_l] f32 gate|up sums of the two-pass (hi + lo operand) GEMM
     bool wq_cache = false;             // keep every dequantised matrix instead (CM_QUANT_PREFILL_CACHE=1, opt-in)
     bool gdn_ck_on = true;                      // cm_debug_set("gdn_chunked"): prompts of >= 64 tokens take the chunk-parallel Gated-Delta-Net scan
     float *gdn_pre_q = nullptr, *gdn_pre_k = nullptr, *gdn_pre_v = nullptr, *gdn_pre_bd = nullptr, *gdn_pre_g = nullptr, *gdn_ck = nullptr;   // GDN prefill scratch
