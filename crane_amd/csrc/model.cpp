@@ -1144,17 +1144,18 @@ int Model::prefill_chunk_rows() const {
     return c < 1 ? 1 : c;
 }
 
-// Rows of one pass over ONE sequence's prompt where the caller left the chunk open: 4096 for hybrid decoders, and 128 more where those are the last.  Their projections are 1024 .. 5120 wide: at 2048
-// rows the tiles of a product fill the chip only with K in slices, whose sums cost a launch and three times the output's bytes; every launch of a pass has a start and an end, and the last rows
-// of a prompt have passes of their own over all weights.  ms, passes of 2048 / so: Qwen3.5-2B 2100 tokens 15.1 / 14.7, 2500 18.0 / 16.8, 4000 25.5 / 23.2, 4165 28.5 / 25.5 (in passes of 4096 26.2), 4500 30.8 /
-// 28.4 (in 4224 30.4); 0.8B 2049 9.7 / 9.3, 3000 13.1 / 11.7, 4165 18.4 / 15.9; 27B 2100 194 / 182, 3000 275 / 246, 4165 379 / 366.  Dense decoders, 8B: 2500 57.6 / 57.3, 3000 69.3 / 71.8: 2048.
-// Several prompts in a pass, images and explicit positions keep the chunk as their limit.  Scratch that the card has no room for twice over is not asked for.
+// Rows of one pass over ONE sequence's prompt where the caller left the chunk open: 4096 for hybrid decoders and for dense ones up to 2048 wide, and 128 more where those are the last.  Their
+// projections are 1024 .. 5120 wide: at 2048 rows the tiles of a product fill the chip only with K in slices, whose sums cost a launch and three times the output's bytes; every launch of a pass
+// has a start and an end, and the last rows of a prompt have passes of their own over all weights.  ms, passes of 2048 / so: Qwen3.5-2B 2100 tokens 15.1 / 14.7, 2500 18.0 / 16.8, 4000 25.5 / 23.2, 4165
+// 28.5 / 25.5 (in passes of 4096 26.2), 4500 30.8 / 28.4 (in 4224 30.4); 0.8B 2200 11.3 / 9.8, 3000 13.1 / 11.7, 4165 18.4 / 15.9; 27B 2100 194 / 182, 3000 275 / 246, 4165 379 / 366; dense, Qwen3-0.6B 2100
+// 8.4 / 7.6, 4000 14.7 / 12.1; 28 layers of width 2048 2100 14.7 / 14.3, 4000 25.9 / 22.9.  8B: 2500 57.6 / 57.3, 3000 69.3 / 71.8, 2176 52.4 / 53.5: 2048.  Several prompts in a pass, images and
+// explicit positions keep the chunk as their limit.  Scratch that the card has no room for twice over is not asked for.
 constexpr int PASS_ROWS = 4096, PASS_TAIL = 128;
 int Model::prefill_pass_rows() const {
     const int c = prefill_chunk_rows();
-    if (!cfg.hybrid || quantized || rccl || opts.prefill_chunk != 0 || max_seq <= c) return c;
+    if ((!cfg.hybrid && cfg.H > 2048) || quantized || rccl || opts.prefill_chunk != 0 || max_seq <= c) return c;
     const int rows = std::min<long>(max_seq, PASS_ROWS + PASS_TAIL);
-    const int qkv_rows = (2 * Hq_l + 2 * Hkv_l) * cfg.D;
+    const int qkv_rows = (cfg.hybrid ? 2 * Hq_l + 2 * Hkv_l : Hq_l + 2 * Hkv_l) * cfg.D;
     const size_t per_row = 4 * ((size_t)2 * cfg.H + std::max(qkv_rows, in_proj_pad) + 3 * (size_t)std::max(cfg.value_dim(), Hq_l * cfg.D) + 2 * (size_t)cfg.key_dim() + I_l + 3 * (size_t)cfg.NV +
                                 (size_t)cfg.NV * GDN_CK_FLOATS / GDN_CK);
     size_t free = 0, total = 0;
@@ -1614,7 +1615,9 @@ void Model::prefill(const uint32_t* ids, size_t n, size_t start_pos) {
     const int H = cfg.H;
     hipStream_t s = stream;
     for (size_t off = 0; off < n;) {
-        const int S = (int)(n - off <= (size_t)pass_rows ? n - off : (size_t)std::min(pass_rows, std::max(chunk, PASS_ROWS)));
+        // the rest, if a pass holds it; less than nine rows behind whole chunks, which no band of a product is for (gemm_band), alone: 2049 tokens of Qwen3.5-2B 16.2 ms in one pass, 15.6 so
+        const size_t rest = n - off, over = rest > (size_t)chunk && rest % (size_t)chunk < 9 ? rest % (size_t)chunk : 0;
+        const int S = (int)(rest <= (size_t)pass_rows ? rest - over : (size_t)std::min(pass_rows, std::max(chunk, PASS_ROWS)));
         const int sp = (int)(start_pos + off);
         CM_HIP(hipStreamSynchronize(s));                       // h_ids reuse
         if (embeds_host != nullptr) {                          // forward_embeds: the caller's hidden rows ARE the layer-0 input

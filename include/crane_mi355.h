@@ -79,7 +79,7 @@ typedef struct cm_opts {
     int32_t  use_graph;        /* 0 default(on), 1 on, -1 off: hipGraph decode step  */
     uint32_t prefill_chunk;    /* tokens per prefill chunk (default 2048,            */
                                /*   PREFILL_CHUNK_SIZE engine/mod.rs:65; one prompt  */
-                               /*   of a hybrid decoder: then 4096 and a short rest) */
+                               /*   of a hybrid or narrow decoder: then up to 4224)  */
     int32_t  prefill_split;    /* prompt pass of the MFMA GEMMs: 0 (default) / 2 = parity mode: activations as bf16 hi + lo (two    */
                                /*   products: the 1e-3 bound of a bf16 checkpoint) and, over QUANTISED weights on the dequantised    */
                                /*   path (K-quants, CM_QUANT_ACT=f32, the hybrid family), the dequantised operand as bf16 hi + lo    */

@@ -61,19 +61,20 @@ def test_one_plane_against_two():
     assert np.isfinite(out[1]).all() and np.abs(out[0] - out[1]).max() < 3e-2 * np.abs(out[0]).max()
 
 
-# a prompt of a hybrid decoder in passes of up to 4096 rows, and 128 more at its end (the chunk left open), against passes of 2048 (the chunk given): one row more than a chunk, as many as a pass takes, one more;
-# a second prompt behind them and a token behind that.  The chunked sums of three Gated-Delta-Net layers and a layer of attention in other orders: the bar of tests/test_gpu_prefill_shares.py
-def test_long_passes():
+# a prompt in passes of up to 4096 rows, and 128 more at its end (the chunk left open), against passes of 2048 (the chunk given): one row more than a chunk (alone in either), nine, as many as a pass takes, one
+# more; a second prompt behind them and a token behind that; a hybrid decoder and a dense one.  The chunked sums of three Gated-Delta-Net layers and a layer of attention in other orders: the bar of tests/test_gpu_prefill_shares.py
+@pytest.mark.parametrize("model,layers", [("qwen3.5-0.8b", 4), ("qwen3-0.6b", 1)])
+def test_long_passes(model, layers):
     from crane_amd import _lib
     from crane_amd.backend import Model
-    cfg = dict(configs.get_config("qwen3.5-0.8b"), vocab_size=512, num_hidden_layers=4)
+    cfg = dict(configs.get_config(model), vocab_size=512, num_hidden_layers=layers)
     ids = np.random.default_rng(5).integers(0, 512, 4400).tolist()
     out = []
     for chunk in (0, 2048):
         m = Model.synthetic(cfg, seed=3, max_seq_len=4608, max_seqs=3, prefill_chunk=chunk)
         try:
             got = []
-            for n in (2049, 4096, 4224, 4225):
+            for n in (2049, 2057, 4096, 4224, 4225):
                 s = m.seq_alloc()
                 got.append(np.asarray(m.seq_forward(s, ids[:n], 0)[0], np.float64).ravel())
                 got.append(np.asarray(m.seq_forward(s, ids[n:n + 130], n)[0], np.float64).ravel())
