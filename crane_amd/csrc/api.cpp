@@ -116,6 +116,23 @@ static void create_ranks(cm_model* h, const std::string& cfg, const cm_opts* opt
     });
 }
 
+namespace {
+// arrays of a test hook on the device
+struct HookMem {
+    std::vector<void*> held;
+    template <class T>
+    T* take(size_t n, const T* from = nullptr) {
+        void* p = nullptr;
+        CM_HIP(hipMalloc(&p, n * sizeof(T)));
+        held.push_back(p);
+        if (from) CM_HIP(hipMemcpy(p, from, n * sizeof(T), hipMemcpyHostToDevice));
+        else CM_HIP(hipMemset(p, 0, n * sizeof(T)));
+        return (T*)p;
+    }
+    ~HookMem() { for (void* p : held) (void)hipFree(p); }
+};
+}  // namespace
+
 extern "C" {
 
 int cm_create(const char* model_dir, const cm_opts* opts, cm_model** out) {
@@ -582,6 +599,44 @@ int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws
 int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats) {
     int bm = 0, bn = 0, ks = 0;
     return cm::gemm_tile_plan(m, n, k, (size_t)ws_floats, norm != 0, &bm, &bn, &ks, nullptr) ? bm * 10000 + bn * 10 + ks : 0;
+}
+
+int cm_debug_rope_rows(const float* rows, int32_t n, int32_t kv_heads, int32_t slices, const float* cos, const float* sin, float* out) {
+    if (!rows || !cos || !sin || !out || n < 1 || n > 4096 || kv_heads < 1 || kv_heads > 64 || slices < 1 || slices > 8) return CM_ERR_INVALID;
+    return guard(nullptr, [&] {
+        const size_t kv = (size_t)n * kv_heads * 128;
+        HookMem m;
+        cm::QkRopeArgs a{};
+        a.qkv = m.take((size_t)slices * 2 * kv, rows); a.parts = slices; a.part = 2 * kv;
+        a.cos = m.take((size_t)n * 64, cos); a.sin = m.take((size_t)n * 64, sin);
+        a.block_table = m.take<int32_t>(1);
+        float* pool = m.take<float>(2 * kv);
+        a.kpool = pool; a.vpool = pool + kv;
+        a.Hkv = kv_heads; a.page = n; a.row_stride = 2 * kv_heads * 128; a.v_off = kv_heads * 128; a.rot_dim = 128; a.scale = 1.f;
+        if (!cm::qknorm_rope_adds_slices(a, 128, 1)) throw CmError(CM_ERR_UNSUPPORTED, "another rotation kernel");
+        cm::launch_qknorm_rope_kv(a, 128, n, 1, 0);
+        CM_HIP(hipGetLastError());
+        CM_HIP(hipMemcpy(out, pool, 2 * kv * sizeof(float), hipMemcpyDeviceToHost));
+    });
+}
+
+int cm_debug_gdn_step(const float* proj, const float* conv_w, const float* state, int32_t heads, float* out) {
+    if (!proj || !conv_w || !state || !out || heads < 1 || heads > 64) return CM_ERR_INVALID;
+    return guard(nullptr, [&] {
+        const size_t kd = (size_t)heads * 128, conv = 3 * kd, row = conv + kd + 2 * (size_t)heads;
+        const std::vector<float> ones(128, 1.f);
+        HookMem m;
+        cm::GdnArgs a{};
+        a.proj = m.take(row, proj); a.conv_w = m.take(conv * 4, conv_w); a.conv_pool = m.take<float>(2 * conv * 3); a.state_pool = m.take(kd * 128, state);
+        a.A_log = m.take<float>((size_t)heads); a.dt_bias = m.take<float>((size_t)heads); a.gnorm_w = m.take(128, ones.data());
+        a.out = m.take<float>(kd); a.st = m.take<cm::StepState>(1);
+        a.gdn_scratch = m.take<float>((size_t)heads * 132); a.gdn_ticket = m.take<int>((size_t)heads);
+        a.NV = heads; a.vpg = 1; a.key_dim = (int)kd; a.gdn_layers = 1; a.n_seq = 1; a.S = 1; a.proj_stride = a.batch_proj_stride = (int)row; a.out_stride = a.batch_out_stride = (int)kd;
+        a.eps = 1e-6f;
+        cm::launch_gdn(a, 0);
+        CM_HIP(hipGetLastError());
+        CM_HIP(hipMemcpy(out, a.out, kd * sizeof(float), hipMemcpyDeviceToHost));
+    });
 }
 
 int cm_debug_attn_group_plan(int32_t pairs, int32_t nrep, int64_t longest, int32_t slices, int32_t num_cu, int32_t most) {

@@ -278,8 +278,7 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs a) {
 #pragma unroll
         for (int j = 0; j < KS; ++j) y += part[j][tid];
         __hip_atomic_store(&yraw[cb * CB + tid], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        float sy = y * y;
-        sy = group_sum(sy, 32);
+        const float sy = group_sum(fmaf(y, y, lane_xor<16>(y * y)), 16);      // (written out: the first sum takes its own square unrounded)
         if (tid == 0) __hip_atomic_store(&yraw[V + cb], sy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // every storing wave drains its write-through stores

@@ -207,11 +207,13 @@ __global__ __launch_bounds__(256) void qknorm_rope_kv4_kernel(QkRopeArgs a_in) {
         }
         const int rp = pos + a.rope_delta, i0 = d0 & 63;
         const f32x4 c4 = *(const f32x4*)(a.cos + (size_t)rp * 64 + i0), s4 = *(const f32x4*)(a.sin + (size_t)rp * 64 + i0);
+        // x c -+ other s: elements 0 and 1 of four with one rounding at the end, 2 and 3 with one more.  Written out, so that pages, and the codes made of rows that have read them, stay
+        // what they are however the compiler would contract these
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float other = lane_xor<16>(xv[e]);           // d < 64: x[d + 64], else x[d - 64]
-            const float lo = d0 < 64 ? xv[e] : other, hi = d0 < 64 ? other : xv[e];
-            xv[e] = d0 < 64 ? lo * c4[e] - hi * s4[e] : lo * s4[e] + hi * c4[e];
+#pragma clang fp contract(off)
+            const float other = lane_xor<16>(xv[e]), p = other * s4[e], y = d0 < 64 ? -p : p;         // other: d < 64: x[d + 64], else x[d - 64]
+            xv[e] = e < 2 ? __builtin_fmaf(xv[e], c4[e], y) : xv[e] * c4[e] + y;
         }
     }
     auto pack4 = [&](const float (&v)[4], u32x2& o) {

@@ -552,6 +552,14 @@ int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws
 /* Test hook (host logic only, no GPU): rows * 10000 + columns * 10 + K slices of the tiles that m prompt rows of such a product run on (norm: one of the rows behind it); 0: another kernel. */
 int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats);
 
+/* Test hook: the keys and values that the rotation of prompts (head_dim 128, no norm) appends to 32-bit pages: rows [slices][n][2 kv_heads][128], cos and sin [n][64];
+ * out [2 (keys, values)][kv_heads][n][128]. */
+int cm_debug_rope_rows(const float* rows, int32_t n, int32_t kv_heads, int32_t slices, const float* cos, const float* sin, float* out);
+
+/* Test hook: one Gated-Delta-Net decode step that normalises itself, at position 0 on `state` [heads][128][128], a key head per value head, A_log and dt_bias 0, norm weights 1:
+ * proj [5 parts: q, k, v, z of heads x 128, b and a of heads], conv_w [3 heads 128][4], out [heads][128]. */
+int cm_debug_gdn_step(const float* proj, const float* conv_w, const float* state, int32_t heads, float* out);
+
 /* Test hook (host logic only, no GPU): among how many blocks the prompt attention shares the keys of a query tile: `rows` queries behind `start` cached
  * tokens, `heads` query heads of 128 or 256. */
 int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32_t head_dim);
