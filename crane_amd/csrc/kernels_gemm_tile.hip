@@ -9,7 +9,8 @@
 //   * the walk is in slots of 32 elements of K, and the requests for a later tile are spread over two or three of the four slots that a tile of activations lasts;
 //   * a request's address is a scalar base, advanced with K, and one 32-bit offset per lane and row band: no 64-bit pointers in vector registers (256 x 256: 230 of 256 registers).
 // Measured (us a launch, real operands back to back, before / here): 24576 x 4096 at 2048 rows 674 / 560, at 452 180 / 145, at 300 158 / 123; 6144 x 4096 at 2048 193 / 162;
-// 4096 x 12288 at 2048 330 / 288 (one round of 128 x 256 either way); 12288 x 2048 at 2048 196 / 171; 4096 x 1024 with gelu at 3172 72 / 60.
+// 4096 x 12288 at 2048 330 / 288 (one round of 128 x 256 either way); 12288 x 2048 at 2048 196 / 171; 4096 x 1024 with gelu at 3172 72 / 60.  (Gate and up in these with a SiLU of
+// fewer roundings than silu_mul's, which takes 1 .. 2 % more: 24576 x 4096 at 2048 rows 545 / 556, at 452 147.7 / 149.)
 //
 // LDS: two stages of activations, 64 deep (an operand row is one whole 128-byte line per stage), and two of weights, 64 deep, or 32 where 256 rows of activations leave 32 KB
 // for them (their lines are fetched twice, which the L1's fill path has room for: 64 KB of lines per 2048 cycles of MFMA at 64 bytes a cycle).  Slot p of a row holds its 16-byte
@@ -23,8 +24,12 @@ namespace cm {
 
 namespace {
 
-// silu(g) u as g / (1 + e^-g) with the hardware's exponential and reciprocal (expf and a division: 11 us of a 256 x 256 tile's 190)
-__device__ __forceinline__ float silu_mul(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u; }
+// silu(g) u with the roundings of the other kernels' epilogues, so that a row has the same bits beside any number of rows (exp2(-1.4427 g) and a bare reciprocal round the exponent:
+// 1.8e-6 of the value at g above -30 where this is 1.4e-7 off; the product is rounded before its planes are taken)
+__device__ __forceinline__ float silu_mul(float g, float u) {
+#pragma clang fp contract(off)
+    return g / (1.0f + expf(-g)) * u;
+}
 template <int NW>
 __device__ __forceinline__ void put_words(uint16_t* p, const uint32_t* w) {
     if constexpr (NW == 4) *(u32x4*)p = (u32x4){w[0], w[1], w[2], w[3]};

@@ -1,8 +1,8 @@
 """Products of more than 128 prompt rows with hi + lo activations (crane_amd/csrc/kernels_gemm_tile.hip): the rule on the host, and on the GPU the same prompt with
 cm_debug_set("gemm256") 1 (these tiles) and 0 (the 128-column kernel).
 
-The tolerance is that of tests/test_gpu_gemm_prompts.py: where K is not split both add the same products in the same order, and SiLU with the hardware's exponential and reciprocal is
-within |g| 2^-24 of expf and a division; where it is split, a sum of K <= 6144 terms moves by about sqrt(K) 2^-24 of its size, and a K or V element lands on the other side of a
+The tolerance is that of tests/test_gpu_gemm_prompts.py: where K is not split both add the same products in the same order and have the same SiLU, so that their rows are equal; where it
+is split, a sum of K <= 6144 terms moves by about sqrt(K) 2^-24 of its size, and a K or V element lands on the other side of a
 16-bit boundary once in a thousand.  2e-3 of the largest logit is ten times what two layers make of that; a tile, a row or a column that is lost or misplaced moves the logits
 by their own size."""
 import numpy as np
@@ -75,5 +75,32 @@ def test_against_the_128_column_kernel(h, i, heads, kv, tokens):
                 rows.append(np.asarray(m.seq_forward(s, ids, 0)[0], np.float64))
                 m.seq_free(s)
             assert np.isfinite(rows[0]).all() and np.abs(rows[0] - rows[1]).max() < TOL * np.abs(rows[1]).max(), n
+    finally:
+        m.close()
+
+
+# whole products in both kernels (no slices of K, no norm in a reduction): the sums have one order and SiLU one rounding, so every bit is the same
+WHOLE = [(2048, 6144, 4096, 0), (2048, 4096, 4096, 1), (2048, 24576, 4096, 0), (2048, 4096, 12288, 1)]
+
+
+def test_the_products_are_whole():
+    assert all(plan(*p)[2] == 1 for p in WHOLE)
+
+
+@pytest.mark.gpu
+def test_the_bits_of_the_128_column_kernel():
+    from crane_amd import configs
+    from crane_amd.backend import Model
+    m = Model.synthetic(dict(configs.get_config("qwen3-8b"), vocab_size=512, num_hidden_layers=2), seed=3, max_seq_len=2048, max_seqs=1)
+    try:
+        for seed in (1, 2):
+            ids = np.random.default_rng(seed).integers(0, 512, 2048).tolist()
+            rows = []
+            for mode in (1, 0):
+                m.debug_set("gemm256", mode)
+                s = m.seq_alloc()
+                rows.append(np.asarray(m.seq_forward(s, ids, 0)[0]).copy())
+                m.seq_free(s)
+            assert np.array_equal(rows[0], rows[1])
     finally:
         m.close()
