@@ -516,6 +516,11 @@ int cm_debug_read(cm_model* h, const char* what, float* out, size_t n) {
         // (the persistent kernel never runs under tensor parallelism and the tower's debug buffers live on rank 0: no '@r' form)
         if (mp != &h->m && (w == "engine_trace" || w.rfind("eng_", 0) == 0 || w == "vision_ms" || w == "deepstack"))
             throw CmError(CM_ERR_INVALID, "cm_debug_read: '" + w + "' has no per-rank form");
+        if (w == "prefill_rows") {         // tokens of several prompts in a pass, rows of a pass over one prompt (fixed with the first prompt)
+            if (n < 2 || !mp->prefill_ready) throw CmError(CM_ERR_INVALID, "prefill_rows: two values, behind the first prompt");
+            out[0] = (float)mp->chunk; out[1] = (float)mp->pass_rows;
+            return;
+        }
         if (w == "engine_trace") { h->m.engine_trace(out, n); return; }
         if (w.rfind("eng_", 0) == 0) {     // value halves of a granule buffer of the persistent kernel (last writer wins)
             static const char* names[cm::ENG_NEDGE] = {"eng_x0", "eng_qkv", "eng_part", "eng_attn", "eng_x1", "eng_h"};
@@ -710,9 +715,11 @@ int cm_debug_set(cm_model* h, const char* key, int64_t value) {
         else if (k == "no_prefill") mm.no_prefill = value != 0;
         else if (k == "quant_prefill") mm.quant_prefill = value != 0;
         else if (k == "prefill_q8") {       // before the first prompt pass of the handle: 0 = prompts over Q8_0-layout weights on the dequantised-to-bf16 GEMMs
-            if (mm.pX != nullptr) throw CmError(CM_ERR_INVALID, "prefill_q8: set before the first prompt pass");
+            if (mm.prefill_ready) throw CmError(CM_ERR_INVALID, "prefill_q8: set before the first prompt pass");
             mm.q8_prefill_want = value != 0;
         }
+        else if (k == "alloc_most") mm.debug_alloc_most = value;
+        else if (k == "free_memory") mm.debug_free = value;
         else if (k == "attn_outq") mm.attn_outq = value != 0;
         else if (k == "prefill_split") mm.prefill_split2 = value < 0 ? mm.default_prefill_split2() : value != 1;   // 1: plain bf16, 0 / 2: hi + lo, -1: back to cm_opts
         // which decode-attention kernel / persistent-kernel mode a step uses (tests and A/B runs; one hipGraph per variant, so

@@ -24,6 +24,7 @@ T* Model::dalloc(size_t n, bool count_weight) {
         if (count_weight) weight_bytes += bytes;
         return (T*)base;
     }
+    if (debug_alloc_most >= 0 && bytes > (size_t)debug_alloc_most) throw CmError(CM_ERR_OOM, "allocation of " + std::to_string(bytes) + " bytes (debug limit)");
     CM_HIP(hipMalloc(&p, bytes));
     // CM_DEBUG_POISON=<byte>[,<first>,<last>]: fill every new allocation (or allocations number first..last of this handle) with
     // the byte -- recycled device memory is not zero, a kernel that reads a buffer before anything wrote it must show up in tests
@@ -1144,100 +1145,117 @@ int Model::prefill_chunk_rows() const {
     return c < 1 ? 1 : c;
 }
 
+// Every buffer of a prompt pass over `rows` rows: f(pointer, elements, cleared)
+template <class F>
+void Model::each_prefill_buffer(int rows_, F&& f) {
+    const size_t H = (size_t)cfg.H, D = (size_t)cfg.D, rows = (size_t)rows_, pad = (rows + 127) / 128 * 128;
+    const size_t qkv_rows = (size_t)(cfg.hybrid ? 2 * Hq_l + 2 * Hkv_l : Hq_l + 2 * Hkv_l) * D, vd = (size_t)(cfg.hybrid ? cfg.value_dim() : 0);
+    const size_t at_cols = std::max((size_t)Hq_l * D, vd);
+    f(pX, rows * H, false);
+    if (rccl) f(pY, rows * H, false);
+    f(pQKV, rows * std::max(qkv_rows, (size_t)in_proj_pad), false);
+    if (cfg.hybrid) {
+        f(pGY, rows * vd, false);
+        f(gdn_pre_q, rows * (size_t)cfg.key_dim(), false);          // three-pass Gated-Delta-Net prefill (kernels_gdn.hip)
+        f(gdn_pre_k, rows * (size_t)cfg.key_dim(), false);
+        f(gdn_pre_v, rows * vd, false);
+        f(gdn_pre_bd, rows * (size_t)cfg.NV * 2, false);
+        f(gdn_pre_g, rows * (size_t)cfg.NV, false);
+        if (cfg.Kd == 128 && cfg.Vd == 128)           // chunk-parallel scan scratch: W | U0 | P | G per (64-token chunk, value head)
+            f(gdn_ck, (rows + GDN_CK - 1) / GDN_CK * (size_t)cfg.NV * GDN_CK_FLOATS, false);
+    }
+    f(pXN_hi, pad * H, true); f(pXN_lo, pad * H, true);
+    f(pQ_hi, pad * (size_t)Hq_l * D, true); f(pQ_lo, pad * (size_t)Hq_l * D, true);
+    f(pAT_hi, pad * at_cols, true); f(pAT_lo, pad * at_cols, true);
+    f(pHH_hi, pad * (size_t)I_l, true); f(pHH_lo, pad * (size_t)I_l, true);
+    if (kvq()) {
+        const size_t shadow = (size_t)max_pages_per_seq * Hkv_l * page * D;
+        f(kshadow, shadow, false); f(vshadow, shadow, false);
+        f(d_ident_bt, (size_t)max_pages_per_seq, false);
+    }
+    if (q8_prefill) {
+        f(pATf, rows * (size_t)Hq_l * D, false);
+        f(pHf, rows * (size_t)I_l, false);                         // silu(gate) * up of the pass, f32 (the down projection's quantiser input)
+        for (LayerW& w : layers)
+            if (!w.full) f(w.ba_pad, 128 * H, true);               // the a / b rows as one zero-padded 128-row GEMM tile
+    }
+    if (quantized && !q8_prefill) {
+        // one dequantised matrix at a time: bf16 hi plane + lo plane (parity mode), and the f32 gate|up sums of the two-pass GEMM
+        wq_scratch_elems = std::max(std::max((size_t)2 * I_l * H, qkv_rows * H), (size_t)in_proj_pad * H);
+        f(wq_scratch, 2 * wq_scratch_elems, false);
+        f(pGU, rows * 2 * (size_t)I_l, false);
+    }
+    f(d_ids, rows, false);
+}
+
 // Rows of one pass over ONE sequence's prompt where the caller left the chunk open: 4096 for hybrid decoders and for dense ones up to 2048 wide, and 128 more where those are the last.  Their
 // projections are 1024 .. 5120 wide: at 2048 rows the tiles of a product fill the chip only with K in slices, whose sums cost a launch and three times the output's bytes; every launch of a pass
 // has a start and an end, and the last rows of a prompt have passes of their own over all weights.  ms, passes of 2048 / so: Qwen3.5-2B 2100 tokens 15.1 / 14.7, 2500 18.0 / 16.8, 4000 25.5 / 23.2, 4165
 // 28.5 / 25.5 (in passes of 4096 26.2), 4500 30.8 / 28.4 (in 4224 30.4); 0.8B 2200 11.3 / 9.8, 3000 13.1 / 11.7, 4165 18.4 / 15.9; 27B 2100 194 / 182, 3000 275 / 246, 4165 379 / 366; dense, Qwen3-0.6B 2100
 // 8.4 / 7.6, 4000 14.7 / 12.1; 28 layers of width 2048 2100 14.7 / 14.3, 4000 25.9 / 22.9.  8B: 2500 57.6 / 57.3, 3000 69.3 / 71.8, 2176 52.4 / 53.5: 2048.  Several prompts in a pass, images and
-// explicit positions keep the chunk as their limit.  Scratch that the card has no room for twice over is not asked for.
+// explicit positions keep the chunk as their limit.  Where the card has not twice the room for all of the longer scratch (what is made later takes its share: groups, images), or turns out not to
+// have it (ensure_prefill_buffers), passes keep the chunk.
 constexpr int PASS_ROWS = 4096, PASS_TAIL = 128;
-int Model::prefill_pass_rows() const {
+int Model::prefill_pass_rows() {
     const int c = prefill_chunk_rows();
     if ((!cfg.hybrid && cfg.H > 2048) || quantized || rccl || opts.prefill_chunk != 0 || max_seq <= c) return c;
     const int rows = std::min<long>(max_seq, PASS_ROWS + PASS_TAIL);
-    const int qkv_rows = (cfg.hybrid ? 2 * Hq_l + 2 * Hkv_l : Hq_l + 2 * Hkv_l) * cfg.D;
-    const size_t per_row = 4 * ((size_t)2 * cfg.H + std::max(qkv_rows, in_proj_pad) + 3 * (size_t)std::max(cfg.value_dim(), Hq_l * cfg.D) + 2 * (size_t)cfg.key_dim() + I_l + 3 * (size_t)cfg.NV +
-                                (size_t)cfg.NV * GDN_CK_FLOATS / GDN_CK);
-    size_t free = 0, total = 0;
-    return hipMemGetInfo(&free, &total) == hipSuccess && (size_t)(rows - c) * per_row * 2 <= free ? rows : c;
+    size_t need = 0, free = 0, total = 0;
+    each_prefill_buffer(rows, [&](auto*& p, size_t n, bool) { need += n * sizeof(*p); });
+    if (hipMemGetInfo(&free, &total) != hipSuccess) { (void)hipGetLastError(); return c; }
+    if (debug_free >= 0) free = (size_t)debug_free;
+    return need <= free / 2 ? rows : c;
 }
 
+// All buffers or none: what a failed allocation leaves behind is given back, and the next prompt asks again
 void Model::ensure_prefill_buffers() {
-    if (pX || layered) return;
+    if (prefill_ready || layered) return;
     const int H = cfg.H, D = cfg.D;
     chunk = prefill_chunk_rows();
-    pass_rows = prefill_pass_rows();
-    const int rows = pass_rows, rows_pad = (rows + 127) / 128 * 128;
     // prompt activations as bf16 hi + lo (two products per GEMM: what the 1e-3 bound of a bf16 checkpoint needs) unless the caller asked
     // for plain bf16 -- or left the choice open (0) on QUANTISED weights: their scratch copy for the GEMMs is already rounded to bf16
     // (2^-9 per weight, tests: 1e-2 of the oracle on the dequantised weights), the activations' low halves would refine past that
     prefill_split2 = default_prefill_split2();
     const int qkv_rows = (cfg.hybrid ? 2 * Hq_l + 2 * Hkv_l : Hq_l + 2 * Hkv_l) * D;
-    prefill_ok = (qkv_rows % 128 == 0) && (H % 128 == 0) && ((2 * I_l) % 128 == 0) && (H % 32 == 0) && (I_l % 32 == 0) &&
-                 (!cfg.hybrid || cfg.value_dim() % 32 == 0);
-    if (!prefill_ok) return;
-    pX = dalloc<float>((size_t)rows * H);
+    if (!((qkv_rows % 128 == 0) && (H % 128 == 0) && ((2 * I_l) % 128 == 0) && (H % 32 == 0) && (I_l % 32 == 0) &&
+          (!cfg.hybrid || cfg.value_dim() % 32 == 0))) return;
     ensure_gemm_workspace();
-    if (rccl) pY = dalloc<float>((size_t)rows * H);
-    pQKV = dalloc<float>((size_t)rows * std::max(qkv_rows, in_proj_pad));
-    if (cfg.hybrid) {
-        pGY = dalloc<float>((size_t)rows * cfg.value_dim());
-        gdn_pre_q = dalloc<float>((size_t)rows * cfg.key_dim());      // three-pass Gated-Delta-Net prefill (kernels_gdn.hip)
-        gdn_pre_k = dalloc<float>((size_t)rows * cfg.key_dim());
-        gdn_pre_v = dalloc<float>((size_t)rows * cfg.value_dim());
-        gdn_pre_bd = dalloc<float>((size_t)rows * cfg.NV * 2);
-        gdn_pre_g = dalloc<float>((size_t)rows * cfg.NV);
-        if (cfg.Kd == 128 && cfg.Vd == 128)           // chunk-parallel scan scratch: W | U0 | P | G per (64-token chunk, value head)
-            gdn_ck = dalloc<float>((size_t)((rows + GDN_CK - 1) / GDN_CK) * cfg.NV * GDN_CK_FLOATS);
-    }
-    auto z = [&](size_t n) {
-        uint16_t* p = dalloc<uint16_t>(n);
-        CM_HIP(hipMemsetAsync(p, 0, n * sizeof(uint16_t), stream));
-        return p;
-    };
-    pXN_hi = z((size_t)rows_pad * H); pXN_lo = z((size_t)rows_pad * H);
-    pQ_hi = z((size_t)rows_pad * Hq_l * D); pQ_lo = z((size_t)rows_pad * Hq_l * D);
-    const size_t at_cols = std::max((size_t)Hq_l * D, (size_t)(cfg.hybrid ? cfg.value_dim() : 0));
-    pAT_hi = z((size_t)rows_pad * at_cols); pAT_lo = z((size_t)rows_pad * at_cols);
-    pHH_hi = z((size_t)rows_pad * I_l); pHH_lo = z((size_t)rows_pad * I_l);
-    if (kvq()) {
-        const size_t shadow = (size_t)max_pages_per_seq * Hkv_l * page * D;
-        kshadow = dalloc<float>(shadow);
-        vshadow = dalloc<float>(shadow);
-        std::vector<int32_t> ident((size_t)max_pages_per_seq);
-        for (int i = 0; i < max_pages_per_seq; ++i) ident[(size_t)i] = i;
-        d_ident_bt = dalloc<int>((size_t)max_pages_per_seq);
-        CM_HIP(hipMemcpy(d_ident_bt, ident.data(), ident.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    }
     // Q8_0-layout weights (GGUF Q8_0 / Q4_0 / Q5_0, every ISQ mode), integer-dot activation mode: the prompt's projections run on the
     // int8 matrix cores in panels of <= 128 rows (prefill_layers) -- the arithmetic of the decode step and of candle's CPU QMatMul
     // (ops/linear.rs:18-51: activation row -> Q8_0 blocks, ggml_vec_dot_q8_0_q8_0 per output), no dequantised copy of any matrix
     q8_prefill = q8_prefill_want && q8_prefill_eligible();
-    if (q8_prefill) {
-        ensure_batch_buffers();                                    // qx_codes / qx_scales pairs (sized for a whole pass there)
-        pATf = dalloc<float>((size_t)rows * Hq_l * D);
-        pHf = dalloc<float>((size_t)rows * I_l);                  // silu(gate) * up of the pass, f32 (the down projection's quantiser input)
-        for (LayerW& w : layers) {
-            if (w.full) continue;
-            w.ba_pad = dalloc<uint16_t>((size_t)128 * H);          // the a / b rows as one zero-padded 128-row GEMM tile
-            CM_HIP(hipMemsetAsync(w.ba_pad, 0, (size_t)128 * H * sizeof(uint16_t), stream));
-            CM_HIP(hipMemcpyAsync(w.ba_pad, w.in_proj_ba, (size_t)2 * cfg.NV * H * sizeof(uint16_t), hipMemcpyDeviceToDevice, stream));
+    if (q8_prefill) ensure_batch_buffers();                        // qx_codes / qx_scales pairs (sized for a whole pass there)
+    for (int rows = prefill_pass_rows();; rows = chunk) {
+        try {
+            each_prefill_buffer(rows, [&](auto*& p, size_t n, bool cleared) {
+                p = dalloc<std::remove_reference_t<decltype(*p)>>(n);
+                if (cleared) CM_HIP(hipMemsetAsync(p, 0, n * sizeof(*p), stream));
+            });
+            CM_HIP(hipHostMalloc((void**)&h_ids, (size_t)rows * sizeof(uint32_t)));
+            pass_rows = rows;
+            break;
+        } catch (const CmError& e) {
+            (void)hipGetLastError();
+            each_prefill_buffer(rows, [&](auto*& p, size_t, bool) { dfree((void*)p); p = nullptr; });
+            if (e.code != CM_ERR_OOM || rows == chunk) throw;
         }
     }
-    if (quantized && !q8_prefill) {
-        // one dequantised matrix at a time: bf16 hi plane + lo plane (parity mode), and the f32 gate|up sums of the two-pass GEMM
-        wq_scratch_elems = std::max(std::max((size_t)2 * I_l * H, (size_t)qkv_rows * H), (size_t)in_proj_pad * H);
-        wq_scratch = dalloc<uint16_t>(2 * wq_scratch_elems);
-        pGU = dalloc<float>((size_t)rows * 2 * I_l);
-        // CM_QUANT_PREFILL_CACHE=1 (opt-in): keep every
-        // dequantised matrix (hi + lo: 4 bytes per weight -- more than the bf16 checkpoint) instead of dequantising it again per pass
-        // (4.5 % of a Q8_0 serving run, before Q8_0-layout models moved to the int8 prompt pass).  An allocation that fails mid-pass
-        // falls back to the scratch (deq_w)
-        wq_cache = false;
-        if (const char* e = getenv("CM_QUANT_PREFILL_CACHE")) wq_cache = atoi(e) != 0;
+    if (kvq()) {
+        std::vector<int32_t> ident((size_t)max_pages_per_seq);
+        for (int i = 0; i < max_pages_per_seq; ++i) ident[(size_t)i] = i;
+        CM_HIP(hipMemcpy(d_ident_bt, ident.data(), ident.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     }
-    d_ids = (uint32_t*)dalloc<int>(rows);
-    CM_HIP(hipHostMalloc((void**)&h_ids, (size_t)rows * sizeof(uint32_t)));
+    if (q8_prefill)
+        for (LayerW& w : layers)
+            if (!w.full) CM_HIP(hipMemcpyAsync(w.ba_pad, w.in_proj_ba, (size_t)2 * cfg.NV * H * sizeof(uint16_t), hipMemcpyDeviceToDevice, stream));
+    // CM_QUANT_PREFILL_CACHE=1 (opt-in): keep every
+    // dequantised matrix (hi + lo: 4 bytes per weight -- more than the bf16 checkpoint) instead of dequantising it again per pass
+    // (4.5 % of a Q8_0 serving run, before Q8_0-layout models moved to the int8 prompt pass).  An allocation that fails mid-pass
+    // falls back to the scratch (deq_w)
+    wq_cache = false;
+    if (quantized && !q8_prefill)
+        if (const char* e = getenv("CM_QUANT_PREFILL_CACHE")) wq_cache = atoi(e) != 0;
+    prefill_ok = prefill_ready = true;
 }
 
 // the decoder layers over the S rows of pX.  The row-wise work (norms, every GEMM) runs once over all rows; what mixes tokens --
@@ -1787,8 +1805,22 @@ void Model::lm_head_rows(int nb, bool want_rows) {
 // batched decode step: step_batch_decode (backend.rs:107-121, qwen3/modeling.rs:1202-1234) without padding,
 // masks or KV copies -- up to MAXB sequences share ONE pass over the weights
 // ------------------------------------------------------------------------------------
+// all buffers or none, as for prompts
 void Model::ensure_batch_buffers() {
     if (stb || layered) return;
+    const size_t mark = allocs.size();
+    try {
+        make_batch_buffers();
+    } catch (...) {
+        (void)hipGetLastError();
+        while (allocs.size() > mark) dfree(allocs.back());
+        if (h_stb) (void)hipHostFree(h_stb);
+        if (h_btb) (void)hipHostFree(h_btb);
+        stb = nullptr; h_stb = nullptr; h_btb = nullptr;       // (the others are made again before anyone looks at them)
+        throw;
+    }
+}
+void Model::make_batch_buffers() {
     const int H = cfg.H, D = cfg.D;
     const size_t attn_rows = (size_t)(cfg.hybrid ? 2 * Hq_l + 2 * Hkv_l : Hq_l + 2 * Hkv_l) * D;
     ldq = (int)std::max(attn_rows, (size_t)in_proj_pad);

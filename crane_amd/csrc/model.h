@@ -238,7 +238,8 @@ struct Model {
 
     // prefill scratch (allocated on first use; sized for pass_rows)
     int chunk = 2048;           // tokens of several prompts in a pass, of a prompt with images
-    int pass_rows = 2048;       // rows of a pass over one prompt: the chunk or more (prefill_pass_rows)
+    int pass_rows = 2048;       // rows of a pass over one prompt: the chunk or more (prefill_pass_rows), fixed with the first prompt
+    bool prefill_ready = false;          // every buffer is there (set last)
     bool prefill_ok = false, prefill_split2 = true;
     int gemm256 = 1;           // prompt-pass / decode-group GEMMs: 0 = never an LDS-DMA kernel, 1 = automatic, 2 = always kernels_gemmw4.hip, 3 = kernels_gemm256.hip only (cm_debug_set("gemm256"))
     float* pX = nullptr;        // [pass_rows, H] f32 residual stream
@@ -281,6 +282,7 @@ struct Model {
     int* pidxb = nullptr;
     int ldq = 0;
     void ensure_batch_buffers();
+    void make_batch_buffers();
     // after_group(g0, nb): called once per <= MAXB group after the stream is idle; logitsb[b * V] (b < nb) is valid
     void decode_batch(const int32_t* sq, const uint32_t* toks, size_t n, float* logits_out, uint32_t* greedy_out,
                       const std::function<void(size_t, int)>* after_group = nullptr);
@@ -327,7 +329,9 @@ struct Model {
     float* pHf = nullptr;              // [pass_rows][I_l] f32 silu(gate) * up rows of the pass
     int q8_xs = QGEMM_MAXM;            // floats between the scale rows of the code buffers in a prompt pass of more than 128 rows
     int prefill_chunk_rows() const;
-    int prefill_pass_rows() const;
+    int prefill_pass_rows();
+    template <class F> void each_prefill_buffer(int rows, F&& f);
+    long long debug_alloc_most = -1, debug_free = -1;      // cm_debug_set: an allocation of more bytes fails, what prefill_pass_rows takes for the card's free memory (-1: as it is)
     bool q8_prefill_eligible() const;
     uint16_t* wq_scratch = nullptr;    // [2][max N*K] bf16 hi | lo planes: one dequantised matrix at a time for the prefill GEMMs
     size_t wq_scratch_elems = 0;

@@ -493,7 +493,8 @@ int cm_bench_kernel(cm_model* m, const char* which, size_t iters, float* ms_out,
 int cm_debug_fill_kv(cm_model* m, size_t ctx, uint64_t seed);
 
 /* Copy an internal device buffer to host for kernel-level parity tests.
- * what: "hidden" (f32 [H] residual after the last forward), "logits". */
+ * what: "hidden" (f32 [H] residual after the last forward), "logits"; "prefill_rows" (behind the first prompt: tokens of several prompts in a pass,
+ * rows of a pass over one prompt). */
 int cm_debug_read(cm_model* m, const char* what, float* out, size_t n);
 
 /* Run ONE quantised projection of `layer` on a host vector: y = W_q . x (plain prologue, store epilogue), in the
@@ -585,7 +586,9 @@ int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32
  * decode hipGraph (CM_TP_GRAPH); "prefill_seg_batch" = 0 / 1: cm_prefill_batch launches RoPE / KV append / attention once per
  * sequence / once for all sequences of the pass; "gdn_defer_norm" = 0 / 1: the Gated-Delta-Net step normalises itself / leaves the
  * gated RMSNorm to out_proj's prologue; "prefill_lo_mask" (measurement only, tools/lo_mask_probe.py): bit 0 QKV, 1 o_proj, 2 gate||up,
- * 3 down_proj -- that GEMM of the prompt pass drops the lo plane of its activations.
+ * 3 down_proj -- that GEMM of the prompt pass drops the lo plane of its activations;
+ * "alloc_most" = n: a device allocation of more than n bytes fails as if the card were full (-1: none does); "free_memory" = n: what the choice of a
+ * pass's rows takes for the card's free bytes (-1: the card's).
  * cm_debug_read("engine_trace") launches the persistent kernel several times on the live state of sequence 0: the K/V rows at
  * the current position and the residual stream are overwritten -- clear the sequence afterwards. */
 int cm_debug_set(cm_model* m, const char* key, int64_t value);
