@@ -1331,53 +1331,45 @@ static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {
     if (a.bias != nullptr) rest.bias = a.bias + most.N;
     return launch_gemm_once(rest, epi, s);
 }
-// What M rows of a product with hi + lo activations take, in seconds.  On tiles of 128 rows (tall: on those of kernels_gemm_tile.hip by their own figures): rounds of blocks, a 64-deep
-// k-tile of 128 x 256 outputs 1.44 us and about 13 us a block around them (measured / so: 24576 x 4096 at 300, 650, 1000, 1400 rows 164 / 164, 248 / 246, 313 / 315, 502 / 493 us); two blocks
-// of 128 x 128 on a CU 1.6 and 10; products of at most 128 rows by their weights
-static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap, bool tall) {
-    int bn = 0, ks = 0;
+// What M rows of a product with hi + lo activations take on the kernel that launch_gemm_once finds for them, in seconds: the tiles of kernels_gemm_tile.hip by their own figures; two blocks of
+// 128 x 128 on a CU 1.6 us per 64-deep k-tile and 10 around them; one row tile of gemm256_kernel 1.44 us at 256 columns and 13; products of at most 128 rows by their weights, which the rows in
+// front of them have just read (118 launches of 9 .. 128 rows over the widths of the 8B and 2B models: 5 % off in the mean square)
+static double gemm_seconds(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
+    int bm = 0, bn = 0, ks = 0;
     const auto split = [&](int cols) { return ks > 1 ? (double)(2 * ks + 1) * M * cols * 4.0 / 5e12 + 4e-6 : 0.0; };
-    if (epi != GEPI_ACT_SPLIT && gemm_rows_plan(M, N, K, ws_floats, &bn, &ks)) {
-        const int blocks = N / bn * ks;
-        return (double)N * K * 2.0 / (M <= 64 ? 4.6e12 : 3.4e12) * ((blocks + 255) / 256 * 256) / blocks + (ks > 1 ? 9e-6 : 4e-6);
-    }
+    if (epi != GEPI_ACT_SPLIT && gemm_rows_plan(M, N, K, ws_floats, &bn, &ks)) return 4.3e-6 + M * 62e-9 + (double)N * K * 2.0 / (M <= 64 ? 5.9e12 : 4.2e12);
     const int tiles_m = (M + 127) / 128;
     const bool tail = epi == GEPI_STORE && gemm_tail_columns(M, N);
     const int cols = N - (tail ? 128 : 0);
-    int bm = 0;
     double best = 0.0;
-    if (tall && gemm_tile_plan(M, cols, K, ws_floats, epi == GEPI_RESADD, &bm, &bn, &ks, &best)) return best + (tail ? 15e-6 : 0.0);
-    if ((!tall || M <= 128) && gemm256_plan(M, cols, K, true, ws_floats, false, &bn, &ks))
-        return (tiles_m * (cols / bn) * ks + 255) / 256 * (K / 64 / ks * 1.44e-6 * bn / 256 + 13e-6) + split(cols) + (tail ? 15e-6 : 0.0);
+    if (gemm_tile_plan(M, cols, K, ws_floats, epi == GEPI_RESADD, &bm, &bn, &ks, &best)) return best + (tail ? 15e-6 : 0.0);
+    if (M <= 128 && gemm256_plan(M, cols, K, true, ws_floats, false, &bn, &ks))
+        return (tiles_m * (cols / bn) * ks + 255) / 256 * (K / 64 / ks * 1.44e-6 * bn / 256 + 13e-6) + split(cols);
     ks = gemm_ksplit(M, N, tiles_m * (N / 128), K / GBK, ws_floats, ksplit_cap);
     return (tiles_m * (N / 128) * ks + 511) / 512 * (K / 64 / ks * 1.6e-6 + 10e-6) + split(N);
 }
-// the rows of the first of two bands that take less time than all rows at once on tiles of 128; 0: all at once
+// the rows of the first of two bands that take less time than all rows at once; 0: all at once
 int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
     if (M <= 256 || N % 128 != 0 || K % 64 != 0 || epi == GEPI_ACT_SPLIT) return 0;
-    const double whole = gemm_seconds(M, N, K, epi, ws_floats, ksplit_cap, false);
+    const double whole = gemm_seconds(M, N, K, epi, ws_floats, ksplit_cap);
     double least = std::min(0.95 * whole, whole - 8e-6);
     int rows = 0;
     for (int m = (M - 9) / 128 * 128; m >= 128 && M - m <= 1024; m -= 128) {
-        const double t = gemm_seconds(m, N, K, epi, ws_floats, ksplit_cap, false) + gemm_seconds(M - m, N, K, epi, ws_floats, ksplit_cap, false) + 2e-6;
+        const double t = gemm_seconds(m, N, K, epi, ws_floats, ksplit_cap) + gemm_seconds(M - m, N, K, epi, ws_floats, ksplit_cap) + 2e-6;
         if (t < least) { least = t; rows = m; }
     }
     return rows;
 }
 // A round of blocks that the last tiles fill to a part takes as long as a full one: a band of rows whose tiles fill their rounds first, the rows behind it on
-// the kernel that suits so few.  What bounds either band is what bounded the whole; the second reads the weights again (24576 x 4096: 44 us of the memory's time
-// against a round of 105).  One launch / two, prompts on width 4096 with 36 layers: 300 tokens 12.8 / 11.8 ms, 520 20.0 / 18.2, 1200 38.1 / 33.6, 1400 44.2 / 37.6;
-// width 2048, 650: 7.5 / 7.1.  The line is a gain of 5 % and 8 us by the figures above: with 5 % alone the products of width 1024 lost (300 tokens 3.32 / 3.45
-// ms, 560 4.30 / 4.41: a launch and a reduction more for a round of 30 us).  Rows of products with an activation behind them and the vision tower's norm stay in one launch (not measured).
+// the kernel that suits so few.  What bounds either band is what bounded the whole; the second reads the weights again.  One launch / two, us of prompts through eight layers: width 4096, 645 tokens
+// 4525 / 4388 (gate and up 512 + 133), 768 4726 / 4521, 1040 6877 / 5918 (1024 + 16 in three products), 1152 7053 / 6478, 1400 7814 / 7608 (down 384 + 1016); width 2048 with Gated-Delta-Net layers,
+// 1290 3546 / 3378, 2060 5427 / 4848, 2304 5718 / 5475, 4165 9739 / 8647.  The line is a gain of 5 % and 8 us by the figures above, which are 5 % off: a band by less of a gain was as often a loss (width
+// 5120, 2000 tokens 10.83 / 11.03 ms), and 5 % alone lost in the products of width 1024, a launch and a reduction more for a round of 30 us.  Rows of products with an activation behind them and the
+// vision tower's norm stay in one launch (not measured).
 static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
     if (a.A_lo == nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
-    const size_t ws = a.ws ? a.ws_floats : 0;
-    const int m = gemm_band(a.M, a.N, a.K, epi, ws, a.ksplit_cap);
+    const int m = gemm_band(a.M, a.N, a.K, epi, a.ws ? a.ws_floats : 0, a.ksplit_cap);
     if (m == 0) return false;
-    // larger tiles and wider ones leave fewer rounds nearly empty: 300 rows of 24576 x 4096 123 us in one launch, 44 more for 44 rows behind 256
-    const double whole = gemm_seconds(a.M, a.N, a.K, epi, ws, a.ksplit_cap, true);
-    const double two = gemm_seconds(m, a.N, a.K, epi, ws, a.ksplit_cap, true) + gemm_seconds(a.M - m, a.N, a.K, epi, ws, a.ksplit_cap, true) + 2e-6;
-    if (two >= std::min(0.95 * whole, whole - 8e-6)) return false;
     const size_t hcols = epi == GEPI_SILUMUL ? (size_t)a.N / 2 : (size_t)a.N;
     for (int part = 0; part < 2; ++part) {
         const size_t r0 = part ? (size_t)m : 0;
