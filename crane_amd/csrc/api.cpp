@@ -644,6 +644,11 @@ int cm_debug_gdn_step(const float* proj, const float* conv_w, const float* state
     });
 }
 
+int cm_debug_attn_prompt_pairs(int32_t rows, int32_t start, int32_t heads, int32_t kv_heads) {
+    if (rows < 1 || start < 0 || heads < 1 || kv_heads < 1) return 0;
+    return cm::attn_prefill_shares(rows, start, heads, 128) == 1 && cm::attn_prompt_pairs(rows, start, heads, heads / kv_heads);
+}
+
 int cm_debug_attn_group_plan(int32_t pairs, int32_t nrep, int64_t longest, int32_t slices, int32_t num_cu, int32_t most) {
     return cm::attn_decode_group_pays(pairs, nrep, longest, slices != 0, num_cu) ? cm::attn_decode_group_split(longest, pairs, num_cu, most) : 0;
 }

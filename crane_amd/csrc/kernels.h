@@ -222,6 +222,8 @@ struct AttnPreArgs {
     const PrefillSegDev* segs = nullptr;
     const int2* tiles = nullptr;
     int ntiles = 0;
+    long long walks = 0;         // their key tiles of 64 together and at most
+    int longest = 0;
     // few queries behind many keys (one sequence): scratch that launch_attn_prefill may share the keys of a query tile among blocks with: nsplit shares of
     // [S][Hq][D] sums and [S][Hq][2] maxima and denominators
     float* ws = nullptr;
@@ -244,6 +246,7 @@ int gemm256_rows(bool split, int M);       // rows of that kernel's tile for an 
 bool launch_gemm256(const GemmArgs& a, int epi, int bn, hipStream_t s);   // kernels_gemm256.hip; a.ksplit set by the caller (launch_gemm)
 int gemmw4_rows(bool split);               // rows of the one-wave-per-SIMD kernel's tile (kernels_gemmw4.hip): 128 with hi + lo activations, 256 plain
 bool launch_gemmw4(const GemmArgs& a, int epi, int bn, hipStream_t s);    // same contract as launch_gemm256
+bool attn_prompt_pairs(int rows, int start, int heads, int nrep);    // whether one prompt's query tiles whose keys nobody shares are launch_attn_prompt_pair's
 int attn_prefill_shares(int rows, int start, int heads, int D);      // blocks that share the keys of a query tile, scratch permitting
 void launch_attn_prompt_pair(const AttnPreArgs& a, int kvt, hipStream_t s);      // kernels_attn_prompt.hip: head_dim 128, an even number of query heads per key head, keys not shared
 void launch_attn_prompt_wide(const AttnPreArgs& a, int kvt, hipStream_t s);      // head_dim 256; a.nsplit shares of the keys

@@ -5,8 +5,8 @@
 // waves of the SIMD hide.  That kernel holds two tiles in 64 registers on their way to the LDS and 69 KB of LDS for four waves, so two waves share a SIMD; here rows go from memory into
 // the LDS directly, eight waves share 64 KB of it and stay within 128 registers, so four do, and the sums are scaled only when a maximum in the wave has moved.  The order of
 // every sum is that kernel's.
-// Measured (us a launch, that kernel / here, 32 heads on 8): 2048 rows 114 / 85, behind 2048 tokens 269 / 188; 1400 rows 65 / 63, 192 / 165; with at most two of its workgroups on every
-// CU that kernel is ahead: 1000 rows 35 / 39, 500 18.6 / 22.7; 16 heads, 2048 rows 60 / 70.
+// Measured (us a launch, that kernel / here, 32 heads on 8): 2048 rows 114 / 85, behind 2048 tokens 269 / 188; 1400 rows behind 2048 tokens 192 / 165; where that kernel's places fill again as the short walks end it
+// is ahead: 1000 rows 35 / 39, 16 heads 2048 rows 60 / 70.  The line stands beside launch_prefill_fast.
 // Two heads in every wave (its fragments shared, two chains, 250 registers): 99 / 191 us in the place of 85 / 188; matrix and vector instructions of the two put side by side by hand: 98 / 195;
 // the waves 4-7 half a tile behind the others (174 registers): 120 / 260.
 //

@@ -1453,13 +1453,26 @@ static int prefill_split(const AttnPreArgs& a, int D) {
     while (n > 1 && (size_t)n * a.S * a.Hq * (D + 2) > a.ws_floats) --n;
     return n;
 }
+// Which of the two head_dim-128 kernels takes query tiles whose walks are `walks` key tiles together (of one head) and `longest` at most.  attn_prefill_fast_kernel has 512 places; a launch of
+// more tiles fills them again as the short ones end, so that what it takes is its longest walk until the work is more than about seven tenths of 512 of those: there attn_prompt_pair_kernel, with all
+// its waves at once, is ahead.  us a layer, that kernel - this one: from the start of a prompt 16 heads 512 / 672 / 704 / 768 / 832 / 1024 tiles (0.52 / 0.67 / 0.70 / 0.77 / 0.83 / 1.02 of 512) -13 /
+// -12 / 0 / +4 / +25 / +30, 32 heads 544 / 672 (0.69) / 704 (0.72) / 896 / 1024 -7 / -6 / +4 / +13 / +22, 24 heads 672 (0.68) / 720 (0.73) -6 / +8, 64 heads 640 (0.69) / 704 (0.75) -2 / +4, 8 heads 528 (0.53) -28; behind 512 tokens 16 heads
+// 560 .. 608 (0.64 .. 0.70) -4 .. -1, 640 (0.74) 0, 32 heads 544 .. 608 (0.72 .. 0.78) -2 .. -1; behind 1024 16 heads 528 (0.69) +2, 576 (0.75) +5; behind 2048 16 heads 512 / 528 / 560 (0.76 / 0.78 / 0.82)
+// -13 / +16 / +11, 32 heads 544 (0.88) +12 .. +16; several prompts of 32 heads 1200 and eight of 64 (0.65) -5, 1300 and 200 (0.72) -5 .. -1, 700 twice (0.75) +1, 300 six times (1.12) +2
+static bool attn_pairs(int heads, int nrep, int tiles, long long walks, int longest) { return nrep % 2 == 0 && heads * tiles > 512 && heads * walks * 10 > 512LL * 7 * longest; }
+bool attn_prompt_pairs(int rows, int start, int heads, int nrep) {
+    const int tiles = (rows + 63) / 64;
+    long long walks = 0;
+    int longest = 0;
+    for (int i = 0; i < tiles; ++i) walks += longest = (start + std::min(64 * (i + 1), rows) + 63) / 64;
+    return attn_pairs(heads, nrep, tiles, walks, longest);
+}
 // causal prompts over 2-byte pages
 static void launch_prefill_fast(AttnPreArgs a, int D, int kvt, hipStream_t s) {
     a.nsplit = prefill_split(a, D);
     const dim3 grid(a.Hq, a.tiles != nullptr ? a.ntiles : (a.S + 63) / 64, a.nsplit);
-    // head_dim 128, more than two workgroups on every CU: half as many with twice the waves (figures beside these kernels)
     if (D == 256) launch_attn_prompt_wide(a, kvt, s);
-    else if (a.nrep % 2 == 0 && a.nsplit == 1 && grid.x * grid.y > 512) launch_attn_prompt_pair(a, kvt, s);
+    else if (a.nsplit == 1 && (a.tiles != nullptr ? attn_pairs(a.Hq, a.nrep, a.ntiles, a.walks, a.longest) : attn_prompt_pairs(a.S, a.start_pos, a.Hq, a.nrep))) launch_attn_prompt_pair(a, kvt, s);
     else if (kvt == KV_F16) hipLaunchKernelGGL((attn_prefill_fast_kernel<KV_F16>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((attn_prefill_fast_kernel<KV_BF16>), grid, dim3(256), 0, s, a);
     if (a.nsplit == 1) return;

@@ -1461,7 +1461,7 @@ void Model::prefill_layers(int S, const PrefillSeg* segs, int nseg, size_t off) 
             at.S = S; at.Hq = Hq_l; at.Hkv = Hkv_l; at.nrep = nrep;
             at.page = page; at.start_pos = 0;
             at.gate = cfg.hybrid ? pQKV + (size_t)Hq_l * D : nullptr; at.gate_stride = qkv_rows;
-            at.segs = d_segtab; at.tiles = d_tiles; at.ntiles = seg_ntiles;
+            at.segs = d_segtab; at.tiles = d_tiles; at.ntiles = seg_ntiles; at.walks = seg_walks; at.longest = seg_longest;
             if (q8p) at.out_f32 = pATf;
             launch_attn_prefill(at, D, kv_f32 ? KV_F32 : kv_mode, s);
         } else
@@ -1606,6 +1606,8 @@ void Model::prefill_multi(const int32_t* sq, const uint32_t* const* ids, const s
         }
         std::stable_sort(tl.begin(), tl.end(), [](const int2& x, const int2& y) { return x.y < y.y; });     // start_pos = 0: key tiles = qt + 1
         seg_ntiles = (int)tl.size();
+        seg_walks = 0;
+        for (const int2& t : tl) seg_walks += seg_longest = t.y + 1;                                                                      // (ascending)
         CM_HIP(hipMemcpy(d_segtab, hs.data(), hs.size() * sizeof(PrefillSegDev), hipMemcpyHostToDevice));
         CM_HIP(hipMemcpy(d_rowseg, rs.data(), rs.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         CM_HIP(hipMemcpy(d_tiles, tl.data(), tl.size() * sizeof(int2), hipMemcpyHostToDevice));

@@ -368,7 +368,8 @@ struct Model {
     PrefillSegDev* d_segtab = nullptr;
     int32_t* d_rowseg = nullptr;
     int2* d_tiles = nullptr;
-    int seg_ntiles = 0;
+    int seg_ntiles = 0, seg_longest = 0;
+    long long seg_walks = 0;
     bool seg_batch = true, seg_tables_ok = false;
     int eng_chunk = 2048;      // dependency chunk of the persistent kernel (2048; 1024 for widths that are only multiples of 1024)
     bool hybrid_engine = false; // CM_ENGINE_HYBRID=1 (or cm_opts.engine = 1): per-layer persistent chain for the hybrid family -- measured slower, opt-in

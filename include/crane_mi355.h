@@ -553,6 +553,10 @@ int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws
 /* Test hook (host logic only, no GPU): rows * 10000 + columns * 10 + K slices of the tiles that m prompt rows of such a product run on (norm: one of the rows behind it); 0: another kernel. */
 int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats);
 
+/* Test hook (host logic only, no GPU): whether `rows` queries of a prompt behind `start` cached tokens, `heads` query heads of 128 on `kv_heads`, take the attention of two heads per workgroup
+ * (csrc/kernels_attn_prompt.hip): 1, or the kernel of one: 0. */
+int cm_debug_attn_prompt_pairs(int32_t rows, int32_t start, int32_t heads, int32_t kv_heads);
+
 /* Test hook: the keys and values that the rotation of prompts (head_dim 128, no norm) appends to 32-bit pages: rows [slices][n][2 kv_heads][128], cos and sin [n][64];
  * out [2 (keys, values)][kv_heads][n][128]. */
 int cm_debug_rope_rows(const float* rows, int32_t n, int32_t kv_heads, int32_t slices, const float* cos, const float* sin, float* out);

@@ -6,9 +6,7 @@ travel as bfloat16 hi + lo planes, 2^-17 of an element where the two land on bot
 import numpy as np
 import pytest
 
-from crane_amd import configs
-
-pytestmark = pytest.mark.gpu
+from crane_amd import _lib, configs
 
 TOL = 2e-5
 
@@ -26,22 +24,41 @@ def _last(m, ids):
     return row
 
 
-# a query tile of one row behind whole ones, whole tiles only, a ragged one; two, four and eight query heads per key head; pages of one tile and of two; both page types; a second pass behind 2048 rows
-@pytest.mark.parametrize("heads,kv,page,dtype,tokens", [(32, 8, 64, "f16", (1025, 1088, 2048, 2300)), (32, 16, 128, "bf16", (1087, 1500)), (32, 4, 128, "f16", (1100,)), (40, 20, 64, "bf16", (833, 900))])
+# whole query tiles, one of one row behind them, a ragged one; two, four and eight query heads per key head; pages of one tile and of two; both page types; a second pass behind 1152 rows
+CASES = [(32, 8, 64, "f16", (1345, 1408, 2048, 2300)), (32, 16, 128, "bf16", (1407, 1500)), (32, 4, 128, "f16", (1409,)), (40, 20, 64, "bf16", (1025, 1088))]
+
+
+def test_the_cases_reach_the_kernel():
+    pairs = _lib.load().cm_debug_attn_prompt_pairs
+    assert all(pairs(min(n, 2048), 0, heads, kv) for heads, kv, _, _, tokens in CASES for n in tokens) and pairs(1148, 1152, 32, 8)
+    assert not any(pairs(n, 0, heads, kv) for heads, kv, chunk in ((32, 8, 512), (32, 16, 512), (32, 4, 512), (40, 20, 384)) for n in range(1, chunk + 1))
+
+
+# both sides of the line (figures beside the rule): prompts from their start, behind cached tokens, an odd number of query heads per key head
+@pytest.mark.parametrize("rows,start,heads,kv,want", [(2048, 0, 16, 8, 0), (2688, 0, 16, 8, 0), (2816, 0, 16, 8, 1), (1344, 0, 32, 8, 0), (1408, 0, 32, 8, 1), (1792, 0, 24, 4, 0), (1920, 0, 24, 4, 1),
+                                                      (4224, 0, 8, 4, 0), (2048, 2048, 16, 8, 0), (2240, 2048, 16, 8, 1), (1088, 2048, 32, 8, 1), (2048, 0, 32, 32, 0), (2048, 2048, 24, 8, 0)])
+def test_the_faster_kernel(rows, start, heads, kv, want):
+    assert _lib.load().cm_debug_attn_prompt_pairs(rows, start, heads, kv) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,page,dtype,tokens", CASES)
 def test_against_portions(heads, kv, page, dtype, tokens):
     ids = np.random.default_rng(heads + kv).integers(0, 512, 2300).tolist()
     rows = []
-    for chunk in (2048, 512 if heads == 32 else 384):
+    for chunk in (2048, 1152, 512) if 2300 in tokens else (2048, 512 if heads == 32 else 384):
         m = _model(heads, kv, chunk, page, dtype)
         try:
             rows.append([_last(m, ids[:n]) for n in tokens])
         finally:
             m.close()
-    for a, b in zip(*rows):
-        assert np.isfinite(a).all() and np.abs(a - b).max() < TOL * np.abs(b).max()
+    for got in rows[:-1]:
+        for a, b in zip(got, rows[-1]):
+            assert np.isfinite(a).all() and np.abs(a - b).max() < TOL * np.abs(b).max()
 
 
 # several sequences in one launch: tiles of every length, sequences of one row and of a tile and one; few rows, whose projection is split and added up by the rotation
+@pytest.mark.gpu
 @pytest.mark.parametrize("lengths", [(1, 65, 700, 64, 310, 900), (3, 40, 17, 60), (9, 1), (150, 120, 30)])
 def test_several_prompts(lengths):
     rng = np.random.default_rng(1)
@@ -59,6 +76,7 @@ def test_several_prompts(lengths):
 
 # head_dim 256 with an output gate (attn_prompt_wide_kernel) against the general kernel, which pages of 32 tokens take: last rows at both ends of a tile's halves and of the query groups, several
 # sequences in a launch; a second pass whose keys are shared (37 and 200 rows behind 320 and 1024: shares of one tile, and of none, to eight).  The same rows and cache as above: 2e-5.
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv,dtype", [(8, 2, "f16"), (4, 4, "bf16"), (16, 4, "f16")])
 def test_wide_heads(heads, kv, dtype):
     from crane_amd.backend import Model
