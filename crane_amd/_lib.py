@@ -24,7 +24,7 @@ EXPORTS = [
     "cm_forward_step_greedy", "cm_clear_kv", "cm_warmup", "cm_generate", "cm_seq_alloc",
     "cm_seq_free", "cm_seq_fork", "cm_seq_len", "cm_seq_truncate", "cm_seq_forward",
     "cm_decode_batch", "cm_prefill_batch", "cm_step_batch", "cm_image_smart_resize", "cm_image_preprocess", "cm_preprocess_last_error", "cm_image_token_id", "cm_vision_features", "cm_vision_encode", "cm_vlm_forward", "cm_embed_tokens", "cm_forward_embeds", "cm_sample", "cm_topk", "cm_read_logits", "cm_engine_create", "cm_engine_destroy", "cm_engine_submit", "cm_engine_cancel",
-    "cm_gguf_config", "cm_checkpoint_inspect", "cm_tp_shard_plan", "cm_engine_step", "cm_engine_step_many", "cm_engine_has_work", "cm_engine_get_stats", "cm_engine_last_error", "cm_bench_decode", "cm_bench_kernel", "cm_debug_fill_kv", "cm_debug_read", "cm_debug_qgemv", "cm_debug_qgemm", "cm_debug_set", "cm_debug_peer_selftest", "cm_debug_qgemm_plan", "cm_debug_lay_router_plan", "cm_debug_attn_group_plan", "cm_debug_attn_prefill_plan", "cm_debug_lay_tile_plan", "cm_debug_lay_tile_shape", "cm_debug_gemm_band", "cm_debug_gemm_tile", "cm_debug_attn_prompt_pairs", "cm_debug_rope_rows", "cm_debug_gdn_step", "cm_debug_lay_attn_shares", "cm_debug_lay_step_out_plan",
+    "cm_gguf_config", "cm_checkpoint_inspect", "cm_tp_shard_plan", "cm_engine_step", "cm_engine_step_many", "cm_engine_has_work", "cm_engine_get_stats", "cm_engine_last_error", "cm_bench_decode", "cm_bench_kernel", "cm_debug_fill_kv", "cm_debug_read", "cm_debug_qgemv", "cm_debug_qgemm", "cm_debug_set", "cm_debug_peer_selftest", "cm_debug_qgemm_plan", "cm_debug_lay_router_plan", "cm_debug_attn_group_plan", "cm_debug_attn_prefill_plan", "cm_debug_lay_tile_plan", "cm_debug_lay_tile_shape", "cm_debug_gemm_band", "cm_debug_gemm_tile", "cm_debug_prefill_pass", "cm_debug_attn_prompt_pairs", "cm_debug_rope_rows", "cm_debug_gdn_step", "cm_debug_lay_attn_shares", "cm_debug_lay_step_out_plan",
 ]
 
 
@@ -157,6 +157,7 @@ def load():
     lib.cm_debug_lay_tile_plan.argtypes = [C.c_int32] * 6
     lib.cm_debug_gemm_band.argtypes = [C.c_int32] * 4 + [C.c_uint64]
     lib.cm_debug_gemm_tile.argtypes = [C.c_int32] * 4 + [C.c_uint64]
+    lib.cm_debug_prefill_pass.argtypes = [C.c_uint64, C.c_int32, C.c_int32]
     lib.cm_debug_attn_prompt_pairs.argtypes = [C.c_int32] * 4
     lib.cm_debug_rope_rows.argtypes = [f32p, C.c_int32, C.c_int32, C.c_int32, f32p, f32p, f32p]
     lib.cm_debug_gdn_step.argtypes = [f32p, f32p, f32p, C.c_int32, f32p]

@@ -644,6 +644,10 @@ int cm_debug_gdn_step(const float* proj, const float* conv_w, const float* state
     });
 }
 
+int cm_debug_prefill_pass(uint64_t rest, int32_t chunk, int32_t pass_rows) {
+    return rest < 1 || chunk < 1 || pass_rows < chunk ? 0 : cm::prefill_next_pass((size_t)rest, chunk, pass_rows);
+}
+
 int cm_debug_attn_prompt_pairs(int32_t rows, int32_t start, int32_t heads, int32_t kv_heads) {
     if (rows < 1 || start < 0 || heads < 1 || kv_heads < 1) return 0;
     return cm::attn_prefill_shares(rows, start, heads, 128) == 1 && cm::attn_prompt_pairs(rows, start, heads, heads / kv_heads);

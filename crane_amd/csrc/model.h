@@ -126,6 +126,8 @@ struct LayeredDeleter { void operator()(Layered* p) const; };
 struct Rccl;         // dlopen'ed RCCL entry points + communicator, or the peer-store transport of an in-process group (tp.cpp)
 struct PeerShared;   // state shared by the ranks of an in-process tensor-parallel group (tp.h)
 
+int prefill_next_pass(size_t rest, int chunk, int pass_rows);      // rows of the next pass of a prompt of which `rest` are left (host rule)
+
 struct Model {
     Config cfg;
     cm_opts opts{};

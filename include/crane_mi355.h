@@ -553,6 +553,9 @@ int cm_debug_gemm_band(int32_t m, int32_t n, int32_t k, int32_t epi, uint64_t ws
 /* Test hook (host logic only, no GPU): rows * 10000 + columns * 10 + K slices of the tiles that m prompt rows of such a product run on (norm: one of the rows behind it); 0: another kernel. */
 int cm_debug_gemm_tile(int32_t m, int32_t n, int32_t k, int32_t norm, uint64_t ws_floats);
 
+/* Test hook (host logic only, no GPU): rows of the next pass of one prompt of which `rest` are left, where several prompts in a pass have `chunk` and one may have `pass_rows`. */
+int cm_debug_prefill_pass(uint64_t rest, int32_t chunk, int32_t pass_rows);
+
 /* Test hook (host logic only, no GPU): whether `rows` queries of a prompt behind `start` cached tokens, `heads` query heads of 128 on `kv_heads`, take the attention of two heads per workgroup
  * (csrc/kernels_attn_prompt.hip): 1, or the kernel of one: 0. */
 int cm_debug_attn_prompt_pairs(int32_t rows, int32_t start, int32_t heads, int32_t kv_heads);
