@@ -144,8 +144,8 @@ struct GemmArgs {
     int ksplit_cap = 0;        // split-K of the 128-wide kernel: at most this many blocks (0: the default 768; the vision tower passes 512)
     int ksplit;             // set by launch_gemm
     int dbg = 0;            // kernels_gemmw4.hip timing experiments (CM_GEMMW4_DBG); 0 in production
-    int wide256 = 1;        // 0: never the LDS-DMA kernels (kernels_gemm_rows.hip / kernels_gemm256.hip / kernels_gemmw4.hip), 1: automatic, 2: always kernels_gemmw4.hip,
-                            // 3: kernels_gemm256.hip only -- A/B switch, cm_debug_set("gemm256")
+    int wide256 = 1;        // 0: never the LDS-DMA kernels (kernels_gemm_rows.hip / kernels_gemm_tile.hip / kernels_gemm256.hip / kernels_gemmw4.hip), 1: automatic, 2: always kernels_gemmw4.hip,
+                            // 3: kernels_gemm256.hip (hi + lo activations of more than 128 rows: kernels_gemm_tile.hip), rows never in two launches -- A/B switch, cm_debug_set("gemm256")
                             // 4: kernels_gemm_rows.hip where its rule takes the sizes, else as 0 (the head of a decode group)
     // GEPI_RESADD with ldc == N only: ALSO write RMSNorm(C row) * norm_w as bf16 hi + lo planes [M][N] -- the A operand of the NEXT
     // GEMM (rmsnorm_rows_kernel's arithmetic).  Fused into the split-K reduction launch when the GEMM splits K (a large decode

@@ -1198,7 +1198,7 @@ static void leave_slices(GemmArgs& a, int epi, hipStream_t s) {
 // The LDS-DMA kernel on full cache lines (kernels_gemm256.hip; one tile of up to 128 rows with hi + lo activations, 256-row tiles with plain bf16 from 512 rows on)
 // where one of its tile widths fills the chip in whole rounds -- (width, k-slices) by a small cost model: rounds of 256 CUs x one block's MFMA time + the f32 partial-tile traffic of a split.  Returns false when the
 // register-staged kernel should run.
-// the column tile and the K slices of such a product; false: not for that kernel
+// the column tile and the K slices of such a product; false: not for that kernel.  (The environment's BN, KS and MIN_BLOCKS steer these launches alone, not those of kernels_gemm_tile.hip.)
 static bool gemm256_plan(int M, int N, int K, bool lo, size_t ws_floats, bool w4, int* bn_out, int* ks_out) {
     static const int force_bn = getenv("CM_GEMM256_BN") ? atoi(getenv("CM_GEMM256_BN")) : 0;     // tuning
     static const int force_ks = getenv("CM_GEMM256_KS") ? atoi(getenv("CM_GEMM256_KS")) : 0;
@@ -1318,7 +1318,7 @@ static bool try_gemm_rows(GemmArgs& a, int epi, hipStream_t s) {
     return true;
 }
 static bool gemm_tail_columns(int M, int N) { return M >= 256 && N >= 512 && N % 192 != 0 && N % 256 == 128; }
-// Prompt rows over a width that no tile of kernels_gemm256.hip divides because of its last 128 columns (the merged in_proj of a Gated-Delta-Net layer:
+// Prompt rows over a width that no tile of the LDS-DMA kernels divides because of its last 128 columns (the merged in_proj of a Gated-Delta-Net layer:
 // 8192 columns and 32 gate columns padded to 128): the wide part there, the last columns alone.  8320 x 2048, 2048 rows: 180 -> 137 us (a prompt of
 // 2048 / 1024 / 300 tokens 18.6 / 10.8 / 5.54 -> 17.8 / 10.2 / 5.49 ms; width 1024: 12.3 / 7.3 / 4.5 -> 12.0 / 7.2 / 4.5)
 static bool try_gemm_tail(GemmArgs& a, int epi, hipStream_t s) {

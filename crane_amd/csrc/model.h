@@ -243,7 +243,7 @@ struct Model {
     int pass_rows = 2048;       // rows of a pass over one prompt: the chunk or more (prefill_pass_rows), fixed with the first prompt
     bool prefill_ready = false;          // every buffer is there (set last)
     bool prefill_ok = false, prefill_split2 = true;
-    int gemm256 = 1;           // prompt-pass / decode-group GEMMs: 0 = never an LDS-DMA kernel, 1 = automatic, 2 = always kernels_gemmw4.hip, 3 = kernels_gemm256.hip only (cm_debug_set("gemm256"))
+    int gemm256 = 1;           // prompt-pass / decode-group GEMMs: 0 = never an LDS-DMA kernel, 1 = automatic, 2 = always kernels_gemmw4.hip, 3 = kernels_gemm256.hip, and kernels_gemm_tile.hip for more than 128 rows with hi + lo activations, each product in one launch (cm_debug_set("gemm256"))
     float* pX = nullptr;        // [pass_rows, H] f32 residual stream
     float* pWS = nullptr;       // split-K workspace of the prefill GEMMs: at most 1024 partial tiles of 128 x 128 f32
     static constexpr size_t gemm_ws_floats = (size_t)1024 * 128 * 128;

@@ -587,7 +587,7 @@ int cm_debug_attn_prefill_plan(int32_t rows, int32_t start, int32_t heads, int32
  * pages never / where it fits on attn_decode_group_kernel, whatever the thresholds above 0; "engine" = 0 / 1 and "engine_full" = 0 / 1: the persistent decode
  * kernel off / on and its per-layer / whole-token mode (only where cm_create found the shapes eligible); "quant_act_int" = 1 / 0
  * and "vision_merger_gelu" = 1 (tanh) / 2 (erf): CM_QUANT_ACT and CM_VISION_MERGER_GELU of the live model; "gemm256" = 0 / 1: the
- * LDS-DMA GEMM of the prompt pass and of large decode groups; "lm_head_gemm_min" = n: decode groups of n or more sequences run
+ * LDS-DMA GEMMs of the prompt pass and of decode groups (3: without those of few rows and with every product in one launch); "lm_head_gemm_min" = n: decode groups of n or more sequences run
  * lm_head as one GEMM + row arg-max (0 = never); "sample_rows" = 0 / 1: the engine's sampled rows through the per-row sampler /
  * one set of launches for all rows (same tokens); "tp_graph" = 0 / 1: RCCL collectives launched eagerly / captured into the
  * decode hipGraph (CM_TP_GRAPH); "prefill_seg_batch" = 0 / 1: cm_prefill_batch launches RoPE / KV append / attention once per

@@ -1,4 +1,4 @@
-"""GPU: the products of long prompts on 128-row tiles (kernels_gemm256.hip) against the 128-column kernel.
+"""GPU: the products of long prompts on the LDS-DMA tiles (kernels_gemm_tile.hip) against the 128-column kernel.
 
 The same prompt with cm_debug_set("gemm256") 1 (automatic) and 0.  Where K is not split both add the same products in the same order; where it is, a sum of
 K <= 6144 terms moves by about sqrt(K) 2^-24 of its size, 5e-6, and a K or V element lands on the other side of a bf16 boundary with probability 5e-6 / 2^-8, one in

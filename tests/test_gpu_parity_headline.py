@@ -198,10 +198,10 @@ def test_large_decode_groups_at_longer_contexts_and_their_fused_launches(name, n
 
 @pytest.mark.parametrize("split", [0, 1])
 def test_wide_gemm_kernel_is_bit_equal_to_the_128_row_kernel(split):
-    """The 256-row LDS-DMA GEMM (kernels_gemm256.hip: global_load_lds tiles, source-side bank swizzle, three LDS stages behind a
-    counted vmcnt) multiplies the same k-tiles in the same order into every accumulator as gemm_bf16_kernel: a 1024-token prompt
-    through either kernel must give IDENTICAL logits wherever neither launch splits K (gate||up at 1024 rows: 256 x 192 tiles),
-    and logits within the split-K summation order elsewhere.  Parity mode (hi + lo planes) and plain bf16 activations."""
+    """The LDS-DMA GEMMs (global_load_lds tiles, source-side bank swizzle: kernels_gemm_tile.hip for hi + lo activations, split 0; kernels_gemm256.hip
+    for plain bf16 ones, split 1) multiply the same k-tiles in the same order into every accumulator as gemm_bf16_kernel: a prompt
+    through either kernel gives the same sums wherever neither launch splits K, and logits within the split-K summation order elsewhere.  (Every bit, where no product is split:
+    tests/test_gpu_gemm_tile.py.)"""
     cfg = configs.get_config("qwen3-8b-2l")
     V = cfg["vocab_size"]
     m = Model.synthetic(cfg, seed=0, max_seq_len=2048, max_seqs=1, prefill_split=split)
@@ -210,7 +210,7 @@ def test_wide_gemm_kernel_is_bit_equal_to_the_128_row_kernel(split):
         for n in (1024, 1536):                       # 4 and 6 m-tiles of 256 rows (1536: a ragged tile count for the XCD order)
             ids = configs.synthetic_prompt(n, V)
             pair = []
-            for mode in (0, 3, 2):                   # 128-row kernel, kernels_gemm256.hip, kernels_gemmw4.hip (round 6: one wave per SIMD, 32 x 32 x 16 MFMAs)
+            for mode in (0, 3, 2):                   # 128-row kernel, kernels_gemm_tile.hip / kernels_gemm256.hip, kernels_gemmw4.hip (round 6: one wave per SIMD, 32 x 32 x 16 MFMAs)
                 m.debug_set("gemm256", mode)
                 m.clear_kv_cache()
                 pair.append(m.forward_step(ids, 0)[0, 0].copy())
