@@ -1363,8 +1363,9 @@ int gemm_band(int M, int N, int K, int epi, size_t ws_floats, int ksplit_cap) {
 // A round of blocks that the last tiles fill to a part takes as long as a full one: a band of rows whose tiles fill their rounds first, the rows behind it on
 // the kernel that suits so few.  What bounds either band is what bounded the whole; the second reads the weights again.  One launch / two, us of prompts through eight layers: width 4096, 645 tokens
 // 4525 / 4388 (gate and up 512 + 133), 768 4726 / 4521, 1040 6877 / 5918 (1024 + 16 in three products), 1152 7053 / 6478, 1400 7814 / 7608 (down 384 + 1016); width 2048 with Gated-Delta-Net layers,
-// 1290 3546 / 3378, 2060 5427 / 4848, 2304 5718 / 5475, 4165 9739 / 8647.  The line is a gain of 5 % and 8 us by the figures above, which are 5 % off: a band by less of a gain was as often a loss (width
-// 5120, 2000 tokens 10.83 / 11.03 ms), and 5 % alone lost in the products of width 1024, a launch and a reduction more for a round of 30 us.  Rows of products with an activation behind them and the
+// 1290 3546 / 3378, 2060 5427 / 4848, 2304 5718 / 5475, 4165 9739 / 8647.  The line is a gain of 5 % and 8 us by the figures above, which are 5 % off: with 5 % alone the products of width
+// 1024 lost, a launch and a reduction more for a round of 30 us.  Width 5120, whose sizes the tiles' prices were not fitted to: 19 of 21 lengths gain up to 10 %, 960 and 2000 tokens lose 1.6 %.
+// Rows of products with an activation behind them and the
 // vision tower's norm stay in one launch (not measured).
 static bool try_gemm_bands(GemmArgs& a, int epi, hipStream_t s) {
     if (a.A_lo == nullptr || a.wide256 != 1 || a.norm_b != nullptr) return false;
